@@ -135,6 +135,21 @@ int launch_gemm_backward(const GemmArgs& dgrad, const GemmArgs& wgrad, bool half
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, bool half, int out_dtype,
                        int splits, bool wide_tiles, float* ws, hipStream_t stream);
 
+// GEMMs of shapes that are not made of whole tiles (gemm_edge.h), on the tile the caller
+// picks: any M, N, contraction and operand size, row strides below kEdgeMaxLd elements (half
+// of that on the tiles of 256 rows).
+enum EdgeTile { EDGE_256x256 = 0, EDGE_256x128 = 1, EDGE_128x128 = 2 };
+constexpr int64_t kEdgeMaxLd = 1LL << 23;
+int launch_gemm_edge_bf16(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32,
+                          EdgeTile tile, hipStream_t stream);
+int launch_gemm_edge_f16(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32,
+                         EdgeTile tile, hipStream_t stream);
+// Both gradients of a layer in one launch of 256 x 256 tiles; tiles_m, tiles_n and wg_first set.
+int launch_gemm_edge_backward_bf16(const GemmArgs& wgrad, const GemmArgs& dgrad, bool dw_f32,
+                                   hipStream_t stream);
+int launch_gemm_edge_backward_f16(const GemmArgs& wgrad, const GemmArgs& dgrad, bool dw_f32,
+                                  hipStream_t stream);
+
 // C = silu(A B^T) * (A B2^T) in one launch (both weight matrices [N][Kc], K-major), for
 // M % 256 == 0, N % 128 == 0, Kc % 64 == 0 and operands below 2 GiB; AXN_ESHAPE otherwise.
 int launch_gemm_swiglu(const GemmArgs& args, bool half, hipStream_t stream);

@@ -1,0 +1,148 @@
+// MFMA GEMMs of shapes that are not made of whole tiles (ragged token counts, odd
+// vocabularies, contractions that are not multiples of 64) and of operands of 2 GiB and more:
+// solo_gemm with EDGE.  Included once per element type (gemm_edge_bf16.hip, gemm_edge_f16.hip:
+// the instances of one type take as long to compile as all of gemm_bf16.hip).
+//
+// What bounds these: the same as the whole-tile kernels (MFMA issue and power), plus the work
+// done for padding, at most one tile row and column.  They replaced a register-staged kernel
+// (128 x 128 tiles, global -> VGPR -> LDS, one barrier per step, 32x32x16 MFMAs).  Measured on
+// MI355X, bf16 unless stated, before -> after:
+//   forward   777 x 14336 x 4096   165 -> 99 us (560 -> 920 TFLOP/s)
+//   forward  3001 x 10240 x 2560   237 -> 166 us (fp16, fp32 result with bias)
+//   backward of the same layer     468 -> 324 us (both products in one launch)
+//   forward  2048 x 50264 x 2048   572 -> 355 us (740 -> 1190 TFLOP/s)
+#pragma once
+#include <atomic>
+
+#include "gemm_solo.h"
+
+namespace axn {
+namespace {
+
+template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF>
+__global__ void __launch_bounds__(256) gemm_edge_kernel(const GemmArgs g) {
+  solo_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, true>(g);
+}
+
+// Both gradients of a layer in one launch, as gemm_backward_kernel.
+template <bool HALF, bool DW_F32>
+__global__ void __launch_bounds__(256) gemm_edge_backward_kernel(const GemmArgs gw, const GemmArgs gd) {
+  const int b = (int)blockIdx.x;
+  if (b >= gw.wg_first && b < gw.wg_first + gw.tiles_m * gw.tiles_n)
+    solo_gemm<256, 256, false, false, AXN_EPI_NONE, DW_F32, HALF, true>(gw);
+  else
+    solo_gemm<256, 256, true, false, AXN_EPI_NONE, false, HALF, true>(gd);
+}
+
+template <int BM, int BN, bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
+int launch_edge_tile(const GemmArgs& in, hipStream_t stream) {
+  GemmArgs g = in;
+  constexpr int COLS = EPI == EPI_SWIGLU ? BN / 2 : BN;   // output columns of a tile
+  g.tiles_m = (g.M + BM - 1) / BM;
+  g.tiles_n = (g.N + COLS - 1) / COLS;
+  const long long nwg = (long long)g.tiles_m * g.tiles_n * (g.splits > 1 ? g.splits : 1);
+  if (nwg > 0x7fffffffLL) {
+    set_error("gemm: too many output tiles (%lld)", nwg);
+    return AXN_ELIMIT;
+  }
+  constexpr size_t lds = 5 * BM * 64 * 2;   // five slots of the A tile's size
+  void (*kern)(const GemmArgs) = gemm_edge_kernel<BM, BN, AK, BKM, EPI, OUT_F32, HALF>;
+  {
+    static std::atomic<unsigned long long> lds_allowed{0};   // per template instance
+    const int rc = allow_lds((const void*)kern, lds, lds_allowed);
+    if (rc != AXN_OK) return rc;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(256), lds, stream, g);
+  AXN_HIP_TRY(hipGetLastError());
+  return AXN_OK;
+}
+
+// Full rounds and the rest, as launch_shape of gemm_bf16.hip cuts whole-tile problems: a last
+// round of at most half of the CUs goes to smaller tiles in a launch of its own.
+template <bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
+int launch_edge_kind(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
+  if (tile == EDGE_128x128) return launch_edge_tile<128, 128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
+  if (tile == EDGE_256x128) return launch_edge_tile<256, 128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
+  const long long tm = (g.M + 255) / 256, tn = (g.N + 255) / 256, tiles = tm * tn;
+  const long long full = tiles / 256 * 256, rest = tiles - full;
+  if (g.splits <= 1 && full > 0 && rest > 0 && rest <= 128 && (full % tm == 0 || full % tn == 0)) {
+    constexpr int64_t esz = OUT_F32 ? 4 : 2;
+    GemmArgs g1 = g, g2 = g;
+    if (full % tm == 0) {  // whole tile columns
+      const int64_t n1 = full / tm * 256;
+      g1.N = (int)n1;
+      g2.N = g.N - (int)n1;
+      g2.B = BKM ? g.B + n1 * g.ldb : g.B + n1;
+      if (g.B2 != nullptr) g2.B2 = BKM ? g.B2 + n1 * g.ldb : g.B2 + n1;
+      g2.C = (char*)g.C + n1 * esz;
+      if (g.bias != nullptr) g2.bias = g.bias + n1;
+      if (g.Z != nullptr) g2.Z = g.Z + n1;
+    } else {  // whole tile rows
+      const int64_t m1 = full / tn * 256;
+      g1.M = (int)m1;
+      g2.M = g.M - (int)m1;
+      g2.A = AK ? g.A + m1 * g.lda : g.A + m1;
+      if (g.A2 != nullptr) g2.A2 = AK ? g.A2 + m1 * g.lda : g.A2 + m1;
+      g2.C = (char*)g.C + m1 * g.ldc * esz;
+      if (g.Z != nullptr) g2.Z = g.Z + m1 * g.ldc;
+    }
+    const int rc = launch_edge_tile<256, 256, AK, BKM, EPI, OUT_F32, HALF>(g1, stream);
+    if (rc != AXN_OK) return rc;
+    return rest > 64 ? launch_edge_tile<256, 128, AK, BKM, EPI, OUT_F32, HALF>(g2, stream)
+                     : launch_edge_tile<128, 128, AK, BKM, EPI, OUT_F32, HALF>(g2, stream);
+  }
+  return launch_edge_tile<256, 256, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
+}
+
+template <bool HALF>
+int launch_edge_layout(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, EdgeTile tile,
+                       hipStream_t stream) {
+  switch (layout) {
+    case GEMM_NT:
+      if (out_f32) {
+        if (epilogue == AXN_EPI_BIAS) return launch_edge_kind<true, true, AXN_EPI_BIAS, true, HALF>(g, tile, stream);
+        if (epilogue == AXN_EPI_BIAS_GELU)
+          return launch_edge_kind<true, true, AXN_EPI_BIAS_GELU, true, HALF>(g, tile, stream);
+        break;
+      }
+      switch (epilogue) {
+        case AXN_EPI_NONE:
+          return launch_edge_kind<true, true, AXN_EPI_NONE, false, HALF>(g, tile, stream);
+        case AXN_EPI_BIAS:
+          return launch_edge_kind<true, true, AXN_EPI_BIAS, false, HALF>(g, tile, stream);
+        case AXN_EPI_BIAS_GELU:
+          return launch_edge_kind<true, true, AXN_EPI_BIAS_GELU, false, HALF>(g, tile, stream);
+        case AXN_EPI_GELU:
+          return launch_edge_kind<true, true, AXN_EPI_GELU, false, HALF>(g, tile, stream);
+      }
+      break;
+    case GEMM_NN:
+      if (out_f32 || epilogue != AXN_EPI_NONE) break;
+      return launch_edge_kind<true, false, AXN_EPI_NONE, false, HALF>(g, tile, stream);
+    case GEMM_TN:
+      if (epilogue != AXN_EPI_NONE) break;
+      return out_f32 ? launch_edge_kind<false, false, AXN_EPI_NONE, true, HALF>(g, tile, stream)
+                     : launch_edge_kind<false, false, AXN_EPI_NONE, false, HALF>(g, tile, stream);
+  }
+  set_error("gemm: unsupported layout/epilogue/output combination");
+  return AXN_EINVAL;
+}
+
+template <bool HALF>
+int launch_edge_backward(const GemmArgs& gw, const GemmArgs& gd, bool dw_f32, hipStream_t stream) {
+  constexpr size_t lds = 5 * 256 * 64 * 2;
+  void (*kern)(const GemmArgs, const GemmArgs) =
+      dw_f32 ? gemm_edge_backward_kernel<HALF, true> : gemm_edge_backward_kernel<HALF, false>;
+  {
+    static std::atomic<unsigned long long> lds_allowed[2];   // per output type of dW
+    const int rc = allow_lds((const void*)kern, lds, lds_allowed[dw_f32 ? 1 : 0]);
+    if (rc != AXN_OK) return rc;
+  }
+  const unsigned nwg = (unsigned)(gw.tiles_m * gw.tiles_n + gd.tiles_m * gd.tiles_n);
+  hipLaunchKernelGGL(kern, dim3(nwg), dim3(256), lds, stream, gw, gd);
+  AXN_HIP_TRY(hipGetLastError());
+  return AXN_OK;
+}
+
+}  // namespace
+}  // namespace axn

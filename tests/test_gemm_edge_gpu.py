@@ -1,0 +1,104 @@
+"""The GEMM kernels with bounds (shapes that are not made of whole tiles) at the sizes where
+they can go wrong: one element around tile edges, contractions that end inside a 64-deep
+stage, outputs that need one, several and cut rounds of tiles.
+
+Operands are small whole numbers, so every partial sum is exact in fp32 and the expected
+result is exact too: the float64 product rounded once to the storage type.  The operands are
+views into buffers whose other elements are NaN, and the outputs views into buffers filled
+with a canary: what lies outside a view is neither read into a result nor written."""
+
+import pytest
+import torch
+
+from axonn_amd import _native as nv
+
+pytestmark = pytest.mark.gpu
+
+CANARY = 7.0
+
+
+def numbers(rows, cols, dtype, gen, pad):
+    """A [rows, cols] view of whole numbers -2 .. 2, NaN around it."""
+    full = torch.full((rows + 3, cols + pad), float("nan"), dtype=dtype, device="cuda")
+    view = full[:rows, :cols]
+    view.copy_(torch.randint(-2, 3, (rows, cols), generator=gen, device="cuda"))
+    return view
+
+
+def canvas(rows, cols, dtype):
+    full = torch.full((rows + 2, cols + 8), CANARY, dtype=dtype, device="cuda")
+    return full, full[:rows, :cols]
+
+
+def check(full, view, want):
+    assert torch.equal(view.double(), want.to(view.dtype).double())
+    view.fill_(CANARY)
+    assert torch.equal(full, torch.full_like(full, CANARY)), "written outside the output"
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 8), (127, 120, 56), (129, 136, 72), (255, 264, 64), (257, 248, 136), (300, 392, 200),
+    (64, 1000, 24), (1000, 128, 1032), (777, 2056, 328),
+    (2049, 2304, 128),      # 9 x 9 tiles of 256 x 128 columns and rows
+    (4000, 4360, 72),       # 288 large tiles: a full round and a cut rest
+    (4100, 4104, 64),       # 289 large tiles that no cut divides
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_edge_kernels_are_exact_and_stay_inside_their_operands(M, N, K, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+    X, W, dY = (numbers(r, c, dtype, gen, 16) for r, c in ((M, K), (N, K), (M, N)))
+    code, ld = nv.dtype_code(dtype), lambda t: t.stride(0)
+    sfx = "" if dtype == torch.bfloat16 else "_f16"
+    stream = nv.current_stream()
+    bias = torch.randint(-3, 4, (N,), generator=gen, device="cuda").float()
+
+    full, y = canvas(M, N, dtype)
+    nv.call("axn_gemm_fwd" + sfx, nv.ptr(X), nv.ptr(W), None, nv.ptr(y), None, M, N, K, ld(X), ld(W),
+            ld(y), nv.EPI_NONE, stream)
+    product = X.double() @ W.double().t()
+    check(full, y, product)
+    nv.call("axn_gemm_fwd" + sfx, nv.ptr(X), nv.ptr(W), nv.ptr(bias), nv.ptr(y), None, M, N, K, ld(X),
+            ld(W), ld(y), nv.EPI_BIAS, stream)
+    check(full, y, product + bias)
+    full32, y32 = canvas(M, N, torch.float32)
+    nv.call("axn_gemm_fwd_f32out", nv.ptr(X), nv.ptr(W), nv.ptr(bias), nv.ptr(y32), None, code, M, N, K,
+            ld(X), ld(W), ld(y32), nv.EPI_BIAS, stream)
+    check(full32, y32, product + bias)
+
+    full, dx = canvas(M, K, dtype)
+    nv.call("axn_gemm_dgrad" + sfx, nv.ptr(dY), nv.ptr(W), nv.ptr(dx), M, N, K, ld(dY), ld(W), ld(dx), stream)
+    want_dx = dY.double() @ W.double()
+    check(full, dx, want_dx)
+
+    full, dw = canvas(N, K, torch.float32)
+    want_dw = dY.double().t() @ X.double()
+    for beta in (0, 1):
+        dw.fill_(3.0)
+        nv.call("axn_gemm_wgrad" + sfx, nv.ptr(dY), nv.ptr(X), nv.ptr(dw), M, N, K, ld(dY), ld(X), ld(dw),
+                beta, nv.F32, stream)
+        check(full, dw, want_dw + 3.0 * beta)
+    # both gradients through the joint entry point, dW in the operands' type
+    fullx, dx = canvas(M, K, dtype)
+    fullw, dw = canvas(N, K, dtype)
+    nv.call("axn_gemm_bwd", nv.ptr(dY), nv.ptr(W), nv.ptr(X), nv.ptr(dx), nv.ptr(dw), code, M, N, K, ld(dY),
+            ld(W), ld(X), ld(dx), ld(dw), 0, code, stream)
+    check(fullx, dx, want_dx)
+    check(fullw, dw, want_dw)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 136, 72), (300, 2056, 200)])
+def test_edge_epilogues_keep_the_pre_activation(M, N, K):
+    """GELU on whole-number pre-activations: the saved Z is exact, Y within one rounding of
+    the exact function of Z (2^-8 relative for bfloat16) plus the erf's 1.5e-7."""
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    X, W = (numbers(r, c, torch.bfloat16, gen, 8) for r, c in ((M, K), (N, K)))
+    bias = torch.randint(-3, 4, (N,), generator=gen, device="cuda").float()
+    for b, epi in ((bias, nv.EPI_BIAS_GELU), (None, nv.EPI_GELU)):
+        fz, z = canvas(M, N, torch.bfloat16)
+        fy, y = canvas(M, N, torch.bfloat16)
+        nv.call("axn_gemm_fwd", nv.ptr(X), nv.ptr(W), nv.ptr(b), nv.ptr(y), nv.ptr(z), M, N, K, X.stride(0),
+                W.stride(0), y.stride(0), epi, nv.current_stream())
+        pre = X.double() @ W.double().t() + (0 if b is None else b)
+        want = torch.nn.functional.gelu(pre)
+        assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2e-7 * pre.abs().clamp(min=1)).all())
+        check(fz, z, pre)

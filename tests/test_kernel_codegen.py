@@ -82,6 +82,18 @@ def test_main_loop_mfma_operands_have_fixed_register_classes(gemm_asm):
                 assert ops[1].startswith("v[") and ops[2].startswith("v["), (name, s)
 
 
+@pytest.mark.parametrize("source", ["gemm_edge_bf16", "gemm_edge_f16"])
+def test_kernels_with_bounds_keep_the_same_properties(tmp_path_factory, source):
+    """No spills, and the accumulators' wait behind the last MFMA, also where the stores are
+    guarded and the columns behind the last multiple of 8 take another way."""
+    kernels = {k: v for k, v in _device_asm(tmp_path_factory, source).items() if "gemm_edge" in k}
+    assert len(kernels) >= 29, sorted(kernels)   # 9 layouts and epilogues x 3 tiles, the joint backward x 2
+    test_solo_kernels_do_not_spill(kernels)
+    test_accumulators_stay_in_their_registers_until_the_last_mfma_has_retired(kernels)
+    for body in kernels.values():
+        assert "v_mfma_f32_16x16x32_" + source.rsplit("_", 1)[1] in body
+
+
 _ASM_CACHE = {}
 
 

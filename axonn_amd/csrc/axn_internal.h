@@ -150,6 +150,12 @@ int launch_gemm_edge_backward_bf16(const GemmArgs& wgrad, const GemmArgs& dgrad,
 int launch_gemm_edge_backward_f16(const GemmArgs& wgrad, const GemmArgs& dgrad, bool dw_f32,
                                   hipStream_t stream);
 
+// Forward products of at most kStreamTokens rows (gemm_stream.hip): a stream over the weights;
+// row strides below kStreamMaxLd elements.
+constexpr int kStreamTokens = 32;
+constexpr int64_t kStreamMaxLd = 1LL << 24;
+int launch_gemm_stream(const GemmArgs& args, int epilogue, bool out_f32, bool half, hipStream_t stream);
+
 // C = silu(A B^T) * (A B2^T) in one launch (both weight matrices [N][Kc], K-major), for
 // M % 256 == 0, N % 128 == 0, Kc % 64 == 0 and operands below 2 GiB; AXN_ESHAPE otherwise.
 int launch_gemm_swiglu(const GemmArgs& args, bool half, hipStream_t stream);

@@ -319,6 +319,9 @@ int launch_split(const GemmArgs& g, bool wide_tiles, hipStream_t stream) {
 template <bool HALF>
 int launch_layout(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32,
                   hipStream_t stream) {
+  if (layout == GEMM_NT && g.M <= kStreamTokens && g.lda < kStreamMaxLd && g.ldb < kStreamMaxLd &&
+      (!out_f32 || epilogue == AXN_EPI_BIAS || epilogue == AXN_EPI_BIAS_GELU))
+    return launch_gemm_stream(g, epilogue, out_f32, HALF, stream);
   switch (layout) {
     case GEMM_NT:
       if (out_f32) {  // 16-bit product + fp32 bias promoted to fp32, as `x + bias` promotes it

@@ -1,0 +1,209 @@
+// Forward products of a few tokens, Y[M, N] = X[M, K] W[N, K]^T with M up to a few dozen (token
+// by token generation, small requests): the weights are read once and hardly computed
+// with, so the kernel is a stream over W with the MFMAs on the side.
+//
+// One workgroup owns 16 R rows of W and all tokens; its waves take the contraction in turn,
+// 64 elements (a 128-byte line of every row) at a time, each through a ring of its own in
+// LDS: no barrier in the loop.  Straight loads into MFMA fragments were the first version:
+// v_mfma_f32_16x16x32 wants 16 rows in 16 consecutive lanes, and a load whose neighbouring lanes
+// lie in different lines runs at a quarter of the L1 rate (2.0 to 3.4 TB/s of weights).  Copies
+// to LDS move whole lines (8 lanes each) and the fragments are read back swizzled
+// (DeepOperand's layout: chunk c of row r at c ^ ((r >> 1) & 7)).  With W as the row operand a
+// lane ends with 4 consecutive output columns of one token.  The waves' sums meet in LDS and
+// are added in wave order, so results do not depend on timing.
+//
+// What bounds it: the weights' way from HBM, and the tokens' from L2, which every workgroup
+// reads again (a CU takes about 60 KB/us in all).  So the workgroups are as tall as it takes
+// to fit one round of the 256 CUs (launch_stream_rows).  Measured on MI355X, cold weights, us:
+//   N x K            16 tokens         32 tokens   register-staged / bounded tile kernel, 16
+//   4096 x 4096      8.0 (4.2 TB/s)    9.9         82 / 52
+//   6144 x 4096      10.8 (4.7 TB/s)   13.0        75 / 54
+//   14336 x 4096     19.6 (6.0 TB/s)   21.1        78 / 62
+//   4096 x 14336     22.3 (5.3 TB/s)   29.8        247 / 161
+//   (about 2.5 us of each are the launch; without the reads of X 16 tokens take 1 to 2 us less)
+#include "gemm_solo.h"
+
+namespace axn {
+namespace {
+
+// D: lines of the contraction a wave has on their way (its ring's slots).
+template <int MT, int R, int NW, int D, int EPI, bool OUT_F32, bool HALF>
+__global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) {
+  constexpr int GROUPS = R + MT;              // 16-row groups copied per line: W's, then X's
+  constexpr uint32_t LINE = GROUPS * 2048;    // bytes of a slot
+  constexpr int COPIES = 2 * GROUPS;
+  static_assert(COPIES * (D - 1) < 64, "outstanding copies the wait can count");
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int n0 = blockIdx.x * (16 * R);
+  char* ring = lds + wave * (D * LINE);
+
+  // Copies: 8 rows of 128 bytes each.  Rows past the end are outside the buffer and come as
+  // zeros; so do the chunks past the contraction's end in its last line.
+  constexpr uint32_t kOutside = 0x80000000u;
+  auto resource = [&](const uint16_t* base, int rows, int64_t ld, int row0) {
+    const int64_t left = ((int64_t)(rows - 1 - row0) * ld + g.Kc) * 2;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(base + row0 * ld), 0, (int)(left < 0x7fffffff ? left : 0x7fffffff),
+                                             0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t rw = resource(g.B, g.N, g.ldb, n0), rx = resource(g.A, g.M, g.lda, 0);
+  uint32_t vw[2], vx[2];   // copy h of a group: rows 8 h .. 8 h + 7
+  int chunk[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int row = 8 * h + (lane >> 3);
+    chunk[h] = (lane & 7) ^ ((row >> 1) & 7);
+    vw[h] = (uint32_t)(row * g.ldb * 2 + chunk[h] * 16);
+    vx[h] = (uint32_t)(row * g.lda * 2 + chunk[h] * 16);
+  }
+  const uint32_t w_group = (uint32_t)(16 * g.ldb * 2), x_group = (uint32_t)(16 * g.lda * 2);
+  const int lines = (g.Kc + 63) / 64;
+  // Workgroups start at different lines: all at the same one, with power-of-two row strides,
+  // they crowd onto few memory channels (N = 14336, R = 2: 27.7 -> 21.4 us).
+  const int rot = (int)((blockIdx.x * 7u) % (unsigned)lines);
+  const int mine = (lines - wave + NW - 1) / NW;   // lines wave, wave + NW, ... (may be 0 or less)
+  auto copy_line = [&](int i) {                    // the wave's i-th line into slot i % D
+    int line = wave + i * NW + rot;
+    if (line >= lines) line -= lines;
+    const int k0 = line * 64;
+    char* to = ring + (i % D) * LINE;
+    const bool cut = k0 + 64 > g.Kc;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool out = cut && k0 + 8 * chunk[h] >= g.Kc;
+      const uint32_t ow = out ? kOutside : vw[h], ox = out ? kOutside : vx[h];
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, LDS_PTR(void, to + j * 2048 + h * 1024), 16, (int)ow,
+                                                 (int)(k0 * 2 + j * w_group), 0, 2);   // non-temporal: read once (4 % on the kernel)
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, LDS_PTR(void, to + (R + j) * 2048 + h * 1024), 16, (int)ox,
+                                                 (int)(k0 * 2 + j * x_group), 0, 0);
+    }
+  };
+
+  f32x4 acc[MT][R];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < R; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto mfma = [&](const bf16x8& a, const bf16x8& b, f32x4& c) {
+    if constexpr (HALF)
+      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c,
+                                                 0, 0, 0);
+    else
+      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  };
+
+  const uint32_t ring0 = (uint32_t)(uintptr_t)LDS_PTR(char, ring);
+  const uint32_t frag0 = (uint32_t)(r * 128 + ((q ^ ((r >> 1) & 7)) << 4));        // first 32 elements
+  const uint32_t frag1 = (uint32_t)(r * 128 + (((4 + q) ^ ((r >> 1) & 7)) << 4));  // last 32
+  auto multiply_line = [&](int i) {
+    const uint32_t at = ring0 + (uint32_t)(i % D) * LINE;
+    bf16x8 f[GROUPS][2];
+    static_for<GROUPS>([&](auto j_) {
+      constexpr int J = decltype(j_)::value;
+      f[J][0] = lds_read_b128<J * 2048>(at + frag0);
+      f[J][1] = lds_read_b128<J * 2048>(at + frag1);
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < GROUPS; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(f[j][h]));   // used behind the wait only
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i2 = 0; i2 < MT; ++i2)
+#pragma unroll
+        for (int j = 0; j < R; ++j) mfma(f[j][h], f[R + i2][h], acc[i2][j]);
+  };
+
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+    if (i < mine) copy_line(i);
+  int i = 0;
+  for (; i + D < mine; ++i) {        // line i has landed when only the D - 1 behind it are on their way
+    wait_vmcnt<COPIES * (D - 1)>();
+    multiply_line(i);
+    copy_line(i + D);                // into the slot whose fragments are in registers now
+  }
+  wait_vmcnt<0>();
+  for (; i < mine; ++i) multiply_line(i);
+
+  // The rings are free once every wave is here.
+  __syncthreads();
+  f32x4* part = (f32x4*)lds;         // [NW][MT * R][64]
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < R; ++j) part[(wave * (MT * R) + m * R + j) * 64 + lane] = acc[m][j];
+  __syncthreads();
+  for (int b = wave; b < MT * R; b += NW) {
+    f32x4 s = part[b * 64 + lane];
+#pragma unroll
+    for (int v = 1; v < NW; ++v) s += part[(v * (MT * R) + b) * 64 + lane];
+    const int row = 16 * (b / R) + r, col = n0 + 16 * (b % R) + 4 * q;
+    if (row >= g.M) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col + e < g.N) store_one<EPI, OUT_F32, HALF>(s[e], g, row, col + e);
+  }
+}
+
+template <int MT, int R, int NW, int D, bool HALF>
+int launch_stream(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
+  constexpr size_t ring = (size_t)NW * D * (R + MT) * 2048, sums = (size_t)NW * MT * R * 1024;
+  constexpr size_t lds = ring > sums ? ring : sums;
+  const dim3 grid((unsigned)((g.N + 16 * R - 1) / (16 * R))), block(NW * 64);
+#define STREAM(EPI, F32)                                                                   \
+  {                                                                                        \
+    void (*kern)(const GemmArgs) = gemm_stream_kernel<MT, R, NW, D, EPI, F32, HALF>;       \
+    static std::atomic<unsigned long long> lds_allowed{0};                                 \
+    const int rc = allow_lds((const void*)kern, lds, lds_allowed);                         \
+    if (rc != AXN_OK) return rc;                                                           \
+    hipLaunchKernelGGL(kern, grid, block, lds, stream, g);                                 \
+  }
+  if (out_f32) {
+    if (epilogue == AXN_EPI_BIAS) STREAM(AXN_EPI_BIAS, true)
+    else STREAM(AXN_EPI_BIAS_GELU, true)
+  } else {
+    switch (epilogue) {
+      case AXN_EPI_NONE: STREAM(AXN_EPI_NONE, false) break;
+      case AXN_EPI_BIAS: STREAM(AXN_EPI_BIAS, false) break;
+      case AXN_EPI_BIAS_GELU: STREAM(AXN_EPI_BIAS_GELU, false) break;
+      default: STREAM(AXN_EPI_GELU, false)
+    }
+  }
+#undef STREAM
+  AXN_HIP_TRY(hipGetLastError());
+  return AXN_OK;
+}
+
+// The smallest R whose workgroups fit one round of the CUs: a second round costs more than
+// taller workgroups (5120 x 4096, 16 tokens: 320 workgroups of 16 rows 12.3 us, 160 of 32
+// rows 10.5; 4096 x 4096: 256 of 16 rows 8.0, 128 of 32 rows 10.1).
+template <int MT, int D1, int D2, bool HALF>
+int launch_stream_rows(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
+  if (g.N <= 16 * 256) return launch_stream<MT, 1, 4, D1, HALF>(g, epilogue, out_f32, stream);
+  if (g.N <= 32 * 256) return launch_stream<MT, 2, 4, D2, HALF>(g, epilogue, out_f32, stream);
+  return launch_stream<MT, 4, 4, 2, HALF>(g, epilogue, out_f32, stream);
+}
+
+template <bool HALF>
+int launch_stream_tokens(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
+  if (g.M <= 16) return launch_stream_rows<1, 4, 3, HALF>(g, epilogue, out_f32, stream);
+  return launch_stream_rows<2, 4, 2, HALF>(g, epilogue, out_f32, stream);
+}
+
+}  // namespace
+
+int launch_gemm_stream(const GemmArgs& g, int epilogue, bool out_f32, bool half, hipStream_t stream) {
+  return half ? launch_stream_tokens<true>(g, epilogue, out_f32, stream)
+              : launch_stream_tokens<false>(g, epilogue, out_f32, stream);
+}
+
+}  // namespace axn

@@ -1,0 +1,61 @@
+"""The forward kernel of a few tokens at the sizes where it can go wrong: one token to the last
+it takes, outputs around its 16-, 32- and 64-row workgroups, contractions shorter than a line,
+ending inside one, and with fewer lines than a workgroup has waves.
+
+Operands are small whole numbers (every sum is exact in fp32) inside buffers of NaN, so the
+expected result is the float64 product rounded once and anything read outside shows."""
+
+import pytest
+import torch
+
+from axonn_amd import _native as nv
+
+pytestmark = pytest.mark.gpu
+
+CANARY = 7.0
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(8, 8), (24, 64), (1000, 72), (4096, 328), (4104, 1024), (8200, 264), (16392, 200)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_few_tokens_are_exact(M, N, K, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+
+    def numbers(rows, cols):
+        full = torch.full((rows + 1, cols + 8), float("nan"), dtype=dtype, device="cuda")
+        full[:rows, :cols] = torch.randint(-2, 3, (rows, cols), generator=gen, device="cuda").to(dtype)
+        return full[:rows, :cols]
+
+    X, W = numbers(M, K), numbers(N, K)
+    bias = torch.randint(-3, 4, (N,), generator=gen, device="cuda").float()
+    product = X.double() @ W.double().t()
+    sfx = "" if dtype == torch.bfloat16 else "_f16"
+    stream = nv.current_stream()
+
+    def canvas(t):
+        full = torch.full((M + 1, N + 8), CANARY, dtype=t, device="cuda")
+        return full, full[:M, :N]
+
+    def check(full, view, want):
+        assert torch.equal(view.double(), want.to(view.dtype).double())
+        view.fill_(CANARY)
+        assert torch.equal(full, torch.full_like(full, CANARY)), "written outside the output"
+
+    full, y = canvas(dtype)
+    for b, epi, want in ((None, nv.EPI_NONE, product), (bias, nv.EPI_BIAS, product + bias)):
+        nv.call("axn_gemm_fwd" + sfx, nv.ptr(X), nv.ptr(W), nv.ptr(b), nv.ptr(y), None, M, N, K, X.stride(0),
+                W.stride(0), y.stride(0), epi, stream)
+        check(full, y, want)
+    full32, y32 = canvas(torch.float32)
+    nv.call("axn_gemm_fwd_f32out", nv.ptr(X), nv.ptr(W), nv.ptr(bias), nv.ptr(y32), None, nv.dtype_code(dtype), M, N,
+            K, X.stride(0), W.stride(0), y32.stride(0), nv.EPI_BIAS, stream)
+    check(full32, y32, product + bias)
+    # GELU: the saved pre-activation is exact, Y within one rounding and the erf's 1.5e-7
+    fz, z = canvas(dtype)
+    nv.call("axn_gemm_fwd" + sfx, nv.ptr(X), nv.ptr(W), nv.ptr(bias), nv.ptr(y), nv.ptr(z), M, N, K, X.stride(0),
+            W.stride(0), y.stride(0), nv.EPI_BIAS_GELU, stream)
+    pre = product + bias
+    want = torch.nn.functional.gelu(pre)
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert bool(((y.double() - want).abs() <= eps * want.abs() + 2e-7 * pre.abs().clamp(min=1)).all())
+    check(fz, z, pre)

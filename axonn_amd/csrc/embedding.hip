@@ -21,6 +21,7 @@
 #include "axn_internal.h"
 
 #include <cstring>
+#include <type_traits>
 
 namespace axn {
 namespace {
@@ -321,20 +322,45 @@ __global__ void __launch_bounds__(64 * SORT_WAVES)
     __syncthreads();   // every lane has read its digit's count before any lane moves one on
     if (active && lane == 63 - __builtin_clzll(same)) cnt[w][d] = off + __builtin_popcountll(same);
     __syncthreads();
-    if (active) {
-      const int dest = off + __builtin_popcountll(same & below);
-      keys_out[dest] = key;
-      vals_out[dest] = val;
-      if (next_hist != nullptr) {
-        const int nx = (key >> next_shift) & ((1 << next_bits) - 1);
-        const int64_t nb = dest / (64 * G * SORT_WAVES);
-        atomicAdd(&next_hist[SCANNED ? (int64_t)nx * nblk + nb : (nb << next_bits) + nx], 1);
-      } else if (key < V) {
-        // last pass: the slots are final, and a row's run starts at the smallest of them
-        // (row_start holds -1 = the largest unsigned value until a slot arrives)
-        atomicMin((unsigned*)&row_start[key], (unsigned)dest);
-      } else {
-        *status = 1;   // an id outside the table
+    // The ids of a text repeat (the most frequent one is a twentieth of all tokens), and an
+    // atomic on one word is one at a time in L2: the lanes that would hit the same word are
+    // joined first, and one of them goes (16384 such ids into 128256 rows: a scatter pass takes
+    // 32 us without, 9 us with it; on ids drawn evenly both take 8).
+    const int dest = off + __builtin_popcountll(same & below);
+    if (next_hist != nullptr) {
+      const int nx = (key >> next_shift) & ((1 << next_bits) - 1);
+      const int nb = dest / (64 * G * SORT_WAVES);
+      // equal next digit, and the same unit: the destinations of `same` are consecutive, so they
+      // lie in at most two units, one of them odd
+      uint64_t joined = same;
+      for (int b = 0; b <= next_bits; ++b) {
+        const bool bit = ((b < next_bits ? nx >> b : nb) & 1) != 0;
+        const uint64_t with = __ballot(active && bit);
+        joined &= bit ? with : ~with;
+      }
+      if (active) {
+        keys_out[dest] = key;
+        vals_out[dest] = val;
+        if ((joined & below) == 0)
+          atomicAdd(&next_hist[SCANNED ? (int64_t)nx * nblk + nb : ((int64_t)nb << next_bits) + nx],
+                    __builtin_popcountll(joined));
+      }
+    } else {
+      // last pass: the slots are final, and a row's run starts at the smallest of them
+      // (row_start holds -1 = the largest unsigned value until a slot arrives).  Lanes of one
+      // digit take their slots in lane order, and equal keys are neighbours among them (the
+      // passes before have sorted the other digits): only the first lane of a run goes.
+      const uint64_t before = same & below;
+      const int prev = before != 0 ? 63 - __builtin_clzll(before) : lane;
+      const int prev_key = __shfl(key, prev, 64);
+      if (active) {
+        keys_out[dest] = key;
+        vals_out[dest] = val;
+        if (key < V) {
+          if (prev == lane || prev_key != key) atomicMin((unsigned*)&row_start[key], (unsigned)dest);
+        } else {
+          *status = 1;   // an id outside the table
+        }
       }
     }
   }
@@ -414,24 +440,29 @@ struct Vec<_Float16> {
   }
 };
 
-// Loads VEC consecutive elements as fp32 (VEC = 4 or 8), 16 bytes per instruction
-// where the type allows.  Gradient rows are read once: non-temporal.
+// VEC consecutive elements of a gradient row (VEC = 2, 4 or 8) as they lie in memory, so that
+// several rows can be on their way before the first is added; 16 bytes per instruction where
+// the type allows.  Gradient rows are read once: non-temporal.
+template <typename T, int VEC>
+struct RowPiece;
 template <int VEC>
-__device__ __forceinline__ void load_row_piece(const float* p, float (&x)[VEC]) {
+struct RowPiece<float, VEC> {
+  static constexpr int W = VEC < 4 ? VEC : 4;
+  typedef float fxv __attribute__((ext_vector_type(W)));
+  fxv v[VEC / W];
+  __device__ __forceinline__ void load(const float* p) {
 #pragma unroll
-  for (int h = 0; h < VEC / 4; ++h) {
-    const f32x4 v = __builtin_nontemporal_load((const f32x4*)p + h);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[4 * h + e] = v[e];
+    for (int h = 0; h < VEC / W; ++h) v[h] = __builtin_nontemporal_load((const fxv*)p + h);
   }
-}
+  __device__ __forceinline__ float get(int e) const { return v[e / W][e % W]; }
+};
 template <int VEC>
-__device__ __forceinline__ void load_row_piece(const uint16_t* p, float (&x)[VEC]) {
+struct RowPiece<uint16_t, VEC> {
   typedef __bf16 bf16xv __attribute__((ext_vector_type(VEC)));
-  const bf16xv v = __builtin_nontemporal_load((const bf16xv*)p);
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) x[e] = (float)v[e];
-}
+  bf16xv v;
+  __device__ __forceinline__ void load(const uint16_t* p) { v = __builtin_nontemporal_load((const bf16xv*)p); }
+  __device__ __forceinline__ float get(int e) const { return (float)v[e]; }
+};
 template <int VEC>
 __device__ __forceinline__ void add_old(const float* p, float (&x)[VEC]) {
   const f32x4 v = *(const f32x4*)p;
@@ -445,23 +476,156 @@ __device__ __forceinline__ void add_old(const uint16_t* p, float (&x)[VEC]) {
   for (int e = 0; e < 8; ++e) x[e] += (float)v[e];
 }
 
+// Adds the gradient rows whose positions lanes i .. i + B - 1 hold in `pos` to acc, in lane
+// order.  All loads come first and under no condition (a lane past the row's end loads the
+// row's last columns): with a condition per row the compiler pairs each load with its addition,
+// and every row waits for the one before.  U pieces of 64 x VEC columns, `col0` this lane's
+// first column.
+template <typename TY, int VEC, int U, int B>
+__device__ __forceinline__ void add_batch(float (&acc)[U][VEC], int i, int pos, const TY* dY, int64_t lddy,
+                                          int64_t col0, int64_t H, bool scaled, float inv) {
+  RowPiece<TY, VEC> g[B][U];
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const TY* row = dY + (int64_t)__builtin_amdgcn_readlane(pos, i + b) * lddy;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t col = col0 + u * 64 * VEC;
+      g[b][u].load(row + (col < H ? col : H - VEC));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);   // (the scheduler, too, would pair them, to save registers)
+#pragma unroll
+  for (int b = 0; b < B; ++b)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < VEC; ++q)
+        acc[u][q] = scaled ? __fmaf_rn(g[b][u].get(q), inv, acc[u][q]) : acc[u][q] + g[b][u].get(q);
+}
+// The same for lanes 0 .. n - 1, B rows on their way at a time.
+template <typename TY, int VEC, int U, int B>
+__device__ __forceinline__ void add_rows(float (&acc)[U][VEC], int n, int pos, const TY* dY, int64_t lddy,
+                                         int64_t col0, int64_t H, bool scaled, float inv, int i = 0) {
+  for (; i + B <= n; i += B) add_batch<TY, VEC, U, B>(acc, i, pos, dY, lddy, col0, H, scaled, inv);
+  if constexpr (B > 1)
+    if (i < n) add_rows<TY, VEC, U, B / 2>(acc, n, pos, dY, lddy, col0, H, scaled, inv, i);
+}
+
+template <typename TW, int VEC, int U>
+__device__ __forceinline__ void store_rows(float (&acc)[U][VEC], TW* dst, int64_t col0, int64_t H, int beta) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (col0 + u * 64 * VEC >= H) break;
+    if (beta != 0) add_old<VEC>(dst + u * 64 * VEC, acc[u]);
+    Vec<TW>::store(dst + u * 64 * VEC, acc[u]);
+  }
+}
+
+// Half a 16-byte vector of the row.
+template <typename TW>
+__device__ __forceinline__ void store_half(const float (&x)[8 / sizeof(TW)], TW* dst, int beta) {
+  constexpr int N = 8 / (int)sizeof(TW);
+  typedef std::conditional_t<sizeof(TW) == 4, float, __bf16> elem;
+  typedef elem half __attribute__((ext_vector_type(N)));
+  half o = beta != 0 ? *(const half*)dst : half{};
+#pragma unroll
+  for (int q = 0; q < N; ++q) o[q] = (elem)(x[q] + (float)o[q]);
+  *(half*)dst = o;
+}
+
+// Rows named by more than EMB_LONG_RUN tokens get waves of their own (below).
+constexpr int EMB_LONG_RUN = 32;
+
+// The slots of `row` among the 64 from slot `first` on: their count, and this lane's position.
+__device__ __forceinline__ int run_in_chunk(const int* __restrict__ keys, const int* __restrict__ vals,
+                                            int64_t first, int64_t T, int row, int lane, int& pos) {
+  const int64_t j = first + lane;
+  const int key = j < T ? keys[j] : -1;
+  pos = j < T ? vals[j] : 0;
+  const uint64_t in = __ballot(key == row);
+  return in == ~0ull ? 64 : __builtin_ctzll(~in);
+}
+
 // One wave per (row, U x 64 x VEC columns): VEC = one 16-byte store of the dW type
 // per lane, U such pieces per lane, 64 x VEC columns apart, so that a wave has U
 // independent loads in flight per gradient row and U KiB of stores behind one
 // look-up of row_start (with one piece per wave the 8192 resident waves of the chip
 // covered 8 MB per memory latency: 4.2 TB/s on a gradient that is mostly zeros).
+//
+// The order of a row's sum is fixed (token order), so a row named by many tokens is a
+// chain of additions, and what it costs is how many gradient rows are on their way at once
+// and how many waves share the row.  A row's slots are read 64 at a time, one per lane, and
+// four (two) gradient rows are in flight.  Rows with more than EMB_LONG_RUN tokens are left to the
+// launch's first `long_blocks` workgroups: one wave per (64 sorted slots, 32 x VEC columns)
+// that looks for such runs among its slots and has 32 (16) gradient rows in flight, so that a
+// long run is spread over all pieces of its row and starts first.  The whole call for 16384
+// tokens x 2048 fp32 whose ids fall off like those of a text, into 128256 rows: 1394 us with one
+// row in flight and every row on the same waves, 239 us so; ids drawn evenly: 230 us both ways.
+// What bounds it now is the store of the 1.05 GB gradient (181 us of one token, 153 us for a
+// plain fill).
 template <typename TY, typename TW, int U>
-__global__ void __launch_bounds__(64 * WAVES_PER_BLOCK)
+__global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
     embedding_bwd_kernel(const int* __restrict__ keys, const int* __restrict__ vals,
                          const int* __restrict__ row_start, const TY* __restrict__ dY, TW* dW,
                          int64_t T, int64_t V, int64_t H, int64_t lddy, int64_t lddw,
-                         int units_per_row, int64_t padding_idx, int scale_by_freq, int beta) {
+                         int units_per_row, int64_t padding_idx, int scale_by_freq, int beta,
+                         int long_blocks, int pieces_per_row) {
   constexpr int VEC = 16 / (int)sizeof(TW);
+  constexpr int LV = VEC / 2;                              // columns of a lane in a long run's wave
+  constexpr int LONG_B = LV * sizeof(TY) > 8 ? 16 : 32;    // its rows in flight: 64 registers
   const int lane = threadIdx.x & 63;
-  const int64_t unit = (int64_t)blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
-  const int64_t row = unit / units_per_row;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if ((int)blockIdx.x < long_blocks) {
+    const int64_t unit = (int64_t)blockIdx.x * WAVES_PER_BLOCK + wave;
+    const int64_t chunk = unit / pieces_per_row * 64;
+    const int64_t col0 = (unit % pieces_per_row * 64 + lane) * LV;
+    const int64_t j = chunk + lane;
+    const int key = j < T ? keys[j] : -1;
+    const bool starts = j < T && key < V && key != padding_idx && (j == 0 || keys[j - 1] != key) &&
+                        j + EMB_LONG_RUN < T && keys[j + EMB_LONG_RUN] == key;
+    for (uint64_t todo = __ballot(starts); todo != 0; todo &= todo - 1) {
+      const int l = __builtin_ctzll(todo);
+      const int row = __builtin_amdgcn_readlane(key, l);
+      const int64_t first = chunk + l;
+      int pos, n;
+      float inv = 1.0f;
+      if (scale_by_freq) {
+        int64_t e = first;
+        do {
+          n = run_in_chunk(keys, vals, e, T, row, lane, pos);
+          e += n;
+        } while (n == 64);
+        inv = 1.0f / (float)(e - first);
+      }
+      float acc[1][LV];
+#pragma unroll
+      for (int q = 0; q < LV; ++q) acc[0][q] = 0.f;
+      n = run_in_chunk(keys, vals, first, T, row, lane, pos);
+      for (int64_t at = first; n > 0; at += 64) {
+        int next_pos = 0;   // looked up while this chunk's rows are added
+        const int next_n = n == 64 ? run_in_chunk(keys, vals, at + 64, T, row, lane, next_pos) : 0;
+        add_rows<TY, LV, 1, LONG_B>(acc, n, pos, dY, lddy, col0, H, scale_by_freq != 0, inv);
+        n = next_n;
+        pos = next_pos;
+      }
+      if (col0 < H) store_half<TW>(acc[0], dW + row * lddw + col0, beta);
+    }
+    return;
+  }
+  // (the wave's number stays a vector here: row_start read through the scalar cache costs 7 %)
+  // (a 64-bit division would be half of what a wave does for a row without tokens: the quotient
+  // of the workgroup's first unit is the scalar unit's, the rest of its units follow)
+  const int64_t unit0 = (int64_t)((int)blockIdx.x - long_blocks) * WAVES_PER_BLOCK;
+  const int64_t row0 = unit0 / units_per_row;
+  int rest = (int)(unit0 - row0 * units_per_row) + (int)(threadIdx.x >> 6);
+  int64_t row = row0;
+  while (rest >= units_per_row) {   // at most WAVES_PER_BLOCK - 1 times
+    rest -= units_per_row;
+    ++row;
+  }
   if (row >= V) return;
-  const int64_t col0 = ((unit % units_per_row) * U * 64 + lane) * VEC;
+  const int64_t col0 = ((int64_t)rest * (U * 64) + lane) * VEC;
   float acc[U][VEC];
 #pragma unroll
   for (int u = 0; u < U; ++u)
@@ -469,37 +633,19 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK)
     for (int q = 0; q < VEC; ++q) acc[u][q] = 0.f;
   const int s = row_start[row];
   if (s >= 0 && row != padding_idx) {
-    float inv = 1.0f;
-    if (scale_by_freq) {
-      int e = s + 1;
-      while (e < T && keys[e] == (int)row) ++e;
-      inv = 1.0f / (float)(e - s);
-    }
-    for (int j = s; j < T; ++j) {
-      if (j != s && keys[j] != (int)row) break;
-      const TY* src = dY + (int64_t)vals[j] * lddy + col0;
-      float g[U][VEC];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (col0 + u * 64 * VEC < H) load_row_piece<VEC>(src + u * 64 * VEC, g[u]);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (col0 + u * 64 * VEC < H) {
-#pragma unroll
-          for (int q = 0; q < VEC; ++q)
-            acc[u][q] = scale_by_freq ? __fmaf_rn(g[u][q], inv, acc[u][q]) : acc[u][q] + g[u][q];
-        }
-    }
+    int pos, n = 1;
+    if (s + 1 >= T || keys[s + 1] != (int)row)   // most rows of a text have one token
+      pos = vals[s];
+    else
+      n = run_in_chunk(keys, vals, s, T, (int)row, lane, pos);
+    if (n > EMB_LONG_RUN) return;   // another wave's
+    const float inv = scale_by_freq ? 1.0f / (float)n : 1.0f;
+    constexpr int B = U * VEC * (int)sizeof(TY) > 64 ? 2 : 4;   // (at most 64 registers of a lane)
+    add_rows<TY, VEC, U, B>(acc, n, pos, dY, lddy, col0, H, scale_by_freq != 0, inv);
   } else if (beta != 0) {
     return;  // nothing to add to this row
   }
-  TW* dst = dW + row * lddw + col0;
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    if (col0 + u * 64 * VEC >= H) break;
-    if (beta != 0) add_old<VEC>(dst + u * 64 * VEC, acc[u]);
-    Vec<TW>::store(dst + u * 64 * VEC, acc[u]);
-  }
+  store_rows<TW, VEC, U>(acc, dW + row * lddw + col0, col0, H, beta);
 }
 
 // ---- max_norm ------------------------------------------------------------------
@@ -700,7 +846,11 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
   const int64_t pieces = (H / vec + 63) / 64;
   const int U = pieces >= 4 ? 4 : pieces >= 2 ? 2 : 1;
   const int upr = (int)((pieces + U - 1) / U);
-  const int64_t blocks = (V * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+  // waves for rows named by many tokens: one per 64 sorted slots and piece
+  const int64_t long_pieces = (H / (vec / 2) + 63) / 64;
+  const int64_t long_blocks =
+      T > EMB_LONG_RUN ? ((T + 63) / 64 * long_pieces + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK : 0;
+  const int64_t blocks = (V * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK + long_blocks;
   if (blocks >= (1LL << 31)) {
     set_error("embedding_bwd: too many rows x columns (%lld blocks)", (long long)blocks);
     return AXN_ELIMIT;
@@ -712,7 +862,7 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
 #define AXN_EMB_BWD_U(TY, TW, UU)                                                               \
   hipLaunchKernelGGL((embedding_bwd_kernel<TY, TW, UU>), grid, block, EMB_BWD_LDS, stream, keys, vals,    \
                      w.row_start, (const TY*)dY, (TW*)dW, T, V, H, lddy, lddw, upr, padding_idx, \
-                     scale_by_freq, beta)
+                     scale_by_freq, beta, (int)long_blocks, (int)long_pieces)
 #define AXN_EMB_BWD(TY, TW)                 \
   do {                                      \
     if (U == 4)                             \

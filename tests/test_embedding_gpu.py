@@ -97,6 +97,40 @@ def test_backward_equals_the_sequential_sum_bit_for_bit(dy_dtype, dw_dtype, T, V
     assert np.array_equal(host(dW), want)
 
 
+@pytest.mark.parametrize("dy_dtype,dw_dtype", [(torch.float32, torch.float32),
+                                               (torch.bfloat16, torch.float32),
+                                               (torch.bfloat16, torch.bfloat16),
+                                               (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("H", [8, 264, 1040, 2056])
+def test_backward_of_rows_named_by_many_tokens(dy_dtype, dw_dtype, H):
+    """Runs around the length from which a row gets waves of its own (32), around the 64 slots
+    looked at in one go and far beyond, at every phase to those 64, one of them the padding row:
+    bit for bit the sequential loop, also accumulating and scaled by frequency."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(H)
+    runs = [1, 31, 32, 33, 34, 7, 63, 64, 65, 2, 96, 127, 128, 129, 40, 300, 33, 1, 33, 500]
+    V = len(runs) + 5
+    ids = torch.repeat_interleave(torch.arange(len(runs), device="cuda"), torch.tensor(runs, device="cuda"))
+    ids = ids[torch.randperm(ids.numel(), device="cuda", generator=g)]
+    dy = (torch.randn(ids.numel(), H, device="cuda", generator=g) * 0.01).to(dy_dtype)
+    old = torch.randn(V, H, device="cuda", generator=g).to(dw_dtype)
+    for padding, accumulate in ((None, False), (15, False), (7, True)):
+        out = old.clone()
+        ops.embedding_bwd(ids, dy, V, padding_idx=padding, out=out, accumulate=accumulate)
+        want = oe.embedding_backward(ids.cpu().numpy(), host(dy), V, padding_idx=padding)
+        if accumulate:
+            want = np.where(want != 0, want + host(old), host(old)).astype(np.float32)
+        if dw_dtype == torch.bfloat16:
+            want = bf16_round(want)
+        assert np.array_equal(host(out), want)
+    dW = ops.embedding_bwd(ids, dy, V, scale_grad_by_freq=True, out_dtype=dw_dtype)
+    want = oe.embedding_backward(ids.cpu().numpy(), host(dy), V, scale_grad_by_freq=True)
+    # the oracle imitates the fused multiply-add through float64: 1 ulp of the sum's terms
+    tol = 2.0 ** -8 if dw_dtype == torch.bfloat16 else 1e-6
+    assert np.allclose(host(dW), want, rtol=tol, atol=1e-9)
+
+
 @pytest.mark.parametrize("T,V", [(700, 3), (513, 1023), (5000, 1024), (40000, 70000), (3000, (1 << 21) + 5),
                                  (100000, 200), ((1 << 18) + 77, 5000), (300000, 1 << 20)])
 def test_backward_over_every_shape_of_the_sort(T, V):

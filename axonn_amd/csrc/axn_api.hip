@@ -293,10 +293,8 @@ size_t axn_gemm_workspace_bytes(int op, int64_t M, int64_t N, int64_t K) {
       N > 0x7fffffff || K > 0x7fffffff)
     return 0;
   GemmArgs g = {};
-  // dense operands: the leading dimensions are the row lengths
-  fill_gemm_args(g, op, nullptr, nullptr, nullptr, M, N, K, op == AXN_GEMM_FWD ? K : N, K,
-                 op == AXN_GEMM_FWD ? N : K);
-  const int s = gemm_splits(kLayoutOfOp[op], g);
+  fill_gemm_args(g, op, nullptr, nullptr, nullptr, M, N, K, 0, 0, 0);
+  const int s = gemm_splits(kLayoutOfOp[op], g.M, g.N, g.Kc).parts;
   return s > 1 ? (size_t)s * (size_t)g.M * (size_t)g.N * sizeof(float) : 0;
 }
 
@@ -321,15 +319,15 @@ static int gemm_ws(const char* name, int op, const void* a, const void* b, void*
   g.bias = bias;
   g.Z = (uint16_t*)zsave;
   const GemmLayout layout = kLayoutOfOp[op];
-  bool wide_tiles = false;
-  const int splits =
-      (workspace != nullptr && epilogue == AXN_EPI_NONE) ? gemm_splits(layout, g, &wide_tiles) : 1;
-  if (splits > 1) {
-    const size_t need = (size_t)splits * (size_t)g.M * (size_t)g.N * sizeof(float);
+  const bool near = lda < kEdgeMaxLd / 2 && ldb < kEdgeMaxLd / 2;   // strides the parts' kernels take
+  const SplitPlan plan =
+      workspace != nullptr && near ? gemm_splits(layout, g.M, g.N, g.Kc) : SplitPlan{1, EDGE_128x128};
+  if (plan.parts > 1) {
+    const size_t need = (size_t)plan.parts * (size_t)g.M * (size_t)g.N * sizeof(float);
     REQUIRE(workspace_bytes >= need, AXN_EINVAL,
             "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
     REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
-    return launch_gemm_splitk(layout, g, half, out_dtype, splits, wide_tiles, (float*)workspace,
+    return launch_gemm_splitk(layout, g, epilogue, half, out_dtype == AXN_F32, plan, (float*)workspace,
                               (hipStream_t)stream);
   }
   return half ? launch_gemm_f16(layout, g, epilogue, out_dtype == AXN_F32, (hipStream_t)stream)

@@ -120,26 +120,27 @@ int launch_gemm_bf16(GemmLayout layout, const GemmArgs& args, int epilogue,
 // The same kernels on IEEE half operands (v_mfma_f32_16x16x32_f16, half outputs).
 int launch_gemm_f16(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32,
                     hipStream_t stream);
-// Split-contraction variant for problems with few output tiles: the number of splits
-// chosen for an [M x N] output over a contraction of Kc (1 = do not split; *wide_tiles:
-// the parts run on 256 x 128 tiles instead of 128 x 128), and the
-// launch: partial products in fp32 to `ws` (splits * M * N floats), then one pass that
-// adds them in split order, adds the old output if args.beta, and stores args.C in
-// out_dtype.  No epilogue.
-int gemm_splits(GemmLayout layout, const GemmArgs& args, bool* wide_tiles = nullptr);
 // dX = dY W and dW (+)= dY^T X of one layer, args as for GEMM_NN and GEMM_TN.  Results are
 // those of the two separate launches bit for bit; when the two problems' tile counts leave
 // CUs idle one after the other but not together, they run as ONE launch (see gemm_bf16.hip).
 int launch_gemm_backward(const GemmArgs& dgrad, const GemmArgs& wgrad, bool half, bool dw_f32,
                          hipStream_t stream);
-int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, bool half, int out_dtype,
-                       int splits, bool wide_tiles, float* ws, hipStream_t stream);
-
 // GEMMs of shapes that are not made of whole tiles (gemm_edge.h), on the tile the caller
 // picks: any M, N, contraction and operand size, row strides below kEdgeMaxLd elements (half
 // of that on the tiles of 256 rows).
 enum EdgeTile { EDGE_256x256 = 0, EDGE_256x128 = 1, EDGE_128x128 = 2 };
 constexpr int64_t kEdgeMaxLd = 1LL << 23;
+// Split contraction for problems with few output tiles: into how many parts and on which
+// tile (parts = 1: do not split), and the launch: partial products in fp32 to `ws`
+// (parts * M * N floats), then one pass that adds them in part order, adds the old output if
+// args.beta, applies the epilogue and stores args.C.
+struct SplitPlan {
+  int parts;
+  EdgeTile tile;
+};
+SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc);
+int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, int epilogue, bool half, bool out_f32,
+                       const SplitPlan& plan, float* ws, hipStream_t stream);
 int launch_gemm_edge_bf16(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32,
                           EdgeTile tile, hipStream_t stream);
 int launch_gemm_edge_f16(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32,
@@ -150,9 +151,11 @@ int launch_gemm_edge_backward_bf16(const GemmArgs& wgrad, const GemmArgs& dgrad,
 int launch_gemm_edge_backward_f16(const GemmArgs& wgrad, const GemmArgs& dgrad, bool dw_f32,
                                   hipStream_t stream);
 
-// Forward products of at most kStreamTokens rows (gemm_stream.hip): a stream over the weights;
-// row strides below kStreamMaxLd elements.
-constexpr int kStreamTokens = 32;
+// Forward products of a few rows (gemm_stream.hip): a stream over the weights; row strides
+// below kStreamMaxLd elements.  Up to 32 rows it is ahead of the tiles with a split contraction
+// everywhere, up to 64 for contractions that are not long (64 rows, us, stream / tiles:
+// 4096 x 4096 13.5 / 15.8, 14336 x 4096 25.9 / 31.6, 4096 x 14336 45 / 32.5).
+inline bool stream_takes(int64_t M, int64_t Kc) { return M <= 32 || (M <= 64 && Kc <= 6144); }
 constexpr int64_t kStreamMaxLd = 1LL << 24;
 int launch_gemm_stream(const GemmArgs& args, int epilogue, bool out_f32, bool half, hipStream_t stream);
 

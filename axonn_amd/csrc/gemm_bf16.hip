@@ -125,31 +125,42 @@ int launch_rest(const GemmArgs& in, hipStream_t stream) {
 }
 
 // ---- shapes that are not made of whole tiles (gemm_edge.h) -----------------------------
-// Estimated microseconds of an M x N output over `stages` 64-deep stages on one tile size,
-// from the whole-tile kernels' measured stage times: 1.29 per stage of a round of 256 x 256
-// tiles, 0.93 of 256 x 128, 1.33 of two 128 x 128 tiles per CU and 0.77 of one, and about
-// 6 per round for the first tiles' way into LDS and the write-back.
-double edge_microseconds(EdgeTile tile, long long M, long long N, long long stages) {
-  auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  const double s = (double)stages;
-  const auto small = [&](long long t) {
-    const long long full = t / 512, rest = t % 512;
-    return (double)full * (1.33 * s + 6) + (rest > 256 ? 1.33 * s + 6 : rest > 0 ? 0.77 * s + 6 : 0.0);
-  };
-  if (tile == EDGE_128x128) return small(tiles(128, 128));
-  if (tile == EDGE_256x128) return (double)((tiles(256, 128) + 255) / 256) * (0.93 * s + 6);
-  const long long t = tiles(256, 256), full = t / 256, rest = t % 256;
-  double us = (double)full * (1.29 * s + 6);
-  if (rest > 0) us += full > 0 && rest <= 64 ? 0.77 * s + 9 : full > 0 && rest <= 128 ? 0.93 * s + 9 : 1.29 * s + 6;
-  return us;
+// Estimated microseconds of one launch of `w` workgroups of a tile size that each walk `stages`
+// 64-deep stages of operands of `mb` megabytes (short runs on MI355X, operands coming from HBM):
+//   main loop   0.69 per stage of 128 x 128 tiles at one workgroup per CU, 1.2 + 0.936 per
+//               stage at two; 2.5 + 0.737 of 256 x 128 tiles; 5.1 + 1.084 of 256 x 256 tiles;
+//               times the rounds of workgroups;
+//   operands    never faster than 1.7 + their bytes at 5.7 TB/s, which they reach only with a
+//               workgroup on every CU (9 % of it with none, linear between).
+// The constants were fitted to 3479 launches: every tile size and split of 220 forward and
+// input-gradient problems of 33 to 3000 tokens and 768 to 14336 features, ragged and whole.
+double launch_microseconds(EdgeTile tile, long long w, double stages, double mb) {
+  const double loop = tile == EDGE_256x256   ? (5.1 + 1.084 * stages) * (double)((w + 255) / 256)
+                      : tile == EDGE_256x128 ? (2.5 + 0.737 * stages) * (double)((w + 255) / 256)
+                      : w <= 256             ? 0.69 * stages
+                                             : (1.2 + 0.936 * stages) * (double)((w + 511) / 512);
+  const double occupied = w >= 256 ? 1.0 : (double)w / 256;
+  const double stream = 1.74 + mb / (5.72 * (0.086 + 0.914 * occupied));
+  return loop > stream ? loop : stream;
+}
+
+// The same for an unsplit M x N output as launch_edge_kind runs it: a last round of at most
+// half of the CUs goes to smaller tiles.
+double edge_microseconds(EdgeTile tile, long long M, long long N, long long Kc) {
+  const int bm = tile == EDGE_128x128 ? 128 : 256, bn = tile == EDGE_256x256 ? 256 : 128;
+  const long long w = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), full = w / 256, rest = w % 256;
+  const double stages = (double)((Kc + 63) / 64), mb = ((double)M + (double)N) * (double)Kc * 2e-6;
+  if (tile == EDGE_256x256 && full > 0 && rest > 0 && rest <= 128)
+    return launch_microseconds(tile, full * 256, stages, mb) +
+           launch_microseconds(rest <= 64 ? EDGE_128x128 : EDGE_256x128, 256, stages, 0.0) + 3.0;
+  return launch_microseconds(tile, w, stages, mb);
 }
 
 EdgeTile edge_tile(long long M, long long N, long long Kc, double* us = nullptr) {
-  const long long stages = (Kc + 63) / 64;
   EdgeTile best = EDGE_256x256;
-  double least = edge_microseconds(best, M, N, stages);
+  double least = edge_microseconds(best, M, N, Kc);
   for (EdgeTile t : {EDGE_256x128, EDGE_128x128}) {
-    const double e = edge_microseconds(t, M, N, stages);
+    const double e = edge_microseconds(t, M, N, Kc);
     if (e < least) {
       least = e;
       best = t;
@@ -269,57 +280,60 @@ int launch_shape(const GemmArgs& g, hipStream_t stream) {
 
 namespace {
 
-// Sum of the fp32 partial products of a split contraction, in split order, plus the
-// old output if beta; one 16-byte store (two for fp32) of 8 columns per lane.
-template <typename LP>
+// Sum of the fp32 partial products of a split contraction, in split order, then the output's
+// epilogue; 8 columns per lane.  Bound by its reads (512 x 8192, 2 parts: 7.3 us for 42 MB).
+template <int EPI, bool OUT_F32, bool HALF>
 __global__ void __launch_bounds__(256)
-    splitk_reduce_kernel(const float* __restrict__ ws, LP* out, int64_t M, int64_t N, int64_t ld,
-                         int splits, int beta) {
+    splitk_reduce_kernel(const float* __restrict__ ws, const GemmArgs g) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t per_row = N / 8;
-  if (idx >= M * per_row) return;
-  const int64_t row = idx / per_row, col = (idx - row * per_row) * 8;
-  const float* p = ws + row * N + col;
+  const int64_t per_row = g.N / 8;
+  if (idx >= (int64_t)g.M * per_row) return;
+  const int64_t row = idx / per_row, col = (idx - row * per_row) * 8, part = (int64_t)g.M * g.N;
+  const float* p = ws + row * g.N + col;
   f32x4 a0 = __builtin_nontemporal_load((const f32x4*)p);
   f32x4 a1 = __builtin_nontemporal_load((const f32x4*)(p + 4));
-  for (int s = 1; s < splits; ++s) {
-    p += M * N;
+  for (int s = 1; s < g.splits; ++s) {
+    p += part;
     a0 += __builtin_nontemporal_load((const f32x4*)p);
     a1 += __builtin_nontemporal_load((const f32x4*)(p + 4));
   }
-  LP* o = out + row * ld + col;
-  if constexpr (sizeof(LP) == 4) {
-    if (beta) {
-      a0 += *(const f32x4*)o;
-      a1 += *(const f32x4*)(o + 4);
-    }
-    *(f32x4*)o = a0;
-    *(f32x4*)(o + 4) = a1;
+  float v[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+  store_row8<EPI, OUT_F32, HALF>(v, g, (int)row, (int)col);
+}
+
+template <bool HALF>
+int launch_reduce(const float* ws, const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
+  const int64_t lanes = (int64_t)g.M * (g.N / 8);
+  const dim3 grid((unsigned)((lanes + 255) / 256)), block(256);
+#define REDUCE(EPI, F32) hipLaunchKernelGGL((splitk_reduce_kernel<EPI, F32, HALF>), grid, block, 0, stream, ws, g)
+  if (out_f32) {
+    if (epilogue == AXN_EPI_BIAS) REDUCE(AXN_EPI_BIAS, true);
+    else if (epilogue == AXN_EPI_BIAS_GELU) REDUCE(AXN_EPI_BIAS_GELU, true);
+    else REDUCE(AXN_EPI_NONE, true);
   } else {
-    typedef LP lpx8 __attribute__((ext_vector_type(8)));
-    float v[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-    if (beta) {
-      const lpx8 old = *(const lpx8*)o;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] += (float)old[e];
+    switch (epilogue) {
+      case AXN_EPI_NONE: REDUCE(AXN_EPI_NONE, false); break;
+      case AXN_EPI_BIAS: REDUCE(AXN_EPI_BIAS, false); break;
+      case AXN_EPI_BIAS_GELU: REDUCE(AXN_EPI_BIAS_GELU, false); break;
+      default: REDUCE(AXN_EPI_GELU, false);
     }
-    lpx8 y;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = (LP)v[e];
-    *(lpx8*)o = y;
   }
+#undef REDUCE
+  AXN_HIP_TRY(hipGetLastError());
+  return AXN_OK;
 }
 
 template <bool AK, bool BKM, bool HALF>
-int launch_split(const GemmArgs& g, bool wide_tiles, hipStream_t stream) {
-  if (wide_tiles) return launch_rest<AK, BKM, AXN_EPI_NONE, true, HALF>(g, stream);
+int launch_split(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
+  if (tile == EDGE_256x256) return launch_solo<256, AK, BKM, AXN_EPI_NONE, true, HALF>(g, stream);
+  if (tile == EDGE_256x128) return launch_rest<AK, BKM, AXN_EPI_NONE, true, HALF>(g, stream);
   return launch_solo<128, AK, BKM, AXN_EPI_NONE, true, HALF>(g, stream);
 }
 
 template <bool HALF>
 int launch_layout(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32,
                   hipStream_t stream) {
-  if (layout == GEMM_NT && g.M <= kStreamTokens && g.lda < kStreamMaxLd && g.ldb < kStreamMaxLd &&
+  if (layout == GEMM_NT && stream_takes(g.M, g.Kc) && g.lda < kStreamMaxLd && g.ldb < kStreamMaxLd &&
       (!out_f32 || epilogue == AXN_EPI_BIAS || epilogue == AXN_EPI_BIAS_GELU))
     return launch_gemm_stream(g, epilogue, out_f32, HALF, stream);
   switch (layout) {
@@ -501,7 +515,7 @@ int launch_backward(const GemmArgs& gd_in, const GemmArgs& gw_in, bool dw_f32, h
       double ud = 0, uw = 0;
       edge_tile(gd.M, gd.N, gd.Kc, &ud);
       edge_tile(gw.M, gw.N, gw.Kc, &uw);
-      return 1.29 * stages_together(tw, sw, td, sd) + 9 < 0.95 * (ud + uw);
+      return 1.084 * stages_together(tw, sw, td, sd) + 15 < 0.95 * (ud + uw);
     });
     if (together) {
       place_together(gd, gw, td, tw, sd, sw);
@@ -532,104 +546,84 @@ int launch_gemm_f16(GemmLayout layout, const GemmArgs& g, int epilogue, bool out
   return launch_layout<true>(layout, g, epilogue, out_f32, stream);
 }
 
-// Few output tiles leave most CUs without work: the contraction is cut into 2, 4 or 8 parts, each
-// at least 512 deep, on 128 x 128 tiles (up to two workgroups per CU) or 256 x 128 tiles (one).
-// Whether, into how many parts and on which tile to split the contraction of a problem with
-// few output tiles: the choice with the smallest estimated time.  The estimate (microseconds
-// on MI355X, operands coming from HBM) of a launch of w workgroups that each walk `stages`
-// 64-deep stages:
-//   main loop   stages x 0.77 (128 x 128 tiles, at most one workgroup per CU), x 1.33 (two
-//               per CU), x 0.93 (256 x 128 tiles: twice the output per stage), times the
-//               rounds of workgroups the launch takes;
-//   operands    never faster than their bytes at 6 TB/s, and at 47 % of that plus the rest in
-//               proportion to the CUs that have a workgroup;
-//   parts       2.1 + parts x 2.5 x (millions of output elements)^0.74 for writing the fp32
-//               partial products and for the pass that adds them.
-// The eight constants were fitted to the choices' measured times over 165 forward and
-// input-gradient problems of 128 to 1024 tokens and 2560 to 14336 features (every choice
-// timed on cold operands): the rule's pick is within 0.6 % of the fastest choice on average
-// and 13 % at worst; the rule it replaced (as many parts as fill the CUs, 256 x 128 tiles
-// first) was 4.4 % off on average and 44 % at worst.
-int gemm_splits(GemmLayout layout, const GemmArgs& g, bool* wide_tiles) {
-  if (wide_tiles != nullptr) *wide_tiles = false;
-  if (g.M % 128 || g.N % 128 || g.Kc % 64) return 1;
-  const bool ak = layout != GEMM_TN, bkm = layout == GEMM_NT;
-  const int64_t a_span = (int64_t)(ak ? g.M : g.Kc) * g.lda * 2;
-  const int64_t b_span = (int64_t)(bkm ? g.N : g.Kc) * g.ldb * 2;
-  if (a_span >= (1LL << 31) || b_span >= (1LL << 31)) return 1;
-  const long long tiles = (long long)(g.M / 128) * (g.N / 128);
-  const long long wide = g.M % 256 == 0 ? (long long)(g.M / 256) * (g.N / 128) : -1;
-  // beyond 128 tiles of either kind an unsplit launch already has a workgroup on half of the CUs
-  if (!(tiles <= 128 || (wide > 0 && wide <= 128))) return 1;
-  const double out_m = (double)g.M * g.N * 1e-6;
-  const double operand_mb = ((double)g.M + g.N) * g.Kc * 2e-6;
-  const double part_cost = 2.529 * std::pow(out_m, 0.736);
-  auto estimate = [&](int parts, bool wide_kind) {
-    const double stages = (double)g.Kc / 64 / parts;
-    const long long w = (wide_kind ? wide : tiles) * parts;
-    const double loop = wide_kind ? stages * 0.928 * (double)((w + 255) / 256)
-                                  : stages * (w <= 256 ? 0.771 : 1.332) * (double)((w + 511) / 512);
-    const double occupied = w >= 256 ? 1.0 : (double)w / 256;
-    const double stream = operand_mb / (5.998 * (0.465 + 0.535 * occupied));
-    return (loop > stream ? loop : stream) + (parts > 1 ? 2.143 + parts * part_cost : 0.0);
-  };
-  double best = estimate(1, false);
-  int best_parts = 1;
-  bool best_wide = false;
-  for (int parts = 2; parts <= 8; parts *= 2) {
-    if (g.Kc % (64 * parts) != 0 || g.Kc / parts < 512) continue;
-    for (int kind = 0; kind < 2; ++kind) {
-      if (kind == 0 ? tiles * parts > 512 : (wide <= 0 || wide * parts > 256)) continue;
-      const double t = estimate(parts, kind == 1);
+// Few output tiles leave most CUs without work: the contraction is cut into parts of at
+// least 512, on the tile and into the number of parts with the smallest estimated time, each part
+// a workgroup per tile.  On top of the launch (launch_microseconds) a split costs
+// 2.96 + parts x 2.02 x (millions of output elements)^0.763 microseconds for writing the fp32
+// partial products and for the pass that adds them.  Over the 220 problems the estimate was
+// fitted to, its pick takes 1.3 % more than the fastest choice on average and 22 % at worst;
+// the rule before (parts of whole shapes only, 2, 4 or 8 of them, on the two smaller tiles) left
+// ragged ones unsplit: 60 x 3520 x 6848 78 -> 20 us, 479 x 832 x 13824 146 -> 31 us, 1111 x 2752 x
+// 6336 70 -> 56 us.
+// It looks at sizes only, not at strides: a caller asks for the workspace by size.
+SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
+  SplitPlan plan = {1, EDGE_128x128};
+  if (layout == GEMM_NT && stream_takes(M, Kc)) return plan;
+  if (N % 8 != 0) return plan;
+  const bool whole = M % 128 == 0 && N % 128 == 0 && Kc % 64 == 0;
+  auto count = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  const long long tiles[3] = {count(256, 256), count(256, 128), count(128, 128)};
+  // beyond 128 large tiles an unsplit launch of them already has half of the CUs; a short
+  // contraction over a ragged shape is left alone
+  if (tiles[EDGE_256x256] > 128 || Kc < (whole ? 1024 : 1536)) return plan;
+  const double mb = ((double)M + (double)N) * (double)Kc * 2e-6;
+  const double part_cost = 2.02 * std::pow((double)M * (double)N * 1e-6, 0.763);
+  const long long stages = (Kc + 63) / 64;
+  double best = 1e30;
+  for (EdgeTile tile : {EDGE_128x128, EDGE_256x128, EDGE_256x256})
+    best = std::fmin(best, launch_microseconds(tile, tiles[tile], (double)stages, mb));
+  for (int parts = 2; parts <= 16 && Kc / parts >= 512; ++parts)
+    for (EdgeTile tile : {EDGE_128x128, EDGE_256x128, EDGE_256x256}) {
+      if (tiles[tile] * parts > (tile == EDGE_128x128 ? 512 : 256)) continue;
+      const double t = launch_microseconds(tile, tiles[tile] * parts, (double)((stages + parts - 1) / parts), mb) +
+                       2.96 + parts * part_cost;
       if (t < best) {
         best = t;
-        best_parts = parts;
-        best_wide = kind == 1;
+        plan = {parts, tile};
       }
     }
-  }
-  if (wide_tiles != nullptr) *wide_tiles = best_wide;
-  return best_parts;
+  return plan;
 }
 
-int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, bool half, int out_dtype,
-                       int splits, bool wide_tiles, float* ws, hipStream_t stream) {
+int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool half, bool out_f32,
+                       const SplitPlan& plan, float* ws, hipStream_t stream) {
   GemmArgs g = in;
   g.C = ws;
   g.ldc = g.N;
   g.beta = 0;
   g.bias = nullptr;
   g.Z = nullptr;
-  g.splits = splits;
-  g.k_split = g.Kc / splits;
+  g.splits = plan.parts;
+  g.k_split = g.Kc / plan.parts;
+  const bool ak = layout != GEMM_TN, bkm = layout == GEMM_NT;
+  const int bm = plan.tile == EDGE_128x128 ? 128 : 256, bn = plan.tile == EDGE_256x256 ? 256 : 128;
+  const bool whole = g.M % bm == 0 && g.N % bn == 0 && g.Kc % (64 * plan.parts) == 0 &&
+                     (int64_t)(ak ? g.M : g.Kc) * g.lda * 2 < (1LL << 31) &&
+                     (int64_t)(bkm ? g.N : g.Kc) * g.ldb * 2 < (1LL << 31);
   int rc;
-  switch (layout) {
-    case GEMM_NT:
-      rc = half ? launch_split<true, true, true>(g, wide_tiles, stream)
-                : launch_split<true, true, false>(g, wide_tiles, stream);
-      break;
-    case GEMM_NN:
-      rc = half ? launch_split<true, false, true>(g, wide_tiles, stream)
-                : launch_split<true, false, false>(g, wide_tiles, stream);
-      break;
-    default:
-      rc = half ? launch_split<false, false, true>(g, wide_tiles, stream)
-                : launch_split<false, false, false>(g, wide_tiles, stream);
+  if (!whole) {
+    rc = half ? launch_gemm_edge_f16(layout, g, AXN_EPI_NONE, true, plan.tile, stream)
+              : launch_gemm_edge_bf16(layout, g, AXN_EPI_NONE, true, plan.tile, stream);
+  } else {
+    switch (layout) {
+      case GEMM_NT:
+        rc = half ? launch_split<true, true, true>(g, plan.tile, stream)
+                  : launch_split<true, true, false>(g, plan.tile, stream);
+        break;
+      case GEMM_NN:
+        rc = half ? launch_split<true, false, true>(g, plan.tile, stream)
+                  : launch_split<true, false, false>(g, plan.tile, stream);
+        break;
+      default:
+        rc = half ? launch_split<false, false, true>(g, plan.tile, stream)
+                  : launch_split<false, false, false>(g, plan.tile, stream);
+    }
   }
   if (rc) return rc;
-  const int64_t lanes = (int64_t)in.M * (in.N / 8);
-  const dim3 grid((unsigned)((lanes + 255) / 256)), block(256);
-  if (out_dtype == AXN_F32)
-    hipLaunchKernelGGL(splitk_reduce_kernel<float>, grid, block, 0, stream, ws, (float*)in.C,
-                       (int64_t)in.M, (int64_t)in.N, in.ldc, splits, in.beta);
-  else if (out_dtype == AXN_F16)
-    hipLaunchKernelGGL(splitk_reduce_kernel<_Float16>, grid, block, 0, stream, ws, (_Float16*)in.C,
-                       (int64_t)in.M, (int64_t)in.N, in.ldc, splits, in.beta);
-  else
-    hipLaunchKernelGGL(splitk_reduce_kernel<__bf16>, grid, block, 0, stream, ws, (__bf16*)in.C,
-                       (int64_t)in.M, (int64_t)in.N, in.ldc, splits, in.beta);
-  AXN_HIP_TRY(hipGetLastError());
-  return AXN_OK;
+  GemmArgs out = in;
+  out.splits = plan.parts;
+  return half ? launch_reduce<true>(ws, out, epilogue, out_f32, stream)
+              : launch_reduce<false>(ws, out, epilogue, out_f32, stream);
 }
 
 }  // namespace axn

@@ -100,6 +100,8 @@ int launch_edge_layout(GemmLayout layout, const GemmArgs& g, int epilogue, bool 
   switch (layout) {
     case GEMM_NT:
       if (out_f32) {
+        if (epilogue == AXN_EPI_NONE && g.splits > 1)   // partial products
+          return launch_edge_kind<true, true, AXN_EPI_NONE, true, HALF>(g, tile, stream);
         if (epilogue == AXN_EPI_BIAS) return launch_edge_kind<true, true, AXN_EPI_BIAS, true, HALF>(g, tile, stream);
         if (epilogue == AXN_EPI_BIAS_GELU)
           return launch_edge_kind<true, true, AXN_EPI_BIAS_GELU, true, HALF>(g, tile, stream);
@@ -117,7 +119,8 @@ int launch_edge_layout(GemmLayout layout, const GemmArgs& g, int epilogue, bool 
       }
       break;
     case GEMM_NN:
-      if (out_f32 || epilogue != AXN_EPI_NONE) break;
+      if (epilogue != AXN_EPI_NONE || (out_f32 && g.splits <= 1)) break;
+      if (out_f32) return launch_edge_kind<true, false, AXN_EPI_NONE, true, HALF>(g, tile, stream);
       return launch_edge_kind<true, false, AXN_EPI_NONE, false, HALF>(g, tile, stream);
     case GEMM_TN:
       if (epilogue != AXN_EPI_NONE) break;

@@ -196,7 +196,8 @@ int launch_stream_rows(const GemmArgs& g, int epilogue, bool out_f32, hipStream_
 template <bool HALF>
 int launch_stream_tokens(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
   if (g.M <= 16) return launch_stream_rows<1, 4, 3, HALF>(g, epilogue, out_f32, stream);
-  return launch_stream_rows<2, 4, 2, HALF>(g, epilogue, out_f32, stream);
+  if (g.M <= 32) return launch_stream_rows<2, 4, 2, HALF>(g, epilogue, out_f32, stream);
+  return launch_stream_rows<4, 2, 2, HALF>(g, epilogue, out_f32, stream);
 }
 
 }  // namespace

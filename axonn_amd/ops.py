@@ -119,8 +119,7 @@ def gemm_fwd(x, w, bias=None, activation=None, save_z=False, out_f32=False):
                     nv.dtype_code(x.dtype), M, N, K, ldx, ldw, N, epi, nv.current_stream())
             return y, z
         y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-        # (the contraction is only divided for a plain product: an epilogue runs unsplit)
-        ws, ws_bytes = _split_workspace(GEMM_FWD, M, N, K, x.device) if epi == nv.EPI_NONE else (None, 0)
+        ws, ws_bytes = _split_workspace(GEMM_FWD, M, N, K, x.device)
         if ws is not None:
             nv.call("axn_gemm_fwd_ws", nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(y), nv.ptr(z),
                     nv.dtype_code(x.dtype), M, N, K, ldx, ldw, N, epi, nv.ptr(ws), ws_bytes,

@@ -102,3 +102,48 @@ def test_edge_epilogues_keep_the_pre_activation(M, N, K):
         want = torch.nn.functional.gelu(pre)
         assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2e-7 * pre.abs().clamp(min=1)).all())
         check(fz, z, pre)
+
+
+@pytest.mark.parametrize("op,M,N,K", [
+    (0, 65, 136, 2056), (0, 129, 392, 4104), (0, 300, 1000, 1608),      # 128 x 128 tiles
+    (0, 520, 2560, 8200), (1, 300, 8200, 2568), (2, 4104, 136, 264),    # 256 wide ones
+    (0, 128, 384, 12224),    # whole tiles whose 191 stages no number of parts divides
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_contraction_of_any_shape_with_its_epilogue(op, M, N, K, dtype):
+    """The contraction cut into parts of unequal length; the pass that adds them applies bias,
+    GELU (pre-activation kept) and beta.  Whole-number operands: every partial sum is exact."""
+    lib, code = nv.load(), nv.dtype_code(dtype)
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    nbytes = lib.axn_gemm_workspace_bytes(op, M, N, K)
+    assert nbytes > 0, "this shape is meant to be split"
+    ws = torch.full((nbytes // 4 + 8,), float("nan"), device="cuda")
+    stream = nv.current_stream()
+    shapes = (((M, K), (N, K), (M, N)), ((M, N), (N, K), (M, K)), ((M, N), (M, K), (N, K)))[op]
+    a, b = (numbers(r, c, dtype, gen, 16) for r, c in shapes[:2])
+    full, c = canvas(*shapes[2], torch.float32 if op == 2 else dtype)
+    tail = (nv.ptr(ws), nbytes, stream)
+    if op == 0:
+        bias = torch.randint(-3, 4, (N,), generator=gen, device="cuda").float()
+        pre = a.double() @ b.double().t()
+        for bb, epi, want in ((None, nv.EPI_NONE, pre), (bias, nv.EPI_BIAS, pre + bias)):
+            nv.call("axn_gemm_fwd_ws", nv.ptr(a), nv.ptr(b), nv.ptr(bb), nv.ptr(c), None, code, M, N, K, a.stride(0),
+                    b.stride(0), c.stride(0), epi, *tail)
+            check(full, c, want)
+        fz, z = canvas(M, N, dtype)
+        nv.call("axn_gemm_fwd_ws", nv.ptr(a), nv.ptr(b), nv.ptr(bias), nv.ptr(c), nv.ptr(z), code, M, N, K,
+                a.stride(0), b.stride(0), c.stride(0), nv.EPI_BIAS_GELU, *tail)
+        want = torch.nn.functional.gelu(pre + bias)   # within one rounding and the erf's 1.5e-7
+        eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        assert bool(((c.double() - want).abs() <= eps * want.abs() + 2e-7 * pre.abs().clamp(min=1)).all())
+        check(fz, z, pre + bias)
+    elif op == 1:
+        nv.call("axn_gemm_dgrad_ws", nv.ptr(a), nv.ptr(b), nv.ptr(c), code, M, N, K, a.stride(0), b.stride(0),
+                c.stride(0), *tail)
+        check(full, c, a.double() @ b.double())
+    else:
+        c.fill_(3.0)
+        nv.call("axn_gemm_wgrad_ws", nv.ptr(a), nv.ptr(b), nv.ptr(c), code, M, N, K, a.stride(0), b.stride(0),
+                c.stride(0), 1, nv.F32, *tail)
+        check(full, c, a.double().t() @ b.double() + 3.0)
+    assert bool(torch.isnan(ws[nbytes // 4:]).all()), "written behind the workspace"

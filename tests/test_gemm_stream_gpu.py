@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 CANARY = 7.0
 
 
-@pytest.mark.parametrize("M", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [(8, 8), (24, 64), (1000, 72), (4096, 328), (4104, 1024), (8200, 264), (16392, 200)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_tokens_are_exact(M, N, K, dtype):

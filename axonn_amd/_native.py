@@ -21,7 +21,7 @@ AXN_ELIMIT = -5
 BF16, F16, F32 = 0, 1, 2
 EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_GELU = 0, 1, 2, 3
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 # Every symbol include/axn.h declares: name -> (restype, argtypes)
 _c = ctypes
@@ -83,6 +83,10 @@ SYMBOLS = {
     "axn_gemm_fwd_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "axn_gemm_dgrad_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     "axn_gemm_wgrad_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
+    "axn_gemm_f32_workspace_bytes": (_sz, [_int, _i64, _i64, _i64]),
+    "axn_gemm_fwd_f32_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
+    "axn_gemm_dgrad_f32_ws": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp]),
+    "axn_gemm_wgrad_f32_ws": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "axn_mt_scan_workspace_bytes": (_sz, [_i64, _i64]),
     "axn_mt_scan": (_int, [_pp, _pi64, _i64, _int, _f32, _f32, _int, _vp, _vp, _sz, _vp]),
     "axn_mt_scan_norm": (_int, [_pp, _pi64, _i64, _int, _f32, _f32, _f32, _int, _vp, _vp, _sz, _vp]),

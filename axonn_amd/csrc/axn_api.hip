@@ -558,35 +558,67 @@ int axn_embedding_renorm(const int64_t* ids, void* W, int dtype, int64_t T, int6
                                  workspace_bytes, (hipStream_t)stream);
 }
 
+size_t axn_gemm_f32_workspace_bytes(int op, int64_t M, int64_t N, int64_t K) {
+  if (op < AXN_GEMM_FWD || op > AXN_GEMM_WGRAD || M < 1 || N < 1 || K < 1 || M > 0x7fffffff ||
+      N > 0x7fffffff || K > 0x7fffffff)
+    return 0;
+  GemmArgs g = {};
+  fill_gemm_args(g, op, nullptr, nullptr, nullptr, M, N, K, 0, 0, 0);
+  return gemm_f32_workspace_bytes(g.M, g.N, g.Kc);
+}
+
+int axn_gemm_fwd_f32_ws(const float* X, const float* W, const float* bias, float* Y,
+                        float* Zsave, int64_t M, int64_t N, int64_t K, int epilogue,
+                        void* workspace, size_t workspace_bytes, void* stream) {
+  const char* name = "axn_gemm_fwd_f32";
+  int rc = check_f32(name, X, W, Y, M, N, K);
+  if (rc) return rc;
+  REQUIRE(epilogue >= AXN_EPI_NONE && epilogue <= AXN_EPI_GELU, AXN_EINVAL,
+          "%s: unknown epilogue %d", name, epilogue);
+  const bool needs_bias = epilogue == AXN_EPI_BIAS || epilogue == AXN_EPI_BIAS_GELU;
+  REQUIRE(!needs_bias || bias != nullptr, AXN_EINVAL,
+          "%s: epilogue %d needs a bias vector", name, epilogue);
+  REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+  return launch_gemm_f32(GEMM_NT, X, W, Y, bias, Zsave, (int)M, (int)N, (int)K, epilogue, 0,
+                         (float*)workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int axn_gemm_dgrad_f32_ws(const float* dY, const float* W, float* dX, int64_t M, int64_t N,
+                          int64_t K, void* workspace, size_t workspace_bytes, void* stream) {
+  const char* name = "axn_gemm_dgrad_f32";
+  int rc = check_f32(name, dY, W, dX, M, N, K);
+  if (rc) return rc;
+  REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+  return launch_gemm_f32(GEMM_NN, dY, W, dX, nullptr, nullptr, (int)M, (int)K, (int)N,
+                         AXN_EPI_NONE, 0, (float*)workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int axn_gemm_wgrad_f32_ws(const float* dY, const float* X, float* dW, int64_t M, int64_t N,
+                          int64_t K, int beta, void* workspace, size_t workspace_bytes,
+                          void* stream) {
+  const char* name = "axn_gemm_wgrad_f32";
+  int rc = check_f32(name, dY, X, dW, M, N, K);
+  if (rc) return rc;
+  REQUIRE(beta == 0 || beta == 1, AXN_EINVAL, "%s: beta must be 0 or 1", name);
+  REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+  return launch_gemm_f32(GEMM_TN, dY, X, dW, nullptr, nullptr, (int)N, (int)K, (int)M,
+                         AXN_EPI_NONE, beta, (float*)workspace, workspace_bytes, (hipStream_t)stream);
+}
+
 int axn_gemm_fwd_f32(const float* X, const float* W, const float* bias, float* Y,
                      float* Zsave, int64_t M, int64_t N, int64_t K, int epilogue,
                      void* stream) {
-  int rc = check_f32("axn_gemm_fwd_f32", X, W, Y, M, N, K);
-  if (rc) return rc;
-  REQUIRE(epilogue >= AXN_EPI_NONE && epilogue <= AXN_EPI_GELU, AXN_EINVAL,
-          "axn_gemm_fwd_f32: unknown epilogue %d", epilogue);
-  const bool needs_bias = epilogue == AXN_EPI_BIAS || epilogue == AXN_EPI_BIAS_GELU;
-  REQUIRE(!needs_bias || bias != nullptr, AXN_EINVAL,
-          "axn_gemm_fwd_f32: epilogue %d needs a bias vector", epilogue);
-  return launch_gemm_f32(GEMM_NT, X, W, Y, bias, Zsave, (int)M, (int)N, (int)K,
-                         epilogue, 0, (hipStream_t)stream);
+  return axn_gemm_fwd_f32_ws(X, W, bias, Y, Zsave, M, N, K, epilogue, nullptr, 0, stream);
 }
 
 int axn_gemm_dgrad_f32(const float* dY, const float* W, float* dX, int64_t M,
                        int64_t N, int64_t K, void* stream) {
-  int rc = check_f32("axn_gemm_dgrad_f32", dY, W, dX, M, N, K);
-  if (rc) return rc;
-  return launch_gemm_f32(GEMM_NN, dY, W, dX, nullptr, nullptr, (int)M, (int)K,
-                         (int)N, AXN_EPI_NONE, 0, (hipStream_t)stream);
+  return axn_gemm_dgrad_f32_ws(dY, W, dX, M, N, K, nullptr, 0, stream);
 }
 
 int axn_gemm_wgrad_f32(const float* dY, const float* X, float* dW, int64_t M,
                        int64_t N, int64_t K, int beta, void* stream) {
-  int rc = check_f32("axn_gemm_wgrad_f32", dY, X, dW, M, N, K);
-  if (rc) return rc;
-  REQUIRE(beta == 0 || beta == 1, AXN_EINVAL, "axn_gemm_wgrad_f32: beta must be 0 or 1");
-  return launch_gemm_f32(GEMM_TN, dY, X, dW, nullptr, nullptr, (int)N, (int)K,
-                         (int)M, AXN_EPI_NONE, beta, (hipStream_t)stream);
+  return axn_gemm_wgrad_f32_ws(dY, X, dW, M, N, K, beta, nullptr, 0, stream);
 }
 
 size_t axn_mt_scan_workspace_bytes(int64_t n, int64_t total) {

@@ -3,7 +3,10 @@
 // same three products as the bf16 path (fully_connected.py:118, :140, :147-151)
 // with fp32 operands, for any M, N, K >= 1.
 //
-// One wave per workgroup owns a (16 FM) x (16 FN) output tile and feeds
+// Two kernels.  gemm_f32_split_kernel forms each fp32 product from six bf16 products on LDS
+// tiles and carries the large problems; gemm_f32_kernel uses the fp32 matrix instruction.
+//
+// gemm_f32_kernel: one wave per workgroup owns a (16 FM) x (16 FN) output tile and feeds
 // v_mfma_f32_16x16x4_f32 (true fp32 products, fp32 accumulate) straight from
 // global memory: no LDS, no barriers.  A 16 x 4 operand block wants, in lane l,
 // the element of one row (r = l % 16) and contraction index q = l / 16; MFMA s of a
@@ -15,14 +18,17 @@
 //   * an operand stored the other way round is read with one FM- (FN-) float load
 //     per contraction index (the lane's FM consecutive rows), and
 //   * a lane stores FN consecutive output columns at once.
-// Full-precision layers are small or rare here: tiles are chosen for many waves
-// (latency hiding by occupancy and by U blocks of loads in flight per wave).
+// Its tiles are chosen for many waves (latency hiding by occupancy and by U blocks of loads
+// in flight per wave).
 #include "axn_internal.h"
 
 namespace axn {
 namespace {
 
+typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
 // Full-precision layers keep the library erff.
 __device__ __forceinline__ float gelu_erff(float z) {
@@ -48,10 +54,10 @@ __device__ __forceinline__ float vec_get(const typename VecOf<F>::type& v, int i
 //   KMAJOR: element (row, k) at base[row * Kc + k]; else at base[k * rows + row]
 //   VEC:    Kc % 4 == 0, a 16-byte aligned base and (unless KMAJOR) rows % F == 0:
 //           vector loads
-//   GUARD:  indices >= Kc read as zero (the tail of the contraction)
+//   GUARD:  indices >= k_end read as zero (the end of a contraction, or of a part of one)
 template <bool KMAJOR, int F, bool VEC, bool GUARD>
 __device__ __forceinline__ void load_block(float (&x)[F][4], const float* __restrict__ base,
-                                           int row0, int rows, int k, int Kc) {
+                                           int row0, int rows, int k, int Kc, int k_end) {
 #pragma unroll
   for (int f = 0; f < F; ++f)
 #pragma unroll
@@ -61,7 +67,7 @@ __device__ __forceinline__ void load_block(float (&x)[F][4], const float* __rest
     for (int f = 0; f < F; ++f) {
       const float* p = base + (int64_t)min(row0 + f, rows - 1) * Kc;
       if (VEC) {  // the four indices are in or out together
-        if (!GUARD || k < Kc) {
+        if (!GUARD || k < k_end) {
           const f32x4 v = *(const f32x4*)(p + k);
 #pragma unroll
           for (int s = 0; s < 4; ++s) x[f][s] = v[s];
@@ -69,14 +75,14 @@ __device__ __forceinline__ void load_block(float (&x)[F][4], const float* __rest
       } else {
 #pragma unroll
         for (int s = 0; s < 4; ++s)
-          if (!GUARD || k + s < Kc) x[f][s] = p[k + s];
+          if (!GUARD || k + s < k_end) x[f][s] = p[k + s];
       }
     }
   } else if (VEC) {  // the F rows are in or out together
     const float* p = base + min(row0, rows - F);
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      if (!GUARD || k + s < Kc) {
+      if (!GUARD || k + s < k_end) {
         const typename VecOf<F>::type v = *(const typename VecOf<F>::type*)(p + (int64_t)(k + s) * rows);
 #pragma unroll
         for (int f = 0; f < F; ++f) x[f][s] = vec_get<F>(v, f);
@@ -87,33 +93,26 @@ __device__ __forceinline__ void load_block(float (&x)[F][4], const float* __rest
       const float* p = base + min(row0 + f, rows - 1);
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        if (!GUARD || k + s < Kc) x[f][s] = p[(int64_t)(k + s) * rows];
+        if (!GUARD || k + s < k_end) x[f][s] = p[(int64_t)(k + s) * rows];
     }
   }
 }
 
-// WAVES > 1: the waves of a workgroup share one tile and take the 16 U-deep chunks of
-// the contraction in turn; their partial sums meet in LDS and are added in wave order.
-template <bool AK, bool BKM, int EPI, int FM, int FN, int U, bool VEC, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES)
-    gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                    float* __restrict__ C, const float* __restrict__ bias,
-                    float* __restrict__ Z, int M, int N, int Kc, int tiles_n, int beta) {
-  const int lane = threadIdx.x & 63;
-  const int wave = WAVES > 1 ? threadIdx.x >> 6 : 0;
-  const int r = lane & 15, q = lane >> 4;
-  const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
-  const int m0 = tm * 16 * FM, n0 = tn * 16 * FN;
-  // Rows and columns past the edge read a valid one: their products land in output
-  // elements that are never stored.
-  const int arow = m0 + FM * r, bcol = n0 + FN * r;
-
-  f32x4 acc[FM][FN];
+template <int FM, int FN>
+__device__ __forceinline__ void clear(f32x4 (&acc)[FM][FN]) {
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
 
+// acc[i][j] += the products of contraction indices [k_begin, k_end) for rows arow + i and columns
+// bcol + j of the lane, in fp32 MFMAs; this wave takes the 16 U-deep chunks first, first + step, ...
+template <bool AK, bool BKM, int FM, int FN, int U, bool VEC>
+__device__ __forceinline__ void direct_tile(f32x4 (&acc)[FM][FN], const float* __restrict__ A,
+                                            const float* __restrict__ B, int arow, int bcol, int M, int N,
+                                            int Kc, int k_begin, int k_end, int first, int step) {
+  const int q = (threadIdx.x & 63) >> 4;
   auto blocks = [&](auto guard_, int k0, auto nblk_) {
     constexpr bool GUARD = decltype(guard_)::value;
     constexpr int NB = decltype(nblk_)::value;
@@ -121,8 +120,8 @@ __global__ void __launch_bounds__(64 * WAVES)
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
       const int k = k0 + 16 * u + 4 * q;
-      load_block<AK, FM, VEC, GUARD>(a[u], A, arow, M, k, Kc);
-      load_block<BKM, FN, VEC, GUARD>(b[u], B, bcol, N, k, Kc);
+      load_block<AK, FM, VEC, GUARD>(a[u], A, arow, M, k, Kc, k_end);
+      load_block<BKM, FN, VEC, GUARD>(b[u], B, bcol, N, k, Kc, k_end);
     }
 #pragma unroll
     for (int u = 0; u < NB; ++u)
@@ -134,32 +133,21 @@ __global__ void __launch_bounds__(64 * WAVES)
           for (int j = 0; j < FN; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i][s], b[u][j][s], acc[i][j], 0, 0, 0);
   };
-
-  const int whole = Kc / (16 * U) * (16 * U);  // the part made of whole chunks
-  for (int k0 = wave * 16 * U; k0 < whole; k0 += WAVES * 16 * U)
+  const int whole = k_begin + (k_end - k_begin) / (16 * U) * (16 * U);  // the part made of whole chunks
+  for (int k0 = k_begin + first * 16 * U; k0 < whole; k0 += step * 16 * U)
     blocks(std::false_type{}, k0, std::integral_constant<int, U>{});
-  for (int k0 = whole + wave * 16; k0 < Kc; k0 += WAVES * 16)
+  for (int k0 = whole + first * 16; k0 < k_end; k0 += step * 16)
     blocks(std::true_type{}, k0, std::integral_constant<int, 1>{});
+}
 
-  if constexpr (WAVES > 1) {
-    __shared__ f32x4 part[WAVES - 1][FM * FN][64];
-    if (wave > 0) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) part[wave - 1][i * FN + j][lane] = acc[i][j];
-    }
-    __syncthreads();
-    if (wave > 0) return;
-#pragma unroll
-    for (int w = 0; w < WAVES - 1; ++w)
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] += part[w][i * FN + j][lane];
-  }
-
-  // Register v of acc[i][j] in lane (r, q) is output row FM (4 q + v) + i, column FN r + j.
+// Stores a wave's 16 FM x 16 FN results at (m0, n0): register v of acc[i][j] in lane (r, q) is
+// output row m0 + FM (4 q + v) + i, column n0 + FN r + j.
+template <int EPI, int FM, int FN, bool VEC>
+__device__ __forceinline__ void store_tile(const f32x4 (&acc)[FM][FN], float* __restrict__ C,
+                                           const float* __restrict__ bias, float* __restrict__ Z, int m0,
+                                           int n0, int M, int N, int beta) {
+  const int r = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+  const int bcol = n0 + FN * r;
   using vec = typename VecOf<FN>::type;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -219,6 +207,218 @@ __global__ void __launch_bounds__(64 * WAVES)
     }
 }
 
+// WAVES > 1: the waves of a workgroup share one tile and take the 16 U-deep chunks of
+// the contraction in turn; their partial sums meet in LDS and are added in wave order.
+template <bool AK, bool BKM, int EPI, int FM, int FN, int U, bool VEC, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+    gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                    float* __restrict__ C, const float* __restrict__ bias,
+                    float* __restrict__ Z, int M, int N, int Kc, int tiles_n, int beta) {
+  const int lane = threadIdx.x & 63;
+  const int wave = WAVES > 1 ? threadIdx.x >> 6 : 0;
+  const int r = lane & 15;
+  const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
+  const int m0 = tm * 16 * FM, n0 = tn * 16 * FN;
+  f32x4 acc[FM][FN];
+  clear(acc);
+  // Rows and columns past the edge read a valid one: their products land in output
+  // elements that are never stored.
+  direct_tile<AK, BKM, FM, FN, U, VEC>(acc, A, B, m0 + FM * r, n0 + FN * r, M, N, Kc, 0, Kc, wave, WAVES);
+
+  if constexpr (WAVES > 1) {
+    __shared__ f32x4 part[WAVES - 1][FM * FN][64];
+    if (wave > 0) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) part[wave - 1][i * FN + j][lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 0; w < WAVES - 1; ++w)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] += part[w][i * FN + j][lane];
+  }
+
+  store_tile<EPI, FM, FN, VEC>(acc, C, bias, Z, m0, n0, M, N, beta);
+}
+
+// ---- fp32 products on the 16-bit matrix units ---------------------------------
+// v_mfma_f32_16x16x4_f32 runs at a sixteenth of the bf16 rate.  A float is the sum of three bf16
+// numbers (8 significant bits each; the remainders are exact), so a product of floats is nine products
+// of bf16, each exact in fp32.  The six that are not below 2^-24 of the whole are taken.  a1 b1 goes to
+// one accumulator, the five smaller ones, least first, to another that is added at the end: its roundings
+// are 2^-8 as large, so the sum sees one rounding per 32 contraction indices (the native instruction: one
+// per 4).  Error against 64 bits, normal operands, native / this: contraction of 128 2.0e-7 / 6.6e-8,
+// 1024 5.7e-7 / 1.9e-7, 4096 (native by four waves) 5.7e-7 / 4.0e-7; in one accumulator 4096 has 1.0e-6.
+//
+// The three parts carry a float's precision where the third is not below bf16's range, and an infinity
+// has no remainder.  So a wave whose results hold a NaN, an infinity or a non-zero magnitude under
+// 2^-64 computes its tile again with native products (direct_tile): operands of 2^-100 cannot reach a
+// result above that bound unnoticed unless their counterparts are above 2^36.
+//
+// Four waves (2 x 2) own a 32 FM x 32 FN tile.  Each thread loads its share of a 32-deep stage into
+// registers one stage ahead, splits it and writes three bf16 planes to LDS ([row][32], 64 bytes a row);
+// splitting before LDS costs each element once a workgroup instead of once a wave.  Row rho of a plane is
+// row F (rho % 32) + rho / 32 of the tile, for both storage orders: the thread that holds F consecutive
+// rows of a contraction-strided operand writes to F places a bank apart from its neighbours', and a
+// lane's fragments are F consecutive rows (columns), as direct_tile and store_tile have them.  A row's
+// 16-byte pieces are permuted by part_of(rho) so that any 16 lanes of a fragment read hit 16 different
+// 16-byte bank groups.  LDS is single-buffered: two or three workgroups share a CU and fill each other's
+// barriers (their splitting and one's matrix instructions overlap).
+// LDS is single-buffered (48 KB for 128 x 128) so that two workgroups share a CU and fill each other's
+// barriers.  2048 x 4096, contraction 1024: 86 us, 200 TFLOP/s of fp32 products (native 201 us); what
+// bounds it is the chain of stores, barrier, fragment reads and matrix instructions of a stage, not one
+// unit: two LDS buffers with one barrier (one workgroup a CU) 122 us, splitting by truncation without the
+// conversions 97, against 98 in the same run.
+template <int F>
+struct Planes {
+  uint16_t at[3][32 * F][32];
+};
+
+__device__ __forceinline__ int part_of(int rho) {
+  const int g = (rho >> 2) & 3;
+  return ((g << 1) ^ ((g >> 1) * 3)) & 3;  // 0 2 3 1
+}
+
+// Four floats as three times four bf16.
+__device__ __forceinline__ void split4(const float (&x)[4], uint2 (&out)[3]) {
+  float rest[4] = {x[0], x[1], x[2], x[3]};
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    uint32_t u[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x2 v = {rest[2 * h], rest[2 * h + 1]};
+      u[h] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+      if (p < 2) {
+        rest[2 * h] -= __builtin_bit_cast(float, u[h] << 16);
+        rest[2 * h + 1] -= __builtin_bit_cast(float, u[h] & 0xffff0000u);
+      }
+    }
+    out[p] = uint2{u[0], u[1]};
+  }
+}
+
+// Row group g (F rows) and quad (4 contraction indices) a thread stages, one of 32 x 8.
+template <bool KMAJOR>
+__device__ __forceinline__ void my_share(int& g, int& quad) {
+  const int t = threadIdx.x;
+  g = KMAJOR ? t >> 3 : t & 31;
+  quad = KMAJOR ? t & 7 : t >> 5;
+}
+
+template <bool KMAJOR, int F>
+__device__ __forceinline__ void put_stage(Planes<F>& lds, const float (&x)[F][4]) {
+  int g, quad;
+  my_share<KMAJOR>(g, quad);
+  const int at = (((quad >> 1) ^ part_of(g)) << 3) + ((quad & 1) << 2);  // 32 i does not change part_of
+#pragma unroll
+  for (int i = 0; i < F; ++i) {
+    uint2 p[3];
+    split4(x[i], p);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) *(uint2*)&lds.at[s][32 * i + g][at] = p[s];
+  }
+}
+
+// The parts of the five smaller products, least first.
+constexpr int kPartA[5] = {2, 0, 1, 1, 0}, kPartB[5] = {0, 2, 1, 0, 1};
+
+template <int FM, int FN>
+__device__ __forceinline__ void split_stage(f32x4 (&acc)[FM][FN], f32x4 (&low)[FM][FN], const Planes<FM>& la,
+                                            const Planes<FN>& lb) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, at = ((lane >> 4) ^ part_of(r)) << 3;
+  const int ra = 16 * (wave >> 1) + r, rb = 16 * (wave & 1) + r;
+  bf16x8 a[FM][3];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) a[i][p] = *(const bf16x8*)&la.at[p][32 * i + ra][at];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    bf16x8 b[3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) b[p] = *(const bf16x8*)&lb.at[p][32 * j + rb][at];
+#pragma unroll
+    for (int t = 0; t < 5; ++t)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+        low[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][kPartA[t]], b[kPartB[t]], low[i][j], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][0], b[0], acc[i][j], 0, 0, 0);
+  }
+}
+
+// parts > 1: workgroup id / tiles is the part, which covers k_part contraction indices and stores
+// its products at C + part * M * N.
+template <bool AK, bool BKM, int EPI, int FM, int FN, bool VEC>
+__global__ void __launch_bounds__(256, 2)
+    gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                          float* __restrict__ C, const float* __restrict__ bias, float* __restrict__ Z,
+                          int M, int N, int Kc, int tiles_m, int tiles_n, int k_part, int beta) {
+  __shared__ Planes<FM> la;
+  __shared__ Planes<FN> lb;
+  const int tiles = tiles_m * tiles_n;
+  const int part = blockIdx.x / tiles, id = blockIdx.x - part * tiles;
+  const int tm = id / tiles_n, tn = id - tm * tiles_n;
+  const int m0 = tm * 32 * FM, n0 = tn * 32 * FN;
+  const int k_begin = part * k_part, k_end = min(Kc, k_begin + k_part);
+  C += (int64_t)part * M * N;
+
+  f32x4 acc[FM][FN], low[FM][FN];
+  clear(acc);
+  clear(low);
+  int ga, qa, gb, qb;
+  my_share<AK>(ga, qa);
+  my_share<BKM>(gb, qb);
+  float xa[FM][4], xb[FN][4];
+  // Rows past the edge read a valid one, indices past the end count as zero.
+  auto fetch = [&](int k0) {
+    if (k0 + 32 <= k_end) {
+      load_block<AK, FM, VEC, false>(xa, A, m0 + FM * ga, M, k0 + 4 * qa, Kc, k_end);
+      load_block<BKM, FN, VEC, false>(xb, B, n0 + FN * gb, N, k0 + 4 * qb, Kc, k_end);
+    } else {
+      load_block<AK, FM, VEC, true>(xa, A, m0 + FM * ga, M, k0 + 4 * qa, Kc, k_end);
+      load_block<BKM, FN, VEC, true>(xb, B, n0 + FN * gb, N, k0 + 4 * qb, Kc, k_end);
+    }
+  };
+  fetch(k_begin);
+  for (int k0 = k_begin; k0 < k_end; k0 += 32) {
+    put_stage<AK, FM>(la, xa);
+    put_stage<BKM, FN>(lb, xb);
+    __syncthreads();
+    if (k0 + 32 < k_end) fetch(k0 + 32);
+    split_stage<FM, FN>(acc, low, la, lb);
+    __syncthreads();
+  }
+
+  const int wave = threadIdx.x >> 6, r = threadIdx.x & 15;
+  const int mw = m0 + 16 * FM * (wave >> 1), nw = n0 + 16 * FN * (wave & 1);
+  bool odd = false;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      acc[i][j] += low[i][j];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float c = fabsf(acc[i][j][v]);
+        odd |= !(c == 0.f || (c >= 0x1p-64f && c <= 0x1.fffffep127f));
+      }
+    }
+  if (__builtin_amdgcn_ballot_w64(odd)) {
+    clear(acc);
+    direct_tile<AK, BKM, FM, FN, 1, VEC>(acc, A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end, 0, 1);
+  }
+  store_tile<EPI, FM, FN, VEC>(acc, C, bias, Z, mw, nw, M, N, beta);
+}
+
 template <bool AK, bool BKM, int EPI, int FM, int FN, int U, int WAVES>
 int launch_tile(const float* A, const float* B, float* C, const float* bias, float* Z, int M,
                 int N, int Kc, int beta, hipStream_t stream) {
@@ -242,7 +442,99 @@ int launch_tile(const float* A, const float* B, float* C, const float* bias, flo
   return AXN_OK;
 }
 
-// The largest of the 64 x 64, 32 x 32 and 16 x 16 tiles (a loaded element is used 4,
+// Adds the parts of a split contraction in part order, then the epilogue.
+template <int EPI, bool VEC>
+__global__ void __launch_bounds__(256)
+    f32_parts_kernel(const float* __restrict__ ws, float* __restrict__ C, const float* __restrict__ bias,
+                     float* __restrict__ Z, int64_t MN, int N, int parts, int beta) {
+  constexpr int W = VEC ? 4 : 1;
+  using vec = typename VecOf<W>::type;
+  const int64_t o = ((int64_t)blockIdx.x * 256 + threadIdx.x) * W;
+  if (o >= MN) return;
+  vec x = __builtin_nontemporal_load((const vec*)(ws + o));
+  for (int p = 1; p < parts; ++p) x += __builtin_nontemporal_load((const vec*)(ws + p * MN + o));
+  if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU) x += *(const vec*)(bias + o % N);
+  if (EPI == AXN_EPI_BIAS_GELU || EPI == AXN_EPI_GELU) {
+    if (Z != nullptr) *(vec*)(Z + o) = x;
+    if constexpr (W == 1) x = gelu_erff(x);
+    else
+#pragma unroll
+      for (int i = 0; i < W; ++i) x[i] = gelu_erff(x[i]);
+  }
+  if (beta) x += *(const vec*)(C + o);
+  *(vec*)(C + o) = x;
+}
+
+// Problems of 2^32 multiply-adds and more are split into bf16 products, with the contraction in as many
+// parts as the estimate below finds fastest (0: not split into products at all).  The line is drawn by
+// results, not by speed (512 x 4096 x 1024 is 61 us natively and 41 split, 64 x 4096 x 1024 18 and 16):
+// Adam divides a gradient by its own magnitude, so where one is next to zero the last bits of a product
+// become 1e-2 of the learning rate (batch 64 through a 1024 - 4096 - 1024 perceptron: one weight moves by
+// 6e-4 of the weights' rms in a step, which is the native kernel's rounding, not the split one's).  Small
+// full-precision networks, where launches and the host bound a step, keep the bits they have; above the
+// line the products bound it and the split ones, 2.4 times as fast and nearer to exact, are taken.
+constexpr double kSplitWork = 4294967296.0;
+
+// Parts of the contraction, by estimated time in us: a 32-deep stage takes 1.85 for a workgroup alone on
+// its CU and 2.7 for two side by side, adding the parts takes a launch and their traffic.  Fitted to
+// 30 problems from 8.6 to 69 GFLOP: 0.3 % off the best number of parts, and 2 % off the best of four tile
+// sizes, on average.  2048 x 1024, contraction 4096: 1 part 217 us, 2 128, 4 99, 8 107.
+struct F32Plan {
+  int parts, k_part;
+};
+F32Plan plan_f32(int64_t M, int64_t N, int64_t Kc, bool may_split) {
+  constexpr int kCUs = 256, kMostParts = 16;
+  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  F32Plan best = {0, 0};
+  if ((double)M * (double)N * (double)Kc < kSplitWork || tiles * kMostParts > 0x7fffffffLL) return best;
+  double least = 0;
+  for (int p = 1; p <= (may_split ? kMostParts : 1); ++p) {
+    const int64_t k_part = ((Kc + p - 1) / p + 31) / 32 * 32;
+    if ((Kc + k_part - 1) / k_part != p) continue;
+    const int64_t load = (tiles * p + kCUs - 1) / kCUs;   // workgroups on the fullest CU
+    double us = (double)(k_part / 32) * ((double)(load / 2) * 2.7 + (double)(load % 2) * 1.85);
+    if (p > 1) us += 3.0 + (p + 1) * (double)M * (double)N * 0.8e-6;
+    if (p == 1 || us < least) least = us, best = {p, (int)k_part};
+  }
+  return best;
+}
+
+template <bool AK, bool BKM, int EPI>
+int launch_split(const float* A, const float* B, float* C, const float* bias, float* Z, int M, int N,
+                      int Kc, int beta, const F32Plan& plan, hipStream_t stream) {
+  constexpr int F = 4;
+  const int tiles_m = (M + 32 * F - 1) / (32 * F), tiles_n = (N + 32 * F - 1) / (32 * F);
+  const dim3 grid((unsigned)((int64_t)tiles_m * tiles_n * plan.parts)), block(256);
+  // as launch_tile's
+  const uintptr_t ptrs = (uintptr_t)A | (uintptr_t)B | (uintptr_t)C | (uintptr_t)bias | (uintptr_t)Z;
+  const bool vec = Kc % 4 == 0 && (AK || M % F == 0) && N % F == 0 && (ptrs & 15u) == 0;
+  if (vec)
+    hipLaunchKernelGGL((gemm_f32_split_kernel<AK, BKM, EPI, F, F, true>), grid, block, 0, stream, A, B, C,
+                       bias, Z, M, N, Kc, tiles_m, tiles_n, plan.k_part, beta);
+  else
+    hipLaunchKernelGGL((gemm_f32_split_kernel<AK, BKM, EPI, F, F, false>), grid, block, 0, stream, A, B, C,
+                       bias, Z, M, N, Kc, tiles_m, tiles_n, plan.k_part, beta);
+  AXN_HIP_TRY(hipGetLastError());
+  return AXN_OK;
+}
+
+template <int EPI>
+int launch_parts(const float* ws, float* C, const float* bias, float* Z, int M, int N, int parts, int beta,
+                 hipStream_t stream) {
+  const int64_t MN = (int64_t)M * N;
+  const uintptr_t ptrs = (uintptr_t)ws | (uintptr_t)C | (uintptr_t)bias | (uintptr_t)Z;
+  const bool vec = N % 4 == 0 && (ptrs & 15u) == 0;
+  const int64_t lanes = vec ? MN / 4 : MN;
+  const dim3 grid((unsigned)((lanes + 255) / 256)), block(256);
+  if (vec)
+    hipLaunchKernelGGL((f32_parts_kernel<EPI, true>), grid, block, 0, stream, ws, C, bias, Z, MN, N, parts, beta);
+  else
+    hipLaunchKernelGGL((f32_parts_kernel<EPI, false>), grid, block, 0, stream, ws, C, bias, Z, MN, N, parts, beta);
+  AXN_HIP_TRY(hipGetLastError());
+  return AXN_OK;
+}
+
+// The native kernel's tile: the largest of 64 x 64, 32 x 32 and 16 x 16 (a loaded element is used 4,
 // 2, 1 times) that still gives the chip's 1024 SIMDs a wave each; smaller tiles keep
 // more loads in flight per wave.  With fewer than 4096 tiles and a contraction of KMIN
 // or more (256 for the smallest tile, 2048 for the middle one; measured: the split
@@ -257,7 +549,19 @@ int launch_waves(long long tiles, const float* A, const float* B, float* C, cons
 
 template <bool AK, bool BKM, int EPI>
 int launch_epi(const float* A, const float* B, float* C, const float* bias, float* Z, int M, int N,
-               int Kc, int beta, hipStream_t stream) {
+               int Kc, int beta, float* ws, size_t ws_bytes, hipStream_t stream) {
+  const F32Plan plan = plan_f32(M, N, Kc, ws != nullptr);
+  if (plan.parts > 1) {
+    const size_t need = (size_t)plan.parts * (size_t)M * (size_t)N * sizeof(float);
+    if (ws_bytes < need) {
+      set_error("gemm_f32: workspace too small (%zu bytes given, %zu needed)", ws_bytes, need);
+      return AXN_EINVAL;
+    }
+    const int rc = launch_split<AK, BKM, AXN_EPI_NONE>(A, B, ws, nullptr, nullptr, M, N, Kc, 0, plan, stream);
+    return rc ? rc : launch_parts<EPI>(ws, C, bias, Z, M, N, plan.parts, beta, stream);
+  }
+  if (plan.parts == 1)
+    return launch_split<AK, BKM, EPI>(A, B, C, bias, Z, M, N, Kc, beta, plan, stream);
   const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64);
   const long long tiles32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
   const long long tiles16 = (long long)((M + 15) / 16) * ((N + 15) / 16);
@@ -270,25 +574,30 @@ int launch_epi(const float* A, const float* B, float* C, const float* bias, floa
 
 }  // namespace
 
+size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t Kc) {
+  const F32Plan plan = plan_f32(M, N, Kc, true);
+  return plan.parts > 1 ? (size_t)plan.parts * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
 int launch_gemm_f32(GemmLayout layout, const float* A, const float* B, float* C,
                     const float* bias, float* Z, int M, int N, int Kc,
-                    int epilogue, int beta, hipStream_t stream) {
+                    int epilogue, int beta, float* ws, size_t ws_bytes, hipStream_t stream) {
   switch (layout) {
     case GEMM_NT:
       switch (epilogue) {
         case AXN_EPI_NONE:
-          return launch_epi<true, true, AXN_EPI_NONE>(A, B, C, bias, Z, M, N, Kc, beta, stream);
+          return launch_epi<true, true, AXN_EPI_NONE>(A, B, C, bias, Z, M, N, Kc, beta, ws, ws_bytes, stream);
         case AXN_EPI_BIAS:
-          return launch_epi<true, true, AXN_EPI_BIAS>(A, B, C, bias, Z, M, N, Kc, beta, stream);
+          return launch_epi<true, true, AXN_EPI_BIAS>(A, B, C, bias, Z, M, N, Kc, beta, ws, ws_bytes, stream);
         case AXN_EPI_BIAS_GELU:
-          return launch_epi<true, true, AXN_EPI_BIAS_GELU>(A, B, C, bias, Z, M, N, Kc, beta, stream);
+          return launch_epi<true, true, AXN_EPI_BIAS_GELU>(A, B, C, bias, Z, M, N, Kc, beta, ws, ws_bytes, stream);
         default:
-          return launch_epi<true, true, AXN_EPI_GELU>(A, B, C, bias, Z, M, N, Kc, beta, stream);
+          return launch_epi<true, true, AXN_EPI_GELU>(A, B, C, bias, Z, M, N, Kc, beta, ws, ws_bytes, stream);
       }
     case GEMM_NN:
-      return launch_epi<true, false, AXN_EPI_NONE>(A, B, C, bias, Z, M, N, Kc, beta, stream);
+      return launch_epi<true, false, AXN_EPI_NONE>(A, B, C, bias, Z, M, N, Kc, beta, ws, ws_bytes, stream);
     default:
-      return launch_epi<false, false, AXN_EPI_NONE>(A, B, C, bias, Z, M, N, Kc, beta, stream);
+      return launch_epi<false, false, AXN_EPI_NONE>(A, B, C, bias, Z, M, N, Kc, beta, ws, ws_bytes, stream);
   }
 }
 

@@ -6,6 +6,8 @@ returns.  None of the arithmetic happens here, and nothing here falls back to a
 torch op: tensors that are not on a GPU are rejected.
 """
 
+import functools
+
 import torch
 
 from . import _native as nv
@@ -70,10 +72,17 @@ _GEMM16 = {torch.bfloat16: "", torch.float16: "_f16"}
 GEMM_FWD, GEMM_DGRAD, GEMM_WGRAD = 0, 1, 2
 
 
-def _split_workspace(op, M, N, K, device):
+@functools.lru_cache(maxsize=4096)
+def _workspace_bytes(op, M, N, K, f32=False):
+    """What the library would use, a function of the sizes alone (about 3 us to work out)."""
+    lib = nv.load()
+    return (lib.axn_gemm_f32_workspace_bytes if f32 else lib.axn_gemm_workspace_bytes)(op, M, N, K)
+
+
+def _split_workspace(op, M, N, K, device, f32=False):
     """Workspace for a GEMM whose contraction the library would divide among workgroups
     (few output tiles), or (None, 0)."""
-    nbytes = nv.load().axn_gemm_workspace_bytes(op, M, N, K)
+    nbytes = _workspace_bytes(op, M, N, K, f32)
     if nbytes == 0:
         return None, 0
     return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
@@ -131,8 +140,9 @@ def gemm_fwd(x, w, bias=None, activation=None, save_z=False, out_f32=False):
         x, w = x.contiguous(), w.contiguous()
         y = torch.empty((M, N), dtype=torch.float32, device=x.device)
         z = torch.empty_like(y) if want_z else None
-        nv.call("axn_gemm_fwd_f32", nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(y), nv.ptr(z),
-                M, N, K, epi, nv.current_stream())
+        ws, ws_bytes = _split_workspace(GEMM_FWD, M, N, K, x.device, f32=True)
+        nv.call("axn_gemm_fwd_f32_ws", nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(y), nv.ptr(z),
+                M, N, K, epi, nv.ptr(ws), ws_bytes, nv.current_stream())
     else:
         raise TypeError("the Linear kernels take bf16, fp16 or fp32 operands, got %s" % x.dtype)
     return y, z
@@ -166,8 +176,9 @@ def gemm_dgrad(dy, w):
     elif dy.dtype == torch.float32:
         dy, w = dy.contiguous(), w.contiguous()
         dx = torch.empty((M, K), dtype=torch.float32, device=dy.device)
-        nv.call("axn_gemm_dgrad_f32", nv.ptr(dy), nv.ptr(w), nv.ptr(dx), M, N, K,
-                nv.current_stream())
+        ws, ws_bytes = _split_workspace(GEMM_DGRAD, M, N, K, dy.device, f32=True)
+        nv.call("axn_gemm_dgrad_f32_ws", nv.ptr(dy), nv.ptr(w), nv.ptr(dx), M, N, K,
+                nv.ptr(ws), ws_bytes, nv.current_stream())
     else:
         raise TypeError("the Linear kernels take bf16, fp16 or fp32 operands, got %s" % dy.dtype)
     return dx
@@ -226,8 +237,9 @@ def gemm_wgrad(dy, x, out=None, accumulate=False, out_dtype=None):
         dy, x = dy.contiguous(), x.contiguous()
         if out is None:
             out = torch.empty((N, K), dtype=torch.float32, device=dy.device)
-        nv.call("axn_gemm_wgrad_f32", nv.ptr(dy), nv.ptr(x), nv.ptr(out), M, N, K,
-                1 if accumulate else 0, nv.current_stream())
+        ws, ws_bytes = _split_workspace(GEMM_WGRAD, M, N, K, dy.device, f32=True)
+        nv.call("axn_gemm_wgrad_f32_ws", nv.ptr(dy), nv.ptr(x), nv.ptr(out), M, N, K,
+                1 if accumulate else 0, nv.ptr(ws), ws_bytes, nv.current_stream())
     else:
         raise TypeError("the Linear kernels take bf16, fp16 or fp32 operands, got %s" % dy.dtype)
     return out
@@ -244,8 +256,8 @@ def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None):
     K = w.shape[1]
     plain16 = (dy.dtype in _GEMM16 and dy.dtype == w.dtype == x.dtype and M > 0
                and not _ragged16(dy.dtype, N, K)
-               and nv.load().axn_gemm_workspace_bytes(GEMM_DGRAD, M, N, K) == 0
-               and nv.load().axn_gemm_workspace_bytes(GEMM_WGRAD, M, N, K) == 0)
+               and _workspace_bytes(GEMM_DGRAD, M, N, K) == 0
+               and _workspace_bytes(GEMM_WGRAD, M, N, K) == 0)
     if not plain16:
         return gemm_dgrad(dy, w), gemm_wgrad(dy, x, out=out, accumulate=accumulate, out_dtype=out_dtype)
     if x.shape != (M, K) or w.shape[0] != N:

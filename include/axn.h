@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define AXN_ABI_VERSION 12
+#define AXN_ABI_VERSION 13
 
 #if defined(__GNUC__)
 #define AXN_API __attribute__((visibility("default")))
@@ -287,6 +287,19 @@ AXN_API int axn_gemm_dgrad_f32(const float* dY, const float* W, float* dX, int64
                        int64_t N, int64_t K, void* stream);
 AXN_API int axn_gemm_wgrad_f32(const float* dY, const float* X, float* dW, int64_t M,
                        int64_t N, int64_t K, int beta, void* stream);
+/* The same given a workspace (16-byte aligned, used by this call alone until it has finished;
+ * NULL: none) for contractions divided among workgroups: axn_gemm_f32_workspace_bytes(op, M, N, K)
+ * bytes, op an axn_gemm_op; 0 if the call would not divide it. */
+AXN_API size_t axn_gemm_f32_workspace_bytes(int op, int64_t M, int64_t N, int64_t K);
+AXN_API int axn_gemm_fwd_f32_ws(const float* X, const float* W, const float* bias,
+                        float* Y, float* Zsave, int64_t M, int64_t N, int64_t K,
+                        int epilogue, void* workspace, size_t workspace_bytes, void* stream);
+AXN_API int axn_gemm_dgrad_f32_ws(const float* dY, const float* W, float* dX, int64_t M,
+                          int64_t N, int64_t K, void* workspace, size_t workspace_bytes,
+                          void* stream);
+AXN_API int axn_gemm_wgrad_f32_ws(const float* dY, const float* X, float* dW, int64_t M,
+                          int64_t N, int64_t K, int beta, void* workspace,
+                          size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * Mixed-precision optimizer step over a list of tensors (multi-tensor).

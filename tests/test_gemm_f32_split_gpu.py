@@ -1,0 +1,81 @@
+"""fp32 products formed from bf16 parts (2^32 multiply-adds and more), whole and ragged, with vector and
+single-element accesses, with the contraction in one part and in several, against 64 bits."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def bound(K):
+    """Norm-wise: the dropped products are under 3 * 2^-24 of a product, the accumulators round once
+    per 32 contraction indices (at random), and the outputs once; twice that."""
+    return 2.0 * 2.0 ** -24 * (4 + (K / 32) ** 0.5)
+
+
+def err(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (2048, 4096, 1024), (2052, 4100, 1028), (2047, 4099, 1027),    # whole, ragged, no vector access
+    (256, 4096, 4128), (260, 4100, 4100), (257, 4099, 4103),       # parts, the last one shorter
+    (8192, 16384, 32), (8196, 16388, 36), (33, 16384, 8192),       # one stage, and a rest; few rows
+])
+def test_products_against_64_bits(M, N, K):
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    X, W, dY = (torch.randn(s, generator=g, device="cuda") for s in ((M, K), (N, K), (M, N)))
+    b = torch.randn(N, generator=g, device="cuda")
+    z64 = X.double() @ W.double().t() + b.double()
+    y, z = ops.gemm_fwd(X, W, bias=b, activation="gelu", save_z=True)
+    assert err(z, z64) < bound(K)
+    assert err(y, torch.nn.functional.gelu(z64)) < bound(K)
+    assert err(ops.gemm_fwd(X, W)[0], z64 - b.double()) < bound(K)
+    assert err(ops.gemm_dgrad(dY, W), dY.double() @ W.double()) < bound(N)
+    dw64 = dY.double().t() @ X.double()
+    dw = ops.gemm_wgrad(dY, X)
+    assert err(dw, dw64) < bound(M)
+    ops.gemm_wgrad(dY, X, out=dw, accumulate=True)
+    assert err(dw, 2 * dw64) < bound(M)
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 4096, 512), (512, 2048, 4096)])
+def test_infinities_and_nans_stay_where_they_belong(M, N, K):
+    """An infinity has no bf16 remainder (inf - inf): results that hold one are those of plain
+    fp32 arithmetic, the others are untouched; the largest floats round to a bf16 infinity."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    X, W = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    X[3, 5], X[70, 9], X[M - 1, K - 1] = float("inf"), float("nan"), -float("inf")
+    W[11, 7] = float("inf")
+    X[200, 8] = 3.4e38           # above the largest bf16
+    W[:, 8] *= 2.0 ** -20
+    want = X.double() @ W.double().t()
+    got = ops.gemm_fwd(X, W)[0]
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()] > 0, want[want.isinf()] > 0)
+    row = got[200].double()
+    ok = row.isfinite()
+    assert err(row[ok], want[200][ok]) < bound(K)
+    plain = torch.ones(M, dtype=torch.bool, device="cuda")
+    plain[[3, 70, 200, M - 1]] = False
+    cols = torch.ones(N, dtype=torch.bool, device="cuda")
+    cols[11] = False
+    assert err(got[plain][:, cols], want[plain][:, cols]) < bound(K)
+
+
+@pytest.mark.parametrize("exponent", [-120, -100, 60])
+def test_magnitudes_beyond_the_parts_keep_full_precision(exponent):
+    """A float of 2^-120 has its third part below bf16's range."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(4)
+    X = torch.randn(2048, 1024, generator=g, device="cuda")
+    W = torch.randn(2048, 1024, generator=g, device="cuda")
+    want = X.double() @ W.double().t()
+    got = ops.gemm_fwd(X * 2.0 ** exponent, W)[0]
+    assert err(got.double() * 2.0 ** -exponent, want) < 1e-6

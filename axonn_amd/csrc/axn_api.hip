@@ -288,14 +288,17 @@ static void fill_gemm_args(GemmArgs& g, int op, const void* a, const void* b, vo
 
 static const GemmLayout kLayoutOfOp[3] = {GEMM_NT, GEMM_NN, GEMM_TN};
 
+static size_t partial_bytes(const SplitPlan& plan, const GemmArgs& g) {
+  return plan.parts > 1 ? (size_t)plan.parts * (size_t)g.M * ((size_t)(g.N + 7) / 8 * 8) * sizeof(float) : 0;
+}
+
 size_t axn_gemm_workspace_bytes(int op, int64_t M, int64_t N, int64_t K) {
   if (op < AXN_GEMM_FWD || op > AXN_GEMM_WGRAD || M < 1 || N < 1 || K < 1 || M > 0x7fffffff ||
       N > 0x7fffffff || K > 0x7fffffff)
     return 0;
   GemmArgs g = {};
   fill_gemm_args(g, op, nullptr, nullptr, nullptr, M, N, K, 0, 0, 0);
-  const int s = gemm_splits(kLayoutOfOp[op], g.M, g.N, g.Kc).parts;
-  return s > 1 ? (size_t)s * (size_t)g.M * (size_t)g.N * sizeof(float) : 0;
+  return partial_bytes(gemm_splits(kLayoutOfOp[op], g.M, g.N, g.Kc), g);
 }
 
 static int gemm_ws(const char* name, int op, const void* a, const void* b, void* c, int dtype,
@@ -323,7 +326,7 @@ static int gemm_ws(const char* name, int op, const void* a, const void* b, void*
   const SplitPlan plan =
       workspace != nullptr && near ? gemm_splits(layout, g.M, g.N, g.Kc) : SplitPlan{1, EDGE_128x128};
   if (plan.parts > 1) {
-    const size_t need = (size_t)plan.parts * (size_t)g.M * (size_t)g.N * sizeof(float);
+    const size_t need = partial_bytes(plan, g);
     REQUIRE(workspace_bytes >= need, AXN_EINVAL,
             "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
     REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
@@ -332,6 +335,56 @@ static int gemm_ws(const char* name, int op, const void* a, const void* b, void*
   }
   return half ? launch_gemm_f16(layout, g, epilogue, out_dtype == AXN_F32, (hipStream_t)stream)
               : launch_gemm_bf16(layout, g, epilogue, out_dtype == AXN_F32, (hipStream_t)stream);
+}
+
+int axn_gemm_any_n(int op, const void* A, const void* B, const float* bias, void* C, void* Zsave,
+                   int dtype, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                   int64_t ldc, int epilogue, int beta, int out_dtype, void* workspace,
+                   size_t workspace_bytes, void* stream) {
+  const char* name = "axn_gemm_any_n";
+  const bool fwd = op == AXN_GEMM_FWD, wgrad = op == AXN_GEMM_WGRAD;
+  REQUIRE(op >= AXN_GEMM_FWD && op <= AXN_GEMM_WGRAD, AXN_EINVAL, "%s: unknown product %d", name, op);
+  REQUIRE(dtype == AXN_BF16 || dtype == AXN_F16, AXN_EINVAL, "%s: dtype must be bf16 or fp16", name);
+  REQUIRE(N >= 1 && N <= 0x7ffffff8, AXN_EINVAL, "%s: N out of range (got %lld)", name, (long long)N);
+  // everything but N itself and the rows of Y: as for the next multiple of 8
+  const int64_t n8 = (N + 7) / 8 * 8;
+  int rc = check_gemm(name, A, B, C, M, n8, K, lda, ldb, fwd ? n8 : ldc, fwd ? K : n8, K, fwd ? n8 : K);
+  if (rc) return rc;
+  REQUIRE(!fwd || ldc >= N, AXN_EINVAL, "%s: leading dimension smaller than the row length", name);
+  rc = check_epilogue(name, epilogue, bias);
+  if (rc) return rc;
+  REQUIRE(fwd || epilogue == AXN_EPI_NONE, AXN_EINVAL, "%s: only the forward has an epilogue", name);
+  REQUIRE(beta == 0 || (beta == 1 && wgrad), AXN_EINVAL, "%s: beta must be 0, or 1 for the weight gradient", name);
+  REQUIRE(out_dtype == dtype ||
+              (out_dtype == AXN_F32 && (wgrad || epilogue == AXN_EPI_BIAS || epilogue == AXN_EPI_BIAS_GELU)),
+          AXN_EINVAL, "%s: unsupported output type", name);
+  GemmArgs g = {};
+  fill_gemm_args(g, op, A, B, C, M, N, K, lda, ldb, ldc);
+  g.beta = beta;
+  g.bias = bias;
+  g.Z = (uint16_t*)Zsave;
+  const bool half = dtype == AXN_F16, out_f32 = out_dtype == AXN_F32;
+  const GemmLayout layout = kLayoutOfOp[op];
+  const bool near = lda < kEdgeMaxLd / 2 && ldb < kEdgeMaxLd / 2;
+  const SplitPlan plan =
+      workspace != nullptr && near ? gemm_splits(layout, g.M, g.N, g.Kc) : SplitPlan{1, EDGE_128x128};
+  if (plan.parts > 1) {
+    const size_t need = partial_bytes(plan, g);
+    REQUIRE(workspace_bytes >= need, AXN_EINVAL,
+            "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
+    REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+    return launch_gemm_splitk(layout, g, epilogue, half, out_f32, plan, (float*)workspace, (hipStream_t)stream);
+  }
+  return half ? launch_gemm_f16(layout, g, epilogue, out_f32, (hipStream_t)stream)
+              : launch_gemm_bf16(layout, g, epilogue, out_f32, (hipStream_t)stream);
+}
+
+int axn_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, void* stream) {
+  const char* name = "axn_pad_rows16";
+  REQUIRE(src && dst, AXN_EINVAL, "%s: null pointer", name);
+  REQUIRE(M >= 1 && N >= 1 && ld >= N, AXN_EINVAL, "%s: M, N >= 1 and ld >= N expected", name);
+  REQUIRE(((uintptr_t)src & 1u) == 0 && aligned16(dst), AXN_EALIGN, "%s: misaligned pointer", name);
+  return launch_pad_rows16(src, dst, M, N, ld, (hipStream_t)stream);
 }
 
 int axn_gemm_fwd_ws(const void* X, const void* W, const float* bias, void* Y, void* Zsave, int dtype,

@@ -132,7 +132,7 @@ enum EdgeTile { EDGE_256x256 = 0, EDGE_256x128 = 1, EDGE_128x128 = 2 };
 constexpr int64_t kEdgeMaxLd = 1LL << 23;
 // Split contraction for problems with few output tiles: into how many parts and on which
 // tile (parts = 1: do not split), and the launch: partial products in fp32 to `ws`
-// (parts * M * N floats), then one pass that adds them in part order, adds the old output if
+// (parts * M * N floats, N rounded up to a multiple of 8), then one pass that adds them in part order, adds the old output if
 // args.beta, applies the epilogue and stores args.C.
 struct SplitPlan {
   int parts;
@@ -181,6 +181,9 @@ size_t dgelu_dbias_workspace_bytes(int64_t M, int64_t N);
 int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
                        float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
                        void* ws, size_t ws_bytes, hipStream_t stream);
+
+// dst[M][8 ceil(N / 8)] = src[M][N] (row stride ld) of 16-bit elements, zeros behind N.
+int launch_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, hipStream_t stream);
 
 // ---- SwiGLU activation of the Llama MLP and its backward -----------------------
 int launch_swiglu_fwd(const void* gate, const void* up, void* out, int dtype, int64_t M,

@@ -282,14 +282,16 @@ namespace {
 
 // Sum of the fp32 partial products of a split contraction, in split order, then the output's
 // epilogue; 8 columns per lane.  Bound by its reads (512 x 8192, 2 parts: 7.3 us for 42 MB).
-template <int EPI, bool OUT_F32, bool HALF>
+// ANY: N is not a multiple of 8, or the output's rows are not 16-byte aligned; the partial products'
+// rows are padded to a multiple of 8.
+template <int EPI, bool OUT_F32, bool HALF, bool ANY>
 __global__ void __launch_bounds__(256)
     splitk_reduce_kernel(const float* __restrict__ ws, const GemmArgs g) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t per_row = g.N / 8;
+  const int64_t per_row = (g.N + 7) / 8;
   if (idx >= (int64_t)g.M * per_row) return;
-  const int64_t row = idx / per_row, col = (idx - row * per_row) * 8, part = (int64_t)g.M * g.N;
-  const float* p = ws + row * g.N + col;
+  const int64_t row = idx / per_row, col = (idx - row * per_row) * 8, part = (int64_t)g.M * per_row * 8;
+  const float* p = ws + row * per_row * 8 + col;
   f32x4 a0 = __builtin_nontemporal_load((const f32x4*)p);
   f32x4 a1 = __builtin_nontemporal_load((const f32x4*)(p + 4));
   for (int s = 1; s < g.splits; ++s) {
@@ -298,14 +300,20 @@ __global__ void __launch_bounds__(256)
     a1 += __builtin_nontemporal_load((const f32x4*)(p + 4));
   }
   float v[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-  store_row8<EPI, OUT_F32, HALF>(v, g, (int)row, (int)col);
+  if (ANY && col + 8 > g.N) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (col + e < g.N) store_one<EPI, OUT_F32, HALF>(v[e], g, (int)row, (int)col + e);
+    return;
+  }
+  store_row8<EPI, OUT_F32, HALF, ANY>(v, g, (int)row, (int)col);
 }
 
-template <bool HALF>
+template <bool HALF, bool ANY>
 int launch_reduce(const float* ws, const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
-  const int64_t lanes = (int64_t)g.M * (g.N / 8);
+  const int64_t lanes = (int64_t)g.M * ((g.N + 7) / 8);
   const dim3 grid((unsigned)((lanes + 255) / 256)), block(256);
-#define REDUCE(EPI, F32) hipLaunchKernelGGL((splitk_reduce_kernel<EPI, F32, HALF>), grid, block, 0, stream, ws, g)
+#define REDUCE(EPI, F32) hipLaunchKernelGGL((splitk_reduce_kernel<EPI, F32, HALF, ANY>), grid, block, 0, stream, ws, g)
   if (out_f32) {
     if (epilogue == AXN_EPI_BIAS) REDUCE(AXN_EPI_BIAS, true);
     else if (epilogue == AXN_EPI_BIAS_GELU) REDUCE(AXN_EPI_BIAS_GELU, true);
@@ -559,7 +567,6 @@ int launch_gemm_f16(GemmLayout layout, const GemmArgs& g, int epilogue, bool out
 SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
   SplitPlan plan = {1, EDGE_128x128};
   if (layout == GEMM_NT && stream_takes(M, Kc)) return plan;
-  if (N % 8 != 0) return plan;
   const bool whole = M % 128 == 0 && N % 128 == 0 && Kc % 64 == 0;
   auto count = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   const long long tiles[3] = {count(256, 256), count(256, 128), count(128, 128)};
@@ -589,7 +596,7 @@ int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool
                        const SplitPlan& plan, float* ws, hipStream_t stream) {
   GemmArgs g = in;
   g.C = ws;
-  g.ldc = g.N;
+  g.ldc = (g.N + 7) / 8 * 8;   // whole vectors a row
   g.beta = 0;
   g.bias = nullptr;
   g.Z = nullptr;
@@ -622,8 +629,11 @@ int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool
   if (rc) return rc;
   GemmArgs out = in;
   out.splits = plan.parts;
-  return half ? launch_reduce<true>(ws, out, epilogue, out_f32, stream)
-              : launch_reduce<false>(ws, out, epilogue, out_f32, stream);
+  if (out.N % 8 != 0 || out.ldc % 8 != 0)
+    return half ? launch_reduce<true, true>(ws, out, epilogue, out_f32, stream)
+                : launch_reduce<false, true>(ws, out, epilogue, out_f32, stream);
+  return half ? launch_reduce<true, false>(ws, out, epilogue, out_f32, stream)
+              : launch_reduce<false, false>(ws, out, epilogue, out_f32, stream);
 }
 
 }  // namespace axn

@@ -461,7 +461,8 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
     __device__ __forceinline__ void start(const uint16_t* base, const uint16_t* base2, bool kmajor,
                                           int rows, int kc, int64_t ld, int row0, int k0) {
       const int64_t first = kmajor ? row0 * ld + k0 : k0 * ld + row0;
-      const int64_t all = kmajor ? (int64_t)(rows - 1) * ld + kc : (int64_t)(kc - 1) * ld + (rows + 7) / 8 * 8;
+      // a row's last 8 elements are copied together: up to 7 of them are padding of the operand's rows
+      const int64_t all = kmajor ? (int64_t)(rows - 1) * ld + (kc + 7) / 8 * 8 : (int64_t)(kc - 1) * ld + (rows + 7) / 8 * 8;
       at[0] = (const char*)(base + first);
       at[1] = base2 != nullptr ? (const char*)(base2 + first) : at[0];
       left = (all - first) * 2;

@@ -66,6 +66,35 @@ def _ragged16(dtype, *dims):
     return dtype in _GEMM16 and any(d % 8 for d in dims)
 
 
+def _any_n(dtype, N, K):
+    """Output features that are no multiple of 8 over input features that are: only dY needs its
+    rows padded, nothing else is copied or cut (2048 x 50257 x 2048: 410 us of copies and fills
+    around the three products before, 64 us after)."""
+    return dtype in _GEMM16 and N % 8 != 0 and K % 8 == 0
+
+
+def _pad_rows(t):
+    """[M, N] -> [M, N rounded up to a multiple of 8], zeros behind the columns."""
+    t, ld = _rows(t)
+    M, N = t.shape
+    out = torch.empty((M, N + (-N) % 8), dtype=t.dtype, device=t.device)
+    nv.call("axn_pad_rows16", nv.ptr(t), nv.ptr(out), M, N, ld, nv.current_stream())
+    return out
+
+
+def _gemm_any_n(op, a, b, out, M, N, K, bias=None, z=None, epilogue=nv.EPI_NONE, accumulate=False):
+    """axn_gemm_any_n; a and b in the order of the product, dY from `_pad_rows`."""
+    a, lda = _prep_bf16(a)
+    b, ldb = _prep_bf16(b)
+    # the forward with an fp32 result has no split kernel for it elsewhere either
+    split = op != GEMM_FWD or out.dtype == a.dtype
+    ws, ws_bytes = _split_workspace(op, M, N, K, a.device) if split else (None, 0)
+    nv.call("axn_gemm_any_n", op, nv.ptr(a), nv.ptr(b), nv.ptr(bias), nv.ptr(out), nv.ptr(z),
+            nv.dtype_code(a.dtype), M, N, K, lda, ldb, N if op == GEMM_FWD else K, epilogue,
+            1 if accumulate else 0, nv.dtype_code(out.dtype), nv.ptr(ws), ws_bytes, nv.current_stream())
+    return out
+
+
 # ------------------------------------------------------------------ GEMMs ----
 # 16-bit operand types of the MFMA kernels -> suffix of their entry points
 _GEMM16 = {torch.bfloat16: "", torch.float16: "_f16"}
@@ -114,6 +143,10 @@ def gemm_fwd(x, w, bias=None, activation=None, save_z=False, out_f32=False):
         return y, (torch.empty_like(y) if want_z else None)
     if out_f32 and (bias is None or x.dtype not in _GEMM16):
         raise ValueError("out_f32 is the promotion of a 16-bit product by an fp32 bias")
+    if _any_n(x.dtype, N, K):
+        y = torch.empty((M, N), dtype=torch.float32 if out_f32 else x.dtype, device=x.device)
+        z = torch.empty((M, N), dtype=x.dtype, device=x.device) if want_z else None
+        return _gemm_any_n(GEMM_FWD, x, w, y, M, N, K, bias, z, epi), z
     if _ragged16(x.dtype, N, K):
         bp = None if bias is None else _pad8(bias.reshape(1, -1), 1).reshape(-1)
         y, z = gemm_fwd(_pad8(x, 1), _pad8(_pad8(w, 1), 0), bp, activation, save_z, out_f32)
@@ -159,6 +192,8 @@ def gemm_dgrad(dy, w):
         raise TypeError("the Linear kernels take bf16, fp16 or fp32 operands, got %s" % dy.dtype)
     if M == 0:
         return torch.empty((0, K), dtype=dy.dtype, device=dy.device)
+    if _any_n(dy.dtype, N, K):
+        return _dgrad_any_n(_pad_rows(dy), w, N)
     if _ragged16(dy.dtype, N, K):
         return gemm_dgrad(_pad8(dy, 1), _pad8(_pad8(w, 1), 0))[:, :K].contiguous()
     if dy.dtype in _GEMM16:
@@ -184,6 +219,31 @@ def gemm_dgrad(dy, w):
     return dx
 
 
+def _dgrad_any_n(dy8, w, N):
+    M, K = dy8.shape[0], w.shape[1]
+    if w.shape[0] != N:
+        raise ValueError("grad_output has %d features, weight is %s" % (N, tuple(w.shape)))
+    return _gemm_any_n(GEMM_DGRAD, dy8, w, torch.empty((M, K), dtype=w.dtype, device=w.device), M, N, K)
+
+
+def _wgrad_any_n(dy8, x, N, out, accumulate, out_dtype):
+    if out_dtype not in (dy8.dtype, torch.float32):
+        raise TypeError("dW must be %s or fp32, got %s" % (dy8.dtype, out_dtype))
+    M, K = x.shape
+    if dy8.shape[0] != M:
+        raise ValueError("grad_output has %d rows, input has %d" % (dy8.shape[0], M))
+    dest = out
+    if dest is None or dest.data_ptr() % 16:   # the kernel writes 16-byte vectors
+        dest = torch.empty((N, K), dtype=out_dtype, device=x.device)
+        if accumulate:
+            dest.copy_(out.view(N, K))
+    _gemm_any_n(GEMM_WGRAD, dy8, x, dest, M, N, K, accumulate=accumulate)
+    if out is None or dest is out:
+        return dest
+    out.view(N, K).copy_(dest)
+    return out
+
+
 def gemm_wgrad(dy, x, out=None, accumulate=False, out_dtype=None):
     """dW = dY^T X, optionally accumulated into `out` (dW += ...).  dy [M,N],
     x [M,K]; the result is [N,K] in `out_dtype` (bf16 or fp32 for bf16 operands)."""
@@ -205,6 +265,8 @@ def gemm_wgrad(dy, x, out=None, accumulate=False, out_dtype=None):
         if out is None:
             return torch.zeros((N, K), dtype=out_dtype, device=dy.device)
         return out if accumulate else out.zero_()
+    if _any_n(dy.dtype, N, K):
+        return _wgrad_any_n(_pad_rows(dy), x, N, out, accumulate, out_dtype)
     if _ragged16(dy.dtype, N, K):
         # the kernel accumulates into a padded copy of the gradient, which is cut back
         tmp = None
@@ -258,6 +320,13 @@ def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None):
                and not _ragged16(dy.dtype, N, K)
                and _workspace_bytes(GEMM_DGRAD, M, N, K) == 0
                and _workspace_bytes(GEMM_WGRAD, M, N, K) == 0)
+    if (_any_n(dy.dtype, N, K) and dy.dtype == w.dtype == x.dtype and M > 0 and tuple(x.shape) == (M, K)
+            and w.shape[0] == N and (out is None or (out.numel() == N * K and out.is_contiguous()))
+            and (out is not None or not accumulate)):
+        dy8 = _pad_rows(dy)   # once for both products
+        if out is not None:
+            out_dtype = out.dtype
+        return _dgrad_any_n(dy8, w, N), _wgrad_any_n(dy8, x, N, out, accumulate, out_dtype or dy.dtype)
     if not plain16:
         return gemm_dgrad(dy, w), gemm_wgrad(dy, x, out=out, accumulate=accumulate, out_dtype=out_dtype)
     if x.shape != (M, K) or w.shape[0] != N:

@@ -178,6 +178,22 @@ AXN_API int axn_gemm_wgrad_ws(const void* dY, const void* X, void* dW, int dtype
                       int beta, int dw_dtype, void* workspace, size_t workspace_bytes,
                       void* stream);
 
+/* The three products for any number N of output features (a head over a vocabulary of 50257):
+ * op an axn_gemm_op, A and B the operands in the order of the calls above, 16-bit of `dtype`.
+ *   FWD    Y[M,N]  rows of ldc >= N elements, any ldc; bias, Zsave (as Y), epilogue as axn_gemm_fwd;
+ *          out_dtype AXN_F32 as axn_gemm_fwd_f32out
+ *   DGRAD, WGRAD   dY rows of lda elements, a multiple of 8; what lies behind column N up to the next
+ *          multiple of 8 must be zero (axn_pad_rows16)
+ * K, the other leading dimensions and pointers: as above.  workspace: axn_gemm_workspace_bytes(op,
+ * M, N, K) bytes, or NULL for no split; beta and an fp32 out_dtype as axn_gemm_wgrad. */
+AXN_API int axn_gemm_any_n(int op, const void* A, const void* B, const float* bias, void* C,
+                   void* Zsave, int dtype, int64_t M, int64_t N, int64_t K, int64_t lda,
+                   int64_t ldb, int64_t ldc, int epilogue, int beta, int out_dtype,
+                   void* workspace, size_t workspace_bytes, void* stream);
+/* dst[M][n8] = src[M][N] of 16-bit elements (rows of ld elements, 2-byte aligned), n8 the next
+ * multiple of 8, zeros behind column N; dst 16-byte aligned. */
+AXN_API int axn_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, void* stream);
+
 /* Gate and up projection of a gated MLP with the activation in the epilogue:
  *   gate = X Wg^T,  up = X Wu^T,  H = silu(gate) * up     (one launch)
  * for `down_proj(act_fn(gate_proj(x)) * up_proj(x))` of the model the reference patches

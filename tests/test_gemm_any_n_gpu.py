@@ -1,0 +1,71 @@
+"""16-bit products with a number of output features that is no multiple of 8: every element against 64
+bits, and nothing written behind the outputs."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def close(got, want, dtype):
+    """One rounding to the result's type on top of fp32 sums (16-bit products are exact in fp32)."""
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -22}[dtype]
+    scale = want.abs().max()
+    return bool(((got.double() - want).abs() <= ulp * want.abs() + 1e-5 * scale).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 8), (3, 9, 72), (16, 1003, 512), (40, 4099, 1024),        # streamed forward
+    (129, 257, 64), (256, 511, 2048), (300, 1001, 4096),             # contractions in parts
+    (512, 20001, 768), (2048, 16391, 256),                           # full rounds and a rest
+])
+def test_products_against_64_bits(M, N, K, dtype):
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    X = torch.randn(M, K, generator=g, device="cuda").to(dtype)
+    W = (torch.randn(N, K, generator=g, device="cuda") * 0.1).to(dtype)
+    dY = torch.randn(M, N, generator=g, device="cuda").to(dtype)
+    b = torch.randn(N, generator=g, device="cuda")
+    X64, W64, dY64 = X.double(), W.double(), dY.double()
+    pre = X64 @ W64.t()
+    assert close(ops.gemm_fwd(X, W)[0], pre, dtype)
+    y, z = ops.gemm_fwd(X, W, bias=b, activation="gelu", save_z=True)
+    assert y.is_contiguous() and close(z, pre + b.double(), dtype)
+    assert close(y, torch.nn.functional.gelu(pre + b.double()), dtype)
+    assert close(ops.gemm_fwd(X, W, bias=b, out_f32=True)[0], pre + b.double(), torch.float32)
+    wide = torch.full((M, N + 5), float("nan"), dtype=dtype, device="cuda")
+    wide[:, 2:N + 2] = dY                                   # rows of an odd stride and offset
+    dx, dw = ops.gemm_bwd(wide[:, 2:N + 2], W, X)
+    assert close(dx, dY64 @ W64, dtype) and close(dw, dY64.t() @ X64, dtype)
+    assert torch.equal(dx, ops.gemm_dgrad(dY, W)) and torch.equal(dw, ops.gemm_wgrad(dY, X))
+    acc = torch.ones(N * K + 1, device="cuda")[1:]           # a flat buffer's view at an odd offset
+    ops.gemm_wgrad(dY, X, out=acc, accumulate=True)
+    assert close(acc.view(N, K), 1 + dY64.t() @ X64, torch.float32)
+    before = dw.double()                                     # rounded once already
+    ops.gemm_wgrad(dY, X, out=dw, accumulate=True)
+    assert close(dw, before + dY64.t() @ X64, dtype)
+
+
+def test_forward_leaves_the_neighbours_alone():
+    """Y at an odd row stride inside a larger buffer: the elements between its rows stay."""
+    from axonn_amd import _native as nv
+
+    M, N, K, ld = 300, 1003, 128, 1007
+    X, W = (torch.randn(n, K, device="cuda").bfloat16() for n in (M, N))
+    buf = torch.full((M * ld + 64,), 7.0, device="cuda").bfloat16()
+    nv.call("axn_gemm_any_n", 0, nv.ptr(X), nv.ptr(W), None, nv.ptr(buf), None, nv.BF16, M, N, K, K, K, ld,
+            nv.EPI_NONE, 0, nv.BF16, None, 0, nv.current_stream())
+    assert close(buf[:M * ld].view(M, ld)[:, :N], X.double() @ W.double().t(), torch.bfloat16)
+    assert bool((buf[:M * ld].view(M, ld)[:, N:] == 7).all()) and bool((buf[M * ld:] == 7).all())
+
+
+@pytest.mark.parametrize("M,N,ld", [(1, 1, 1), (3, 17, 17), (5, 24, 31), (70, 1003, 1005)])
+def test_pad_rows(M, N, ld):
+    from axonn_amd import ops
+
+    src = torch.randn(M, ld, device="cuda").half()[:, :N]
+    out = ops._pad_rows(src)
+    assert out.shape == (M, N + (-N) % 8)
+    assert torch.equal(out[:, :N], src) and not out[:, N:].any()

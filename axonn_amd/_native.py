@@ -20,6 +20,7 @@ AXN_ELIMIT = -5
 
 BF16, F16, F32 = 0, 1, 2
 EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_GELU = 0, 1, 2, 3
+BIAS_16BIT = 0x100   # with an epilogue: the bias has the operands' 16-bit type
 
 ABI_VERSION = 13
 

@@ -57,7 +57,7 @@ int check_gemm(const char* name, const void* a, const void* b, const void* c,
   return AXN_OK;
 }
 
-int check_epilogue(const char* name, int epilogue, const float* bias) {
+int check_epilogue(const char* name, int epilogue, const void* bias) {
   REQUIRE(epilogue >= AXN_EPI_NONE && epilogue <= AXN_EPI_GELU, AXN_EINVAL,
           "%s: unknown epilogue %d", name, epilogue);
   const bool needs_bias = epilogue == AXN_EPI_BIAS || epilogue == AXN_EPI_BIAS_GELU;
@@ -337,7 +337,7 @@ static int gemm_ws(const char* name, int op, const void* a, const void* b, void*
               : launch_gemm_bf16(layout, g, epilogue, out_dtype == AXN_F32, (hipStream_t)stream);
 }
 
-int axn_gemm_any_n(int op, const void* A, const void* B, const float* bias, void* C, void* Zsave,
+int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void* C, void* Zsave,
                    int dtype, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                    int64_t ldc, int epilogue, int beta, int out_dtype, void* workspace,
                    size_t workspace_bytes, void* stream) {
@@ -351,6 +351,8 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const float* bias, void
   int rc = check_gemm(name, A, B, C, M, n8, K, lda, ldb, fwd ? n8 : ldc, fwd ? K : n8, K, fwd ? n8 : K);
   if (rc) return rc;
   REQUIRE(!fwd || ldc >= N, AXN_EINVAL, "%s: leading dimension smaller than the row length", name);
+  const bool bias16 = (epilogue & AXN_BIAS_16BIT) != 0;
+  epilogue &= ~(int)AXN_BIAS_16BIT;
   rc = check_epilogue(name, epilogue, bias);
   if (rc) return rc;
   REQUIRE(fwd || epilogue == AXN_EPI_NONE, AXN_EINVAL, "%s: only the forward has an epilogue", name);
@@ -362,6 +364,7 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const float* bias, void
   fill_gemm_args(g, op, A, B, C, M, N, K, lda, ldb, ldc);
   g.beta = beta;
   g.bias = bias;
+  g.bias16 = bias16 ? 1 : 0;
   g.Z = (uint16_t*)Zsave;
   const bool half = dtype == AXN_F16, out_f32 = out_dtype == AXN_F32;
   const GemmLayout layout = kLayoutOfOp[op];

@@ -85,7 +85,8 @@ struct GemmArgs {
   const uint16_t* A;
   const uint16_t* B;
   void* C;            // bf16 or fp32, row-major [M][N]
-  const float* bias;  // [N] or null
+  const void* bias;   // [N] or null: fp32, or the operands' type if bias16
+  int bias16;
   uint16_t* Z;        // optional pre-activation copy, bf16 [M][N], ld = ldc
   int M, N, Kc;
   int64_t lda, ldb, ldc;
@@ -109,6 +110,11 @@ struct GemmArgs {
   const uint16_t* A2;
   int k_first;
 };
+
+// Address of the bias of output column n.
+inline const void* bias_at(const GemmArgs& g, int64_t n) {
+  return g.bias == nullptr ? nullptr : (const char*)g.bias + n * (g.bias16 ? 2 : 4);
+}
 
 enum GemmLayout { GEMM_NT = 0, GEMM_NN = 1, GEMM_TN = 2 };
 // GEMM_NT: A K-major, B K-major   (forward  Y  = X  W^T)

@@ -75,7 +75,7 @@ int launch_edge_kind(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
       g2.B = BKM ? g.B + n1 * g.ldb : g.B + n1;
       if (g.B2 != nullptr) g2.B2 = BKM ? g.B2 + n1 * g.ldb : g.B2 + n1;
       g2.C = (char*)g.C + n1 * esz;
-      if (g.bias != nullptr) g2.bias = g.bias + n1;
+      g2.bias = bias_at(g, n1);
       if (g.Z != nullptr) g2.Z = g.Z + n1;
     } else {  // whole tile rows
       const int64_t m1 = full / tn * 256;

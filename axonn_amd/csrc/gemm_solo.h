@@ -80,12 +80,18 @@ __device__ __forceinline__ void store_row8(float (&v)[8], const GemmArgs& g, int
   using f32x4_mem = typename Unaligned<f32x4, ANY ? 4 : 16>::type;
   const int64_t o = (int64_t)row * g.ldc + col;
   if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU) {
-    const f32x4 b0 = *(const f32x4*)(g.bias + col);
-    const f32x4 b1 = *(const f32x4*)(g.bias + col + 4);
+    if (g.bias16) {   // widened here: a launch before the product that widens it costs more than the product of a small layer
+      const lpx8 b = *(const lpx8*)((const uint16_t*)g.bias + col);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[e] += b0[e];
-      v[4 + e] += b1[e];
+      for (int e = 0; e < 8; ++e) v[e] += (float)b[e];
+    } else {
+      const f32x4 b0 = *(const f32x4*)((const float*)g.bias + col);
+      const f32x4 b1 = *(const f32x4*)((const float*)g.bias + col + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] += b0[e];
+        v[4 + e] += b1[e];
+      }
     }
   }
   if (EPI == AXN_EPI_BIAS_GELU || EPI == AXN_EPI_GELU) {
@@ -126,7 +132,8 @@ template <int EPI, bool OUT_F32, bool HALF>
 __device__ __forceinline__ void store_one(float x, const GemmArgs& g, int row, int col) {
   using lp = std::conditional_t<HALF, _Float16, __bf16>;
   const int64_t o = (int64_t)row * g.ldc + col;
-  if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU) x += g.bias[col];
+  if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU)
+    x += g.bias16 ? (float)((const lp*)g.bias)[col] : ((const float*)g.bias)[col];
   if (EPI == AXN_EPI_BIAS_GELU || EPI == AXN_EPI_GELU) {
     if (g.Z != nullptr) *((lp*)g.Z + o) = (lp)x;
     x = gelu_exact(x);

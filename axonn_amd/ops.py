@@ -132,9 +132,13 @@ def gemm_fwd(x, w, bias=None, activation=None, save_z=False, out_f32=False):
     if w.shape[1] != K:
         raise ValueError("weight is %s, input has %d features" % (tuple(w.shape), K))
     if bias is not None:
-        bias = bias.float().contiguous()
         if bias.numel() != N:
             raise ValueError("bias has %d elements, expected %d" % (bias.numel(), N))
+        # the 16-bit kernels read a bias of their operands' type as it is
+        if bias.dtype == x.dtype and x.dtype in _GEMM16 and bias.is_contiguous() and bias.data_ptr() % 16 == 0:
+            epi |= nv.BIAS_16BIT
+        else:
+            bias = bias.float().contiguous()
     want_z = activation is not None and save_z
     if x.dtype not in _GEMM16 and x.dtype != torch.float32:
         raise TypeError("the Linear kernels take bf16, fp16 or fp32 operands, got %s" % x.dtype)
@@ -143,33 +147,15 @@ def gemm_fwd(x, w, bias=None, activation=None, save_z=False, out_f32=False):
         return y, (torch.empty_like(y) if want_z else None)
     if out_f32 and (bias is None or x.dtype not in _GEMM16):
         raise ValueError("out_f32 is the promotion of a 16-bit product by an fp32 bias")
-    if _any_n(x.dtype, N, K):
+    if x.dtype in _GEMM16 and K % 8 == 0:
         y = torch.empty((M, N), dtype=torch.float32 if out_f32 else x.dtype, device=x.device)
         z = torch.empty((M, N), dtype=x.dtype, device=x.device) if want_z else None
         return _gemm_any_n(GEMM_FWD, x, w, y, M, N, K, bias, z, epi), z
-    if _ragged16(x.dtype, N, K):
+    if x.dtype in _GEMM16:
         bp = None if bias is None else _pad8(bias.reshape(1, -1), 1).reshape(-1)
         y, z = gemm_fwd(_pad8(x, 1), _pad8(_pad8(w, 1), 0), bp, activation, save_z, out_f32)
         return y[:, :N].contiguous(), (None if z is None else z[:, :N].contiguous())
-    if x.dtype in _GEMM16:
-        x, ldx = _prep_bf16(x)
-        w, ldw = _prep_bf16(w)
-        z = torch.empty((M, N), dtype=x.dtype, device=x.device) if want_z else None
-        if out_f32:
-            y = torch.empty((M, N), dtype=torch.float32, device=x.device)
-            nv.call("axn_gemm_fwd_f32out", nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(y), nv.ptr(z),
-                    nv.dtype_code(x.dtype), M, N, K, ldx, ldw, N, epi, nv.current_stream())
-            return y, z
-        y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-        ws, ws_bytes = _split_workspace(GEMM_FWD, M, N, K, x.device)
-        if ws is not None:
-            nv.call("axn_gemm_fwd_ws", nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(y), nv.ptr(z),
-                    nv.dtype_code(x.dtype), M, N, K, ldx, ldw, N, epi, nv.ptr(ws), ws_bytes,
-                    nv.current_stream())
-            return y, z
-        nv.call("axn_gemm_fwd" + _GEMM16[x.dtype], nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(y), nv.ptr(z),
-                M, N, K, ldx, ldw, N, epi, nv.current_stream())
-    elif x.dtype == torch.float32:
+    if x.dtype == torch.float32:
         x, w = x.contiguous(), w.contiguous()
         y = torch.empty((M, N), dtype=torch.float32, device=x.device)
         z = torch.empty_like(y) if want_z else None

@@ -181,12 +181,13 @@ AXN_API int axn_gemm_wgrad_ws(const void* dY, const void* X, void* dW, int dtype
 /* The three products for any number N of output features (a head over a vocabulary of 50257):
  * op an axn_gemm_op, A and B the operands in the order of the calls above, 16-bit of `dtype`.
  *   FWD    Y[M,N]  rows of ldc >= N elements, any ldc; bias, Zsave (as Y), epilogue as axn_gemm_fwd;
- *          out_dtype AXN_F32 as axn_gemm_fwd_f32out
+ *          out_dtype AXN_F32 as axn_gemm_fwd_f32out; epilogue | AXN_BIAS_16BIT: a 16-bit bias
  *   DGRAD, WGRAD   dY rows of lda elements, a multiple of 8; what lies behind column N up to the next
  *          multiple of 8 must be zero (axn_pad_rows16)
  * K, the other leading dimensions and pointers: as above.  workspace: axn_gemm_workspace_bytes(op,
  * M, N, K) bytes, or NULL for no split; beta and an fp32 out_dtype as axn_gemm_wgrad. */
-AXN_API int axn_gemm_any_n(int op, const void* A, const void* B, const float* bias, void* C,
+#define AXN_BIAS_16BIT 0x100 /* with the epilogue: bias is of `dtype` instead of fp32 */
+AXN_API int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void* C,
                    void* Zsave, int dtype, int64_t M, int64_t N, int64_t K, int64_t lda,
                    int64_t ldb, int64_t ldc, int epilogue, int beta, int out_dtype,
                    void* workspace, size_t workspace_bytes, void* stream);

@@ -69,3 +69,23 @@ def test_pad_rows(M, N, ld):
     out = ops._pad_rows(src)
     assert out.shape == (M, N + (-N) % 8)
     assert torch.equal(out[:, :N], src) and not out[:, N:].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(5, 1003, 64), (40, 72, 512), (256, 512, 256), (130, 264, 4096),
+                                   (129, 1001, 64), (2304, 4096, 128)])
+def test_bias_of_the_operands_type_equals_its_fp32_copy(M, N, K, dtype):
+    """Streamed, whole, ragged and split products; a bias at an odd offset is widened beforehand."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(N)
+    X, W = (torch.randn(n, K, generator=g, device="cuda").to(dtype) for n in (M, N))
+    b = torch.randn(N + 1, generator=g, device="cuda").to(dtype)
+    for bias in (b[:N], b[1:]):
+        for act in (None, "gelu"):
+            got = ops.gemm_fwd(X, W, bias=bias, activation=act, save_z=True)
+            want = ops.gemm_fwd(X, W, bias=bias.float(), activation=act, save_z=True)
+            assert torch.equal(got[0], want[0])
+            assert act is None or torch.equal(got[1], want[1])
+    pre = X.double() @ W.double().t() + b[:N].double()
+    assert close(ops.gemm_fwd(X, W, bias=b[:N])[0], pre, dtype)

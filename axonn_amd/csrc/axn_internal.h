@@ -147,6 +147,9 @@ struct SplitPlan {
 SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc);
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, int epilogue, bool half, bool out_f32,
                        const SplitPlan& plan, float* ws, hipStream_t stream);
+// Row strides from kEdgeMaxLd on, both operands addressed with 64 bits (gemm_far.hip).
+int launch_gemm_far(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32, bool half,
+                    hipStream_t stream);
 int launch_gemm_edge_bf16(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32,
                           EdgeTile tile, hipStream_t stream);
 int launch_gemm_edge_f16(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32,

@@ -173,10 +173,7 @@ EdgeTile edge_tile(long long M, long long N, long long Kc, double* us = nullptr)
 int launch_edge(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, bool half,
                 hipStream_t stream) {
   const int64_t ld = g.lda > g.ldb ? g.lda : g.ldb;
-  if (ld >= kEdgeMaxLd) {
-    set_error("gemm: row strides must stay below %lld elements", (long long)kEdgeMaxLd);
-    return AXN_ELIMIT;
-  }
+  if (ld >= kEdgeMaxLd) return launch_gemm_far(layout, g, epilogue, out_f32, half, stream);
   const EdgeTile tile = ld >= kEdgeMaxLd / 2 ? EDGE_128x128 : edge_tile(g.M, g.N, g.Kc);
   return half ? launch_gemm_edge_f16(layout, g, epilogue, out_f32, tile, stream)
               : launch_gemm_edge_bf16(layout, g, epilogue, out_f32, tile, stream);

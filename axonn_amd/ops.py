@@ -43,9 +43,14 @@ def _bf16_ok(t, ld):
     return t.data_ptr() % 16 == 0 and ld % 8 == 0
 
 
+# Rows further apart than this are packed first (the last token of every sequence of a long prompt,
+# `hidden[:, -1, :]`): the fast kernels' offsets are 32 bits wide.
+_FAR_ROWS = 1 << 22
+
+
 def _prep_bf16(t):
     t, ld = _rows(t)
-    if not _bf16_ok(t, ld):
+    if not _bf16_ok(t, ld) or (ld >= _FAR_ROWS and ld > t.shape[1]):
         t = t.contiguous().clone()
         ld = t.shape[1]
     return t, ld

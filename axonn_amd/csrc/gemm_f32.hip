@@ -140,6 +140,32 @@ __device__ __forceinline__ void direct_tile(f32x4 (&acc)[FM][FN], const float* _
     blocks(std::true_type{}, k0, std::integral_constant<int, 1>{});
 }
 
+// Whether the lane's operands hold a non-zero number under 2^-62 (a product of two that are larger is
+// a normal number).
+template <bool AK, bool BKM, int FM, int FN, bool VEC>
+__device__ __forceinline__ bool tiny_operands(const float* __restrict__ A, const float* __restrict__ B, int arow,
+                                              int bcol, int M, int N, int Kc, int k_begin, int k_end) {
+  const int q = (threadIdx.x & 63) >> 4;
+  bool tiny = false;
+  auto chunk = [&](auto guard_, int k0) {
+    constexpr bool GUARD = decltype(guard_)::value;
+    float a[FM][4], b[FN][4];
+    load_block<AK, FM, VEC, GUARD>(a, A, arow, M, k0 + 4 * q, Kc, k_end);
+    load_block<BKM, FN, VEC, GUARD>(b, B, bcol, N, k0 + 4 * q, Kc, k_end);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) tiny |= a[i][s] != 0.f && fabsf(a[i][s]) < 0x1p-62f;
+#pragma unroll
+      for (int j = 0; j < FN; ++j) tiny |= b[j][s] != 0.f && fabsf(b[j][s]) < 0x1p-62f;
+    }
+  };
+  const int whole = k_begin + (k_end - k_begin) / 16 * 16;
+  for (int k0 = k_begin; k0 < whole; k0 += 16) chunk(std::false_type{}, k0);
+  if (whole < k_end) chunk(std::true_type{}, whole);
+  return tiny;
+}
+
 // Stores a wave's 16 FM x 16 FN results at (m0, n0): register v of acc[i][j] in lane (r, q) is
 // output row m0 + FM (4 q + v) + i, column n0 + FN r + j.
 template <int EPI, int FM, int FN, bool VEC>
@@ -258,7 +284,11 @@ __global__ void __launch_bounds__(64 * WAVES)
 // The three parts carry a float's precision where the third is not below bf16's range, and an infinity
 // has no remainder.  So a wave whose results hold a NaN, an infinity or a non-zero magnitude under
 // 2^-64 computes its tile again with native products (direct_tile): operands of 2^-100 cannot reach a
-// result above that bound unnoticed unless their counterparts are above 2^36.
+// result above that bound unnoticed unless their counterparts are above 2^36.  The bf16 instruction takes
+// subnormal operands as zero, so a wave with a result of exactly zero looks through its operands for
+// tiny ones first; those of zero rows (padding) have none and keep their zeros
+// (2048 x 4096 x 1024 in a row of launches: 106 us, with half of the rows zero 142, with a zero row in every wave
+// 198; four chunks of the look in flight made no difference).
 //
 // Four waves (2 x 2) own a 32 FM x 32 FN tile.  Each thread loads its share of a 32-deep stage into
 // registers one stage ahead, splits it and writes three bf16 planes to LDS ([row][32], 64 bytes a row);
@@ -267,8 +297,7 @@ __global__ void __launch_bounds__(64 * WAVES)
 // rows of a contraction-strided operand writes to F places a bank apart from its neighbours', and a
 // lane's fragments are F consecutive rows (columns), as direct_tile and store_tile have them.  A row's
 // 16-byte pieces are permuted by part_of(rho) so that any 16 lanes of a fragment read hit 16 different
-// 16-byte bank groups.  LDS is single-buffered: two or three workgroups share a CU and fill each other's
-// barriers (their splitting and one's matrix instructions overlap).
+// 16-byte bank groups.
 // LDS is single-buffered (48 KB for 128 x 128) so that two workgroups share a CU and fill each other's
 // barriers.  2048 x 4096, contraction 1024: 86 us, 200 TFLOP/s of fp32 products (native 201 us); what
 // bounds it is the chain of stores, barrier, fragment reads and matrix instructions of a stage, not one
@@ -400,7 +429,7 @@ __global__ void __launch_bounds__(256, 2)
 
   const int wave = threadIdx.x >> 6, r = threadIdx.x & 15;
   const int mw = m0 + 16 * FM * (wave >> 1), nw = n0 + 16 * FN * (wave & 1);
-  bool odd = false;
+  bool odd = false, zero = false;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -410,8 +439,11 @@ __global__ void __launch_bounds__(256, 2)
       for (int v = 0; v < 4; ++v) {
         const float c = fabsf(acc[i][j][v]);
         odd |= !(c == 0.f || (c >= 0x1p-64f && c <= 0x1.fffffep127f));
+        zero |= c == 0.f;
       }
     }
+  if (!__builtin_amdgcn_ballot_w64(odd) && __builtin_amdgcn_ballot_w64(zero))
+    odd = tiny_operands<AK, BKM, FM, FN, VEC>(A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end);
   if (__builtin_amdgcn_ballot_w64(odd)) {
     clear(acc);
     direct_tile<AK, BKM, FM, FN, 1, VEC>(acc, A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end, 0, 1);

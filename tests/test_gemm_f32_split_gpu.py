@@ -79,3 +79,23 @@ def test_magnitudes_beyond_the_parts_keep_full_precision(exponent):
     want = X.double() @ W.double().t()
     got = ops.gemm_fwd(X * 2.0 ** exponent, W)[0]
     assert err(got.double() * 2.0 ** -exponent, want) < 1e-6
+
+
+@pytest.mark.parametrize("M,N,K", [(2050, 2049, 1030), (2052, 2052, 1032)])
+@pytest.mark.parametrize("exponent", [-132, -140, -145])
+def test_subnormal_operands_are_not_taken_as_zero(M, N, K, exponent):
+    """The bf16 instruction flushes them. Whole multiples of 2^exponent, sums below 2^(exponent + 20):
+    every one is a multiple of 2^-149, so the exact results are floats."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    X = torch.randint(-2, 3, (M, K), generator=g, device="cuda").float()
+    W = torch.randint(-2, 3, (N, K), generator=g, device="cuda").float()
+    X[7], W[:, 9] = 0, 0
+    tiny = (X.double() * 2.0 ** exponent).float()
+    got = ops.gemm_fwd(tiny, W)[0]
+    assert torch.equal(got.double() * 2.0 ** -exponent, X.double() @ W.double().t())
+    mixed = X.clone()
+    mixed[:, 1:] = 0              # one subnormal column among zeros, split over parts
+    mixed[:, 0] = tiny[:, 0]
+    assert torch.equal(ops.gemm_fwd(mixed, W)[0].double(), mixed.double() @ W.double().t())

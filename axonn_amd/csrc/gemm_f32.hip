@@ -140,11 +140,10 @@ __device__ __forceinline__ void direct_tile(f32x4 (&acc)[FM][FN], const float* _
     blocks(std::true_type{}, k0, std::integral_constant<int, 1>{});
 }
 
-// Whether the lane's operands hold a non-zero number under 2^-62 (a product of two that are larger is
-// a normal number).
+// Whether the lane's operands hold a non-zero number under `bound`.
 template <bool AK, bool BKM, int FM, int FN, bool VEC>
 __device__ __forceinline__ bool tiny_operands(const float* __restrict__ A, const float* __restrict__ B, int arow,
-                                              int bcol, int M, int N, int Kc, int k_begin, int k_end) {
+                                              int bcol, int M, int N, int Kc, int k_begin, int k_end, float bound) {
   const int q = (threadIdx.x & 63) >> 4;
   bool tiny = false;
   auto chunk = [&](auto guard_, int k0) {
@@ -155,9 +154,9 @@ __device__ __forceinline__ bool tiny_operands(const float* __restrict__ A, const
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i) tiny |= a[i][s] != 0.f && fabsf(a[i][s]) < 0x1p-62f;
+      for (int i = 0; i < FM; ++i) tiny |= a[i][s] != 0.f && fabsf(a[i][s]) < bound;
 #pragma unroll
-      for (int j = 0; j < FN; ++j) tiny |= b[j][s] != 0.f && fabsf(b[j][s]) < 0x1p-62f;
+      for (int j = 0; j < FN; ++j) tiny |= b[j][s] != 0.f && fabsf(b[j][s]) < bound;
     }
   };
   const int whole = k_begin + (k_end - k_begin) / 16 * 16;
@@ -281,14 +280,23 @@ __global__ void __launch_bounds__(64 * WAVES)
 // per 4).  Error against 64 bits, normal operands, native / this: contraction of 128 2.0e-7 / 6.6e-8,
 // 1024 5.7e-7 / 1.9e-7, 4096 (native by four waves) 5.7e-7 / 4.0e-7; in one accumulator 4096 has 1.0e-6.
 //
-// The three parts carry a float's precision where the third is not below bf16's range, and an infinity
-// has no remainder.  So a wave whose results hold a NaN, an infinity or a non-zero magnitude under
-// 2^-64 computes its tile again with native products (direct_tile): operands of 2^-100 cannot reach a
-// result above that bound unnoticed unless their counterparts are above 2^36.  The bf16 instruction takes
-// subnormal operands as zero, so a wave with a result of exactly zero looks through its operands for
-// tiny ones first; those of zero rows (padding) have none and keep their zeros
-// (2048 x 4096 x 1024 in a row of launches: 106 us, with half of the rows zero 142, with a zero row in every wave
-// 198; four chunks of the look in flight made no difference).
+// A result that is one product (a row with one non-zero element) misses the three dropped products: at
+// most 1.7 x 2^-24 off, the native one 1.0 x 2^-24; with two more of the three it is 1.0 again and the kernel
+// 16 to 22 % slower (2048 x 1024, contraction 4096: 97 us, 111), which sums, nearer to exact as they are, do
+// not pay for.
+//
+// What three bf16 numbers cannot carry, and where the native products (direct_tile) take over, wave by wave:
+//   * an infinity has no remainder, the largest floats round to one, and partial products far below the
+//     result lose bits: a wave whose results hold a NaN, an infinity or a non-zero magnitude under 2^-64;
+//   * the conversion rounds to multiples of 2^-133 (the matrix instruction itself keeps subnormals), so a
+//     number under 2^-110 is off by up to 2^-134.  Times less than 2^16 that is nothing to a result of 2^-64
+//     and more.  A workgroup that staged a larger number has its waves look through their operands for
+//     numbers under 2^-110;
+//   * a result of exactly zero may be one that was lost: those waves look for numbers under 2^-62 (a product
+//     of two that are larger is a normal number).  Zero rows (padding) have none and keep their zeros.
+// A look costs what reading the operands once more costs (2048 x 4096 x 1024 in a row of launches: 106 us, with
+// half of the rows zero 142, with a zero row in every wave 198; four chunks of the look in flight made no
+// difference); the largest magnitude, kept while staging, half an instruction an element.
 //
 // Four waves (2 x 2) own a 32 FM x 32 FN tile.  Each thread loads its share of a 32-deep stage into
 // registers one stage ahead, splits it and writes three bf16 planes to LDS ([row][32], 64 bytes a row);
@@ -354,6 +362,16 @@ __device__ __forceinline__ void put_stage(Planes<F>& lds, const float (&x)[F][4]
   }
 }
 
+// The larger of m and the magnitudes (fmaxf would quiet NaNs first, an instruction each).
+template <int F>
+__device__ __forceinline__ float max_magnitude(float m, const float (&x)[F][4]) {
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int s = 0; s < 4; s += 2) asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(x[i][s]), "v"(x[i][s + 1]));
+  return m;
+}
+
 // The parts of the five smaller products, least first.
 constexpr int kPartA[5] = {2, 0, 1, 1, 0}, kPartB[5] = {0, 2, 1, 0, 1};
 
@@ -393,6 +411,7 @@ __global__ void __launch_bounds__(256, 2)
                           int M, int N, int Kc, int tiles_m, int tiles_n, int k_part, int beta) {
   __shared__ Planes<FM> la;
   __shared__ Planes<FN> lb;
+  __shared__ int large;   // an operand of 2^16 and more was staged
   const int tiles = tiles_m * tiles_n;
   const int part = blockIdx.x / tiles, id = blockIdx.x - part * tiles;
   const int tm = id / tiles_n, tn = id - tm * tiles_n;
@@ -417,15 +436,20 @@ __global__ void __launch_bounds__(256, 2)
       load_block<BKM, FN, VEC, true>(xb, B, n0 + FN * gb, N, k0 + 4 * qb, Kc, k_end);
     }
   };
+  float largest = 0.f;
+  if (threadIdx.x == 0) large = 0;
   fetch(k_begin);
   for (int k0 = k_begin; k0 < k_end; k0 += 32) {
     put_stage<AK, FM>(la, xa);
     put_stage<BKM, FN>(lb, xb);
+    largest = max_magnitude(max_magnitude(largest, xa), xb);
     __syncthreads();
     if (k0 + 32 < k_end) fetch(k0 + 32);
     split_stage<FM, FN>(acc, low, la, lb);
     __syncthreads();
   }
+  if (largest >= 0x1p16f) large = 1;
+  __syncthreads();
 
   const int wave = threadIdx.x >> 6, r = threadIdx.x & 15;
   const int mw = m0 + 16 * FM * (wave >> 1), nw = n0 + 16 * FN * (wave & 1);
@@ -442,8 +466,10 @@ __global__ void __launch_bounds__(256, 2)
         zero |= c == 0.f;
       }
     }
-  if (!__builtin_amdgcn_ballot_w64(odd) && __builtin_amdgcn_ballot_w64(zero))
-    odd = tiny_operands<AK, BKM, FM, FN, VEC>(A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end);
+  const bool zeros = __builtin_amdgcn_ballot_w64(zero) != 0;
+  if (!__builtin_amdgcn_ballot_w64(odd) && (zeros || large))
+    odd = tiny_operands<AK, BKM, FM, FN, VEC>(A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end,
+                                              zeros ? 0x1p-62f : 0x1p-110f);
   if (__builtin_amdgcn_ballot_w64(odd)) {
     clear(acc);
     direct_tile<AK, BKM, FM, FN, 1, VEC>(acc, A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end, 0, 1);

@@ -99,3 +99,69 @@ def test_subnormal_operands_are_not_taken_as_zero(M, N, K, exponent):
     mixed[:, 1:] = 0              # one subnormal column among zeros, split over parts
     mixed[:, 0] = tiny[:, 0]
     assert torch.equal(ops.gemm_fwd(mixed, W)[0].double(), mixed.double() @ W.double().t())
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 2048, 1024), (2050, 2049, 1030), (260, 4100, 4100)])
+@pytest.mark.parametrize("small,large", [(-118, 60), (-122, 70), (-130, 100), (-145, 120)])
+def test_small_operands_times_large_ones_keep_full_precision(M, N, K, small, large):
+    """Numbers around 2^small times ones around 2^large, in one operand or the other: results of ordinary
+    magnitude, of numbers whose last bits lie below bf16's multiples of 2^-133."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(6)
+    X, W, dY = (torch.randn(s, generator=g, device="cuda").double() for s in ((M, K), (N, K), (M, N)))
+    low = lambda t: (t * 2.0 ** small).float()   # noqa: E731
+    high = lambda t: (t * 2.0 ** large).float()   # noqa: E731
+    for got, a, b in ((ops.gemm_fwd(low(X), high(W))[0], low(X), high(W).t()),
+                      (ops.gemm_fwd(high(X), low(W))[0], high(X), low(W).t()),
+                      (ops.gemm_dgrad(high(dY), low(W)), high(dY), low(W)),
+                      (ops.gemm_wgrad(low(dY), high(X)), low(dY).t(), high(X))):
+        assert err(got, a.double() @ b.double()) < bound(max(M, N, K))
+
+
+def test_a_small_operand_beside_ordinary_ones():
+    """One term of a sum is a subnormal times a large number, the others are ordinary: the result is neither
+    small nor zero, and without the one term it is 1."""
+    from axonn_amd import ops
+
+    X, W = torch.zeros(2048, 1024, device="cuda"), torch.zeros(2048, 1024, device="cuda")
+    X[:, 0], W[:, 0] = 1, 1
+    X[:, 9], W[:, 9] = 2.0 ** -140, 2.0 ** 120
+    W[1000:, 9] = 2.0 ** 126
+    want = X.double() @ W.double().t()
+    assert torch.equal(ops.gemm_fwd(X, W)[0], want.float())
+    assert torch.equal(ops.gemm_fwd(W, X)[0], want.t().float())
+
+
+def test_large_operands_beside_ordinary_ones():
+    """Numbers of 2^16 and more, nothing small: whole multiples, exact either way."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    X, W = (torch.randint(-7, 8, (2050, 1030), generator=g, device="cuda").float() for _ in range(2))
+    X *= 2.0 ** 17
+    assert torch.equal(ops.gemm_fwd(X, W)[0].double(), X.double() @ W.double().t())
+
+
+def test_products_of_two_small_operands():
+    """2^-70 times 2^-70: whole multiples of 2^-140, exact in subnormal floats."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(7)
+    X, W = (torch.randint(-2, 3, s, generator=g, device="cuda").float() for s in ((2050, 1030), (2049, 1030)))
+    got = ops.gemm_fwd(X * 2.0 ** -70, W * 2.0 ** -70)[0]
+    assert torch.equal(got.double() * 2.0 ** 140, X.double() @ W.double().t())
+
+
+def test_a_result_of_one_product():
+    """Rows with one non-zero element: the dropped products are under 2^-24 of the product, the sum of the two
+    accumulators rounds once."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(8)
+    X, W = torch.zeros(2048, 1024, device="cuda"), torch.randn(2048, 1024, generator=g, device="cuda")
+    X[torch.arange(2048), torch.randint(0, 1024, (2048,), generator=g, device="cuda").cpu()] = \
+        torch.randn(2048, generator=g, device="cuda")
+    want = X.double() @ W.double().t()
+    got = ops.gemm_fwd(X, W)[0]
+    assert bool(((got.double() - want).abs() <= 2.0 * 2.0 ** -24 * want.abs()).all())

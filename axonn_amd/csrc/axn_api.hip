@@ -620,7 +620,7 @@ size_t axn_gemm_f32_workspace_bytes(int op, int64_t M, int64_t N, int64_t K) {
     return 0;
   GemmArgs g = {};
   fill_gemm_args(g, op, nullptr, nullptr, nullptr, M, N, K, 0, 0, 0);
-  return gemm_f32_workspace_bytes(g.M, g.N, g.Kc);
+  return gemm_f32_workspace_bytes(kLayoutOfOp[op], g.M, g.N, g.Kc);
 }
 
 int axn_gemm_fwd_f32_ws(const float* X, const float* W, const float* bias, float* Y,

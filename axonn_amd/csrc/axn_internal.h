@@ -183,7 +183,7 @@ int launch_gemm_f32(GemmLayout layout, const float* A, const float* B, float* C,
                     const float* bias, float* Z, int M, int N, int Kc,
                     int epilogue, int beta, float* ws, size_t ws_bytes, hipStream_t stream);
 // Workspace for a contraction in parts (0: it would not be split); ws == nullptr: no split.
-size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t Kc);
+size_t gemm_f32_workspace_bytes(GemmLayout layout, int64_t M, int64_t N, int64_t Kc);
 
 // ---- elementwise backward of the bias/GELU epilogue ----------------------
 size_t dgelu_dbias_workspace_bytes(int64_t M, int64_t N);

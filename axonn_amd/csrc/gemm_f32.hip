@@ -523,36 +523,67 @@ __global__ void __launch_bounds__(256)
   *(vec*)(C + o) = x;
 }
 
-// Problems of 2^32 multiply-adds and more are split into bf16 products, with the contraction in as many
-// parts as the estimate below finds fastest (0: not split into products at all).  The line is drawn by
-// results, not by speed (512 x 4096 x 1024 is 61 us natively and 41 split, 64 x 4096 x 1024 18 and 16):
-// Adam divides a gradient by its own magnitude, so where one is next to zero the last bits of a product
-// become 1e-2 of the learning rate (batch 64 through a 1024 - 4096 - 1024 perceptron: one weight moves by
-// 6e-4 of the weights' rms in a step, which is the native kernel's rounding, not the split one's).  Small
-// full-precision networks, where launches and the host bound a step, keep the bits they have; above the
-// line the products bound it and the split ones, 2.4 times as fast and nearer to exact, are taken.
+// Problems of 2^32 multiply-adds and more may be split into bf16 products, with the contraction in as many
+// parts as the estimate below finds fastest.  Smaller ones keep the native kernel and its bits, although by
+// speed the line could lie lower (512 x 4096 x 1024 is 61 us natively and 41 split, 64 x 4096 x 1024 18 and
+// 16): Adam divides a gradient by its own magnitude, so where one is next to zero the last bits of a product
+// become 1e-2 of the learning rate, and small full-precision networks, whose steps the launches and the host
+// bound, would take other steps than before for little.  (One step of a 1024 - 4096 - 1024 perceptron against
+// 64 bits, largest difference of a weight over the weights' rms: batch 64 native 7e-4; batch 1024, which is
+// above the line, native 3.2e-4, split 0.9e-4.)
 constexpr double kSplitWork = 4294967296.0;
+
+// Output tiles of the native kernel: the largest of 64 x 64, 32 x 32 and 16 x 16 (a loaded element is used
+// 4, 2, 1 times) that still gives the chip's 1024 SIMDs a wave each; smaller tiles keep more loads in flight
+// per wave.
+struct NativeTiles {
+  int size;
+  long long count;
+};
+NativeTiles native_tiles(int64_t M, int64_t N) {
+  const auto count = [&](int64_t t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t); };
+  if (count(64) >= 1024) return {64, count(64)};
+  if (count(32) >= 1024) return {32, count(32)};
+  return {16, count(16)};
+}
+
+// Its estimated time in us: the products of whole tiles at a rate per tile size and storage order (NT, NN,
+// TN), which the smallest tile reaches with 320, 1200 and 440 tiles.
+double native_us(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
+  constexpr double kRate64[3] = {65, 70, 55}, kRate32[3] = {60, 55, 42}, kRate16[3] = {35, 30, 22};   // TFLOP/s
+  constexpr double kFull16[3] = {320, 1200, 440};
+  const NativeTiles t = native_tiles(M, N);
+  double rate = t.size == 64 ? kRate64[layout] : t.size == 32 ? kRate32[layout] : kRate16[layout];
+  if (t.size == 16 && t.count < kFull16[layout]) rate *= (double)t.count / kFull16[layout];
+  return 2e-6 * (double)t.count * t.size * t.size * (double)Kc / rate;
+}
 
 // Parts of the contraction, by estimated time in us: a 32-deep stage takes 1.85 for a workgroup alone on
 // its CU and 2.7 for two side by side, adding the parts takes a launch and their traffic.  Fitted to
 // 30 problems from 8.6 to 69 GFLOP: 0.3 % off the best number of parts, and 2 % off the best of four tile
 // sizes, on average.  2048 x 1024, contraction 4096: 1 part 217 us, 2 128, 4 99, 8 107.
+// Thin outputs, whose 128 x 128 tiles are mostly padding, and few tiles over a long contraction without a
+// workspace for parts are left to the native kernel where that is estimated to be faster (us, forward,
+// native / split): 8 x 8192 over 65536 424 / 685, 15744 x 10 over 38831 679 / 1171, 128 x 128 over 2^18
+// 1207 / 920 with a workspace and 14374 in one part.  Over 70 problems of 2^32 to 2^34.5 multiply-adds in the
+// three storage orders the pick takes 0.5 % more than the faster of the two on average, 36 % at worst (41 %
+// without a workspace); always split: 2.2 % and 73 % (140 % and 14 times).
 struct F32Plan {
-  int parts, k_part;
+  int parts, k_part;   // parts 0: native
 };
-F32Plan plan_f32(int64_t M, int64_t N, int64_t Kc, bool may_split) {
+F32Plan plan_f32(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, bool may_split) {
   constexpr int kCUs = 256, kMostParts = 16;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   F32Plan best = {0, 0};
   if ((double)M * (double)N * (double)Kc < kSplitWork || tiles * kMostParts > 0x7fffffffLL) return best;
-  double least = 0;
+  double least = native_us(layout, M, N, Kc);
   for (int p = 1; p <= (may_split ? kMostParts : 1); ++p) {
     const int64_t k_part = ((Kc + p - 1) / p + 31) / 32 * 32;
     if ((Kc + k_part - 1) / k_part != p) continue;
     const int64_t load = (tiles * p + kCUs - 1) / kCUs;   // workgroups on the fullest CU
     double us = (double)(k_part / 32) * ((double)(load / 2) * 2.7 + (double)(load % 2) * 1.85);
     if (p > 1) us += 3.0 + (p + 1) * (double)M * (double)N * 0.8e-6;
-    if (p == 1 || us < least) least = us, best = {p, (int)k_part};
+    if (us < least) least = us, best = {p, (int)k_part};
   }
   return best;
 }
@@ -592,11 +623,9 @@ int launch_parts(const float* ws, float* C, const float* bias, float* Z, int M, 
   return AXN_OK;
 }
 
-// The native kernel's tile: the largest of 64 x 64, 32 x 32 and 16 x 16 (a loaded element is used 4,
-// 2, 1 times) that still gives the chip's 1024 SIMDs a wave each; smaller tiles keep
-// more loads in flight per wave.  With fewer than 4096 tiles and a contraction of KMIN
-// or more (256 for the smallest tile, 2048 for the middle one; measured: the split
-// loses on the largest tile and on shorter contractions), four waves share a tile.
+// With fewer than 4096 of the native kernel's tiles and a contraction of KMIN or more (256 for the smallest
+// tile, 2048 for the middle one; measured: the split loses on the largest tile and on shorter contractions),
+// four waves share a tile.
 template <bool AK, bool BKM, int EPI, int FM, int FN, int U, int KMIN>
 int launch_waves(long long tiles, const float* A, const float* B, float* C, const float* bias,
                  float* Z, int M, int N, int Kc, int beta, hipStream_t stream) {
@@ -608,7 +637,8 @@ int launch_waves(long long tiles, const float* A, const float* B, float* C, cons
 template <bool AK, bool BKM, int EPI>
 int launch_epi(const float* A, const float* B, float* C, const float* bias, float* Z, int M, int N,
                int Kc, int beta, float* ws, size_t ws_bytes, hipStream_t stream) {
-  const F32Plan plan = plan_f32(M, N, Kc, ws != nullptr);
+  constexpr GemmLayout layout = !AK ? GEMM_TN : BKM ? GEMM_NT : GEMM_NN;
+  const F32Plan plan = plan_f32(layout, M, N, Kc, ws != nullptr);
   if (plan.parts > 1) {
     const size_t need = (size_t)plan.parts * (size_t)M * (size_t)N * sizeof(float);
     if (ws_bytes < need) {
@@ -620,20 +650,18 @@ int launch_epi(const float* A, const float* B, float* C, const float* bias, floa
   }
   if (plan.parts == 1)
     return launch_split<AK, BKM, EPI>(A, B, C, bias, Z, M, N, Kc, beta, plan, stream);
-  const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64);
-  const long long tiles32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
-  const long long tiles16 = (long long)((M + 15) / 16) * ((N + 15) / 16);
-  if (tiles64 >= 1024)
+  const NativeTiles t = native_tiles(M, N);
+  if (t.size == 64)
     return launch_tile<AK, BKM, EPI, 4, 4, 2, 1>(A, B, C, bias, Z, M, N, Kc, beta, stream);
-  if (tiles32 >= 1024)
-    return launch_waves<AK, BKM, EPI, 2, 2, 4, 2048>(tiles32, A, B, C, bias, Z, M, N, Kc, beta, stream);
-  return launch_waves<AK, BKM, EPI, 1, 1, 8, 256>(tiles16, A, B, C, bias, Z, M, N, Kc, beta, stream);
+  if (t.size == 32)
+    return launch_waves<AK, BKM, EPI, 2, 2, 4, 2048>(t.count, A, B, C, bias, Z, M, N, Kc, beta, stream);
+  return launch_waves<AK, BKM, EPI, 1, 1, 8, 256>(t.count, A, B, C, bias, Z, M, N, Kc, beta, stream);
 }
 
 }  // namespace
 
-size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t Kc) {
-  const F32Plan plan = plan_f32(M, N, Kc, true);
+size_t gemm_f32_workspace_bytes(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
+  const F32Plan plan = plan_f32(layout, M, N, Kc, true);
   return plan.parts > 1 ? (size_t)plan.parts * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 

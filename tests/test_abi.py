@@ -68,6 +68,15 @@ def test_workspace_queries():
     assert lib.axn_embedding_workspace_bytes(T, 0) == 0 and lib.axn_embedding_workspace_bytes(-1, V) == 0
 
 
+def test_fp32_workspace_queries():
+    """Parts for problems of 2^32 multiply-adds and more, except thin ones, which the native kernel does faster."""
+    q = nv.load().axn_gemm_f32_workspace_bytes
+    assert q(0, 64, 1024, 4096) == 0                                                  # below the line
+    assert q(0, 2048, 4096, 1024) == 0 and q(0, 512, 4096, 2048) > 0                   # one part, several
+    assert q(0, 300, 2048, 8192) > 0 and q(1, 300, 8192, 2048) > 0 and q(2, 8192, 300, 2048) > 0
+    assert q(0, 8, 8192, 65536) == 0 and q(0, 8192, 8, 65536) == 0 and q(0, 16, 16384, 16384) == 0
+
+
 def _err():
     return nv.load().axn_last_error().decode()
 

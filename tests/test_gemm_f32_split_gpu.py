@@ -165,3 +165,24 @@ def test_a_result_of_one_product():
     want = X.double() @ W.double().t()
     got = ops.gemm_fwd(X, W)[0]
     assert bool(((got.double() - want).abs() <= 2.0 * 2.0 ** -24 * want.abs()).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 1 << 18), (300, 2048, 8192), (8, 8192, 65536)])
+def test_few_tiles_without_a_workspace_are_left_to_the_native_kernel(M, N, K):
+    """A workgroup or a few would walk the whole contraction.  Half of the rows are below 2^32 multiply-adds:
+    the same bits."""
+    from axonn_amd import _native as nv
+
+    g = torch.Generator(device="cuda").manual_seed(10)
+    X, W = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+
+    def forward(rows):
+        y = torch.empty(rows, N, device="cuda")
+        nv.call("axn_gemm_fwd_f32", nv.ptr(X), nv.ptr(W), None, nv.ptr(y), None, rows, N, K, nv.EPI_NONE,
+                nv.current_stream())
+        return y
+
+    assert M // 2 * N * K < 2 ** 32
+    assert torch.equal(forward(M)[:M // 2], forward(M // 2))
+    # four waves share a tile, the native instruction rounds once per 4 indices (at random); twice that
+    assert err(forward(M), X.double() @ W.double().t()) < 2.0 * 2.0 ** -24 * (4 + (K / 16) ** 0.5)

@@ -323,16 +323,21 @@ static int gemm_ws(const char* name, int op, const void* a, const void* b, void*
   g.Z = (uint16_t*)zsave;
   const GemmLayout layout = kLayoutOfOp[op];
   const bool near = lda < kEdgeMaxLd / 2 && ldb < kEdgeMaxLd / 2;   // strides the parts' kernels take
-  const SplitPlan plan =
-      workspace != nullptr && near ? gemm_splits(layout, g.M, g.N, g.Kc) : SplitPlan{1, EDGE_128x128};
+  SplitPlan plan = workspace != nullptr && near ? gemm_splits(layout, g.M, g.N, g.Kc) : SplitPlan{1, EDGE_128x128};
   if (plan.parts > 1) {
     const size_t need = partial_bytes(plan, g);
-    REQUIRE(workspace_bytes >= need, AXN_EINVAL,
+    const bool given = workspace_bytes >= need && aligned16(workspace);
+    // an epilogue or a ragged shape: the plain GEMM, as before such products were divided
+    const bool may_do_without =
+        epilogue != AXN_EPI_NONE || g.M % 128 != 0 || g.N % 128 != 0 || g.Kc % 64 != 0;
+    if (!given && may_do_without) plan.parts = 1;
+    REQUIRE(given || may_do_without || workspace_bytes >= need, AXN_EINVAL,
             "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
-    REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+    REQUIRE(given || may_do_without, AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+  }
+  if (plan.parts > 1)
     return launch_gemm_splitk(layout, g, epilogue, half, out_dtype == AXN_F32, plan, (float*)workspace,
                               (hipStream_t)stream);
-  }
   return half ? launch_gemm_f16(layout, g, epilogue, out_dtype == AXN_F32, (hipStream_t)stream)
               : launch_gemm_bf16(layout, g, epilogue, out_dtype == AXN_F32, (hipStream_t)stream);
 }

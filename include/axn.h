@@ -154,16 +154,19 @@ AXN_API int axn_gemm_fwd_f32out(const void* X, const void* W, const float* bias,
 /* Variants of the three GEMMs that divide the contraction among workgroups, given a
  * workspace.  No reference counterpart: torch picks such kernels inside its GEMM library.
  *   A problem with few output tiles (a short batch, a narrow shard) leaves most CUs
- *   without work: the contraction is cut into 2, 4 or 8 parts whose fp32 partial
- *   products a second pass adds in a fixed order (epilogue NONE only; results are
- *   reproducible bit for bit).
- *   axn_gemm_workspace_bytes(op, M, N, K): bytes the call below would use for dense
- *   operands and epilogue NONE, 0 if it would not split.  op, M, N, K as in the call.
+ *   without work: the contraction is cut into 2 to 16 parts whose fp32 partial products a
+ *   second pass adds in a fixed order and gives the output's epilogue, Zsave and beta (results
+ *   are reproducible bit for bit).  Any shape the plain GEMM takes, whole tiles or ragged.
+ *   axn_gemm_workspace_bytes(op, M, N, K): bytes the call below uses, 0 if it would not
+ *   split.  op, M, N, K as in the call, whatever its epilogue (operands with rows 2^22
+ *   elements or more apart are not split).
  *   axn_gemm_*_ws: arguments as axn_gemm_fwd / _dgrad / _wgrad, plus dtype (AXN_BF16 or
  *   AXN_F16) of the 16-bit operands and results, and the workspace (16-byte aligned, used
  *   by this call alone until it has finished; contents need not be initialised).
- *   workspace == NULL, an epilogue, or a shape that does not profit: the call is the
- *   plain GEMM. */
+ *   workspace == NULL, or a shape that does not profit: the call is the plain GEMM.  A
+ *   workspace that is too small is AXN_EINVAL, a misaligned one AXN_EALIGN, for a product of
+ *   whole 128 x 128 tiles and 64-deep stages without an epilogue; with an epilogue or a
+ *   ragged shape the call is then the plain GEMM. */
 typedef enum axn_gemm_op { AXN_GEMM_FWD = 0, AXN_GEMM_DGRAD = 1, AXN_GEMM_WGRAD = 2 } axn_gemm_op;
 AXN_API size_t axn_gemm_workspace_bytes(int op, int64_t M, int64_t N, int64_t K);
 AXN_API int axn_gemm_fwd_ws(const void* X, const void* W, const float* bias, void* Y, void* Zsave,

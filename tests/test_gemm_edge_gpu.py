@@ -147,3 +147,20 @@ def test_split_contraction_of_any_shape_with_its_epilogue(op, M, N, K, dtype):
                 c.stride(0), 1, nv.F32, *tail)
         check(full, c, a.double().t() @ b.double() + 3.0)
     assert bool(torch.isnan(ws[nbytes // 4:]).all()), "written behind the workspace"
+
+
+@pytest.mark.parametrize("M,N,K,epi", [(256, 512, 4096, nv.EPI_BIAS), (300, 1000, 1608, nv.EPI_NONE)])
+@pytest.mark.parametrize("nbytes,offset", [(64, 0), (1 << 24, 4)])
+def test_a_workspace_too_small_or_misaligned_with_an_epilogue_or_a_ragged_shape(M, N, K, epi, nbytes, offset):
+    """The plain GEMM, bit for bit, and the workspace is left alone."""
+    assert nv.load().axn_gemm_workspace_bytes(0, M, N, K) > 64
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x, w = (numbers(r, K, torch.bfloat16, gen, 16) for r in (M, N))
+    bias = torch.randn(N, generator=gen, device="cuda")
+    ws = torch.full((nbytes + 16,), 7, dtype=torch.uint8, device="cuda")
+    got, want = (torch.empty(M, N, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    args = (M, N, K, x.stride(0), w.stride(0), N, epi)
+    nv.call("axn_gemm_fwd_ws", nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(got), None, nv.BF16, *args,
+            ws.data_ptr() + offset, nbytes, nv.current_stream())
+    nv.call("axn_gemm_fwd", nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(want), None, *args, nv.current_stream())
+    assert torch.equal(got, want) and bool((ws == 7).all())

@@ -356,6 +356,7 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void*
   int rc = check_gemm(name, A, B, C, M, n8, K, lda, ldb, fwd ? n8 : ldc, fwd ? K : n8, K, fwd ? n8 : K);
   if (rc) return rc;
   REQUIRE(!fwd || ldc >= N, AXN_EINVAL, "%s: leading dimension smaller than the row length", name);
+  REQUIRE(Zsave == nullptr || aligned16(Zsave), AXN_EALIGN, "%s: Zsave must be 16-byte aligned", name);
   const bool bias16 = (epilogue & AXN_BIAS_16BIT) != 0;
   epilogue &= ~(int)AXN_BIAS_16BIT;
   rc = check_epilogue(name, epilogue, bias);

@@ -123,6 +123,13 @@ def test_gemm_argument_errors():
     assert lib.axn_gemm_dgrad_f16(A, None, A, 8, 8, 8, 8, 8, 8, None) == nv.AXN_EINVAL
     assert lib.axn_gemm_wgrad_f16(A, A, A, 8, 8, 8, 8, 8, 8, 0, nv.BF16, None) == nv.AXN_EINVAL
     assert "fp16 or fp32" in _err()
+    # any number of output features: the pre-activation is stored in 16-byte vectors, as Y's first row
+    fn = lib.axn_gemm_any_n
+    half_aligned = ctypes.c_void_p(0x1008)
+    for n, ld in ((16, 16), (17, 17)):
+        assert fn(0, A, A, A, A, half_aligned, nv.BF16, 8, n, 8, 8, 8, ld, nv.EPI_BIAS_GELU, 0, nv.BF16, None, 0,
+                  None) == nv.AXN_EALIGN
+        assert "Zsave" in _err()
     # split-contraction variants
     ws = lib.axn_gemm_dgrad_ws
     assert ws(A, A, A, nv.F32, 512, 8192, 3584, 8192, 3584, 3584, A, 1 << 30, None) == nv.AXN_EINVAL

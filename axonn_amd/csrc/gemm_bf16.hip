@@ -228,6 +228,11 @@ int launch_whole(const GemmArgs& g, hipStream_t stream) {
 // The two parts run one after the other on the caller's stream.
 template <bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
 int launch_shape(const GemmArgs& g, hipStream_t stream) {
+  if constexpr (EPI != EPI_PAIR) {
+    // output rows that are not 16-byte aligned (axn_gemm_any_n): the kernels with bounds store them
+    constexpr GemmLayout layout = !AK ? GEMM_TN : BKM ? GEMM_NT : GEMM_NN;
+    if (g.ldc % 8 != 0) return launch_edge(layout, g, EPI, OUT_F32, HALF, stream);
+  }
   if (g.M % 256 == 0 && g.N % 256 == 0 && g.Kc % 64 == 0 && g.splits <= 1) {
     const long long tm = g.M / 256, tn = g.N / 256, tiles = tm * tn;
     const long long full = tiles / 256 * 256, rest = tiles - full;

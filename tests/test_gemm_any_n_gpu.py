@@ -61,6 +61,37 @@ def test_forward_leaves_the_neighbours_alone():
     assert bool((buf[:M * ld].view(M, ld)[:, N:] == 7).all()) and bool((buf[M * ld:] == 7).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 1024, 64), (128, 128, 64), (512, 1024, 128), (2304, 2048, 64),
+                                   (3072, 2048, 64), (4096, 4096, 64), (4352, 4096, 64), (256, 512, 4096)])
+@pytest.mark.parametrize("out_f32", [False, True])
+def test_forward_of_whole_tiles_at_odd_row_strides(M, N, K, out_f32):
+    """Rows of Y that start anywhere are stored by kernels that do not take them for 16-byte aligned, whatever
+    the shape: streamed, each tile size, full rounds and a rest, a contraction in parts.  Exact whole numbers."""
+    from axonn_amd import _native as nv
+    from launches import launches
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    X, W = (torch.randint(-2, 3, (n, K), generator=g, device="cuda").bfloat16() for n in (M, N))
+    b = torch.randint(-3, 4, (N,), generator=g, device="cuda").float()
+    want = X.double() @ W.double().t() + b
+    nbytes = nv.load().axn_gemm_workspace_bytes(0, M, N, K)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device="cuda")
+    dtype = torch.float32 if out_f32 else torch.bfloat16
+    for ld in (N + 1, N + 3, N + 8):
+        buf = torch.full((M * ld + 64,), 7.0, device="cuda", dtype=dtype)
+
+        def forward():
+            nv.call("axn_gemm_any_n", 0, nv.ptr(X), nv.ptr(W), nv.ptr(b), nv.ptr(buf), None, nv.BF16, M, N, K, K, K,
+                    ld, nv.EPI_BIAS, 0, nv.dtype_code(dtype), nv.ptr(ws), nbytes, nv.current_stream())
+
+        names = [name for name, _ in launches(forward)]
+        last = names[-1]   # of parts: the pass that adds them, with element-aligned rows
+        if ld % 8:
+            assert "edge_kernel" in last or "stream_kernel" in last or last.endswith("Lb1EEEvPKfNS_8GemmArgsE"), names
+        assert torch.equal(buf[:M * ld].view(M, ld)[:, :N].double(), want.to(dtype).double())
+        assert bool((buf[:M * ld].view(M, ld)[:, N:] == 7).all()) and bool((buf[M * ld:] == 7).all())
+
+
 @pytest.mark.parametrize("M,N,ld", [(1, 1, 1), (3, 17, 17), (5, 24, 31), (70, 1003, 1005)])
 def test_pad_rows(M, N, ld):
     from axonn_amd import ops

@@ -111,6 +111,22 @@ struct GemmArgs {
   int k_first;
 };
 
+// Sizes go up to 2^31 - 1: what is rounded up to tiles or stages is computed in 64 bits.
+__host__ __device__ constexpr int64_t ceil_div(int64_t n, int64_t by) { return (n + by - 1) / by; }
+// The 64-deep stages of a contraction of kc that part `part` of `parts` covers.
+struct StageRange {
+  int first, count;
+};
+__host__ __device__ constexpr StageRange stages_of_part(int kc, int part, int parts) {
+  const int all = (int)ceil_div(kc, 64);   // at most 2^25, times 16 parts 2^29
+  if (parts <= 1) return {0, all};
+  const int first = part * all / parts;
+  return {first, (part + 1) * all / parts - first};
+}
+static_assert(stages_of_part(0x7fffffff, 0, 1).count == 1 << 25 && stages_of_part(0x7fffffff, 15, 16).first == 15 << 21 &&
+                  stages_of_part(0x7fffffff, 15, 16).count == 1 << 21,
+              "the longest contraction");
+
 // Address of the bias of output column n.
 inline const void* bias_at(const GemmArgs& g, int64_t n) {
   return g.bias == nullptr ? nullptr : (const char*)g.bias + n * (g.bias16 ? 2 : 4);

@@ -189,8 +189,8 @@ int launch_whole(const GemmArgs& g, hipStream_t stream) {
   const bool deep = g.Kc % 64 == 0;
   const bool whole256 = (g.M % 256 == 0) && (g.N % 256 == 0) && deep;
   const bool whole128 = (g.M % 128 == 0) && (g.N % 128 == 0) && deep;
-  const long long tiles256 = (long long)((g.M + 255) / 256) * ((g.N + 255) / 256);
-  const long long tiles128 = (long long)((g.M + 127) / 128) * ((g.N + 127) / 128);
+  const long long tiles256 = ceil_div(g.M, 256) * ceil_div(g.N, 256);
+  const long long tiles128 = ceil_div(g.M, 128) * ceil_div(g.N, 128);
   // The one-wave-per-SIMD kernel addresses its operands with 32-bit byte offsets.
   const int64_t a_span = (int64_t)(AK ? g.M : g.Kc) * g.lda * 2;
   const int64_t b_span = (int64_t)(BKM ? g.N : g.Kc) * g.ldb * 2;
@@ -290,7 +290,7 @@ template <int EPI, bool OUT_F32, bool HALF, bool ANY>
 __global__ void __launch_bounds__(256)
     splitk_reduce_kernel(const float* __restrict__ ws, const GemmArgs g) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t per_row = (g.N + 7) / 8;
+  const int64_t per_row = ceil_div(g.N, 8);
   if (idx >= (int64_t)g.M * per_row) return;
   const int64_t row = idx / per_row, col = (idx - row * per_row) * 8, part = (int64_t)g.M * per_row * 8;
   const float* p = ws + row * per_row * 8 + col;
@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(256)
 
 template <bool HALF, bool ANY>
 int launch_reduce(const float* ws, const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
-  const int64_t lanes = (int64_t)g.M * ((g.N + 7) / 8);
+  const int64_t lanes = (int64_t)g.M * ceil_div(g.N, 8);
   const dim3 grid((unsigned)((lanes + 255) / 256)), block(256);
 #define REDUCE(EPI, F32) hipLaunchKernelGGL((splitk_reduce_kernel<EPI, F32, HALF, ANY>), grid, block, 0, stream, ws, g)
   if (out_f32) {
@@ -471,8 +471,8 @@ bool plan_together(PlannedTogether (&plans)[4], int& next, long long td, long lo
 }
 // The problem with the longer tiles takes the first workgroups.
 void place_together(GemmArgs& gd, GemmArgs& gw, long long td, long long tw, long long sd, long long sw) {
-  gw.tiles_m = (gw.M + 255) / 256, gw.tiles_n = (gw.N + 255) / 256, gw.wg_first = sw >= sd ? 0 : (int)td;
-  gd.tiles_m = (gd.M + 255) / 256, gd.tiles_n = (gd.N + 255) / 256, gd.wg_first = sw >= sd ? (int)tw : 0;
+  gw.tiles_m = (int)ceil_div(gw.M, 256), gw.tiles_n = (int)ceil_div(gw.N, 256), gw.wg_first = sw >= sd ? 0 : (int)td;
+  gd.tiles_m = (int)ceil_div(gd.M, 256), gd.tiles_n = (int)ceil_div(gd.N, 256), gd.wg_first = sw >= sd ? (int)tw : 0;
   gw.splits = gd.splits = 0;
 }
 
@@ -516,9 +516,8 @@ int launch_backward(const GemmArgs& gd_in, const GemmArgs& gw_in, bool dw_f32, h
     return (g.M % 128 != 0 || g.N % 128 != 0 || g.Kc % 64 != 0) && g.lda < kEdgeMaxLd / 2 && g.ldb < kEdgeMaxLd / 2;
   };
   if (ragged(gd) && ragged(gw)) {
-    const long long td = (long long)((gd.M + 255) / 256) * ((gd.N + 255) / 256);
-    const long long tw = (long long)((gw.M + 255) / 256) * ((gw.N + 255) / 256);
-    const long long sd = (gd.Kc + 63) / 64, sw = (gw.Kc + 63) / 64;
+    const long long td = ceil_div(gd.M, 256) * ceil_div(gd.N, 256), tw = ceil_div(gw.M, 256) * ceil_div(gw.N, 256);
+    const long long sd = ceil_div(gd.Kc, 64), sw = ceil_div(gw.Kc, 64);
     static thread_local PlannedTogether plans[4] = {};
     static thread_local int next_plan = 0;
     const bool together = plan_together(plans, next_plan, td, tw, sd, sw, [&] {
@@ -598,7 +597,7 @@ int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool
                        const SplitPlan& plan, float* ws, hipStream_t stream) {
   GemmArgs g = in;
   g.C = ws;
-  g.ldc = (g.N + 7) / 8 * 8;   // whole vectors a row
+  g.ldc = ceil_div(g.N, 8) * 8;   // whole vectors a row
   g.beta = 0;
   g.bias = nullptr;
   g.Z = nullptr;

@@ -38,8 +38,8 @@ template <int BM, int BN, bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
 int launch_edge_tile(const GemmArgs& in, hipStream_t stream) {
   GemmArgs g = in;
   constexpr int COLS = EPI == EPI_SWIGLU ? BN / 2 : BN;   // output columns of a tile
-  g.tiles_m = (g.M + BM - 1) / BM;
-  g.tiles_n = (g.N + COLS - 1) / COLS;
+  g.tiles_m = (int)ceil_div(g.M, BM);
+  g.tiles_n = (int)ceil_div(g.N, COLS);
   const long long nwg = (long long)g.tiles_m * g.tiles_n * (g.splits > 1 ? g.splits : 1);
   if (nwg > 0x7fffffffLL) {
     set_error("gemm: too many output tiles (%lld)", nwg);
@@ -63,7 +63,7 @@ template <bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
 int launch_edge_kind(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
   if (tile == EDGE_128x128) return launch_edge_tile<128, 128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
   if (tile == EDGE_256x128) return launch_edge_tile<256, 128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
-  const long long tm = (g.M + 255) / 256, tn = (g.N + 255) / 256, tiles = tm * tn;
+  const long long tm = ceil_div(g.M, 256), tn = ceil_div(g.N, 256), tiles = tm * tn;
   const long long full = tiles / 256 * 256, rest = tiles - full;
   if (g.splits <= 1 && full > 0 && rest > 0 && rest <= 128 && (full % tm == 0 || full % tn == 0)) {
     constexpr int64_t esz = OUT_F32 ? 4 : 2;

@@ -134,10 +134,11 @@ __device__ __forceinline__ void direct_tile(f32x4 (&acc)[FM][FN], const float* _
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i][s], b[u][j][s], acc[i][j], 0, 0, 0);
   };
   const int whole = k_begin + (k_end - k_begin) / (16 * U) * (16 * U);  // the part made of whole chunks
-  for (int k0 = k_begin + first * 16 * U; k0 < whole; k0 += step * 16 * U)
-    blocks(std::false_type{}, k0, std::integral_constant<int, U>{});
-  for (int k0 = whole + first * 16; k0 < k_end; k0 += step * 16)
-    blocks(std::true_type{}, k0, std::integral_constant<int, 1>{});
+  // (unsigned: past the end of the longest contraction an int overflows)
+  for (unsigned k0 = k_begin + first * 16 * U; k0 < (unsigned)whole; k0 += step * 16 * U)
+    blocks(std::false_type{}, (int)k0, std::integral_constant<int, U>{});
+  for (unsigned k0 = whole + first * 16; k0 < (unsigned)k_end; k0 += step * 16)
+    blocks(std::true_type{}, (int)k0, std::integral_constant<int, 1>{});
 }
 
 // Whether the lane's operands hold a non-zero number under `bound`.
@@ -416,7 +417,8 @@ __global__ void __launch_bounds__(256, 2)
   const int part = blockIdx.x / tiles, id = blockIdx.x - part * tiles;
   const int tm = id / tiles_n, tn = id - tm * tiles_n;
   const int m0 = tm * 32 * FM, n0 = tn * 32 * FN;
-  const int k_begin = part * k_part, k_end = min(Kc, k_begin + k_part);
+  // (unsigned: past the end of the longest contraction an int overflows)
+  const unsigned k_begin = part * k_part, k_end = min((unsigned)Kc, k_begin + k_part);
   C += (int64_t)part * M * N;
 
   f32x4 acc[FM][FN], low[FM][FN];
@@ -427,7 +429,7 @@ __global__ void __launch_bounds__(256, 2)
   my_share<BKM>(gb, qb);
   float xa[FM][4], xb[FN][4];
   // Rows past the edge read a valid one, indices past the end count as zero.
-  auto fetch = [&](int k0) {
+  auto fetch = [&](unsigned k0) {
     if (k0 + 32 <= k_end) {
       load_block<AK, FM, VEC, false>(xa, A, m0 + FM * ga, M, k0 + 4 * qa, Kc, k_end);
       load_block<BKM, FN, VEC, false>(xb, B, n0 + FN * gb, N, k0 + 4 * qb, Kc, k_end);
@@ -439,7 +441,7 @@ __global__ void __launch_bounds__(256, 2)
   float largest = 0.f;
   if (threadIdx.x == 0) large = 0;
   fetch(k_begin);
-  for (int k0 = k_begin; k0 < k_end; k0 += 32) {
+  for (unsigned k0 = k_begin; k0 < k_end; k0 += 32) {
     put_stage<AK, FM>(la, xa);
     put_stage<BKM, FN>(lb, xb);
     largest = max_magnitude(max_magnitude(largest, xa), xb);
@@ -480,7 +482,7 @@ __global__ void __launch_bounds__(256, 2)
 template <bool AK, bool BKM, int EPI, int FM, int FN, int U, int WAVES>
 int launch_tile(const float* A, const float* B, float* C, const float* bias, float* Z, int M,
                 int N, int Kc, int beta, hipStream_t stream) {
-  const long long tiles_m = (M + 16 * FM - 1) / (16 * FM), tiles_n = (N + 16 * FN - 1) / (16 * FN);
+  const long long tiles_m = ceil_div(M, 16 * FM), tiles_n = ceil_div(N, 16 * FN);
   const long long nwg = tiles_m * tiles_n;
   if (nwg > 0x7fffffffLL) {
     set_error("gemm_f32: too many output tiles (%lld)", nwg);
@@ -583,7 +585,7 @@ F32Plan plan_f32(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, bool may_s
     const int64_t load = (tiles * p + kCUs - 1) / kCUs;   // workgroups on the fullest CU
     double us = (double)(k_part / 32) * ((double)(load / 2) * 2.7 + (double)(load % 2) * 1.85);
     if (p > 1) us += 3.0 + (p + 1) * (double)M * (double)N * 0.8e-6;
-    if (us < least) least = us, best = {p, (int)k_part};
+    if (us < least) least = us, best = {p, (int)(k_part < Kc ? k_part : Kc)};   // (one part of the longest: 2^31)
   }
   return best;
 }
@@ -592,7 +594,7 @@ template <bool AK, bool BKM, int EPI>
 int launch_split(const float* A, const float* B, float* C, const float* bias, float* Z, int M, int N,
                       int Kc, int beta, const F32Plan& plan, hipStream_t stream) {
   constexpr int F = 4;
-  const int tiles_m = (M + 32 * F - 1) / (32 * F), tiles_n = (N + 32 * F - 1) / (32 * F);
+  const int tiles_m = (int)ceil_div(M, 32 * F), tiles_n = (int)ceil_div(N, 32 * F);
   const dim3 grid((unsigned)((int64_t)tiles_m * tiles_n * plan.parts)), block(256);
   // as launch_tile's
   const uintptr_t ptrs = (uintptr_t)A | (uintptr_t)B | (uintptr_t)C | (uintptr_t)bias | (uintptr_t)Z;

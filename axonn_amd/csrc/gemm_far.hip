@@ -92,8 +92,8 @@ __global__ void __launch_bounds__(64) gemm_far_kernel(const GemmArgs g, int epil
 template <bool HALF>
 int launch_far(GemmLayout layout, const GemmArgs& in, int epilogue, bool out_f32, hipStream_t stream) {
   GemmArgs g = in;
-  g.tiles_m = (int)(((int64_t)g.M + 31) / 32);
-  g.tiles_n = (int)(((int64_t)g.N + 31) / 32);
+  g.tiles_m = (int)ceil_div(g.M, 32);
+  g.tiles_n = (int)ceil_div(g.N, 32);
   const long long nwg = (long long)g.tiles_m * g.tiles_n;
   if (nwg > 0x7fffffffLL) {
     set_error("gemm: too many output tiles (%lld)", nwg);

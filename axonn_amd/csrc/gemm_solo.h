@@ -435,9 +435,10 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   const int m0 = tm * BM, n0 = tn * (SWIGLU ? BN / 2 : BN);
   int KP, s0;
   if constexpr (EDGE) {
-    const int S = (g.Kc + PK - 1) / PK;
-    s0 = g.splits > 1 ? (int)((int64_t)split * S / g.splits) : 0;
-    KP = (g.splits > 1 ? (int)((int64_t)(split + 1) * S / g.splits) : S) - s0;
+    static_assert(PK == 64, "stages_of_part");
+    const StageRange part = stages_of_part(g.Kc, split, g.splits);
+    s0 = part.first;
+    KP = part.count;
   } else {
     KP = (g.splits > 1 ? g.k_split : g.Kc) / PK;
     s0 = split * KP;
@@ -469,7 +470,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
                                           int rows, int kc, int64_t ld, int row0, int k0) {
       const int64_t first = kmajor ? row0 * ld + k0 : k0 * ld + row0;
       // a row's last 8 elements are copied together: up to 7 of them are padding of the operand's rows
-      const int64_t all = kmajor ? (int64_t)(rows - 1) * ld + (kc + 7) / 8 * 8 : (int64_t)(kc - 1) * ld + (rows + 7) / 8 * 8;
+      const int64_t all = kmajor ? (int64_t)(rows - 1) * ld + ceil_div(kc, 8) * 8 : (int64_t)(kc - 1) * ld + ceil_div(rows, 8) * 8;
       at[0] = (const char*)(base + first);
       at[1] = base2 != nullptr ? (const char*)(base2 + first) : at[0];
       left = (all - first) * 2;
@@ -642,7 +643,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
     vb = OB::dma_offset(g.ldb, 0, wave, lane, b_is);
     va_end = va;
     vb_end = vb;
-    const int over = (s0 + KP) * PK - g.Kc;   // contraction elements the last stage lacks
+    const int over = (int)((int64_t)(s0 + KP) * PK - g.Kc);   // contraction elements the last stage lacks
     if (over > 0) {
       if (A_KMAJOR && 8 * OA::dma_chunk(wave, lane) >= PK - over) va_end = kOutside;
       if (B_KMAJOR && 8 * OB::dma_chunk(wave, lane) >= PK - over) vb_end = kOutside;

@@ -158,7 +158,7 @@ template <int MT, int R, int NW, int D, bool HALF>
 int launch_stream(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
   constexpr size_t ring = (size_t)NW * D * (R + MT) * 2048, sums = (size_t)NW * MT * R * 1024;
   constexpr size_t lds = ring > sums ? ring : sums;
-  const dim3 grid((unsigned)((g.N + 16 * R - 1) / (16 * R))), block(NW * 64);
+  const dim3 grid((unsigned)ceil_div(g.N, 16 * R)), block(NW * 64);
 #define STREAM(EPI, F32)                                                                   \
   {                                                                                        \
     void (*kern)(const GemmArgs) = gemm_stream_kernel<MT, R, NW, D, EPI, F32, HALF>;       \

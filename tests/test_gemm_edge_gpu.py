@@ -164,3 +164,19 @@ def test_a_workspace_too_small_or_misaligned_with_an_epilogue_or_a_ragged_shape(
             ws.data_ptr() + offset, nbytes, nv.current_stream())
     nv.call("axn_gemm_fwd", nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.ptr(want), None, *args, nv.current_stream())
     assert torch.equal(got, want) and bool((ws == 7).all())
+
+
+def test_the_longest_contractions():
+    """A weight gradient over 2^31 - 8 tokens: the stages of 64 and their parts are counted past 2^31.  Zeros
+    but for the first and the last rows and one in each part."""
+    M = 2 ** 31 - 8
+    if torch.cuda.mem_get_info()[0] < 90e9:
+        pytest.skip("needs 69 GB")
+    from axonn_amd import ops
+
+    dy, x = (torch.zeros((M, 8), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    want = torch.zeros(8, 8, dtype=torch.float64, device="cuda")
+    for i, row in enumerate([0, 1, M - 1, M - 2, M - 70] + [p * (M // 16) + 5 for p in range(16)]):
+        dy[row, i % 8], x[row, (3 * i) % 8] = 1, i + 1
+        want[i % 8, (3 * i) % 8] += i + 1
+    assert torch.equal(ops.gemm_wgrad(dy, x, out_dtype=torch.float32).double(), want)

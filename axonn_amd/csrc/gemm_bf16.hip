@@ -454,19 +454,20 @@ double stages_together(long long t1, long long s1, long long t2, long long s2) {
 }
 
 // Whether two tile sets run in one launch; the answers for the last few shapes of a thread
-// are kept, a training loop asks for the same ones again and again.
+// are kept, a training loop asks for the same ones again and again.  The key holds all that
+// `ends_earlier` looks at.
 struct PlannedTogether {
-  long long td, tw, sd, sw;
+  long long key[4];
   bool together;
 };
 template <class F>
-bool plan_together(PlannedTogether (&plans)[4], int& next, long long td, long long tw, long long sd,
-                   long long sw, F&& ends_earlier) {
+bool plan_together(PlannedTogether (&plans)[4], int& next, long long k0, long long k1, long long k2, long long k3,
+                   F&& ends_earlier) {
   for (const PlannedTogether& p : plans)
-    if (p.td == td && p.tw == tw && p.sd == sd && p.sw == sw) return p.together;
+    if (p.key[0] == k0 && p.key[1] == k1 && p.key[2] == k2 && p.key[3] == k3) return p.together;
   PlannedTogether& p = plans[next];
   next = (next + 1) % 4;
-  p = {td, tw, sd, sw, td + tw <= 4096 && ends_earlier()};
+  p = {{k0, k1, k2, k3}, ends_earlier()};
   return p.together;
 }
 // The problem with the longer tiles takes the first workgroups.
@@ -493,7 +494,8 @@ int launch_backward(const GemmArgs& gd_in, const GemmArgs& gw_in, bool dw_f32, h
     static thread_local PlannedTogether plans[4] = {};
     static thread_local int next_plan = 0;
     const bool together = plan_together(plans, next_plan, td, tw, sd, sw, [&] {
-      return stages_together(tw, sw, td, sd) < 0.95 * (stages_alone(td, sd) + stages_alone(tw, sw));
+      return td + tw <= 4096 &&
+             stages_together(tw, sw, td, sd) < 0.95 * (stages_alone(td, sd) + stages_alone(tw, sw));
     });
     if (together) {
       place_together(gd, gw, td, tw, sd, sw);
@@ -520,7 +522,8 @@ int launch_backward(const GemmArgs& gd_in, const GemmArgs& gw_in, bool dw_f32, h
     const long long sd = ceil_div(gd.Kc, 64), sw = ceil_div(gw.Kc, 64);
     static thread_local PlannedTogether plans[4] = {};
     static thread_local int next_plan = 0;
-    const bool together = plan_together(plans, next_plan, td, tw, sd, sw, [&] {
+    const bool together = plan_together(plans, next_plan, gd.M, gd.N, gd.Kc, 0, [&] {
+      if (td + tw > 4096) return false;
       double ud = 0, uw = 0;
       edge_tile(gd.M, gd.N, gd.Kc, &ud);
       edge_tile(gw.M, gw.N, gw.Kc, &uw);

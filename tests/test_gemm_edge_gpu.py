@@ -7,10 +7,13 @@ result is exact too: the float64 product rounded once to the storage type.  The 
 views into buffers whose other elements are NaN, and the outputs views into buffers filled
 with a canary: what lies outside a view is neither read into a result nor written."""
 
+import threading
+
 import pytest
 import torch
 
 from axonn_amd import _native as nv
+from launches import launches
 
 pytestmark = pytest.mark.gpu
 
@@ -180,3 +183,28 @@ def test_the_longest_contractions():
         dy[row, i % 8], x[row, (3 * i) % 8] = 1, i + 1
         want[i % 8, (3 * i) % 8] += i + 1
     assert torch.equal(ops.gemm_wgrad(dy, x, out_dtype=torch.float32).double(), want)
+
+
+def backward(M, N, K, dtype=torch.bfloat16):
+    """A call of the joint entry point on operands of ones."""
+    dy, w, x = (torch.ones(s, dtype=dtype, device="cuda") for s in ((M, N), (N, K), (M, K)))
+    dx, dw = torch.empty(M, K, dtype=dtype, device="cuda"), torch.empty(N, K, dtype=dtype, device="cuda")
+    return lambda: nv.call("axn_gemm_bwd", nv.ptr(dy), nv.ptr(w), nv.ptr(x), nv.ptr(dx), nv.ptr(dw),
+                           nv.dtype_code(dtype), M, N, K, N, K, K, K, K, 0, nv.dtype_code(dtype), nv.current_stream())
+
+
+def test_a_shape_is_planned_alike_whatever_was_asked_before():
+    """Two ragged shapes with the same numbers of tiles and stages, one of them better in one launch: the plan
+    that a thread keeps for the first is not taken for the second."""
+    shapes = [(3783, 2520, 3080), (3783, 2520, 3208)]
+    found = {}
+
+    def plan(order):
+        found[tuple(order)] = [launches(backward(*shapes[i])) for i in order]
+
+    for order in ((0, 1), (1, 0)):   # a thread's plans are its own
+        t = threading.Thread(target=plan, args=(order,))
+        t.start()
+        t.join()
+    assert found[0, 1] == found[1, 0][::-1]
+    assert [len(f) for f in found[0, 1]] != [1, 1], "the second is meant to differ from the first"

@@ -177,10 +177,20 @@ int launch_gemm_edge_backward_f16(const GemmArgs& wgrad, const GemmArgs& dgrad, 
                                   hipStream_t stream);
 
 // Forward products of a few rows (gemm_stream.hip): a stream over the weights; row strides
-// below kStreamMaxLd elements.  Up to 32 rows it is ahead of the tiles with a split contraction
-// everywhere, up to 64 for contractions that are not long (64 rows, us, stream / tiles:
-// 4096 x 4096 13.5 / 15.8, 14336 x 4096 25.9 / 31.6, 4096 x 14336 45 / 32.5).
-inline bool stream_takes(int64_t M, int64_t Kc) { return M <= 32 || (M <= 64 && Kc <= 6144); }
+// below kStreamMaxLd elements.
+constexpr int64_t kStreamMaxRows = 64;
+// Whether it is also ahead of tiles with the contraction in parts.  Those lose on many weights and win where a
+// few workgroups would walk a long contraction; the line lies where they meet over 360 shapes of 1 to 64 rows,
+// 64 to 14336 outputs and contractions of 1024 to 65536 (cold weights; the pick is 0.5 % off the faster one on
+// average, 14 % at worst).  us, stream / tiles:
+//   64 rows   512 x 4096 12.5 / 11.4    512 x 5120 15.9 / 12.7   4096 x 8192 23.5 / 24.0   4096 x 14336 47 / 37
+//   32 rows   512 x 8192 13.5 / 14.5    512 x 28672 51 / 31      4096 x 28672 66 / 64      8192 x 65536 207 / 232
+//   8 rows    512 x 14336 15.3 / 18.7   512 x 65536 56 / 55      4096 x 65536 84 / 143
+inline bool stream_ahead(int64_t M, int64_t N, int64_t Kc) {
+  if (M > kStreamMaxRows) return false;
+  if (N >= 8192 || (N >= 4096 && M <= 32)) return true;
+  return M * Kc <= (N >= 4096 ? 524288 : 196608);
+}
 constexpr int64_t kStreamMaxLd = 1LL << 24;
 int launch_gemm_stream(const GemmArgs& args, int epilogue, bool out_f32, bool half, hipStream_t stream);
 

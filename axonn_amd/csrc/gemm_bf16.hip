@@ -343,7 +343,7 @@ int launch_split(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
 template <bool HALF>
 int launch_layout(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32,
                   hipStream_t stream) {
-  if (layout == GEMM_NT && stream_takes(g.M, g.Kc) && g.lda < kStreamMaxLd && g.ldb < kStreamMaxLd &&
+  if (layout == GEMM_NT && g.M <= kStreamMaxRows && g.lda < kStreamMaxLd && g.ldb < kStreamMaxLd &&
       (!out_f32 || epilogue == AXN_EPI_BIAS || epilogue == AXN_EPI_BIAS_GELU))
     return launch_gemm_stream(g, epilogue, out_f32, HALF, stream);
   switch (layout) {
@@ -570,7 +570,7 @@ int launch_gemm_f16(GemmLayout layout, const GemmArgs& g, int epilogue, bool out
 // It looks at sizes only, not at strides: a caller asks for the workspace by size.
 SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
   SplitPlan plan = {1, EDGE_128x128};
-  if (layout == GEMM_NT && stream_takes(M, Kc)) return plan;
+  if (layout == GEMM_NT && stream_ahead(M, N, Kc)) return plan;
   const bool whole = M % 128 == 0 && N % 128 == 0 && Kc % 64 == 0;
   auto count = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   const long long tiles[3] = {count(256, 256), count(256, 128), count(128, 128)};

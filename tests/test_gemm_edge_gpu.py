@@ -110,6 +110,7 @@ def test_edge_epilogues_keep_the_pre_activation(M, N, K):
 @pytest.mark.parametrize("op,M,N,K", [
     (0, 65, 136, 2056), (0, 129, 392, 4104), (0, 300, 1000, 1608),      # 128 x 128 tiles
     (0, 520, 2560, 8200), (1, 300, 8200, 2568), (2, 4104, 136, 264),    # 256 wide ones
+    (0, 24, 520, 16384), (0, 1, 8, 200000), (0, 64, 4096, 8200),         # few rows, a long contraction
     (0, 128, 384, 12224),    # whole tiles whose 191 stages no number of parts divides
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -37,9 +37,8 @@ __global__ void __launch_bounds__(256) gemm_edge_backward_kernel(const GemmArgs 
 template <int BM, int BN, bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
 int launch_edge_tile(const GemmArgs& in, hipStream_t stream) {
   GemmArgs g = in;
-  constexpr int COLS = EPI == EPI_SWIGLU ? BN / 2 : BN;   // output columns of a tile
   g.tiles_m = (int)ceil_div(g.M, BM);
-  g.tiles_n = (int)ceil_div(g.N, COLS);
+  g.tiles_n = (int)ceil_div(g.N, BN);
   const long long nwg = (long long)g.tiles_m * g.tiles_n * (g.splits > 1 ? g.splits : 1);
   if (nwg > 0x7fffffffLL) {
     set_error("gemm: too many output tiles (%lld)", nwg);
@@ -73,7 +72,6 @@ int launch_edge_kind(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
       g1.N = (int)n1;
       g2.N = g.N - (int)n1;
       g2.B = BKM ? g.B + n1 * g.ldb : g.B + n1;
-      if (g.B2 != nullptr) g2.B2 = BKM ? g.B2 + n1 * g.ldb : g.B2 + n1;
       g2.C = (char*)g.C + n1 * esz;
       g2.bias = bias_at(g, n1);
       if (g.Z != nullptr) g2.Z = g.Z + n1;
@@ -82,7 +80,6 @@ int launch_edge_kind(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
       g1.M = (int)m1;
       g2.M = g.M - (int)m1;
       g2.A = AK ? g.A + m1 * g.lda : g.A + m1;
-      if (g.A2 != nullptr) g2.A2 = AK ? g.A2 + m1 * g.lda : g.A2 + m1;
       g2.C = (char*)g.C + m1 * g.ldc * esz;
       if (g.Z != nullptr) g2.Z = g.Z + m1 * g.ldc;
     }

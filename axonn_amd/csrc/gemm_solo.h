@@ -1,6 +1,6 @@
 // Device code of the one-wave-per-SIMD MFMA GEMM kernels (solo_gemm), shared by the
 // translation units that instantiate it: gemm_bf16.hip (shapes made of whole tiles) and
-// gemm_edge.hip (every other shape).
+// gemm_edge_bf16.hip, gemm_edge_f16.hip (every other shape).
 #pragma once
 #include <atomic>
 #include <utility>
@@ -409,6 +409,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   // Two-term product: stages 0 .. k_first / 64 - 1 copy from (A, B), the others from
   // (A2, B2); everything behind the copies is unchanged.
   constexpr bool PAIR = EPI == EPI_PAIR;
+  static_assert(!EDGE || (!SWIGLU && !PAIR), "whole tiles only");
   static_assert(!PAIR || (A_KMAJOR && !B_KMAJOR), "the two-term product is the dgrad layout");
   static_assert(!SWIGLU || (BM == 256 && BN == 256 && A_KMAJOR && B_KMAJOR && !OUT_F32),
                 "the gate/up forward runs on the 256 x 256 tile with contraction-contiguous operands");
@@ -454,7 +455,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
       __builtin_amdgcn_make_buffer_rsrc((void*)(SWIGLU ? g.B2 : g.B), 0, (int)b_bytes, 0x00020000);
   // the pair the copies read from (PAIR only: switched once, two stages before the
   // first stage of the second pair)
-  __amdgpu_buffer_rsrc_t ra_cur = ra_rsrc, rb_cur = rb_rsrc, rb2_cur = rb2_rsrc;
+  __amdgpu_buffer_rsrc_t ra_cur = ra_rsrc, rb_cur = rb_rsrc;
   uint32_t a_is = 0, b_is = 0, va = 0, vb = 0;   // per-lane copy offsets of the current tile
   const uint32_t a_step = (uint32_t)((A_KMAJOR ? (int64_t)PK : (int64_t)PK * g.lda) * 2);
   const uint32_t b_step = (uint32_t)((B_KMAJOR ? (int64_t)PK : (int64_t)PK * g.ldb) * 2);
@@ -464,28 +465,26 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   // EDGE: where the next A / B tile to copy starts and how many bytes of the operand lie
   // behind that point.
   struct Walk {
-    const char* at[2];   // [1]: the up weights of the gate/up forward
+    const char* at;
     int64_t left, step;
-    __device__ __forceinline__ void start(const uint16_t* base, const uint16_t* base2, bool kmajor,
-                                          int rows, int kc, int64_t ld, int row0, int k0) {
+    __device__ __forceinline__ void start(const uint16_t* base, bool kmajor, int rows, int kc, int64_t ld, int row0,
+                                          int k0) {
       const int64_t first = kmajor ? row0 * ld + k0 : k0 * ld + row0;
       // a row's last 8 elements are copied together: up to 7 of them are padding of the operand's rows
       const int64_t all = kmajor ? (int64_t)(rows - 1) * ld + ceil_div(kc, 8) * 8 : (int64_t)(kc - 1) * ld + ceil_div(rows, 8) * 8;
-      at[0] = (const char*)(base + first);
-      at[1] = base2 != nullptr ? (const char*)(base2 + first) : at[0];
+      at = (const char*)(base + first);
       left = (all - first) * 2;
       step = (kmajor ? (int64_t)PK : (int64_t)PK * ld) * 2;
     }
     // (left is positive: only stages that exist are copied; its halves are looked at one by
     // one because there is no scalar 64-bit order comparison)
-    __device__ __forceinline__ __amdgpu_buffer_rsrc_t resource(int which) const {
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t resource() const {
       const uint32_t lo = (uint32_t)left;
       const uint32_t n = (uint32_t)(left >> 32) != 0u || lo > 0x7fffffffu ? 0x7fffffffu : lo;
-      return __builtin_amdgcn_make_buffer_rsrc((void*)at[which], 0, (int)n, 0x00020000);
+      return __builtin_amdgcn_make_buffer_rsrc((void*)at, 0, (int)n, 0x00020000);
     }
     __device__ __forceinline__ void advance() {
-      at[0] += step;
-      if (SWIGLU) at[1] += step;
+      at += step;
       left -= step;
     }
   };
@@ -512,8 +511,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   auto copy_b = [&](auto c_) {
     constexpr int I = decltype(c_)::value;
     if constexpr (EDGE) {
-      constexpr int IO = SWIGLU ? 2 * (I / 4) + I % 2 : I;   // as below
-      OB::template dma_one<I, IO>(SWIGLU && I % 4 >= 2 ? rb2_cur : rb_cur, vb, 0, b_is, lds + wslot, wave);
+      OB::template dma_one<I>(rb_cur, vb, 0, b_is, lds + wslot, wave);
     } else if constexpr (SWIGLU) {
       // copies 4 h + {0, 1} of a half h bring 64 gate rows, 4 h + {2, 3} the 64 up rows
       // with the same indices: both are rows 64 h + 32 (I % 2) .. of their matrix
@@ -528,7 +526,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   auto a_done = [&]() {
     if constexpr (EDGE) {
       walk_a.advance();
-      ra_cur = walk_a.resource(0);
+      ra_cur = walk_a.resource();
     } else {
       ka += a_step;
     }
@@ -537,8 +535,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   auto b_done = [&]() {
     if constexpr (EDGE) {
       walk_b.advance();
-      rb_cur = walk_b.resource(0);
-      if constexpr (SWIGLU) rb2_cur = walk_b.resource(1);
+      rb_cur = walk_b.resource();
     } else {
       kb += b_step;
     }
@@ -634,11 +631,10 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
 
   uint32_t va_end = 0, vb_end = 0;   // EDGE: the copy offsets of the operand's last stage
   if constexpr (EDGE) {
-    walk_a.start(g.A, nullptr, A_KMAJOR, g.M, PAIR ? g.k_first : g.Kc, g.lda, m0, s0 * PK);
-    walk_b.start(g.B, SWIGLU ? g.B2 : nullptr, B_KMAJOR, g.N, PAIR ? g.k_first : g.Kc, g.ldb, n0, s0 * PK);
-    ra_cur = walk_a.resource(0);
-    rb_cur = walk_b.resource(0);
-    if constexpr (SWIGLU) rb2_cur = walk_b.resource(1);
+    walk_a.start(g.A, A_KMAJOR, g.M, g.Kc, g.lda, m0, s0 * PK);
+    walk_b.start(g.B, B_KMAJOR, g.N, g.Kc, g.ldb, n0, s0 * PK);
+    ra_cur = walk_a.resource();
+    rb_cur = walk_b.resource();
     va = OA::dma_offset(g.lda, 0, wave, lane, a_is);
     vb = OB::dma_offset(g.ldb, 0, wave, lane, b_is);
     va_end = va;
@@ -692,17 +688,10 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
     const uint32_t b2_bytes = (uint32_t)((int64_t)(g.Kc - g.k_first) * g.ldb * 2);
     for (int p = 0; p < KP - 2; ++p) {
       if (p == kp1 - 2) {  // this stage copies the tiles of stage kp1, the second pair's first
-        if constexpr (EDGE) {
-          walk_a.start(g.A2, nullptr, true, g.M, g.Kc - g.k_first, g.lda, m0, 0);
-          walk_b.start(g.B2, nullptr, false, g.N, g.Kc - g.k_first, g.ldb, n0, 0);
-          ra_cur = walk_a.resource(0);
-          rb_cur = walk_b.resource(0);
-        } else {
-          ra_cur = __builtin_amdgcn_make_buffer_rsrc((void*)g.A2, 0, (int)a_bytes, 0x00020000);
-          rb_cur = __builtin_amdgcn_make_buffer_rsrc((void*)g.B2, 0, (int)b2_bytes, 0x00020000);
-          ka = 0;
-          kb = 0;
-        }
+        ra_cur = __builtin_amdgcn_make_buffer_rsrc((void*)g.A2, 0, (int)a_bytes, 0x00020000);
+        rb_cur = __builtin_amdgcn_make_buffer_rsrc((void*)g.B2, 0, (int)b2_bytes, 0x00020000);
+        ka = 0;
+        kb = 0;
       }
       stage(T{}, F{});
     }
@@ -743,7 +732,6 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
         const f32x4 ul = acc[i][2 * t + FRN / 2], uh = acc[i][2 * t + 1 + FRN / 2];
         const float vg[8] = {gl[0], gl[1], gl[2], gl[3], gh[0], gh[1], gh[2], gh[3]};
         const float vu[8] = {ul[0], ul[1], ul[2], ul[3], uh[0], uh[1], uh[2], uh[3]};
-        if (EDGE && (orow + 16 * i >= g.M || hcol + 32 * t >= g.N)) continue;
         store_swiglu8<HALF>(vg, vu, g, orow + 16 * i, hcol + 32 * t);
       }
   } else {

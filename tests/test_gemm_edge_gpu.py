@@ -194,6 +194,33 @@ def backward(M, N, K, dtype=torch.bfloat16):
                            nv.dtype_code(dtype), M, N, K, N, K, K, K, K, 0, nv.dtype_code(dtype), nv.current_stream())
 
 
+@pytest.mark.parametrize("M,N,K", [(2210, 2160, 2088), (3001, 10240, 2560),   # one of either order: the weight
+                                   (1402, 2056, 4024), (3783, 2520, 3208)])   # gradient's tiles longer, or not
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_both_gradients_of_a_ragged_shape_in_one_launch(M, N, K, dtype):
+    """Workgroups of both products side by side: exact, inside their views, equal to the separate calls."""
+    names = launches(backward(M, N, K, dtype))
+    assert len(names) == 1 and "gemm_edge_backward_kernel" in names[0][0], "this shape is meant to go together"
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    dY, W, X = (numbers(r, c, dtype, gen, 16) for r, c in ((M, N), (N, K), (M, K)))
+    code, ld, stream = nv.dtype_code(dtype), lambda t: t.stride(0), nv.current_stream()
+    sfx = "" if dtype == torch.bfloat16 else "_f16"
+    want_dx, want_dw = dY.double() @ W.double(), dY.double().t() @ X.double()
+    for out, beta in ((dtype, 0), (dtype, 1), (torch.float32, 0), (torch.float32, 1)):
+        fullx, dx = canvas(M, K, dtype)
+        fullw, dw = canvas(N, K, out)
+        dw.fill_(3.0)
+        nv.call("axn_gemm_bwd", nv.ptr(dY), nv.ptr(W), nv.ptr(X), nv.ptr(dx), nv.ptr(dw), code, M, N, K, ld(dY),
+                ld(W), ld(X), ld(dx), ld(dw), beta, nv.dtype_code(out), stream)
+        alone_x, alone_w = torch.empty(M, K, dtype=dtype, device="cuda"), torch.full((N, K), 3.0, dtype=out, device="cuda")
+        nv.call("axn_gemm_dgrad" + sfx, nv.ptr(dY), nv.ptr(W), nv.ptr(alone_x), M, N, K, ld(dY), ld(W), K, stream)
+        nv.call("axn_gemm_wgrad" + sfx, nv.ptr(dY), nv.ptr(X), nv.ptr(alone_w), M, N, K, ld(dY), ld(X), K, beta,
+                nv.dtype_code(out), stream)
+        assert torch.equal(dx, alone_x) and torch.equal(dw, alone_w)
+        check(fullx, dx, want_dx)
+        check(fullw, dw, want_dw + 3.0 * beta)
+
+
 def test_a_shape_is_planned_alike_whatever_was_asked_before():
     """Two ragged shapes with the same numbers of tiles and stages, one of them better in one launch: the plan
     that a thread keeps for the first is not taken for the second."""

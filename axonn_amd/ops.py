@@ -91,7 +91,7 @@ def _gemm_any_n(op, a, b, out, M, N, K, bias=None, z=None, epilogue=nv.EPI_NONE,
     """axn_gemm_any_n; a and b in the order of the product, dY from `_pad_rows`."""
     a, lda = _prep_bf16(a)
     b, ldb = _prep_bf16(b)
-    # the forward with an fp32 result has no split kernel for it elsewhere either
+    # (a forward with an fp32 result, autocast's, could be divided too; its times are not measured)
     split = op != GEMM_FWD or out.dtype == a.dtype
     ws, ws_bytes = _split_workspace(op, M, N, K, a.device) if split else (None, 0)
     nv.call("axn_gemm_any_n", op, nv.ptr(a), nv.ptr(b), nv.ptr(bias), nv.ptr(out), nv.ptr(z),

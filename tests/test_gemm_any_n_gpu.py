@@ -4,6 +4,9 @@ bits, and nothing written behind the outputs."""
 import pytest
 import torch
 
+from axonn_amd import _native as nv
+from launches import launches
+
 pytestmark = pytest.mark.gpu
 
 
@@ -50,8 +53,6 @@ def test_products_against_64_bits(M, N, K, dtype):
 
 def test_forward_leaves_the_neighbours_alone():
     """Y at an odd row stride inside a larger buffer: the elements between its rows stay."""
-    from axonn_amd import _native as nv
-
     M, N, K, ld = 300, 1003, 128, 1007
     X, W = (torch.randn(n, K, device="cuda").bfloat16() for n in (M, N))
     buf = torch.full((M * ld + 64,), 7.0, device="cuda").bfloat16()
@@ -67,9 +68,6 @@ def test_forward_leaves_the_neighbours_alone():
 def test_forward_of_whole_tiles_at_odd_row_strides(M, N, K, out_f32):
     """Rows of Y that start anywhere are stored by kernels that do not take them for 16-byte aligned, whatever
     the shape: streamed, each tile size, full rounds and a rest, a contraction in parts.  Exact whole numbers."""
-    from axonn_amd import _native as nv
-    from launches import launches
-
     g = torch.Generator(device="cuda").manual_seed(M)
     X, W = (torch.randint(-2, 3, (n, K), generator=g, device="cuda").bfloat16() for n in (M, N))
     b = torch.randint(-3, 4, (N,), generator=g, device="cuda").float()
@@ -90,6 +88,36 @@ def test_forward_of_whole_tiles_at_odd_row_strides(M, N, K, out_f32):
             assert "edge_kernel" in last or "stream_kernel" in last or last.endswith("Lb1EEEvPKfNS_8GemmArgsE"), names
         assert torch.equal(buf[:M * ld].view(M, ld)[:, :N].double(), want.to(dtype).double())
         assert bool((buf[:M * ld].view(M, ld)[:, N:] == 7).all()) and bool((buf[M * ld:] == 7).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 512, 4096), (129, 392, 4104), (300, 1001, 4096), (64, 520, 8192)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("narrow", [False, True])
+def test_fp32_results_of_a_contraction_in_parts(M, N, K, dtype, narrow):
+    """The pass that adds the parts with an fp32 result: bias (fp32 or of the operands' type), GELU with the
+    pre-activation kept.  Whole numbers: sums are exact, GELU within the erf's 1.5e-7."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    X, W = (torch.randint(-2, 3, (n, K), generator=g, device="cuda").to(dtype) for n in (M, N))
+    b = torch.randint(-3, 4, (N,), generator=g, device="cuda").to(dtype if narrow else torch.float32)
+    nbytes = nv.load().axn_gemm_workspace_bytes(0, M, N, K)
+    assert nbytes > 0, "this shape is meant to be split"
+    ws = torch.full((nbytes // 4 + 8,), float("nan"), device="cuda")
+    y, z = torch.empty(M, N, device="cuda"), torch.empty(M, N, dtype=dtype, device="cuda")
+    pre = X.double() @ W.double().t() + b.double()
+    for epi in (nv.EPI_BIAS, nv.EPI_BIAS_GELU):
+        def forward():
+            nv.call("axn_gemm_any_n", 0, nv.ptr(X), nv.ptr(W), nv.ptr(b), nv.ptr(y), nv.ptr(z), nv.dtype_code(dtype), M,
+                    N, K, K, K, N, epi | (nv.BIAS_16BIT if narrow else 0), 0, nv.F32, nv.ptr(ws), nbytes,
+                    nv.current_stream())
+
+        assert "splitk_reduce_kernel" in launches(forward)[-1][0]
+        if epi == nv.EPI_BIAS:
+            assert torch.equal(y.double(), pre)
+        else:
+            want = torch.nn.functional.gelu(pre)
+            assert bool(((y.double() - want).abs() <= 2.0 ** -23 * want.abs() + 2e-7 * pre.abs().clamp(min=1)).all())
+            assert torch.equal(z, pre.to(dtype))
+    assert bool(torch.isnan(ws[nbytes // 4:]).all()), "written behind the workspace"
 
 
 @pytest.mark.parametrize("M,N,ld", [(1, 1, 1), (3, 17, 17), (5, 24, 31), (70, 1003, 1005)])

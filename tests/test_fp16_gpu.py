@@ -3,7 +3,7 @@ is fp16 autocast under a loss scaler) with the CPU oracle, through the C ABI.
 
 The half GEMMs are the bf16 kernels with another MFMA mnemonic and another conversion
 in the epilogue, so the tests walk each kernel (256- and 128-wide tiles of the
-one-wave-per-SIMD kernel, the register-staged kernel with and without edges), each
+one-wave-per-SIMD kernel, the same with bounds, the stream over the weights), each
 storage order and each epilogue once more.  Tolerance: fp16 keeps 11 significant bits,
 so against the float64 oracle on the same fp16 inputs the final rounding leaves about
 3e-4 normwise; the bar is 1e-3 (ten times tighter than the bf16 bar), 1e-5 with an fp32
@@ -41,7 +41,7 @@ def half_inputs(M, N, K, seed, x_std=1.0, w_std=0.02, g_std=1e-2):
 
 
 SHAPES = [
-    (32, 64, 64), (100, 72, 40), (1, 8, 16), (257, 264, 72),      # register-staged, ragged
+    (32, 64, 64), (100, 72, 40), (1, 8, 16), (257, 264, 72),      # few tokens, ragged
     (128, 128, 64), (256, 384, 192), (512, 1024, 1024),           # 128-wide tiles
     (4096, 3072, 128), (2304, 4096, 320),                         # 256-wide tiles
 ]

@@ -88,7 +88,7 @@ def test_fused_epilogues_match_oracle(M, N, K, epilogue):
 def test_forward_with_fp32_result_matches_oracle(M, N, K, epilogue, dtype):
     """The forward whose sum with the fp32 bias stays fp32 (what type promotion makes of the
     reference's `x + bias` under autocast): only fp32 accumulation error is left, on every
-    tile shape (register-staged, 128 x 128, whole rounds of 256 x 256 plus a rest)."""
+    kernel (streamed, with bounds, 128 x 128, whole rounds of 256 x 256 plus a rest)."""
     from axonn_amd import ops
 
     g = torch.Generator().manual_seed(M + N + K)

@@ -281,10 +281,12 @@ __global__ void __launch_bounds__(64 * WAVES)
 // per 4).  Error against 64 bits, normal operands, native / this: contraction of 128 2.0e-7 / 6.6e-8,
 // 1024 5.7e-7 / 1.9e-7, 4096 (native by four waves) 5.7e-7 / 4.0e-7; in one accumulator 4096 has 1.0e-6.
 //
-// A result that is one product (a row with one non-zero element) misses the three dropped products: at
-// most 1.7 x 2^-24 off, the native one 1.0 x 2^-24; with two more of the three it is 1.0 again and the kernel
-// 16 to 22 % slower (2048 x 1024, contraction 4096: 97 us, 111), which sums, nearer to exact as they are, do
-// not pay for.
+// Results that are one or two products (rows with as many non-zero elements) miss what the dropped products
+// hold: against 64 bits, in 2^-24 of the sum of the magnitudes, native / this: one product 1.0 / 1.7 at most
+// and 0.424 / 0.435 rms, two 2.0 / 2.7 and 0.521 / 0.537; from three on the native instruction's rounding of
+// every product weighs more (rms of 3 0.602 / 0.585, of 8 0.902 / 0.642, of 64 2.40 / 0.86).  With two more of
+// the three products one is 1.0 again and the kernel 16 to 22 % slower (2048 x 1024, contraction 4096: 97 us,
+// 111), which dense sums, nearer to exact as they are, do not pay for.
 //
 // What three bf16 numbers cannot carry, and where the native products (direct_tile) take over, wave by wave:
 //   * an infinity has no remainder, the largest floats round to one, and partial products far below the

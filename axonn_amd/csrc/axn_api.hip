@@ -301,6 +301,16 @@ size_t axn_gemm_workspace_bytes(int op, int64_t M, int64_t N, int64_t K) {
   return partial_bytes(gemm_splits(kLayoutOfOp[op], g.M, g.N, g.Kc), g);
 }
 
+// Whether axn_gemm_*_ws refuse a workspace that is too small or misaligned instead of running the plain
+// GEMM: the products that were the first to be divided.
+static bool refuses_small_workspace(GemmLayout layout, const GemmArgs& g, int epilogue) {
+  const int64_t tiles = (int64_t)(g.M / 128) * (g.N / 128);
+  const bool few = tiles <= 128 || (g.M % 256 == 0 && tiles <= 256);
+  const bool small = (int64_t)(layout == GEMM_TN ? g.Kc : g.M) * g.lda < (1LL << 30) &&
+                     (int64_t)(layout == GEMM_NT ? g.N : g.Kc) * g.ldb < (1LL << 30);
+  return epilogue == AXN_EPI_NONE && g.M % 128 == 0 && g.N % 128 == 0 && g.Kc % 128 == 0 && few && small;
+}
+
 static int gemm_ws(const char* name, int op, const void* a, const void* b, void* c, int dtype,
                    int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int beta,
                    int out_dtype, void* workspace, size_t workspace_bytes, void* stream,
@@ -327,13 +337,11 @@ static int gemm_ws(const char* name, int op, const void* a, const void* b, void*
   if (plan.parts > 1) {
     const size_t need = partial_bytes(plan, g);
     const bool given = workspace_bytes >= need && aligned16(workspace);
-    // an epilogue or a ragged shape: the plain GEMM, as before such products were divided
-    const bool may_do_without =
-        epilogue != AXN_EPI_NONE || g.M % 128 != 0 || g.N % 128 != 0 || g.Kc % 64 != 0;
-    if (!given && may_do_without) plan.parts = 1;
-    REQUIRE(given || may_do_without || workspace_bytes >= need, AXN_EINVAL,
+    const bool refused = refuses_small_workspace(layout, g, epilogue);
+    if (!given && !refused) plan.parts = 1;
+    REQUIRE(given || !refused || workspace_bytes >= need, AXN_EINVAL,
             "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
-    REQUIRE(given || may_do_without, AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+    REQUIRE(given || !refused, AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
   }
   if (plan.parts > 1)
     return launch_gemm_splitk(layout, g, epilogue, half, out_dtype == AXN_F32, plan, (float*)workspace,

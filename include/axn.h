@@ -164,9 +164,10 @@ AXN_API int axn_gemm_fwd_f32out(const void* X, const void* W, const float* bias,
  *   AXN_F16) of the 16-bit operands and results, and the workspace (16-byte aligned, used
  *   by this call alone until it has finished; contents need not be initialised).
  *   workspace == NULL, or a shape that does not profit: the call is the plain GEMM.  A
- *   workspace that is too small is AXN_EINVAL, a misaligned one AXN_EALIGN, for a product of
- *   whole 128 x 128 tiles and 64-deep stages without an epilogue; with an epilogue or a
- *   ragged shape the call is then the plain GEMM. */
+ *   workspace that is too small is AXN_EINVAL, a misaligned one AXN_EALIGN, for a product
+ *   without an epilogue of whole 128 x 128 tiles, at most 128 of them or of 256 x 128 ones,
+ *   over a contraction that is a multiple of 128, with operands below 2 GiB; otherwise the
+ *   call is then the plain GEMM. */
 typedef enum axn_gemm_op { AXN_GEMM_FWD = 0, AXN_GEMM_DGRAD = 1, AXN_GEMM_WGRAD = 2 } axn_gemm_op;
 AXN_API size_t axn_gemm_workspace_bytes(int op, int64_t M, int64_t N, int64_t K);
 AXN_API int axn_gemm_fwd_ws(const void* X, const void* W, const float* bias, void* Y, void* Zsave,

@@ -236,3 +236,22 @@ def test_a_shape_is_planned_alike_whatever_was_asked_before():
         t.join()
     assert found[0, 1] == found[1, 0][::-1]
     assert [len(f) for f in found[0, 1]] != [1, 1], "the second is meant to differ from the first"
+
+
+@pytest.mark.parametrize("op,M,N,K", [(0, 256, 512, 4160), (1, 128, 8896, 256), (2, 4160, 256, 384),   # an odd number of stages
+                                      (0, 640, 3584, 8192)])                                         # 140 tiles
+def test_a_workspace_too_small_for_whole_tiles_that_do_not_halve_or_are_many(op, M, N, K):
+    """The plain GEMM, bit for bit."""
+    assert nv.load().axn_gemm_workspace_bytes(op, M, N, K) > 64
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    rows = {0: ((M, K), (N, K), (M, N)), 1: ((M, N), (N, K), (M, K)), 2: ((M, N), (M, K), (N, K))}[op]
+    a, b = (torch.randn(s, generator=gen, device="cuda").bfloat16() for s in rows[:2])
+    ws = torch.zeros(64, dtype=torch.uint8, device="cuda")
+    got, want = (torch.empty(rows[2], dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    name, none, last = {0: ("axn_gemm_fwd", (None,), (nv.EPI_NONE,)), 1: ("axn_gemm_dgrad", (), ()),
+                        2: ("axn_gemm_wgrad", (), (0, nv.BF16))}[op]
+    dims = (M, N, K, a.shape[1], b.shape[1], rows[2][1])
+    nv.call(name + "_ws", nv.ptr(a), nv.ptr(b), *none, nv.ptr(got), *none, nv.BF16, *dims, *last, nv.ptr(ws), 64,
+            nv.current_stream())
+    nv.call(name, nv.ptr(a), nv.ptr(b), *none, nv.ptr(want), *none, *dims, *last, nv.current_stream())
+    assert torch.equal(got, want)

@@ -383,8 +383,11 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void*
   const bool half = dtype == AXN_F16, out_f32 = out_dtype == AXN_F32;
   const GemmLayout layout = kLayoutOfOp[op];
   const bool near = lda < kEdgeMaxLd / 2 && ldb < kEdgeMaxLd / 2;
-  const SplitPlan plan =
+  SplitPlan plan =
       workspace != nullptr && near ? gemm_splits(layout, g.M, g.N, g.Kc) : SplitPlan{1, EDGE_128x128};
+  // (forwards of a few rows were streams whatever the workspace)
+  if (fwd && M <= kStreamMaxRows && (workspace_bytes < partial_bytes(plan, g) || !aligned16(workspace)))
+    plan.parts = 1;
   if (plan.parts > 1) {
     const size_t need = partial_bytes(plan, g);
     REQUIRE(workspace_bytes >= need, AXN_EINVAL,

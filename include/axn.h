@@ -189,7 +189,8 @@ AXN_API int axn_gemm_wgrad_ws(const void* dY, const void* X, void* dW, int dtype
  *   DGRAD, WGRAD   dY rows of lda elements, a multiple of 8; what lies behind column N up to the next
  *          multiple of 8 must be zero (axn_pad_rows16)
  * K, the other leading dimensions and pointers: as above.  workspace: axn_gemm_workspace_bytes(op,
- * M, N, K) bytes, or NULL for no split; beta and an fp32 out_dtype as axn_gemm_wgrad. */
+ * M, N, K) bytes, or NULL for no split (less or misaligned is refused, for a forward of up to 64 rows
+ * no split either); beta and an fp32 out_dtype as axn_gemm_wgrad. */
 #define AXN_BIAS_16BIT 0x100 /* with the epilogue: bias is of `dtype` instead of fp32 */
 AXN_API int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void* C,
                    void* Zsave, int dtype, int64_t M, int64_t N, int64_t K, int64_t lda,

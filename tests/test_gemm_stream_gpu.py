@@ -60,3 +60,18 @@ def test_few_tokens_are_exact(M, N, K, dtype):
     eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     assert bool(((y.double() - want).abs() <= eps * want.abs() + 2e-7 * pre.abs().clamp(min=1)).all())
     check(fz, z, pre)
+
+
+@pytest.mark.parametrize("M,N,K", [(32, 512, 28672), (16, 64, 14336), (64, 512, 5120)])
+@pytest.mark.parametrize("nbytes,offset", [(16, 0), (1 << 24, 4)])
+def test_a_workspace_too_small_or_misaligned_for_parts(M, N, K, nbytes, offset):
+    """Streamed, as without one, bit for bit, and the workspace is left alone."""
+    assert nv.load().axn_gemm_workspace_bytes(0, M, N, K) > 16
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    X, W = (torch.randn(r, K, generator=gen, device="cuda").bfloat16() for r in (M, N))
+    ws = torch.full((nbytes + 16,), 7, dtype=torch.uint8, device="cuda")
+    got, want = (torch.empty(M, N, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    for out, where, size in ((got, ws.data_ptr() + offset, nbytes), (want, None, 0)):
+        nv.call("axn_gemm_any_n", 0, nv.ptr(X), nv.ptr(W), None, nv.ptr(out), None, nv.BF16, M, N, K, K, K, N,
+                nv.EPI_NONE, 0, nv.BF16, where, size, nv.current_stream())
+    assert torch.equal(got, want) and bool((ws == 7).all())

@@ -107,11 +107,11 @@ __device__ __forceinline__ void clear(f32x4 (&acc)[FM][FN]) {
 }
 
 // acc[i][j] += the products of contraction indices [k_begin, k_end) for rows arow + i and columns
-// bcol + j of the lane, in fp32 MFMAs; this wave takes the 16 U-deep chunks first, first + step, ...
-template <bool AK, bool BKM, int FM, int FN, int U, bool VEC>
+// bcol + j of the lane, in fp32 MFMAs; this wave takes the 16 U-deep chunks first, first + STEP, ...
+template <bool AK, bool BKM, int FM, int FN, int U, bool VEC, int STEP>
 __device__ __forceinline__ void direct_tile(f32x4 (&acc)[FM][FN], const float* __restrict__ A,
                                             const float* __restrict__ B, int arow, int bcol, int M, int N,
-                                            int Kc, int k_begin, int k_end, int first, int step) {
+                                            int Kc, int k_begin, int k_end, int first) {
   const int q = (threadIdx.x & 63) >> 4;
   auto blocks = [&](auto guard_, int k0, auto nblk_) {
     constexpr bool GUARD = decltype(guard_)::value;
@@ -134,11 +134,16 @@ __device__ __forceinline__ void direct_tile(f32x4 (&acc)[FM][FN], const float* _
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i][s], b[u][j][s], acc[i][j], 0, 0, 0);
   };
   const int whole = k_begin + (k_end - k_begin) / (16 * U) * (16 * U);  // the part made of whole chunks
-  // (unsigned: past the end of the longest contraction an int overflows)
-  for (unsigned k0 = k_begin + first * 16 * U; k0 < (unsigned)whole; k0 += step * 16 * U)
-    blocks(std::false_type{}, (int)k0, std::integral_constant<int, U>{});
-  for (unsigned k0 = whole + first * 16; k0 < (unsigned)k_end; k0 += step * 16)
-    blocks(std::true_type{}, (int)k0, std::integral_constant<int, 1>{});
+  // (left by a difference: past the end of the longest contraction an int overflows, and with unsigned or
+  // counted chunks the compiler keeps fewer loads in flight)
+  for (int k0 = k_begin + first * 16 * U; k0 < whole; k0 += STEP * 16 * U) {
+    blocks(std::false_type{}, k0, std::integral_constant<int, U>{});
+    if (whole - k0 <= STEP * 16 * U) break;
+  }
+  for (int k0 = whole + first * 16; k0 < k_end; k0 += STEP * 16) {
+    blocks(std::true_type{}, k0, std::integral_constant<int, 1>{});
+    if (k_end - k0 <= STEP * 16) break;
+  }
 }
 
 // Whether the lane's operands hold a non-zero number under `bound`.
@@ -249,7 +254,7 @@ __global__ void __launch_bounds__(64 * WAVES)
   clear(acc);
   // Rows and columns past the edge read a valid one: their products land in output
   // elements that are never stored.
-  direct_tile<AK, BKM, FM, FN, U, VEC>(acc, A, B, m0 + FM * r, n0 + FN * r, M, N, Kc, 0, Kc, wave, WAVES);
+  direct_tile<AK, BKM, FM, FN, U, VEC, WAVES>(acc, A, B, m0 + FM * r, n0 + FN * r, M, N, Kc, 0, Kc, wave);
 
   if constexpr (WAVES > 1) {
     __shared__ f32x4 part[WAVES - 1][FM * FN][64];
@@ -419,8 +424,8 @@ __global__ void __launch_bounds__(256, 2)
   const int part = blockIdx.x / tiles, id = blockIdx.x - part * tiles;
   const int tm = id / tiles_n, tn = id - tm * tiles_n;
   const int m0 = tm * 32 * FM, n0 = tn * 32 * FN;
-  // (unsigned: past the end of the longest contraction an int overflows)
-  const unsigned k_begin = part * k_part, k_end = min((unsigned)Kc, k_begin + k_part);
+  // (differences: past the end of the longest contraction an int overflows)
+  const int k_begin = part * k_part, k_end = Kc - k_begin < k_part ? Kc : k_begin + k_part;
   C += (int64_t)part * M * N;
 
   f32x4 acc[FM][FN], low[FM][FN];
@@ -431,8 +436,8 @@ __global__ void __launch_bounds__(256, 2)
   my_share<BKM>(gb, qb);
   float xa[FM][4], xb[FN][4];
   // Rows past the edge read a valid one, indices past the end count as zero.
-  auto fetch = [&](unsigned k0) {
-    if (k0 + 32 <= k_end) {
+  auto fetch = [&](int k0) {
+    if (k_end - k0 >= 32) {
       load_block<AK, FM, VEC, false>(xa, A, m0 + FM * ga, M, k0 + 4 * qa, Kc, k_end);
       load_block<BKM, FN, VEC, false>(xb, B, n0 + FN * gb, N, k0 + 4 * qb, Kc, k_end);
     } else {
@@ -443,14 +448,16 @@ __global__ void __launch_bounds__(256, 2)
   float largest = 0.f;
   if (threadIdx.x == 0) large = 0;
   fetch(k_begin);
-  for (unsigned k0 = k_begin; k0 < k_end; k0 += 32) {
+  for (int k0 = k_begin; k0 < k_end; k0 += 32) {
     put_stage<AK, FM>(la, xa);
     put_stage<BKM, FN>(lb, xb);
     largest = max_magnitude(max_magnitude(largest, xa), xb);
     __syncthreads();
-    if (k0 + 32 < k_end) fetch(k0 + 32);
+    const bool last = k_end - k0 <= 32;
+    if (!last) fetch(k0 + 32);
     split_stage<FM, FN>(acc, low, la, lb);
     __syncthreads();
+    if (last) break;
   }
   if (largest >= 0x1p16f) large = 1;
   __syncthreads();
@@ -476,7 +483,7 @@ __global__ void __launch_bounds__(256, 2)
                                               zeros ? 0x1p-62f : 0x1p-110f);
   if (__builtin_amdgcn_ballot_w64(odd)) {
     clear(acc);
-    direct_tile<AK, BKM, FM, FN, 1, VEC>(acc, A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end, 0, 1);
+    direct_tile<AK, BKM, FM, FN, 1, VEC, 1>(acc, A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end, 0);
   }
   store_tile<EPI, FM, FN, VEC>(acc, C, bias, Z, mw, nw, M, N, beta);
 }

@@ -134,33 +134,52 @@ int launch_rest(const GemmArgs& in, hipStream_t stream) {
 //               workgroup on every CU (9 % of it with none, linear between).
 // The constants were fitted to 3479 launches: every tile size and split of 220 forward and
 // input-gradient problems of 33 to 3000 tokens and 768 to 14336 features, ragged and whole.
-double launch_microseconds(EdgeTile tile, long long w, double stages, double mb) {
-  const double loop = tile == EDGE_256x256   ? (5.1 + 1.084 * stages) * (double)((w + 255) / 256)
-                      : tile == EDGE_256x128 ? (2.5 + 0.737 * stages) * (double)((w + 255) / 256)
-                      : w <= 256             ? 0.69 * stages
-                                             : (1.2 + 0.936 * stages) * (double)((w + 511) / 512);
+// `epilogue`: what the output's epilogue adds to a round, on each of the four.
+struct EpilogueTime {
+  double us[4];
+};
+double launch_microseconds(EdgeTile tile, long long w, double stages, double mb, const EpilogueTime& epilogue = {}) {
+  const double* e = epilogue.us;
+  const double loop = tile == EDGE_256x256   ? (5.1 + 1.084 * stages + e[0]) * (double)((w + 255) / 256)
+                      : tile == EDGE_256x128 ? (2.5 + 0.737 * stages + e[1]) * (double)((w + 255) / 256)
+                      : w <= 256             ? 0.69 * stages + e[2]
+                                             : (1.2 + 0.936 * stages + e[3]) * (double)((w + 511) / 512);
   const double occupied = w >= 256 ? 1.0 : (double)w / 256;
   const double stream = 1.74 + mb / (5.72 * (0.086 + 0.914 * occupied));
   return loop > stream ? loop : stream;
 }
 
+// One wave a SIMD has nothing to run beside its epilogue; two workgroups on a CU have each other's main loop.
+// Bias, or (bias and) GELU, and each of an fp32 result and a saved pre-activation on top.  Fitted with the
+// constants above held, to 2400 ragged forwards of 65 to 8192 rows, 64 to 16384 outputs and contractions of 192
+// to 4096; over 5000 others the pick takes 0.3 % more than the best of the three tiles on average and 30 % at
+// worst (without it 1.6 % and 69 %: 6144 x 2880 x 384 with bias 44 us on the large tile, 35 on the small).
+EpilogueTime epilogue_time(const GemmArgs& g, int epilogue, bool out_f32) {
+  if (epilogue == AXN_EPI_NONE) return {};
+  const bool gelu = epilogue != AXN_EPI_BIAS;
+  EpilogueTime t = gelu ? EpilogueTime{15.5, 7.8, 3.9, 1.4} : EpilogueTime{6.6, 3.3, 1.6, 0.0};
+  const double more[4] = {1.9, 1.1, 0.7, 1.1};
+  for (int i = 0; i < 4; ++i) t.us[i] += more[i] * ((out_f32 ? 1 : 0) + (gelu && g.Z != nullptr ? 1 : 0));
+  return t;
+}
+
 // The same for an unsplit M x N output as launch_edge_kind runs it: a last round of at most
 // half of the CUs goes to smaller tiles.
-double edge_microseconds(EdgeTile tile, long long M, long long N, long long Kc) {
+double edge_microseconds(EdgeTile tile, long long M, long long N, long long Kc, const EpilogueTime& epilogue) {
   const int bm = tile == EDGE_128x128 ? 128 : 256, bn = tile == EDGE_256x256 ? 256 : 128;
   const long long w = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), full = w / 256, rest = w % 256;
   const double stages = (double)((Kc + 63) / 64), mb = ((double)M + (double)N) * (double)Kc * 2e-6;
   if (tile == EDGE_256x256 && full > 0 && rest > 0 && rest <= 128)
-    return launch_microseconds(tile, full * 256, stages, mb) +
-           launch_microseconds(rest <= 64 ? EDGE_128x128 : EDGE_256x128, 256, stages, 0.0) + 3.0;
-  return launch_microseconds(tile, w, stages, mb);
+    return launch_microseconds(tile, full * 256, stages, mb, epilogue) +
+           launch_microseconds(rest <= 64 ? EDGE_128x128 : EDGE_256x128, 256, stages, 0.0, epilogue) + 3.0;
+  return launch_microseconds(tile, w, stages, mb, epilogue);
 }
 
-EdgeTile edge_tile(long long M, long long N, long long Kc, double* us = nullptr) {
+EdgeTile edge_tile(long long M, long long N, long long Kc, const EpilogueTime& epilogue = {}, double* us = nullptr) {
   EdgeTile best = EDGE_256x256;
-  double least = edge_microseconds(best, M, N, Kc);
+  double least = edge_microseconds(best, M, N, Kc, epilogue);
   for (EdgeTile t : {EDGE_256x128, EDGE_128x128}) {
-    const double e = edge_microseconds(t, M, N, Kc);
+    const double e = edge_microseconds(t, M, N, Kc, epilogue);
     if (e < least) {
       least = e;
       best = t;
@@ -174,7 +193,9 @@ int launch_edge(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32
                 hipStream_t stream) {
   const int64_t ld = g.lda > g.ldb ? g.lda : g.ldb;
   if (ld >= kEdgeMaxLd) return launch_gemm_far(layout, g, epilogue, out_f32, half, stream);
-  const EdgeTile tile = ld >= kEdgeMaxLd / 2 ? EDGE_128x128 : edge_tile(g.M, g.N, g.Kc);
+  const EdgeTile tile = ld >= kEdgeMaxLd / 2
+                            ? EDGE_128x128
+                            : edge_tile(g.M, g.N, g.Kc, epilogue_time(g, epilogue, out_f32));
   return half ? launch_gemm_edge_f16(layout, g, epilogue, out_f32, tile, stream)
               : launch_gemm_edge_bf16(layout, g, epilogue, out_f32, tile, stream);
 }
@@ -525,8 +546,8 @@ int launch_backward(const GemmArgs& gd_in, const GemmArgs& gw_in, bool dw_f32, h
     const bool together = plan_together(plans, next_plan, gd.M, gd.N, gd.Kc, 0, [&] {
       if (td + tw > 4096) return false;
       double ud = 0, uw = 0;
-      edge_tile(gd.M, gd.N, gd.Kc, &ud);
-      edge_tile(gw.M, gw.N, gw.Kc, &uw);
+      edge_tile(gd.M, gd.N, gd.Kc, {}, &ud);
+      edge_tile(gw.M, gw.N, gw.Kc, {}, &uw);
       return 1.084 * stages_together(tw, sw, td, sd) + 15 < 0.95 * (ud + uw);
     });
     if (together) {

@@ -255,3 +255,33 @@ def test_a_workspace_too_small_for_whole_tiles_that_do_not_halve_or_are_many(op,
             nv.current_stream())
     nv.call(name, nv.ptr(a), nv.ptr(b), *none, nv.ptr(want), *none, *dims, *last, nv.current_stream())
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,N,K,none,bias,gelu", [(777, 14336, 1032, 256, 256, 128), (1591, 10752, 392, 256, 128, 128),
+                                                  (2001, 4104, 2056, 256, 256, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_the_tile_of_a_ragged_forward_follows_its_epilogue(M, N, K, none, bias, gelu, dtype):
+    """Whole numbers: the product, its sum with the bias and the saved pre-activation are exact on either tile,
+    GELU as above."""
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    X, W = (numbers(r, K, dtype, gen, 16) for r in (M, N))
+    b = torch.randint(-3, 4, (N,), generator=gen, device="cuda").float()
+    product = X.double() @ W.double().t()
+    sfx = "" if dtype == torch.bfloat16 else "_f16"
+    for epi, tile, pre in ((nv.EPI_NONE, none, product), (nv.EPI_BIAS, bias, product + b),
+                           (nv.EPI_BIAS_GELU, gelu, product + b)):
+        fy, y = canvas(M, N, dtype)
+        fz, z = canvas(M, N, dtype)
+        call = lambda: nv.call(   # noqa: E731
+            "axn_gemm_fwd" + sfx, nv.ptr(X), nv.ptr(W), nv.ptr(b) if epi else None, nv.ptr(y),
+            nv.ptr(z) if epi == nv.EPI_BIAS_GELU else None, M, N, K, X.stride(0), W.stride(0), y.stride(0), epi,
+            nv.current_stream())
+        name = launches(call)[0][0]
+        assert "gemm_edge_kernel" in name and ("%d, %d" % (tile, tile) in name or "Li%dELi%dE" % (tile, tile) in name), name
+        if epi == nv.EPI_BIAS_GELU:
+            want = torch.nn.functional.gelu(pre)
+            eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+            assert bool(((y.double() - want).abs() <= eps * want.abs() + 2e-7 * pre.abs().clamp(min=1)).all())
+            check(fz, z, pre)
+        else:
+            check(fy, y, pre)

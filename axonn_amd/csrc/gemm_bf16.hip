@@ -329,7 +329,9 @@ __global__ void __launch_bounds__(256)
       if (col + e < g.N) store_one<EPI, OUT_F32, HALF>(v[e], g, (int)row, (int)col + e);
     return;
   }
-  store_row8<EPI, OUT_F32, HALF, ANY>(v, g, (int)row, (int)col);
+  float bias[8];
+  load_bias8<EPI, HALF>(bias, g, (int)col);
+  store_row8<EPI, OUT_F32, HALF, ANY>(v, bias, g, (int)row, (int)col);
 }
 
 template <bool HALF, bool ANY>

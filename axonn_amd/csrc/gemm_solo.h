@@ -67,32 +67,43 @@ struct Unaligned {
   typedef V type __attribute__((aligned(A)));
 };
 
+// The bias of 8 consecutive columns in fp32; a 16-bit one is widened here: a launch before the product that
+// widens it costs more than the product of a small layer.
+template <int EPI, bool HALF>
+__device__ __forceinline__ void load_bias8(float (&bias)[8], const GemmArgs& g, int col) {
+  using lpx8 = std::conditional_t<HALF, f16x8, bf16x8>;
+  if (EPI != AXN_EPI_BIAS && EPI != AXN_EPI_BIAS_GELU) return;
+  if (g.bias16) {
+    const lpx8 b = *(const lpx8*)((const uint16_t*)g.bias + col);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) bias[e] = (float)b[e];
+  } else {
+    const f32x4 b0 = *(const f32x4*)((const float*)g.bias + col);
+    const f32x4 b1 = *(const f32x4*)((const float*)g.bias + col + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      bias[e] = b0[e];
+      bias[4 + e] = b1[e];
+    }
+  }
+}
+
 // Epilogue of 8 consecutive columns of one output row, held in fp32: bias,
 // exact GELU with optional save of the pre-activation, accumulation into the
 // existing output (beta), conversion and one 16- or 32-byte store.
 // HALF: the 16-bit storage type is IEEE half instead of bfloat16.
 // ANY: rows of C and Z have the alignment of one element (else 16 bytes).
+// bias: the 8 columns', from load_bias8 (a load in here would be repeated for every row, behind the stores).
 template <int EPI, bool OUT_F32, bool HALF, bool ANY = false>
-__device__ __forceinline__ void store_row8(float (&v)[8], const GemmArgs& g, int row, int col) {
+__device__ __forceinline__ void store_row8(float (&v)[8], const float (&bias)[8], const GemmArgs& g, int row, int col) {
   using lp = std::conditional_t<HALF, _Float16, __bf16>;
   using lpx8 = std::conditional_t<HALF, f16x8, bf16x8>;
   using lpx8_mem = typename Unaligned<lpx8, ANY ? 2 : 16>::type;
   using f32x4_mem = typename Unaligned<f32x4, ANY ? 4 : 16>::type;
   const int64_t o = (int64_t)row * g.ldc + col;
   if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU) {
-    if (g.bias16) {   // widened here: a launch before the product that widens it costs more than the product of a small layer
-      const lpx8 b = *(const lpx8*)((const uint16_t*)g.bias + col);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] += (float)b[e];
-    } else {
-      const f32x4 b0 = *(const f32x4*)((const float*)g.bias + col);
-      const f32x4 b1 = *(const f32x4*)((const float*)g.bias + col + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] += b0[e];
-        v[4 + e] += b1[e];
-      }
-    }
+    for (int e = 0; e < 8; ++e) v[e] += bias[e];
   }
   if (EPI == AXN_EPI_BIAS_GELU || EPI == AXN_EPI_GELU) {
     if (g.Z != nullptr) {
@@ -742,6 +753,10 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
     // stored one by one, which keeps that path out of the unrolled stores.  The ring slot
     // behind the last stage's two is free: no wave reads or fills it any more.
     [[maybe_unused]] float* tail = (float*)(lds + sa) + wave * (WTM * 8);
+    float bias[FRN / 2][8];
+#pragma unroll
+    for (int t = 0; t < FRN / 2; ++t)
+      if (!EDGE || ocol + 32 * t + 8 <= g.N) load_bias8<EP, HALF>(bias[t], g, ocol + 32 * t);
 #pragma unroll
     for (int i = 0; i < FRM; ++i)
 #pragma unroll
@@ -758,7 +773,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
             continue;
           }
         }
-        store_row8<EP, OUT_F32, HALF, EDGE>(v, go, row, col);
+        store_row8<EP, OUT_F32, HALF, EDGE>(v, bias[t], go, row, col);
       }
     if constexpr (EDGE) {
       const int end = g.N / 8 * 8, first = n0 + wn * WTN;

@@ -180,16 +180,18 @@ int launch_gemm_edge_backward_f16(const GemmArgs& wgrad, const GemmArgs& dgrad, 
 // below kStreamMaxLd elements.
 constexpr int64_t kStreamMaxRows = 64;
 // Whether it is also ahead of tiles with the contraction in parts.  Those lose on many weights and win where a
-// few workgroups would walk a long contraction; the line lies where they meet over 360 shapes of 1 to 64 rows,
-// 64 to 14336 outputs and contractions of 1024 to 65536 (cold weights; the pick is 0.5 % off the faster one on
-// average, 14 % at worst).  us, stream / tiles:
+// few workgroups would walk a long contraction; the line lies where they meet over 41397 shapes of 1 to 64 rows,
+// 64 to 16384 outputs and contractions of 1024 to 65536 (cold weights, in rows of calls; the pick is 0.2 % off the
+// faster one on average, 39 % at worst).  It moves with the share of the CUs that the stream's workgroups fill:
+// 3072 outputs and more fill three quarters of them.  us, stream / tiles:
 //   64 rows   512 x 4096 12.5 / 11.4    512 x 5120 15.9 / 12.7   4096 x 8192 23.5 / 24.0   4096 x 14336 47 / 37
 //   32 rows   512 x 8192 13.5 / 14.5    512 x 28672 51 / 31      4096 x 28672 66 / 64      8192 x 65536 207 / 232
-//   8 rows    512 x 14336 15.3 / 18.7   512 x 65536 56 / 55      4096 x 65536 84 / 143
+//   15 rows   3904 x 16256 24 / 40      64 x 14144 17.6 / 18.5   64 x 14656 (16 rows) 18.6 / 18.3
+//   8 rows    512 x 14336 15.3 / 18.7   512 x 65536 56 / 55      4032 x 30336 40 / 58      4096 x 65536 84 / 143
 inline bool stream_ahead(int64_t M, int64_t N, int64_t Kc) {
   if (M > kStreamMaxRows) return false;
-  if (N >= 8192 || (N >= 4096 && M <= 32)) return true;
-  return M * Kc <= (N >= 4096 ? 524288 : 196608);
+  if (M <= 8 || N >= 8192 || (N >= 4096 && M <= 32) || (N >= 3072 && M <= 16)) return true;
+  return M * Kc <= (N >= 3072 ? 524288 : 225000);
 }
 constexpr int64_t kStreamMaxLd = 1LL << 24;
 int launch_gemm_stream(const GemmArgs& args, int epilogue, bool out_f32, bool half, hipStream_t stream);

@@ -61,7 +61,8 @@ def test_workspace_queries():
     # few tokens: a stream over the weights, unless a few workgroups would walk a long contraction
     for m, n, k, parts in ((16, 4096, 14336, 0), (32, 4096, 65536, 0), (64, 14336, 14336, 0), (64, 4096, 8192, 0),
                            (64, 512, 2048, 0), (8, 512, 14336, 0), (64, 512, 5120, 1), (32, 512, 28672, 1),
-                           (16, 64, 14336, 1), (64, 4096, 14336, 1)):
+                           (16, 64, 14336, 1), (64, 4096, 14336, 1), (15, 3904, 16256, 0), (8, 1024, 57344, 0),
+                           (14, 3072, 14336, 0), (24, 3584, 14336, 0), (40, 3584, 14336, 1)):
         assert (lib.axn_gemm_workspace_bytes(0, m, n, k) > 0) == bool(parts), (m, n, k)
     # embedding: four int32 arrays over the tokens, one over the rows, and the sort's digit
     # counts (17 key bits = two passes of 9 and 8 bits, one count per digit and 512 tokens)

@@ -190,8 +190,9 @@ constexpr int64_t kStreamMaxRows = 64;
 //   8 rows    512 x 14336 15.3 / 18.7   512 x 65536 56 / 55      4032 x 30336 40 / 58      4096 x 65536 84 / 143
 inline bool stream_ahead(int64_t M, int64_t N, int64_t Kc) {
   if (M > kStreamMaxRows) return false;
-  if (M <= 8 || N >= 8192 || (N >= 4096 && M <= 32) || (N >= 3072 && M <= 16)) return true;
-  return M * Kc <= (N >= 3072 ? 524288 : 225000);
+  if (N >= 8192 || (N >= 4096 && M <= 32) || (N >= 3072 && M <= 16)) return true;
+  if (N >= 3072) return M * Kc <= 524288;
+  return Kc <= 65536 && (M <= 8 || M * Kc <= 225000);
 }
 constexpr int64_t kStreamMaxLd = 1LL << 24;
 int launch_gemm_stream(const GemmArgs& args, int epilogue, bool out_f32, bool half, hipStream_t stream);

@@ -333,7 +333,7 @@ __global__ void __launch_bounds__(64 * SORT_WAVES)
       // equal next digit, and the same unit: the destinations of `same` are consecutive, so they
       // lie in at most two units, one of them odd
       uint64_t joined = same;
-      for (int b = 0; b <= next_bits; ++b) {
+      for (int b = 0; b <= next_bits && __ballot(active) != 0; ++b) {
         const bool bit = ((b < next_bits ? nx >> b : nb) & 1) != 0;
         const uint64_t with = __ballot(active && bit);
         joined &= bit ? with : ~with;
@@ -569,13 +569,14 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
     embedding_bwd_kernel(const int* __restrict__ keys, const int* __restrict__ vals,
                          const int* __restrict__ row_start, const TY* __restrict__ dY, TW* dW,
                          int64_t T, int64_t V, int64_t H, int64_t lddy, int64_t lddw,
-                         int units_per_row, int64_t padding_idx, int scale_by_freq, int beta,
-                         int long_blocks, int pieces_per_row) {
+                         int64_t padding_idx, int units_per_row, int long_blocks, int scale_by_freq,
+                         int beta, int pieces_per_row) {
   constexpr int VEC = 16 / (int)sizeof(TW);
   constexpr int LV = VEC / 2;                              // columns of a lane in a long run's wave
   constexpr int LONG_B = LV * sizeof(TY) > 8 ? 16 : 32;    // its rows in flight: 64 registers
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // (units_per_row and long_blocks lie side by side and come with one load, not with a second one here)
   if ((int)blockIdx.x < long_blocks) {
     const int64_t unit = (int64_t)blockIdx.x * WAVES_PER_BLOCK + wave;
     const int64_t chunk = unit / pieces_per_row * 64;
@@ -614,15 +615,19 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
     return;
   }
   // (the wave's number stays a vector here: row_start read through the scalar cache costs 7 %)
-  // (a 64-bit division would be half of what a wave does for a row without tokens: the quotient
-  // of the workgroup's first unit is the scalar unit's, the rest of its units follow)
+  // (a 64-bit division would be half of what a wave does for a row without tokens.  4 tokens, 146388 x 2240
+  // bf16, beta: 55 us; 61 with the scalar unit's 64-bit quotient of the workgroup's first unit and a loop over its
+  // other units)
   const int64_t unit0 = (int64_t)((int)blockIdx.x - long_blocks) * WAVES_PER_BLOCK;
-  const int64_t row0 = unit0 / units_per_row;
-  int rest = (int)(unit0 - row0 * units_per_row) + (int)(threadIdx.x >> 6);
-  int64_t row = row0;
-  while (rest >= units_per_row) {   // at most WAVES_PER_BLOCK - 1 times
-    rest -= units_per_row;
-    ++row;
+  int64_t row = unit0 + (int)(threadIdx.x >> 6);
+  int rest = 0;
+  if (units_per_row != 1) {   // (rows of up to 1024 fp32 or 2048 16-bit elements need no division)
+    const int64_t unit = row;
+    if (unit0 <= 0x7ffffff0)
+      row = (uint32_t)unit / (uint32_t)units_per_row;
+    else
+      row = unit / units_per_row;
+    rest = (int)(unit - row * units_per_row);
   }
   if (row >= V) return;
   const int64_t col0 = ((int64_t)rest * (U * 64) + lane) * VEC;
@@ -861,8 +866,8 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
   const dim3 grid((unsigned)blocks), block(64 * WAVES_PER_BLOCK);
 #define AXN_EMB_BWD_U(TY, TW, UU)                                                               \
   hipLaunchKernelGGL((embedding_bwd_kernel<TY, TW, UU>), grid, block, EMB_BWD_LDS, stream, keys, vals,    \
-                     w.row_start, (const TY*)dY, (TW*)dW, T, V, H, lddy, lddw, upr, padding_idx, \
-                     scale_by_freq, beta, (int)long_blocks, (int)long_pieces)
+                     w.row_start, (const TY*)dY, (TW*)dW, T, V, H, lddy, lddw, padding_idx, upr, \
+                     (int)long_blocks, scale_by_freq, beta, (int)long_pieces)
 #define AXN_EMB_BWD(TY, TW)                 \
   do {                                      \
     if (U == 4)                             \

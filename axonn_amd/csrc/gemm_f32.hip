@@ -108,7 +108,7 @@ __device__ __forceinline__ void clear(f32x4 (&acc)[FM][FN]) {
 
 // acc[i][j] += the products of contraction indices [k_begin, k_end) for rows arow + i and columns
 // bcol + j of the lane, in fp32 MFMAs; this wave takes the 16 U-deep chunks first, first + STEP, ...
-template <bool AK, bool BKM, int FM, int FN, int U, bool VEC, int STEP>
+template <bool AK, bool BKM, int FM, int FN, int U, bool VEC, int STEP, bool LONG>
 __device__ __forceinline__ void direct_tile(f32x4 (&acc)[FM][FN], const float* __restrict__ A,
                                             const float* __restrict__ B, int arow, int bcol, int M, int N,
                                             int Kc, int k_begin, int k_end, int first) {
@@ -134,15 +134,16 @@ __device__ __forceinline__ void direct_tile(f32x4 (&acc)[FM][FN], const float* _
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i][s], b[u][j][s], acc[i][j], 0, 0, 0);
   };
   const int whole = k_begin + (k_end - k_begin) / (16 * U) * (16 * U);  // the part made of whole chunks
-  // (left by a difference: past the end of the longest contraction an int overflows, and with unsigned or
-  // counted chunks the compiler keeps fewer loads in flight)
+  // LONG: the loops are left by a difference, for an index past the end of the longest contraction overflows an
+  // int.  The test costs an instruction or two a chunk, but 12 % where the addresses are strided (256 x 4480 x 1992,
+  // input gradient), and unsigned, 64-bit or counted indices leave fewer loads in flight: a variant of its own.
   for (int k0 = k_begin + first * 16 * U; k0 < whole; k0 += STEP * 16 * U) {
     blocks(std::false_type{}, k0, std::integral_constant<int, U>{});
-    if (whole - k0 <= STEP * 16 * U) break;
+    if (LONG && whole - k0 <= STEP * 16 * U) break;
   }
   for (int k0 = whole + first * 16; k0 < k_end; k0 += STEP * 16) {
     blocks(std::true_type{}, k0, std::integral_constant<int, 1>{});
-    if (k_end - k0 <= STEP * 16) break;
+    if (LONG && k_end - k0 <= STEP * 16) break;
   }
 }
 
@@ -240,7 +241,7 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[FM][FN], float* __
 
 // WAVES > 1: the waves of a workgroup share one tile and take the 16 U-deep chunks of
 // the contraction in turn; their partial sums meet in LDS and are added in wave order.
-template <bool AK, bool BKM, int EPI, int FM, int FN, int U, bool VEC, int WAVES>
+template <bool AK, bool BKM, int EPI, int FM, int FN, int U, bool VEC, int WAVES, bool LONG>
 __global__ void __launch_bounds__(64 * WAVES)
     gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
                     float* __restrict__ C, const float* __restrict__ bias,
@@ -254,7 +255,7 @@ __global__ void __launch_bounds__(64 * WAVES)
   clear(acc);
   // Rows and columns past the edge read a valid one: their products land in output
   // elements that are never stored.
-  direct_tile<AK, BKM, FM, FN, U, VEC, WAVES>(acc, A, B, m0 + FM * r, n0 + FN * r, M, N, Kc, 0, Kc, wave);
+  direct_tile<AK, BKM, FM, FN, U, VEC, WAVES, LONG>(acc, A, B, m0 + FM * r, n0 + FN * r, M, N, Kc, 0, Kc, wave);
 
   if constexpr (WAVES > 1) {
     __shared__ f32x4 part[WAVES - 1][FM * FN][64];
@@ -304,7 +305,8 @@ __global__ void __launch_bounds__(64 * WAVES)
 //     of two that are larger is a normal number).  Zero rows (padding) have none and keep their zeros.
 // A look costs what reading the operands once more costs (2048 x 4096 x 1024 in a row of launches: 106 us, with
 // half of the rows zero 142, with a zero row in every wave 198; four chunks of the look in flight made no
-// difference); the largest magnitude, kept while staging, half an instruction an element.
+// difference); the largest magnitude, kept while staging, half an instruction an element (0 to 2 % of
+// the kernel, 6 % of a weight gradient: 4096 x 2048 x 2048 163 -> 171 us).
 //
 // Four waves (2 x 2) own a 32 FM x 32 FN tile.  Each thread loads its share of a 32-deep stage into
 // registers one stage ahead, splits it and writes three bf16 planes to LDS ([row][32], 64 bytes a row);
@@ -483,12 +485,12 @@ __global__ void __launch_bounds__(256, 2)
                                               zeros ? 0x1p-62f : 0x1p-110f);
   if (__builtin_amdgcn_ballot_w64(odd)) {
     clear(acc);
-    direct_tile<AK, BKM, FM, FN, 1, VEC, 1>(acc, A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end, 0);
+    direct_tile<AK, BKM, FM, FN, 1, VEC, 1, true>(acc, A, B, mw + FM * r, nw + FN * r, M, N, Kc, k_begin, k_end, 0);
   }
   store_tile<EPI, FM, FN, VEC>(acc, C, bias, Z, mw, nw, M, N, beta);
 }
 
-template <bool AK, bool BKM, int EPI, int FM, int FN, int U, int WAVES>
+template <bool AK, bool BKM, int EPI, int FM, int FN, int U, int WAVES, bool LONG = false>
 int launch_tile(const float* A, const float* B, float* C, const float* bias, float* Z, int M,
                 int N, int Kc, int beta, hipStream_t stream) {
   const long long tiles_m = ceil_div(M, 16 * FM), tiles_n = ceil_div(N, 16 * FN);
@@ -502,10 +504,10 @@ int launch_tile(const float* A, const float* B, float* C, const float* bias, flo
   const uintptr_t ptrs = (uintptr_t)A | (uintptr_t)B | (uintptr_t)C | (uintptr_t)bias | (uintptr_t)Z;
   const bool vec = Kc % 4 == 0 && (AK || M % FM == 0) && N % FN == 0 && (ptrs & 15u) == 0;
   if (vec)
-    hipLaunchKernelGGL((gemm_f32_kernel<AK, BKM, EPI, FM, FN, U, true, WAVES>), dim3((unsigned)nwg),
+    hipLaunchKernelGGL((gemm_f32_kernel<AK, BKM, EPI, FM, FN, U, true, WAVES, LONG>), dim3((unsigned)nwg),
                        dim3(64 * WAVES), 0, stream, A, B, C, bias, Z, M, N, Kc, (int)tiles_n, beta);
   else
-    hipLaunchKernelGGL((gemm_f32_kernel<AK, BKM, EPI, FM, FN, U, false, WAVES>), dim3((unsigned)nwg),
+    hipLaunchKernelGGL((gemm_f32_kernel<AK, BKM, EPI, FM, FN, U, false, WAVES, LONG>), dim3((unsigned)nwg),
                        dim3(64 * WAVES), 0, stream, A, B, C, bias, Z, M, N, Kc, (int)tiles_n, beta);
   AXN_HIP_TRY(hipGetLastError());
   return AXN_OK;
@@ -645,6 +647,10 @@ int launch_waves(long long tiles, const float* A, const float* B, float* C, cons
   return launch_tile<AK, BKM, EPI, FM, FN, U, 1>(A, B, C, bias, Z, M, N, Kc, beta, stream);
 }
 
+// Contractions whose loops would step past 2^31 - 1 (by four waves' chunks of 128 at most).
+constexpr int kLongContraction = 0x7fffffff - 512;
+static_assert((long long)kLongContraction + 4 * 16 * 8 <= 0x7fffffff, "the last step of the other variants");
+
 template <bool AK, bool BKM, int EPI>
 int launch_epi(const float* A, const float* B, float* C, const float* bias, float* Z, int M, int N,
                int Kc, int beta, float* ws, size_t ws_bytes, hipStream_t stream) {
@@ -662,6 +668,8 @@ int launch_epi(const float* A, const float* B, float* C, const float* bias, floa
   if (plan.parts == 1)
     return launch_split<AK, BKM, EPI>(A, B, C, bias, Z, M, N, Kc, beta, plan, stream);
   const NativeTiles t = native_tiles(M, N);
+  if (Kc > kLongContraction)
+    return launch_tile<AK, BKM, EPI, 1, 1, 4, 4, true>(A, B, C, bias, Z, M, N, Kc, beta, stream);
   if (t.size == 64)
     return launch_tile<AK, BKM, EPI, 4, 4, 2, 1>(A, B, C, bias, Z, M, N, Kc, beta, stream);
   if (t.size == 32)

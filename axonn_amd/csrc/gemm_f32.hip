@@ -305,8 +305,8 @@ __global__ void __launch_bounds__(64 * WAVES)
 //     of two that are larger is a normal number).  Zero rows (padding) have none and keep their zeros.
 // A look costs what reading the operands once more costs (2048 x 4096 x 1024 in a row of launches: 106 us, with
 // half of the rows zero 142, with a zero row in every wave 198; four chunks of the look in flight made no
-// difference); the largest magnitude, kept while staging, half an instruction an element (0 to 2 % of
-// the kernel, 6 % of a weight gradient: 4096 x 2048 x 2048 163 -> 171 us).
+// difference); the largest magnitude, kept while staging, half an instruction an element (nothing
+// measurable, 3 to 4 % of a weight gradient: 4096 x 2048 x 2048 170 -> 176 us).
 //
 // Four waves (2 x 2) own a 32 FM x 32 FN tile.  Each thread loads its share of a 32-deep stage into
 // registers one stage ahead, splits it and writes three bf16 planes to LDS ([row][32], 64 bytes a row);
@@ -426,8 +426,9 @@ __global__ void __launch_bounds__(256, 2)
   const int part = blockIdx.x / tiles, id = blockIdx.x - part * tiles;
   const int tm = id / tiles_n, tn = id - tm * tiles_n;
   const int m0 = tm * 32 * FM, n0 = tn * 32 * FN;
-  // (differences: past the end of the longest contraction an int overflows)
-  const int k_begin = part * k_part, k_end = Kc - k_begin < k_part ? Kc : k_begin + k_part;
+  // (unsigned: past the end of the longest contraction an int overflows; loops left by a difference are 2 %
+  // slower here)
+  const unsigned k_begin = part * k_part, k_end = min((unsigned)Kc, k_begin + k_part);
   C += (int64_t)part * M * N;
 
   f32x4 acc[FM][FN], low[FM][FN];
@@ -438,8 +439,8 @@ __global__ void __launch_bounds__(256, 2)
   my_share<BKM>(gb, qb);
   float xa[FM][4], xb[FN][4];
   // Rows past the edge read a valid one, indices past the end count as zero.
-  auto fetch = [&](int k0) {
-    if (k_end - k0 >= 32) {
+  auto fetch = [&](unsigned k0) {
+    if (k0 + 32 <= k_end) {
       load_block<AK, FM, VEC, false>(xa, A, m0 + FM * ga, M, k0 + 4 * qa, Kc, k_end);
       load_block<BKM, FN, VEC, false>(xb, B, n0 + FN * gb, N, k0 + 4 * qb, Kc, k_end);
     } else {
@@ -450,16 +451,14 @@ __global__ void __launch_bounds__(256, 2)
   float largest = 0.f;
   if (threadIdx.x == 0) large = 0;
   fetch(k_begin);
-  for (int k0 = k_begin; k0 < k_end; k0 += 32) {
+  for (unsigned k0 = k_begin; k0 < k_end; k0 += 32) {
     put_stage<AK, FM>(la, xa);
     put_stage<BKM, FN>(lb, xb);
     largest = max_magnitude(max_magnitude(largest, xa), xb);
     __syncthreads();
-    const bool last = k_end - k0 <= 32;
-    if (!last) fetch(k0 + 32);
+    if (k0 + 32 < k_end) fetch(k0 + 32);
     split_stage<FM, FN>(acc, low, la, lb);
     __syncthreads();
-    if (last) break;
   }
   if (largest >= 0x1p16f) large = 1;
   __syncthreads();

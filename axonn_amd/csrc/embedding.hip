@@ -14,8 +14,9 @@
 //   3. one wave per 64 x 16 bytes of a dW row walks that row's run of sorted
 //      slots, adds the dY rows in ascending token order in fp32 and stores the
 //      row once; rows no token names are stored as zeros (beta = 0) or left alone
-//      (beta = 1).  Every dW byte is written exactly once and never read unless
-//      beta = 1, so a fresh gradient needs no separate clear.
+//      (beta = 1).  dW is never read unless beta = 1.  Where the table has at least twice as
+//      many rows as there are tokens, the sort's launches write the zeros, to the whole table,
+//      beside the sort, and step 3 takes one wave per sorted slot.
 // The max_norm renormalisation of the looked-up rows reuses steps 1 and 2: one
 // wave per row that occurs, so a row named by many tokens is scaled once.
 #include "axn_internal.h"
@@ -58,6 +59,33 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK)
   __builtin_nontemporal_store(v, out + t * ldo + piece);
 }
 
+// One 16-byte store, non-temporal and written through (nt + sc1): the dense weight gradient
+// is written once, row after row, and read much later.  (The s_nop: the wait states a store
+// of more than 8 bytes needs before its data registers are written again are the
+// compiler's to insert for its own stores, not for this one.)
+template <typename V>
+__device__ __forceinline__ void store_through(V v, void* p) {
+  static_assert(sizeof(V) == 16, "one 16-byte store");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+
+// Zeros for a part of the gradient, written by the workgroups of a sort launch behind the
+// `sort_blocks` that sort: a sort of a few thousand tokens keeps 32 workgroups busy for 25 us
+// in three launches, and the rest of the chip writes the gradient meanwhile.
+struct Fill {
+  u32x4* first;          // 16-byte vectors
+  int64_t count;
+  int64_t sort_blocks;
+};
+constexpr int FILL_THREADS = 256;   // one vector a lane: see SORT_FILL_LDS
+__device__ __forceinline__ bool fill_zeros(const Fill& fill) {
+  const int64_t b = (int64_t)blockIdx.x - fill.sort_blocks;
+  if (b < 0) return false;
+  const int64_t i = b * FILL_THREADS + threadIdx.x;
+  if (i < fill.count) store_through(u32x4{0u, 0u, 0u, 0u}, fill.first + i);
+  return true;
+}
+
 // ---- sorting the token positions by id ---------------------------------------
 // Stable least-significant-digit radix sort of (key, position) pairs, keys over [0, V]
 // (V for an id outside [0, V): those sort behind every row), in 1 to 4 passes of at most
@@ -82,6 +110,10 @@ constexpr int SORT_FUSED_BATCH = 1 << 17;   // tokens (at most 64 workgroups) up
 constexpr int SORT_WAVES = 4;        // waves per workgroup
 constexpr int SORT_MAX_BITS = 10;    // digit width: 1024 counters per wave in LDS
 constexpr int SORT_MAX_PASSES = 4;
+// LDS of a workgroup in launches that also clear the gradient: 24 waves per CU, where a fill is fastest (7.3
+// TB/s; 6.8 with 32).  What the kernels declare themselves comes off it.
+constexpr int SORT_FILL_LDS = 27136;
+constexpr int SORT_PREPARE_LDS = 4 << SORT_MAX_BITS, SORT_SCATTER_LDS = SORT_WAVES * (4 << SORT_MAX_BITS) + 64;
 
 struct SortPlan {
   int passes;
@@ -98,20 +130,22 @@ __device__ __forceinline__ int key_of_id(int64_t id, int64_t V) {
 }
 
 // keys[i], vals[i] = i, pass 0's counts; row_start[v] = -1, status = 0, the later passes'
-// counts cleared.
+// counts cleared.  (row_start is not wanted where the gradient goes slot by slot.)
 template <int G>
 __global__ void __launch_bounds__(64 * SORT_WAVES)
     embedding_sort_prepare_kernel(const int64_t* __restrict__ ids, int* __restrict__ keys,
                                   int* __restrict__ vals, int* __restrict__ row_start, int* status,
                                   int* __restrict__ hist0, int* __restrict__ hist_rest,
                                   int64_t hist_rest_ints, int64_t T, int64_t V, int64_t nblk,
-                                  int bits0, bool block_major) {
+                                  int bits0, bool block_major, const Fill fill) {
   __shared__ int cnt[1 << SORT_MAX_BITS];
+  if (fill_zeros(fill)) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
+  const int64_t nthreads = fill.sort_blocks * blockDim.x;
   for (int64_t i = gtid; i < hist_rest_ints; i += nthreads) hist_rest[i] = 0;
-  for (int64_t i = gtid; i < V; i += nthreads) row_start[i] = -1;
+  if (row_start != nullptr)
+    for (int64_t i = gtid; i < V; i += nthreads) row_start[i] = -1;
   if (gtid == 0) *status = 0;
   const int nd = 1 << bits0;
   for (int d = threadIdx.x; d < nd; d += 64 * SORT_WAVES) cnt[d] = 0;
@@ -227,8 +261,10 @@ __global__ void __launch_bounds__(64 * SORT_WAVES)
                                   int* __restrict__ keys_out, int* __restrict__ vals_out,
                                   const int* __restrict__ base, int* __restrict__ next_hist,
                                   int* __restrict__ row_start, int* status, int64_t T, int64_t V,
-                                  int64_t nblk, int shift, int bits, int next_shift, int next_bits) {
+                                  int64_t nblk, int shift, int bits, int next_shift, int next_bits,
+                                  const Fill fill) {
   __shared__ int cnt[SORT_WAVES][1 << SORT_MAX_BITS];
+  if (fill_zeros(fill)) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t blk = blockIdx.x;
   const int nd = 1 << bits;
@@ -357,7 +393,8 @@ __global__ void __launch_bounds__(64 * SORT_WAVES)
         keys_out[dest] = key;
         vals_out[dest] = val;
         if (key < V) {
-          if (prev == lane || prev_key != key) atomicMin((unsigned*)&row_start[key], (unsigned)dest);
+          if (row_start != nullptr && (prev == lane || prev_key != key))
+            atomicMin((unsigned*)&row_start[key], (unsigned)dest);
         } else {
           *status = 1;   // an id outside the table
         }
@@ -368,16 +405,6 @@ __global__ void __launch_bounds__(64 * SORT_WAVES)
 
 // ---- backward ------------------------------------------------------------------
 // One 16-byte vector of a table row as fp32 values.
-// One 16-byte store, non-temporal and written through (nt + sc1): the dense weight gradient
-// is written once, row after row, and read much later.  (The s_nop: the wait states a store
-// of more than 8 bytes needs before its data registers are written again are the
-// compiler's to insert for its own stores, not for this one.)
-template <typename V>
-__device__ __forceinline__ void store_through(V v, void* p) {
-  static_assert(sizeof(V) == 16, "one 16-byte store");
-  asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
-}
-
 template <typename T>
 struct Vec;
 template <>
@@ -522,18 +549,23 @@ __device__ __forceinline__ void store_rows(float (&acc)[U][VEC], TW* dst, int64_
   }
 }
 
-// Half a 16-byte vector of the row.
-template <typename TW>
-__device__ __forceinline__ void store_half(const float (&x)[8 / sizeof(TW)], TW* dst, int beta) {
-  constexpr int N = 8 / (int)sizeof(TW);
+// Part of a 16-byte vector of the row.
+template <typename TW, int VEC>
+__device__ __forceinline__ void store_part(const float (&x)[VEC], TW* dst, int beta) {
   typedef std::conditional_t<sizeof(TW) == 4, float, __bf16> elem;
-  typedef elem half __attribute__((ext_vector_type(N)));
-  half o = beta != 0 ? *(const half*)dst : half{};
+  typedef elem part __attribute__((ext_vector_type(VEC)));
+  part o = beta != 0 ? *(const part*)dst : part{};
 #pragma unroll
-  for (int q = 0; q < N; ++q) o[q] = (elem)(x[q] + (float)o[q]);
-  *(half*)dst = o;
+  for (int q = 0; q < VEC; ++q) o[q] = (elem)(x[q] + (float)o[q]);
+  *(part*)dst = o;
 }
 
+// Table rows per token from which on the gradient is cleared by the sort's launches and then goes slot by
+// slot.  Ids drawn evenly (the most rows written twice), 128256 rows x 2048, row by row -> slot by slot, us:
+//   tokens          128256      64128       32064       16032       250
+//   fp32            420 -> 458  319 -> 317  264 -> 240  234 -> 196  187 -> 147
+//   bf16            237 -> 243  181 -> 164  153 -> 124  136 -> 101   99 -> 77
+constexpr int64_t EMB_SLOT_ROWS = 2;
 // Rows named by more than EMB_LONG_RUN tokens get waves of their own (below).
 constexpr int EMB_LONG_RUN = 32;
 
@@ -557,14 +589,20 @@ __device__ __forceinline__ int run_in_chunk(const int* __restrict__ keys, const 
 // chain of additions, and what it costs is how many gradient rows are on their way at once
 // and how many waves share the row.  A row's slots are read 64 at a time, one per lane, and
 // four (two) gradient rows are in flight.  Rows with more than EMB_LONG_RUN tokens are left to the
-// launch's first `long_blocks` workgroups: one wave per (64 sorted slots, 32 x VEC columns)
-// that looks for such runs among its slots and has 32 (16) gradient rows in flight, so that a
+// launch's first `long_blocks` workgroups: one wave per (64 sorted slots, 16 x VEC columns)
+// that looks for such runs among its slots and has 64 (32) gradient rows in flight, so that a
 // long run is spread over all pieces of its row and starts first.  The whole call for 16384
 // tokens x 2048 fp32 whose ids fall off like those of a text, into 128256 rows: 1394 us with one
-// row in flight and every row on the same waves, 239 us so; ids drawn evenly: 230 us both ways.
-// What bounds it now is the store of the 1.05 GB gradient (181 us of one token, 153 us for a
-// plain fill).
-template <typename TY, typename TW, int U>
+// row in flight and every row on the same waves, 239 with pieces twice as wide and half as many rows in flight
+// (the most frequent row, a twelfth of the tokens, was the launch's longest chain), 203 us so and slot by slot.
+// What bounds it now is the store of the 1.05 GB gradient (147 us of 250 tokens, 153 us for a
+// plain fill) and the way of 134 MB of gradient rows behind it.
+//
+// SLOTS: one wave per (sorted slot, U x 64 x VEC columns) instead, for a gradient whose other rows are
+// zeros already (beta = 0: the sort's launches write them, see Fill) or stay as they are (beta = 1).  Only a
+// run's first slot has work.  At most T rows are then written twice, but the zeros go at a fill's rate and under
+// the sort.
+template <typename TY, typename TW, int U, bool SLOTS>
 __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
     embedding_bwd_kernel(const int* __restrict__ keys, const int* __restrict__ vals,
                          const int* __restrict__ row_start, const TY* __restrict__ dY, TW* dW,
@@ -572,8 +610,8 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
                          int64_t padding_idx, int units_per_row, int long_blocks, int scale_by_freq,
                          int beta, int pieces_per_row) {
   constexpr int VEC = 16 / (int)sizeof(TW);
-  constexpr int LV = VEC / 2;                              // columns of a lane in a long run's wave
-  constexpr int LONG_B = LV * sizeof(TY) > 8 ? 16 : 32;    // its rows in flight: 64 registers
+  constexpr int LV = VEC / 4;                                 // columns of a lane in a long run's wave
+  constexpr int LONG_B = 256 / (LV * (int)sizeof(TY));        // its rows in flight: 64 registers
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   // (units_per_row and long_blocks lie side by side and come with one load, not with a second one here)
@@ -610,7 +648,7 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
         n = next_n;
         pos = next_pos;
       }
-      if (col0 < H) store_half<TW>(acc[0], dW + row * lddw + col0, beta);
+      if (col0 < H) store_part<TW, LV>(acc[0], dW + row * lddw + col0, beta);
     }
     return;
   }
@@ -629,15 +667,25 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
       row = unit / units_per_row;
     rest = (int)(unit - row * units_per_row);
   }
-  if (row >= V) return;
   const int64_t col0 = ((int64_t)rest * (U * 64) + lane) * VEC;
   float acc[U][VEC];
 #pragma unroll
   for (int u = 0; u < U; ++u)
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[u][q] = 0.f;
-  const int s = row_start[row];
-  if (s >= 0 && row != padding_idx) {
+  int s;
+  if constexpr (SLOTS) {
+    const int64_t slot = row;   // (fewer than 2^31)
+    if (slot >= T) return;
+    const int key = keys[slot], before = slot > 0 ? keys[slot - 1] : -1;
+    if (key == before || key >= V || key == padding_idx) return;
+    s = (int)slot;
+    row = key;
+  } else {
+    if (row >= V) return;
+    s = row_start[row];
+  }
+  if (SLOTS || (s >= 0 && row != padding_idx)) {
     int pos, n = 1;
     if (s + 1 >= T || keys[s + 1] != (int)row)   // most rows of a text have one token
       pos = vals[s];
@@ -754,8 +802,10 @@ inline bool carve(void* ws, size_t ws_bytes, int64_t T, int64_t V, Workspace* ou
 
 // Fills ws with the sorted (key, position) pairs and row_start; on return
 // *keys and *vals point at the sorted arrays.
+// With `zeros`, the launches also clear that many bytes there, an equal share each, and row_start is left alone.
 int sort_token_positions(const int64_t* ids, int64_t T, int64_t V, const Workspace& w,
-                         const int** keys, const int** vals, hipStream_t stream) {
+                         const int** keys, const int** vals, hipStream_t stream, bool want_row_start = true,
+                         void* zeros = nullptr, size_t zero_bytes = 0) {
   const SortPlan pl = plan_sort(T, V);
   if (pl.nblk >= (1LL << 31) ||
       pl.hist_ints >= ((size_t)1 << 40)) {
@@ -768,16 +818,26 @@ int sort_token_positions(const int64_t* ids, int64_t T, int64_t V, const Workspa
   int64_t fill_blocks = (V + 4 * 256 - 1) / (4 * 256);
   if (fill_blocks > 1024) fill_blocks = 1024;
   const int64_t prep_blocks = seg_blocks > fill_blocks ? seg_blocks : (fill_blocks > 0 ? fill_blocks : 1);
+  int* const row_start = want_row_start ? w.row_start : nullptr;
+  const int64_t vectors = (int64_t)(zero_bytes / 16), shares = 1 + (T > 0 ? pl.passes : 0);
+  auto fill_of = [&](int64_t share, int64_t sort_blocks) {
+    const int64_t first = vectors / shares * share, end = share + 1 == shares ? vectors : vectors / shares * (share + 1);
+    return Fill{(u32x4*)zeros + first, end - first, sort_blocks};
+  };
+  auto blocks_with = [](const Fill& fill) {
+    return (unsigned)(fill.sort_blocks + (fill.count + FILL_THREADS - 1) / FILL_THREADS);
+  };
   int* hist_rest = w.hist + pl.hist_ofs[1];
   const int64_t hist_rest_ints = pl.passes > 1 ? (int64_t)(pl.hist_ints - pl.hist_ofs[1]) : 0;
-  if (pl.groups == 2)
-    hipLaunchKernelGGL(embedding_sort_prepare_kernel<2>, dim3((unsigned)prep_blocks), block, 0, stream, ids,
-                       w.keys_a, w.vals_a, w.row_start, w.status, w.hist, hist_rest, hist_rest_ints, T, V,
-                       pl.nblk, pl.bits[0], pl.fused_scan);
-  else
-    hipLaunchKernelGGL(embedding_sort_prepare_kernel<8>, dim3((unsigned)prep_blocks), block, 0, stream, ids,
-                       w.keys_a, w.vals_a, w.row_start, w.status, w.hist, hist_rest, hist_rest_ints, T, V,
-                       pl.nblk, pl.bits[0], pl.fused_scan);
+  {
+    const Fill fill = fill_of(0, prep_blocks);
+    void (*prepare)(const int64_t*, int*, int*, int*, int*, int*, int*, int64_t, int64_t, int64_t, int64_t, int,
+                    bool, Fill) =
+        pl.groups == 2 ? embedding_sort_prepare_kernel<2> : embedding_sort_prepare_kernel<8>;
+    hipLaunchKernelGGL(prepare, dim3(blocks_with(fill)), block, vectors > 0 ? SORT_FILL_LDS - SORT_PREPARE_LDS : 0,
+                       stream, ids, w.keys_a, w.vals_a, row_start, w.status, w.hist, hist_rest, hist_rest_ints, T, V,
+                       pl.nblk, pl.bits[0], pl.fused_scan, fill);
+  }
   AXN_HIP_TRY(hipGetLastError());
   const int *kin = w.keys_a, *vin = w.vals_a;
   int *kout = w.keys_b, *vout = w.vals_b;
@@ -791,14 +851,16 @@ int sort_token_positions(const int64_t* ids, int64_t T, int64_t V, const Workspa
       }
       const bool more = p + 1 < pl.passes;
       void (*scatter)(const int*, const int*, int*, int*, const int*, int*, int*, int*, int64_t, int64_t,
-                      int64_t, int, int, int, int) =
+                      int64_t, int, int, int, int, Fill) =
           pl.fused_scan ? (pl.groups == 2 ? embedding_sort_scatter_kernel<2, false>
                                           : embedding_sort_scatter_kernel<8, false>)
                         : embedding_sort_scatter_kernel<8, true>;
-      hipLaunchKernelGGL(scatter, dim3((unsigned)seg_blocks), block, 0, stream, kin, vin, kout, vout,
-                         (const int*)hist, more ? w.hist + pl.hist_ofs[p + 1] : nullptr, w.row_start,
+      const Fill fill = fill_of(p + 1, seg_blocks);
+      hipLaunchKernelGGL(scatter, dim3(blocks_with(fill)), block,
+                         vectors > 0 ? SORT_FILL_LDS - SORT_SCATTER_LDS : 0, stream, kin, vin, kout, vout,
+                         (const int*)hist, more ? w.hist + pl.hist_ofs[p + 1] : nullptr, row_start,
                          w.status, T, V, pl.nblk, pl.shift[p], pl.bits[p], more ? pl.shift[p + 1] : 0,
-                         more ? pl.bits[p + 1] : 0);
+                         more ? pl.bits[p + 1] : 0, fill);
       AXN_HIP_TRY(hipGetLastError());
       const int* tk = kin; kin = kout; kout = (int*)tk;
       const int* tv = vin; vin = vout; vout = (int*)tv;
@@ -852,22 +914,31 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
   const int U = pieces >= 4 ? 4 : pieces >= 2 ? 2 : 1;
   const int upr = (int)((pieces + U - 1) / U);
   // waves for rows named by many tokens: one per 64 sorted slots and piece
-  const int64_t long_pieces = (H / (vec / 2) + 63) / 64;
+  const int64_t long_pieces = (H / (vec / 4) + 63) / 64;
   const int64_t long_blocks =
       T > EMB_LONG_RUN ? ((T + 63) / 64 * long_pieces + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK : 0;
-  const int64_t blocks = (V * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK + long_blocks;
-  if (blocks >= (1LL << 31)) {
+  const bool slots = T <= V / EMB_SLOT_ROWS && (beta != 0 || lddw == H);
+  const int64_t blocks = ((slots ? T : V) * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK + long_blocks;
+  const size_t zero_bytes = slots && beta == 0 ? (size_t)V * (size_t)H * (dw_dtype == AXN_F32 ? 4 : 2) : 0;
+  if (blocks + (int64_t)(zero_bytes / (16 * FILL_THREADS)) >= (1LL << 31)) {
     set_error("embedding_bwd: too many rows x columns (%lld blocks)", (long long)blocks);
     return AXN_ELIMIT;
   }
   const int *keys = nullptr, *vals = nullptr;
-  int rc = sort_token_positions(ids, T, V, w, &keys, &vals, stream);
-  if (rc) return rc;
+  int rc = sort_token_positions(ids, T, V, w, &keys, &vals, stream, !slots, dW, zero_bytes);
+  if (rc || blocks == 0) return rc;
   const dim3 grid((unsigned)blocks), block(64 * WAVES_PER_BLOCK);
-#define AXN_EMB_BWD_U(TY, TW, UU)                                                               \
-  hipLaunchKernelGGL((embedding_bwd_kernel<TY, TW, UU>), grid, block, EMB_BWD_LDS, stream, keys, vals,    \
+#define AXN_EMB_BWD_US(TY, TW, UU, SLOTS)                                                       \
+  hipLaunchKernelGGL((embedding_bwd_kernel<TY, TW, UU, SLOTS>), grid, block, EMB_BWD_LDS, stream, keys, vals,    \
                      w.row_start, (const TY*)dY, (TW*)dW, T, V, H, lddy, lddw, padding_idx, upr, \
                      (int)long_blocks, scale_by_freq, beta, (int)long_pieces)
+#define AXN_EMB_BWD_U(TY, TW, UU)           \
+  do {                                      \
+    if (slots)                              \
+      AXN_EMB_BWD_US(TY, TW, UU, true);     \
+    else                                    \
+      AXN_EMB_BWD_US(TY, TW, UU, false);    \
+  } while (0)
 #define AXN_EMB_BWD(TY, TW)                 \
   do {                                      \
     if (U == 4)                             \
@@ -885,6 +956,7 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
     AXN_EMB_BWD(uint16_t, float);
   else
     AXN_EMB_BWD(uint16_t, uint16_t);
+#undef AXN_EMB_BWD_US
 #undef AXN_EMB_BWD_U
 #undef AXN_EMB_BWD
   AXN_HIP_TRY(hipGetLastError());

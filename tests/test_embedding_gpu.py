@@ -154,6 +154,39 @@ def test_backward_over_every_shape_of_the_sort(T, V):
     assert np.array_equal(host(dW), want)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,V,H", [(1, 2, 8), (1, 1, 8), (500, 1000, 264), (500, 999, 264), (3, 4096, 2056),
+                                   (0, 300, 40), (2500, (1 << 20) + 3, 8), (140000, 280000, 16)])
+def test_backward_on_either_side_of_two_table_rows_a_token(dtype, T, V, H):
+    """From two table rows a token on the sort's launches clear the gradient and the rows with tokens are
+    written behind them: tables smaller and larger than what a launch's workgroups clear, one to three passes,
+    no tokens at all, ids outside the table, the padding row, a gradient that held something else, and one
+    with room between its rows (which nothing may write to)."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(T + V)
+    u = torch.rand(T, device="cuda", generator=g)
+    ids = torch.where(torch.rand(T, device="cuda", generator=g) < 0.5, u * V, u * u * u * 9).long().clamp_(0, V - 1)
+    if T > 2:
+        ids[1], ids[T // 2] = V, -1
+    dy = (torch.randn(T, H, device="cuda", generator=g) * 0.01).to(dtype)
+    padding = int(ids[0]) if T else None
+    want = oe.embedding_backward(ids.cpu().numpy(), host(dy), V, padding_idx=padding)
+    if dtype == torch.bfloat16:
+        want = bf16_round(want)
+    out = torch.full((V, H), 7.0, device="cuda", dtype=dtype)
+    ops.embedding_bwd(ids, dy, V, padding_idx=padding, out=out)
+    assert np.array_equal(host(out), want)
+    wide = torch.full((V, H + 8), 7.0, device="cuda", dtype=dtype)
+    ops.embedding_bwd(ids, dy, V, padding_idx=padding, out=wide[:, :H])
+    assert np.array_equal(host(wide[:, :H]), want) and bool((wide[:, H:] == 7.0).all())
+    ops.embedding_bwd(ids, dy, V, padding_idx=padding, out=out, accumulate=True)
+    twice = 2 * oe.embedding_backward(ids.cpu().numpy(), host(dy), V, padding_idx=padding)
+    if dtype == torch.bfloat16:   # the sum is added to the rounded gradient and rounded again
+        twice = bf16_round(want + twice / 2)
+    assert np.array_equal(host(out), twice)
+
+
 def test_backward_padding_row_repeated_ids_and_determinism():
     """A tenth of the tokens name one row, another tenth the padding row; the sum of 400
     terms depends on its order, and the kernel's order is the token order."""

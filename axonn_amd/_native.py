@@ -22,7 +22,7 @@ BF16, F16, F32 = 0, 1, 2
 EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_GELU = 0, 1, 2, 3
 BIAS_16BIT = 0x100   # with an epilogue: the bias has the operands' 16-bit type
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 # Every symbol include/axn.h declares: name -> (restype, argtypes)
 _c = ctypes
@@ -71,6 +71,7 @@ SYMBOLS = {
                                  _int, _vp, _sz, _vp]),
     "axn_dgelu_dbias": (_int, [_vp, _vp, _vp, _int, _vp, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "axn_gemm_swiglu_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _i64, _vp]),
+    "axn_gemm_swiglu_fwd_few": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _i64, _vp]),
     "axn_gemm_dgrad_pair": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp]),
     "axn_dgelu_dbias_workspace_bytes": (_sz, [_i64, _i64]),
     "axn_swiglu_fwd": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _i64, _vp]),

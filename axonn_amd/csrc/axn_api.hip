@@ -433,17 +433,15 @@ int axn_gemm_wgrad_ws(const void* dY, const void* X, void* dW, int dtype, int64_
                  beta, dw_dtype, workspace, workspace_bytes, stream);
 }
 
-int axn_gemm_swiglu_fwd(const void* X, const void* Wg, const void* Wu, void* H, void* gate_save,
-                        void* up_save, int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx,
-                        int64_t ldw, int64_t ldh, void* stream) {
-  const char* name = "axn_gemm_swiglu_fwd";
+static int swiglu_args(const char* name, GemmArgs& g, const void* X, const void* Wg, const void* Wu, void* H,
+                       void* gate_save, void* up_save, int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                       int64_t ldw, int64_t ldh) {
   REQUIRE(dtype == AXN_BF16 || dtype == AXN_F16, AXN_EINVAL, "%s: dtype must be bf16 or fp16", name);
   int rc = check_gemm(name, X, Wg, H, M, N, K, ldx, ldw, ldh, K, K, N);
   if (rc) return rc;
   REQUIRE(Wu != nullptr, AXN_EINVAL, "%s: null operand pointer", name);
   REQUIRE(aligned16(Wu) && aligned16(gate_save) && aligned16(up_save), AXN_EALIGN,
           "%s: operand pointers must be 16-byte aligned", name);
-  GemmArgs g = {};
   g.A = (const uint16_t*)X;
   g.B = (const uint16_t*)Wg;
   g.B2 = (const uint16_t*)Wu;
@@ -456,7 +454,28 @@ int axn_gemm_swiglu_fwd(const void* X, const void* Wg, const void* Wu, void* H, 
   g.lda = ldx;
   g.ldb = ldw;
   g.ldc = ldh;
-  return launch_gemm_swiglu(g, dtype == AXN_F16, (hipStream_t)stream);
+  return AXN_OK;
+}
+
+int axn_gemm_swiglu_fwd(const void* X, const void* Wg, const void* Wu, void* H, void* gate_save,
+                        void* up_save, int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                        int64_t ldw, int64_t ldh, void* stream) {
+  GemmArgs g = {};
+  const int rc = swiglu_args("axn_gemm_swiglu_fwd", g, X, Wg, Wu, H, gate_save, up_save, dtype, M, N, K, ldx, ldw, ldh);
+  return rc ? rc : launch_gemm_swiglu(g, dtype == AXN_F16, (hipStream_t)stream);
+}
+
+int axn_gemm_swiglu_fwd_few(const void* X, const void* Wg, const void* Wu, void* H, void* gate_save,
+                            void* up_save, int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                            int64_t ldw, int64_t ldh, void* stream) {
+  const char* name = "axn_gemm_swiglu_fwd_few";
+  GemmArgs g = {};
+  const int rc = swiglu_args(name, g, X, Wg, Wu, H, gate_save, up_save, dtype, M, N, K, ldx, ldw, ldh);
+  if (rc) return rc;
+  REQUIRE(M <= kStreamMaxRows && ldx < kStreamMaxLd && ldw < kStreamMaxLd, AXN_ESHAPE,
+          "%s: at most %lld rows and row strides below %lld elements (got M=%lld, %lld and %lld)", name,
+          (long long)kStreamMaxRows, (long long)kStreamMaxLd, (long long)M, (long long)ldx, (long long)ldw);
+  return launch_gemm_stream_swiglu(g, dtype == AXN_F16, (hipStream_t)stream);
 }
 
 int axn_gemm_dgrad_pair(const void* dY1, const void* W1, const void* dY2, const void* W2, void* dX,

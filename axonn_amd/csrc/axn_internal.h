@@ -109,6 +109,8 @@ struct GemmArgs {
   // the leading dimensions of A and B.
   const uint16_t* A2;
   int k_first;
+  // Gate/up forward of a few rows (launch_gemm_stream_swiglu): output columns that start at the same line.
+  int start_rows;
 };
 
 // Sizes go up to 2^31 - 1: what is rounded up to tiles or stages is computed in 64 bits.
@@ -196,6 +198,9 @@ inline bool stream_ahead(int64_t M, int64_t N, int64_t Kc) {
 }
 constexpr int64_t kStreamMaxLd = 1LL << 24;
 int launch_gemm_stream(const GemmArgs& args, int epilogue, bool out_f32, bool half, hipStream_t stream);
+// The gate/up forward (launch_gemm_swiglu) of up to kStreamMaxRows rows, N a multiple of 8; the two products of up
+// to 32 rows are those of launch_gemm_stream bit for bit.
+int launch_gemm_stream_swiglu(const GemmArgs& args, bool half, hipStream_t stream);
 
 // C = silu(A B^T) * (A B2^T) in one launch (both weight matrices [N][Kc], K-major), for
 // M % 256 == 0, N % 128 == 0, Kc % 64 == 0 and operands below 2 GiB; AXN_ESHAPE otherwise.

@@ -26,18 +26,42 @@
 namespace axn {
 namespace {
 
+// Gate/up forward: 4 consecutive columns of one row (of a multiple of 8), as store_swiglu8.
+template <bool HALF>
+__device__ __forceinline__ void store_swiglu4(const f32x4& vg, const f32x4& vu, const GemmArgs& g, int row, int col) {
+  using lp = std::conditional_t<HALF, _Float16, __bf16>;
+  typedef lp lpx4 __attribute__((ext_vector_type(4)));
+  const int64_t o = (int64_t)row * g.ldc + col;
+  lpx4 gate, up, out;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    gate[e] = (lp)vg[e];
+    up[e] = (lp)vu[e];
+    const float x = (float)gate[e];
+    out[e] = (lp)(x * sigmoid_f(x) * (float)up[e]);
+  }
+  if (g.G != nullptr) *(lpx4*)(g.G + o) = gate;
+  if (g.U != nullptr) *(lpx4*)(g.U + o) = up;
+  *(lpx4*)((uint16_t*)g.C + o) = out;
+}
+
 // D: lines of the contraction a wave has on their way (its ring's slots).
 template <int MT, int R, int NW, int D, int EPI, bool OUT_F32, bool HALF>
-__global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) {
+__device__ __forceinline__ void stream_gemm(const GemmArgs& g) {
   constexpr int GROUPS = R + MT;              // 16-row groups copied per line: W's, then X's
   constexpr uint32_t LINE = GROUPS * 2048;    // bytes of a slot
   constexpr int COPIES = 2 * GROUPS;
+  // Gate/up forward: the first half of W's groups are rows of the gate weights, the second half the rows of
+  // the up weights with the same indices.
+  constexpr bool SWIGLU = EPI == EPI_SWIGLU;
+  constexpr int RO = SWIGLU ? R / 2 : R;      // 16-column groups of the output
+  static_assert(!SWIGLU || (R % 2 == 0 && !OUT_F32), "pairs of groups");
   static_assert(COPIES * (D - 1) < 64, "outstanding copies the wait can count");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
-  const int n0 = blockIdx.x * (16 * R);
+  const int n0 = blockIdx.x * (16 * RO);
   char* ring = lds + wave * (D * LINE);
 
   // Copies: 8 rows of 128 bytes each.  Rows past the end are outside the buffer and come as
@@ -49,6 +73,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) 
                                              0x00020000);
   };
   const __amdgpu_buffer_rsrc_t rw = resource(g.B, g.N, g.ldb, n0), rx = resource(g.A, g.M, g.lda, 0);
+  const __amdgpu_buffer_rsrc_t rw2 = SWIGLU ? resource(g.B2, g.N, g.ldb, n0) : rw;
   uint32_t vw[2], vx[2];   // copy h of a group: rows 8 h .. 8 h + 7
   int chunk[2];
 #pragma unroll
@@ -62,7 +87,9 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) 
   const int lines = (g.Kc + 63) / 64;
   // Workgroups start at different lines: all at the same one, with power-of-two row strides,
   // they crowd onto few memory channels (N = 14336, R = 2: 27.7 -> 21.4 us).
-  const int rot = (int)((blockIdx.x * 7u) % (unsigned)lines);
+  // (The gate/up forward starts where the two products of their own would: the same sums.)
+  const unsigned start = SWIGLU ? (unsigned)n0 / (unsigned)g.start_rows : blockIdx.x;
+  const int rot = (int)((start * 7u) % (unsigned)lines);
   const int mine = (lines - wave + NW - 1) / NW;   // lines wave, wave + NW, ... (may be 0 or less)
   auto copy_line = [&](int i) {                    // the wave's i-th line into slot i % D
     int line = wave + i * NW + rot;
@@ -76,8 +103,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) 
       const uint32_t ow = out ? kOutside : vw[h], ox = out ? kOutside : vx[h];
 #pragma unroll
       for (int j = 0; j < R; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, LDS_PTR(void, to + j * 2048 + h * 1024), 16, (int)ow,
-                                                 (int)(k0 * 2 + j * w_group), 0, 2);   // non-temporal: read once (4 % on the kernel)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(j < RO ? rw : rw2, LDS_PTR(void, to + j * 2048 + h * 1024), 16,
+                                                 (int)ow, (int)(k0 * 2 + (j % RO) * w_group), 0, 2);   // non-temporal: read once (4 % on the kernel)
 #pragma unroll
       for (int j = 0; j < MT; ++j)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, LDS_PTR(void, to + (R + j) * 2048 + h * 1024), 16, (int)ox,
@@ -142,10 +169,23 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) 
 #pragma unroll
     for (int j = 0; j < R; ++j) part[(wave * (MT * R) + m * R + j) * 64 + lane] = acc[m][j];
   __syncthreads();
-  for (int b = wave; b < MT * R; b += NW) {
+  auto total = [&](int b) {
     f32x4 s = part[b * 64 + lane];
 #pragma unroll
     for (int v = 1; v < NW; ++v) s += part[(v * (MT * R) + b) * 64 + lane];
+    return s;
+  };
+  if constexpr (SWIGLU) {
+    for (int b = wave; b < MT * RO; b += NW) {
+      const int m = b / RO, j = b % RO;
+      const f32x4 gate = total(m * R + j), up = total(m * R + RO + j);
+      const int row = 16 * m + r, col = n0 + 16 * j + 4 * q;
+      if (row < g.M && col < g.N) store_swiglu4<HALF>(gate, up, g, row, col);
+    }
+    return;
+  }
+  for (int b = wave; b < MT * R; b += NW) {
+    const f32x4 s = total(b);
     const int row = 16 * (b / R) + r, col = n0 + 16 * (b % R) + 4 * q;
     if (row >= g.M) continue;
 #pragma unroll
@@ -154,10 +194,24 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) 
   }
 }
 
+template <int MT, int R, int NW, int D, int EPI, bool OUT_F32, bool HALF>
+__global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) {
+  stream_gemm<MT, R, NW, D, EPI, OUT_F32, HALF>(g);
+}
+template <int MT, int R, int NW, int D, bool HALF>
+__global__ void __launch_bounds__(NW * 64) gemm_gate_up_stream_kernel(const GemmArgs g) {
+  stream_gemm<MT, R, NW, D, EPI_SWIGLU, false, HALF>(g);
+}
+
+// The rings, or the waves' sums behind them.
+constexpr size_t stream_lds(int MT, int R, int NW, int D) {
+  const size_t ring = (size_t)NW * D * (R + MT) * 2048, sums = (size_t)NW * MT * R * 1024;
+  return ring > sums ? ring : sums;
+}
+
 template <int MT, int R, int NW, int D, bool HALF>
 int launch_stream(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
-  constexpr size_t ring = (size_t)NW * D * (R + MT) * 2048, sums = (size_t)NW * MT * R * 1024;
-  constexpr size_t lds = ring > sums ? ring : sums;
+  constexpr size_t lds = stream_lds(MT, R, NW, D);
   const dim3 grid((unsigned)ceil_div(g.N, 16 * R)), block(NW * 64);
 #define STREAM(EPI, F32)                                                                   \
   {                                                                                        \
@@ -186,10 +240,12 @@ int launch_stream(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t str
 // The smallest R whose workgroups fit one round of the CUs: a second round costs more than
 // taller workgroups (5120 x 4096, 16 tokens: 320 workgroups of 16 rows 12.3 us, 160 of 32
 // rows 10.5; 4096 x 4096: 256 of 16 rows 8.0, 128 of 32 rows 10.1).
+int stream_groups(int N) { return N <= 16 * 256 ? 1 : N <= 32 * 256 ? 2 : 4; }
 template <int MT, int D1, int D2, bool HALF>
 int launch_stream_rows(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
-  if (g.N <= 16 * 256) return launch_stream<MT, 1, 4, D1, HALF>(g, epilogue, out_f32, stream);
-  if (g.N <= 32 * 256) return launch_stream<MT, 2, 4, D2, HALF>(g, epilogue, out_f32, stream);
+  const int groups = stream_groups(g.N);
+  if (groups == 1) return launch_stream<MT, 1, 4, D1, HALF>(g, epilogue, out_f32, stream);
+  if (groups == 2) return launch_stream<MT, 2, 4, D2, HALF>(g, epilogue, out_f32, stream);
   return launch_stream<MT, 4, 4, 2, HALF>(g, epilogue, out_f32, stream);
 }
 
@@ -200,7 +256,49 @@ int launch_stream_tokens(const GemmArgs& g, int epilogue, bool out_f32, hipStrea
   return launch_stream_rows<4, 2, 2, HALF>(g, epilogue, out_f32, stream);
 }
 
+// The gate/up forward: R / 2 groups of 16 rows of either matrix a workgroup.  Two workgroups fit a CU with
+// R up to 4, so that both matrices are one round of twice as many; taller ones read the tokens less often.
+// us of 16 and 64 tokens (cold weights, N x K), two products and the activation before -> R = 2, 4, 8:
+//              16 tokens                          64 tokens
+//   2816 x 1024   11.8 -> 4.9, 5.9, 8.3           14.3 -> 6.5, 8.4, 13.7
+//   5632 x 2048   16.0 -> 11.1, 10.0, 14.6        23.5 -> 18.2, 13.9, 22.7
+//   8192 x 3072   23.1 -> 17.7, 17.7, 23.3        33.8 -> 28.6, 22.1, 32.9
+//   11008 x 4096  38.6 -> 29.6, 34.6, 31.3        54.1 -> 47.9, 46.3, 40.3
+//   14336 x 4096  45.2 -> 38.1, 37.8, 38.0        57.6 -> 63.0, 49.6, 43.1
+// (R = 8 of more than 32 tokens with two waves: with four its rings are larger than LDS.)  16384 x 4096 at 16
+// tokens: 40.2 us, 6.7 TB/s.
+template <int MT, int R, int NW, int D, bool HALF>
+int launch_gate_up_stream(const GemmArgs& in, hipStream_t stream) {
+  constexpr size_t lds = stream_lds(MT, R, NW, D);
+  GemmArgs g = in;
+  g.start_rows = 16 * stream_groups(g.N);
+  void (*kern)(const GemmArgs) = gemm_gate_up_stream_kernel<MT, R, NW, D, HALF>;
+  static std::atomic<unsigned long long> lds_allowed{0};
+  const int rc = allow_lds((const void*)kern, lds, lds_allowed);
+  if (rc != AXN_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(g.N, 8 * R)), dim3(NW * 64), lds, stream, g);
+  AXN_HIP_TRY(hipGetLastError());
+  return AXN_OK;
+}
+template <int MT, int D2, bool HALF>
+int launch_stream_swiglu(const GemmArgs& g, hipStream_t stream) {
+  if (g.N <= 16 * 256 || (g.N > 32 * 256 && MT == 1))
+    return launch_gate_up_stream<MT, 2, 4, D2, HALF>(g, stream);
+  if (g.N <= 32 * 256) return launch_gate_up_stream<MT, 4, 4, 2, HALF>(g, stream);
+  return launch_gate_up_stream<MT, 8, MT == 4 ? 2 : 4, 2, HALF>(g, stream);
+}
+template <bool HALF>
+int launch_stream_swiglu_tokens(const GemmArgs& g, hipStream_t stream) {
+  if (g.M <= 16) return launch_stream_swiglu<1, 3, HALF>(g, stream);
+  if (g.M <= 32) return launch_stream_swiglu<2, 2, HALF>(g, stream);
+  return launch_stream_swiglu<4, 2, HALF>(g, stream);
+}
+
 }  // namespace
+
+int launch_gemm_stream_swiglu(const GemmArgs& g, bool half, hipStream_t stream) {
+  return half ? launch_stream_swiglu_tokens<true>(g, stream) : launch_stream_swiglu_tokens<false>(g, stream);
+}
 
 int launch_gemm_stream(const GemmArgs& g, int epilogue, bool out_f32, bool half, hipStream_t stream) {
   return half ? launch_stream_tokens<true>(g, epilogue, out_f32, stream)

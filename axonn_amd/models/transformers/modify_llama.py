@@ -10,7 +10,8 @@ forward passes to Hugging Face.  Here
   and the product as one kernel (`SwiGLU`, axn_swiglu_fwd / axn_swiglu_bwd) when
   the activation is SiLU - or, for 16-bit layers without bias and whole-tile shapes,
   both projections and the activation as one launch (`GateUpSwiGLU`,
-  axn_gemm_swiglu_fwd), with the same results bit for bit;
+  axn_gemm_swiglu_fwd), with the same results bit for bit; so are up to 64 tokens without
+  gradients (axn_gemm_swiglu_fwd_few);
 * the attention projections are swapped after the original constructor has run,
   instead of restating that constructor (:12-73): the constructor's other fields
   changed across transformers releases, the four projections did not.  At a
@@ -60,12 +61,12 @@ class GateUpSwiGLU(torch.autograd.Function):
 
     @staticmethod
     @torch.amp.custom_fwd(device_type="cuda")
-    def forward(ctx, x, w_gate, w_up, shape):
+    def forward(ctx, x, w_gate, w_up, shape, save=True):
         dt = _compute_dtype(x, w_gate.reshape(shape))
         x2 = x.reshape(-1, x.shape[-1]).to(dt)
-        needs_grad = any(ctx.needs_input_grad[:3])
+        needs_grad = save and any(ctx.needs_input_grad[:3])
         h, gate, up = ops.gemm_swiglu_fwd(x2, w_gate.reshape(shape).to(dt), w_up.reshape(shape).to(dt),
-                                          save=needs_grad)
+                                          save=needs_grad, few=not save and x2.shape[0] <= 64)
         ctx.save_for_backward(x2, w_gate, w_up, gate, up)
         ctx.shape, ctx.input_shape, ctx.compute_dtype = shape, x.shape, dt
         return h.reshape(*x.shape[:-1], shape[0])
@@ -91,12 +92,13 @@ class GateUpSwiGLU(torch.autograd.Function):
             grad_wg = _weight_grad(dgate, x2, w_gate)
         if ctx.needs_input_grad[2]:
             grad_wu = _weight_grad(dup, x2, w_up)
-        return grad_x, grad_wg, grad_wu, None
+        return grad_x, grad_wg, grad_wu, None, None
 
 
 def _one_launch_gate_up(mlp, x):
     """The MLP's gate/up pair qualifies for the one-launch forward: SiLU, no biases,
-    plain layers on one rank, 16-bit compute type and whole-tile shapes."""
+    plain layers on one rank, 16-bit compute type and whole-tile shapes, or up to 64 tokens without
+    gradients (generation)."""
     g, u = mlp.gate_proj, mlp.up_proj
     if not (getattr(mlp, "_axonn_fused_swiglu", False) and x.is_cuda):
         return False
@@ -106,7 +108,13 @@ def _one_launch_gate_up(mlp, x):
     if not torch.is_autocast_enabled("cuda") and not (x.dtype == g.weight.dtype == u.weight.dtype):
         return False
     tokens = x.numel() // max(x.shape[-1], 1)
-    return ops.gemm_swiglu_supported(tokens, g.local_out_features, g.local_in_features, dt)
+    sizes = tokens, g.local_out_features, g.local_in_features, dt
+    if torch.is_grad_enabled() or tokens > 64:
+        return ops.gemm_swiglu_supported(*sizes)
+    # (layers that something watches or has replaced are called themselves)
+    return (type(g) is type(u) is Linear and not (g._forward_hooks or g._forward_pre_hooks or u._forward_hooks
+                                                  or u._forward_pre_hooks)
+            and x.shape[-1] == g.local_in_features and ops.gemm_swiglu_few_supported(*sizes))
 
 
 def modified_mlp_init(self, config):
@@ -126,7 +134,8 @@ def modified_mlp_init(self, config):
 def modified_mlp_forward(self, x):
     if _one_launch_gate_up(self, x):
         shape = (self.gate_proj.local_out_features, self.gate_proj.local_in_features)
-        return self.down_proj(GateUpSwiGLU.apply(x, self.gate_proj.weight, self.up_proj.weight, shape))
+        return self.down_proj(GateUpSwiGLU.apply(x, self.gate_proj.weight, self.up_proj.weight, shape,
+                                                 torch.is_grad_enabled()))
     gate, up = self.gate_proj(x), self.up_proj(x)
     if getattr(self, "_axonn_fused_swiglu", False) and gate.is_cuda and gate.dtype == up.dtype \
             and gate.dtype in (torch.bfloat16, torch.float16, torch.float32):

@@ -445,10 +445,18 @@ def gemm_swiglu_supported(M, N, K, dtype):
             and M * K * 2 < 2 ** 31 and N * K * 2 < 2 ** 31)
 
 
-def gemm_swiglu_fwd(x, w_gate, w_up, save=True):
+def gemm_swiglu_few_supported(M, N, K, dtype):
+    """The same for few tokens: shapes whose two products would each be a stream over their
+    weights (see axn_gemm_swiglu_fwd_few)."""
+    return (dtype in _GEMM16 and 0 < M <= 64 and N > 0 and N % 8 == 0 and K > 0 and K % 8 == 0
+            and K < _FAR_ROWS and _workspace_bytes(GEMM_FWD, M, N, K) == 0)
+
+
+def gemm_swiglu_fwd(x, w_gate, w_up, save=True, few=False):
     """silu(X Wg^T) * (X Wu^T) in one launch.  x [M,K], w_gate / w_up [N,K], bf16 or
     fp16.  Returns (h, gate, up); gate and up (the pre-activations, for the backward
-    pass) are None unless `save`.  Callers check `gemm_swiglu_supported` first."""
+    pass) are None unless `save`.  Callers check `gemm_swiglu_supported` first, or
+    `gemm_swiglu_few_supported` for `few`."""
     _require_gpu(x, w_gate, w_up)
     if not (x.dtype == w_gate.dtype == w_up.dtype):
         raise TypeError("operand dtypes differ: %s, %s, %s" % (x.dtype, w_gate.dtype, w_up.dtype))
@@ -468,8 +476,8 @@ def gemm_swiglu_fwd(x, w_gate, w_up, save=True):
     h = torch.empty((M, N), dtype=x.dtype, device=x.device)
     gate = torch.empty_like(h) if save else None
     up = torch.empty_like(h) if save else None
-    nv.call("axn_gemm_swiglu_fwd", nv.ptr(x), nv.ptr(w_gate), nv.ptr(w_up), nv.ptr(h), nv.ptr(gate),
-            nv.ptr(up), nv.dtype_code(x.dtype), M, N, K, ldx, ldg, N, nv.current_stream())
+    nv.call("axn_gemm_swiglu_fwd_few" if few else "axn_gemm_swiglu_fwd", nv.ptr(x), nv.ptr(w_gate),
+            nv.ptr(w_up), nv.ptr(h), nv.ptr(gate), nv.ptr(up), nv.dtype_code(x.dtype), M, N, K, ldx, ldg, N, nv.current_stream())
     return h, gate, up
 
 

@@ -179,6 +179,18 @@ def test_gate_up_forward_argument_errors():
     assert "M % 256 == 0" in _err()
 
 
+def test_gate_up_forward_of_few_rows_argument_errors():
+    f = nv.load().axn_gemm_swiglu_fwd_few
+    ok = (nv.BF16, 16, 128, 64, 64, 64, 128, None)
+    assert f(A, A, None, A, A, A, *ok) == nv.AXN_EINVAL                  # no up weights
+    assert f(A, A, A, A, A, A, nv.F32, *ok[1:]) == nv.AXN_EINVAL         # 16-bit types only
+    assert f(A, A, A, A, ctypes.c_void_p(0x1008), A, *ok) == nv.AXN_EALIGN
+    assert f(A, A, A, A, None, None, nv.BF16, 16, 132, 64, 64, 64, 136, None) == nv.AXN_ESHAPE  # N % 8
+    assert f(A, A, A, A, None, None, nv.BF16, 65, 128, 64, 64, 64, 128, None) == nv.AXN_ESHAPE  # a row too many
+    assert f(A, A, A, A, None, None, nv.BF16, 16, 128, 64, 64, 1 << 24, 128, None) == nv.AXN_ESHAPE
+    assert "axn_gemm_swiglu_fwd_few" in _err()
+
+
 def test_dgrad_pair_argument_errors():
     f = nv.load().axn_gemm_dgrad_pair
     tail = (128, 128, 128, 128, 128, 128, None)      # N2, K, lddy, ldw, lddx, stream

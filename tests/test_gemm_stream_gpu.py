@@ -75,3 +75,52 @@ def test_a_workspace_too_small_or_misaligned_for_parts(M, N, K, nbytes, offset):
         nv.call("axn_gemm_any_n", 0, nv.ptr(X), nv.ptr(W), None, nv.ptr(out), None, nv.BF16, M, N, K, K, K, N,
                 nv.EPI_NONE, 0, nv.BF16, where, size, nv.current_stream())
     assert torch.equal(got, want) and bool((ws == 7).all())
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(8, 8), (24, 64), (1000, 72), (4096, 328), (4104, 1024), (8192, 264), (8200, 264),
+                                 (16392, 200), (72, 8200)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gate_up_of_few_tokens(M, N, K, dtype):
+    """Pre-activations of whole numbers are exact, the activation is the separate kernel's on them bit for bit,
+    nothing is written outside the outputs, and random operands of up to 32 tokens give the two products' bits."""
+    from axonn_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+
+    def rows(n, fill):
+        full = torch.full((n + 1, K + 8), float("nan"), dtype=dtype, device="cuda")
+        full[:n, :K] = fill(n).to(dtype)
+        return full[:n, :K]
+
+    def whole(n):
+        return torch.randint(-2, 3, (n, K), generator=gen, device="cuda")
+
+    X, G, U = rows(M, whole), rows(N, whole), rows(N, whole)
+    full = [torch.full((M + 1, N + 8), CANARY, dtype=dtype, device="cuda") for _ in range(3)]
+    h, gate, up = (f[:M, :N] for f in full)
+    nv.call("axn_gemm_swiglu_fwd_few", nv.ptr(X), nv.ptr(G), nv.ptr(U), nv.ptr(h), nv.ptr(gate), nv.ptr(up),
+            nv.dtype_code(dtype), M, N, K, K + 8, K + 8, N + 8, nv.current_stream())
+    assert torch.equal(gate.double(), (X.double() @ G.double().t()).to(dtype).double())
+    assert torch.equal(up.double(), (X.double() @ U.double().t()).to(dtype).double())
+    assert torch.equal(h, ops.swiglu_fwd(gate.contiguous(), up.contiguous()))
+    for f, view in zip(full, (h, gate, up)):
+        view.fill_(CANARY)
+        assert torch.equal(f, torch.full_like(f, CANARY)), "written outside the output"
+
+    def random(n):
+        return torch.randn(n, K, generator=gen, device="cuda") * 0.1
+
+    X, G, U = rows(M, random), rows(N, random), rows(N, random)
+    h, none_g, none_u = ops.gemm_swiglu_fwd(X, G, U, save=False, few=True)
+    assert none_g is None and none_u is None
+    sfx = "" if dtype == torch.bfloat16 else "_f16"
+    for w, out in ((G, gate), (U, up)):   # (without a workspace: always the stream)
+        nv.call("axn_gemm_fwd" + sfx, nv.ptr(X), nv.ptr(w), None, nv.ptr(out), None, M, N, K, K + 8, K + 8, N + 8,
+                nv.EPI_NONE, nv.current_stream())
+    want = ops.swiglu_fwd(gate.contiguous(), up.contiguous())
+    if M <= 32:
+        assert torch.equal(h, want)
+    else:   # other order of sums: a rounding of each factor and of the product
+        eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        assert ((h.double() - want.double()).norm() / want.double().norm()) < 4 * eps

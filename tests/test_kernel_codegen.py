@@ -142,6 +142,30 @@ def test_stream_kernels_touch_no_fragment_before_its_wait(tmp_path_factory):
         assert reads > 0, name
 
 
+def test_gate_up_stream_kernels_touch_no_fragment_before_its_wait(tmp_path_factory):
+    """The same for the gate/up forward of a few tokens."""
+    kernels = {k: v for k, v in _device_asm(tmp_path_factory, "gemm_stream").items() if "gate_up_stream" in k}
+    assert len(kernels) == 18, len(kernels)   # 3 token ranges x 3 heights x 2 types
+    for name, body in kernels.items():
+        assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", body), name
+        pending, reads, in_asm = set(), 0, False
+        for line in body.split("\n"):
+            in_asm = (in_asm or "#APP" in line or "#ASMSTART" in line) and "#NO_APP" not in line and "#ASMEND" not in line
+            s = line.split(";")[0].strip()
+            used = {int(v) for v in re.findall(r"\bv(\d+)\b", s)}
+            for a, b in re.findall(r"\bv\[(\d+):(\d+)\]", s):
+                used |= set(range(int(a), int(b) + 1))
+            if in_asm and s.startswith("ds_read_b128"):   # (not the compiler's own reads)
+                reads += 1
+                first, last = map(int, re.search(r"v\[(\d+):(\d+)\]", s).groups())
+                pending |= set(range(first, last + 1))
+            elif s.startswith("s_waitcnt") and "lgkmcnt(0)" in s:
+                pending = set()
+            else:
+                assert not used & pending, (name, s)
+        assert reads > 0, name
+
+
 @pytest.mark.parametrize("source", ["stream_probe", "embedding"])
 def test_hand_written_stores_are_followed_by_their_wait_states(tmp_path_factory, source):
     """A store of more than 8 bytes needs wait states before its data registers are written

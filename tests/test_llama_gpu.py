@@ -297,6 +297,37 @@ def test_gate_up_forward_rejects_what_it_cannot_run():
         ops.gemm_swiglu_fwd(x.float(), w.float(), w.float())
 
 
+@pytest.mark.parametrize("tokens", [1, 32, 64, 65])
+def test_generation_runs_gate_up_in_one_launch(tokens):
+    """Up to 64 tokens without gradients: one launch, the output of the three calls; with gradients on, with a
+    hook on a projection, and past 64 tokens the projections are called themselves."""
+    from launches import launches
+    from transformers import LlamaConfig
+    from transformers.models.llama.modeling_llama import LlamaMLP
+
+    import axonn_amd.axonn as ax
+    from axonn_amd.models.transformers import modify_llama, parallelize
+
+    ax.init(1, 1, 1, 1)
+    cfg = LlamaConfig(hidden_size=128, intermediate_size=384, num_attention_heads=4, num_key_value_heads=2,
+                      num_hidden_layers=1, vocab_size=32)
+    with parallelize(cfg):
+        mlp = LlamaMLP(cfg)
+    mlp.forward = modify_llama.modified_mlp_forward.__get__(mlp)
+    mlp = mlp.cuda().bfloat16()
+    x = torch.randn(1, tokens, 128, device="cuda").bfloat16()
+    separate = mlp(x).detach()   # gradients on
+    with torch.no_grad():
+        assert len(launches(lambda: mlp(x))) == (2 if tokens <= 64 else 4)
+        fused = mlp(x)
+        handle = mlp.up_proj.register_forward_hook(lambda module, args, out: out * 0)
+        assert torch.equal(mlp(x), torch.zeros_like(x))
+        handle.remove()
+    if tokens <= 32 or tokens > 64:
+        assert torch.equal(fused, separate)
+    assert rel(np64(fused), np64(separate)) < 1e-2
+
+
 def test_mlp_with_one_launch_gate_up_equals_the_separate_path(monkeypatch):
     """The patched MLP at a whole-tile shape takes the one-launch gate/up forward; with
     that path switched off it takes three launches.  Output and weight gradients agree bit

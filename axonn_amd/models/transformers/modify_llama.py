@@ -29,10 +29,9 @@ _original_mlp_forward = None
 
 
 class SwiGLU(torch.autograd.Function):
-    """silu(gate) * up with a one-pass backward."""
+    """silu(gate) * up with a one-pass backward.  (No torch.amp decorators here and below: see AsyncLinear.)"""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
     def forward(ctx, gate, up):
         shape = gate.shape
         g2, u2 = gate.reshape(-1, shape[-1]), up.reshape(-1, shape[-1])
@@ -41,7 +40,6 @@ class SwiGLU(torch.autograd.Function):
         return ops.swiglu_fwd(g2, u2).reshape(shape)
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, grad_out):
         g2, u2 = ctx.saved_tensors
         d2 = grad_out.reshape(-1, ctx.shape[-1]).to(g2.dtype)
@@ -60,7 +58,6 @@ class GateUpSwiGLU(torch.autograd.Function):
     results), and the two wgrads as one launch."""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
     def forward(ctx, x, w_gate, w_up, shape, save=True):
         dt = _compute_dtype(x, w_gate.reshape(shape))
         x2 = x.reshape(-1, x.shape[-1]).to(dt)
@@ -72,7 +69,6 @@ class GateUpSwiGLU(torch.autograd.Function):
         return h.reshape(*x.shape[:-1], shape[0])
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, grad_out):
         x2, w_gate, w_up, gate, up = ctx.saved_tensors
         dt = ctx.compute_dtype

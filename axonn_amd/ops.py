@@ -22,7 +22,7 @@ EPILOGUES = {
 
 def _require_gpu(*tensors):
     for t in tensors:
-        if t is not None and not t.is_cuda:
+        if not (t is None or t.is_cuda):
             raise RuntimeError(
                 "axonn_amd kernels run on the GPU only; got a tensor on %s" % t.device
             )
@@ -49,6 +49,10 @@ _FAR_ROWS = 1 << 22
 
 
 def _prep_bf16(t):
+    if t.dim() == 2 and t.is_contiguous():   # nearly always (the rest of this costs 0.5 us more)
+        ld = t.shape[1]
+        if ld % 8 == 0 and t.data_ptr() % 16 == 0:
+            return t, ld
     t, ld = _rows(t)
     if not _bf16_ok(t, ld) or (ld >= _FAR_ROWS and ld > t.shape[1]):
         t = t.contiguous().clone()
@@ -345,6 +349,11 @@ def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None):
     return dx, out
 
 
+@functools.lru_cache(maxsize=4096)
+def _dbias_workspace_bytes(M, N):
+    return nv.load().axn_dgelu_dbias_workspace_bytes(M, N)
+
+
 def dgelu_dbias(dy, z=None, want_dbias=True, dbias_out=None, accumulate=False):
     """dZ = dY * gelu'(Z) (when z is given) and dbias = column sums of dZ (fp32).
     Returns (dz, dbias); dz is dy itself when z is None."""
@@ -394,7 +403,7 @@ def dgelu_dbias(dy, z=None, want_dbias=True, dbias_out=None, accumulate=False):
         dbias = dbias_out if dbias_out is not None else torch.empty(N, dtype=torch.float32, device=dy.device)
         if dbias.dtype != torch.float32 or dbias.numel() != N:
             raise ValueError("dbias must be fp32 with %d elements" % N)
-        ws_bytes = nv.load().axn_dgelu_dbias_workspace_bytes(M, N)
+        ws_bytes = _dbias_workspace_bytes(M, N)
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dy.device)
     elif z is None:
         return dy, None

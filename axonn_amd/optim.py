@@ -219,16 +219,10 @@ class CPUAdam(Optimizer):
             beta1, beta2 = group["betas"]
             hp = ops.adam_hparams(t, group["lr"], beta1, beta2, group["eps"],
                                   group["weight_decay"])
-            ops.mt_adam(
-                [grads[lo:hi]],
-                [self.model_params_fp32[lo:hi]],
-                [self.exp_avg[lo:hi]],
-                [self.exp_avg_sq[lo:hi]],
-                [self.model_params_fp16[lo:hi]] if self._writes_lowp else None,
-                hp,
-                inv_scale=inv_scale,
-                scan=scan,
-            )
+            whole = hi - lo == grads.numel()   # one group: the buffers themselves
+            g, p, m, v, low = ([t if whole else t[lo:hi]] for t in (
+                grads, self.model_params_fp32, self.exp_avg, self.exp_avg_sq, self.model_params_fp16))
+            ops.mt_adam(g, p, m, v, low if self._writes_lowp else None, hp, inv_scale=inv_scale, scan=scan)
         skipped = False
         if scan is not None:
             skipped = bool(scan.found_inf.item())  # one 4-byte read back per step

@@ -287,3 +287,36 @@ def test_feature_counts_that_are_not_multiples_of_eight(dtype, in_f, out_f):
         assert rel(y, yr.detach()) < tol and rel(x.grad, xr.grad) < tol
         assert rel(layer.weight.grad, ref.weight.grad) < tol
         assert rel(layer.bias.grad, ref.bias.grad) < tol
+
+
+@pytest.mark.parametrize("autocast", [False, True])
+@pytest.mark.parametrize("shape", [(24,), (5, 24), (3, 7, 24), (1, 24)])
+def test_results_do_not_depend_on_grad_mode_or_on_where_backward_is_called(shape, autocast):
+    """Without gradients nothing is kept for a backward pass; a backward pass called inside an autocast
+    region computes what it computes outside, in the forward's type."""
+    from axonn_amd.intra_layer import Linear
+
+    torch.manual_seed(3)
+    own = torch.float32 if autocast else torch.bfloat16
+    layers = [Linear(24, 40, bias=bias, fused_activation=act).cuda().to(own)
+              for bias, act in ((True, "gelu"), (True, None), (False, "gelu"), (False, None))]
+    for layer in layers:
+        with torch.no_grad():
+            for p in layer.parameters():
+                p.normal_(0, 0.1)
+        x = torch.randn(*shape, device="cuda").to(own).requires_grad_(True)
+        found = []
+        for backward_inside in (False, True):
+            x.grad = None
+            layer.zero_grad(set_to_none=True)
+            with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+                y = layer(x)
+                with torch.no_grad():
+                    assert torch.equal(layer(x), y)
+            dy = torch.linspace(-1, 1, y.numel(), device="cuda").reshape(y.shape).to(y.dtype)
+            with torch.autocast("cuda", dtype=torch.float16, enabled=backward_inside):
+                y.backward(dy)
+            assert y.shape == (*shape[:-1], 40) and x.grad.shape == x.shape and x.grad.dtype == own
+            found.append([y.detach(), x.grad] + [p.grad for p in layer.parameters()])
+        for a, b in zip(*found):
+            assert a.dtype == b.dtype and torch.equal(a, b)

@@ -19,9 +19,9 @@
 namespace axn {
 namespace {
 
-template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF>
+template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF, bool ODD = false>
 __global__ void __launch_bounds__(256) gemm_edge_kernel(const GemmArgs g) {
-  solo_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, true>(g);
+  solo_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, true, ODD>(g);
 }
 
 // Both gradients of a layer in one launch, as gemm_backward_kernel.
@@ -34,8 +34,12 @@ __global__ void __launch_bounds__(256) gemm_edge_backward_kernel(const GemmArgs 
     solo_gemm<256, 256, true, false, AXN_EPI_NONE, false, HALF, true>(gd);
 }
 
-template <int BM, int BN, bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
+template <int BM, int BN, bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF, bool ODD = false>
 int launch_edge_tile(const GemmArgs& in, hipStream_t stream) {
+  // Only the forward's output rows can be odd (the others have the width of an input); those of heads over
+  // vocabularies are, which have neither bias nor activation.
+  if constexpr (!ODD && AK && BKM && EPI == AXN_EPI_NONE && !OUT_F32)
+    if (in.ldc % 2 != 0 && !in.beta) return launch_edge_tile<BM, BN, AK, BKM, EPI, OUT_F32, HALF, true>(in, stream);
   GemmArgs g = in;
   g.tiles_m = (int)ceil_div(g.M, BM);
   g.tiles_n = (int)ceil_div(g.N, BN);
@@ -45,7 +49,7 @@ int launch_edge_tile(const GemmArgs& in, hipStream_t stream) {
     return AXN_ELIMIT;
   }
   constexpr size_t lds = 5 * BM * 64 * 2;   // five slots of the A tile's size
-  void (*kern)(const GemmArgs) = gemm_edge_kernel<BM, BN, AK, BKM, EPI, OUT_F32, HALF>;
+  void (*kern)(const GemmArgs) = gemm_edge_kernel<BM, BN, AK, BKM, EPI, OUT_F32, HALF, ODD>;
   {
     static std::atomic<unsigned long long> lds_allowed{0};   // per template instance
     const int rc = allow_lds((const void*)kern, lds, lds_allowed);

@@ -138,6 +138,48 @@ __device__ __forceinline__ void store_row8(float (&v)[8], const float (&bias)[8]
   }
 }
 
+// An output row of 16-bit elements that starts 2 bytes off a 4-byte boundary (every second row of an odd row
+// stride): a lane stores its predecessor's last element and its own first seven, on the boundary.  Stores off
+// it cost 5 us a round of 256 x 256 tiles: 2048 x 50257, contraction 2048 418 us (50256 and 50258 columns,
+// whose rows start on 4-byte boundaries, 385 and 388), this way 388 as well (in short
+// runs 357 -> 337; 777 x 19999, 768 43.8 -> 36.3).
+// y: the lane's 8 columns; before: the dword with the predecessor's last one (lead: there is none, the
+// wave's first columns); end: nobody takes the lane's own last one.
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+// before <- the same of the lane whose byte index is `from`.  One statement that nothing moves across: of the
+// builtin the compiler takes every row's exchange ahead of the first store, and spills.
+__device__ __forceinline__ void lanes_16_down(uint32_t (&b)[4], int from) {
+  asm volatile("ds_bpermute_b32 %0, %4, %0\n\tds_bpermute_b32 %1, %4, %1\n\tds_bpermute_b32 %2, %4, %2\n\t"
+               "ds_bpermute_b32 %3, %4, %3\n\ts_waitcnt lgkmcnt(0)"
+               : "+&v"(b[0]), "+&v"(b[1]), "+&v"(b[2]), "+&v"(b[3])
+               : "v"(from));
+}
+__device__ __forceinline__ void lanes_16_down(uint32_t (&b)[2], int from) {
+  asm volatile("ds_bpermute_b32 %0, %2, %0\n\tds_bpermute_b32 %1, %2, %1\n\ts_waitcnt lgkmcnt(0)"
+               : "+&v"(b[0]), "+&v"(b[1])
+               : "v"(from));
+}
+__device__ __forceinline__ void store_row8_odd(uint16_t* to, const u32x4& y, uint32_t before, bool lead, bool end) {
+  typedef typename Unaligned<u32x4, 4>::type u32x4_mem;
+  struct __attribute__((packed, aligned(4))) u32x3_mem {
+    uint32_t d[3];
+  };
+  const bool off = ((uintptr_t)to & 2) != 0;
+  u32x4 v = y;
+  if (off) {
+    v[0] = (y[0] << 16) | (before >> 16);
+#pragma unroll
+    for (int d = 1; d < 4; ++d) v[d] = (y[d] << 16) | (y[d - 1] >> 16);
+  }
+  if (off && lead) {
+    *to = (uint16_t)y[0];
+    *(u32x3_mem*)(to + 1) = u32x3_mem{{v[1], v[2], v[3]}};
+  } else {
+    *(u32x4_mem*)((char*)to - (off ? 2 : 0)) = v;
+  }
+  if (off && end) to[7] = (uint16_t)(y[3] >> 16);
+}
+
 // The same for one element.
 template <int EPI, bool OUT_F32, bool HALF>
 __device__ __forceinline__ void store_one(float x, const GemmArgs& g, int row, int col) {
@@ -393,9 +435,11 @@ __device__ __forceinline__ void wait_vmcnt() {
 //     contraction steps of one tile and not the whole operand: operands of any size, row
 //     strides up to 2^22 elements (2^23 on the 128 x 128 tile).  A resource per copy instead
 //     put 340 scalar and vector instructions into a stage and made it 60 % longer;
-//   * stores of rows and columns inside the output only, with the alignment of one element.
+//   * stores of rows and columns inside the output only, with the alignment of one element.  ODD: the
+//     output's row stride is odd (store_row8_odd; a kernel of its own: with both epilogues in one the
+//     compiler converts what both store ahead of their branch, and spills).
 template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF,
-          bool EDGE = false>
+          bool EDGE = false, bool ODD = false>
 __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   constexpr uint32_t kOutside = 0x80000000u;
   constexpr int WTM = BM / 2, WTN = BN / 2, FRM = BM / 32, FRN = BN / 32;
@@ -757,24 +801,62 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
 #pragma unroll
     for (int t = 0; t < FRN / 2; ++t)
       if (!EDGE || ocol + 32 * t + 8 <= g.N) load_bias8<EP, HALF>(bias[t], g, ocol + 32 * t);
+    static_assert(!ODD || (EDGE && A_KMAJOR && B_KMAJOR && EP == AXN_EPI_NONE && !OUT_F32), "store_row8_odd");
+    if constexpr (ODD) {
+      using lp = std::conditional_t<HALF, _Float16, __bf16>;
+      using lpx8 = std::conditional_t<HALF, f16x8, bf16x8>;
 #pragma unroll
-    for (int i = 0; i < FRM; ++i)
+      for (int i = 0; i < FRM; ++i) {
+        const int row = orow + 16 * i;
+        u32x4 y[FRN / 2];
+        uint32_t before[FRN / 2];   // of each 8 columns: the dword with the one before them
 #pragma unroll
-      for (int t = 0; t < FRN / 2; ++t) {
-        const f32x4 lo = acc[i][2 * t], hi = acc[i][2 * t + 1];
-        float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        const int row = orow + 16 * i, col = ocol + 32 * t;
-        if constexpr (EDGE) {
+        for (int t = 0; t < FRN / 2; ++t) {
+          lpx8 y8;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            y8[e] = (lp)acc[i][2 * t][e];
+            y8[4 + e] = (lp)acc[i][2 * t + 1][e];
+          }
+          y[t] = __builtin_bit_cast(u32x4, y8);
+          // it lies in the lane 16 further down; for lanes 0 .. 15 in lanes 48 .. 63 at t - 1
+          before[t] = lane >= 48 ? (t > 0 ? y[t - 1][3] : 0u) : y[t][3];
+        }
+        lanes_16_down(before, ((lane + 48) & 63) * 4);
+#pragma unroll
+        for (int t = 0; t < FRN / 2; ++t) {
+          const int col = ocol + 32 * t;
           if (row >= g.M || col >= g.N) continue;
           if (col + 8 > g.N) {
             f32x4* to = (f32x4*)(tail + ((lane & 15) + 16 * i) * 8);
-            to[0] = lo;
-            to[1] = hi;
+            to[0] = acc[i][2 * t];
+            to[1] = acc[i][2 * t + 1];
             continue;
           }
+          store_row8_odd((uint16_t*)go.C + (int64_t)row * go.ldc + col, y[t], before[t], t == 0 && lane < 16,
+                         (t == FRN / 2 - 1 && lane >= 48) || col + 16 > g.N);
         }
-        store_row8<EP, OUT_F32, HALF, EDGE>(v, bias[t], go, row, col);
       }
+    } else {
+#pragma unroll
+      for (int i = 0; i < FRM; ++i)
+#pragma unroll
+        for (int t = 0; t < FRN / 2; ++t) {
+          const f32x4 lo = acc[i][2 * t], hi = acc[i][2 * t + 1];
+          float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          const int row = orow + 16 * i, col = ocol + 32 * t;
+          if constexpr (EDGE) {
+            if (row >= g.M || col >= g.N) continue;
+            if (col + 8 > g.N) {
+              f32x4* to = (f32x4*)(tail + ((lane & 15) + 16 * i) * 8);
+              to[0] = lo;
+              to[1] = hi;
+              continue;
+            }
+          }
+          store_row8<EP, OUT_F32, HALF, EDGE>(v, bias[t], go, row, col);
+        }
+    }
     if constexpr (EDGE) {
       const int end = g.N / 8 * 8, first = n0 + wn * WTN;
       if (end < g.N && end >= first && end < first + WTN) {

@@ -148,3 +148,27 @@ def test_bias_of_the_operands_type_equals_its_fp32_copy(M, N, K, dtype):
             assert act is None or torch.equal(got[1], want[1])
     pre = X.double() @ W.double().t() + b[:N].double()
     assert close(ops.gemm_fwd(X, W, bias=b[:N])[0], pre, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(65, 1, 64), (65, 7, 64), (129, 127, 64), (300, 129, 128), (257, 255, 72),
+                                   (700, 1016, 64), (2100, 4093, 64), (3000, 7003, 64), (2048, 16385, 64)])
+def test_odd_rows_hold_what_even_rows_hold(M, N, K, dtype):
+    """The forward's output at odd row strides, on every tile and with every number of columns behind the last
+    whole vector: the bits of the same product at an even stride, and nothing between the rows is touched."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    X, W = (torch.randn(n, K, generator=g, device="cuda").to(dtype) for n in (M, N))
+
+    def product(ld):
+        buf = torch.full((M * ld + 64,), 7.0, device="cuda", dtype=dtype)
+        nv.call("axn_gemm_any_n", 0, nv.ptr(X), nv.ptr(W), None, nv.ptr(buf), None, nv.dtype_code(dtype), M, N, K, K,
+                K, ld, nv.EPI_NONE, 0, nv.dtype_code(dtype), None, 0, nv.current_stream())
+        assert bool((buf[M * ld:] == 7).all())
+        rows = buf[:M * ld].view(M, ld)
+        assert bool((rows[:, N:] == 7).all())
+        return rows[:, :N]
+
+    even = product(N + N % 2)
+    assert close(even, X.double() @ W.double().t(), dtype)
+    assert torch.equal(product(N + 1 - N % 2), even)
+    assert torch.equal(product(N + 5 - N % 2), even)

@@ -189,6 +189,22 @@ EdgeTile edge_tile(long long M, long long N, long long Kc, const EpilogueTime& e
   return best;
 }
 
+// Outputs made of whole 128 x 128 tiles but not of larger ones: whether the small tile without bounds is ahead
+// of the larger ones with them.  Two workgroups share a CU and do not run in rounds, so its time grows
+// evenly with their number.  Larger tiles have to be estimated 5 % faster, beyond one round of them, where the
+// power cap stretches the estimate, 20 %.  us, small tile / larger ones, of M x N, contraction:
+//   2048 x 50304, 2048  442 / 363      8192 x 5504, 2048  149 / 134   2048 x 5504, 8192 (weight gradient)  163 / 139
+//   4096 x 50304, 768   398 / 298      4096 x 3200, 3200   83 / 67    3200 x 10240, 2560 (input gradient)  143 / 158
+//   896 x 14336, 4096    99 / 82       8192 x 1920, 1920   52 / 46    2176 x 4096, 4096, GELU               83 / 87
+bool small_tile_ahead(long long M, long long N, long long Kc, const EpilogueTime& epilogue) {
+  const double w = (double)(M / 128) * (double)(N / 128), stages = (double)(Kc / 64);
+  const double alone = 0.69 * stages + epilogue.us[2], shared = 1.2 + 0.936 * stages + epilogue.us[3];
+  const double small = w <= 256 ? alone : w <= 512 ? alone + (shared - alone) * (w - 256) / 256 : shared * w / 512;
+  double large = 0;
+  if (edge_tile(M, N, Kc, epilogue, &large) == EDGE_128x128) return true;
+  return small < large * (ceil_div(M, 256) * ceil_div(N, 256) <= 256 ? 1.05 : 1.2);
+}
+
 int launch_edge(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, bool half,
                 hipStream_t stream) {
   const int64_t ld = g.lda > g.ldb ? g.lda : g.ldb;
@@ -227,8 +243,12 @@ int launch_whole(const GemmArgs& g, hipStream_t stream) {
   // (+4..11 % against the small tile, measured at 80, 96, 112 and 128 tiles).
   if (small_spans && whole256 && tiles256 > 64 && tiles256 <= 128)
     return launch_rest<AK, BKM, EPI, OUT_F32, HALF>(g, stream);
-  if (small_spans && whole128 && tiles128 < (1LL << 31))
-    return launch_solo<128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
+  if (small_spans && whole128 && tiles128 < (1LL << 31)) {
+    bool small_tile = true;
+    if constexpr (EPI != EPI_PAIR)
+      small_tile = whole256 || small_tile_ahead(g.M, g.N, g.Kc, epilogue_time(g, EPI, OUT_F32));
+    if (small_tile) return launch_solo<128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
+  }
   if constexpr (EPI == EPI_PAIR) {
     set_error("gemm_pair: needs whole 128 x 128 tiles, contractions that are multiples of 64 and "
               "operands below 2 GiB (got M=%d, N=%d, K=%d)", g.M, g.N, g.Kc);

@@ -285,3 +285,25 @@ def test_the_tile_of_a_ragged_forward_follows_its_epilogue(M, N, K, none, bias, 
             check(fz, z, pre)
         else:
             check(fy, y, pre)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols,kc", [(3968, 3968, 1024), (1920, 4096, 1920), (640, 2176, 4096), (3200, 3200, 192)])
+def test_outputs_of_whole_small_tiles_only(rows, cols, kc, dtype):
+    """Multiples of 128 that are none of 256 take the tile with bounds that is estimated to be faster, or the
+    small one: every product against 64 bits (one rounding to 16 bits of an fp32 sum)."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(rows + kc)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device="cuda").to(dtype)   # noqa: E731
+    a, b = draw(rows, kc), draw(cols, kc)
+    at, bt = a.t().contiguous(), b.t().contiguous()
+    want = a.double() @ b.double().t()
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for got in (ops.gemm_fwd(a, b)[0], ops.gemm_dgrad(a, bt), ops.gemm_wgrad(at, bt)):
+        assert bool(((got.double() - want).abs() <= ulp * want.abs() + 1e-5 * want.abs().max()).all())
+    y, z = ops.gemm_fwd(a * 0.05, b, bias=torch.ones(cols, device="cuda"), activation="gelu", save_z=True)
+    pre = (a * 0.05).double() @ b.double().t() + 1
+    assert bool(((z.double() - pre).abs() <= ulp * pre.abs() + 1e-5 * pre.abs().max()).all())
+    gelu = torch.nn.functional.gelu(pre)
+    assert bool(((y.double() - gelu).abs() <= ulp * gelu.abs() + 1e-5 * gelu.abs().max()).all())

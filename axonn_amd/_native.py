@@ -88,6 +88,7 @@ SYMBOLS = {
     "axn_gemm_any_n": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _i64, _int,
                               _int, _int, _vp, _sz, _vp]),
     "axn_pad_rows16": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
+    "axn_pad_rows16_to": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "axn_gemm_f32_workspace_bytes": (_sz, [_int, _i64, _i64, _i64]),
     "axn_gemm_fwd_f32_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "axn_gemm_dgrad_f32_ws": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp]),

@@ -399,12 +399,21 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void*
               : launch_gemm_bf16(layout, g, epilogue, out_f32, (hipStream_t)stream);
 }
 
-int axn_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, void* stream) {
-  const char* name = "axn_pad_rows16";
+static int pad_rows16(const char* name, const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst,
+                      void* stream) {
   REQUIRE(src && dst, AXN_EINVAL, "%s: null pointer", name);
   REQUIRE(M >= 1 && N >= 1 && ld >= N, AXN_EINVAL, "%s: M, N >= 1 and ld >= N expected", name);
+  REQUIRE(ld_dst >= N && ld_dst % 8 == 0, AXN_EINVAL, "%s: ld_dst >= N and a multiple of 8 expected", name);
   REQUIRE(((uintptr_t)src & 1u) == 0 && aligned16(dst), AXN_EALIGN, "%s: misaligned pointer", name);
-  return launch_pad_rows16(src, dst, M, N, ld, (hipStream_t)stream);
+  return launch_pad_rows16(src, dst, M, N, ld, ld_dst, (hipStream_t)stream);
+}
+
+int axn_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, void* stream) {
+  return pad_rows16("axn_pad_rows16", src, dst, M, N, ld, (N + 7) / 8 * 8, stream);
+}
+
+int axn_pad_rows16_to(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst, void* stream) {
+  return pad_rows16("axn_pad_rows16_to", src, dst, M, N, ld, ld_dst, stream);
 }
 
 int axn_gemm_fwd_ws(const void* X, const void* W, const float* bias, void* Y, void* Zsave, int dtype,

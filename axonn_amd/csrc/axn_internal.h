@@ -226,7 +226,8 @@ int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
                        void* ws, size_t ws_bytes, hipStream_t stream);
 
 // dst[M][8 ceil(N / 8)] = src[M][N] (row stride ld) of 16-bit elements, zeros behind N.
-int launch_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, hipStream_t stream);
+int launch_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst,
+                      hipStream_t stream);
 
 // ---- SwiGLU activation of the Llama MLP and its backward -----------------------
 int launch_swiglu_fwd(const void* gate, const void* up, void* out, int dtype, int64_t M,

@@ -379,7 +379,7 @@ int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
 
 // ---- rows of any width, padded with zeros to a multiple of 8 elements -----------------
 // Bound by its bytes: 8 elements a lane, the reads with the alignment of one element (2048 x 50257:
-// 64 us, 6.4 TB/s).
+// 64 us, 6.4 TB/s).  The destination's rows are ld_dst elements apart, zeros up to there.
 namespace {
 struct __attribute__((packed, aligned(2))) Any8 {
   uint4 v;
@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(256)
                       int64_t ld, int64_t per_row) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= M * per_row) return;
-  const int64_t row = idx / per_row, col = (idx - row * per_row) * 8;
+  const int64_t row = idx / per_row, col = (idx - row * per_row) * 8;   // per_row groups of 8 in a padded row
   const uint16_t* from = src + row * ld + col;
   uint4 v = {0, 0, 0, 0};
   if (col + 8 <= N) {
@@ -406,8 +406,9 @@ __global__ void __launch_bounds__(256)
 }
 }  // namespace
 
-int launch_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, hipStream_t stream) {
-  const int64_t per_row = (N + 7) / 8, groups = (M * per_row + 255) / 256;
+int launch_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst,
+                      hipStream_t stream) {
+  const int64_t per_row = ld_dst / 8, groups = (M * per_row + 255) / 256;
   if (groups > 0x7fffffffLL) {
     set_error("pad_rows16: too many elements");
     return AXN_ELIMIT;

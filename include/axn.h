@@ -199,6 +199,9 @@ AXN_API int axn_gemm_any_n(int op, const void* A, const void* B, const void* bia
 /* dst[M][n8] = src[M][N] of 16-bit elements (rows of ld elements, 2-byte aligned), n8 the next
  * multiple of 8, zeros behind column N; dst 16-byte aligned. */
 AXN_API int axn_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, void* stream);
+/* The same with destination rows of ld_dst elements, a multiple of 8, zeros up to there. */
+AXN_API int axn_pad_rows16_to(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst,
+                              void* stream);
 
 /* Gate and up projection of a gated MLP with the activation in the epilogue:
  *   gate = X Wg^T,  up = X Wu^T,  H = silu(gate) * up     (one launch)

@@ -172,3 +172,21 @@ def test_odd_rows_hold_what_even_rows_hold(M, N, K, dtype):
     assert close(even, X.double() @ W.double().t(), dtype)
     assert torch.equal(product(N + 1 - N % 2), even)
     assert torch.equal(product(N + 5 - N % 2), even)
+
+
+@pytest.mark.parametrize("M,N,ld", [(3, 4097, 4103), (70, 5000, 5000), (300, 4159, 4160), (9, 4160, 4161)])
+def test_wide_rows_are_padded_to_whole_lines(M, N, ld):
+    """Rows of 4096 elements and more start on 128-byte lines, with zeros up to the next row."""
+    from axonn_amd import ops
+
+    src = torch.randn(M, ld, device="cuda").bfloat16()[:, :N]
+    out = ops._pad_rows(src)
+    assert out.shape == (M, N + (-N) % 8) and out.stride(0) == N + (-N) % 64
+    assert torch.equal(out[:, :N], src)
+    assert not out.as_strided((M, out.stride(0)), (out.stride(0), 1))[:, N:].any()
+    w, x = torch.randn(N, 64, device="cuda").bfloat16(), torch.randn(M, 64, device="cuda").bfloat16()
+    dx, dw = ops.gemm_bwd(src, w, x) if N % 8 else (ops._dgrad_any_n(out, w, N),
+                                                   ops._wgrad_any_n(out, x, N, None, False, src.dtype))
+    for got, want in ((dx, src.double() @ w.double()), (dw, src.double().t() @ x.double())):
+        # bf16 rounding of the result and fp32 sums
+        assert float((got.double() - want).norm() / want.norm()) < 2.0 ** -8

@@ -3,7 +3,7 @@
 // which is what autograd derives from the reference's `x + bias`
 // (axonn/intra_layer/fully_connected.py:348) followed by the caller's exact-erf
 // nn.GELU.  Lanes move 16 bytes (8 bf16 columns); column sums are kept in
-// registers over a band of rows, combined through LDS, written as one fp32
+// registers over a band's rows, combined through LDS, written as one fp32
 // partial row per band and reduced over bands in a fixed order by a second
 // kernel, so the result does not depend on scheduling.
 //
@@ -25,7 +25,6 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int EW_TX = 64;          // lanes along columns (8 columns each)
 constexpr int EW_TY = 4;           // row phases per workgroup
 constexpr int EW_COLS = EW_TX * 8; // 512 columns per workgroup
-constexpr int EW_BAND = 128;       // rows per workgroup (dGELU + dbias: column sums per band)
 // Non-temporal loads of dY and Z: 12 % faster when the operands come from HBM (62 -> 55 us),
 // 12 % slower when the memory-side cache holds them, which is the case in a training step
 // (dY was written by the layer behind a moment ago): off.
@@ -124,13 +123,15 @@ __device__ __forceinline__ void widen8(const Raw8<float>::type& v, float (&x)[8]
 // A thread walks its rows in groups of EW_GROUP: the loads of the next group are issued
 // before the stores of this one.  The memory counter of a wave is in order, so a load
 // behind a store returns only after the store is acknowledged; with the loads in front,
-// a wave waits for one store round trip per group and not per row.  Worth 3 % at
-// 8192 x 5120 bf16 (56.7 -> 55.1 us on MI355X): with 2.5 waves per SIMD the kernel is
-// bound by its arithmetic (about 24 operations per element) and by how little there is to
-// hide latency with, not by the memory system.  Shorter bands do not help (32 rows:
-// 68 us; the column sums then cost more than the better balance gains).  Rows of different
+// a wave waits for one store round trip per group and not per row (3 % at 8192 x 5120 bf16).
+// Band b is the chunks b, b + bands, b + 2 bands, ...: all workgroups together walk down one compact
+// window of the operands, where consecutive rows a band had each its own (us, from HBM, bf16: 8192 x 5120
+// 56.5 -> 51.3, 8192 x 14336 153 -> 136, 5000 x 8192 69 -> 50, sums alone 24.6 -> 17.0).  What bounds it is the
+// memory system, at 4.9 to 5.2 TB/s, beside about 24 operations an element.  Rows of different
 // groups never overlap, so dZ may still alias dY.
 constexpr int EW_GROUP = 4;
+constexpr int EW_CHUNK = EW_TY * EW_GROUP;   // rows a workgroup has in flight
+constexpr int EW_TURNS = 8;                  // most chunks a workgroup walks where that fills the chip
 
 template <typename T, bool HAS_Z>
 __global__ void __launch_bounds__(EW_TX* EW_TY)
@@ -139,9 +140,7 @@ __global__ void __launch_bounds__(EW_TX* EW_TY)
   typedef typename Raw8<T>::type raw;
   const int tx = threadIdx.x % EW_TX, ty = threadIdx.x / EW_TX;
   const int64_t col = (int64_t)blockIdx.x * EW_COLS + tx * 8;
-  const int64_t r0 = (int64_t)blockIdx.y * EW_BAND;
-  int64_t r1 = r0 + EW_BAND;
-  if (r1 > M) r1 = M;
+  const int64_t step = (int64_t)gridDim.y * EW_CHUNK;
   float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (col < N) {
     raw gy[EW_GROUP], gz[EW_GROUP];
@@ -149,15 +148,15 @@ __global__ void __launch_bounds__(EW_TX* EW_TY)
 #pragma unroll
       for (int u = 0; u < EW_GROUP; ++u) {
         const int64_t r = first + u * EW_TY;
-        if (r < r1) {
+        if (r < M) {
           gy[u] = load_raw8(dY + r * ld + col);
           if (HAS_Z) gz[u] = load_raw8(Z + r * ld + col);
         }
       }
     };
-    int64_t first = r0 + ty;
+    int64_t first = (int64_t)blockIdx.y * EW_CHUNK + ty;
     fetch(first);
-    while (first < r1) {
+    while (first < M) {
       float g[EW_GROUP][8];
 #pragma unroll
       for (int u = 0; u < EW_GROUP; ++u) {
@@ -169,12 +168,12 @@ __global__ void __launch_bounds__(EW_TX* EW_TY)
           for (int e = 0; e < 8; ++e) g[u][e] *= dgelu_exact(z[e]);
         }
       }
-      const int64_t next = first + EW_GROUP * EW_TY;
-      if (next < r1) fetch(next);
+      const int64_t next = first + step;
+      if (next < M) fetch(next);
 #pragma unroll
       for (int u = 0; u < EW_GROUP; ++u) {
         const int64_t r = first + u * EW_TY;
-        if (r < r1) {
+        if (r < M) {
           // g becomes what was stored: the sum of what wgrad reads
           if (HAS_Z) store8(dZ + r * ld + col, g[u]);
 #pragma unroll
@@ -197,24 +196,24 @@ __global__ void __launch_bounds__(EW_TX* EW_TY)
   }
 }
 
-// Column sums over the band partials in a fixed order: 64 columns per workgroup,
-// the bands split in 4 consecutive quarters summed by 4 threads each in band
-// order, the quarters then combined as (q0 + q1) + (q2 + q3).
-__global__ void __launch_bounds__(256)
+// Column sums over the band partials in a fixed order: 64 columns per workgroup, thread q of a
+// column's 16 adds bands q, q + 16, ..., the 16 sums are then added in order.
+__global__ void __launch_bounds__(1024)
     dbias_reduce_kernel(const float* partial, float* dbias, int64_t bands,
                         int64_t N, int beta) {
-  __shared__ float red[4][64];
+  __shared__ float red[16][64];
   const int tx = threadIdx.x & 63, q = threadIdx.x >> 6;
   const int64_t c = (int64_t)blockIdx.x * 64 + tx;
-  const int64_t per = (bands + 3) / 4;
-  const int64_t b0 = q * per, b1 = (b0 + per < bands) ? b0 + per : bands;
   float s = 0.f;
   if (c < N)
-    for (int64_t b = b0; b < b1; ++b) s += partial[b * N + c];
+#pragma unroll 4
+    for (int64_t b = q; b < bands; b += 16) s += partial[b * N + c];
   red[q][tx] = s;
   __syncthreads();
   if (q == 0 && c < N) {
-    const float t = (red[0][tx] + red[1][tx]) + (red[2][tx] + red[3][tx]);
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t += red[i][tx];
     dbias[c] = beta ? dbias[c] + t : t;
   }
 }
@@ -319,18 +318,38 @@ int launch_swiglu_bwd(const void* dout, const void* gate, const void* up, void* 
   return AXN_OK;
 }
 
+namespace {
+// Bands of the dGELU + dbias pass: as many as leave a workgroup one to eight chunks of rows, at most 640 workgroups
+// where there is a choice (the sums' traffic grows with them), and of those the number whose fullest CU has the
+// fewest chunks to walk.  Bands of 128 consecutive rows left 64 to 500 rows to 8 to 32 CUs (us, before -> now):
+// fp32 2048 x 4096 25.2 -> 20.2, 2900 x 6144 59.3 -> 47.1; bf16 256 x 4096 without sums 16 -> 9.
+int64_t dgelu_bands(int64_t M, int64_t N) {
+  const int64_t cols = (N + EW_COLS - 1) / EW_COLS, chunks = (M + EW_CHUNK - 1) / EW_CHUNK;
+  int64_t best = 0, least = 0;
+  for (int64_t turns = 1; turns <= EW_TURNS; ++turns) {
+    const int64_t bands = (chunks + turns - 1) / turns;
+    if (bands * cols > 640 && turns < EW_TURNS) continue;
+    const int64_t walk = (bands * cols + 255) / 256 * turns;
+    if (best == 0 || walk < least) best = bands, least = walk;
+  }
+  return best;
+}
+size_t band_sums_bytes(int64_t bands, int64_t N) { return (size_t)bands * (size_t)N * sizeof(float); }
+}  // namespace
+
 size_t dgelu_dbias_workspace_bytes(int64_t M, int64_t N) {
-  if (M <= 0 || N <= 0) return 0;
-  return (size_t)((M + EW_BAND - 1) / EW_BAND) * (size_t)N * sizeof(float);
+  return M <= 0 || N <= 0 ? 0 : band_sums_bytes(dgelu_bands(M, N), N);
 }
 
 int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
                        float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
                        void* ws, size_t ws_bytes, hipStream_t stream) {
-  const int64_t bands = (M + EW_BAND - 1) / EW_BAND;
+  int64_t bands = dgelu_bands(M, N);
+  // (a workspace for a sum per 128 rows is enough)
+  if (dbias != nullptr && ws_bytes < band_sums_bytes(bands, N)) bands = (M + EW_TURNS * EW_CHUNK - 1) / (EW_TURNS * EW_CHUNK);
   float* partial = nullptr;
   if (dbias != nullptr) {
-    if (ws == nullptr || ws_bytes < dgelu_dbias_workspace_bytes(M, N)) {
+    if (ws == nullptr || ws_bytes < band_sums_bytes(bands, N)) {
       set_error("dgelu_dbias: workspace too small (%zu bytes given, %zu needed)",
                 ws_bytes, dgelu_dbias_workspace_bytes(M, N));
       return AXN_EINVAL;
@@ -371,7 +390,7 @@ int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
   AXN_HIP_TRY(hipGetLastError());
   if (dbias != nullptr) {
     hipLaunchKernelGGL(dbias_reduce_kernel, dim3((unsigned)((N + 63) / 64)),
-                       dim3(256), 0, stream, partial, dbias, bands, N, beta);
+                       dim3(1024), 0, stream, partial, dbias, bands, N, beta);
     AXN_HIP_TRY(hipGetLastError());
   }
   return AXN_OK;

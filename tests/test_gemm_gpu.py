@@ -110,6 +110,39 @@ def test_forward_with_fp32_result_matches_oracle(M, N, K, epilogue, dtype):
         ops.gemm_fwd(X.cuda(), W.cuda(), out_f32=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("M,N", [(1, 8), (15, 520), (17, 512), (129, 1032), (257, 4104), (2900, 6144), (3001, 1024)])
+def test_dgelu_dbias_rows_dealt_to_bands(M, N, dtype):
+    """One chunk of 16 rows, a chunk begun, several turns; with the workspace that is asked for and with one
+    for a sum per 128 rows."""
+    from axonn_amd import _native as nv, ops
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    dY = torch.randn(M, N, generator=g, device="cuda").to(dtype)
+    Z = torch.randn(M, N, generator=g, device="cuda").to(dtype)
+    dz, db = ops.dgelu_dbias(dY, Z)
+    z = Z.double()
+    want = dY.double() * (torch.erfc(-z / 2 ** 0.5) / 2 + z * torch.exp(-z * z / 2) / (2 * torch.pi) ** 0.5)
+    # Phi to 1.5e-7, a few fp32 roundings, the stored type's
+    step = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[dtype]
+    assert bool(((dz.double() - want).abs() <= step * want.abs() + 2.0 ** -20 * dY.double().abs() + 2.0 ** -24).all())
+    bound = (M + 16) * 2.0 ** -24 * dz.double().abs().sum(0) + 1e-30   # M additions in fp32
+    if dtype == torch.float16:
+        # the stored product is rounded once, the summed one by way of fp32: where that falls on a tie (one in
+        # 2^13) they are a step apart; eight such elements in a column of 3001
+        bound += 8 * 2.0 ** -10 * dz.double().abs().amax(0)
+    assert bool(((db.double() - dz.double().sum(0)).abs() <= bound).all())
+    rows = (M + 127) // 128
+    ws = torch.full((rows * N,), float("nan"), device="cuda")
+    dz2, db2 = torch.empty_like(dz), torch.empty(N, device="cuda")
+    nv.call("axn_dgelu_dbias", nv.ptr(dY), nv.ptr(Z), nv.ptr(dz2), nv.dtype_code(dtype), nv.ptr(db2), M, N, N, 0,
+            nv.ptr(ws), rows * N * 4, nv.current_stream())
+    assert torch.equal(dz2, dz) and bool(((db2.double() - dz.double().sum(0)).abs() <= bound).all())
+    _, db3 = ops.dgelu_dbias(dz)   # the sums alone
+    assert bool(((db3.double() - dz.double().sum(0)).abs() <= bound).all())
+
+
+
 def test_dgelu_dbias_matches_oracle():
     from axonn_amd import ops
 

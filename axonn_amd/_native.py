@@ -87,6 +87,9 @@ SYMBOLS = {
     "axn_gemm_wgrad_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "axn_gemm_any_n": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _i64, _int,
                               _int, _int, _vp, _sz, _vp]),
+    "axn_gemm_bwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _int]),
+    "axn_gemm_bwd_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+                               _int, _int, _vp, _sz, _vp]),
     "axn_pad_rows16": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
     "axn_pad_rows16_to": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "axn_gemm_f32_workspace_bytes": (_sz, [_int, _i64, _i64, _i64]),

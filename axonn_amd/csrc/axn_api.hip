@@ -399,6 +399,39 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void*
               : launch_gemm_bf16(layout, g, epilogue, out_f32, (hipStream_t)stream);
 }
 
+size_t axn_gemm_bwd_workspace_bytes(int64_t M, int64_t N, int64_t K, int beta) {
+  if (M < 1 || N < 1 || K < 1 || M > 0x7fffffff || N > 0x7ffffff8 || K > 0x7fffffff || K % 8 != 0) return 0;
+  return (size_t)gemm_backward_parts(M, N, K, beta != 0) * (size_t)M * (size_t)K * sizeof(float);
+}
+
+int axn_gemm_bwd_ws(const void* dY, const void* W, const void* X, void* dX, void* dW, int dtype, int64_t M, int64_t N,
+                    int64_t K, int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t lddw, int beta,
+                    int dw_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  const char* name = "axn_gemm_bwd_ws";
+  REQUIRE(dtype == AXN_BF16 || dtype == AXN_F16, AXN_EINVAL, "%s: dtype must be bf16 or fp16", name);
+  const bool half = dtype == AXN_F16;
+  REQUIRE(N >= 1 && N <= 0x7ffffff8, AXN_EINVAL, "%s: N out of range (got %lld)", name, (long long)N);
+  const int64_t n8 = (N + 7) / 8 * 8;
+  int rc = check_gemm(name, dY, W, dX, M, n8, K, lddy, ldw, lddx, n8, K, K);
+  if (rc) return rc;
+  rc = check_gemm(name, dY, X, dW, M, n8, K, lddy, ldx, lddw, n8, K, K);
+  if (rc) return rc;
+  REQUIRE(beta == 0 || beta == 1, AXN_EINVAL, "%s: beta must be 0 or 1", name);
+  REQUIRE(dw_dtype == dtype || dw_dtype == AXN_F32, AXN_EINVAL, "%s: dW must be %s or fp32", name,
+          half ? "fp16" : "bf16");
+  const int parts = gemm_backward_parts(M, N, K, beta != 0);
+  REQUIRE(parts > 1 && workspace != nullptr && workspace_bytes >= (size_t)parts * (size_t)M * (size_t)K * sizeof(float),
+          AXN_EINVAL, "%s: workspace too small, or sizes that axn_gemm_bwd_workspace_bytes has none for", name);
+  REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+  REQUIRE(lddy < kEdgeMaxLd / 2 && ldw < kEdgeMaxLd / 2 && ldx < kEdgeMaxLd / 2, AXN_ESHAPE,
+          "%s: row strides below %lld elements expected", name, (long long)(kEdgeMaxLd / 2));
+  GemmArgs gd = {}, gw = {};
+  fill_gemm_args(gd, AXN_GEMM_DGRAD, dY, W, dX, M, N, K, lddy, ldw, lddx);
+  fill_gemm_args(gw, AXN_GEMM_WGRAD, dY, X, dW, M, N, K, lddy, ldx, lddw);
+  gw.beta = beta;
+  return launch_gemm_backward_parts(gd, gw, half, dw_dtype == AXN_F32, parts, (float*)workspace, (hipStream_t)stream);
+}
+
 static int pad_rows16(const char* name, const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst,
                       void* stream) {
   REQUIRE(src && dst, AXN_EINVAL, "%s: null pointer", name);

@@ -162,9 +162,14 @@ struct SplitPlan {
   int parts;
   EdgeTile tile;
 };
-SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc);
+SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, double* us = nullptr);
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, int epilogue, bool half, bool out_f32,
                        const SplitPlan& plan, float* ws, hipStream_t stream);
+// The parts of the input gradient's contraction if both gradients of a layer (dY[M][N], W[N][K], X[M][K]) are
+// estimated to be faster in one launch than in two, or 0; add: dW += ...; ws holds the parts, parts * M * K floats.
+int gemm_backward_parts(int64_t M, int64_t N, int64_t K, bool add);
+int launch_gemm_backward_parts(const GemmArgs& dgrad, const GemmArgs& wgrad, bool half, bool dw_f32, int parts,
+                               float* ws, hipStream_t stream);
 // Row strides from kEdgeMaxLd on, both operands addressed with 64 bits (gemm_far.hip).
 int launch_gemm_far(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32, bool half,
                     hipStream_t stream);

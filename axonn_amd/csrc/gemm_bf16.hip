@@ -601,6 +601,11 @@ int launch_gemm_f16(GemmLayout layout, const GemmArgs& g, int epilogue, bool out
   return launch_layout<true>(layout, g, epilogue, out_f32, stream);
 }
 
+namespace {
+constexpr double kPartsMicroseconds = 2.96;
+double part_microseconds(int64_t M, int64_t N) { return 2.02 * std::pow((double)M * (double)N * 1e-6, 0.763); }
+}  // namespace
+
 // Few output tiles leave most CUs without work: the contraction is cut into parts of at
 // least 512, on the tile and into the number of parts with the smallest estimated time, each part
 // a workgroup per tile.  On top of the launch (launch_microseconds) a split costs
@@ -611,7 +616,7 @@ int launch_gemm_f16(GemmLayout layout, const GemmArgs& g, int epilogue, bool out
 // ragged ones unsplit: 60 x 3520 x 6848 78 -> 20 us, 479 x 832 x 13824 146 -> 31 us, 1111 x 2752 x
 // 6336 70 -> 56 us.
 // It looks at sizes only, not at strides: a caller asks for the workspace by size.
-SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
+SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, double* us) {
   SplitPlan plan = {1, EDGE_128x128};
   if (layout == GEMM_NT && stream_ahead(M, N, Kc)) return plan;
   const bool whole = M % 128 == 0 && N % 128 == 0 && Kc % 64 == 0;
@@ -621,7 +626,7 @@ SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
   // contraction over a ragged shape is left alone
   if (tiles[EDGE_256x256] > 128 || Kc < (whole ? 1024 : 1536)) return plan;
   const double mb = ((double)M + (double)N) * (double)Kc * 2e-6;
-  const double part_cost = 2.02 * std::pow((double)M * (double)N * 1e-6, 0.763);
+  const double part_cost = part_microseconds(M, N);
   const long long stages = (Kc + 63) / 64;
   double best = 1e30;
   for (EdgeTile tile : {EDGE_128x128, EDGE_256x128, EDGE_256x256})
@@ -630,12 +635,13 @@ SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
     for (EdgeTile tile : {EDGE_128x128, EDGE_256x128, EDGE_256x256}) {
       if (tiles[tile] * parts > (tile == EDGE_128x128 ? 512 : 256)) continue;
       const double t = launch_microseconds(tile, tiles[tile] * parts, (double)((stages + parts - 1) / parts), mb) +
-                       2.96 + parts * part_cost;
+                       kPartsMicroseconds + parts * part_cost;
       if (t < best) {
         best = t;
         plan = {parts, tile};
       }
     }
+  if (us != nullptr) *us = best;
   return plan;
 }
 
@@ -681,6 +687,69 @@ int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool
                 : launch_reduce<false, true>(ws, out, epilogue, out_f32, stream);
   return half ? launch_reduce<true, false>(ws, out, epilogue, out_f32, stream)
               : launch_reduce<false, false>(ws, out, epilogue, out_f32, stream);
+}
+
+// ---- both gradients in one launch, the input gradient's contraction in parts -----------
+// An input gradient of few tiles and its weight gradient each end in a ramp and a last wave of their own; in one
+// launch the shorter tiles fill what the longer leave.  us, two launches and the sum / one and the sum: 1722 x 5888
+// x 1024 69 / 55, 1376 x 9088 x 2112 141 / 118, 599 x 32000 x 1088 143 / 118, 777 x 6144 x 4096 105 / 86.
+namespace {
+// Time until n1 tiles of s1 and then n2 of s2, each on the CU that is free first, are done.
+double filled(long long n1, double s1, long long n2, double s2) {
+  const long long rounds = n1 / 256, more = n1 % 256;   // `more` CUs have a tile of the first kind on top
+  const auto room = [&](double t) {
+    const double a = t - (double)(rounds + 1) * s1, b = t - (double)rounds * s1;
+    return (double)more * (a > 0 ? std::floor(a / s2) : 0) + (double)(256 - more) * (b > 0 ? std::floor(b / s2) : 0);
+  };
+  double lo = (double)(rounds + (more > 0 ? 1 : 0)) * s1, hi = lo + (double)(n2 / 256 + 1) * s2;
+  while (hi - lo > 0.25) {
+    const double mid = 0.5 * (lo + hi);
+    (room(mid) >= (double)n2 ? hi : lo) = mid;
+  }
+  return hi;
+}
+
+}  // namespace
+
+// The parts are the input gradient's own, so that its bits are the same either way.  The estimate: 2.2 us and 1.45
+// a stage of a time that lies between the work's average over the CUs and that of the fullest one (0.3 to 0.7), a
+// tile counting 3 stages more than it has, 6 where it reads dW to add to it, and the parts' cost; fitted to 65
+// problems of 64 to 3564 tokens with 2 to 16 parts each (7 % rms).  The two launches, whose estimate is 8 % low, and
+// 20 % beyond 100 us, where the power cap stretches it, have to be slower.  Of 110 other problems 25 take one launch,
+// 0.76 to 1.03 of the time of two, 0.89 on average; adding to dW 21, 0.72 to 0.99.  Up to 192 rows a weight gradient
+// is nearly all stores, and two launches are as fast (151 x 11392 x 4992: 75 us, 79 in one).
+int gemm_backward_parts(int64_t M, int64_t N, int64_t K, bool add) {
+  if (M <= 192) return 0;
+  double apart_d = 0, apart_w = 0;
+  const int parts = gemm_splits(GEMM_NN, M, K, N, &apart_d).parts;
+  const long long tw = ceil_div(N, 256) * ceil_div(K, 256);
+  if (parts <= 1 || tw > 65536 || gemm_splits(GEMM_TN, N, K, M).parts > 1) return 0;
+  edge_tile(N, K, M, {}, &apart_w);
+  if (add) apart_w += 0.5 * (double)N * (double)K * 2e-6 / 5.72;   // reading dW, half of it hidden
+  const long long td = ceil_div(M, 256) * ceil_div(K, 256) * parts;
+  const double d = (double)(ceil_div(ceil_div(N, 64), parts) + 3), w = (double)(ceil_div(M, 64) + (add ? 6 : 3));
+  const double fullest = d >= w ? filled(td, d, tw, w) : filled(tw, w, td, d);
+  const double average = ((double)td * d + (double)tw * w) / 256;
+  const double us = 2.2 + 1.45 * (0.7 * fullest + 0.3 * average) + kPartsMicroseconds + parts * part_microseconds(M, K);
+  const double apart = apart_d + apart_w;
+  return us < apart * (apart < 100 ? 1.08 : 1.2) ? parts : 0;
+}
+
+int launch_gemm_backward_parts(const GemmArgs& dgrad, const GemmArgs& wgrad, bool half, bool dw_f32, int parts,
+                               float* ws, hipStream_t stream) {
+  GemmArgs gd = dgrad, gw = wgrad;
+  const long long td = ceil_div(gd.M, 256) * ceil_div(gd.N, 256), tw = ceil_div(gw.M, 256) * ceil_div(gw.N, 256);
+  place_together(gd, gw, td * parts, tw, ceil_div(ceil_div(gd.Kc, 64), parts), ceil_div(gw.Kc, 64));
+  gd.C = ws;
+  gd.ldc = ceil_div(gd.N, 8) * 8;
+  gd.splits = parts;
+  const int rc = half ? launch_gemm_edge_backward_f16(gw, gd, dw_f32, stream)
+                      : launch_gemm_edge_backward_bf16(gw, gd, dw_f32, stream);
+  if (rc) return rc;
+  GemmArgs out = dgrad;
+  out.splits = parts;
+  return half ? launch_reduce<true, false>(ws, out, AXN_EPI_NONE, false, stream)
+              : launch_reduce<false, false>(ws, out, AXN_EPI_NONE, false, stream);
 }
 
 }  // namespace axn

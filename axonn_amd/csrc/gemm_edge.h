@@ -24,14 +24,15 @@ __global__ void __launch_bounds__(256) gemm_edge_kernel(const GemmArgs g) {
   solo_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, true, ODD>(g);
 }
 
-// Both gradients of a layer in one launch, as gemm_backward_kernel.
-template <bool HALF, bool DW_F32>
+// Both gradients of a layer in one launch, as gemm_backward_kernel.  PARTS: the input gradient's contraction is
+// in parts (fp32 partial products).
+template <bool HALF, bool DW_F32, bool PARTS>
 __global__ void __launch_bounds__(256) gemm_edge_backward_kernel(const GemmArgs gw, const GemmArgs gd) {
   const int b = (int)blockIdx.x;
   if (b >= gw.wg_first && b < gw.wg_first + gw.tiles_m * gw.tiles_n)
     solo_gemm<256, 256, false, false, AXN_EPI_NONE, DW_F32, HALF, true>(gw);
   else
-    solo_gemm<256, 256, true, false, AXN_EPI_NONE, false, HALF, true>(gd);
+    solo_gemm<256, 256, true, false, AXN_EPI_NONE, PARTS, HALF, true>(gd);
 }
 
 template <int BM, int BN, bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF, bool ODD = false>
@@ -132,20 +133,28 @@ int launch_edge_layout(GemmLayout layout, const GemmArgs& g, int epilogue, bool 
   return AXN_EINVAL;
 }
 
-template <bool HALF>
-int launch_edge_backward(const GemmArgs& gw, const GemmArgs& gd, bool dw_f32, hipStream_t stream) {
+template <bool HALF, bool DW_F32, bool PARTS>
+int launch_edge_backward_kind(const GemmArgs& gw, const GemmArgs& gd, hipStream_t stream) {
   constexpr size_t lds = 5 * 256 * 64 * 2;
-  void (*kern)(const GemmArgs, const GemmArgs) =
-      dw_f32 ? gemm_edge_backward_kernel<HALF, true> : gemm_edge_backward_kernel<HALF, false>;
+  void (*kern)(const GemmArgs, const GemmArgs) = gemm_edge_backward_kernel<HALF, DW_F32, PARTS>;
   {
-    static std::atomic<unsigned long long> lds_allowed[2];   // per output type of dW
-    const int rc = allow_lds((const void*)kern, lds, lds_allowed[dw_f32 ? 1 : 0]);
+    static std::atomic<unsigned long long> lds_allowed{0};   // per template instance
+    const int rc = allow_lds((const void*)kern, lds, lds_allowed);
     if (rc != AXN_OK) return rc;
   }
-  const unsigned nwg = (unsigned)(gw.tiles_m * gw.tiles_n + gd.tiles_m * gd.tiles_n);
+  const unsigned nwg = (unsigned)(gw.tiles_m * gw.tiles_n + gd.tiles_m * gd.tiles_n * (PARTS ? gd.splits : 1));
   hipLaunchKernelGGL(kern, dim3(nwg), dim3(256), lds, stream, gw, gd);
   AXN_HIP_TRY(hipGetLastError());
   return AXN_OK;
+}
+
+template <bool HALF>
+int launch_edge_backward(const GemmArgs& gw, const GemmArgs& gd, bool dw_f32, hipStream_t stream) {
+  if (gd.splits > 1)
+    return dw_f32 ? launch_edge_backward_kind<HALF, true, true>(gw, gd, stream)
+                  : launch_edge_backward_kind<HALF, false, true>(gw, gd, stream);
+  return dw_f32 ? launch_edge_backward_kind<HALF, true, false>(gw, gd, stream)
+                : launch_edge_backward_kind<HALF, false, false>(gw, gd, stream);
 }
 
 }  // namespace

@@ -121,6 +121,12 @@ def _workspace_bytes(op, M, N, K, f32=False):
     return (lib.axn_gemm_f32_workspace_bytes if f32 else lib.axn_gemm_workspace_bytes)(op, M, N, K)
 
 
+@functools.lru_cache(maxsize=4096)
+def _bwd_workspace_bytes(M, N, K, beta):
+    """Workspace with which both gradients are faster in one launch, the input gradient's contraction in parts."""
+    return nv.load().axn_gemm_bwd_workspace_bytes(M, N, K, beta)
+
+
 def _split_workspace(op, M, N, K, device, f32=False):
     """Workspace for a GEMM whose contraction the library would divide among workgroups
     (few output tiles), or (None, 0)."""
@@ -306,15 +312,48 @@ def gemm_wgrad(dy, x, out=None, accumulate=False, out_dtype=None):
     return out
 
 
+def _bwd_in_parts(dy, w, x, out, accumulate, out_dtype):
+    """gemm_bwd through axn_gemm_bwd_ws, or None for what that does not take."""
+    (M, N), K = dy.shape, w.shape[1]
+    if out is not None:
+        if out.numel() != N * K or not out.is_contiguous() or out.data_ptr() % 16:
+            return None
+        out_dtype = out.dtype
+    elif accumulate:
+        return None
+    out_dtype = out_dtype or dy.dtype
+    if out_dtype not in (dy.dtype, torch.float32):
+        return None
+    dy, lddy = _prep_bf16(_pad_rows(dy) if N % 8 else dy)
+    w, ldw = _prep_bf16(w)
+    x, ldx = _prep_bf16(x)
+    if max(lddy, ldw, ldx) >= _FAR_ROWS:
+        return None
+    dx = torch.empty((M, K), dtype=dy.dtype, device=dy.device)
+    if out is None:
+        out = torch.empty((N, K), dtype=out_dtype, device=dy.device)
+    beta = 1 if accumulate else 0
+    ws_bytes = _bwd_workspace_bytes(M, N, K, beta)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dy.device)
+    nv.call("axn_gemm_bwd_ws", nv.ptr(dy), nv.ptr(w), nv.ptr(x), nv.ptr(dx), nv.ptr(out), nv.dtype_code(dy.dtype),
+            M, N, K, lddy, ldw, ldx, K, K, beta, nv.dtype_code(out_dtype), nv.ptr(ws), ws_bytes, nv.current_stream())
+    return dx, out
+
+
 def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None):
     """(dX, dW) = (dY W, dY^T X) of one layer, dW optionally accumulated into `out`: the two
     products of AsyncLinear.backward (axonn/intra_layer/fully_connected.py:140, :147-151)
     through ONE entry point, which runs both in a single launch where their tile counts
     would each leave CUs idle in a launch of their own.  Results equal gemm_dgrad and
-    gemm_wgrad bit for bit; shapes the joint entry point does not take go through those."""
+    gemm_wgrad bit for bit; shapes the joint entry points do not take go through those."""
     _require_gpu(dy, w, x, out)
     M, N = dy.shape
     K = w.shape[1]
+    if (dy.dtype in _GEMM16 and dy.dtype == w.dtype == x.dtype and M > 0 and K % 8 == 0
+            and tuple(x.shape) == (M, K) and w.shape[0] == N and _bwd_workspace_bytes(M, N, K, 1 if accumulate else 0)):
+        both = _bwd_in_parts(dy, w, x, out, accumulate, out_dtype)
+        if both is not None:
+            return both
     plain16 = (dy.dtype in _GEMM16 and dy.dtype == w.dtype == x.dtype and M > 0
                and not _ragged16(dy.dtype, N, K)
                and _workspace_bytes(GEMM_DGRAD, M, N, K) == 0

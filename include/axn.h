@@ -196,6 +196,15 @@ AXN_API int axn_gemm_any_n(int op, const void* A, const void* B, const void* bia
                    void* Zsave, int dtype, int64_t M, int64_t N, int64_t K, int64_t lda,
                    int64_t ldb, int64_t ldc, int epilogue, int beta, int out_dtype,
                    void* workspace, size_t workspace_bytes, void* stream);
+/* Both gradients of a layer in one launch, as axn_gemm_bwd, the input gradient's contraction in parts that are added
+ * in a second one: for sizes whose input gradient alone has too few tiles.  The operands as axn_gemm_any_n's DGRAD and
+ * WGRAD (any N), row strides below 2^22 elements; results equal those calls' with their workspaces bit for bit.
+ * workspace: axn_gemm_bwd_workspace_bytes(M, N, K, beta) bytes, 16-byte aligned; where that is 0 the two products are
+ * faster by themselves, and this call refuses. */
+AXN_API size_t axn_gemm_bwd_workspace_bytes(int64_t M, int64_t N, int64_t K, int beta);
+AXN_API int axn_gemm_bwd_ws(const void* dY, const void* W, const void* X, void* dX, void* dW, int dtype, int64_t M,
+                    int64_t N, int64_t K, int64_t lddy, int64_t ldw, int64_t ldx, int64_t lddx, int64_t lddw,
+                    int beta, int dw_dtype, void* workspace, size_t workspace_bytes, void* stream);
 /* dst[M][n8] = src[M][N] of 16-bit elements (rows of ld elements, 2-byte aligned), n8 the next
  * multiple of 8, zeros behind column N; dst 16-byte aligned. */
 AXN_API int axn_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, void* stream);

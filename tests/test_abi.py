@@ -116,6 +116,18 @@ def test_gemm_argument_errors():
     assert fb(A, A, None, A, A, nv.BF16, 8, 8, 8, 8, 8, 8, 8, 8, 0, nv.BF16, None) == nv.AXN_EINVAL
     assert fb(A, A, A, A, A, nv.BF16, 8, 12, 8, 16, 8, 8, 8, 8, 0, nv.BF16, None) == nv.AXN_ESHAPE
     assert "axn_gemm_bwd" in _err()
+    # the same with the input gradient in parts: only sizes that have a workspace, with that workspace
+    need = lib.axn_gemm_bwd_workspace_bytes(777, 6144, 4096, 0)
+    assert need > 0 and need % (777 * 4096 * 4) == 0
+    assert lib.axn_gemm_bwd_workspace_bytes(777, 6144, 4092, 0) == lib.axn_gemm_bwd_workspace_bytes(0, 8, 8, 1) == 0
+    fp = lib.axn_gemm_bwd_ws
+    sizes = (777, 6144, 4096, 6144, 4096, 4096, 4096, 4096)
+    assert fp(A, A, A, A, A, nv.BF16, *sizes, 0, nv.BF16, A, need - 1, None) == nv.AXN_EINVAL
+    assert fp(A, A, A, A, A, nv.BF16, *sizes, 0, nv.BF16, None, need, None) == nv.AXN_EINVAL
+    assert fp(A, A, A, A, A, nv.BF16, 8, 8, 8, 8, 8, 8, 8, 8, 0, nv.BF16, A, need, None) == nv.AXN_EINVAL
+    assert fp(A, A, A, A, A, nv.F32, *sizes, 0, nv.F32, A, need, None) == nv.AXN_EINVAL
+    assert fp(A, A, A, A, A, nv.BF16, 777, 6144, 4096, 1 << 22, 4096, 4096, 4096, 4096, 0, nv.BF16, A, need,
+              None) == nv.AXN_ESHAPE
     # fp32 result: the promotion of an fp32 bias, so only with a bias epilogue
     fo = lib.axn_gemm_fwd_f32out
     assert fo(A, A, A, A, None, nv.BF16, 8, 8, 8, 8, 8, 8, nv.EPI_NONE, None) == nv.AXN_EINVAL

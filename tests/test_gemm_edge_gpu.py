@@ -307,3 +307,42 @@ def test_outputs_of_whole_small_tiles_only(rows, cols, kc, dtype):
     assert bool(((z.double() - pre).abs() <= ulp * pre.abs() + 1e-5 * pre.abs().max()).all())
     gelu = torch.nn.functional.gelu(pre)
     assert bool(((y.double() - gelu).abs() <= ulp * gelu.abs() + 1e-5 * gelu.abs().max()).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,beta,dw_f32", [
+    (649, 4032, 2176, 1, False), (2466, 4800, 1216, 0, False),      # longer tiles of dX, of dW first
+    (2400, 4803, 1216, 1, True), (777, 6144, 4096, 0, True),        # any N; an fp32 dW
+    (193, 9920, 5120, 0, False), (974, 50257, 768, 1, False),       # the fewest rows; ten parts
+])
+def test_both_gradients_in_one_launch_with_the_contraction_in_parts(M, N, K, beta, dw_f32, dtype):
+    """Against the two calls, bit for bit, the operands in buffers of NaN, the outputs in canvases, the workspace
+    exactly as large as it has to be."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(N)
+    need = nv.load().axn_gemm_bwd_workspace_bytes(M, N, K, beta)
+    assert need > 0
+    dY = torch.full((M + 3, N + (-N) % 8 + 8), float("nan"), dtype=dtype, device="cuda")[:M]
+    dY[:, N:N + (-N) % 8] = 0
+    dY = dY[:, :N]
+    dY.copy_(torch.randn(M, N, generator=g, device="cuda"))
+    W, X = numbers(N, K, dtype, g, 8), numbers(M, K, dtype, g, 16)
+    W.copy_(torch.randn(N, K, generator=g, device="cuda") * 0.1)
+    dw_dtype = torch.float32 if dw_f32 else dtype
+    fx, dx = canvas(M, K, dtype)
+    fw, dw = canvas(N, K, dw_dtype)
+    start = torch.ones(N, K, dtype=dw_dtype, device="cuda")
+    if beta:
+        dw.copy_(start)
+    ws = torch.full((need // 4 + 64,), float("nan"), device="cuda")
+    nv.call("axn_gemm_bwd_ws", nv.ptr(dY), nv.ptr(W), nv.ptr(X), nv.ptr(dx), nv.ptr(dw), nv.dtype_code(dtype), M, N, K,
+            dY.stride(0), W.stride(0), X.stride(0), dx.stride(0), dw.stride(0), beta, nv.dtype_code(dw_dtype),
+            nv.ptr(ws), need, nv.current_stream())
+    assert bool(torch.isnan(ws[need // 4:]).all()), "written behind the workspace"
+    want_dx = ops.gemm_dgrad(dY, W)
+    want_dw = ops.gemm_wgrad(dY, X, out=start if beta else None, accumulate=bool(beta), out_dtype=dw_dtype)
+    both = ops.gemm_bwd(dY, W, X, out_dtype=dw_dtype)
+    assert torch.equal(both[0], want_dx)
+    check(fx, dx, want_dx)
+    check(fw, dw, want_dw)

@@ -126,12 +126,12 @@ __device__ __forceinline__ void widen8(const Raw8<float>::type& v, float (&x)[8]
 // a wave waits for one store round trip per group and not per row (3 % at 8192 x 5120 bf16).
 // Band b is the chunks b, b + bands, b + 2 bands, ...: all workgroups together walk down one compact
 // window of the operands, where consecutive rows a band had each its own (us, from HBM, bf16: 8192 x 5120
-// 56.5 -> 51.3, 8192 x 14336 153 -> 136, 5000 x 8192 69 -> 50, sums alone 24.6 -> 17.0).  What bounds it is the
-// memory system, at 4.9 to 5.2 TB/s, beside about 24 operations an element.  Rows of different
+// 56.5 -> 48.5, 8192 x 14336 153 -> 136, 5000 x 8192 69 -> 45, sums alone 24.6 -> 17.0).  What bounds it is the
+// memory system, at 4.9 to 5.4 TB/s, beside about 24 operations an element.  Rows of different
 // groups never overlap, so dZ may still alias dY.
 constexpr int EW_GROUP = 4;
 constexpr int EW_CHUNK = EW_TY * EW_GROUP;   // rows a workgroup has in flight
-constexpr int EW_TURNS = 8;                  // most chunks a workgroup walks where that fills the chip
+constexpr int EW_TURNS = 16;                 // most chunks a workgroup walks where that fills the chip
 
 template <typename T, bool HAS_Z>
 __global__ void __launch_bounds__(EW_TX* EW_TY)
@@ -319,34 +319,38 @@ int launch_swiglu_bwd(const void* dout, const void* gate, const void* up, void* 
 }
 
 namespace {
-// Bands of the dGELU + dbias pass: as many as leave a workgroup one to eight chunks of rows, at most 640 workgroups
-// where there is a choice (the sums' traffic grows with them), and of those the number whose fullest CU has the
-// fewest chunks to walk.  Bands of 128 consecutive rows left 64 to 500 rows to 8 to 32 CUs (us, before -> now):
-// fp32 2048 x 4096 25.2 -> 20.2, 2900 x 6144 59.3 -> 47.1; bf16 256 x 4096 without sums 16 -> 9.
+// Bands of the dGELU + dbias pass: as many as leave a workgroup one to sixteen chunks of rows, at most 640
+// workgroups where there is a choice (the sums' traffic grows with them; from eight chunks on there is none), and of
+// those the number whose fullest CU has the fewest chunks to walk.  Bands of 128 consecutive rows left 64 to 500 rows
+// to 8 to 32 CUs (us, before -> now): fp32 2048 x 4096 25.2 -> 20.2, 2900 x 6144 59.3 -> 40.0; bf16 256 x 4096 without
+// sums 16 -> 9.  With no more than eight chunks 8192 x 5120 takes 640 workgroups, which are 3 for half of the CUs and 2
+// for the others (bf16 51.7 us, with 470 48.5), 5000 x 8192 49.4 and 45.2.
 int64_t dgelu_bands(int64_t M, int64_t N) {
   const int64_t cols = (N + EW_COLS - 1) / EW_COLS, chunks = (M + EW_CHUNK - 1) / EW_CHUNK;
   int64_t best = 0, least = 0;
   for (int64_t turns = 1; turns <= EW_TURNS; ++turns) {
     const int64_t bands = (chunks + turns - 1) / turns;
-    if (bands * cols > 640 && turns < EW_TURNS) continue;
+    if (bands * cols > 640 && turns < 8) continue;
     const int64_t walk = (bands * cols + 255) / 256 * turns;
     if (best == 0 || walk < least) best = bands, least = walk;
   }
   return best;
 }
+constexpr int EW_SUM_ROWS = 128;   // a workspace for a sum per so many rows is always enough
 size_t band_sums_bytes(int64_t bands, int64_t N) { return (size_t)bands * (size_t)N * sizeof(float); }
 }  // namespace
 
 size_t dgelu_dbias_workspace_bytes(int64_t M, int64_t N) {
-  return M <= 0 || N <= 0 ? 0 : band_sums_bytes(dgelu_bands(M, N), N);
+  if (M <= 0 || N <= 0) return 0;
+  const int64_t bands = dgelu_bands(M, N), enough = (M + EW_SUM_ROWS - 1) / EW_SUM_ROWS;
+  return band_sums_bytes(bands > enough ? bands : enough, N);
 }
 
 int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
                        float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
                        void* ws, size_t ws_bytes, hipStream_t stream) {
   int64_t bands = dgelu_bands(M, N);
-  // (a workspace for a sum per 128 rows is enough)
-  if (dbias != nullptr && ws_bytes < band_sums_bytes(bands, N)) bands = (M + EW_TURNS * EW_CHUNK - 1) / (EW_TURNS * EW_CHUNK);
+  if (dbias != nullptr && ws_bytes < band_sums_bytes(bands, N)) bands = (M + EW_SUM_ROWS - 1) / EW_SUM_ROWS;
   float* partial = nullptr;
   if (dbias != nullptr) {
     if (ws == nullptr || ws_bytes < band_sums_bytes(bands, N)) {
@@ -357,7 +361,7 @@ int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
     partial = (float*)ws;
   }
   const dim3 grid((unsigned)((N + EW_COLS - 1) / EW_COLS), (unsigned)bands);
-  if (bands > 65535) {
+  if ((M + EW_SUM_ROWS - 1) / EW_SUM_ROWS > 65535) {   // (never fewer than bands where there are many)
     set_error("dgelu_dbias: too many rows (%lld)", (long long)M);
     return AXN_ELIMIT;
   }

@@ -317,10 +317,11 @@ __global__ void __launch_bounds__(64 * WAVES)
 // 16-byte pieces are permuted by part_of(rho) so that any 16 lanes of a fragment read hit 16 different
 // 16-byte bank groups.
 // LDS is single-buffered (48 KB for 128 x 128) so that two workgroups share a CU and fill each other's
-// barriers.  2048 x 4096, contraction 1024: 86 us, 200 TFLOP/s of fp32 products (native 201 us); what
-// bounds it is the chain of stores, barrier, fragment reads and matrix instructions of a stage, not one
-// unit: two LDS buffers with one barrier (one workgroup a CU) 122 us, splitting by truncation without the
-// conversions 97, against 98 in the same run.
+// barriers.  2048 x 4096, contraction 1024: 86 us, 200 TFLOP/s of fp32 products (native 201 us), in a row of launches
+// 110.  What bounds it is the work of a stage together, six products and both operands' splitting in every workgroup
+// (matrix cores busy 47 % of the time, vector instructions 30 %, at 2.17 GHz): two LDS buffers with one barrier (one
+// workgroup a CU) 122 us, splitting by truncation without the conversions 97, against 98 in the same run; the next
+// stage's splitting between the matrix instructions 110 to 117 us against 107 to 112.
 template <int F>
 struct Planes {
   uint16_t at[3][32 * F][32];

@@ -2,10 +2,10 @@
 //   dZ = dY * gelu'(Z)   and   dbias[n] = sum_m dZ[m, n]
 // which is what autograd derives from the reference's `x + bias`
 // (axonn/intra_layer/fully_connected.py:348) followed by the caller's exact-erf
-// nn.GELU.  Lanes move 16 bytes (8 bf16 columns); column sums are kept in
-// registers over a band's rows, combined through LDS, written as one fp32
-// partial row per band and reduced over bands in a fixed order by a second
-// kernel, so the result does not depend on scheduling.
+// nn.GELU.  Lanes move 16 bytes (8 bf16 columns); column sums are formed over
+// bands of 128 rows, written as one fp32 partial row per band and reduced over
+// bands in a fixed order by a second kernel, so the result does not depend on
+// scheduling.
 //
 // Also here: the SwiGLU activation of the Llama MLP, h = silu(gate) * up, and its
 // backward, each one HBM pass.  The reference's Llama patch
@@ -25,10 +25,6 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int EW_TX = 64;          // lanes along columns (8 columns each)
 constexpr int EW_TY = 4;           // row phases per workgroup
 constexpr int EW_COLS = EW_TX * 8; // 512 columns per workgroup
-// Non-temporal loads of dY and Z: 12 % faster when the operands come from HBM (62 -> 55 us),
-// 12 % slower when the memory-side cache holds them, which is the case in a training step
-// (dY was written by the layer behind a moment ago): off.
-constexpr bool DGELU_NT = false;
 // SwiGLU has no sums to carry down the rows: one row piece per wave, the workgroups handed
 // out in row-major order, so that the chip reads and writes one compact window of every
 // operand (4096 x 14336 bf16 from HBM: forward 76 -> 59 us, backward 131 -> 98 us against
@@ -90,130 +86,136 @@ __device__ __forceinline__ void store8(float* p, float (&x)[8]) {
   *(f32x4*)(p + 4) = f32x4{x[4], x[5], x[6], x[7]};
 }
 
-// Raw 8-column pieces of a row, so that a group of rows can be in flight as loads before
-// any of it is converted.
+// Raw 8-column pieces of a row (16-byte aligned), as they lie in memory.
+typedef float f32x8 __attribute__((ext_vector_type(8), aligned(16)));
 template <typename T> struct Raw8;
-template <> struct Raw8<uint16_t> { typedef bf16x8 type; };
-template <> struct Raw8<_Float16> { typedef f16x8 type; };
-template <> struct Raw8<float> { struct type { f32x4 lo, hi; }; };
-template <typename T>
-__device__ __forceinline__ typename Raw8<T>::type load_raw8(const T* p) {
-  if constexpr (DGELU_NT && sizeof(T) == 2) {
-    return __builtin_nontemporal_load((const typename Raw8<T>::type*)p);
-  } else {
-    return *(const typename Raw8<T>::type*)p;
-  }
-}
-__device__ __forceinline__ void widen8(const bf16x8& v, float (&x)[8]) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = (float)v[e];
-}
-__device__ __forceinline__ void widen8(const f16x8& v, float (&x)[8]) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = (float)v[e];
-}
-__device__ __forceinline__ void widen8(const Raw8<float>::type& v, float (&x)[8]) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    x[e] = v.lo[e];
-    x[4 + e] = v.hi[e];
-  }
+template <> struct Raw8<uint16_t> { typedef bf16x8 type; typedef __bf16 element; };
+template <> struct Raw8<_Float16> { typedef f16x8 type; typedef _Float16 element; };
+template <> struct Raw8<float> { typedef f32x8 type; typedef float element; };
+
+// fp16(g * d) rounded once.
+__device__ __forceinline__ _Float16 product_f16(float d, _Float16 g) {
+  _Float16 r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(r) : "v"(d), "v"(g));
+  return r;
 }
 
-// A thread walks its rows in groups of EW_GROUP: the loads of the next group are issued
-// before the stores of this one.  The memory counter of a wave is in order, so a load
-// behind a store returns only after the store is acknowledged; with the loads in front,
-// a wave waits for one store round trip per group and not per row (3 % at 8192 x 5120 bf16).
-// Band b is the chunks b, b + bands, b + 2 bands, ...: all workgroups together walk down one compact
-// window of the operands, where consecutive rows a band had each its own (us, from HBM, bf16: 8192 x 5120
-// 56.5 -> 48.5, 8192 x 14336 153 -> 136, 5000 x 8192 69 -> 45, sums alone 24.6 -> 17.0).  What bounds it is the
-// memory system, at 4.9 to 5.4 TB/s, beside about 24 operations an element.  Rows of different
-// groups never overlap, so dZ may still alias dY.
-constexpr int EW_GROUP = 4;
-constexpr int EW_CHUNK = EW_TY * EW_GROUP;   // rows a workgroup has in flight
-constexpr int EW_TURNS = 16;                 // most chunks a workgroup walks where that fills the chip
+// A workgroup takes 128 columns of a band of 128 rows, 64 or 32 rows at a time: every thread one piece of 8 columns,
+// which it stores and leaves in LDS, and then (512 threads) one column and phase whose sum it carries down the band:
+// phase p adds rows p, p + 4, p + 8, ... one after the other, the four phases are added in pairs.  Two LDS buffers: the
+// barrier behind the next rows is the one that frees these.
+//
+// Bound by memory: 252 MB of bf16 8192 x 5120 and their sums in 52 us from HBM (4.9 TB/s), 42 where the memory-side
+// cache holds the operands.  The order of the sums is that of one workgroup of 256 threads walking 512 columns of a
+// band row by row, which had 64 to 500 rows on 8 to 32 CUs; bands dealt out in chunks of 16 rows balance too,
+// but add in another order, up to 1.6 times as far from 64 bits.  us with the sums, (HBM | cache), walk row by row,
+// chunks, so:
+//   bf16 8192 x 5120 62 | 51, 52 | 45, 52 | 42    2048 x 4096 22 | 21, 17 | 15, 16 | 13    256 x 4096 18, 8, 8
+//   bf16 8192 x 14336 154, 137, 138               2900 x 6144 36 | 33, 26 | 23, 28 | 23    3001 x 10240 43 | 37, 41 | 34, 41 | 34
+//   fp32 8192 x 5120 110, 101, 101                2900 x 6144 64 | 46, 44 | 36, 48 | 38    5000 x 8192 112, 96, 88
+//   sums alone, bf16 8192 x 5120 22, 18, 19       2900 x 6144 12.5, 11.8, 12.7             fp32 2900 x 6144 19.7, 15.9, 19.0
+// 1024 threads are ahead of 512 by 2 % on 16-bit dGELU and behind by 3 to 8 % on fp32 and on sums alone (bf16 8192 x
+// 5120 18.7 us, with 1024 19.6); 64 columns or 256, and the loads of the next rows ahead of the stores were no faster.
+// Non-temporal loads of dY and Z (bf16 8192 x 5120) are 10 % faster from HBM (47 us) and 12 % slower from the
+// cache (47), which holds dY in a training step (the layer behind wrote it a moment ago): plain ones.
+// Every thread has read its piece before it stores it, so dZ may alias dY.
+constexpr int DG_BAND = 128, DG_COLS = 128, DG_PIECES = DG_COLS / 8;
+template <typename T, bool HAS_Z>
+constexpr int DG_THREADS = HAS_Z && sizeof(T) == 2 ? 1024 : 512;
 
 template <typename T, bool HAS_Z>
-__global__ void __launch_bounds__(EW_TX* EW_TY)
-    dgelu_dbias_kernel(const T* dY, const T* Z, T* dZ, float* partial, int64_t M,
-                       int64_t N, int64_t ld) {
+__global__ void __launch_bounds__((DG_THREADS<T, HAS_Z>))
+    dgelu_dbias_kernel(const T* dY, const T* Z, T* dZ, float* partial, int64_t M, int64_t N, int64_t ld) {
   typedef typename Raw8<T>::type raw;
-  const int tx = threadIdx.x % EW_TX, ty = threadIdx.x / EW_TX;
-  const int64_t col = (int64_t)blockIdx.x * EW_COLS + tx * 8;
-  const int64_t step = (int64_t)gridDim.y * EW_CHUNK;
-  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (col < N) {
-    raw gy[EW_GROUP], gz[EW_GROUP];
-    auto fetch = [&](int64_t first) {
+  typedef typename Raw8<T>::element element;
+  constexpr int ROWS = DG_THREADS<T, HAS_Z> / DG_PIECES;   // at a time
+  static_assert(ROWS % 4 == 0 && DG_BAND % ROWS == 0 && DG_THREADS<T, HAS_Z> >= 4 * DG_COLS, "a thread for each phase and column");
+  // fp32: the sums take in the product unrounded, from its factors
+  constexpr bool FACTORS = HAS_Z && std::is_same_v<T, float>;
+  __shared__ __attribute__((aligned(16))) element rows[2][FACTORS ? 2 : 1][ROWS][DG_COLS];
+  __shared__ float phases[4][DG_COLS];
+  const int piece = threadIdx.x % DG_PIECES, row0 = threadIdx.x / DG_PIECES;
+  const int c = threadIdx.x % DG_COLS, phase = threadIdx.x / DG_COLS;
+  const int64_t col0 = (int64_t)blockIdx.x * DG_COLS, band0 = (int64_t)blockIdx.y * DG_BAND;
+  const int64_t col = col0 + piece * 8;
+  float sum = 0.f;
 #pragma unroll
-      for (int u = 0; u < EW_GROUP; ++u) {
-        const int64_t r = first + u * EW_TY;
-        if (r < M) {
-          gy[u] = load_raw8(dY + r * ld + col);
-          if (HAS_Z) gz[u] = load_raw8(Z + r * ld + col);
+  for (int step = 0; step < DG_BAND / ROWS; ++step) {
+    const int64_t row = band0 + step * ROWS + row0;
+    raw add = raw{}, factor = raw{};   // zeros outside
+    if (row < M && col < N) {
+      add = *(const raw*)(dY + row * ld + col);
+      if constexpr (HAS_Z) {
+        const raw z = *(const raw*)(Z + row * ld + col);
+        raw out;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float d = dgelu_exact((float)z[e]);
+          float g = (float)add[e] * d;
+          if constexpr (FACTORS) {
+            factor[e] = d;
+            out[e] = g;
+          } else if constexpr (std::is_same_v<T, _Float16>) {
+            // stored: rounded to fp32 and then to fp16; added: the same, but in the first two columns of a piece
+            // the product rounded once (what the sums of fp16 layers have been; one step apart on ties)
+            asm("" : "+v"(g));
+            out[e] = (_Float16)g;
+            add[e] = e < 2 ? product_f16(d, add[e]) : out[e];
+          } else {
+            add[e] = out[e] = (__bf16)g;   // the sum of what wgrad reads
+          }
         }
+        *(raw*)(dZ + row * ld + col) = out;
       }
-    };
-    int64_t first = (int64_t)blockIdx.y * EW_CHUNK + ty;
-    fetch(first);
-    while (first < M) {
-      float g[EW_GROUP][8];
+    }
+    if (partial == nullptr) continue;
+    *(raw*)&rows[step & 1][0][row0][piece * 8] = add;
+    if constexpr (FACTORS) *(raw*)&rows[step & 1][1][row0][piece * 8] = factor;
+    __syncthreads();
+    if (phase >= 4) continue;
 #pragma unroll
-      for (int u = 0; u < EW_GROUP; ++u) {
-        widen8(gy[u], g[u]);
-        if (HAS_Z) {
-          float z[8];
-          widen8(gz[u], z);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) g[u][e] *= dgelu_exact(z[e]);
-        }
-      }
-      const int64_t next = first + step;
-      if (next < M) fetch(next);
-#pragma unroll
-      for (int u = 0; u < EW_GROUP; ++u) {
-        const int64_t r = first + u * EW_TY;
-        if (r < M) {
-          // g becomes what was stored: the sum of what wgrad reads
-          if (HAS_Z) store8(dZ + r * ld + col, g[u]);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) s[e] += g[u][e];
-        }
-      }
-      first = next;
+    for (int r = 0; r < ROWS; r += 4) {
+      const float x = (float)rows[step & 1][0][phase + r][c];
+      if constexpr (FACTORS)
+        sum = __builtin_fmaf(x, rows[step & 1][1][phase + r][c], sum);
+      else
+        sum += x;
     }
   }
   if (partial == nullptr) return;
-  __shared__ float red[EW_TY][EW_COLS];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) red[ty][tx * 8 + e] = s[e];
+  if (phase < 4) phases[phase][c] = sum;
   __syncthreads();
-  for (int c = threadIdx.x; c < EW_COLS; c += EW_TX * EW_TY) {
-    const int64_t gc = (int64_t)blockIdx.x * EW_COLS + c;
-    if (gc < N)
-      partial[(int64_t)blockIdx.y * N + gc] =
-          (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
-  }
+  if (phase == 0 && col0 + c < N)
+    partial[(int64_t)blockIdx.y * N + col0 + c] = (phases[0][c] + phases[1][c]) + (phases[2][c] + phases[3][c]);
 }
 
-// Column sums over the band partials in a fixed order: 64 columns per workgroup, thread q of a
-// column's 16 adds bands q, q + 16, ..., the 16 sums are then added in order.
-__global__ void __launch_bounds__(1024)
+// Column sums over the band partials in a fixed order: 64 columns per workgroup, the bands split in 4
+// consecutive quarters summed by 4 threads each in band order (8 loads on their way), the quarters then
+// combined as (q0 + q1) + (q2 + q3).
+__global__ void __launch_bounds__(256)
     dbias_reduce_kernel(const float* partial, float* dbias, int64_t bands,
                         int64_t N, int beta) {
-  __shared__ float red[16][64];
+  __shared__ float red[4][64];
   const int tx = threadIdx.x & 63, q = threadIdx.x >> 6;
   const int64_t c = (int64_t)blockIdx.x * 64 + tx;
+  const int64_t per = (bands + 3) / 4;
+  const int64_t b1 = (q + 1) * per < bands ? (q + 1) * per : bands;
   float s = 0.f;
-  if (c < N)
-#pragma unroll 4
-    for (int64_t b = q; b < bands; b += 16) s += partial[b * N + c];
+  if (c < N) {
+    int64_t b = q * per;
+    for (; b + 8 <= b1; b += 8) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = partial[(b + i) * N + c];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s += v[i];
+    }
+    for (; b < b1; ++b) s += partial[b * N + c];
+  }
   red[q][tx] = s;
   __syncthreads();
   if (q == 0 && c < N) {
-    float t = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) t += red[i][tx];
+    const float t = (red[0][tx] + red[1][tx]) + (red[2][tx] + red[3][tx]);
     dbias[c] = beta ? dbias[c] + t : t;
   }
 }
@@ -318,83 +320,51 @@ int launch_swiglu_bwd(const void* dout, const void* gate, const void* up, void* 
   return AXN_OK;
 }
 
-namespace {
-// Bands of the dGELU + dbias pass: as many as leave a workgroup one to sixteen chunks of rows, at most 640
-// workgroups where there is a choice (the sums' traffic grows with them; from eight chunks on there is none), and of
-// those the number whose fullest CU has the fewest chunks to walk.  Bands of 128 consecutive rows left 64 to 500 rows
-// to 8 to 32 CUs (us, before -> now): fp32 2048 x 4096 25.2 -> 20.2, 2900 x 6144 59.3 -> 40.0; bf16 256 x 4096 without
-// sums 16 -> 9.  With no more than eight chunks 8192 x 5120 takes 640 workgroups, which are 3 for half of the CUs and 2
-// for the others (bf16 51.7 us, with 470 48.5), 5000 x 8192 49.4 and 45.2.
-int64_t dgelu_bands(int64_t M, int64_t N) {
-  const int64_t cols = (N + EW_COLS - 1) / EW_COLS, chunks = (M + EW_CHUNK - 1) / EW_CHUNK;
-  int64_t best = 0, least = 0;
-  for (int64_t turns = 1; turns <= EW_TURNS; ++turns) {
-    const int64_t bands = (chunks + turns - 1) / turns;
-    if (bands * cols > 640 && turns < 8) continue;
-    const int64_t walk = (bands * cols + 255) / 256 * turns;
-    if (best == 0 || walk < least) best = bands, least = walk;
-  }
-  return best;
-}
-constexpr int EW_SUM_ROWS = 128;   // a workspace for a sum per so many rows is always enough
-size_t band_sums_bytes(int64_t bands, int64_t N) { return (size_t)bands * (size_t)N * sizeof(float); }
-}  // namespace
-
 size_t dgelu_dbias_workspace_bytes(int64_t M, int64_t N) {
   if (M <= 0 || N <= 0) return 0;
-  const int64_t bands = dgelu_bands(M, N), enough = (M + EW_SUM_ROWS - 1) / EW_SUM_ROWS;
-  return band_sums_bytes(bands > enough ? bands : enough, N);
+  return (size_t)((M + DG_BAND - 1) / DG_BAND) * (size_t)N * sizeof(float);
 }
 
 int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
                        float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
                        void* ws, size_t ws_bytes, hipStream_t stream) {
-  int64_t bands = dgelu_bands(M, N);
-  if (dbias != nullptr && ws_bytes < band_sums_bytes(bands, N)) bands = (M + EW_SUM_ROWS - 1) / EW_SUM_ROWS;
+  const int64_t bands = (M + DG_BAND - 1) / DG_BAND;
   float* partial = nullptr;
   if (dbias != nullptr) {
-    if (ws == nullptr || ws_bytes < band_sums_bytes(bands, N)) {
+    if (ws == nullptr || ws_bytes < dgelu_dbias_workspace_bytes(M, N)) {
       set_error("dgelu_dbias: workspace too small (%zu bytes given, %zu needed)",
                 ws_bytes, dgelu_dbias_workspace_bytes(M, N));
       return AXN_EINVAL;
     }
     partial = (float*)ws;
   }
-  const dim3 grid((unsigned)((N + EW_COLS - 1) / EW_COLS), (unsigned)bands);
-  if ((M + EW_SUM_ROWS - 1) / EW_SUM_ROWS > 65535) {   // (never fewer than bands where there are many)
+  const dim3 grid((unsigned)((N + DG_COLS - 1) / DG_COLS), (unsigned)bands);
+  if (bands > 65535) {
     set_error("dgelu_dbias: too many rows (%lld)", (long long)M);
     return AXN_ELIMIT;
   }
-  const dim3 block(EW_TX * EW_TY);
-  if (dtype == AXN_F32) {
-    const float *y = (const float*)dY, *z = (const float*)Z;
-    if (Z != nullptr)
-      hipLaunchKernelGGL((dgelu_dbias_kernel<float, true>), grid, block, 0, stream,
-                         y, z, (float*)dZ, partial, M, N, ld);
-    else
-      hipLaunchKernelGGL((dgelu_dbias_kernel<float, false>), grid, block, 0, stream,
-                         y, z, (float*)dZ, partial, M, N, ld);
-  } else if (dtype == AXN_F16) {
-    const _Float16 *y = (const _Float16*)dY, *z = (const _Float16*)Z;
-    if (Z != nullptr)
-      hipLaunchKernelGGL((dgelu_dbias_kernel<_Float16, true>), grid, block, 0, stream, y, z,
-                         (_Float16*)dZ, partial, M, N, ld);
-    else
-      hipLaunchKernelGGL((dgelu_dbias_kernel<_Float16, false>), grid, block, 0, stream, y, z,
-                         (_Float16*)dZ, partial, M, N, ld);
-  } else {
-    const uint16_t *y = (const uint16_t*)dY, *z = (const uint16_t*)Z;
-    if (Z != nullptr)
-      hipLaunchKernelGGL((dgelu_dbias_kernel<uint16_t, true>), grid, block, 0,
-                         stream, y, z, (uint16_t*)dZ, partial, M, N, ld);
-    else
-      hipLaunchKernelGGL((dgelu_dbias_kernel<uint16_t, false>), grid, block, 0,
-                         stream, y, z, (uint16_t*)dZ, partial, M, N, ld);
-  }
+#define AXN_DGELU(T, HAS_Z)                                                                                  \
+  hipLaunchKernelGGL((dgelu_dbias_kernel<T, HAS_Z>), grid, dim3(DG_THREADS<T, HAS_Z>), 0, stream, (const T*)dY, \
+                     (const T*)Z, (T*)dZ, partial, M, N, ld)
+#define AXN_DGELU_TYPE(T)    \
+  do {                       \
+    if (Z != nullptr)        \
+      AXN_DGELU(T, true);    \
+    else                     \
+      AXN_DGELU(T, false);   \
+  } while (0)
+  if (dtype == AXN_F32)
+    AXN_DGELU_TYPE(float);
+  else if (dtype == AXN_F16)
+    AXN_DGELU_TYPE(_Float16);
+  else
+    AXN_DGELU_TYPE(uint16_t);
+#undef AXN_DGELU_TYPE
+#undef AXN_DGELU
   AXN_HIP_TRY(hipGetLastError());
   if (dbias != nullptr) {
     hipLaunchKernelGGL(dbias_reduce_kernel, dim3((unsigned)((N + 63) / 64)),
-                       dim3(1024), 0, stream, partial, dbias, bands, N, beta);
+                       dim3(256), 0, stream, partial, dbias, bands, N, beta);
     AXN_HIP_TRY(hipGetLastError());
   }
   return AXN_OK;

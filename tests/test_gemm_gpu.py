@@ -141,6 +141,53 @@ def test_dgelu_dbias_rows_dealt_to_bands(M, N, dtype):
     _, db3 = ops.dgelu_dbias(dz)   # the sums alone
     assert bool(((db3.double() - dz.double().sum(0)).abs() <= bound).all())
 
+def sums_by_bands(x):
+    """Column sums of fp32 `x` in the order of axn_dgelu_dbias: rows p, p + 4, p + 8, ... of a band of 128 one after
+    the other, the four phases in pairs; the bands in four quarters of consecutive ones, the quarters in pairs."""
+    M, N = x.shape
+    bands = (M + 127) // 128
+    x = torch.cat([x, x.new_zeros(bands * 128 - M, N)]).view(bands, 32, 4, N)
+    phase = x.new_zeros(bands, 4, N)
+    for i in range(32):
+        phase = phase + x[:, i]
+    band = (phase[:, 0] + phase[:, 1]) + (phase[:, 2] + phase[:, 3])
+    per = (bands + 3) // 4
+    quarter = x.new_zeros(4, N)
+    for q in range(4):
+        for b in range(q * per, min((q + 1) * per, bands)):
+            quarter[q] = quarter[q] + band[b]
+    return (quarter[0] + quarter[1]) + (quarter[2] + quarter[3])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("M,N", [(1, 8), (31, 136), (33, 128), (129, 1032), (257, 4104), (1700, 520), (2900, 6144)])
+def test_dgelu_dbias_adds_in_the_order_of_its_bands(M, N, dtype):
+    """The bias gradient bit for bit: its order of sums is part of what a step reproduces."""
+    from axonn_amd import _native as nv, ops
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    dY = (torch.randn(M, N, generator=g, device="cuda") + 0.2).to(dtype)
+    assert torch.equal(ops.dgelu_dbias(dY)[1], sums_by_bands(dY.float()))
+    wide = torch.zeros(M, N + 8, device="cuda", dtype=dtype)
+    wide[:, :N] = dY
+    start = torch.randn(N, generator=g, device="cuda")
+    _, db = ops.dgelu_dbias(wide[:, :N], dbias_out=start.clone(), accumulate=True)
+    assert torch.equal(db, start + sums_by_bands(dY.float()))
+    Z = torch.randn(M, N, generator=g, device="cuda").to(dtype)
+    dz, db = ops.dgelu_dbias(dY, Z)
+    want = sums_by_bands(dz.float())
+    if dtype == torch.bfloat16:
+        assert torch.equal(db, want)
+    elif dtype == torch.float16:   # (the first two columns of eight add products rounded once, see the kernel)
+        assert torch.equal(db.view(-1, 8)[:, 2:], want.view(-1, 8)[:, 2:])
+    inplace = dY.clone()   # dZ over dY
+    ws = torch.full(((M + 127) // 128 * N + 8,), float("nan"), device="cuda")
+    db2 = torch.empty_like(db)
+    need = nv.load().axn_dgelu_dbias_workspace_bytes(M, N)
+    assert need == (M + 127) // 128 * N * 4
+    nv.call("axn_dgelu_dbias", nv.ptr(inplace), nv.ptr(Z), nv.ptr(inplace), nv.dtype_code(dtype), nv.ptr(db2), M, N, N,
+            0, nv.ptr(ws), need, nv.current_stream())
+    assert torch.equal(inplace, dz) and torch.equal(db2, db) and bool(torch.isnan(ws[-8:]).all())
 
 
 def test_dgelu_dbias_matches_oracle():

@@ -203,8 +203,8 @@ inline bool stream_ahead(int64_t M, int64_t N, int64_t Kc) {
 }
 constexpr int64_t kStreamMaxLd = 1LL << 24;
 int launch_gemm_stream(const GemmArgs& args, int epilogue, bool out_f32, bool half, hipStream_t stream);
-// The gate/up forward (launch_gemm_swiglu) of up to kStreamMaxRows rows, N a multiple of 8; the two products of up
-// to 32 rows are those of launch_gemm_stream bit for bit.
+// The gate/up forward (launch_gemm_swiglu) of up to kStreamMaxRows rows, N a multiple of 8; the two products are
+// those of launch_gemm_stream bit for bit.
 int launch_gemm_stream_swiglu(const GemmArgs& args, bool half, hipStream_t stream);
 
 // C = silu(A B^T) * (A B2^T) in one launch (both weight matrices [N][Kc], K-major), for

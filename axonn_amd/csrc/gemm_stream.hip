@@ -45,12 +45,15 @@ __device__ __forceinline__ void store_swiglu4(const f32x4& vg, const f32x4& vu, 
   *(lpx4*)((uint16_t*)g.C + o) = out;
 }
 
-// D: lines of the contraction a wave has on their way (its ring's slots).
-template <int MT, int R, int NW, int D, int EPI, bool OUT_F32, bool HALF>
+// D: lines of the contraction a wave has on their way (its ring's slots); DX: of those, slots for X.  With one, a
+// line's part of X follows when the line before it is in registers: it comes from L2, and four waves have each other's
+// latency, which rings too large for LDS leave room for.
+template <int MT, int R, int NW, int D, int DX, int EPI, bool OUT_F32, bool HALF>
 __device__ __forceinline__ void stream_gemm(const GemmArgs& g) {
   constexpr int GROUPS = R + MT;              // 16-row groups copied per line: W's, then X's
-  constexpr uint32_t LINE = GROUPS * 2048;    // bytes of a slot
+  constexpr uint32_t WLINE = R * 2048, XLINE = MT * 2048;   // bytes of a slot
   constexpr int COPIES = 2 * GROUPS;
+  static_assert(DX == D || (DX == 1 && D == 2), "slots of X");
   // Gate/up forward: the first half of W's groups are rows of the gate weights, the second half the rows of
   // the up weights with the same indices.
   constexpr bool SWIGLU = EPI == EPI_SWIGLU;
@@ -62,7 +65,8 @@ __device__ __forceinline__ void stream_gemm(const GemmArgs& g) {
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
   const int n0 = blockIdx.x * (16 * RO);
-  char* ring = lds + wave * (D * LINE);
+  char* const ring = lds + wave * (D * WLINE + DX * XLINE);
+  char* const xring = ring + D * WLINE;
 
   // Copies: 8 rows of 128 bytes each.  Rows past the end are outside the buffer and come as
   // zeros; so do the chunks past the contraction's end in its last line.
@@ -91,23 +95,25 @@ __device__ __forceinline__ void stream_gemm(const GemmArgs& g) {
   const unsigned start = SWIGLU ? (unsigned)n0 / (unsigned)g.start_rows : blockIdx.x;
   const int rot = (int)((start * 7u) % (unsigned)lines);
   const int mine = (lines - wave + NW - 1) / NW;   // lines wave, wave + NW, ... (may be 0 or less)
-  auto copy_line = [&](int i) {                    // the wave's i-th line into slot i % D
+  // the wave's i-th line of W into slot i % D, of X into slot i % DX
+  auto copy = [&](int i, bool of_w, bool of_x) {
     int line = wave + i * NW + rot;
     if (line >= lines) line -= lines;
     const int k0 = line * 64;
-    char* to = ring + (i % D) * LINE;
+    char* const to = ring + (i % D) * WLINE;
+    char* const xto = xring + (i % DX) * XLINE;
     const bool cut = k0 + 64 > g.Kc;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const bool out = cut && k0 + 8 * chunk[h] >= g.Kc;
       const uint32_t ow = out ? kOutside : vw[h], ox = out ? kOutside : vx[h];
 #pragma unroll
-      for (int j = 0; j < R; ++j)
+      for (int j = 0; of_w && j < R; ++j)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(j < RO ? rw : rw2, LDS_PTR(void, to + j * 2048 + h * 1024), 16,
                                                  (int)ow, (int)(k0 * 2 + (j % RO) * w_group), 0, 2);   // non-temporal: read once (4 % on the kernel)
 #pragma unroll
-      for (int j = 0; j < MT; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, LDS_PTR(void, to + (R + j) * 2048 + h * 1024), 16, (int)ox,
+      for (int j = 0; of_x && j < MT; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, LDS_PTR(void, xto + j * 2048 + h * 1024), 16, (int)ox,
                                                  (int)(k0 * 2 + j * x_group), 0, 0);
     }
   };
@@ -125,22 +131,25 @@ __device__ __forceinline__ void stream_gemm(const GemmArgs& g) {
       c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   };
 
-  const uint32_t ring0 = (uint32_t)(uintptr_t)LDS_PTR(char, ring);
+  const uint32_t ring0 = (uint32_t)(uintptr_t)LDS_PTR(char, ring), xring0 = ring0 + D * WLINE;
   const uint32_t frag0 = (uint32_t)(r * 128 + ((q ^ ((r >> 1) & 7)) << 4));        // first 32 elements
   const uint32_t frag1 = (uint32_t)(r * 128 + (((4 + q) ^ ((r >> 1) & 7)) << 4));  // last 32
-  auto multiply_line = [&](int i) {
-    const uint32_t at = ring0 + (uint32_t)(i % D) * LINE;
+  // `then`: called when the line's fragments are in registers and its slots are free
+  auto multiply_line = [&](int i, auto then) {
+    const uint32_t at = ring0 + (uint32_t)(i % D) * WLINE, xat = xring0 + (uint32_t)(i % DX) * XLINE;
     bf16x8 f[GROUPS][2];
     static_for<GROUPS>([&](auto j_) {
       constexpr int J = decltype(j_)::value;
-      f[J][0] = lds_read_b128<J * 2048>(at + frag0);
-      f[J][1] = lds_read_b128<J * 2048>(at + frag1);
+      const uint32_t from = J < R ? at : xat;
+      f[J][0] = lds_read_b128<(J < R ? J : J - R) * 2048>(from + frag0);
+      f[J][1] = lds_read_b128<(J < R ? J : J - R) * 2048>(from + frag1);
     });
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
     for (int j = 0; j < GROUPS; ++j)
 #pragma unroll
       for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(f[j][h]));   // used behind the wait only
+    then();
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -149,17 +158,34 @@ __device__ __forceinline__ void stream_gemm(const GemmArgs& g) {
         for (int j = 0; j < R; ++j) mfma(f[j][h], f[R + i2][h], acc[i2][j]);
   };
 
+  auto nothing = [] {};
+  if constexpr (DX == D) {
 #pragma unroll
-  for (int i = 0; i < D; ++i)
-    if (i < mine) copy_line(i);
-  int i = 0;
-  for (; i + D < mine; ++i) {        // line i has landed when only the D - 1 behind it are on their way
-    wait_vmcnt<COPIES * (D - 1)>();
-    multiply_line(i);
-    copy_line(i + D);                // into the slot whose fragments are in registers now
+    for (int i = 0; i < D; ++i)
+      if (i < mine) copy(i, true, true);
+    int i = 0;
+    for (; i + D < mine; ++i) {        // line i has landed when only the D - 1 behind it are on their way
+      wait_vmcnt<COPIES * (D - 1)>();
+      multiply_line(i, nothing);
+      copy(i + D, true, true);         // into the slot whose fragments are in registers now
+    }
+    wait_vmcnt<0>();
+    for (; i < mine; ++i) multiply_line(i, nothing);
+  } else {
+    // On their way, in this order: W's line i, X's line i, W's line i + 1.
+    if (mine > 0) copy(0, true, true);
+    if (mine > 1) copy(1, true, false);
+    for (int i = 0; i < mine; ++i) {
+      if (i + 1 < mine)
+        wait_vmcnt<2 * R>();
+      else
+        wait_vmcnt<0>();
+      multiply_line(i, [&] {
+        if (i + 1 < mine) copy(i + 1, false, true);
+        if (i + 2 < mine) copy(i + 2, true, false);
+      });
+    }
   }
-  wait_vmcnt<0>();
-  for (; i < mine; ++i) multiply_line(i);
 
   // The rings are free once every wave is here.
   __syncthreads();
@@ -196,22 +222,22 @@ __device__ __forceinline__ void stream_gemm(const GemmArgs& g) {
 
 template <int MT, int R, int NW, int D, int EPI, bool OUT_F32, bool HALF>
 __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(const GemmArgs g) {
-  stream_gemm<MT, R, NW, D, EPI, OUT_F32, HALF>(g);
+  stream_gemm<MT, R, NW, D, D, EPI, OUT_F32, HALF>(g);
 }
-template <int MT, int R, int NW, int D, bool HALF>
+template <int MT, int R, int NW, int D, int DX, bool HALF>
 __global__ void __launch_bounds__(NW * 64) gemm_gate_up_stream_kernel(const GemmArgs g) {
-  stream_gemm<MT, R, NW, D, EPI_SWIGLU, false, HALF>(g);
+  stream_gemm<MT, R, NW, D, DX, EPI_SWIGLU, false, HALF>(g);
 }
 
 // The rings, or the waves' sums behind them.
-constexpr size_t stream_lds(int MT, int R, int NW, int D) {
-  const size_t ring = (size_t)NW * D * (R + MT) * 2048, sums = (size_t)NW * MT * R * 1024;
+constexpr size_t stream_lds(int MT, int R, int NW, int D, int DX) {
+  const size_t ring = (size_t)NW * (D * R + DX * MT) * 2048, sums = (size_t)NW * MT * R * 1024;
   return ring > sums ? ring : sums;
 }
 
 template <int MT, int R, int NW, int D, bool HALF>
 int launch_stream(const GemmArgs& g, int epilogue, bool out_f32, hipStream_t stream) {
-  constexpr size_t lds = stream_lds(MT, R, NW, D);
+  constexpr size_t lds = stream_lds(MT, R, NW, D, D);
   const dim3 grid((unsigned)ceil_div(g.N, 16 * R)), block(NW * 64);
 #define STREAM(EPI, F32)                                                                   \
   {                                                                                        \
@@ -263,16 +289,19 @@ int launch_stream_tokens(const GemmArgs& g, int epilogue, bool out_f32, hipStrea
 //   2816 x 1024   11.8 -> 4.9, 5.9, 8.3           14.3 -> 6.5, 8.4, 13.7
 //   5632 x 2048   16.0 -> 11.1, 10.0, 14.6        23.5 -> 18.2, 13.9, 22.7
 //   8192 x 3072   23.1 -> 17.7, 17.7, 23.3        33.8 -> 28.6, 22.1, 32.9
-//   11008 x 4096  38.6 -> 29.6, 34.6, 31.3        54.1 -> 47.9, 46.3, 40.3
-//   14336 x 4096  45.2 -> 38.1, 37.8, 38.0        57.6 -> 63.0, 49.6, 43.1
-// (R = 8 of more than 32 tokens with two waves: with four its rings are larger than LDS.)  16384 x 4096 at 16
-// tokens: 40.2 us, 6.7 TB/s.
-template <int MT, int R, int NW, int D, bool HALF>
+//   11008 x 4096  38.6 -> 29.6, 34.6, 31.3        54.1 -> 47.9, 46.3, 38.5
+//   14336 x 4096  45.2 -> 38.1, 37.8, 38.0        57.6 -> 63.0, 49.6, 43.2
+// (R = 8 of more than 32 tokens with one slot for X a wave: with two its rings are larger than LDS.  With two slots
+// and two waves, whose sums are twice as long, 40.8 and 43.7; 28672 x 8192 157, so 153.)  16384 x 4096 at 16 tokens:
+// 40.2 us, 6.7 TB/s.
+template <int MT, int R, int D, int DX, bool HALF>
 int launch_gate_up_stream(const GemmArgs& in, hipStream_t stream) {
-  constexpr size_t lds = stream_lds(MT, R, NW, D);
+  constexpr int NW = 4;
+  constexpr size_t lds = stream_lds(MT, R, NW, D, DX);
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
   GemmArgs g = in;
   g.start_rows = 16 * stream_groups(g.N);
-  void (*kern)(const GemmArgs) = gemm_gate_up_stream_kernel<MT, R, NW, D, HALF>;
+  void (*kern)(const GemmArgs) = gemm_gate_up_stream_kernel<MT, R, NW, D, DX, HALF>;
   static std::atomic<unsigned long long> lds_allowed{0};
   const int rc = allow_lds((const void*)kern, lds, lds_allowed);
   if (rc != AXN_OK) return rc;
@@ -283,9 +312,9 @@ int launch_gate_up_stream(const GemmArgs& in, hipStream_t stream) {
 template <int MT, int D2, bool HALF>
 int launch_stream_swiglu(const GemmArgs& g, hipStream_t stream) {
   if (g.N <= 16 * 256 || (g.N > 32 * 256 && MT == 1))
-    return launch_gate_up_stream<MT, 2, 4, D2, HALF>(g, stream);
-  if (g.N <= 32 * 256) return launch_gate_up_stream<MT, 4, 4, 2, HALF>(g, stream);
-  return launch_gate_up_stream<MT, 8, MT == 4 ? 2 : 4, 2, HALF>(g, stream);
+    return launch_gate_up_stream<MT, 2, D2, D2, HALF>(g, stream);
+  if (g.N <= 32 * 256) return launch_gate_up_stream<MT, 4, 2, 2, HALF>(g, stream);
+  return launch_gate_up_stream<MT, 8, 2, MT == 4 ? 1 : 2, HALF>(g, stream);
 }
 template <bool HALF>
 int launch_stream_swiglu_tokens(const GemmArgs& g, hipStream_t stream) {

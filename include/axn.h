@@ -230,8 +230,8 @@ AXN_API int axn_gemm_swiglu_fwd(const void* X, const void* Wg, const void* Wu, v
                                 int64_t K, int64_t ldx, int64_t ldw, int64_t ldh, void* stream);
 
 /* The same for 1 to 64 rows of X (token by token generation) and any N and K that are multiples of 8, row
- * strides below 2^24 elements (AXN_ESHAPE otherwise): a stream over both weight matrices.  Sums of more than 32
- * rows may be in another order than axn_gemm_fwd's. */
+ * strides below 2^24 elements (AXN_ESHAPE otherwise): a stream over both weight matrices.  The two products are
+ * axn_gemm_fwd's bit for bit. */
 AXN_API int axn_gemm_swiglu_fwd_few(const void* X, const void* Wg, const void* Wu, void* H,
                                     void* gate_save, void* up_save, int dtype, int64_t M, int64_t N,
                                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldh, void* stream);

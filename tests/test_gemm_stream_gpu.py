@@ -124,3 +124,23 @@ def test_gate_up_of_few_tokens(M, N, K, dtype):
     else:   # other order of sums: a rounding of each factor and of the product
         eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
         assert ((h.double() - want.double()).norm() / want.double().norm()) < 4 * eps
+
+
+@pytest.mark.parametrize("M", [33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(8200, 8), (8200, 264), (9000, 72), (11008, 1160), (16392, 200), (8256, 4096)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gate_up_of_33_to_64_tokens_gives_the_bits_of_the_two_products(M, N, K, dtype):
+    """Over more than 8192 outputs, where a wave has one slot for the tokens: lines of the contraction on one to
+    four waves, one to many a wave."""
+    from axonn_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    X, G, U = (torch.randn(n, K, generator=gen, device="cuda").to(dtype) * s for n, s in ((M, 1), (N, 0.1), (N, 0.1)))
+    h, gate, up = ops.gemm_swiglu_fwd(X, G, U, save=True, few=True)
+    sfx = "" if dtype == torch.bfloat16 else "_f16"
+    want = [torch.empty_like(h), torch.empty_like(h)]
+    for w, out in zip((G, U), want):   # (without a workspace: always the stream)
+        nv.call("axn_gemm_fwd" + sfx, nv.ptr(X), nv.ptr(w), None, nv.ptr(out), None, M, N, K, K, K, N, nv.EPI_NONE,
+                nv.current_stream())
+    assert torch.equal(gate, want[0]) and torch.equal(up, want[1])
+    assert torch.equal(h, ops.swiglu_fwd(*want))

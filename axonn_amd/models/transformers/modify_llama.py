@@ -19,6 +19,7 @@ forward passes to Hugging Face.  Here
 """
 
 import torch
+from torch.nn.modules import module as module_hooks
 from transformers.models.llama.modeling_llama import LlamaAttention, LlamaMLP, ACT2FN
 
 from axonn_amd import ops
@@ -91,12 +92,29 @@ class GateUpSwiGLU(torch.autograd.Function):
         return grad_x, grad_wg, grad_wu, None, None
 
 
+_linear_forward = Linear.forward
+
+
+def _called_as_linear(layer):
+    """Calling `layer` does what Linear does with its weight and nothing else: its forward is neither rebound on
+    the instance (offloading and quantisation do that) nor on the class, and no hook of its own or of all modules
+    runs with it.  (What Module's own short cut looks at, and the replacements.)"""
+    return (type(layer) is Linear and "forward" not in layer.__dict__ and Linear.forward is _linear_forward
+            and layer.__dict__.get("_compiled_call_impl") is None
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
+                     or layer._backward_pre_hooks or module_hooks._global_forward_hooks
+                     or module_hooks._global_forward_pre_hooks or module_hooks._global_backward_hooks
+                     or module_hooks._global_backward_pre_hooks))
+
+
 def _one_launch_gate_up(mlp, x):
     """The MLP's gate/up pair qualifies for the one-launch forward: SiLU, no biases,
     plain layers on one rank, 16-bit compute type and whole-tile shapes, or up to 64 tokens without
-    gradients (generation)."""
+    gradients (generation).  Layers that something watches or has replaced are called themselves."""
     g, u = mlp.gate_proj, mlp.up_proj
     if not (getattr(mlp, "_axonn_fused_swiglu", False) and x.is_cuda):
+        return False
+    if not (_called_as_linear(g) and _called_as_linear(u)):
         return False
     if g.bias is not None or u.bias is not None or g.fused_activation or u.fused_activation:
         return False
@@ -107,10 +125,7 @@ def _one_launch_gate_up(mlp, x):
     sizes = tokens, g.local_out_features, g.local_in_features, dt
     if torch.is_grad_enabled() or tokens > 64:
         return ops.gemm_swiglu_supported(*sizes)
-    # (layers that something watches or has replaced are called themselves)
-    return (type(g) is type(u) is Linear and not (g._forward_hooks or g._forward_pre_hooks or u._forward_hooks
-                                                  or u._forward_pre_hooks)
-            and x.shape[-1] == g.local_in_features and ops.gemm_swiglu_few_supported(*sizes))
+    return x.shape[-1] == g.local_in_features and ops.gemm_swiglu_few_supported(*sizes)
 
 
 def modified_mlp_init(self, config):

@@ -328,6 +328,55 @@ def test_generation_runs_gate_up_in_one_launch(tokens):
     assert rel(np64(fused), np64(separate)) < 1e-2
 
 
+@pytest.mark.parametrize("tokens,grad", [(1, False), (16, False), (64, False), (256, False), (256, True)])
+def test_replaced_and_watched_projections_are_called(tokens, grad, monkeypatch):
+    """A projection whose forward is rebound on the instance or on the class, or that a hook of all modules watches,
+    is called itself, at sizes that run in one launch otherwise."""
+    from transformers import LlamaConfig
+    from transformers.models.llama.modeling_llama import LlamaMLP
+
+    import axonn_amd.axonn as ax
+    from axonn_amd.intra_layer import Linear
+    from axonn_amd.models.transformers import modify_llama, parallelize
+
+    ax.init(1, 1, 1, 1)
+    cfg = LlamaConfig(hidden_size=128, intermediate_size=384, num_attention_heads=4, num_key_value_heads=2,
+                      num_hidden_layers=1, vocab_size=32)
+    with parallelize(cfg):
+        mlp = LlamaMLP(cfg)
+    mlp.forward = modify_llama.modified_mlp_forward.__get__(mlp)
+    mlp = mlp.cuda().bfloat16()
+    x = torch.randn(1, tokens, 128, device="cuda").bfloat16()
+    with torch.set_grad_enabled(grad):
+        assert modify_llama._one_launch_gate_up(mlp, x)
+        plain = mlp(x)
+        for name in ("gate_proj", "up_proj"):
+            layer = getattr(mlp, name)
+            own = layer.forward
+            layer.forward = lambda *args: own(*args) * 0     # as offloading and quantisation attach themselves
+            assert not mlp(x).any()
+            del layer.forward
+            handle = layer.register_forward_pre_hook(lambda module, args: (args[0] * 0,))
+            assert not mlp(x).any()
+            handle.remove()
+        seen = []
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda module, args, out: seen.append(module))
+        mlp(x)
+        handle.remove()
+        assert mlp.gate_proj in seen and mlp.up_proj in seen
+        with monkeypatch.context() as patch:
+            original = Linear.forward
+            patch.setattr(Linear, "forward", lambda self, *args: original(self, *args) * 0)
+            assert not mlp(x).any()
+        assert torch.equal(mlp(x), plain)
+        if grad:
+            called = []
+            handle = mlp.up_proj.register_full_backward_hook(lambda module, gi, go: called.append(module))
+            mlp(x.clone().requires_grad_(True)).sum().backward()
+            handle.remove()
+            assert called == [mlp.up_proj]
+
+
 def test_mlp_with_one_launch_gate_up_equals_the_separate_path(monkeypatch):
     """The patched MLP at a whole-tile shape takes the one-launch gate/up forward; with
     that path switched off it takes three launches.  Output and weight gradients agree bit

@@ -715,9 +715,18 @@ double filled(long long n1, double s1, long long n2, double s2) {
 // a stage of a time that lies between the work's average over the CUs and that of the fullest one (0.3 to 0.7), a
 // tile counting 3 stages more than it has, 6 where it reads dW to add to it, and the parts' cost; fitted to 65
 // problems of 64 to 3564 tokens with 2 to 16 parts each (7 % rms).  The two launches, whose estimate is 8 % low, and
-// 20 % beyond 100 us, where the power cap stretches it, have to be slower.  Of 110 other problems 25 take one launch,
-// 0.76 to 1.03 of the time of two, 0.89 on average; adding to dW 21, 0.72 to 0.99.  Up to 192 rows a weight gradient
+// 20 % beyond 100 us, where the power cap stretches it, have to be slower.  Up to 192 rows a weight gradient
 // is nearly all stores, and two launches are as fast (151 x 11392 x 4992: 75 us, 79 in one).
+// Where that estimate is not enough, from 758 problems that it takes (481 of whole 128 x 128 x 64 tiles, whose two
+// launches have kernels without bounds; us, two launches / one):
+//   too few tiles in all to fill the CUs, which smaller tiles of a launch alone do        1536 x 3072 x 1024  37 / 44
+//   at most 64 tiles of dX, unless they run beside one round of stores of dW + ...        256 x 11136 x 1664  45 / 50
+//   more than 200 tiles of dX (nearly a round of their own) of a whole-tile problem, unless the estimate is well ahead
+//                                                                                         512 x 11008 x 8192 186 / 196
+//   adding to dW in tiles that reach past its edge where those of two launches do not      256 x 18560 x 5632 209 / 236
+//   adding to more than 256 tiles of dW from at most 256 rows with bounds                  237 x 13312 x 5376 154 / 180
+// Of 284 problems drawn anew that it then takes (121 whole), one launch has 0.90 of the time of two on average, seven
+// take 2 to 5 % longer.
 int gemm_backward_parts(int64_t M, int64_t N, int64_t K, bool add) {
   if (M <= 192) return 0;
   double apart_d = 0, apart_w = 0;
@@ -727,12 +736,15 @@ int gemm_backward_parts(int64_t M, int64_t N, int64_t K, bool add) {
   edge_tile(N, K, M, {}, &apart_w);
   if (add) apart_w += 0.5 * (double)N * (double)K * 2e-6 / 5.72;   // reading dW, half of it hidden
   const long long td = ceil_div(M, 256) * ceil_div(K, 256) * parts;
+  const bool whole = M % 64 == 0 && N % 128 == 0 && K % 128 == 0, large = N % 256 == 0 && K % 256 == 0;
+  if (td + tw <= 160 || (td <= 64 && !(add && tw <= 256))) return 0;
+  if (add && (whole ? !large : M <= 256 && tw > 256)) return 0;
   const double d = (double)(ceil_div(ceil_div(N, 64), parts) + 3), w = (double)(ceil_div(M, 64) + (add ? 6 : 3));
   const double fullest = d >= w ? filled(td, d, tw, w) : filled(tw, w, td, d);
   const double average = ((double)td * d + (double)tw * w) / 256;
   const double us = 2.2 + 1.45 * (0.7 * fullest + 0.3 * average) + kPartsMicroseconds + parts * part_microseconds(M, K);
   const double apart = apart_d + apart_w;
-  return us < apart * (apart < 100 ? 1.08 : 1.2) ? parts : 0;
+  return us < apart * (apart < 100 ? 1.08 : whole && td > 200 ? 1.1 : 1.2) ? parts : 0;
 }
 
 int launch_gemm_backward_parts(const GemmArgs& dgrad, const GemmArgs& wgrad, bool half, bool dw_f32, int parts,

@@ -191,6 +191,21 @@ def test_gate_up_forward_argument_errors():
     assert "M % 256 == 0" in _err()
 
 
+@pytest.mark.parametrize("M,N,K,beta,joint", [
+    # where one launch of both gradients was measured slower than two, and neighbours where it is faster
+    (1536, 3072, 1024, 0, False), (1280, 2560, 1280, 0, False), (1536, 6144, 1024, 0, True),
+    (256, 11136, 1664, 0, False), (256, 9728, 1792, 1, False), (768, 4864, 1792, 1, True),
+    (512, 11008, 8192, 0, False), (1024, 32000, 3584, 0, False), (1280, 15360, 2304, 0, True),
+    (256, 18560, 5632, 1, False), (512, 13312, 3712, 1, False), (249, 25472, 4864, 1, False), (237, 13312, 5376, 1, False),
+    (256, 14336, 4096, 0, True), (1376, 9088, 2112, 0, True), (649, 4032, 2176, 1, True), (1024, 6144, 4096, 0, True),
+])
+def test_sizes_whose_gradients_take_one_launch(M, N, K, beta, joint):
+    parts = nv.load().axn_gemm_bwd_workspace_bytes(M, N, K, beta) // (M * K * 4)
+    assert (parts > 1) == joint
+    if joint:   # the input gradient's own parts
+        assert parts * M * K * 4 == nv.load().axn_gemm_workspace_bytes(1, M, N, K)
+
+
 def test_gate_up_forward_of_few_rows_argument_errors():
     f = nv.load().axn_gemm_swiglu_fwd_few
     ok = (nv.BF16, 16, 128, 64, 64, 64, 128, None)

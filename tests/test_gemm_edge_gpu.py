@@ -346,3 +346,11 @@ def test_both_gradients_in_one_launch_with_the_contraction_in_parts(M, N, K, bet
     assert torch.equal(both[0], want_dx)
     check(fx, dx, want_dx)
     check(fw, dw, want_dw)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,beta,dw_f32", [(256, 14336, 4096, 0, False), (768, 4864, 1792, 1, True),
+                                               (1024, 6144, 4096, 0, False), (640, 6016, 3200, 0, True)])
+def test_both_gradients_in_one_launch_of_whole_tiles(M, N, K, beta, dw_f32, dtype):
+    """Against the kernels without bounds that the two calls take here."""
+    test_both_gradients_in_one_launch_with_the_contraction_in_parts(M, N, K, beta, dw_f32, dtype)

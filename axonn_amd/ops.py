@@ -82,14 +82,18 @@ def _any_n(dtype, N, K):
     return dtype in _GEMM16 and N % 8 != 0 and K % 8 == 0
 
 
+def _padded_width(N):
+    """Row stride of `_pad_rows`' result.  Wide rows start on whole 128-byte lines: a tile's copies, 128 bytes of a
+    row each, else take two (input gradient of 2048 x 50257 x 2048 with rows of 50264 elements 358 us, of 50304 323;
+    of 700 x 19999 x 768 50.1 and 47.3)."""
+    return N + (-N) % (64 if N >= 4096 else 8)
+
+
 def _pad_rows(t):
-    """[M, N] -> [M, N rounded up to a multiple of 8], zeros behind the columns.  Wide rows start on whole
-    128-byte lines: a tile's copies, 128 bytes of a row each, else take two (input gradient of 2048 x 50257
-    x 2048 with rows of 50264 elements 358 us, of 50304 323; of 700 x 19999 x 768 50.1 and 47.3)."""
+    """[M, N] -> [M, N rounded up to a multiple of 8], zeros behind the columns."""
     t, ld = _rows(t)
     M, N = t.shape
-    n8 = N + (-N) % 8
-    ld_out = N + (-N) % 64 if N >= 4096 else n8
+    n8, ld_out = N + (-N) % 8, _padded_width(N)
     out = torch.empty((M, ld_out), dtype=t.dtype, device=t.device)
     nv.call("axn_pad_rows16_to", nv.ptr(t), nv.ptr(out), M, N, ld, ld_out, nv.current_stream())
     return out if ld_out == n8 else out[:, :n8]
@@ -324,11 +328,11 @@ def _bwd_in_parts(dy, w, x, out, accumulate, out_dtype):
     out_dtype = out_dtype or dy.dtype
     if out_dtype not in (dy.dtype, torch.float32):
         return None
+    if max(_padded_width(N) if N % 8 else N, K) >= _FAR_ROWS:   # (views with rows that far apart are packed below)
+        return None
     dy, lddy = _prep_bf16(_pad_rows(dy) if N % 8 else dy)
     w, ldw = _prep_bf16(w)
     x, ldx = _prep_bf16(x)
-    if max(lddy, ldw, ldx) >= _FAR_ROWS:
-        return None
     dx = torch.empty((M, K), dtype=dy.dtype, device=dy.device)
     if out is None:
         out = torch.empty((N, K), dtype=out_dtype, device=dy.device)

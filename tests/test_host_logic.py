@@ -303,3 +303,19 @@ def test_parallelize_patches_every_family_the_reference_patches(family, n_linear
         cfg.architectures = ["GPT2LMHeadModel"]
         with parallelize(cfg):
             pass
+
+
+def test_gradients_in_one_launch_are_refused_before_anything_is_copied(monkeypatch):
+    """Rows too long for the joint launch: the pass that pads dY is left to the calls that take them."""
+    from axonn_amd import ops
+
+    padded = []
+    monkeypatch.setattr(ops, "_pad_rows", lambda t: padded.append(t) or t)
+    monkeypatch.setattr(ops, "_prep_bf16", lambda t: padded.append(t) or (t, t.shape[1]))
+    monkeypatch.setattr(ops, "_FAR_ROWS", 128)
+    dy, x = torch.zeros(4, 121).bfloat16(), torch.zeros(4, 16).bfloat16()
+    w = torch.zeros(121, 16).bfloat16()
+    assert ops._bwd_in_parts(dy, w, x, None, False, None) is None      # 121 + 7 = 128
+    assert ops._bwd_in_parts(dy[:, :8], torch.zeros(8, 128).bfloat16(), torch.zeros(4, 128).bfloat16(), None, False,
+                             None) is None
+    assert not padded

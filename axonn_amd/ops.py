@@ -83,10 +83,20 @@ def _any_n(dtype, N, K):
 
 
 def _padded_width(N):
-    """Row stride of `_pad_rows`' result.  Wide rows start on whole 128-byte lines: a tile's copies, 128 bytes of a
+    """Row stride of `_pad_rows`' result.  Rows start on whole 128-byte lines: a tile's copies, 128 bytes of a
     row each, else take two (input gradient of 2048 x 50257 x 2048 with rows of 50264 elements 358 us, of 50304 323;
-    of 700 x 19999 x 768 50.1 and 47.3)."""
-    return N + (-N) % (64 if N >= 4096 else 8)
+    padding and both gradients of 256 to 2048 rows x 4100 to 20000 columns, inputs of 768 and 2048: 0 to 4 % less, 8 %
+    beyond 30000).  Rows of 1000 to 4000 gain 0 to 3 % on the GPU and lose 3 us of host time to the view
+    without the padding (700 x 1501 x 2048 29.5 -> 32.9 us).  Strides 1/128 or 1/256 beyond a power of two are left out:
+    the rows of a tile crowd onto few memory channels (both gradients of 2048 x 33001 x 2048 with rows of 33024 elements
+    542 us, of 33088 487; 2048 x 32885 x 2048, 32896 585, 32960 486; 2048 x 16453 x 768, 16512 164, 16576 145)."""
+    if N < 4096:
+        return N + (-N) % 8
+    ld = N + (-N) % 64
+    power = 1 << (ld.bit_length() - 1)
+    while ld - power in (power // 256, power // 128):
+        ld += 64
+    return ld
 
 
 def _pad_rows(t):

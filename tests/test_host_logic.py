@@ -319,3 +319,13 @@ def test_gradients_in_one_launch_are_refused_before_anything_is_copied(monkeypat
     assert ops._bwd_in_parts(dy[:, :8], torch.zeros(8, 128).bfloat16(), torch.zeros(4, 128).bfloat16(), None, False,
                              None) is None
     assert not padded
+
+
+def test_padded_rows_start_on_lines_and_off_the_crowded_strides():
+    from axonn_amd import ops
+
+    for N in [1, 9, 1023, 1025, 4097, 8193, 8250, 16385, 16449, 16500, 20201, 32833, 32890, 33001, 50257, 65700, 66001]:
+        ld = ops._padded_width(N)
+        assert N <= ld < N + (256 if N >= 4096 else 8) and ld % (64 if N >= 4096 else 8) == 0
+    assert [ops._padded_width(n) for n in (8250, 16440, 16500, 32890, 33001, 50257)] == [8320, 16576, 16576, 32960,
+                                                                                          33088, 50304]

@@ -22,7 +22,7 @@ BF16, F16, F32 = 0, 1, 2
 EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_GELU = 0, 1, 2, 3
 BIAS_16BIT = 0x100   # with an epilogue: the bias has the operands' 16-bit type
 
-ABI_VERSION = 14
+ABI_VERSION = 15   # another one with every change of the entry points below
 
 # Every symbol include/axn.h declares: name -> (restype, argtypes)
 _c = ctypes
@@ -143,15 +143,15 @@ def load():
         except ImportError:
             pass
         lib = ctypes.CDLL(_LIB_PATH)
-        for name, (restype, argtypes) in SYMBOLS.items():
-            fn = getattr(lib, name)
-            fn.restype = restype
-            fn.argtypes = argtypes
-        if lib.axn_abi_version() != ABI_VERSION:
+        if lib.axn_abi_version() != ABI_VERSION:   # (before the entry points, of which another version may lack some)
             raise ImportError(
                 "libaxn_gfx950.so has ABI version %d, this package needs %d"
                 % (lib.axn_abi_version(), ABI_VERSION)
             )
+        for name, (restype, argtypes) in SYMBOLS.items():
+            fn = getattr(lib, name)
+            fn.restype = restype
+            fn.argtypes = argtypes
         _lib = lib
     return _lib
 

@@ -5,6 +5,7 @@ the GPU (so all of this runs on a host without one)."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -29,6 +30,24 @@ def test_library_loads_and_exports_every_declared_symbol():
     for name in declared_symbols():
         assert hasattr(lib, name), "libaxn_gfx950.so does not export %s" % name
     assert nv.load().axn_abi_version() == nv.ABI_VERSION
+
+
+def test_the_version_goes_with_the_entry_points():
+    """A change of the entry points takes a version of its own: raise it together with what is written here."""
+    assert (nv.ABI_VERSION, len(nv.SYMBOLS)) == (15, 43)
+
+
+def test_a_library_of_another_version_is_refused_by_its_version(tmp_path, monkeypatch):
+    """Also one that lacks entry points: the message names the versions, not the first missing symbol."""
+    source = tmp_path / "old.c"
+    source.write_text("int axn_abi_version(void) { return 14; }\n")
+    old = tmp_path / "libold.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(old), str(source)], check=True)
+    monkeypatch.setattr(nv, "_LIB_PATH", str(old))
+    monkeypatch.setattr(nv, "_lib", None)
+    with pytest.raises(ImportError, match="ABI version 14"):
+        nv.load()
+    assert nv._lib is None
 
 
 def test_library_is_a_gfx950_code_object():

@@ -311,10 +311,10 @@ int launch_gate_up_stream(const GemmArgs& in, hipStream_t stream) {
 }
 template <int MT, int D2, bool HALF>
 int launch_stream_swiglu(const GemmArgs& g, hipStream_t stream) {
-  if (g.N <= 16 * 256 || (g.N > 32 * 256 && MT == 1))
-    return launch_gate_up_stream<MT, 2, D2, D2, HALF>(g, stream);
-  if (g.N <= 32 * 256) return launch_gate_up_stream<MT, 4, 2, 2, HALF>(g, stream);
-  return launch_gate_up_stream<MT, 8, 2, MT == 4 ? 1 : 2, HALF>(g, stream);
+  if (g.N > 16 * 256 && g.N <= 32 * 256) return launch_gate_up_stream<MT, 4, 2, 2, HALF>(g, stream);
+  if constexpr (MT > 1)
+    if (g.N > 32 * 256) return launch_gate_up_stream<MT, 8, 2, MT == 4 ? 1 : 2, HALF>(g, stream);
+  return launch_gate_up_stream<MT, 2, D2, D2, HALF>(g, stream);
 }
 template <bool HALF>
 int launch_stream_swiglu_tokens(const GemmArgs& g, hipStream_t stream) {

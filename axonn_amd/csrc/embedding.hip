@@ -917,7 +917,10 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
   const int64_t long_pieces = (H / (vec / 4) + 63) / 64;
   const int64_t long_blocks =
       T > EMB_LONG_RUN ? ((T + 63) / 64 * long_pieces + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK : 0;
-  const bool slots = T <= V / EMB_SLOT_ROWS && (beta != 0 || lddw == H);
+  // (a launch has fewer than 2^32 threads: one for each 16 bytes it clears, and those that sort)
+  const int64_t clearing = 1 + (T > 0 ? plan_sort(T, V).passes : 0);
+  const bool clears = lddw == H && V * (H / vec) / clearing < 0xd0000000LL;
+  const bool slots = T <= V / EMB_SLOT_ROWS && (beta != 0 || clears);
   const int64_t blocks = ((slots ? T : V) * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK + long_blocks;
   const size_t zero_bytes = slots && beta == 0 ? (size_t)V * (size_t)H * (dw_dtype == AXN_F32 ? 4 : 2) : 0;
   if (blocks + (int64_t)(zero_bytes / (16 * FILL_THREADS)) >= (1LL << 31)) {

@@ -187,6 +187,25 @@ def test_backward_on_either_side_of_two_table_rows_a_token(dtype, T, V, H):
     assert np.array_equal(host(out), twice)
 
 
+@pytest.mark.parametrize("T", [0, 1])
+def test_gradient_of_a_table_larger_than_one_launch_can_clear(T):
+    """68.7 GB and more of a gradient without tokens: 2^32 pieces of 16 bytes, and as many threads, are one too many."""
+    from axonn_amd import ops
+
+    V, H = (1 << 23) + 5, 2048
+    if torch.cuda.mem_get_info()[0] < 90 * 10 ** 9:
+        pytest.skip("needs 90 GB")
+    out = torch.empty(V, H, device="cuda", dtype=torch.float32)
+    for rows in out.split(1 << 20):
+        rows.fill_(7.0)
+    ids = torch.tensor([V - 1], device="cuda")[:T]
+    ops.embedding_bwd(ids, torch.ones(T, H, device="cuda"), V, out=out)
+    assert bool((out[V - 1] == float(T)).all())
+    assert not any(bool(rows.any()) for rows in out[:V - 1].split(1 << 20))
+    del out
+    torch.cuda.empty_cache()
+
+
 def test_backward_padding_row_repeated_ids_and_determinism():
     """A tenth of the tokens name one row, another tenth the padding row; the sum of 400
     terms depends on its order, and the kernel's order is the token order."""

@@ -18,6 +18,17 @@ int hip_fail(hipError_t e, const char* what);
     if (e__ != hipSuccess) return ::axn::hip_fail(e__, #expr); \
   } while (0)
 
+// ---- launches of many workgroups ---------------------------------------------------
+// A launch has fewer than 2^32 threads in a dimension; beyond, the grid wraps without an error.  So the workgroups
+// of a launch that may have that many go on in the next dimension, kMostBlocks (of up to 1024 threads) at a time, and
+// some behind the last one with nothing to do.  (A constant: the size of the grid would be another load.)
+constexpr int64_t kMostBlocks = 1 << 21;
+inline dim3 grid_of(int64_t blocks) {
+  return blocks <= kMostBlocks ? dim3((unsigned)blocks)
+                               : dim3((unsigned)kMostBlocks, (unsigned)((blocks + kMostBlocks - 1) / kMostBlocks));
+}
+__device__ __forceinline__ int64_t block_number() { return (int64_t)blockIdx.y * kMostBlocks + blockIdx.x; }
+
 // ---- exact-erf GELU -----------------------------------------------------------
 // gelu(x) = x * Phi(x), Phi(x) = (1 + erf(x / sqrt 2)) / 2, the definition behind
 // torch.nn.GELU() (approximate='none').  The library erff costs about 100 VALU

@@ -136,7 +136,7 @@ __global__ void __launch_bounds__((DG_THREADS<T, HAS_Z>))
   __shared__ float phases[4][DG_COLS];
   const int piece = threadIdx.x % DG_PIECES, row0 = threadIdx.x / DG_PIECES;
   const int c = threadIdx.x % DG_COLS, phase = threadIdx.x / DG_COLS;
-  const int64_t col0 = (int64_t)blockIdx.x * DG_COLS, band0 = (int64_t)blockIdx.y * DG_BAND;
+  const int64_t col0 = (blockIdx.z * kMostBlocks + blockIdx.x) * DG_COLS, band0 = (int64_t)blockIdx.y * DG_BAND;
   const int64_t col = col0 + piece * 8;
   float sum = 0.f;
 #pragma unroll
@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(256)
                         int64_t N, int beta) {
   __shared__ float red[4][64];
   const int tx = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int64_t c = (int64_t)blockIdx.x * 64 + tx;
+  const int64_t c = block_number() * 64 + tx;
   const int64_t per = (bands + 3) / 4;
   const int64_t b1 = (q + 1) * per < bands ? (q + 1) * per : bands;
   float s = 0.f;
@@ -225,8 +225,8 @@ __global__ void __launch_bounds__(EW_TX* EW_TY)
     swiglu_fwd_kernel(const T* gate, const T* up, T* out, int64_t M, int64_t N, int64_t ld) {
   const int tx = threadIdx.x % EW_TX, ty = threadIdx.x / EW_TX;
   const int64_t col_blocks = (N + EW_COLS - 1) / EW_COLS;
-  const int64_t band = blockIdx.x / col_blocks;
-  const int64_t col = (int64_t)(blockIdx.x - band * col_blocks) * EW_COLS + tx * 8;
+  const int64_t number = block_number(), band = number / col_blocks;
+  const int64_t col = (number - band * col_blocks) * EW_COLS + tx * 8;
   if (col >= N) return;
   const int64_t r0 = band * SWIGLU_BAND;
   const int64_t r1 = (r0 + SWIGLU_BAND < M) ? r0 + SWIGLU_BAND : M;
@@ -249,8 +249,8 @@ __global__ void __launch_bounds__(EW_TX* EW_TY)
                       int64_t N, int64_t ld, int64_t ld_out) {
   const int tx = threadIdx.x % EW_TX, ty = threadIdx.x / EW_TX;
   const int64_t col_blocks = (N + EW_COLS - 1) / EW_COLS;
-  const int64_t band = blockIdx.x / col_blocks;
-  const int64_t col = (int64_t)(blockIdx.x - band * col_blocks) * EW_COLS + tx * 8;
+  const int64_t number = block_number(), band = number / col_blocks;
+  const int64_t col = (number - band * col_blocks) * EW_COLS + tx * 8;
   if (col >= N) return;
   const int64_t r0 = band * SWIGLU_BAND;
   const int64_t r1 = (r0 + SWIGLU_BAND < M) ? r0 + SWIGLU_BAND : M;
@@ -277,11 +277,11 @@ int launch_swiglu_fwd(const void* gate, const void* up, void* out, int dtype, in
                       int64_t N, int64_t ld, hipStream_t stream) {
   const int64_t bands = (M + SWIGLU_BAND - 1) / SWIGLU_BAND;
   const int64_t blocks = bands * ((N + EW_COLS - 1) / EW_COLS);
-  if (blocks > 0x7fffffffLL) {
+  if (blocks > 0x7fffffffLL - kMostBlocks) {
     set_error("swiglu: too many elements (%lld x %lld)", (long long)M, (long long)N);
     return AXN_ELIMIT;
   }
-  const dim3 grid((unsigned)blocks), block(EW_TX * EW_TY);
+  const dim3 grid = grid_of(blocks), block(EW_TX * EW_TY);
   if (dtype == AXN_F32)
     hipLaunchKernelGGL(swiglu_fwd_kernel<float>, grid, block, 0, stream, (const float*)gate,
                        (const float*)up, (float*)out, M, N, ld);
@@ -300,11 +300,11 @@ int launch_swiglu_bwd(const void* dout, const void* gate, const void* up, void* 
                       hipStream_t stream) {
   const int64_t bands = (M + SWIGLU_BAND - 1) / SWIGLU_BAND;
   const int64_t blocks = bands * ((N + EW_COLS - 1) / EW_COLS);
-  if (blocks > 0x7fffffffLL) {
+  if (blocks > 0x7fffffffLL - kMostBlocks) {
     set_error("swiglu: too many elements (%lld x %lld)", (long long)M, (long long)N);
     return AXN_ELIMIT;
   }
-  const dim3 grid((unsigned)blocks), block(EW_TX * EW_TY);
+  const dim3 grid = grid_of(blocks), block(EW_TX * EW_TY);
   if (dtype == AXN_F32)
     hipLaunchKernelGGL(swiglu_bwd_kernel<float>, grid, block, 0, stream, (const float*)dout,
                        (const float*)gate, (const float*)up, (float*)dgate, (float*)dup, M, N, ld, ld_out);
@@ -338,7 +338,7 @@ int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
     }
     partial = (float*)ws;
   }
-  const dim3 grid((unsigned)((N + DG_COLS - 1) / DG_COLS), (unsigned)bands);
+  const dim3 columns = grid_of((N + DG_COLS - 1) / DG_COLS), grid(columns.x, (unsigned)bands, columns.y);
   if (bands > 65535) {
     set_error("dgelu_dbias: too many rows (%lld)", (long long)M);
     return AXN_ELIMIT;
@@ -363,7 +363,7 @@ int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
 #undef AXN_DGELU
   AXN_HIP_TRY(hipGetLastError());
   if (dbias != nullptr) {
-    hipLaunchKernelGGL(dbias_reduce_kernel, dim3((unsigned)((N + 63) / 64)),
+    hipLaunchKernelGGL(dbias_reduce_kernel, grid_of((N + 63) / 64),
                        dim3(256), 0, stream, partial, dbias, bands, N, beta);
     AXN_HIP_TRY(hipGetLastError());
   }
@@ -381,7 +381,7 @@ struct __attribute__((packed, aligned(2))) Any8 {
 __global__ void __launch_bounds__(256)
     pad_rows16_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int64_t M, int64_t N,
                       int64_t ld, int64_t per_row) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t idx = block_number() * 256 + threadIdx.x;
   if (idx >= M * per_row) return;
   const int64_t row = idx / per_row, col = (idx - row * per_row) * 8;   // per_row groups of 8 in a padded row
   const uint16_t* from = src + row * ld + col;
@@ -402,11 +402,11 @@ __global__ void __launch_bounds__(256)
 int launch_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst,
                       hipStream_t stream) {
   const int64_t per_row = ld_dst / 8, groups = (M * per_row + 255) / 256;
-  if (groups > 0x7fffffffLL) {
+  if (groups > 0x7fffffffLL - kMostBlocks) {
     set_error("pad_rows16: too many elements");
     return AXN_ELIMIT;
   }
-  hipLaunchKernelGGL(pad_rows16_kernel, dim3((unsigned)groups), dim3(256), 0, stream, (const uint16_t*)src,
+  hipLaunchKernelGGL(pad_rows16_kernel, grid_of(groups), dim3(256), 0, stream, (const uint16_t*)src,
                      (uint16_t*)dst, M, N, ld, per_row);
   AXN_HIP_TRY(hipGetLastError());
   return AXN_OK;

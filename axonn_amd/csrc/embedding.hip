@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK)
                          u32x4* __restrict__ out, int64_t T, int64_t V, int64_t pieces,
                          int64_t ldw, int64_t ldo, int units_per_row, int* status) {
   const int lane = threadIdx.x & 63;
-  const int64_t unit = (int64_t)blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
+  const int64_t unit = block_number() * WAVES_PER_BLOCK + (threadIdx.x >> 6);
   const int64_t t = unit / units_per_row;
   if (t >= T) return;
   const int64_t piece = (unit % units_per_row) * 64 + lane;
@@ -615,8 +615,9 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   // (units_per_row and long_blocks lie side by side and come with one load, not with a second one here)
-  if ((int)blockIdx.x < long_blocks) {
-    const int64_t unit = (int64_t)blockIdx.x * WAVES_PER_BLOCK + wave;
+  const int block = (int)block_number();   // (less than 2^31)
+  if (block < long_blocks) {
+    const int64_t unit = (int64_t)block * WAVES_PER_BLOCK + wave;
     const int64_t chunk = unit / pieces_per_row * 64;
     const int64_t col0 = (unit % pieces_per_row * 64 + lane) * LV;
     const int64_t j = chunk + lane;
@@ -656,7 +657,7 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
   // (a 64-bit division would be half of what a wave does for a row without tokens.  4 tokens, 146388 x 2240
   // bf16, beta: 55 us; 61 with the scalar unit's 64-bit quotient of the workgroup's first unit and a loop over its
   // other units)
-  const int64_t unit0 = (int64_t)((int)blockIdx.x - long_blocks) * WAVES_PER_BLOCK;
+  const int64_t unit0 = (int64_t)(block - long_blocks) * WAVES_PER_BLOCK;
   int64_t row = unit0 + (int)(threadIdx.x >> 6);
   int rest = 0;
   if (units_per_row != 1) {   // (rows of up to 1024 fp32 or 2048 16-bit elements need no division)
@@ -710,7 +711,7 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK)
     embedding_renorm_kernel(const int* __restrict__ row_start, TW* W, int64_t V, int64_t H,
                             int64_t ldw, float max_norm, float norm_type) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
+  const int64_t row = block_number() * WAVES_PER_BLOCK + (threadIdx.x >> 6);
   if (row >= V) return;
   if (row_start[row] < 0) return;
   constexpr int N = Vec<TW>::N;
@@ -887,11 +888,11 @@ int launch_embedding_fwd(const int64_t* ids, const void* W, void* out, int elem_
   const int upr = (int)((pieces + 63) / 64);
   const int64_t blocks = (T * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
   if (blocks == 0) return AXN_OK;
-  if (blocks >= (1LL << 31)) {
+  if (blocks >= (1LL << 31) - kMostBlocks) {
     set_error("embedding_fwd: too many tokens x columns (%lld blocks)", (long long)blocks);
     return AXN_ELIMIT;
   }
-  hipLaunchKernelGGL(embedding_fwd_kernel, dim3((unsigned)blocks), dim3(64 * WAVES_PER_BLOCK), 0,
+  hipLaunchKernelGGL(embedding_fwd_kernel, grid_of(blocks), dim3(64 * WAVES_PER_BLOCK), 0,
                      stream, ids, (const u32x4*)W, (u32x4*)out, T, V, pieces, ldw / per_piece,
                      ldo / per_piece, upr, status);
   AXN_HIP_TRY(hipGetLastError());
@@ -923,14 +924,14 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
   const bool slots = T <= V / EMB_SLOT_ROWS && (beta != 0 || clears);
   const int64_t blocks = ((slots ? T : V) * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK + long_blocks;
   const size_t zero_bytes = slots && beta == 0 ? (size_t)V * (size_t)H * (dw_dtype == AXN_F32 ? 4 : 2) : 0;
-  if (blocks + (int64_t)(zero_bytes / (16 * FILL_THREADS)) >= (1LL << 31)) {
+  if (blocks >= (1LL << 31) - kMostBlocks) {
     set_error("embedding_bwd: too many rows x columns (%lld blocks)", (long long)blocks);
     return AXN_ELIMIT;
   }
   const int *keys = nullptr, *vals = nullptr;
   int rc = sort_token_positions(ids, T, V, w, &keys, &vals, stream, !slots, dW, zero_bytes);
   if (rc || blocks == 0) return rc;
-  const dim3 grid((unsigned)blocks), block(64 * WAVES_PER_BLOCK);
+  const dim3 grid = grid_of(blocks), block(64 * WAVES_PER_BLOCK);
 #define AXN_EMB_BWD_US(TY, TW, UU, SLOTS)                                                       \
   hipLaunchKernelGGL((embedding_bwd_kernel<TY, TW, UU, SLOTS>), grid, block, EMB_BWD_LDS, stream, keys, vals,    \
                      w.row_start, (const TY*)dY, (TW*)dW, T, V, H, lddy, lddw, padding_idx, upr, \
@@ -978,8 +979,7 @@ int launch_embedding_renorm(const int64_t* ids, void* W, int dtype, int64_t T, i
   const int *keys = nullptr, *vals = nullptr;
   int rc = sort_token_positions(ids, T, V, w, &keys, &vals, stream);
   if (rc) return rc;
-  const dim3 grid((unsigned)((V + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK)),
-      block(64 * WAVES_PER_BLOCK);
+  const dim3 grid = grid_of((V + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK), block(64 * WAVES_PER_BLOCK);
   if (dtype == AXN_F32)
     hipLaunchKernelGGL(embedding_renorm_kernel<float>, grid, block, 0, stream, w.row_start,
                        (float*)W, V, H, ldw, max_norm, norm_type);

@@ -206,6 +206,27 @@ def test_gradient_of_a_table_larger_than_one_launch_can_clear(T):
     torch.cuda.empty_cache()
 
 
+def test_launches_of_more_than_2_to_the_32_threads():
+    """A wave a token or a table row, 2^26 and more of them: what lies behind the first 2^26 is done, too."""
+    from axonn_amd import ops
+
+    many = (1 << 26) + 9
+    weight = torch.arange(40, device="cuda", dtype=torch.float32).view(10, 4)
+    ids = torch.arange(many, device="cuda") % 10
+    out = ops.embedding_fwd(ids, weight)
+    for rows, these in zip(out.split(1 << 24), ids.split(1 << 24)):   # (as a whole torch's lookup wraps)
+        assert torch.equal(rows, weight[these])
+    del ids, out
+    wide = torch.full((many, 8), 7.0, device="cuda")     # (room between the rows: row by row)
+    ids = torch.tensor([0, many - 1, many - 1], device="cuda")
+    ops.embedding_bwd(ids, torch.ones(3, 4, device="cuda"), many, out=wide[:, :4])
+    rows = wide[:, :4].sum(1)
+    assert rows[0] == 4 and rows[-1] == 8 and int(rows.count_nonzero()) == 2 and bool((wide[:, 4:] == 7).all())
+    ops.embedding_renorm_(wide[:, 4:], ids, 1.0)         # rows of norm 14
+    norms = wide[:, 4:].norm(dim=1)
+    assert abs(float(norms[-1]) - 1) < 1e-5 and abs(float(norms[0]) - 1) < 1e-5 and bool((norms[1:-1] == 14).all())
+
+
 def test_backward_padding_row_repeated_ids_and_determinism():
     """A tenth of the tokens name one row, another tenth the padding row; the sum of 400
     terms depends on its order, and the kernel's order is the token order."""

@@ -190,6 +190,24 @@ def test_dgelu_dbias_adds_in_the_order_of_its_bands(M, N, dtype):
     assert torch.equal(inplace, dz) and torch.equal(db2, db) and bool(torch.isnan(ws[-8:]).all())
 
 
+@pytest.mark.parametrize("dtype,N", [(torch.bfloat16, (1 << 29) + 24), (torch.float32, (1 << 30) + 24)])
+def test_dgelu_dbias_over_more_columns_than_a_grid_has_threads(dtype, N):
+    """One row, so the sums are the row itself."""
+    from axonn_amd import ops
+
+    dY = torch.zeros(1, N, device="cuda", dtype=dtype)
+    at = torch.tensor([0, 1000, N // 2 + 3, N - 25, N - 24, N - 1], device="cuda")
+    dY[0, at] = torch.arange(1.0, 7.0, device="cuda", dtype=dtype)
+    _, db = ops.dgelu_dbias(dY)
+    assert torch.equal(db[at], dY[0, at].float()) and int(db.count_nonzero()) == 6
+    del db
+    if dtype == torch.bfloat16:
+        dz, db = ops.dgelu_dbias(dY, torch.ones_like(dY))
+        few, _ = ops.dgelu_dbias(dY[:, at].repeat(8, 4), torch.ones(8, 24, device="cuda", dtype=dtype))
+        assert torch.equal(dz[0, at], few[0, :6]) and int(dz.count_nonzero()) == 6
+        assert torch.equal(db[at], few[0, :6].float())
+
+
 def test_dgelu_dbias_matches_oracle():
     from axonn_amd import ops
 

@@ -227,6 +227,36 @@ def test_launches_of_more_than_2_to_the_32_threads():
     assert abs(float(norms[-1]) - 1) < 1e-5 and abs(float(norms[0]) - 1) < 1e-5 and bool((norms[1:-1] == 14).all())
 
 
+@pytest.mark.parametrize("offset", [0, 1, 7, 8])
+@pytest.mark.parametrize("T,V,H", [(1, 2, 4), (2, 5, 12), (1, 3, 72), (3, 77, 36), (0, 40, 8), (5, 1001, 84), (700, 2100, 260)])
+def test_a_gradient_anywhere_in_memory_is_cleared_and_nothing_around_it(T, V, H, offset):
+    """The sort's launches share the clearing; their shares end on lines of memory, wherever the table starts."""
+    from axonn_amd import ops
+
+    full = torch.full((V * H + 72,), 7.0, device="cuda")
+    out = full[4 * offset:4 * offset + V * H].view(V, H)
+    ids = (torch.arange(T, device="cuda") * 13) % V
+    dy = torch.randn(T, H, device="cuda")
+    ops.embedding_bwd(ids, dy, V, out=out)
+    want = torch.zeros(V, H, device="cuda", dtype=torch.float64).index_add_(0, ids, dy.double())
+    assert float((out.double() - want).abs().max()) <= 1e-5
+    assert bool((full[:4 * offset] == 7).all()) and bool((full[4 * offset + V * H:] == 7).all())
+
+
+def test_shares_of_the_clearing_start_on_lines():
+    """11 x 3 x 256 + 3 pieces of 16 bytes in three launches: even shares would start the second launch's 16 bytes
+    behind a line and take a workgroup for one piece."""
+    from launches import launches
+
+    from axonn_amd import ops
+
+    V, H = 2817, 12   # 3 pieces a row
+    ids, dy, out = torch.tensor([5], device="cuda"), torch.ones(1, H, device="cuda"), torch.empty(V, H, device="cuda")
+    grids = dict(launches(lambda: ops.embedding_bwd(ids, dy, V, out=out)))
+    prepare = [n for name, n in grids.items() if "prepare" in name]
+    assert prepare == [3 + 11]   # three workgroups for the sort's own tables, 2816 of the 2817 pieces
+
+
 def test_backward_padding_row_repeated_ids_and_determinism():
     """A tenth of the tokens name one row, another tenth the padding row; the sum of 400
     terms depends on its order, and the kernel's order is the token order."""

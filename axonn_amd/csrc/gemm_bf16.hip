@@ -191,8 +191,11 @@ EdgeTile edge_tile(long long M, long long N, long long Kc, const EpilogueTime& e
 
 // Outputs made of whole 128 x 128 tiles but not of larger ones: whether the small tile without bounds is ahead
 // of the larger ones with them.  Two workgroups share a CU and do not run in rounds, so its time grows
-// evenly with their number.  Larger tiles have to be estimated 5 % faster, beyond one round of them, where the
-// power cap stretches the estimate, 20 %.  us, small tile / larger ones, of M x N, contraction:
+// evenly with their number.  Larger tiles have to be estimated 8 % faster, beyond one round of them, where the
+// power cap stretches the estimate, 27 % (of 277 problems drawn those between 20 and 26 % took 1.01 of the small tile's
+// time on average, up to 1.14; the ones beyond either line 0.92 and 0.90).  They do not add to the output: reading it in
+// tiles that reach past its edge costs more than they gain (91 of them 1.01 on average, up to 1.22: 640 x
+// 7040 x 6528 91 / 110).  us, small tile / larger ones, of M x N, contraction:
 //   2048 x 50304, 2048  442 / 363      8192 x 5504, 2048  149 / 134   2048 x 5504, 8192 (weight gradient)  163 / 139
 //   4096 x 50304, 768   398 / 298      4096 x 3200, 3200   83 / 67    3200 x 10240, 2560 (input gradient)  143 / 158
 //   896 x 14336, 4096    99 / 82       8192 x 1920, 1920   52 / 46    2176 x 4096, 4096, GELU               83 / 87
@@ -202,7 +205,7 @@ bool small_tile_ahead(long long M, long long N, long long Kc, const EpilogueTime
   const double small = w <= 256 ? alone : w <= 512 ? alone + (shared - alone) * (w - 256) / 256 : shared * w / 512;
   double large = 0;
   if (edge_tile(M, N, Kc, epilogue, &large) == EDGE_128x128) return true;
-  return small < large * (ceil_div(M, 256) * ceil_div(N, 256) <= 256 ? 1.05 : 1.2);
+  return small < large * (ceil_div(M, 256) * ceil_div(N, 256) <= 256 ? 1.08 : 1.27);
 }
 
 int launch_edge(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, bool half,
@@ -219,8 +222,9 @@ int launch_edge(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32
 // Kernel selection.  Problems made of whole 256 x 256 tiles, more than 128 of
 // them (half of the CUs) and not just above one round of 256, take the
 // one-wave-per-SIMD kernel at that tile size, 65..128 of them take it at 256 x 128;
-// other problems made of whole 128 x 128 tiles take it at 128 x 128; ragged
-// shapes, and operands too large for 32-bit byte offsets, take the kernels of gemm_edge.h.
+// other problems made of whole 128 x 128 tiles take it at 128 x 128, or the larger tiles of
+// gemm_edge.h where small_tile_ahead says so; ragged shapes, and operands too large for 32-bit
+// byte offsets, take the kernels of gemm_edge.h.
 template <bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
 int launch_whole(const GemmArgs& g, hipStream_t stream) {
   const bool deep = g.Kc % 64 == 0;
@@ -246,7 +250,7 @@ int launch_whole(const GemmArgs& g, hipStream_t stream) {
   if (small_spans && whole128 && tiles128 < (1LL << 31)) {
     bool small_tile = true;
     if constexpr (EPI != EPI_PAIR)
-      small_tile = whole256 || small_tile_ahead(g.M, g.N, g.Kc, epilogue_time(g, EPI, OUT_F32));
+      small_tile = whole256 || g.beta || small_tile_ahead(g.M, g.N, g.Kc, epilogue_time(g, EPI, OUT_F32));
     if (small_tile) return launch_solo<128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
   }
   if constexpr (EPI == EPI_PAIR) {

@@ -354,3 +354,22 @@ def test_both_gradients_in_one_launch_with_the_contraction_in_parts(M, N, K, bet
 def test_both_gradients_in_one_launch_of_whole_tiles(M, N, K, beta, dw_f32, dtype):
     """Against the kernels without bounds that the two calls take here."""
     test_both_gradients_in_one_launch_with_the_contraction_in_parts(M, N, K, beta, dw_f32, dtype)
+
+
+@pytest.mark.parametrize("op,rows,cols,kc,beta,edge", [
+    (2, 7040, 6528, 640, 1, False), (2, 3584, 4224, 384, 1, False), (2, 7040, 6528, 640, 0, False),
+    (1, 6272, 7936, 1408, 0, False), (0, 7040, 4736, 3712, 0, False), (2, 2944, 2688, 768, 0, False),
+    (0, 896, 14336, 4096, 0, True), (0, 8192, 5504, 2048, 0, True), (2, 2048, 5504, 8192, 0, True),
+    (2, 2048, 5504, 8192, 1, False),
+])
+def test_the_tile_of_outputs_of_whole_small_tiles(op, rows, cols, kc, beta, edge):
+    """Larger tiles with bounds where they are measured faster: clearly estimated so, and never to add to dW."""
+    from launches import launches
+
+    M, N, K = {0: (rows, cols, kc), 1: (rows, kc, cols), 2: (kc, rows, cols)}[op]
+    a, b = {0: ((M, K), (N, K)), 1: ((M, N), (N, K)), 2: ((M, N), (M, K))}[op]
+    a, b = torch.zeros(a, device="cuda").bfloat16(), torch.zeros(b, device="cuda").bfloat16()
+    c = torch.zeros(rows, cols, device="cuda").bfloat16()
+    call = lambda: nv.call("axn_gemm_any_n", op, nv.ptr(a), nv.ptr(b), None, nv.ptr(c), None, nv.BF16, M, N, K,   # noqa: E731
+                           a.shape[1], b.shape[1], cols, nv.EPI_NONE, beta, nv.BF16, None, 0, nv.current_stream())
+    assert ["edge" in name for name, _ in launches(call)][0] == edge

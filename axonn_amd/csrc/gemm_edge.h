@@ -38,9 +38,11 @@ __global__ void __launch_bounds__(256) gemm_edge_backward_kernel(const GemmArgs 
 template <int BM, int BN, bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF, bool ODD = false>
 int launch_edge_tile(const GemmArgs& in, hipStream_t stream) {
   // Only the forward's output rows can be odd (the others have the width of an input); those of heads over
-  // vocabularies are, which have neither bias nor activation.
+  // vocabularies are, which have neither bias nor activation.  Up to 80 rows, few of a tile, the exchange costs what
+  // the stores gain (us, plain / so: 78 x 1013, 448 6.6 / 7.3, 70 x 688, 1192 10.4 / 11.0; 65 to 80 rows 1.02 of the
+  // time on average up to contractions of 1200 and 1.00 beyond, 81 to 96 rows 1.00, 113 to 128 0.94).
   if constexpr (!ODD && AK && BKM && EPI == AXN_EPI_NONE && !OUT_F32)
-    if (in.ldc % 2 != 0 && !in.beta) return launch_edge_tile<BM, BN, AK, BKM, EPI, OUT_F32, HALF, true>(in, stream);
+    if (in.ldc % 2 != 0 && !in.beta && in.M > 80) return launch_edge_tile<BM, BN, AK, BKM, EPI, OUT_F32, HALF, true>(in, stream);
   GemmArgs g = in;
   g.tiles_m = (int)ceil_div(g.M, BM);
   g.tiles_n = (int)ceil_div(g.N, BN);

@@ -190,3 +190,24 @@ def test_wide_rows_are_padded_to_whole_lines(M, N, ld):
     for got, want in ((dx, src.double() @ w.double()), (dw, src.double().t() @ x.double())):
         # bf16 rounding of the result and fp32 sums
         assert float((got.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("M,N,K,odd", [(70, 689, 1192, False), (80, 1013, 448, False), (81, 1013, 448, True),
+                                       (300, 50257, 64, True)])
+def test_rows_from_which_odd_strides_take_the_exchange(M, N, K, odd):
+    from launches import launches
+
+    X, W = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
+    out, even = torch.empty(M, N, device="cuda").bfloat16(), torch.empty(M, N + 1, device="cuda").bfloat16()
+
+    def call(to):
+        nv.call("axn_gemm_any_n", 0, nv.ptr(X), nv.ptr(W), None, nv.ptr(to), None, nv.BF16, M, N, K, K, K, to.shape[1],
+                nv.EPI_NONE, 0, nv.BF16, None, 0, nv.current_stream())
+
+    def kernels(to):
+        return [name for name, _ in launches(lambda: call(to))]
+
+    assert (kernels(out) != kernels(even)) == odd
+    call(out)
+    call(even)
+    assert torch.equal(out, even[:, :N])

@@ -89,8 +89,9 @@ def _padded_width(N):
     beyond 30000).  Rows of 1000 to 4000 gain 0 to 3 % on the GPU and lose 3 us of host time to the view
     without the padding (700 x 1501 x 2048 29.5 -> 32.9 us).  Strides 1/128 or 1/256 beyond a power of two are left out:
     the rows of a tile crowd onto few memory channels (both gradients of 2048 x 33001 x 2048 with rows of 33024 elements
-    542 us, of 33088 487; 2048 x 32885 x 2048, 32896 585, 32960 486; 2048 x 16453 x 768, 16512 164, 16576 145)."""
-    if N < 4096:
+    542 us, of 33088 487; 2048 x 32885 x 2048, 32896 585, 32960 486; 2048 x 16453 x 768, 16512 164, 16576 145).
+    Near _FAR_ROWS and beyond, rows have nothing between them: `_prep_bf16` would pack them again for each product."""
+    if N < 4096 or N > _FAR_ROWS - 256:
         return N + (-N) % 8
     ld = N + (-N) % 64
     power = 1 << (ld.bit_length() - 1)

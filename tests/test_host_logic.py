@@ -329,3 +329,15 @@ def test_padded_rows_start_on_lines_and_off_the_crowded_strides():
         assert N <= ld < N + (256 if N >= 4096 else 8) and ld % (64 if N >= 4096 else 8) == 0
     assert [ops._padded_width(n) for n in (8250, 16440, 16500, 32890, 33001, 50257)] == [8320, 16576, 16576, 32960,
                                                                                           33088, 50304]
+
+
+def test_padded_rows_as_long_as_far_rows_are_not_packed_again(monkeypatch):
+    """A row stride beyond `_FAR_ROWS` that has a gap is packed by `_prep_bf16`: what `_pad_rows` makes has none."""
+    from axonn_amd import ops
+
+    monkeypatch.setattr(ops, "_FAR_ROWS", 1 << 13)
+    for N in [4097, 7935, 7937, 8121, 8129, 8185, 8191, 8193, 8255, 16385, 33001]:
+        ld, n8 = ops._padded_width(N), N + (-N) % 8
+        dy8 = torch.zeros(2, ld).bfloat16()[:, :n8]
+        at, stride = ops._prep_bf16(dy8)
+        assert at.data_ptr() == dy8.data_ptr() and stride == ld

@@ -241,7 +241,7 @@ int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
                        float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
                        void* ws, size_t ws_bytes, hipStream_t stream);
 
-// dst[M][8 ceil(N / 8)] = src[M][N] (row stride ld) of 16-bit elements, zeros behind N.
+// dst[M][ld_dst] = src[M][N] (row stride ld) of 16-bit elements, zeros behind N; ld_dst a multiple of 8.
 int launch_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst,
                       hipStream_t stream);
 

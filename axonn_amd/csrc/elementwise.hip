@@ -101,23 +101,37 @@ __device__ __forceinline__ _Float16 product_f16(float d, _Float16 g) {
 // phase p adds rows p, p + 4, p + 8, ... one after the other, the four phases are added in pairs.  Two LDS buffers: the
 // barrier behind the next rows is the one that frees these.
 //
-// Bound by memory: 252 MB of bf16 8192 x 5120 and their sums in 52 us from HBM (4.9 TB/s), 42 where the memory-side
+// Bound by memory: 252 MB of bf16 8192 x 5120 and their sums in 50 us from HBM (5.0 TB/s), 41 where the memory-side
 // cache holds the operands.  The order of the sums is that of one workgroup of 256 threads walking 512 columns of a
 // band row by row, which had 64 to 500 rows on 8 to 32 CUs; bands dealt out in chunks of 16 rows balance too,
 // but add in another order, up to 1.6 times as far from 64 bits.  us with the sums, (HBM | cache), walk row by row,
 // chunks, so:
-//   bf16 8192 x 5120 62 | 51, 52 | 45, 52 | 42    2048 x 4096 22 | 21, 17 | 15, 16 | 13    256 x 4096 18, 8, 8
-//   bf16 8192 x 14336 154, 137, 138               2900 x 6144 36 | 33, 26 | 23, 28 | 23    3001 x 10240 43 | 37, 41 | 34, 41 | 34
-//   fp32 8192 x 5120 110, 101, 101                2900 x 6144 64 | 46, 44 | 36, 48 | 38    5000 x 8192 112, 96, 88
-//   sums alone, bf16 8192 x 5120 22, 18, 19       2900 x 6144 12.5, 11.8, 12.7             fp32 2900 x 6144 19.7, 15.9, 19.0
+//   bf16 8192 x 5120 62 | 51, 53 | 45, 50 | 41    2048 x 4096 22 | 21, 17 | 14, 15 | 14    256 x 4096 18, 7, 7
+//   bf16 8192 x 14336 155, 135, 126               2900 x 6144 36 | 33, 26 | 23, 27 | 23    3001 x 10240 43 | 37, 40 | 34, 39 | 33
+//   fp32 8192 x 5120 110, 101, 99                 2900 x 6144 64 | 46, 44 | 36, 48 | 37    5000 x 8192 108, 95, 87
+//   sums alone, bf16 8192 x 5120 22, 18, 19       2900 x 6144 13.0, 12.4, 13.5             fp32 2900 x 6144 19.5, 15.8, 18.9
 // 1024 threads are ahead of 512 by 2 % on 16-bit dGELU and behind by 3 to 8 % on fp32 and on sums alone (bf16 8192 x
-// 5120 18.7 us, with 1024 19.6); 64 columns or 256, and the loads of the next rows ahead of the stores were no faster.
+// 5120 18.7 us, with 1024 19.6); 64 columns or 256 (fp32: 5 % slower), the loads of the next rows ahead of the stores and
+// those of the whole band ahead of the first sums (2 to 5 % slower) were no faster.
 // Non-temporal loads of dY and Z (bf16 8192 x 5120) are 10 % faster from HBM (47 us) and 12 % slower from the
 // cache (47), which holds dY in a training step (the layer behind wrote it a moment ago): plain ones.
 // Every thread has read its piece before it stores it, so dZ may alias dY.
 constexpr int DG_BAND = 128, DG_COLS = 128, DG_PIECES = DG_COLS / 8;
 template <typename T, bool HAS_Z>
 constexpr int DG_THREADS = HAS_Z && sizeof(T) == 2 ? 1024 : 512;
+
+// The workgroup's 128 columns.  Workgroups go to the 8 XCDs in turn, each with an L2 of its own: one XCD takes columns
+// side by side, so that a 128-byte line that two of them share is read, and written, by one L2 (rows that do not
+// start on lines share one line in three of 16-bit types).  fp32 (TURN): other columns in the next band, because
+// 512 bytes of rows 4096 (32768) bytes apart lie in two of the 16 channels of an L2.  us in launch order, side by side,
+// turned:   bf16 8192 x 5896 64, 54, 57   12000 x 8200 151, 117, 121   sums alone 8192 x 14344 49, 37, 42
+//           fp32 16384 x 1024 44, 44, 34  4096 x 3048 34, 29, 27       sums alone 3000 x 8192 19, 23, 19
+template <bool TURN>
+__device__ __forceinline__ unsigned column_group() {
+  const unsigned n = gridDim.x, xcd = blockIdx.x & 7, each = n >> 3;
+  const unsigned at = xcd * each + min(xcd, n & 7u) + (blockIdx.x >> 3);
+  return TURN ? (at + (blockIdx.y & 7) * max(each, 1u)) % n : at;
+}
 
 template <typename T, bool HAS_Z>
 __global__ void __launch_bounds__((DG_THREADS<T, HAS_Z>))
@@ -132,7 +146,8 @@ __global__ void __launch_bounds__((DG_THREADS<T, HAS_Z>))
   __shared__ float phases[4][DG_COLS];
   const int piece = threadIdx.x % DG_PIECES, row0 = threadIdx.x / DG_PIECES;
   const int c = threadIdx.x % DG_COLS, phase = threadIdx.x / DG_COLS;
-  const int64_t col0 = (blockIdx.z * kMostBlocks + blockIdx.x) * DG_COLS, band0 = (int64_t)blockIdx.y * DG_BAND;
+  const unsigned at = column_group<sizeof(T) == 4>();
+  const int64_t col0 = (blockIdx.z * kMostBlocks + at) * DG_COLS, band0 = (int64_t)blockIdx.y * DG_BAND;
   const int64_t col = col0 + piece * 8;
   float sum = 0.f;
 #pragma unroll

@@ -190,6 +190,22 @@ def test_dgelu_dbias_adds_in_the_order_of_its_bands(M, N, dtype):
     assert torch.equal(inplace, dz) and torch.equal(db2, db) and bool(torch.isnan(ws[-8:]).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_dgelu_dbias_takes_every_group_of_columns_in_every_band(dtype):
+    """Each number of 128-column groups modulo the 8 XCDs, more bands than XCDs."""
+    from axonn_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    dY = torch.randn(9 * 128 + 5, 25 * 128, generator=g, device="cuda").to(dtype)
+    Z = torch.randn(dY.shape, generator=g, device="cuda").to(dtype)
+    dz_all, db_all = ops.dgelu_dbias(dY, Z)
+    sums = sums_by_bands(dY.float())
+    for N in [8, 128, *range(136, 25 * 128, 128), 25 * 128]:
+        assert torch.equal(ops.dgelu_dbias(dY[:, :N])[1], sums[:N])
+        dz, db = ops.dgelu_dbias(dY[:, :N], Z[:, :N])
+        assert torch.equal(dz, dz_all[:, :N]) and torch.equal(db, db_all[:N])
+
+
 @pytest.mark.parametrize("dtype,N", [(torch.bfloat16, (1 << 29) + 24), (torch.float32, (1 << 30) + 24)])
 def test_dgelu_dbias_over_more_columns_than_a_grid_has_threads(dtype, N):
     """One row, so the sums are the row itself."""

@@ -568,6 +568,13 @@ __device__ __forceinline__ void store_part(const float (&x)[VEC], TW* dst, int b
 constexpr int64_t EMB_SLOT_ROWS = 2;
 // Rows named by more than EMB_LONG_RUN tokens get waves of their own (below).
 constexpr int EMB_LONG_RUN = 32;
+// Workgroups that are resident together (256 CUs, 4 each: EMB_BWD_LDS).  Where all do not fit and those of the other
+// rows take three quarters of the room at most, these start first: behind the long runs' they went where one
+// ended first, several to a CU, and the launch waited for them.  Elsewhere the long runs, the longest chains, do.
+// us, long runs first / so: 8192 tokens drawn evenly from 512 rows x 3640, fp32 into bf16 (256 and 928 workgroups) 75 / 44,
+// 16384 from 1024 x 1832 84 / 50, 8192 from 3000 x 1832 (750, 480) 39 / 35; as in a text 16384 from 512 x 3640 186 / 172; but
+// 2000 from 1024 x 3640 (1024, 456) 32 / 35.
+constexpr int64_t EMB_RESIDENT = 4 * 256;
 
 // The slots of `row` among the 64 from slot `first` on: their count, and this lane's position.
 __device__ __forceinline__ int run_in_chunk(const int* __restrict__ keys, const int* __restrict__ vals,
@@ -595,6 +602,8 @@ __device__ __forceinline__ int run_in_chunk(const int* __restrict__ keys, const 
 // tokens x 2048 fp32 whose ids fall off like those of a text, into 128256 rows: 1394 us with one
 // row in flight and every row on the same waves, 239 with pieces twice as wide and half as many rows in flight
 // (the most frequent row, a twelfth of the tokens, was the launch's longest chain), 203 us so and slot by slot.
+// (Twice as many waves that find no long run cost 1 to 6 % of tables with fewer than two rows a token whose ids
+// are drawn evenly, 30000 x 512 x 3640 108 -> 113 us; as in a text these take 0.72 to 0.90 of the time.)
 // What bounds it now is the store of the 1.05 GB gradient (147 us of 250 tokens, 153 us for a
 // plain fill) and the way of 134 MB of gradient rows behind it.
 //
@@ -607,17 +616,17 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
     embedding_bwd_kernel(const int* __restrict__ keys, const int* __restrict__ vals,
                          const int* __restrict__ row_start, const TY* __restrict__ dY, TW* dW,
                          int64_t T, int64_t V, int64_t H, int64_t lddy, int64_t lddw,
-                         int64_t padding_idx, int units_per_row, int long_blocks, int scale_by_freq,
+                         int64_t padding_idx, int units_per_row, int long_blocks, int long_at, int rows_at, int scale_by_freq,
                          int beta, int pieces_per_row) {
   constexpr int VEC = 16 / (int)sizeof(TW);
   constexpr int LV = VEC / 4;                                 // columns of a lane in a long run's wave
   constexpr int LONG_B = LV * (int)sizeof(TY) <= 4 ? 64 : 32; // its rows in flight: a chunk, or 64 registers
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  // (units_per_row and long_blocks lie side by side and come with one load, not with a second one here)
+  // (units_per_row and the block numbers lie side by side and come with one load, not with a second one here)
   const int block = (int)block_number();   // (less than 2^31)
-  if (block < long_blocks) {
-    const int64_t unit = (int64_t)block * WAVES_PER_BLOCK + wave;
+  if ((unsigned)(block - long_at) < (unsigned)long_blocks) {
+    const int64_t unit = (int64_t)(block - long_at) * WAVES_PER_BLOCK + wave;
     const int64_t chunk = unit / pieces_per_row * 64;
     const int64_t col0 = (unit % pieces_per_row * 64 + lane) * LV;
     const int64_t j = chunk + lane;
@@ -657,7 +666,7 @@ __global__ void __launch_bounds__(64 * WAVES_PER_BLOCK, 4)
   // (a 64-bit division would be half of what a wave does for a row without tokens.  4 tokens, 146388 x 2240
   // bf16, beta: 55 us; 61 with the scalar unit's 64-bit quotient of the workgroup's first unit and a loop over its
   // other units)
-  const int64_t unit0 = (int64_t)(block - long_blocks) * WAVES_PER_BLOCK;
+  const int64_t unit0 = (int64_t)(block - rows_at) * WAVES_PER_BLOCK;
   int64_t row = unit0 + (int)(threadIdx.x >> 6);
   int rest = 0;
   if (units_per_row != 1) {   // (rows of up to 1024 fp32 or 2048 16-bit elements need no division)
@@ -929,7 +938,9 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
   const int64_t clearing = 1 + (T > 0 ? plan_sort(T, V).passes : 0);
   const bool clears = lddw == H && V * (H / vec) / clearing < 0xd0000000LL;
   const bool slots = T <= V / EMB_SLOT_ROWS && (beta != 0 || clears);
-  const int64_t blocks = ((slots ? T : V) * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK + long_blocks;
+  const int64_t row_blocks = ((slots ? T : V) * upr + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+  const int64_t blocks = row_blocks + long_blocks;
+  const bool rows_first = row_blocks <= EMB_RESIDENT * 3 / 4 && blocks > EMB_RESIDENT;
   const size_t zero_bytes = slots && beta == 0 ? (size_t)V * (size_t)H * (dw_dtype == AXN_F32 ? 4 : 2) : 0;
   if (blocks >= (1LL << 31) - kMostBlocks) {
     set_error("embedding_bwd: too many rows x columns (%lld blocks)", (long long)blocks);
@@ -942,7 +953,8 @@ int launch_embedding_bwd(const int64_t* ids, const void* dY, void* dW, int dy_dt
 #define AXN_EMB_BWD_US(TY, TW, UU, SLOTS)                                                       \
   hipLaunchKernelGGL((embedding_bwd_kernel<TY, TW, UU, SLOTS>), grid, block, EMB_BWD_LDS, stream, keys, vals,    \
                      w.row_start, (const TY*)dY, (TW*)dW, T, V, H, lddy, lddw, padding_idx, upr, \
-                     (int)long_blocks, scale_by_freq, beta, (int)long_pieces)
+                     (int)long_blocks, rows_first ? (int)row_blocks : 0, rows_first ? 0 : (int)long_blocks, \
+                     scale_by_freq, beta, (int)long_pieces)
 #define AXN_EMB_BWD_U(TY, TW, UU)           \
   do {                                      \
     if (slots)                              \

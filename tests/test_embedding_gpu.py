@@ -187,6 +187,24 @@ def test_backward_on_either_side_of_two_table_rows_a_token(dtype, T, V, H):
     assert np.array_equal(host(out), twice)
 
 
+@pytest.mark.parametrize("V", [1100, 1121, 1536, 1537])
+def test_backward_whichever_rows_start_first(V):
+    """464 workgroups for long runs and 550 to 769 for the other rows: within a round of 1024, and either side of 768."""
+    from axonn_amd import ops
+
+    T, H = 4096, 1832
+    g = torch.Generator(device="cuda").manual_seed(V)
+    ids = torch.randint(0, V, (T,), device="cuda", generator=g)
+    ids[torch.randperm(T, device="cuda", generator=g)[:300]] = V - 1
+    ids[::50] = 3
+    dy = torch.randn(T, H, device="cuda", generator=g)
+    dW = ops.embedding_bwd(ids, dy, V, padding_idx=7)
+    want = oe.embedding_backward(ids.cpu().numpy(), host(dy), V, padding_idx=7)
+    assert np.array_equal(host(dW), want)
+    dW = ops.embedding_bwd(ids, dy, V, padding_idx=7, out=dW, accumulate=True)
+    assert np.allclose(host(dW), 2 * want, rtol=1e-6, atol=0)
+
+
 @pytest.mark.parametrize("T", [0, 1])
 def test_gradient_of_a_table_larger_than_one_launch_can_clear(T):
     """68.7 GB and more of a gradient without tokens: 2^32 pieces of 16 bytes, and as many threads, are one too many."""

@@ -719,7 +719,8 @@ double filled(long long n1, double s1, long long n2, double s2) {
 // a stage of a time that lies between the work's average over the CUs and that of the fullest one (0.3 to 0.7), a
 // tile counting 3 stages more than it has, 6 where it reads dW to add to it, and the parts' cost; fitted to 65
 // problems of 64 to 3564 tokens with 2 to 16 parts each (7 % rms).  The two launches, whose estimate is 8 % low, and
-// 20 % beyond 100 us, where the power cap stretches it, have to be slower.  Up to 192 rows a weight gradient
+// 15 % beyond 100 us, where the power cap stretches it, have to be slower (up to 20 %: of 1100 problems drawn 243
+// more in one launch, 0.98 of the time of two, a twelfth of them 3 to 15 % slower).  Up to 192 rows a weight gradient
 // is nearly all stores, and two launches are as fast (151 x 11392 x 4992: 75 us, 79 in one).
 // Where that estimate is not enough, from 758 problems that it takes (481 of whole 128 x 128 x 64 tiles, whose two
 // launches have kernels without bounds; us, two launches / one):
@@ -729,8 +730,8 @@ double filled(long long n1, double s1, long long n2, double s2) {
 //                                                                                         512 x 11008 x 8192 186 / 196
 //   adding to dW in tiles that reach past its edge where those of two launches do not      256 x 18560 x 5632 209 / 236
 //   adding to more than 256 tiles of dW from at most 256 rows with bounds                  237 x 13312 x 5376 154 / 180
-// Of 284 problems drawn anew that it then takes (121 whole), one launch has 0.90 of the time of two on average, seven
-// take 2 to 5 % longer.
+// Of 857 problems drawn anew that it then takes, one launch has 0.88 of the time of two on average, 13 take 3 to 13 %
+// longer (3223 x 11176 x 1920, fp32 dW, 257 / 285; 512 x 5632 x 3328 64 / 69).
 int gemm_backward_parts(int64_t M, int64_t N, int64_t K, bool add) {
   if (M <= 192) return 0;
   double apart_d = 0, apart_w = 0;
@@ -748,7 +749,7 @@ int gemm_backward_parts(int64_t M, int64_t N, int64_t K, bool add) {
   const double average = ((double)td * d + (double)tw * w) / 256;
   const double us = 2.2 + 1.45 * (0.7 * fullest + 0.3 * average) + kPartsMicroseconds + parts * part_microseconds(M, K);
   const double apart = apart_d + apart_w;
-  return us < apart * (apart < 100 ? 1.08 : whole && td > 200 ? 1.1 : 1.2) ? parts : 0;
+  return us < apart * (apart < 100 ? 1.08 : whole && td > 200 ? 1.1 : 1.15) ? parts : 0;
 }
 
 int launch_gemm_backward_parts(const GemmArgs& dgrad, const GemmArgs& wgrad, bool half, bool dw_f32, int parts,

@@ -217,6 +217,8 @@ def test_gate_up_forward_argument_errors():
     (512, 11008, 8192, 0, False), (1024, 32000, 3584, 0, False), (1280, 15360, 2304, 0, True),
     (256, 18560, 5632, 1, False), (512, 13312, 3712, 1, False), (249, 25472, 4864, 1, False), (237, 13312, 5376, 1, False),
     (256, 14336, 4096, 0, True), (1376, 9088, 2112, 0, True), (649, 4032, 2176, 1, True), (1024, 6144, 4096, 0, True),
+    (2100, 7424, 1536, 1, False), (3136, 11392, 1152, 0, False), (2688, 11203, 768, 0, False), (2944, 13824, 2048, 0, False),
+    (2624, 12189, 512, 0, True), (3584, 8707, 1024, 1, True),
 ])
 def test_sizes_whose_gradients_take_one_launch(M, N, K, beta, joint):
     parts = nv.load().axn_gemm_bwd_workspace_bytes(M, N, K, beta) // (M * K * 4)

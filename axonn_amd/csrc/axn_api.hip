@@ -342,6 +342,7 @@ static int gemm_ws(const char* name, int op, const void* a, const void* b, void*
     REQUIRE(given || !refused || workspace_bytes >= need, AXN_EINVAL,
             "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
     REQUIRE(given || !refused, AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
+    if (given) plan = gemm_plan(layout, g.M, g.N, g.Kc);
   }
   if (plan.parts > 1)
     return launch_gemm_splitk(layout, g, epilogue, half, out_dtype == AXN_F32, plan, (float*)workspace,
@@ -393,7 +394,9 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void*
     REQUIRE(workspace_bytes >= need, AXN_EINVAL,
             "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
     REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
-    return launch_gemm_splitk(layout, g, epilogue, half, out_f32, plan, (float*)workspace, (hipStream_t)stream);
+    plan = gemm_plan(layout, g.M, g.N, g.Kc);
+    if (plan.parts > 1)
+      return launch_gemm_splitk(layout, g, epilogue, half, out_f32, plan, (float*)workspace, (hipStream_t)stream);
   }
   return half ? launch_gemm_f16(layout, g, epilogue, out_f32, (hipStream_t)stream)
               : launch_gemm_bf16(layout, g, epilogue, out_f32, (hipStream_t)stream);

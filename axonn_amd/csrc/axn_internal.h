@@ -163,7 +163,11 @@ int launch_gemm_backward(const GemmArgs& dgrad, const GemmArgs& wgrad, bool half
 // GEMMs of shapes that are not made of whole tiles (gemm_edge.h), on the tile the caller
 // picks: any M, N, contraction and operand size, row strides below kEdgeMaxLd elements (half
 // of that on the tiles of 256 rows).
-enum EdgeTile { EDGE_256x256 = 0, EDGE_256x128 = 1, EDGE_128x128 = 2 };
+// FED_*: tiles of gemm_fed_tiles.h, one workgroup on a CU.
+enum EdgeTile {
+  EDGE_256x256 = 0, EDGE_256x128 = 1, EDGE_128x128 = 2,
+  FED_64x64, FED_96x64, FED_64x128, FED_96x128, FED_128x128, FED_96x192, FED_128x192, FED_160x192, FED_128x256
+};
 constexpr int64_t kEdgeMaxLd = 1LL << 23;
 // Split contraction for problems with few output tiles: into how many parts and on which
 // tile (parts = 1: do not split), and the launch: partial products in fp32 to `ws`
@@ -174,6 +178,9 @@ struct SplitPlan {
   EdgeTile tile;
 };
 SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, double* us = nullptr);
+// What a call with the workspace for gemm_splits' parts does: those parts on the tile that is estimated to be fastest,
+// or the contraction in one part where a smaller tile is faster still.
+SplitPlan gemm_plan(GemmLayout layout, int64_t M, int64_t N, int64_t Kc);
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, int epilogue, bool half, bool out_f32,
                        const SplitPlan& plan, float* ws, hipStream_t stream);
 // The parts of the input gradient's contraction if both gradients of a layer (dY[M][N], W[N][K], X[M][K]) are
@@ -188,6 +195,11 @@ int launch_gemm_edge_bf16(GemmLayout layout, const GemmArgs& args, int epilogue,
                           EdgeTile tile, hipStream_t stream);
 int launch_gemm_edge_f16(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32,
                          EdgeTile tile, hipStream_t stream);
+// The same on a FED_* tile; row strides below kEdgeMaxLd / 2.
+int launch_gemm_fed_nt_bf16(const GemmArgs& args, int epilogue, bool out_f32, EdgeTile tile, hipStream_t stream);
+int launch_gemm_fed_nt_f16(const GemmArgs& args, int epilogue, bool out_f32, EdgeTile tile, hipStream_t stream);
+int launch_gemm_fed_nn_tn_bf16(GemmLayout layout, const GemmArgs& args, bool out_f32, EdgeTile tile, hipStream_t stream);
+int launch_gemm_fed_nn_tn_f16(GemmLayout layout, const GemmArgs& args, bool out_f32, EdgeTile tile, hipStream_t stream);
 // Both gradients of a layer in one launch of 256 x 256 tiles; tiles_m, tiles_n and wg_first set.
 int launch_gemm_edge_backward_bf16(const GemmArgs& wgrad, const GemmArgs& dgrad, bool dw_f32,
                                    hipStream_t stream);

@@ -18,8 +18,7 @@
 //     works on a compact block of neighbouring tiles.
 //
 // One-wave-per-SIMD kernels (solo_gemm: gemm_*_solo_kernel at 256 x 256 and 128 x 128
-// tiles, gemm_*_rest_kernel at 256 x 128, gemm_*_swiglu_kernel; shapes made of whole
-// tiles, contraction % 64 == 0, operands below 2 GiB): 4 waves, one per SIMD, each a
+// tiles, gemm_*_swiglu_kernel; shapes made of whole tiles, contraction % 64 == 0, operands below 2 GiB): 4 waves, one per SIMD, each a
 // quarter of the tile on v_mfma_f32_16x16x32_{bf16,f16}; operand tiles go global -> LDS
 // directly (buffer loads to LDS, 16 bytes per lane, no registers) into a ring of five
 // 64-deep tiles; each wave pipelines its share of the copies and its LDS fragment reads
@@ -31,6 +30,10 @@
 // gate/up forward of a gated MLP gathers its column operand from two weight matrices
 // and applies silu(gate) * up in the epilogue.
 //
+// Kernels with copying waves of their own (fed_gemm: gemm_*_rest_kernel at 256 x 128, and the tiles of
+// gemm_fed_tiles.h): rests, and outputs that small tiles cover in one round of workgroups or two, of any shape
+// (fed_tile, gemm_plan).
+//
 // Everything else (ragged shapes, contractions that are not multiples of 64, operands of
 // 2 GiB and more) runs on the same main loop with bounds: gemm_edge.h.
 #include <atomic>
@@ -39,7 +42,7 @@
 #include <queue>
 #include <vector>
 
-#include "gemm_solo.h"
+#include "gemm_fed.h"
 
 namespace axn {
 namespace {
@@ -54,12 +57,12 @@ __global__ void __launch_bounds__(256) gemm_f16_solo_kernel(const GemmArgs g) {
 }
 // The 256 x 128 tile of the launches that finish a problem.
 template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32>
-__global__ void __launch_bounds__(256) gemm_bf16_rest_kernel(const GemmArgs g) {
-  solo_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, false>(g);
+__global__ void __launch_bounds__(512) gemm_bf16_rest_kernel(const GemmArgs g) {
+  fed_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, false, false>(g);
 }
 template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32>
-__global__ void __launch_bounds__(256) gemm_f16_rest_kernel(const GemmArgs g) {
-  solo_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, true>(g);
+__global__ void __launch_bounds__(512) gemm_f16_rest_kernel(const GemmArgs g) {
+  fed_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, true, false>(g);
 }
 
 // Weight gradient and input gradient of one layer in one launch, 256 x 256 tiles: the
@@ -110,7 +113,7 @@ int launch_rest(const GemmArgs& in, hipStream_t stream) {
   GemmArgs g = in;
   g.tiles_m = g.M / 256;
   g.tiles_n = g.N / 128;
-  constexpr size_t lds = 5 * 256 * 64 * 2;  // five slots of the A tile's size
+  constexpr size_t lds = kFedLds<256, 128>;
   void (*kern)(const GemmArgs) = gemm_bf16_rest_kernel<AK, BKM, EPI, OUT_F32>;
   if constexpr (HALF) kern = gemm_f16_rest_kernel<AK, BKM, EPI, OUT_F32>;
   {
@@ -119,7 +122,7 @@ int launch_rest(const GemmArgs& in, hipStream_t stream) {
     if (rc != AXN_OK) return rc;
   }
   const int splits = g.splits > 1 ? g.splits : 1;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(g.tiles_m * g.tiles_n * splits)), dim3(256), lds, stream, g);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(g.tiles_m * g.tiles_n * splits)), dim3(512), lds, stream, g);
   AXN_HIP_TRY(hipGetLastError());
   return AXN_OK;
 }
@@ -208,6 +211,98 @@ bool small_tile_ahead(long long M, long long N, long long Kc, const EpilogueTime
   return small < large * (ceil_div(M, 256) * ceil_div(N, 256) <= 256 ? 1.08 : 1.27);
 }
 
+// ---- outputs of one round of small tiles, or two (gemm_fed_tiles.h) ------------------------
+struct FedTile {
+  EdgeTile tile;
+  int bm, bn;
+  // Estimated microseconds of a launch, for each operand order: a round of workgroups, a stage of it, a megabyte of
+  // operands (with a workgroup on every CU) and one of output.
+  float round[3], stage[3], operands[3], output[3];
+};
+// Fitted to 17288 launches on MI355X, cold operands: every tile, in 1 to 16 parts, of 1441 products of 1 to 8192 tokens
+// and 256 to 14336 features as training and inference have them; 8 to 14 % rms, but alike for a problem's tiles.
+constexpr FedTile kFedTiles[] = {
+    {FED_64x64, 64, 64, {1.29f, 2.08f, 2.13f}, {0.175f, 0.208f, 0.077f}, {0.140f, 0.073f, 0.719f}, {0.79f, 0.70f, 0.00f}},
+    {FED_96x64, 96, 64, {1.40f, 1.93f, 2.99f}, {0.276f, 0.295f, 0.270f}, {0.072f, 0.045f, 0.227f}, {0.65f, 0.63f, 0.05f}},
+    {FED_64x128, 64, 128, {1.52f, 2.06f, 3.15f}, {0.330f, 0.343f, 0.277f}, {0.073f, 0.047f, 0.208f}, {0.58f, 0.61f, 0.11f}},
+    {FED_96x128, 96, 128, {1.69f, 2.08f, 3.26f}, {0.400f, 0.417f, 0.371f}, {0.065f, 0.038f, 0.194f}, {0.51f, 0.56f, 0.14f}},
+    {FED_128x128, 128, 128, {1.93f, 2.39f, 3.55f}, {0.470f, 0.504f, 0.425f}, {0.058f, 0.024f, 0.147f}, {0.47f, 0.51f, 0.15f}},
+    {FED_96x192, 96, 192, {1.84f, 2.10f, 3.74f}, {0.512f, 0.533f, 0.491f}, {0.064f, 0.039f, 0.134f}, {0.46f, 0.51f, 0.13f}},
+    {FED_128x192, 128, 192, {2.52f, 2.67f, 4.01f}, {0.564f, 0.595f, 0.528f}, {0.051f, 0.030f, 0.121f}, {0.45f, 0.48f, 0.15f}},
+    {FED_160x192, 160, 192, {3.00f, 2.88f, 4.33f}, {0.609f, 0.662f, 0.620f}, {0.044f, 0.022f, 0.104f}, {0.41f, 0.44f, 0.15f}},
+    {FED_128x256, 128, 256, {2.98f, 2.92f, 4.40f}, {0.683f, 0.686f, 0.627f}, {0.049f, 0.031f, 0.114f}, {0.39f, 0.42f, 0.15f}},
+    {EDGE_256x128, 256, 128, {3.35f, 2.45f, 4.41f}, {0.748f, 0.784f, 0.678f}, {0.010f, 0.000f, 0.091f}, {0.39f, 0.46f, 0.16f}},
+};
+
+double fed_microseconds(const FedTile& t, GemmLayout layout, long long M, long long N, long long Kc, int parts,
+                        double epilogue) {
+  const long long w = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * parts;
+  const double rounds = (double)((w + 255) / 256), occupied = w >= 256 ? 1.0 : (double)w / 256;
+  const double mb = ((double)M + (double)N) * (double)Kc * 2e-6;
+  const double out = (double)M * (double)N * (parts > 1 ? 4e-6 * parts : 2e-6);
+  // rows of a contraction that does not fill 128-byte lines: the copies of a stage take two lines a row
+  const double lines = layout != GEMM_TN && Kc % 64 != 0 ? 1.3 : 1.0;
+  const double stages = (double)((Kc + 63) / 64 + parts - 1) / parts;
+  return rounds * (t.round[layout] + t.stage[layout] * lines * stages + epilogue * (t.bm * t.bn) / 32768.0) +
+         t.operands[layout] * mb / occupied + t.output[layout] * out;
+}
+
+// The best of them for a contraction in `parts`, or null.  More than two rounds of workgroups are left to larger
+// tiles, and so are contractions of many stages to those of more than 64 columns: 64-column tiles read 128 bytes of a
+// row of W or X at a time, which at some strides crowd onto few memory channels (446 x 2048 over 7168, rows of W of
+// 4096 bytes, 41 us, 31 on larger tiles).  A weight gradient over few tokens is all stores, whatever its tile.
+const FedTile* best_fed_tile(GemmLayout layout, long long M, long long N, long long Kc, int parts, double epilogue,
+                             double* us) {
+  const FedTile* best = nullptr;
+  if (layout == GEMM_TN && Kc < 192) return best;
+  for (const FedTile& t : kFedTiles) {
+    const long long w = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * parts;
+    if (w > (parts > 1 ? 256 : 512)) continue;
+    if (t.bn == 64 && Kc > (layout == GEMM_NT ? 4096 : 2560) * parts) continue;
+    const double e = fed_microseconds(t, layout, M, N, Kc, parts, epilogue);
+    if (best == nullptr || e < *us) {
+      best = &t;
+      *us = e;
+    }
+  }
+  return best;
+}
+
+// What the estimates above, of the other tiles, come to on cold operands: they leave out the output's way.  (Fitted to
+// the same products, 10 % rms.)
+double other_microseconds(GemmLayout layout, double us, long long M, long long N) {
+  const double out = (double)M * (double)N * 2e-6;
+  return layout == GEMM_TN ? 1.03 * us + 0.12 * out + 2.4 : layout == GEMM_NT ? 1.06 * us + 0.35 * out + 0.2 : 1.03 * us + 0.35 * out + 0.7;
+}
+
+// The fed tile of a contraction in one part, or null where the others are ahead or less than 5 % behind.  With the parts
+// of gemm_plan, 700 products drawn anew have 0.85 (forward), 0.86 (input gradient) and 0.98 (weight gradient) of the
+// time they had on average; 18 got 4 to 11 % slower (385 x 2848 over 3648 26 -> 29 us).  us, before / so, outputs over
+// contractions, operands from HBM: 512 x 8192, 3584 43.0 / 38.5; 777 x 6144, 4096 60 / 51; 250 x 1024, 1024 14.8 / 7.7;
+// 2006 x 2432, 1088 19.3 / 17.1; weight gradient 2440 x 2240, 800 18.6 / 16.6.
+const FedTile* fed_tile(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32) {
+  if (g.splits > 1 || (g.lda > g.ldb ? g.lda : g.ldb) >= kEdgeMaxLd / 2) return nullptr;
+  const bool bias = epilogue == AXN_EPI_BIAS, gelu = epilogue == AXN_EPI_BIAS_GELU || epilogue == AXN_EPI_GELU;
+  const double extra = (bias ? 3.3 : gelu ? 7.8 : 0.0) + (bias || gelu ? 1.1 * ((out_f32 ? 1 : 0) + (gelu && g.Z != nullptr ? 1 : 0)) : 0.0);
+  double us = 0, other = 0;
+  const FedTile* t = best_fed_tile(layout, g.M, g.N, g.Kc, 1, extra, &us);
+  if (t == nullptr) return nullptr;
+  edge_tile(g.M, g.N, g.Kc, epilogue_time(g, epilogue, out_f32), &other);
+  return us < 0.95 * other_microseconds(layout, other, g.M, g.N) ? t : nullptr;
+}
+
+int launch_fed(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, bool half, EdgeTile tile,
+               hipStream_t stream) {
+  if (tile == EDGE_256x128)
+    return half ? launch_gemm_edge_f16(layout, g, epilogue, out_f32, tile, stream)
+                : launch_gemm_edge_bf16(layout, g, epilogue, out_f32, tile, stream);
+  if (layout == GEMM_NT)
+    return half ? launch_gemm_fed_nt_f16(g, epilogue, out_f32, tile, stream)
+                : launch_gemm_fed_nt_bf16(g, epilogue, out_f32, tile, stream);
+  return half ? launch_gemm_fed_nn_tn_f16(layout, g, out_f32, tile, stream)
+              : launch_gemm_fed_nn_tn_bf16(layout, g, out_f32, tile, stream);
+}
+
 int launch_edge(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, bool half,
                 hipStream_t stream) {
   const int64_t ld = g.lda > g.ldb ? g.lda : g.ldb;
@@ -274,9 +369,11 @@ int launch_whole(const GemmArgs& g, hipStream_t stream) {
 template <bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
 int launch_shape(const GemmArgs& g, hipStream_t stream) {
   if constexpr (EPI != EPI_PAIR) {
+    constexpr GemmLayout order = !AK ? GEMM_TN : BKM ? GEMM_NT : GEMM_NN;
+    if (const FedTile* t = fed_tile(order, g, EPI, OUT_F32))
+      return launch_fed(order, g, EPI, OUT_F32, HALF, t->tile, stream);
     // output rows that are not 16-byte aligned (axn_gemm_any_n): the kernels with bounds store them
-    constexpr GemmLayout layout = !AK ? GEMM_TN : BKM ? GEMM_NT : GEMM_NN;
-    if (g.ldc % 8 != 0) return launch_edge(layout, g, EPI, OUT_F32, HALF, stream);
+    if (g.ldc % 8 != 0) return launch_edge(order, g, EPI, OUT_F32, HALF, stream);
   }
   if (g.M % 256 == 0 && g.N % 256 == 0 && g.Kc % 64 == 0 && g.splits <= 1) {
     const long long tm = g.M / 256, tn = g.N / 256, tiles = tm * tn;
@@ -316,6 +413,11 @@ int launch_shape(const GemmArgs& g, hipStream_t stream) {
         const int64_t b_span = (int64_t)(BKM ? g2.N : g2.Kc) * g2.ldb * 2;
         if (rest > 64 && a_span < (1LL << 31) && b_span < (1LL << 31))
           return launch_rest<AK, BKM, EPI, OUT_F32, HALF>(g2, stream);
+        if constexpr (EPI != EPI_PAIR) {
+          constexpr GemmLayout order = !AK ? GEMM_TN : BKM ? GEMM_NT : GEMM_NN;
+          if (const FedTile* t = fed_tile(order, g2, EPI, OUT_F32))
+            return launch_fed(order, g2, EPI, OUT_F32, HALF, t->tile, stream);
+        }
         return launch_whole<AK, BKM, EPI, OUT_F32, HALF>(g2, stream);
       }
     }
@@ -649,6 +751,41 @@ SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, doubl
   return plan;
 }
 
+// The parts that a sum of the fp32 products reads and writes, and the launch it is: fitted to 2 to 16 parts.
+static double sum_microseconds(int64_t M, int64_t N, int parts) {
+  return 2.5 + (double)M * (double)N * (4 * parts + 2) * 1e-6 / 7.0;
+}
+
+SplitPlan gemm_plan(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
+  double other = 0, us = 0, one = 0;
+  SplitPlan plan = gemm_splits(layout, M, N, Kc, &other);
+  if (plan.parts <= 1) return plan;
+  other = 0.95 * other_microseconds(layout, other, M, N);
+  if (const FedTile* t = best_fed_tile(layout, M, N, Kc, plan.parts, 0, &us)) {
+    us += sum_microseconds(M, N, plan.parts);
+    if (us < other) {
+      other = us;
+      plan.tile = t->tile;
+    }
+  }
+  // The input gradient of a layer whose gradients take one launch keeps the parts it has there.
+  if (best_fed_tile(layout, M, N, Kc, 1, 0, &one) != nullptr && one < other &&
+      !(layout == GEMM_NN && (gemm_backward_parts(M, Kc, N, false) > 0 || gemm_backward_parts(M, Kc, N, true) > 0)))
+    plan.parts = 1;
+  return plan;
+}
+
+static int launch_sum(const GemmArgs& in, int epilogue, bool half, bool out_f32, int parts, const float* ws,
+                      hipStream_t stream) {
+  GemmArgs out = in;
+  out.splits = parts;
+  if (out.N % 8 != 0 || out.ldc % 8 != 0)
+    return half ? launch_reduce<true, true>(ws, out, epilogue, out_f32, stream)
+                : launch_reduce<false, true>(ws, out, epilogue, out_f32, stream);
+  return half ? launch_reduce<true, false>(ws, out, epilogue, out_f32, stream)
+              : launch_reduce<false, false>(ws, out, epilogue, out_f32, stream);
+}
+
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool half, bool out_f32,
                        const SplitPlan& plan, float* ws, hipStream_t stream) {
   GemmArgs g = in;
@@ -659,6 +796,10 @@ int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool
   g.Z = nullptr;
   g.splits = plan.parts;
   g.k_split = g.Kc / plan.parts;
+  if (plan.tile > EDGE_128x128) {
+    const int rc = launch_fed(layout, g, AXN_EPI_NONE, true, half, plan.tile, stream);
+    return rc ? rc : launch_sum(in, epilogue, half, out_f32, plan.parts, ws, stream);
+  }
   const bool ak = layout != GEMM_TN, bkm = layout == GEMM_NT;
   const int bm = plan.tile == EDGE_128x128 ? 128 : 256, bn = plan.tile == EDGE_256x256 ? 256 : 128;
   const bool whole = g.M % bm == 0 && g.N % bn == 0 && g.Kc % (64 * plan.parts) == 0 &&
@@ -683,14 +824,7 @@ int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool
                   : launch_split<false, false, false>(g, plan.tile, stream);
     }
   }
-  if (rc) return rc;
-  GemmArgs out = in;
-  out.splits = plan.parts;
-  if (out.N % 8 != 0 || out.ldc % 8 != 0)
-    return half ? launch_reduce<true, true>(ws, out, epilogue, out_f32, stream)
-                : launch_reduce<false, true>(ws, out, epilogue, out_f32, stream);
-  return half ? launch_reduce<true, false>(ws, out, epilogue, out_f32, stream)
-              : launch_reduce<false, false>(ws, out, epilogue, out_f32, stream);
+  return rc ? rc : launch_sum(in, epilogue, half, out_f32, plan.parts, ws, stream);
 }
 
 // ---- both gradients in one launch, the input gradient's contraction in parts -----------
@@ -763,10 +897,7 @@ int launch_gemm_backward_parts(const GemmArgs& dgrad, const GemmArgs& wgrad, boo
   const int rc = half ? launch_gemm_edge_backward_f16(gw, gd, dw_f32, stream)
                       : launch_gemm_edge_backward_bf16(gw, gd, dw_f32, stream);
   if (rc) return rc;
-  GemmArgs out = dgrad;
-  out.splits = parts;
-  return half ? launch_reduce<true, false>(ws, out, AXN_EPI_NONE, false, stream)
-              : launch_reduce<false, false>(ws, out, AXN_EPI_NONE, false, stream);
+  return launch_sum(dgrad, AXN_EPI_NONE, half, false, parts, ws, stream);
 }
 
 }  // namespace axn

@@ -154,6 +154,15 @@ __device__ __forceinline__ void lanes_16_down(uint32_t (&b)[4], int from) {
                : "+&v"(b[0]), "+&v"(b[1]), "+&v"(b[2]), "+&v"(b[3])
                : "v"(from));
 }
+__device__ __forceinline__ void lanes_16_down(uint32_t (&b)[3], int from) {
+  asm volatile("ds_bpermute_b32 %0, %3, %0\n\tds_bpermute_b32 %1, %3, %1\n\tds_bpermute_b32 %2, %3, %2\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "+&v"(b[0]), "+&v"(b[1]), "+&v"(b[2])
+               : "v"(from));
+}
+__device__ __forceinline__ void lanes_16_down(uint32_t (&b)[1], int from) {
+  asm volatile("ds_bpermute_b32 %0, %1, %0\n\ts_waitcnt lgkmcnt(0)" : "+&v"(b[0]) : "v"(from));
+}
 __device__ __forceinline__ void lanes_16_down(uint32_t (&b)[2], int from) {
   asm volatile("ds_bpermute_b32 %0, %2, %0\n\tds_bpermute_b32 %1, %2, %1\n\ts_waitcnt lgkmcnt(0)"
                : "+&v"(b[0]), "+&v"(b[1])
@@ -259,6 +268,9 @@ __device__ __forceinline__ s16x4 lds_read_tr16_b64(uint32_t addr) {
 //   MN-major tile [64][256] : 512-byte rows; 64-byte chunk c of contraction row k
 //                             lives at chunk c ^ (k & 3); read with the transposing
 //                             ds_read_b64_tr_b16 (two per fragment)
+// Tiles of other heights (multiples of 32 rows) differ in the MN-major swizzle alone: four contraction rows
+// that are read together have to lie in four different 64-byte quarters of the 256 bytes that the banks span.
+// Rows of an odd number of chunks do so by themselves, rows of 2, 6, 10 ... chunks with c ^ ((k >> 1) & 1).
 //
 // PERMUTED (the operand that supplies the output columns): fragment j holds the
 // tile rows 32 (j / 2) + 8 (q / 4) + 4 (j % 2) + q % 4 in its lane-rows
@@ -268,7 +280,7 @@ __device__ __forceinline__ s16x4 lds_read_tr16_b64(uint32_t addr) {
 // registers without a transpose through LDS.  Its K-major swizzle is
 // chunk ^ (((r >> 1) & 1) | ((r >> 3) & 3) << 1), which again gives the 16 rows
 // of a fragment quarter 16 distinct (row parity, chunk) pairs.
-template <bool KMAJOR, bool PERMUTED, int ROWS_ /* 256 or 128 */>
+template <bool KMAJOR, bool PERMUTED, int ROWS_ /* a multiple of 32, up to 256 */>
 struct DeepOperand {
   static constexpr int ROWS = ROWS_;
   static constexpr int PK = 64;
@@ -276,11 +288,14 @@ struct DeepOperand {
   static constexpr int NW = 4;
   static constexpr int DMA_N = BYTES / 1024 / NW;  // 8 or 4 copies per wave
   static constexpr int FR = ROWS / 32;             // 16-row fragments of a wave's half of the rows
-  static constexpr int NADDR = KMAJOR ? 2 : FR / 2;
+  static constexpr int NADDR = KMAJOR ? 2 : (FR + 1) / 2;
   static constexpr int LPR = ROWS / 8;             // MN-major: lanes per contraction row of a copy
 
   __device__ __forceinline__ static int kmajor_swizzle(int row) {
     return PERMUTED ? (((row >> 1) & 1) | (((row >> 3) & 3) << 1)) : ((row >> 1) & 7);
+  }
+  __device__ __forceinline__ static int mnmajor_swizzle(int k) {
+    return ROWS / 32 % 4 == 0 ? k & 3 : ROWS / 32 % 2 == 0 ? (k >> 1) & 1 : 0;
   }
 
   // Byte offset of this lane's 16 bytes for copy 0 of the tile at contraction
@@ -288,12 +303,13 @@ struct DeepOperand {
   // lands at tile + (4 i + wave) * 1024 + 16 l; the swizzle is applied here.
   __device__ __forceinline__ static uint32_t dma_offset(int64_t ld, int row0, int wave,
                                                         int lane, uint32_t& istride) {
-    if (KMAJOR) {
+    if constexpr (KMAJOR) {
       const int row = wave * 8 + (lane >> 3);              // + 32 i
       const int c = (lane & 7) ^ kmajor_swizzle(row);      // 32 i does not change the swizzle
       istride = (uint32_t)(32 * ld * 2);
       return (uint32_t)(((int64_t)(row0 + row) * ld + c * 8) * 2);
     } else {
+      static_assert(64 % LPR == 0, "copies of whole contraction rows: 256 or 128 rows");
       constexpr int KPI = 64 / LPR;                    // contraction rows per copy: 2 or 4
       const int k = wave * KPI + lane / LPR;           // + 4 KPI i
       const int p16 = lane % LPR;
@@ -301,6 +317,13 @@ struct DeepOperand {
       istride = (uint32_t)(4 * KPI * ld * 2);
       return (uint32_t)(((int64_t)k * ld + row0 + (c64 * 4 + (p16 & 3)) * 8) * 2);
     }
+  }
+
+  // MN-major, tiles of any height: this lane's byte offset for copy i (contraction rows end inside a copy).
+  __device__ __forceinline__ static uint32_t mnmajor_copy(int64_t ld, int wave, int lane, int i) {
+    const int at = (NW * i + wave) * 1024 + 16 * lane, k = at / (ROWS * 2), b = at % (ROWS * 2);
+    const int col = ((b >> 6) ^ mnmajor_swizzle(k)) * 32 + (b & 63) / 2;
+    return (uint32_t)(((int64_t)k * ld + col) * 2);
   }
 
   // K-major: the 8 contraction elements 8 c .. 8 c + 7 of the tile that this lane copies
@@ -342,7 +365,7 @@ struct DeepOperand {
 #pragma unroll
       for (int h = 0; h < NADDR; ++h) {
         const int colbyte = (wrow0 + h * 32 + (PERMUTED ? 8 : 4) * (lane & 3)) * 2;
-        a[h] = (uint32_t)(k * (ROWS * 2) + ((((colbyte >> 6) ^ kq) << 6) | (colbyte & 63)));
+        a[h] = (uint32_t)(k * (ROWS * 2) + ((((colbyte >> 6) ^ mnmajor_swizzle(kq)) << 6) | (colbyte & 63)));
       }
     }
   }
@@ -362,6 +385,33 @@ struct DeepOperand {
   }
 };
 
+// With bounds: where the next A / B tile to copy starts and how many bytes of the operand lie
+// behind that point.
+struct OperandWalk {
+  const char* at;
+  int64_t left, step;
+  __device__ __forceinline__ void start(const uint16_t* base, bool kmajor, int rows, int kc, int64_t ld, int row0,
+                                        int k0) {
+    const int64_t first = kmajor ? row0 * ld + k0 : k0 * ld + row0;
+    // a row's last 8 elements are copied together: up to 7 of them are padding of the operand's rows
+    const int64_t all = kmajor ? (int64_t)(rows - 1) * ld + ceil_div(kc, 8) * 8 : (int64_t)(kc - 1) * ld + ceil_div(rows, 8) * 8;
+    at = (const char*)(base + first);
+    left = (all - first) * 2;
+    step = (kmajor ? (int64_t)64 : (int64_t)64 * ld) * 2;
+  }
+  // (left is positive: only stages that exist are copied; its halves are looked at one by
+  // one because there is no scalar 64-bit order comparison)
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t resource() const {
+    const uint32_t lo = (uint32_t)left;
+    const uint32_t n = (uint32_t)(left >> 32) != 0u || lo > 0x7fffffffu ? 0x7fffffffu : lo;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)at, 0, (int)n, 0x00020000);
+  }
+  __device__ __forceinline__ void advance() {
+    at += step;
+    left -= step;
+  }
+};
+
 // Waits for every outstanding LDS read; the fragments flow through the
 // statement, so no MFMA on them can move above the wait.
 __device__ __forceinline__ void wait_all_fragments(bf16x8 (&fa)[8], bf16x8 (&fb)[8]) {
@@ -369,11 +419,6 @@ __device__ __forceinline__ void wait_all_fragments(bf16x8 (&fa)[8], bf16x8 (&fb)
                : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fa[4]), "+v"(fa[5]),
                  "+v"(fa[6]), "+v"(fa[7]), "+v"(fb[0]), "+v"(fb[1]), "+v"(fb[2]), "+v"(fb[3]),
                  "+v"(fb[4]), "+v"(fb[5]), "+v"(fb[6]), "+v"(fb[7]));
-}
-__device__ __forceinline__ void wait_all_fragments(bf16x8 (&fa)[8], bf16x8 (&fb)[4]) {
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fa[4]), "+v"(fa[5]),
-                 "+v"(fa[6]), "+v"(fa[7]), "+v"(fb[0]), "+v"(fb[1]), "+v"(fb[2]), "+v"(fb[3]));
 }
 __device__ __forceinline__ void wait_all_fragments(bf16x8 (&fa)[4], bf16x8 (&fb)[4]) {
   asm volatile("s_waitcnt lgkmcnt(0)"
@@ -392,6 +437,99 @@ __device__ __forceinline__ void settle_accumulators(f32x4 (&a)[4]) {
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Output of a wave's accumulators: rows m_first .., columns n_first .. of C.  With the permuted column fragments a
+// lane owns, per block row i and block pair t, the 8 consecutive columns 32 t + 8 (l / 16) .. + 7 of row
+// 16 i + l % 16: they go out straight from the registers, 64 contiguous bytes per row and instruction.
+// EDGE: rows and columns inside the output only; tail: 8 floats a row in LDS that are the wave's own.
+// APART: one block row after the other (left to itself the compiler works on several at once, and spills where a
+// wave has 256 registers).
+template <int EPI, bool OUT_F32, bool HALF, bool EDGE, bool ODD, bool APART = false, int FRM, int FRN>
+__device__ __forceinline__ void store_blocks(f32x4 (&acc)[FRM][FRN], const GemmArgs& g, int split, int m_first,
+                                             int n_first, int lane, [[maybe_unused]] float* tail) {
+  constexpr int WTM = FRM * 16, WTN = FRN * 16;
+  const int orow = m_first + (lane & 15), ocol = n_first + 8 * (lane >> 4);
+  GemmArgs go = g;  // a split writes its own fp32 partial product
+  if (OUT_F32 && g.splits > 1) go.C = (float*)g.C + (int64_t)split * g.M * g.ldc;
+  constexpr int EP = EPI == EPI_PAIR ? (int)AXN_EPI_NONE : EPI;
+  // EDGE: the columns behind the last multiple of 8 of the output go through LDS and are
+  // stored one by one, which keeps that path out of the unrolled stores.
+  float bias[FRN / 2][8];
+#pragma unroll
+  for (int t = 0; t < FRN / 2; ++t)
+    if (!EDGE || ocol + 32 * t + 8 <= g.N) load_bias8<EP, HALF>(bias[t], g, ocol + 32 * t);
+  static_assert(!ODD || (EDGE && EP == AXN_EPI_NONE && !OUT_F32), "store_row8_odd");
+  if constexpr (ODD) {
+    using lp = std::conditional_t<HALF, _Float16, __bf16>;
+    using lpx8 = std::conditional_t<HALF, f16x8, bf16x8>;
+#pragma unroll
+    for (int i = 0; i < FRM; ++i) {
+      const int row = orow + 16 * i;
+      u32x4 y[FRN / 2];
+      uint32_t before[FRN / 2];   // of each 8 columns: the dword with the one before them
+#pragma unroll
+      for (int t = 0; t < FRN / 2; ++t) {
+        lpx8 y8;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          y8[e] = (lp)acc[i][2 * t][e];
+          y8[4 + e] = (lp)acc[i][2 * t + 1][e];
+        }
+        y[t] = __builtin_bit_cast(u32x4, y8);
+        // it lies in the lane 16 further down; for lanes 0 .. 15 in lanes 48 .. 63 at t - 1
+        before[t] = lane >= 48 ? (t > 0 ? y[t - 1][3] : 0u) : y[t][3];
+      }
+      lanes_16_down(before, ((lane + 48) & 63) * 4);
+#pragma unroll
+      for (int t = 0; t < FRN / 2; ++t) {
+        const int col = ocol + 32 * t;
+        if (row >= g.M || col >= g.N) continue;
+        if (col + 8 > g.N) {
+          f32x4* to = (f32x4*)(tail + ((lane & 15) + 16 * i) * 8);
+          to[0] = acc[i][2 * t];
+          to[1] = acc[i][2 * t + 1];
+          continue;
+        }
+        store_row8_odd((uint16_t*)go.C + (int64_t)row * go.ldc + col, y[t], before[t], t == 0 && lane < 16,
+                       (t == FRN / 2 - 1 && lane >= 48) || col + 16 > g.N);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < FRM; ++i) {
+      if constexpr (APART) {
+#pragma unroll
+        for (int j = 0; j < FRN; ++j) asm volatile("" : "+a"(acc[i][j])::"memory");
+      }
+#pragma unroll
+      for (int t = 0; t < FRN / 2; ++t) {
+        const f32x4 lo = acc[i][2 * t], hi = acc[i][2 * t + 1];
+        float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        const int row = orow + 16 * i, col = ocol + 32 * t;
+        if constexpr (EDGE) {
+          if (row >= g.M || col >= g.N) continue;
+          if (col + 8 > g.N) {
+            f32x4* to = (f32x4*)(tail + ((lane & 15) + 16 * i) * 8);
+            to[0] = lo;
+            to[1] = hi;
+            continue;
+          }
+        }
+        store_row8<EP, OUT_F32, HALF, EDGE>(v, bias[t], go, row, col);
+      }
+    }
+  }
+  if constexpr (EDGE) {
+    const int end = g.N / 8 * 8, first = n_first;
+    if (end < g.N && end >= first && end < first + WTN) {
+#pragma unroll 1
+      for (int k = lane; k < WTM * 8; k += 64) {
+        const int row = m_first + k / 8, col = end + k % 8;
+        if (row < g.M && col < g.N) store_one<EP, OUT_F32, HALF>(tail[k], go, row, col);
+      }
+    }
+  }
 }
 
 // TILE = 256: 4 waves, one per SIMD, each owning 128 x 128 of the 256 x 256 tile:
@@ -413,11 +551,6 @@ __device__ __forceinline__ void wait_vmcnt() {
 // TILE = 128 is the same schedule on a 128 x 128 tile for problems that do not
 // fill the chip with 256 x 256 tiles: 64 x 64 per wave (4 x 4 blocks, 16 MFMAs per
 // step, 4 copies per tile and wave), an 80 KiB ring, two workgroups per CU.
-//
-// BM x BN = 256 x 128 is the tile of the launches that finish a problem after its full
-// rounds of 256 x 256 tiles: a rest of r <= 128 large tiles makes 2 r <= 256 of these,
-// one per CU, and needs 3/4 of the global -> LDS bytes per MFMA of the 128 x 128 tile.
-// Its ring has five slots of the larger (A) tile's size.
 //
 // EDGE: any M, N and contraction, operands of any size.  The main loop is the same; what is
 // added is
@@ -453,8 +586,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   constexpr int READ_EVERY = (NM / 2) / NFRAG;     // a fragment read every .. MFMAs, first half of a step
   constexpr int COPY_EVERY_A = (NM / 2) / NCA;     // a copy every .. MFMAs, second half
   constexpr int COPY_EVERY_B = (NM / 2) / NCB;
-  static_assert((BM == 256 || BM == 128) && (BN == 256 || BN == 128) && BM >= BN,
-                "tile sizes with a schedule below");
+  static_assert((BM == 256 || BM == 128) && BM == BN, "tile sizes with a schedule below");
   static_assert(READ_EVERY >= 1 && COPY_EVERY_A >= 1 && COPY_EVERY_B >= 1, "schedule fits a step");
   // Gate/up forward: the B tile's 256 rows are, per 128-row half (one wave column), 64
   // rows of the gate weights and the 64 rows of the up weights with the same indices, so
@@ -465,6 +597,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   // (A2, B2); everything behind the copies is unchanged.
   constexpr bool PAIR = EPI == EPI_PAIR;
   static_assert(!EDGE || (!SWIGLU && !PAIR), "whole tiles only");
+  static_assert(!ODD || (A_KMAJOR && B_KMAJOR), "the forward");
   static_assert(!PAIR || (A_KMAJOR && !B_KMAJOR), "the two-term product is the dgrad layout");
   static_assert(!SWIGLU || (BM == 256 && BN == 256 && A_KMAJOR && B_KMAJOR && !OUT_F32),
                 "the gate/up forward runs on the 256 x 256 tile with contraction-contiguous operands");
@@ -517,33 +650,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   uint32_t ka = 0, kb = 0;  // byte offsets of the next A / B tile to copy
   uint32_t wslot = 0;       // ring slot (byte offset) the next copied tile takes
 
-  // EDGE: where the next A / B tile to copy starts and how many bytes of the operand lie
-  // behind that point.
-  struct Walk {
-    const char* at;
-    int64_t left, step;
-    __device__ __forceinline__ void start(const uint16_t* base, bool kmajor, int rows, int kc, int64_t ld, int row0,
-                                          int k0) {
-      const int64_t first = kmajor ? row0 * ld + k0 : k0 * ld + row0;
-      // a row's last 8 elements are copied together: up to 7 of them are padding of the operand's rows
-      const int64_t all = kmajor ? (int64_t)(rows - 1) * ld + ceil_div(kc, 8) * 8 : (int64_t)(kc - 1) * ld + ceil_div(rows, 8) * 8;
-      at = (const char*)(base + first);
-      left = (all - first) * 2;
-      step = (kmajor ? (int64_t)PK : (int64_t)PK * ld) * 2;
-    }
-    // (left is positive: only stages that exist are copied; its halves are looked at one by
-    // one because there is no scalar 64-bit order comparison)
-    __device__ __forceinline__ __amdgpu_buffer_rsrc_t resource() const {
-      const uint32_t lo = (uint32_t)left;
-      const uint32_t n = (uint32_t)(left >> 32) != 0u || lo > 0x7fffffffu ? 0x7fffffffu : lo;
-      return __builtin_amdgcn_make_buffer_rsrc((void*)at, 0, (int)n, 0x00020000);
-    }
-    __device__ __forceinline__ void advance() {
-      at += step;
-      left -= step;
-    }
-  };
-  Walk walk_a, walk_b;
+  OperandWalk walk_a, walk_b;   // EDGE
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(char, lds);
   uint32_t ra0[OA::NADDR], rb0[OB::NADDR];
@@ -769,13 +876,8 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
   for (int i = 0; i < FRM; ++i) settle_accumulators(acc[i]);
-  // With the permuted column fragments a lane owns, per block row i and block
-  // pair t, the 8 consecutive columns 32 t + 8 (l / 16) .. + 7 of row 16 i + l % 16:
-  // they go out straight from the registers, 64 contiguous bytes per row and
-  // instruction.
-  const int orow = m0 + wm * WTM + (lane & 15);
-  const int ocol = n0 + wn * WTN + 8 * (lane >> 4);
   if constexpr (SWIGLU) {
+    const int orow = m0 + wm * WTM + (lane & 15);
     // blocks 0..3 of a lane's row hold 64 gate columns, blocks 4..7 the up values of the
     // same columns
     const int hcol = n0 + wn * (WTN / 2) + 8 * (lane >> 4);
@@ -790,83 +892,9 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
         store_swiglu8<HALF>(vg, vu, g, orow + 16 * i, hcol + 32 * t);
       }
   } else {
-    GemmArgs go = g;  // a split writes its own fp32 partial product
-    if (OUT_F32 && g.splits > 1) go.C = (float*)g.C + (int64_t)split * g.M * g.ldc;
-    constexpr int EP = PAIR ? (int)AXN_EPI_NONE : EPI;
-    // EDGE: the columns behind the last multiple of 8 of the output go through LDS and are
-    // stored one by one, which keeps that path out of the unrolled stores.  The ring slot
-    // behind the last stage's two is free: no wave reads or fills it any more.
-    [[maybe_unused]] float* tail = (float*)(lds + sa) + wave * (WTM * 8);
-    float bias[FRN / 2][8];
-#pragma unroll
-    for (int t = 0; t < FRN / 2; ++t)
-      if (!EDGE || ocol + 32 * t + 8 <= g.N) load_bias8<EP, HALF>(bias[t], g, ocol + 32 * t);
-    static_assert(!ODD || (EDGE && A_KMAJOR && B_KMAJOR && EP == AXN_EPI_NONE && !OUT_F32), "store_row8_odd");
-    if constexpr (ODD) {
-      using lp = std::conditional_t<HALF, _Float16, __bf16>;
-      using lpx8 = std::conditional_t<HALF, f16x8, bf16x8>;
-#pragma unroll
-      for (int i = 0; i < FRM; ++i) {
-        const int row = orow + 16 * i;
-        u32x4 y[FRN / 2];
-        uint32_t before[FRN / 2];   // of each 8 columns: the dword with the one before them
-#pragma unroll
-        for (int t = 0; t < FRN / 2; ++t) {
-          lpx8 y8;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            y8[e] = (lp)acc[i][2 * t][e];
-            y8[4 + e] = (lp)acc[i][2 * t + 1][e];
-          }
-          y[t] = __builtin_bit_cast(u32x4, y8);
-          // it lies in the lane 16 further down; for lanes 0 .. 15 in lanes 48 .. 63 at t - 1
-          before[t] = lane >= 48 ? (t > 0 ? y[t - 1][3] : 0u) : y[t][3];
-        }
-        lanes_16_down(before, ((lane + 48) & 63) * 4);
-#pragma unroll
-        for (int t = 0; t < FRN / 2; ++t) {
-          const int col = ocol + 32 * t;
-          if (row >= g.M || col >= g.N) continue;
-          if (col + 8 > g.N) {
-            f32x4* to = (f32x4*)(tail + ((lane & 15) + 16 * i) * 8);
-            to[0] = acc[i][2 * t];
-            to[1] = acc[i][2 * t + 1];
-            continue;
-          }
-          store_row8_odd((uint16_t*)go.C + (int64_t)row * go.ldc + col, y[t], before[t], t == 0 && lane < 16,
-                         (t == FRN / 2 - 1 && lane >= 48) || col + 16 > g.N);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < FRM; ++i)
-#pragma unroll
-        for (int t = 0; t < FRN / 2; ++t) {
-          const f32x4 lo = acc[i][2 * t], hi = acc[i][2 * t + 1];
-          float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          const int row = orow + 16 * i, col = ocol + 32 * t;
-          if constexpr (EDGE) {
-            if (row >= g.M || col >= g.N) continue;
-            if (col + 8 > g.N) {
-              f32x4* to = (f32x4*)(tail + ((lane & 15) + 16 * i) * 8);
-              to[0] = lo;
-              to[1] = hi;
-              continue;
-            }
-          }
-          store_row8<EP, OUT_F32, HALF, EDGE>(v, bias[t], go, row, col);
-        }
-    }
-    if constexpr (EDGE) {
-      const int end = g.N / 8 * 8, first = n0 + wn * WTN;
-      if (end < g.N && end >= first && end < first + WTN) {
-#pragma unroll 1
-        for (int k = lane; k < WTM * 8; k += 64) {
-          const int row = m0 + wm * WTM + k / 8, col = end + k % 8;
-          if (row < g.M && col < g.N) store_one<EP, OUT_F32, HALF>(tail[k], go, row, col);
-        }
-      }
-    }
+    // (the ring slot behind the last stage's two is free: no wave reads or fills it any more)
+    store_blocks<EPI, OUT_F32, HALF, EDGE, ODD>(acc, g, split, m0 + wm * WTM, n0 + wn * WTN, lane,
+                                                (float*)(lds + sa) + wave * (WTM * 8));
   }
 }
 

@@ -506,7 +506,11 @@ int axn_gemm_swiglu_fwd(const void* X, const void* Wg, const void* Wu, void* H, 
                         void* up_save, int dtype, int64_t M, int64_t N, int64_t K, int64_t ldx,
                         int64_t ldw, int64_t ldh, void* stream) {
   GemmArgs g = {};
+  const bool any = (dtype & AXN_ANY_SIZES) != 0;
+  dtype &= ~(int)AXN_ANY_SIZES;
   const int rc = swiglu_args("axn_gemm_swiglu_fwd", g, X, Wg, Wu, H, gate_save, up_save, dtype, M, N, K, ldx, ldw, ldh);
+  bool taken;
+  if (rc == AXN_OK && any) return launch_gemm_swiglu_any(g, dtype == AXN_F16, false, (hipStream_t)stream, taken);
   return rc ? rc : launch_gemm_swiglu(g, dtype == AXN_F16, (hipStream_t)stream);
 }
 

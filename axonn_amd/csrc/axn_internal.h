@@ -233,6 +233,9 @@ int launch_gemm_stream_swiglu(const GemmArgs& args, bool half, hipStream_t strea
 // C = silu(A B^T) * (A B2^T) in one launch (both weight matrices [N][Kc], K-major), for
 // M % 256 == 0, N % 128 == 0, Kc % 64 == 0 and operands below 2 GiB; AXN_ESHAPE otherwise.
 int launch_gemm_swiglu(const GemmArgs& args, bool half, hipStream_t stream);
+// The same for any M, N a multiple of 8 (gemm_gate_up.hip), on the tile that is estimated to be fastest; row strides
+// below kEdgeMaxLd / 2.  unless_largest: nothing is launched (taken is false) where that is 256 x 256, or within 5 %.
+int launch_gemm_swiglu_any(const GemmArgs& args, bool half, bool unless_largest, hipStream_t stream, bool& taken);
 
 // C[M x N] = A B + A2 B2, A / A2 K-major [M][k1], [M][k2], B / B2 MN-major [k1][N], [k2][N]
 // (two input-gradient products added in the accumulators): args.Kc = k1 + k2,

@@ -553,6 +553,11 @@ int launch_gemm_swiglu(const GemmArgs& in, bool half, hipStream_t stream) {
               "2 GiB (got M=%d, N=%d, K=%d)", g.M, g.N, g.Kc);
     return AXN_ESHAPE;
   }
+  if (g.lda < kEdgeMaxLd / 2 && g.ldb < kEdgeMaxLd / 2) {   // few large tiles, or a last round of few: others
+    bool taken = false;
+    const int rc = launch_gemm_swiglu_any(g, half, true, stream, taken);
+    if (taken) return rc;
+  }
   g.tiles_m = g.M / 256;
   g.tiles_n = g.N / 128;
   g.splits = 0;

@@ -6,19 +6,6 @@
 namespace axn {
 namespace {
 
-// Passes fragments through a statement, behind the wait for them.
-template <int N>
-__device__ __forceinline__ void tie_fragments(bf16x8 (&f)[N]) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));
-}
-// The same for a row of accumulators (see the end of solo_gemm).
-template <int N>
-__device__ __forceinline__ void tie_accumulators(f32x4 (&a)[N]) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+a"(a[i]));
-}
-
 // Stages that fit into a CU's LDS, at most five.
 template <int BM, int BN>
 constexpr int kFedStages = 163840 / ((BM + BN) * 128) < 5 ? 163840 / ((BM + BN) * 128) : 5;
@@ -57,13 +44,14 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
   using OB = DeepOperand<B_KMAJOR, true, BN>;
   constexpr uint32_t STAGE = OA::BYTES + OB::BYTES;
   constexpr int NCA = OA::DMA_N, NCB = OB::DMA_N, NC = NCA + NCB;   // copies per stage and copying wave
-  constexpr bool PAIR = EPI == EPI_PAIR;
+  constexpr bool PAIR = EPI == EPI_PAIR, SWIGLU = EPI == EPI_SWIGLU;
   constexpr int READ_EVERY = NM / NFRAG >= 2 ? 2 : 1;   // a fragment read every .. MFMAs, from a step's first on
   static_assert(BM % 32 == 0 && BN % 64 == 0 && NM >= NFRAG, "blocks of a wave, and a place for every read in a step");
   static_assert(4 * NM + 8 * NFRAG <= 232, "accumulators and two sets of fragments leave room for addresses");
   static_assert(NST >= 3 && (NST - 1) * NC <= 63, "the count of a wait has six bits");
   static_assert(!PAIR || (A_KMAJOR && !B_KMAJOR), "the two-term product is the dgrad layout");
   static_assert(!ODD || (A_KMAJOR && B_KMAJOR), "the forward");
+  static_assert(!SWIGLU || (BN % 128 == 0 && A_KMAJOR && B_KMAJOR && !OUT_F32), "gate and up rows of a wave column");
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -78,15 +66,16 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
     }
     tile_of_workgroup(pid, g.tiles_m, g.tiles_n, tm, tn);
   }
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * BM, n0 = tn * (SWIGLU ? BN / 2 : BN);
   const StageRange part = stages_of_part(g.Kc, split, g.splits);
   const int s0 = part.first, KP = part.count;
 
   if (wave8 >= 4) {
-    OperandWalk wa, wb;
+    OperandWalk wa, wb, wb2;   // (wb2: SWIGLU, the up weights')
     const int kfirst = PAIR ? g.k_first : g.Kc;
     wa.start(g.A, A_KMAJOR, g.M, kfirst, g.lda, m0, s0 * PK);
     wb.start(g.B, B_KMAJOR, g.N, kfirst, g.ldb, n0, s0 * PK);
+    if constexpr (SWIGLU) wb2.start(g.B2, B_KMAJOR, g.N, g.Kc, g.ldb, n0, s0 * PK);
     // per-lane offsets of the copies: one and a stride (K-major), or one for each copy
     uint32_t ais = 0, bis = 0, va[A_KMAJOR ? 1 : NCA], vb[B_KMAJOR ? 1 : NCB];
     if constexpr (A_KMAJOR) {
@@ -114,6 +103,11 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
         if (B_KMAJOR && 8 * OB::dma_chunk(wave, lane) >= PK - over) vb[0] = kOutside;
       }
       const __amdgpu_buffer_rsrc_t ra = wa.resource(), rb = wb.resource();
+      [[maybe_unused]] __amdgpu_buffer_rsrc_t rb2 = rb;
+      if constexpr (SWIGLU) {
+        rb2 = wb2.resource();
+        wb2.advance();
+      }
       char* at = lds + slot;
       static_for<NCA>([&](auto c) {
         constexpr int I = decltype(c)::value;
@@ -122,7 +116,10 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
       });
       static_for<NCB>([&](auto c) {
         constexpr int I = decltype(c)::value;
-        if constexpr (B_KMAJOR) OB::template dma_one<I>(rb, vb[0], 0, bis, at + OA::BYTES, wave);
+        if constexpr (SWIGLU) {
+          constexpr GateUpCopy from = gate_up_copy(BN, I);
+          OB::template dma_one<I, from.at>(from.up ? rb2 : rb, vb[0], 0, bis, at + OA::BYTES, wave);
+        } else if constexpr (B_KMAJOR) OB::template dma_one<I>(rb, vb[0], 0, bis, at + OA::BYTES, wave);
         else OB::template dma_one<I, 0>(rb, vb[I], 0, 0, at + OA::BYTES, wave);
       });
       wa.advance();
@@ -191,9 +188,7 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
       constexpr int ST = decltype(st_)::value;
       bf16x8(&fa)[FRM] = ST ? fa1 : fa0;
       bf16x8(&fb)[FRN] = ST ? fb1 : fb0;
-      asm volatile("s_waitcnt lgkmcnt(0)");   // every read of this set was issued during the previous step
-      tie_fragments(fa);
-      tie_fragments(fb);
+      wait_all_fragments(fa, fb);   // every read of this set was issued during the previous step
       if constexpr (ST == 1 && !LAST) __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
       static_for<NM>([&](auto m_) {
@@ -222,10 +217,14 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
   for (int i = 0; i < FRM; ++i) tie_accumulators(acc[i]);
-  // (s is the slot behind the last stage's: no wave reads or fills it any more)
-  constexpr bool APART = EPI != AXN_EPI_NONE && !PAIR;
-  store_blocks<EPI, OUT_F32, HALF, EDGE, ODD, APART>(acc, g, split, m0 + wm * (BM / 2), n0 + wn * (BN / 2), lane,
-                                                     (float*)(lds + s) + wave * (FRM * 16 * 8));
+  if constexpr (SWIGLU) {
+    store_gate_up<HALF, EDGE>(acc, g, m0 + wm * (BM / 2), n0 + wn * (BN / 4), lane);
+  } else {
+    // (s is the slot behind the last stage's: no wave reads or fills it any more)
+    constexpr bool APART = EPI != AXN_EPI_NONE && !PAIR;
+    store_blocks<EPI, OUT_F32, HALF, EDGE, ODD, APART>(acc, g, split, m0 + wm * (BM / 2), n0 + wn * (BN / 2), lane,
+                                                       (float*)(lds + s) + wave * (FRM * 16 * 8));
+  }
 }
 
 }  // namespace

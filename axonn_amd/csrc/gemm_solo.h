@@ -412,27 +412,24 @@ struct OperandWalk {
   }
 };
 
-// Waits for every outstanding LDS read; the fragments flow through the
-// statement, so no MFMA on them can move above the wait.
-__device__ __forceinline__ void wait_all_fragments(bf16x8 (&fa)[8], bf16x8 (&fb)[8]) {
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fa[4]), "+v"(fa[5]),
-                 "+v"(fa[6]), "+v"(fa[7]), "+v"(fb[0]), "+v"(fb[1]), "+v"(fb[2]), "+v"(fb[3]),
-                 "+v"(fb[4]), "+v"(fb[5]), "+v"(fb[6]), "+v"(fb[7]));
+// Passes fragments through a statement, so that no MFMA on them can move above it.
+template <int N>
+__device__ __forceinline__ void tie_fragments(bf16x8 (&f)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));
 }
-__device__ __forceinline__ void wait_all_fragments(bf16x8 (&fa)[4], bf16x8 (&fb)[4]) {
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fb[0]), "+v"(fb[1]),
-                 "+v"(fb[2]), "+v"(fb[3]));
+// Waits for every outstanding LDS read of both operands' fragments.
+template <int NA, int NB>
+__device__ __forceinline__ void wait_all_fragments(bf16x8 (&fa)[NA], bf16x8 (&fb)[NB]) {
+  asm volatile("s_waitcnt lgkmcnt(0)");
+  tie_fragments(fa);
+  tie_fragments(fb);
 }
-// Passes a row of accumulators through a statement (see the end of the kernel).
-__device__ __forceinline__ void settle_accumulators(f32x4 (&a)[8]) {
-  asm volatile("s_nop 3"
-               : "+a"(a[0]), "+a"(a[1]), "+a"(a[2]), "+a"(a[3]), "+a"(a[4]), "+a"(a[5]),
-                 "+a"(a[6]), "+a"(a[7]));
-}
-__device__ __forceinline__ void settle_accumulators(f32x4 (&a)[4]) {
-  asm volatile("s_nop 3" : "+a"(a[0]), "+a"(a[1]), "+a"(a[2]), "+a"(a[3]));
+// The same for a row of accumulators (see the end of solo_gemm).
+template <int N>
+__device__ __forceinline__ void tie_accumulators(f32x4 (&a)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+a"(a[i]));
 }
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
@@ -532,6 +529,40 @@ __device__ __forceinline__ void store_blocks(f32x4 (&acc)[FRM][FRN], const GemmA
   }
 }
 
+// The gate/up forward: the tile's B rows are, per wave column, a half of gate rows and then the up rows with the same
+// indices, so that a lane ends with a gate value in accumulator block j and the up value of the same output element in
+// block j + FRN / 2.  Copy i brings 32 rows: those of the gate or the up weights from row 32 at on.
+struct GateUpCopy {
+  bool up;
+  int at;
+};
+constexpr GateUpCopy gate_up_copy(int bn, int i) {
+  const int a_half = bn / 64, of_one = a_half / 2;   // copies a wave column, of one of the two matrices
+  return {i % a_half >= of_one, i / a_half * of_one + i % of_one};
+}
+template <bool HALF, bool EDGE, int FRM, int FRN>
+__device__ __forceinline__ void store_gate_up(f32x4 (&acc)[FRM][FRN], const GemmArgs& g, int m_first, int n_first,
+                                              int lane) {
+  const int orow = m_first + (lane & 15), ocol = n_first + 8 * (lane >> 4);
+#pragma unroll
+  for (int i = 0; i < FRM; ++i) {
+    if constexpr (EDGE) {   // (one block row after the other, as store_blocks)
+#pragma unroll
+      for (int j = 0; j < FRN; ++j) asm volatile("" : "+a"(acc[i][j])::"memory");
+    }
+#pragma unroll
+    for (int t = 0; t < FRN / 4; ++t) {
+      const int row = orow + 16 * i, col = ocol + 32 * t;
+      if (EDGE && (row >= g.M || col >= g.N)) continue;   // (N is a multiple of 8)
+      const f32x4 gl = acc[i][2 * t], gh = acc[i][2 * t + 1];
+      const f32x4 ul = acc[i][2 * t + FRN / 2], uh = acc[i][2 * t + 1 + FRN / 2];
+      const float vg[8] = {gl[0], gl[1], gl[2], gl[3], gh[0], gh[1], gh[2], gh[3]};
+      const float vu[8] = {ul[0], ul[1], ul[2], ul[3], uh[0], uh[1], uh[2], uh[3]};
+      store_swiglu8<HALF>(vg, vu, g, row, col);
+    }
+  }
+}
+
 // TILE = 256: 4 waves, one per SIMD, each owning 128 x 128 of the 256 x 256 tile:
 // 8 x 8 blocks of 16 x 16, 256 accumulator registers, 64 MFMAs per 32-deep step.
 // A wave pipelines against itself: while the MFMAs of one step run on one
@@ -586,20 +617,17 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   constexpr int READ_EVERY = (NM / 2) / NFRAG;     // a fragment read every .. MFMAs, first half of a step
   constexpr int COPY_EVERY_A = (NM / 2) / NCA;     // a copy every .. MFMAs, second half
   constexpr int COPY_EVERY_B = (NM / 2) / NCB;
-  static_assert((BM == 256 || BM == 128) && BM == BN, "tile sizes with a schedule below");
+  static_assert((BM == 128 && BN == 128) || (BM <= 256 && BN == 256), "tile sizes with a schedule below");
   static_assert(READ_EVERY >= 1 && COPY_EVERY_A >= 1 && COPY_EVERY_B >= 1, "schedule fits a step");
-  // Gate/up forward: the B tile's 256 rows are, per 128-row half (one wave column), 64
-  // rows of the gate weights and the 64 rows of the up weights with the same indices, so
-  // that a lane ends with a gate value in accumulator block j and the up value of the
-  // same output element in block j + 4.  The tile covers 128 output columns.
+  // Gate/up forward (gate_up_copy): the tile covers 128 output columns.
   constexpr bool SWIGLU = EPI == EPI_SWIGLU;
   // Two-term product: stages 0 .. k_first / 64 - 1 copy from (A, B), the others from
   // (A2, B2); everything behind the copies is unchanged.
   constexpr bool PAIR = EPI == EPI_PAIR;
-  static_assert(!EDGE || (!SWIGLU && !PAIR), "whole tiles only");
+  static_assert(!EDGE || !PAIR, "whole tiles only");
   static_assert(!ODD || (A_KMAJOR && B_KMAJOR), "the forward");
   static_assert(!PAIR || (A_KMAJOR && !B_KMAJOR), "the two-term product is the dgrad layout");
-  static_assert(!SWIGLU || (BM == 256 && BN == 256 && A_KMAJOR && B_KMAJOR && !OUT_F32),
+  static_assert(!SWIGLU || (BN == 256 && A_KMAJOR && B_KMAJOR && !OUT_F32),
                 "the gate/up forward runs on the 256 x 256 tile with contraction-contiguous operands");
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -644,13 +672,14 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   // the pair the copies read from (PAIR only: switched once, two stages before the
   // first stage of the second pair)
   __amdgpu_buffer_rsrc_t ra_cur = ra_rsrc, rb_cur = rb_rsrc;
+  [[maybe_unused]] __amdgpu_buffer_rsrc_t rb2_cur = rb2_rsrc;   // EDGE: the up weights'
   uint32_t a_is = 0, b_is = 0, va = 0, vb = 0;   // per-lane copy offsets of the current tile
   const uint32_t a_step = (uint32_t)((A_KMAJOR ? (int64_t)PK : (int64_t)PK * g.lda) * 2);
   const uint32_t b_step = (uint32_t)((B_KMAJOR ? (int64_t)PK : (int64_t)PK * g.ldb) * 2);
   uint32_t ka = 0, kb = 0;  // byte offsets of the next A / B tile to copy
   uint32_t wslot = 0;       // ring slot (byte offset) the next copied tile takes
 
-  OperandWalk walk_a, walk_b;   // EDGE
+  OperandWalk walk_a, walk_b, walk_b2;   // EDGE
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(char, lds);
   uint32_t ra0[OA::NADDR], rb0[OB::NADDR];
@@ -672,13 +701,14 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   };
   auto copy_b = [&](auto c_) {
     constexpr int I = decltype(c_)::value;
-    if constexpr (EDGE) {
+    if constexpr (SWIGLU) {
+      constexpr GateUpCopy from = gate_up_copy(BN, I);
+      if constexpr (EDGE)
+        OB::template dma_one<I, from.at>(from.up ? rb2_cur : rb_cur, vb, 0, b_is, lds + wslot, wave);
+      else
+        OB::template dma_one<I, from.at>(from.up ? rb2_rsrc : rb_rsrc, vb, kb, b_is, lds + wslot, wave);
+    } else if constexpr (EDGE) {
       OB::template dma_one<I>(rb_cur, vb, 0, b_is, lds + wslot, wave);
-    } else if constexpr (SWIGLU) {
-      // copies 4 h + {0, 1} of a half h bring 64 gate rows, 4 h + {2, 3} the 64 up rows
-      // with the same indices: both are rows 64 h + 32 (I % 2) .. of their matrix
-      constexpr int IO = 2 * (I / 4) + I % 2;
-      OB::template dma_one<I, IO>(I % 4 < 2 ? rb_rsrc : rb2_rsrc, vb, kb, b_is, lds + wslot, wave);
     } else if constexpr (PAIR) {
       OB::template dma_one<I>(rb_cur, vb, kb, b_is, lds + wslot, wave);
     } else {
@@ -698,6 +728,10 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
     if constexpr (EDGE) {
       walk_b.advance();
       rb_cur = walk_b.resource();
+      if constexpr (SWIGLU) {
+        walk_b2.advance();
+        rb2_cur = walk_b2.resource();
+      }
     } else {
       kb += b_step;
     }
@@ -797,6 +831,10 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
     walk_b.start(g.B, B_KMAJOR, g.N, g.Kc, g.ldb, n0, s0 * PK);
     ra_cur = walk_a.resource();
     rb_cur = walk_b.resource();
+    if constexpr (SWIGLU) {
+      walk_b2.start(g.B2, B_KMAJOR, g.N, g.Kc, g.ldb, n0, s0 * PK);
+      rb2_cur = walk_b2.resource();
+    }
     va = OA::dma_offset(g.lda, 0, wave, lane, a_is);
     vb = OB::dma_offset(g.ldb, 0, wave, lane, b_is);
     va_end = va;
@@ -835,7 +873,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
 #pragma unroll
     for (int j = 0; j < FRN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int i = 0; i < FRM; ++i) settle_accumulators(acc[i]);
+  for (int i = 0; i < FRM; ++i) tie_accumulators(acc[i]);
   if (KP > 1) {
     wait_vmcnt<NCA + NCB>();
   } else {
@@ -875,22 +913,9 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   // latency; the epilogue can only read the values these statements return.
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < FRM; ++i) settle_accumulators(acc[i]);
+  for (int i = 0; i < FRM; ++i) tie_accumulators(acc[i]);
   if constexpr (SWIGLU) {
-    const int orow = m0 + wm * WTM + (lane & 15);
-    // blocks 0..3 of a lane's row hold 64 gate columns, blocks 4..7 the up values of the
-    // same columns
-    const int hcol = n0 + wn * (WTN / 2) + 8 * (lane >> 4);
-#pragma unroll
-    for (int i = 0; i < FRM; ++i)
-#pragma unroll
-      for (int t = 0; t < FRN / 4; ++t) {
-        const f32x4 gl = acc[i][2 * t], gh = acc[i][2 * t + 1];
-        const f32x4 ul = acc[i][2 * t + FRN / 2], uh = acc[i][2 * t + 1 + FRN / 2];
-        const float vg[8] = {gl[0], gl[1], gl[2], gl[3], gh[0], gh[1], gh[2], gh[3]};
-        const float vu[8] = {ul[0], ul[1], ul[2], ul[3], uh[0], uh[1], uh[2], uh[3]};
-        store_swiglu8<HALF>(vg, vu, g, orow + 16 * i, hcol + 32 * t);
-      }
+    store_gate_up<HALF, EDGE>(acc, g, m0 + wm * WTM, n0 + wn * (WTN / 2), lane);
   } else {
     // (the ring slot behind the last stage's two is free: no wave reads or fills it any more)
     store_blocks<EPI, OUT_F32, HALF, EDGE, ODD>(acc, g, split, m0 + wm * WTM, n0 + wn * WTN, lane,

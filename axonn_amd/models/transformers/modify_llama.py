@@ -8,10 +8,10 @@ forward passes to Hugging Face.  Here
 * the MLP is rebuilt the same way (`modified_mlp_init`, :76-95), and its forward
   `down_proj(act_fn(gate_proj(x)) * up_proj(x))` additionally runs the activation
   and the product as one kernel (`SwiGLU`, axn_swiglu_fwd / axn_swiglu_bwd) when
-  the activation is SiLU - or, for 16-bit layers without bias and whole-tile shapes,
-  both projections and the activation as one launch (`GateUpSwiGLU`,
-  axn_gemm_swiglu_fwd), with the same results bit for bit; so are up to 64 tokens without
-  gradients (axn_gemm_swiglu_fwd_few);
+  the activation is SiLU - or, for 16-bit layers without bias, both projections and the
+  activation as one launch (`GateUpSwiGLU`, axn_gemm_swiglu_fwd): whole-tile shapes, with the
+  same results bit for bit, other numbers of tokens beyond 64 where the products are large, and
+  up to 64 tokens without gradients (axn_gemm_swiglu_fwd_few);
 * the attention projections are swapped after the original constructor has run,
   instead of restating that constructor (:12-73): the constructor's other fields
   changed across transformers releases, the four projections did not.  At a
@@ -24,7 +24,7 @@ from transformers.models.llama.modeling_llama import LlamaAttention, LlamaMLP, A
 
 from axonn_amd import ops
 from axonn_amd.intra_layer import Linear
-from axonn_amd.intra_layer.fully_connected import _compute_dtype, _weight_grad
+from axonn_amd.intra_layer.fully_connected import _backward_products, _compute_dtype, _weight_grad
 
 _original_mlp_forward = None
 
@@ -63,8 +63,10 @@ class GateUpSwiGLU(torch.autograd.Function):
         dt = _compute_dtype(x, w_gate.reshape(shape))
         x2 = x.reshape(-1, x.shape[-1]).to(dt)
         needs_grad = save and any(ctx.needs_input_grad[:3])
-        h, gate, up = ops.gemm_swiglu_fwd(x2, w_gate.reshape(shape).to(dt), w_up.reshape(shape).to(dt),
-                                          save=needs_grad, few=not save and x2.shape[0] <= 64)
+        few = not save and x2.shape[0] <= 64
+        h, gate, up = ops.gemm_swiglu_fwd(
+            x2, w_gate.reshape(shape).to(dt), w_up.reshape(shape).to(dt), save=needs_grad, few=few,
+            any_sizes=not few and not ops.gemm_swiglu_supported(x2.shape[0], *shape, dt))
         ctx.save_for_backward(x2, w_gate, w_up, gate, up)
         ctx.shape, ctx.input_shape, ctx.compute_dtype = shape, x.shape, dt
         return h.reshape(*x.shape[:-1], shape[0])
@@ -79,6 +81,14 @@ class GateUpSwiGLU(torch.autograd.Function):
         # within +-3 % of them at the Llama-3-8B shape and was dropped.
         dgate, dup = ops.swiglu_bwd(d2, gate, up)
         grad_x = grad_wg = grad_wu = None
+        if not ops.gemm_dgrad_pair_supported(x2.shape[0], n, n, k, dt):
+            # as the two projections called by themselves, and autograd's sum
+            need = ctx.needs_input_grad
+            grad_x, grad_wg = _backward_products(dgate, w_gate.reshape(ctx.shape).to(dt), x2, w_gate, need[0], need[1])
+            dx_up, grad_wu = _backward_products(dup, w_up.reshape(ctx.shape).to(dt), x2, w_up, need[0], need[2])
+            if need[0]:
+                grad_x = (grad_x + dx_up).reshape(ctx.input_shape)
+            return grad_x, grad_wg, grad_wu, None, None
         if ctx.needs_input_grad[0]:
             # both products through one set of accumulators, rounded once (two products and
             # an add where the shape does not fit the one-pass kernel)
@@ -124,7 +134,10 @@ def _one_launch_gate_up(mlp, x):
     tokens = x.numel() // max(x.shape[-1], 1)
     sizes = tokens, g.local_out_features, g.local_in_features, dt
     if torch.is_grad_enabled() or tokens > 64:
-        return ops.gemm_swiglu_supported(*sizes)
+        # (a weight that autocast casts is kept for the backward pass by the projections themselves)
+        return ops.gemm_swiglu_supported(*sizes) or (
+            x.shape[-1] == g.local_in_features and ops.gemm_swiglu_any_supported(*sizes)
+            and (g.weight.dtype == u.weight.dtype == dt or not torch.is_grad_enabled()))
     return x.shape[-1] == g.local_in_features and ops.gemm_swiglu_few_supported(*sizes)
 
 

@@ -224,7 +224,10 @@ AXN_API int axn_pad_rows16_to(const void* src, void* dst, int64_t M, int64_t N, 
  * axn_gemm_fwd twice followed by axn_swiglu_fwd bit for bit.
  * Shapes: M % 256 == 0, N % 128 == 0, K % 64 == 0, every operand below 2 GiB
  * (AXN_ESHAPE otherwise: use the three separate calls); pointers 16-byte aligned,
- * leading dimensions multiples of 8. */
+ * leading dimensions multiples of 8.
+ * With dtype | AXN_ANY_SIZES: any M, N and K multiples of 8, operands of any size, row strides
+ * below 2^22 elements.  The results are those of products whose contraction is in one part. */
+#define AXN_ANY_SIZES 0x100
 AXN_API int axn_gemm_swiglu_fwd(const void* X, const void* Wg, const void* Wu, void* H,
                                 void* gate_save, void* up_save, int dtype, int64_t M, int64_t N,
                                 int64_t K, int64_t ldx, int64_t ldw, int64_t ldh, void* stream);

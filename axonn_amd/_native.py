@@ -21,6 +21,8 @@ AXN_ELIMIT = -5
 BF16, F16, F32 = 0, 1, 2
 EPI_NONE, EPI_BIAS, EPI_BIAS_GELU, EPI_GELU = 0, 1, 2, 3
 BIAS_16BIT = 0x100   # with an epilogue: the bias has the operands' 16-bit type
+DY_F32, DBIAS_16BIT = 0x100, 0x200   # with the dtype of axn_dgelu_dbias: dY is fp32; dbias is not
+ROUNDED = 0x100      # with F32 as an input gradient's output type: 16-bit values
 ANY_SIZES = 0x100    # with the dtype of axn_gemm_swiglu_fwd: sizes that are not made of whole tiles
 
 ABI_VERSION = 15   # another one with every change of the entry points below

@@ -371,6 +371,8 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void*
   rc = check_epilogue(name, epilogue, bias);
   if (rc) return rc;
   REQUIRE(fwd || epilogue == AXN_EPI_NONE, AXN_EINVAL, "%s: only the forward has an epilogue", name);
+  const bool widen = op == AXN_GEMM_DGRAD && out_dtype == (AXN_F32 | AXN_ROUNDED);
+  if (widen) out_dtype = dtype;
   REQUIRE(beta == 0 || (beta == 1 && wgrad), AXN_EINVAL, "%s: beta must be 0, or 1 for the weight gradient", name);
   REQUIRE(out_dtype == dtype ||
               (out_dtype == AXN_F32 && (wgrad || epilogue == AXN_EPI_BIAS || epilogue == AXN_EPI_BIAS_GELU)),
@@ -396,8 +398,16 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void*
     REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
     plan = gemm_plan(layout, g.M, g.N, g.Kc);
     if (plan.parts > 1)
-      return launch_gemm_splitk(layout, g, epilogue, half, out_f32, plan, (float*)workspace, (hipStream_t)stream);
+      return launch_gemm_splitk(layout, g, epilogue, half, out_f32, plan, (float*)workspace, (hipStream_t)stream, widen);
+    if (widen) {   // in one part after all: 16 bits into the workspace, which is larger than that
+      REQUIRE(ldc == K, AXN_ESHAPE, "%s: a rounded fp32 result has no gaps between its rows", name);
+      g.C = workspace;
+      rc = half ? launch_gemm_f16(layout, g, epilogue, false, (hipStream_t)stream)
+                : launch_gemm_bf16(layout, g, epilogue, false, (hipStream_t)stream);
+      return rc ? rc : launch_widen(workspace, (float*)C, half, M * K, (hipStream_t)stream);
+    }
   }
+  REQUIRE(!widen, AXN_EINVAL, "%s: a rounded fp32 result needs the workspace", name);
   return half ? launch_gemm_f16(layout, g, epilogue, out_f32, (hipStream_t)stream)
               : launch_gemm_bf16(layout, g, epilogue, out_f32, (hipStream_t)stream);
 }
@@ -564,20 +574,26 @@ int axn_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
                     float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
                     void* workspace, size_t workspace_bytes, void* stream) {
   const char* name = "axn_dgelu_dbias";
+  const bool wide = (dtype & AXN_DY_F32) != 0, dbias16 = (dtype & AXN_DBIAS_16BIT) != 0;
+  dtype &= ~(int)(AXN_DY_F32 | AXN_DBIAS_16BIT);
   REQUIRE(dY != nullptr, AXN_EINVAL, "%s: dY is null", name);
+  REQUIRE((!wide && !dbias16) || dtype == AXN_BF16 || dtype == AXN_F16, AXN_EINVAL,
+          "%s: an fp32 dY or a 16-bit dbias goes with a 16-bit dtype", name);
+  REQUIRE(!dbias16 || beta == 0, AXN_EINVAL, "%s: a 16-bit dbias is not added to", name);
+  REQUIRE(!wide || dZ != nullptr, AXN_EINVAL, "%s: an fp32 dY is rounded into dZ", name);
   REQUIRE(dtype == AXN_BF16 || dtype == AXN_F16 || dtype == AXN_F32, AXN_EINVAL,
           "%s: unknown dtype %d", name, dtype);
   REQUIRE(M >= 1 && N >= 1, AXN_EINVAL, "%s: M and N must be >= 1", name);
   REQUIRE(N % 8 == 0, AXN_ESHAPE, "%s: N must be a multiple of 8", name);
   REQUIRE(ld >= N && ld % 8 == 0, AXN_EALIGN,
           "%s: ld must be >= N and a multiple of 8", name);
-  REQUIRE((Z == nullptr) == (dZ == nullptr), AXN_EINVAL,
+  REQUIRE((Z == nullptr) == (dZ == nullptr) || (wide && dZ != nullptr), AXN_EINVAL,
           "%s: Z and dZ must be given together", name);
-  REQUIRE(Z != nullptr || dbias != nullptr, AXN_EINVAL, "%s: nothing to compute", name);
+  REQUIRE(Z != nullptr || dbias != nullptr || wide, AXN_EINVAL, "%s: nothing to compute", name);
   REQUIRE(aligned16(dY) && aligned16(Z) && aligned16(dZ), AXN_EALIGN,
           "%s: pointers must be 16-byte aligned", name);
   REQUIRE(beta == 0 || beta == 1, AXN_EINVAL, "%s: beta must be 0 or 1", name);
-  return launch_dgelu_dbias(dY, Z, dZ, dtype, dbias, M, N, ld, beta, workspace,
+  return launch_dgelu_dbias(dY, Z, dZ, dtype, wide, dbias, dbias16, M, N, ld, beta, workspace,
                             workspace_bytes, (hipStream_t)stream);
 }
 

@@ -181,8 +181,9 @@ SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, doubl
 // What a call with the workspace for gemm_splits' parts does: those parts on the tile that is estimated to be fastest,
 // or the contraction in one part where a smaller tile is faster still.
 SplitPlan gemm_plan(GemmLayout layout, int64_t M, int64_t N, int64_t Kc);
+// widen (input gradient): the result is rounded to the operands' type and stored as fp32.
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, int epilogue, bool half, bool out_f32,
-                       const SplitPlan& plan, float* ws, hipStream_t stream);
+                       const SplitPlan& plan, float* ws, hipStream_t stream, bool widen = false);
 // The parts of the input gradient's contraction if both gradients of a layer (dY[M][N], W[N][K], X[M][K]) are
 // estimated to be faster in one launch than in two, or 0; add: dW += ...; ws holds the parts, parts * M * K floats.
 int gemm_backward_parts(int64_t M, int64_t N, int64_t K, bool add);
@@ -252,9 +253,11 @@ size_t gemm_f32_workspace_bytes(GemmLayout layout, int64_t M, int64_t N, int64_t
 
 // ---- elementwise backward of the bias/GELU epilogue ----------------------
 size_t dgelu_dbias_workspace_bytes(int64_t M, int64_t N);
-int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
-                       float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
-                       void* ws, size_t ws_bytes, hipStream_t stream);
+// wide: dY is fp32, rounded to dtype; dbias16: dbias has dtype.
+int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype, bool wide, void* dbias, bool dbias16,
+                       int64_t M, int64_t N, int64_t ld, int beta, void* ws, size_t ws_bytes, hipStream_t stream);
+// dst = src, n (a multiple of 8) 16-bit elements as fp32.
+int launch_widen(const void* src, float* dst, bool half, int64_t n, hipStream_t stream);
 
 // dst[M][ld_dst] = src[M][N] (row stride ld) of 16-bit elements, zeros behind N; ld_dst a multiple of 8.
 int launch_pad_rows16(const void* src, void* dst, int64_t M, int64_t N, int64_t ld, int64_t ld_dst,

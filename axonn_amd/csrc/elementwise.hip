@@ -133,10 +133,14 @@ __device__ __forceinline__ unsigned column_group() {
   return TURN ? (at + (blockIdx.y & 7) * max(each, 1u)) % n : at;
 }
 
-template <typename T, bool HAS_Z>
+// WIDE: dY is fp32 (a 16-bit layer's fp32 bias makes its result, and so its gradient, fp32) and rounded to T on the way,
+// as a cast before this pass would round it; without Z the rounded values are stored.  A cast of its own reads dY once
+// more than that and its result is read twice: 3001 x 10240, fp16, sums alone: cast 34 us and 16.5 after it -> 37.
+template <typename T, bool HAS_Z, bool WIDE>
 __global__ void __launch_bounds__((DG_THREADS<T, HAS_Z>))
-    dgelu_dbias_kernel(const T* dY, const T* Z, T* dZ, float* partial, int64_t M, int64_t N, int64_t ld) {
+    dgelu_dbias_kernel(const void* dY, const T* Z, T* dZ, float* partial, int64_t M, int64_t N, int64_t ld) {
   typedef typename Raw8<T>::type raw;
+  static_assert(!WIDE || sizeof(T) == 2, "rounds to a 16-bit type");
   typedef typename Raw8<T>::element element;
   constexpr int ROWS = DG_THREADS<T, HAS_Z> / DG_PIECES;   // at a time
   static_assert(ROWS % 4 == 0 && DG_BAND % ROWS == 0 && DG_THREADS<T, HAS_Z> >= 4 * DG_COLS, "a thread for each phase and column");
@@ -155,7 +159,14 @@ __global__ void __launch_bounds__((DG_THREADS<T, HAS_Z>))
     const int64_t row = band0 + step * ROWS + row0;
     raw add = raw{}, factor = raw{};   // zeros outside
     if (row < M && col < N) {
-      add = *(const raw*)(dY + row * ld + col);
+      if constexpr (WIDE) {
+        const f32x8 wide = *(const f32x8*)((const float*)dY + row * ld + col);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) add[e] = (element)wide[e];
+        if constexpr (!HAS_Z) *(raw*)(dZ + row * ld + col) = add;
+      } else {
+        add = *(const raw*)((const T*)dY + row * ld + col);
+      }
       if constexpr (HAS_Z) {
         const raw z = *(const raw*)(Z + row * ld + col);
         raw out;
@@ -202,9 +213,11 @@ __global__ void __launch_bounds__((DG_THREADS<T, HAS_Z>))
 
 // Column sums over the band partials in a fixed order: 64 columns per workgroup, the bands split in 4
 // consecutive quarters summed by 4 threads each in band order (8 loads on their way), the quarters then
-// combined as (q0 + q1) + (q2 + q3).
+// combined as (q0 + q1) + (q2 + q3).  OUT: the sums' type (a 16-bit parameter's gradient straight away, where a cast
+// would be one more launch).
+template <typename OUT>
 __global__ void __launch_bounds__(256)
-    dbias_reduce_kernel(const float* partial, float* dbias, int64_t bands,
+    dbias_reduce_kernel(const float* partial, OUT* dbias, int64_t bands,
                         int64_t N, int beta) {
   __shared__ float red[4][64];
   const int tx = threadIdx.x & 63, q = threadIdx.x >> 6;
@@ -227,7 +240,7 @@ __global__ void __launch_bounds__(256)
   __syncthreads();
   if (q == 0 && c < N) {
     const float t = (red[0][tx] + red[1][tx]) + (red[2][tx] + red[3][tx]);
-    dbias[c] = beta ? dbias[c] + t : t;
+    dbias[c] = (OUT)(beta ? (float)dbias[c] + t : t);
   }
 }
 
@@ -336,9 +349,8 @@ size_t dgelu_dbias_workspace_bytes(int64_t M, int64_t N) {
   return (size_t)((M + DG_BAND - 1) / DG_BAND) * (size_t)N * sizeof(float);
 }
 
-int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
-                       float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
-                       void* ws, size_t ws_bytes, hipStream_t stream) {
+int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype, bool wide, void* dbias, bool dbias16,
+                       int64_t M, int64_t N, int64_t ld, int beta, void* ws, size_t ws_bytes, hipStream_t stream) {
   const int64_t bands = (M + DG_BAND - 1) / DG_BAND;
   float* partial = nullptr;
   if (dbias != nullptr) {
@@ -354,30 +366,62 @@ int launch_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
     set_error("dgelu_dbias: too many rows (%lld)", (long long)M);
     return AXN_ELIMIT;
   }
-#define AXN_DGELU(T, HAS_Z)                                                                                  \
-  hipLaunchKernelGGL((dgelu_dbias_kernel<T, HAS_Z>), grid, dim3(DG_THREADS<T, HAS_Z>), 0, stream, (const T*)dY, \
-                     (const T*)Z, (T*)dZ, partial, M, N, ld)
-#define AXN_DGELU_TYPE(T)    \
-  do {                       \
-    if (Z != nullptr)        \
-      AXN_DGELU(T, true);    \
-    else                     \
-      AXN_DGELU(T, false);   \
+#define AXN_DGELU(T, HAS_Z, WIDE)                                                                                       \
+  hipLaunchKernelGGL((dgelu_dbias_kernel<T, HAS_Z, WIDE>), grid, dim3(DG_THREADS<T, HAS_Z>), 0, stream, dY, (const T*)Z, \
+                     (T*)dZ, partial, M, N, ld)
+#define AXN_DGELU_TYPE(T, WIDE)  \
+  do {                           \
+    if (Z != nullptr)            \
+      AXN_DGELU(T, true, WIDE);  \
+    else                         \
+      AXN_DGELU(T, false, WIDE); \
   } while (0)
   if (dtype == AXN_F32)
-    AXN_DGELU_TYPE(float);
+    AXN_DGELU_TYPE(float, false);
+  else if (dtype == AXN_F16 && wide)
+    AXN_DGELU_TYPE(_Float16, true);
   else if (dtype == AXN_F16)
-    AXN_DGELU_TYPE(_Float16);
+    AXN_DGELU_TYPE(_Float16, false);
+  else if (wide)
+    AXN_DGELU_TYPE(uint16_t, true);
   else
-    AXN_DGELU_TYPE(uint16_t);
+    AXN_DGELU_TYPE(uint16_t, false);
 #undef AXN_DGELU_TYPE
 #undef AXN_DGELU
   AXN_HIP_TRY(hipGetLastError());
   if (dbias != nullptr) {
-    hipLaunchKernelGGL(dbias_reduce_kernel, grid_of((N + 63) / 64),
-                       dim3(256), 0, stream, partial, dbias, bands, N, beta);
+#define AXN_REDUCE(OUT) \
+  hipLaunchKernelGGL(dbias_reduce_kernel<OUT>, grid_of((N + 63) / 64), dim3(256), 0, stream, partial, (OUT*)dbias, bands, N, beta)
+    if (!dbias16)
+      AXN_REDUCE(float);
+    else if (dtype == AXN_F16)
+      AXN_REDUCE(_Float16);
+    else
+      AXN_REDUCE(__bf16);
+#undef AXN_REDUCE
     AXN_HIP_TRY(hipGetLastError());
   }
+  return AXN_OK;
+}
+
+// 16-bit elements as fp32: bound by its bytes.
+namespace {
+template <typename T>
+__global__ void __launch_bounds__(256) widen_kernel(const T* __restrict__ src, float* __restrict__ dst, int64_t n8) {
+  const int64_t i = block_number() * 256 + threadIdx.x;
+  if (i >= n8) return;
+  float x[8];
+  load8(src + i * 8, x);
+  store8(dst + i * 8, x);
+}
+}  // namespace
+int launch_widen(const void* src, float* dst, bool half, int64_t n, hipStream_t stream) {
+  const dim3 grid = grid_of((n / 8 + 255) / 256);
+  if (half)
+    hipLaunchKernelGGL(widen_kernel<_Float16>, grid, dim3(256), 0, stream, (const _Float16*)src, dst, n / 8);
+  else
+    hipLaunchKernelGGL(widen_kernel<uint16_t>, grid, dim3(256), 0, stream, (const uint16_t*)src, dst, n / 8);
+  AXN_HIP_TRY(hipGetLastError());
   return AXN_OK;
 }
 

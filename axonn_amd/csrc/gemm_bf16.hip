@@ -449,6 +449,11 @@ __global__ void __launch_bounds__(256)
     a1 += __builtin_nontemporal_load((const f32x4*)(p + 4));
   }
   float v[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+  if constexpr (EPI == EPI_WIDEN) {
+    using lp = std::conditional_t<HALF, _Float16, __bf16>;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (float)(lp)v[e];
+  }
   if (ANY && col + 8 > g.N) {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
@@ -466,7 +471,8 @@ int launch_reduce(const float* ws, const GemmArgs& g, int epilogue, bool out_f32
   const dim3 grid((unsigned)((lanes + 255) / 256)), block(256);
 #define REDUCE(EPI, F32) hipLaunchKernelGGL((splitk_reduce_kernel<EPI, F32, HALF, ANY>), grid, block, 0, stream, ws, g)
   if (out_f32) {
-    if (epilogue == AXN_EPI_BIAS) REDUCE(AXN_EPI_BIAS, true);
+    if (epilogue == EPI_WIDEN) REDUCE(EPI_WIDEN, true);
+    else if (epilogue == AXN_EPI_BIAS) REDUCE(AXN_EPI_BIAS, true);
     else if (epilogue == AXN_EPI_BIAS_GELU) REDUCE(AXN_EPI_BIAS_GELU, true);
     else REDUCE(AXN_EPI_NONE, true);
   } else {
@@ -792,7 +798,11 @@ static int launch_sum(const GemmArgs& in, int epilogue, bool half, bool out_f32,
 }
 
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool half, bool out_f32,
-                       const SplitPlan& plan, float* ws, hipStream_t stream) {
+                       const SplitPlan& plan, float* ws, hipStream_t stream, bool widen) {
+  if (widen) {
+    epilogue = EPI_WIDEN;
+    out_f32 = true;
+  }
   GemmArgs g = in;
   g.C = ws;
   g.ldc = ceil_div(g.N, 8) * 8;   // whole vectors a row

@@ -23,6 +23,8 @@ constexpr int EPI_SWIGLU = 100;
 // Internal: no epilogue, but the contraction runs through two operand pairs one after the
 // other (C = A B + A2 B2).
 constexpr int EPI_PAIR = 101;
+// Internal, of the sum of parts: the result rounded to the 16-bit type and stored as fp32.
+constexpr int EPI_WIDEN = 102;
 #define LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
 
 template <int... I, class F>

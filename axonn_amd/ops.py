@@ -201,8 +201,9 @@ def gemm_fwd(x, w, bias=None, activation=None, save_z=False, out_f32=False):
     return y, z
 
 
-def gemm_dgrad(dy, w):
-    """dX = dY W.  dy [M,N], w [N,K]."""
+def gemm_dgrad(dy, w, widen=False):
+    """dX = dY W.  dy [M,N], w [N,K].  widen: dX may come as fp32, its values rounded to the operands' type (where
+    the pass that adds the contraction's parts writes it so, instead of a cast behind it)."""
     _require_gpu(dy, w)
     if dy.dtype != w.dtype:
         raise TypeError("grad_output is %s but weight is %s" % (dy.dtype, w.dtype))
@@ -219,8 +220,13 @@ def gemm_dgrad(dy, w):
     if dy.dtype in _GEMM16:
         dy, lddy = _prep_bf16(dy)
         w, ldw = _prep_bf16(w)
-        dx = torch.empty((M, K), dtype=dy.dtype, device=dy.device)
         ws, ws_bytes = _split_workspace(GEMM_DGRAD, M, N, K, dy.device)
+        if widen and ws is not None and max(lddy, ldw) < _FAR_ROWS:
+            dx = torch.empty((M, K), dtype=torch.float32, device=dy.device)
+            nv.call("axn_gemm_any_n", GEMM_DGRAD, nv.ptr(dy), nv.ptr(w), None, nv.ptr(dx), None, nv.dtype_code(dy.dtype),
+                    M, N, K, lddy, ldw, K, nv.EPI_NONE, 0, nv.F32 | nv.ROUNDED, nv.ptr(ws), ws_bytes, nv.current_stream())
+            return dx
+        dx = torch.empty((M, K), dtype=dy.dtype, device=dy.device)
         if ws is not None:
             nv.call("axn_gemm_dgrad_ws", nv.ptr(dy), nv.ptr(w), nv.ptr(dx),
                     nv.dtype_code(dy.dtype), M, N, K, lddy, ldw, K, nv.ptr(ws), ws_bytes,
@@ -355,12 +361,12 @@ def _bwd_in_parts(dy, w, x, out, accumulate, out_dtype):
     return dx, out
 
 
-def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None):
+def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None, widen=False):
     """(dX, dW) = (dY W, dY^T X) of one layer, dW optionally accumulated into `out`: the two
     products of AsyncLinear.backward (axonn/intra_layer/fully_connected.py:140, :147-151)
     through ONE entry point, which runs both in a single launch where their tile counts
     would each leave CUs idle in a launch of their own.  Results equal gemm_dgrad and
-    gemm_wgrad bit for bit; shapes the joint entry points do not take go through those."""
+    gemm_wgrad bit for bit; shapes the joint entry points do not take go through those (widen: as gemm_dgrad)."""
     _require_gpu(dy, w, x, out)
     M, N = dy.shape
     K = w.shape[1]
@@ -381,7 +387,7 @@ def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None):
             out_dtype = out.dtype
         return _dgrad_any_n(dy8, w, N), _wgrad_any_n(dy8, x, N, out, accumulate, out_dtype or dy.dtype)
     if not plain16:
-        return gemm_dgrad(dy, w), gemm_wgrad(dy, x, out=out, accumulate=accumulate, out_dtype=out_dtype)
+        return gemm_dgrad(dy, w, widen), gemm_wgrad(dy, x, out=out, accumulate=accumulate, out_dtype=out_dtype)
     if x.shape != (M, K) or w.shape[0] != N:
         raise ValueError("shapes do not match: dY %s, W %s, X %s" % (tuple(dy.shape), tuple(w.shape),
                                                                      tuple(x.shape)))
@@ -412,10 +418,17 @@ def _dbias_workspace_bytes(M, N):
     return nv.load().axn_dgelu_dbias_workspace_bytes(M, N)
 
 
-def dgelu_dbias(dy, z=None, want_dbias=True, dbias_out=None, accumulate=False):
+def dgelu_dbias(dy, z=None, want_dbias=True, dbias_out=None, accumulate=False, dtype=None, dbias_dtype=None):
     """dZ = dY * gelu'(Z) (when z is given) and dbias = column sums of dZ (fp32).
-    Returns (dz, dbias); dz is dy itself when z is None."""
+    Returns (dz, dbias); dz is dy itself when z is None.  dtype (bf16 or fp16, with an fp32 dy): dy rounded to it, dz
+    of it.  dbias_dtype: dbias comes in it where the sums' kernel writes it (the type of a 16-bit dz), else in fp32."""
     _require_gpu(dy, z, dbias_out)
+    wide = dtype in _GEMM16 and dy.dtype == torch.float32
+    if wide and (dy.dim() != 2 or dy.shape[1] % 8 or dy.shape[0] == 0
+                 or (z is not None and (z.dtype != dtype or z.shape != dy.shape))):
+        dy, wide = dy.to(dtype), False
+    elif dtype is not None and not wide and dy.dtype != dtype:
+        dy = dy.to(dtype)
     if dy.dtype not in (torch.bfloat16, torch.float16, torch.float32):
         raise TypeError("bf16, fp16 or fp32 expected, got %s" % dy.dtype)
     if dy.dim() == 2 and dy.shape[1] % 8:   # ragged width: zero-padded columns, results cut back
@@ -448,24 +461,34 @@ def dgelu_dbias(dy, z=None, want_dbias=True, dbias_out=None, accumulate=False):
                 dbias.zero_()
         return (torch.empty_like(dy) if z is not None else dy), dbias
     if z is not None:
-        if z.dtype != dy.dtype or z.shape != dy.shape:
+        if not wide and (z.dtype != dy.dtype or z.shape != dy.shape):
             raise ValueError("z must match dy in dtype and shape")
         if not z.is_contiguous() or ld != N:
             z = z.contiguous()
             dy = dy.contiguous()
             ld = N
-        dz = torch.empty_like(dy)
+    elif wide and ld != N:
+        dy = dy.contiguous()
+        ld = N
+    if z is not None or wide:
+        dz = torch.empty((M, N), dtype=dtype if wide else dy.dtype, device=dy.device)
+    code = nv.dtype_code(dtype) | nv.DY_F32 if wide else nv.dtype_code(dy.dtype)
     dbias = None
     ws, ws_bytes = None, 0
-    if want_dbias:
+    if want_dbias and dbias_out is None and dbias_dtype in _GEMM16 and dbias_dtype == (dtype if wide else dy.dtype):
+        dbias = torch.empty(N, dtype=dbias_dtype, device=dy.device)
+        code |= nv.DBIAS_16BIT
+        ws_bytes = _dbias_workspace_bytes(M, N)
+        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dy.device)
+    elif want_dbias:
         dbias = dbias_out if dbias_out is not None else torch.empty(N, dtype=torch.float32, device=dy.device)
         if dbias.dtype != torch.float32 or dbias.numel() != N:
             raise ValueError("dbias must be fp32 with %d elements" % N)
         ws_bytes = _dbias_workspace_bytes(M, N)
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dy.device)
-    elif z is None:
+    elif z is None and not wide:
         return dy, None
-    nv.call("axn_dgelu_dbias", nv.ptr(dy), nv.ptr(z), nv.ptr(dz), nv.dtype_code(dy.dtype),
+    nv.call("axn_dgelu_dbias", nv.ptr(dy), nv.ptr(z), nv.ptr(dz), code,
             nv.ptr(dbias), M, N, ld, 1 if (accumulate and dbias_out is not None) else 0,
             nv.ptr(ws), ws_bytes, nv.current_stream())
     return (dz if dz is not None else dy), dbias

@@ -108,7 +108,12 @@ AXN_API int axn_gemm_wgrad(const void* dY, const void* X, void* dW, int64_t M,
  * AXN_F32), row stride ld; dbias is fp32.  N % 8 == 0, pointers 16-byte
  * aligned, ld % 8 == 0.  Deterministic: column partial sums go through
  * `workspace` (axn_dgelu_dbias_workspace_bytes, needed only when dbias is
- * given) and are reduced in a fixed order.  dZ may alias dY. */
+ * given) and are reduced in a fixed order.  dZ may alias dY.
+ * dtype | AXN_DY_F32 (16-bit types): dY is fp32 and rounded to dtype first (a 16-bit product
+ * with an fp32 bias has an fp32 result and gradient); dZ is required, and without Z receives
+ * the rounded dY.  dtype | AXN_DBIAS_16BIT (16-bit types, beta 0): dbias is of dtype. */
+#define AXN_DY_F32 0x100
+#define AXN_DBIAS_16BIT 0x200
 AXN_API int axn_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
                     float* dbias, int64_t M, int64_t N, int64_t ld, int beta,
                     void* workspace, size_t workspace_bytes, void* stream);
@@ -190,7 +195,10 @@ AXN_API int axn_gemm_wgrad_ws(const void* dY, const void* X, void* dW, int dtype
  *          multiple of 8 must be zero (axn_pad_rows16)
  * K, the other leading dimensions and pointers: as above.  workspace: axn_gemm_workspace_bytes(op,
  * M, N, K) bytes, or NULL for no split (less or misaligned is refused, for a forward of up to 64 rows
- * no split either); beta and an fp32 out_dtype as axn_gemm_wgrad. */
+ * no split either); beta and an fp32 out_dtype as axn_gemm_wgrad.
+ *   DGRAD with out_dtype AXN_F32 | AXN_ROUNDED and the workspace, ldc == K: the result is rounded to
+ *          dtype and stored as fp32 (the gradient of an fp32 input that was cast for the product). */
+#define AXN_ROUNDED 0x100
 #define AXN_BIAS_16BIT 0x100 /* with the epilogue: bias is of `dtype` instead of fp32 */
 AXN_API int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void* C,
                    void* Zsave, int dtype, int64_t M, int64_t N, int64_t K, int64_t lda,

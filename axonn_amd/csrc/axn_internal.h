@@ -103,8 +103,9 @@ struct GemmArgs {
   int64_t lda, ldb, ldc;
   int tiles_m, tiles_n;
   int beta;  // 0: C = AB ; 1: C += AB
-  // First workgroup of this problem in a launch that runs two problems (launch_gemm_backward).
-  int wg_first;
+  // First workgroup of this problem in a launch that runs two problems (launch_gemm_backward), and how many of its
+  // last tiles are four workgroups each.
+  int wg_first, quartered;
   // Split of the contraction over workgroups (splits > 1): workgroup id / tiles is the
   // split, which covers k_split contraction elements and writes its fp32 partial
   // product to C + split * M * ldc.  0 or 1: no split.

@@ -66,16 +66,33 @@ __global__ void __launch_bounds__(512) gemm_f16_rest_kernel(const GemmArgs g) {
 }
 
 // Weight gradient and input gradient of one layer in one launch, 256 x 256 tiles: the
-// workgroups [gw.wg_first, gw.wg_first + gw's tiles) compute dW = dY^T X, the others dX = dY W.
+// workgroups [gw.wg_first, gw.wg_first + gw's) compute dW = dY^T X, the others dX = dY W.
 // The host puts the problem with the longer tiles first; the dispatcher hands workgroups
 // out in index order, so a CU takes a tile of the other product as soon as it is free.
+// The second problem's last `quartered` tiles, those that would start when few are left, are four
+// workgroups of 128 x 128 each, in the same order of sums: a tile that one CU would work on alone ends in
+// less than half the time on four.  8192 x 5120 x 2560, 200 tiles of 128 stages and 320 of 80, the last 8
+// of them alone on 56 idle CUs: 363 -> 343 us; 4096 x 2560 x 2560 104 -> 90, 4096 x 14336 x 2560 434 -> 416.
+template <bool A_KMAJOR, bool B_KMAJOR, bool OUT_F32, bool HALF>
+__device__ __forceinline__ void backward_tile(const GemmArgs& g, int pid) {
+  const int whole = g.tiles_m * g.tiles_n - g.quartered;
+  int tm, tn;
+  if (pid < whole) {
+    tile_of_workgroup(pid, g.tiles_m, g.tiles_n, tm, tn);
+    solo_gemm<256, 256, A_KMAJOR, B_KMAJOR, AXN_EPI_NONE, OUT_F32, HALF>(g, tm, tn, 0);
+  } else {
+    const int q = pid - whole;
+    tile_of_workgroup(whole + q / 4, g.tiles_m, g.tiles_n, tm, tn);
+    solo_gemm<128, 128, A_KMAJOR, B_KMAJOR, AXN_EPI_NONE, OUT_F32, HALF>(g, 2 * tm + q % 4 / 2, 2 * tn + q % 2, 0);
+  }
+}
 template <bool HALF, bool DW_F32>
 __global__ void __launch_bounds__(256) gemm_backward_kernel(const GemmArgs gw, const GemmArgs gd) {
   const int b = (int)blockIdx.x;
-  if (b >= gw.wg_first && b < gw.wg_first + gw.tiles_m * gw.tiles_n)
-    solo_gemm<256, 256, false, false, AXN_EPI_NONE, DW_F32, HALF>(gw);
+  if (b >= gw.wg_first && b < gw.wg_first + gw.tiles_m * gw.tiles_n + 3 * gw.quartered)
+    backward_tile<false, false, DW_F32, HALF>(gw, b - gw.wg_first);
   else
-    solo_gemm<256, 256, true, false, AXN_EPI_NONE, false, HALF>(gd);
+    backward_tile<true, false, false, HALF>(gd, b - gd.wg_first);
 }
 
 // The gate/up forward of a gated MLP: silu(A B^T) * (A B2^T), 256 rows x 128 columns of
@@ -591,50 +608,62 @@ double stages_alone(long long tiles, long long stages) {
   return (double)((full + 1) * stages);
 }
 // The same for one launch that holds both problems, longer tiles first: every CU takes the
-// next tile when it is free (a heap of the CUs' busy times: a few thousand steps).
-double stages_together(long long t1, long long s1, long long t2, long long s2) {
+// next tile when it is free (a heap of the CUs' busy times: a few thousand steps).  The last `quartered` tiles of the
+// second problem are four of kQuarter of their stages each; last: how many of its tiles end with the launch.
+constexpr double kQuarter = 0.5;   // 0.45 to 0.55 us a stage of a 128 x 128 tile alone on its CU, 1.04 to 1.3 of a large one
+double stages_together(long long t1, long long s1, long long t2, long long s2, long long quartered = 0,
+                       long long* last = nullptr) {
   if (s1 < s2) {
     std::swap(t1, t2);
     std::swap(s1, s2);
   }
-  std::priority_queue<long long, std::vector<long long>, std::greater<long long>> cus;
+  std::priority_queue<double, std::vector<double>, std::greater<double>> cus;
   for (int c = 0; c < 256; ++c) cus.push(0);
-  long long end = 0;
-  auto place = [&](long long tiles, long long stages) {
+  double end = 0;
+  long long at_end = 0;
+  auto place = [&](long long tiles, double stages) {
     for (long long i = 0; i < tiles; ++i) {
-      const long long t = cus.top() + stages;
+      const double t = cus.top() + stages;
       cus.pop();
       cus.push(t);
+      if (t > end) at_end = 0;
       end = t > end ? t : end;
+      if (t == end) ++at_end;
     }
   };
-  place(t1, s1);
-  place(t2, s2);
-  return (double)end;
+  place(t1, (double)s1);
+  place(t2 - quartered, (double)s2);
+  place(4 * quartered, kQuarter * (double)s2);
+  if (last != nullptr) *last = at_end;
+  return end;
 }
 
 // Whether two tile sets run in one launch; the answers for the last few shapes of a thread
 // are kept, a training loop asks for the same ones again and again.  The key holds all that
 // `ends_earlier` looks at.
+struct Together {
+  bool together;
+  int quartered = 0;
+};
 struct PlannedTogether {
   long long key[4];
-  bool together;
+  Together plan;
 };
 template <class F>
-bool plan_together(PlannedTogether (&plans)[4], int& next, long long k0, long long k1, long long k2, long long k3,
-                   F&& ends_earlier) {
+Together plan_together(PlannedTogether (&plans)[4], int& next, long long k0, long long k1, long long k2, long long k3,
+                       F&& ends_earlier) {
   for (const PlannedTogether& p : plans)
-    if (p.key[0] == k0 && p.key[1] == k1 && p.key[2] == k2 && p.key[3] == k3) return p.together;
+    if (p.key[0] == k0 && p.key[1] == k1 && p.key[2] == k2 && p.key[3] == k3) return p.plan;
   PlannedTogether& p = plans[next];
   next = (next + 1) % 4;
   p = {{k0, k1, k2, k3}, ends_earlier()};
-  return p.together;
+  return p.plan;
 }
 // The problem with the longer tiles takes the first workgroups.
 void place_together(GemmArgs& gd, GemmArgs& gw, long long td, long long tw, long long sd, long long sw) {
   gw.tiles_m = (int)ceil_div(gw.M, 256), gw.tiles_n = (int)ceil_div(gw.N, 256), gw.wg_first = sw >= sd ? 0 : (int)td;
   gd.tiles_m = (int)ceil_div(gd.M, 256), gd.tiles_n = (int)ceil_div(gd.N, 256), gd.wg_first = sw >= sd ? (int)tw : 0;
-  gw.splits = gd.splits = 0;
+  gw.splits = gd.splits = gw.quartered = gd.quartered = 0;
 }
 
 template <bool HALF>
@@ -653,12 +682,18 @@ int launch_backward(const GemmArgs& gd_in, const GemmArgs& gw_in, bool dw_f32, h
     // MI355X at 8192 x 5120 x 2560: 320 tiles of 80 stages and 200 of 128)
     static thread_local PlannedTogether plans[4] = {};
     static thread_local int next_plan = 0;
-    const bool together = plan_together(plans, next_plan, td, tw, sd, sw, [&] {
-      return td + tw <= 4096 &&
-             stages_together(tw, sw, td, sd) < 0.95 * (stages_alone(td, sd) + stages_alone(tw, sw));
+    const Together plan = plan_together(plans, next_plan, td, tw, sd, sw, [&]() -> Together {
+      if (td + tw > 4096) return {false};
+      long long last = 0;
+      const double end = stages_together(tw, sw, td, sd, 0, &last);
+      if (end >= 0.95 * (stages_alone(td, sd) + stages_alone(tw, sw))) return {false};
+      // few tiles that end the launch: a quarter each where that ends it 5 % earlier
+      const bool few = last <= 64 && last < (sw >= sd ? td : tw);
+      return {true, few && stages_together(tw, sw, td, sd, last) < 0.95 * end ? (int)last : 0};
     });
-    if (together) {
+    if (plan.together) {
       place_together(gd, gw, td, tw, sd, sw);
+      (sw >= sd ? gd : gw).quartered = plan.quartered;
       constexpr size_t lds = 5 * 256 * 64 * 2;
       void (*kern)(const GemmArgs, const GemmArgs) =
           dw_f32 ? gemm_backward_kernel<HALF, true> : gemm_backward_kernel<HALF, false>;
@@ -667,7 +702,7 @@ int launch_backward(const GemmArgs& gd_in, const GemmArgs& gw_in, bool dw_f32, h
         const int rc = allow_lds((const void*)kern, lds, lds_allowed[dw_f32 ? 1 : 0]);
         if (rc != AXN_OK) return rc;
       }
-      hipLaunchKernelGGL(kern, dim3((unsigned)(tw + td)), dim3(256), lds, stream, gw, gd);
+      hipLaunchKernelGGL(kern, dim3((unsigned)(tw + td + 3 * plan.quartered)), dim3(256), lds, stream, gw, gd);
       AXN_HIP_TRY(hipGetLastError());
       return AXN_OK;
     }
@@ -682,14 +717,14 @@ int launch_backward(const GemmArgs& gd_in, const GemmArgs& gw_in, bool dw_f32, h
     const long long sd = ceil_div(gd.Kc, 64), sw = ceil_div(gw.Kc, 64);
     static thread_local PlannedTogether plans[4] = {};
     static thread_local int next_plan = 0;
-    const bool together = plan_together(plans, next_plan, gd.M, gd.N, gd.Kc, 0, [&] {
-      if (td + tw > 4096) return false;
+    const Together plan = plan_together(plans, next_plan, gd.M, gd.N, gd.Kc, 0, [&]() -> Together {
+      if (td + tw > 4096) return {false};
       double ud = 0, uw = 0;
       edge_tile(gd.M, gd.N, gd.Kc, {}, &ud);
       edge_tile(gw.M, gw.N, gw.Kc, {}, &uw);
-      return 1.084 * stages_together(tw, sw, td, sd) + 15 < 0.95 * (ud + uw);
+      return {1.084 * stages_together(tw, sw, td, sd) + 15 < 0.95 * (ud + uw)};
     });
-    if (together) {
+    if (plan.together) {
       place_together(gd, gw, td, tw, sd, sw);
       return HALF ? launch_gemm_edge_backward_f16(gw, gd, dw_f32, stream)
                   : launch_gemm_edge_backward_bf16(gw, gd, dw_f32, stream);

@@ -606,7 +606,7 @@ __device__ __forceinline__ void store_gate_up(f32x4 (&acc)[FRM][FRN], const Gemm
 //     compiler converts what both store ahead of their branch, and spills).
 template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF,
           bool EDGE = false, bool ODD = false>
-__device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
+__device__ __forceinline__ void solo_gemm(const GemmArgs& g, const int tm, const int tn, const int split) {
   constexpr uint32_t kOutside = 0x80000000u;
   constexpr int WTM = BM / 2, WTN = BN / 2, FRM = BM / 32, FRN = BN / 32;
   constexpr int PK = 64, NSLOT = 5;
@@ -641,16 +641,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
 
   f32x4 acc[FRM][FRN];
 
-  // This workgroup's tile and, for a split contraction, its part: KP stages from stage s0 on.
-  int tm, tn, split = 0;
-  {
-    int pid = blockIdx.x - g.wg_first;
-    if (g.splits > 1) {
-      split = pid / (g.tiles_m * g.tiles_n);
-      pid -= split * (g.tiles_m * g.tiles_n);
-    }
-    tile_of_workgroup(pid, g.tiles_m, g.tiles_n, tm, tn);
-  }
+  // tm, tn: this workgroup's tile; for a split contraction its part, KP stages from stage s0 on.
   const int m0 = tm * BM, n0 = tn * (SWIGLU ? BN / 2 : BN);
   int KP, s0;
   if constexpr (EDGE) {
@@ -923,6 +914,19 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
     store_blocks<EPI, OUT_F32, HALF, EDGE, ODD>(acc, g, split, m0 + wm * WTM, n0 + wn * WTN, lane,
                                                 (float*)(lds + sa) + wave * (WTM * 8));
   }
+}
+
+// The tile, and the part of the contraction, of a workgroup of a launch of its own or of a range of one.
+template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF,
+          bool EDGE = false, bool ODD = false>
+__device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
+  int tm, tn, split = 0, pid = blockIdx.x - g.wg_first;
+  if (g.splits > 1) {
+    split = pid / (g.tiles_m * g.tiles_n);
+    pid -= split * (g.tiles_m * g.tiles_n);
+  }
+  tile_of_workgroup(pid, g.tiles_m, g.tiles_n, tm, tn);
+  solo_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, EDGE, ODD>(g, tm, tn, split);
 }
 
 // The dynamic LDS size a kernel may ask for is an attribute of the kernel on a device: set

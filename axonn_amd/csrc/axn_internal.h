@@ -179,8 +179,8 @@ struct SplitPlan {
   EdgeTile tile;
 };
 SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, double* us = nullptr);
-// What a call with the workspace for gemm_splits' parts does: those parts on the tile that is estimated to be fastest,
-// or the contraction in one part where a smaller tile is faster still.
+// What a call with the workspace for gemm_splits' parts does: those parts or fewer, on the tile that is estimated to
+// be fastest.
 SplitPlan gemm_plan(GemmLayout layout, int64_t M, int64_t N, int64_t Kc);
 // widen (input gradient): the result is rounded to the operands' type and stored as fp32.
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, int epilogue, bool half, bool out_f32,

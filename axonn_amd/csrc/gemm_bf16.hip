@@ -320,15 +320,56 @@ int launch_fed(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32,
               : launch_gemm_fed_nn_tn_bf16(layout, g, out_f32, tile, stream);
 }
 
+// `full` whole tile columns, or rows, of 256 x 256 tiles and the rest of a problem, or false if no cut gives them.
+bool cut_problem(GemmLayout layout, const GemmArgs& g, bool out_f32, long long full, GemmArgs& g1, GemmArgs& g2) {
+  const long long tm = ceil_div(g.M, 256), tn = ceil_div(g.N, 256);
+  const int64_t esz = out_f32 ? 4 : 2;
+  g1 = g2 = g;
+  if (full % tm == 0) {  // whole tile columns
+    const int64_t n1 = full / tm * 256;
+    g1.N = (int)n1;
+    g2.N = g.N - (int)n1;
+    g2.B = layout == GEMM_NT ? g.B + n1 * g.ldb : g.B + n1;
+    if (g.B2 != nullptr) g2.B2 = layout == GEMM_NT ? g.B2 + n1 * g.ldb : g.B2 + n1;
+    g2.C = (char*)g.C + n1 * esz;
+    g2.bias = bias_at(g, n1);
+    if (g.Z != nullptr) g2.Z = g.Z + n1;
+    return true;
+  }
+  if (full % tn != 0) return false;
+  const int64_t m1 = full / tn * 256;   // whole tile rows
+  g1.M = (int)m1;
+  g2.M = g.M - (int)m1;
+  g2.A = layout == GEMM_TN ? g.A + m1 : g.A + m1 * g.lda;
+  if (g.A2 != nullptr) g2.A2 = layout == GEMM_TN ? g.A2 + m1 : g.A2 + m1 * g.lda;
+  g2.C = (char*)g.C + m1 * g.ldc * esz;
+  if (g.Z != nullptr) g2.Z = g.Z + m1 * g.ldc;
+  return true;
+}
+
+// Full rounds and the rest, as launch_shape cuts whole-tile problems: a last round of at most half of the CUs goes to
+// smaller tiles in a launch of its own (2048 x 50257 over 2048, 40 tiles of 1576 left: 128 x 128 tiles
+// two to a CU 30 us, fed ones 21; weight gradient 24, 22).
 int launch_edge(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, bool half,
                 hipStream_t stream) {
   const int64_t ld = g.lda > g.ldb ? g.lda : g.ldb;
   if (ld >= kEdgeMaxLd) return launch_gemm_far(layout, g, epilogue, out_f32, half, stream);
-  const EdgeTile tile = ld >= kEdgeMaxLd / 2
-                            ? EDGE_128x128
-                            : edge_tile(g.M, g.N, g.Kc, epilogue_time(g, epilogue, out_f32));
-  return half ? launch_gemm_edge_f16(layout, g, epilogue, out_f32, tile, stream)
-              : launch_gemm_edge_bf16(layout, g, epilogue, out_f32, tile, stream);
+  const auto launch = [&](const GemmArgs& a, EdgeTile tile) {
+    return half ? launch_gemm_edge_f16(layout, a, epilogue, out_f32, tile, stream)
+                : launch_gemm_edge_bf16(layout, a, epilogue, out_f32, tile, stream);
+  };
+  if (ld >= kEdgeMaxLd / 2) return launch(g, EDGE_128x128);
+  const EdgeTile tile = edge_tile(g.M, g.N, g.Kc, epilogue_time(g, epilogue, out_f32));
+  const long long tiles = ceil_div(g.M, 256) * ceil_div(g.N, 256), full = tiles / 256 * 256, rest = tiles - full;
+  GemmArgs g1, g2;
+  if (tile == EDGE_256x256 && full > 0 && rest > 0 && rest <= 128 && cut_problem(layout, g, out_f32, full, g1, g2)) {
+    const int rc = launch(g1, tile);
+    if (rc != AXN_OK) return rc;
+    if (const FedTile* t = fed_tile(layout, g2, epilogue, out_f32))
+      return launch_fed(layout, g2, epilogue, out_f32, half, t->tile, stream);
+    return launch(g2, rest > 64 ? EDGE_256x128 : EDGE_128x128);
+  }
+  return launch(g, tile);
 }
 
 // Kernel selection.  Problems made of whole 256 x 256 tiles, more than 128 of
@@ -393,33 +434,12 @@ int launch_shape(const GemmArgs& g, hipStream_t stream) {
     if (g.ldc % 8 != 0) return launch_edge(order, g, EPI, OUT_F32, HALF, stream);
   }
   if (g.M % 256 == 0 && g.N % 256 == 0 && g.Kc % 64 == 0 && g.splits <= 1) {
-    const long long tm = g.M / 256, tn = g.N / 256, tiles = tm * tn;
+    const long long tiles = (long long)(g.M / 256) * (g.N / 256);
     const long long full = tiles / 256 * 256, rest = tiles - full;
     if (full > 0 && rest > 0 && rest <= 128) {
-      constexpr int64_t esz = OUT_F32 ? 4 : 2;
-      GemmArgs g1 = g, g2 = g;
-      bool cut = false;
-      if (full % tm == 0) {  // whole tile columns
-        const int64_t n1 = full / tm * 256;
-        g1.N = (int)n1;
-        g2.N = g.N - (int)n1;
-        g2.B = BKM ? g.B + n1 * g.ldb : g.B + n1;
-        if (g.B2 != nullptr) g2.B2 = BKM ? g.B2 + n1 * g.ldb : g.B2 + n1;
-        g2.C = (char*)g.C + n1 * esz;
-        g2.bias = bias_at(g, n1);
-        if (g.Z != nullptr) g2.Z = g.Z + n1;
-        cut = true;
-      } else if (full % tn == 0) {  // whole tile rows
-        const int64_t m1 = full / tn * 256;
-        g1.M = (int)m1;
-        g2.M = g.M - (int)m1;
-        g2.A = AK ? g.A + m1 * g.lda : g.A + m1;
-        if (g.A2 != nullptr) g2.A2 = AK ? g.A2 + m1 * g.lda : g.A2 + m1;
-        g2.C = (char*)g.C + m1 * g.ldc * esz;
-        if (g.Z != nullptr) g2.Z = g.Z + m1 * g.ldc;
-        cut = true;
-      }
-      if (cut) {
+      GemmArgs g1, g2;
+      constexpr GemmLayout order = !AK ? GEMM_TN : BKM ? GEMM_NT : GEMM_NN;
+      if (cut_problem(order, g, OUT_F32, full, g1, g2)) {
         const int rc = launch_whole<AK, BKM, EPI, OUT_F32, HALF>(g1, stream);
         if (rc != AXN_OK) return rc;
         // More than 64 tiles left: 256 x 128 tiles, one per CU on more than half of the CUs
@@ -431,7 +451,6 @@ int launch_shape(const GemmArgs& g, hipStream_t stream) {
         if (rest > 64 && a_span < (1LL << 31) && b_span < (1LL << 31))
           return launch_rest<AK, BKM, EPI, OUT_F32, HALF>(g2, stream);
         if constexpr (EPI != EPI_PAIR) {
-          constexpr GemmLayout order = !AK ? GEMM_TN : BKM ? GEMM_NT : GEMM_NN;
           if (const FedTile* t = fed_tile(order, g2, EPI, OUT_F32))
             return launch_fed(order, g2, EPI, OUT_F32, HALF, t->tile, stream);
         }
@@ -803,21 +822,23 @@ static double sum_microseconds(int64_t M, int64_t N, int parts) {
 }
 
 SplitPlan gemm_plan(GemmLayout layout, int64_t M, int64_t N, int64_t Kc) {
-  double other = 0, us = 0, one = 0;
+  double other = 0;
   SplitPlan plan = gemm_splits(layout, M, N, Kc, &other);
   if (plan.parts <= 1) return plan;
-  other = 0.95 * other_microseconds(layout, other, M, N);
-  if (const FedTile* t = best_fed_tile(layout, M, N, Kc, plan.parts, 0, &us)) {
-    us += sum_microseconds(M, N, plan.parts);
-    if (us < other) {
-      other = us;
-      plan.tile = t->tile;
+  double least = 0.95 * other_microseconds(layout, other, M, N);
+  // The input gradient of a layer whose gradients take one launch keeps the parts it has there.
+  const bool kept = layout == GEMM_NN && (gemm_backward_parts(M, Kc, N, false) > 0 || gemm_backward_parts(M, Kc, N, true) > 0);
+  const int most = plan.parts;   // what the workspace holds
+  for (int parts = kept ? most : 1; parts <= most; ++parts) {
+    double us = 0;
+    const FedTile* t = best_fed_tile(layout, M, N, Kc, parts, 0, &us);
+    if (t == nullptr) continue;
+    if (parts > 1) us += sum_microseconds(M, N, parts);
+    if (us < least) {
+      least = us;
+      plan = {parts, t->tile};
     }
   }
-  // The input gradient of a layer whose gradients take one launch keeps the parts it has there.
-  if (best_fed_tile(layout, M, N, Kc, 1, 0, &one) != nullptr && one < other &&
-      !(layout == GEMM_NN && (gemm_backward_parts(M, Kc, N, false) > 0 || gemm_backward_parts(M, Kc, N, true) > 0)))
-    plan.parts = 1;
   return plan;
 }
 

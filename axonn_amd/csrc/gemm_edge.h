@@ -68,38 +68,10 @@ int launch_edge_tile(const GemmArgs& in, hipStream_t stream) {
   return AXN_OK;
 }
 
-// Full rounds and the rest, as launch_shape of gemm_bf16.hip cuts whole-tile problems: a last
-// round of at most half of the CUs goes to smaller tiles in a launch of its own.
 template <bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
 int launch_edge_kind(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
   if (tile == EDGE_128x128) return launch_edge_tile<128, 128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
   if (tile == EDGE_256x128) return launch_edge_tile<256, 128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
-  const long long tm = ceil_div(g.M, 256), tn = ceil_div(g.N, 256), tiles = tm * tn;
-  const long long full = tiles / 256 * 256, rest = tiles - full;
-  if (g.splits <= 1 && full > 0 && rest > 0 && rest <= 128 && (full % tm == 0 || full % tn == 0)) {
-    constexpr int64_t esz = OUT_F32 ? 4 : 2;
-    GemmArgs g1 = g, g2 = g;
-    if (full % tm == 0) {  // whole tile columns
-      const int64_t n1 = full / tm * 256;
-      g1.N = (int)n1;
-      g2.N = g.N - (int)n1;
-      g2.B = BKM ? g.B + n1 * g.ldb : g.B + n1;
-      g2.C = (char*)g.C + n1 * esz;
-      g2.bias = bias_at(g, n1);
-      if (g.Z != nullptr) g2.Z = g.Z + n1;
-    } else {  // whole tile rows
-      const int64_t m1 = full / tn * 256;
-      g1.M = (int)m1;
-      g2.M = g.M - (int)m1;
-      g2.A = AK ? g.A + m1 * g.lda : g.A + m1;
-      g2.C = (char*)g.C + m1 * g.ldc * esz;
-      if (g.Z != nullptr) g2.Z = g.Z + m1 * g.ldc;
-    }
-    const int rc = launch_edge_tile<256, 256, AK, BKM, EPI, OUT_F32, HALF>(g1, stream);
-    if (rc != AXN_OK) return rc;
-    return rest > 64 ? launch_edge_tile<256, 128, AK, BKM, EPI, OUT_F32, HALF>(g2, stream)
-                     : launch_edge_tile<128, 128, AK, BKM, EPI, OUT_F32, HALF>(g2, stream);
-  }
   return launch_edge_tile<256, 256, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
 }
 

@@ -6,6 +6,8 @@ library is missing, loading raises, and every compute entry point needs a GPU.
 """
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -110,6 +112,9 @@ SYMBOLS = {
 
 _lib = None
 _probe_lib = None
+# axn_fast.so (csrc/fast.cpp): the host side of the usual Linear calls, same kernels.  None before `load` and where it is
+# not built: every caller then goes the general way, which it also goes where a function of `fast` answers None.
+fast = None
 _lock = threading.Lock()
 
 
@@ -125,9 +130,25 @@ def lib_path():
     return _LIB_PATH
 
 
+def _load_fast(lib):
+    path = os.path.join(os.path.dirname(_LIB_PATH), "axn_fast.so")
+    if not os.path.exists(path):
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("axn_fast", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("axn_fast", loader))
+    loader.exec_module(module)
+    if module.ABI_VERSION != ABI_VERSION:
+        raise ImportError("axn_fast.so has ABI version %d, this package needs %d" % (module.ABI_VERSION, ABI_VERSION))
+    import torch
+
+    dtype_code(torch.float32)   # (fills the table that callers of `fast` look types up in)
+    module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in module.entry_points()})
+    return module
+
+
 def load():
     """Loads the library once and types its entry points.  Raises if it is absent."""
-    global _lib
+    global _lib, fast
     if _lib is not None:
         return _lib
     with _lock:
@@ -155,6 +176,7 @@ def load():
             fn = getattr(lib, name)
             fn.restype = restype
             fn.argtypes = argtypes
+        fast = _load_fast(lib)
         _lib = lib
     return _lib
 

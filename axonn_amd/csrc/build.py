@@ -1,5 +1,7 @@
 """Builds libaxn_gfx950.so (the product library) and libaxn_probe_gfx950.so (streaming
-yardsticks for benchmarks, include/axn_probe.h) from the HIP sources in this directory.
+yardsticks for benchmarks, include/axn_probe.h) from the HIP sources in this directory, and
+axn_fast.so (fast.cpp), the host side of the usual Linear calls, with the host compiler
+against the headers of the PyTorch that imports it.
 
     python -m axonn_amd.csrc.build
 
@@ -11,6 +13,7 @@ runtime PyTorch has already loaded.
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -18,6 +21,7 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 LIB_DIR = os.path.join(os.path.dirname(HERE), "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libaxn_gfx950.so")
 PROBE_LIB_PATH = os.path.join(LIB_DIR, "libaxn_probe_gfx950.so")
+FAST_PATH = os.path.join(LIB_DIR, "axn_fast.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = ["axn_api.hip", "gemm_bf16.hip", "gemm_edge_bf16.hip", "gemm_edge_f16.hip",
@@ -54,6 +58,22 @@ def _run(cmd):
     return out
 
 
+def build_fast():
+    """Compiles and links axn_fast.so.  Its libraries are PyTorch's, found by soname in the process that has them."""
+    import torch
+
+    base = os.path.dirname(torch.__file__)
+    tmp = FAST_PATH + ".tmp"
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+          "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
+          *("-isystem" + d for d in (os.path.join(base, "include"), os.path.join(base, "include", "torch", "csrc", "api", "include"),
+                                     os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+                                     sysconfig.get_paths()["include"])),
+          "-I" + os.path.join(ROOT, "include"), os.path.join(HERE, "fast.cpp"), "-o", tmp, "-L" + os.path.join(base, "lib"),
+          "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"])
+    os.replace(tmp, FAST_PATH)   # (a running process keeps the file it has mapped)
+
+
 def build_library(verbose=False, extra_flags=()):
     """Compiles every source and links the shared library; returns its path."""
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -67,8 +87,10 @@ def build_library(verbose=False, extra_flags=()):
         return obj
 
     every = SOURCES + PROBE_SOURCES
-    with ThreadPoolExecutor(max_workers=min(len(every), os.cpu_count() or 1)) as pool:
+    with ThreadPoolExecutor(max_workers=min(len(every) + 1, os.cpu_count() or 1)) as pool:
+        fast = pool.submit(build_fast)
         objs = list(pool.map(compile_one, every))
+        fast.result()
     for path, part in ((LIB_PATH, objs[:len(SOURCES)]), (PROBE_LIB_PATH, objs[len(SOURCES):])):
         out = _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *part, "-o", path])
         if verbose and out.strip():

@@ -157,6 +157,10 @@ def gemm_fwd(x, w, bias=None, activation=None, save_z=False, out_f32=False):
     save_z).  out_f32 (16-bit operands with a bias): y is fp32, the sum with the fp32
     bias left unrounded, as type promotion leaves the reference's `x + bias`
     (axonn/intra_layer/fully_connected.py:348) under autocast."""
+    if nv.fast is not None and activation in (None, "gelu"):
+        done = nv.fast.gemm_fwd(x, w, bias, activation is not None, save_z, out_f32)
+        if done is not None:
+            return done
     _require_gpu(x, w, bias)
     if x.dtype != w.dtype:
         raise TypeError("input is %s but weight is %s" % (x.dtype, w.dtype))
@@ -367,6 +371,11 @@ def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None, widen=False):
     through ONE entry point, which runs both in a single launch where their tile counts
     would each leave CUs idle in a launch of their own.  Results equal gemm_dgrad and
     gemm_wgrad bit for bit; shapes the joint entry points do not take go through those (widen: as gemm_dgrad)."""
+    if (out is None) == (not accumulate):
+        dw_dtype = out.dtype if out is not None else out_dtype or dy.dtype
+        done = layer_bwd(dy, None, w, x, out, True, True, False, None, dw_dtype, widen)
+        if done is not None:
+            return done[0], (done[1].view(w.shape) if out is None else out)
     _require_gpu(dy, w, x, out)
     M, N = dy.shape
     K = w.shape[1]
@@ -411,6 +420,17 @@ def gemm_bwd(dy, w, x, out=None, accumulate=False, out_dtype=None, widen=False):
             M, N, K, lddy, ldw, ldx, K, K, 1 if accumulate else 0, nv.dtype_code(out_dtype),
             nv.current_stream())
     return dx, out
+
+
+def layer_bwd(dy, z, w, x, out, need_dx, need_dw, want_dbias, bias_dtype, dw_dtype, widen=False):
+    """The backward of one layer, act(x W^T + b), in one call: dgelu_dbias and then the products, as the functions above
+    and below launch them (dW is added to `out` if that is given).  (dX, dW, dbias), dW flat, None for what is not
+    wanted; or None for operands that are not dense, aligned and of usual sizes, which take those functions."""
+    if nv.fast is None:
+        return None
+    codes = nv._DTYPE_CODES
+    return nv.fast.backward(dy, z, w, x, out, need_dx, need_dw, want_dbias, codes.get(bias_dtype, nv.F32),
+                            codes.get(dw_dtype, -1), widen)
 
 
 @functools.lru_cache(maxsize=4096)

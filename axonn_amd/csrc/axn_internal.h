@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "axn.h"
 
 namespace axn {
@@ -304,5 +306,18 @@ int launch_mt_scale(void* const* h_g, const int64_t* h_sizes, int64_t n,
                     int g_dtype, float inv_scale, const axn_scan_result* scan,
                     int use_clip, hipStream_t stream);
 
+
+// The dynamic LDS size a kernel may ask for is an attribute of the kernel on a device: set
+// on a kernel's first launch on each device, not on every launch.  `done` is the
+// per-kernel-instance record (one bit per device).
+inline int allow_lds(const void* kern, size_t lds, std::atomic<unsigned long long>& done) {
+  int dev = 0;
+  AXN_HIP_TRY(hipGetDevice(&dev));
+  const unsigned long long bit = 1ull << (dev & 63);
+  if (done.load(std::memory_order_acquire) & bit) return AXN_OK;
+  AXN_HIP_TRY(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  done.fetch_or(bit, std::memory_order_release);
+  return AXN_OK;
+}
 
 }  // namespace axn

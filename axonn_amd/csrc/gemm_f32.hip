@@ -3,8 +3,9 @@
 // same three products as the bf16 path (fully_connected.py:118, :140, :147-151)
 // with fp32 operands, for any M, N, K >= 1.
 //
-// Two kernels.  gemm_f32_split_kernel forms each fp32 product from six bf16 products on LDS
-// tiles and carries the large problems; gemm_f32_kernel uses the fp32 matrix instruction.
+// Three kernels.  gemm_f32_split_kernel forms each fp32 product from six bf16 products on LDS
+// tiles and carries the large problems; gemm_f32_kernel and gemm_f32_copied_kernel use the fp32 matrix
+// instruction, in the same order of sums: they give the same bits.
 //
 // gemm_f32_kernel: one wave per workgroup owns a (16 FM) x (16 FN) output tile and feeds
 // v_mfma_f32_16x16x4_f32 (true fp32 products, fp32 accumulate) straight from
@@ -19,7 +20,11 @@
 //     per contraction index (the lane's FM consecutive rows), and
 //   * a lane stores FN consecutive output columns at once.
 // Its tiles are chosen for many waves (latency hiding by occupancy and by U blocks of loads
-// in flight per wave).
+// in flight per wave).  It takes any size and alignment, and is left with the short contractions of the rest.
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
 #include "axn_internal.h"
 
 namespace axn {
@@ -172,6 +177,60 @@ __device__ __forceinline__ bool tiny_operands(const float* __restrict__ A, const
   return tiny;
 }
 
+// Stores FN results of a row, columns bcol ...
+template <int EPI, int FN, bool VEC>
+__device__ __forceinline__ void store_row(float (&x)[FN], float* __restrict__ C, const float* __restrict__ bias,
+                                          float* __restrict__ Z, int row, int bcol, int M, int N, int beta) {
+  using vec = typename VecOf<FN>::type;
+  if (row >= M) return;
+  const int64_t o = (int64_t)row * N + bcol;
+  if (VEC) {  // N % FN == 0: the lane's FN columns are in or out together
+    if (bcol >= N) return;
+    if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU) {
+      const vec bv = *(const vec*)(bias + bcol);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) x[j] += vec_get<FN>(bv, j);
+    }
+    vec y;
+    if (EPI == AXN_EPI_BIAS_GELU || EPI == AXN_EPI_GELU) {
+      if (Z != nullptr) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          if constexpr (FN == 1) y = x[j];
+          else y[j] = x[j];
+        }
+        *(vec*)(Z + o) = y;
+      }
+#pragma unroll
+      for (int j = 0; j < FN; ++j) x[j] = gelu_erff(x[j]);
+    }
+    if (beta) {
+      const vec old = *(const vec*)(C + o);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) x[j] += vec_get<FN>(old, j);
+    }
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      if constexpr (FN == 1) y = x[j];
+      else y[j] = x[j];
+    }
+    *(vec*)(C + o) = y;
+  } else {
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      if (bcol + j >= N) continue;
+      float t = x[j];
+      if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU) t += bias[bcol + j];
+      if (EPI == AXN_EPI_BIAS_GELU || EPI == AXN_EPI_GELU) {
+        if (Z != nullptr) Z[o + j] = t;
+        t = gelu_erff(t);
+      }
+      if (beta) t += C[o + j];
+      C[o + j] = t;
+    }
+  }
+}
+
 // Stores a wave's 16 FM x 16 FN results at (m0, n0): register v of acc[i][j] in lane (r, q) is
 // output row m0 + FM (4 q + v) + i, column n0 + FN r + j.
 template <int EPI, int FM, int FN, bool VEC>
@@ -179,63 +238,14 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[FM][FN], float* __
                                            const float* __restrict__ bias, float* __restrict__ Z, int m0,
                                            int n0, int M, int N, int beta) {
   const int r = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
-  const int bcol = n0 + FN * r;
-  using vec = typename VecOf<FN>::type;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int row = m0 + FM * (4 * q + v) + i;
-      if (row >= M) continue;
-      const int64_t o = (int64_t)row * N + bcol;
       float x[FN];
 #pragma unroll
       for (int j = 0; j < FN; ++j) x[j] = acc[i][j][v];
-      if (VEC) {  // N % FN == 0: the lane's FN columns are in or out together
-        if (bcol >= N) continue;
-        if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU) {
-          const vec bv = *(const vec*)(bias + bcol);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) x[j] += vec_get<FN>(bv, j);
-        }
-        vec y;
-        if (EPI == AXN_EPI_BIAS_GELU || EPI == AXN_EPI_GELU) {
-          if (Z != nullptr) {
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-              if constexpr (FN == 1) y = x[j];
-              else y[j] = x[j];
-            }
-            *(vec*)(Z + o) = y;
-          }
-#pragma unroll
-          for (int j = 0; j < FN; ++j) x[j] = gelu_erff(x[j]);
-        }
-        if (beta) {
-          const vec old = *(const vec*)(C + o);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) x[j] += vec_get<FN>(old, j);
-        }
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          if constexpr (FN == 1) y = x[j];
-          else y[j] = x[j];
-        }
-        *(vec*)(C + o) = y;
-      } else {
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          if (bcol + j >= N) continue;
-          float t = x[j];
-          if (EPI == AXN_EPI_BIAS || EPI == AXN_EPI_BIAS_GELU) t += bias[bcol + j];
-          if (EPI == AXN_EPI_BIAS_GELU || EPI == AXN_EPI_GELU) {
-            if (Z != nullptr) Z[o + j] = t;
-            t = gelu_erff(t);
-          }
-          if (beta) t += C[o + j];
-          C[o + j] = t;
-        }
-      }
+      store_row<EPI, FN, VEC>(x, C, bias, Z, m0 + FM * (4 * q + v) + i, n0 + FN * r, M, N, beta);
     }
 }
 
@@ -276,6 +286,269 @@ __global__ void __launch_bounds__(64 * WAVES)
   }
 
   store_tile<EPI, FM, FN, VEC>(acc, C, bias, Z, m0, n0, M, N, beta);
+}
+
+// ---- the native products with their operands copied to LDS ahead -----------------------
+constexpr uint32_t kOutside = 0x80000000u;   // an offset behind every buffer: the copy writes zeros
+
+// One operand of a unit, 32 contraction indices of 16 F rows (columns), in a wave's own LDS: 2 F copies of 1 KB.
+//   KMAJOR: [row 16 i + r][32], row F r + i of the tile; the eight 16-byte pieces of a row are permuted by r / 2, so that
+//           the 16 lanes of a fragment read hit 16 different bank groups
+//   else    two blocks of 16 contraction indices, [4 s + q][16 F], index 4 q + s of the block
+template <bool KMAJOR, int F>
+struct Copied {
+  static constexpr int COPIES = 2 * F, BYTES = 2048 * F;
+  const char* base;
+  int64_t left;           // bytes of the operand from there on
+  uint32_t pitch, offset[KMAJOR ? 2 : 1];
+  int index[2], Kc;       // KMAJOR: first contraction index of the lane's piece
+  __device__ __forceinline__ void start(const float* from, int first, int rows, int K) {
+    const int lane = threadIdx.x & 63;
+    Kc = K;
+    if constexpr (KMAJOR) {
+      base = (const char*)(from + (int64_t)first * K);
+      left = ((int64_t)rows - first) * K * 4;
+      pitch = (uint32_t)K * 4;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        index[p] = 4 * ((lane & 7) ^ (4 * p + (lane >> 4)));
+        offset[p] = (uint32_t)(F * (8 * p + (lane >> 3))) * pitch + (uint32_t)index[p] * 4;
+      }
+    } else {
+      base = (const char*)(from + first);
+      left = ((int64_t)rows * K - first) * 4;
+      pitch = (uint32_t)rows * 4;
+      if constexpr (F == 4) offset[0] = (uint32_t)(4 * (lane >> 4)) * pitch + 16 * (lane & 15);
+      else if constexpr (F == 2) offset[0] = (uint32_t)(4 * ((lane >> 3) & 3) + (lane >> 5)) * pitch + 16 * (lane & 7);
+      else offset[0] = (uint32_t)(4 * ((lane >> 2) & 3) + (lane >> 4)) * pitch + 16 * (lane & 3);
+    }
+  }
+  // Starts the copies of contraction indices k .. k + 31; those behind the end come as zeros.
+  __device__ __forceinline__ void copy(int k, char* lds) const {
+    const int64_t skip = (int64_t)k * (KMAJOR ? 4 : pitch);
+    const int64_t rest = left - skip;
+    const int n = k >= Kc ? 0 : rest > 0x7fffffff ? 0x7fffffff : (int)rest;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(base + (k >= Kc ? 0 : skip)), 0, n, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < COPIES; ++j) {
+      uint32_t at;
+      if constexpr (KMAJOR) at = k + index[j & 1] < Kc ? offset[j & 1] + (uint32_t)(j >> 1) * pitch : kOutside;
+      else at = offset[0] + (uint32_t)(16 * (j / F) + (F == 4 ? j % 4 : F == 2 ? 2 * (j % 2) : 0)) * pitch;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(lds + 1024 * j), 16, (int)at,
+                                               0, 0, 0);
+    }
+  }
+  // Where the lane's reads of block u start.
+  __device__ __forceinline__ static uint32_t read_at(int u) {
+    const int r = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+    if constexpr (KMAJOR) return 128 * r + 16 * (((4 * u + q) ^ (r >> 1)) & 7);
+    else return u * (BYTES / 2) + 64 * F * q + 4 * F * r;
+  }
+};
+
+// An operand's fragments of a block of 16 contraction indices.  KMAJOR: k[i] holds indices 4 q .. 4 q + 3 of row i, else
+// m[s] rows 0 .. F - 1 of index 4 q + s.
+template <bool KMAJOR, int F>
+struct Fragments {
+  f32x4 k[F];
+  __device__ __forceinline__ float at(int i, int s) const { return k[i][s]; }
+};
+template <int F>
+struct Fragments<false, F> {
+  typename VecOf<F>::type m[4];
+  __device__ __forceinline__ float at(int i, int s) const { return vec_get<F>(m[s], i); }
+};
+// Both operands' fragments of the blocks that a step multiplies between two waits: four blocks (two units) at F = 1, two
+// at F = 2, one of the two at F = 4.  pa, pb: where the lane's reads of blocks 0 and 1 of a unit start.
+#define AXN_RD(size, to, from, at) "ds_read_" size " %" #to ", %" #from " offset:" #at "\n\t"
+#define AXN_RD4(size, t0, t1, t2, t3, from, a0, a1, a2, a3) \
+  AXN_RD(size, t0, from, a0) AXN_RD(size, t1, from, a1) AXN_RD(size, t2, from, a2) AXN_RD(size, t3, from, a3)
+#define AXN_WAIT "s_waitcnt lgkmcnt(0)"
+#define AXN_V4(x, y, z, w) "=&v"(x), "=&v"(y), "=&v"(z), "=&v"(w)
+#define AXN_M(f) AXN_V4(f.m[0], f.m[1], f.m[2], f.m[3])
+#define AXN_K(f) AXN_V4(f.k[0], f.k[1], f.k[2], f.k[3])
+__device__ __forceinline__ void read_step(Fragments<true, 1> (&a)[4], Fragments<true, 1> (&b)[4], const uint32_t (&pa)[2],
+                                          const uint32_t (&pb)[2]) {
+  asm volatile(AXN_RD("b128", 0, 8, 0) AXN_RD("b128", 4, 10, 0) AXN_RD("b128", 1, 9, 0) AXN_RD("b128", 5, 11, 0)
+               AXN_RD("b128", 2, 8, 4096) AXN_RD("b128", 6, 10, 4096) AXN_RD("b128", 3, 9, 4096) AXN_RD("b128", 7, 11, 4096) AXN_WAIT
+               : AXN_V4(a[0].k[0], a[1].k[0], a[2].k[0], a[3].k[0]), AXN_V4(b[0].k[0], b[1].k[0], b[2].k[0], b[3].k[0])
+               : "v"(pa[0]), "v"(pa[1]), "v"(pb[0]), "v"(pb[1]) : "memory");
+}
+__device__ __forceinline__ void read_step(Fragments<true, 1> (&a)[4], Fragments<false, 1> (&b)[4], const uint32_t (&pa)[2],
+                                          const uint32_t (&pb)[2]) {
+  asm volatile(AXN_RD("b128", 0, 20, 0) AXN_RD("b128", 1, 21, 0) AXN_RD("b128", 2, 20, 4096) AXN_RD("b128", 3, 21, 4096)
+               AXN_RD4("b32", 4, 5, 6, 7, 22, 0, 256, 512, 768) AXN_RD4("b32", 8, 9, 10, 11, 22, 1024, 1280, 1536, 1792)
+               AXN_RD4("b32", 12, 13, 14, 15, 22, 4096, 4352, 4608, 4864) AXN_RD4("b32", 16, 17, 18, 19, 22, 5120, 5376, 5632, 5888) AXN_WAIT
+               : AXN_V4(a[0].k[0], a[1].k[0], a[2].k[0], a[3].k[0]), AXN_M(b[0]), AXN_M(b[1]), AXN_M(b[2]), AXN_M(b[3])
+               : "v"(pa[0]), "v"(pa[1]), "v"(pb[0]) : "memory");
+}
+__device__ __forceinline__ void read_step(Fragments<true, 2> (&a)[2], Fragments<true, 2> (&b)[2], const uint32_t (&pa)[2],
+                                          const uint32_t (&pb)[2]) {
+  asm volatile(AXN_RD("b128", 0, 8, 0) AXN_RD("b128", 1, 8, 2048) AXN_RD("b128", 4, 10, 0) AXN_RD("b128", 5, 10, 2048)
+               AXN_RD("b128", 2, 9, 0) AXN_RD("b128", 3, 9, 2048) AXN_RD("b128", 6, 11, 0) AXN_RD("b128", 7, 11, 2048) AXN_WAIT
+               : AXN_V4(a[0].k[0], a[0].k[1], a[1].k[0], a[1].k[1]), AXN_V4(b[0].k[0], b[0].k[1], b[1].k[0], b[1].k[1])
+               : "v"(pa[0]), "v"(pa[1]), "v"(pb[0]), "v"(pb[1]) : "memory");
+}
+__device__ __forceinline__ void read_step(Fragments<true, 2> (&a)[2], Fragments<false, 2> (&b)[2], const uint32_t (&pa)[2],
+                                          const uint32_t (&pb)[2]) {
+  asm volatile(AXN_RD("b128", 0, 12, 0) AXN_RD("b128", 1, 12, 2048) AXN_RD("b128", 2, 13, 0) AXN_RD("b128", 3, 13, 2048)
+               AXN_RD4("b64", 4, 5, 6, 7, 14, 0, 512, 1024, 1536) AXN_RD4("b64", 8, 9, 10, 11, 14, 2048, 2560, 3072, 3584) AXN_WAIT
+               : AXN_V4(a[0].k[0], a[0].k[1], a[1].k[0], a[1].k[1]), AXN_M(b[0]), AXN_M(b[1])
+               : "v"(pa[0]), "v"(pa[1]), "v"(pb[0]) : "memory");
+}
+__device__ __forceinline__ void read_step(Fragments<false, 2> (&a)[2], Fragments<false, 2> (&b)[2], const uint32_t (&pa)[2],
+                                          const uint32_t (&pb)[2]) {
+  asm volatile(AXN_RD4("b64", 0, 1, 2, 3, 16, 0, 512, 1024, 1536) AXN_RD4("b64", 8, 9, 10, 11, 17, 0, 512, 1024, 1536)
+               AXN_RD4("b64", 4, 5, 6, 7, 16, 2048, 2560, 3072, 3584) AXN_RD4("b64", 12, 13, 14, 15, 17, 2048, 2560, 3072, 3584) AXN_WAIT
+               : AXN_M(a[0]), AXN_M(a[1]), AXN_M(b[0]), AXN_M(b[1]) : "v"(pa[0]), "v"(pb[0]) : "memory");
+}
+__device__ __forceinline__ void read_block(Fragments<true, 4>& a, Fragments<true, 4>& b, uint32_t pa, uint32_t pb) {
+  asm volatile(AXN_RD4("b128", 0, 1, 2, 3, 8, 0, 2048, 4096, 6144) AXN_RD4("b128", 4, 5, 6, 7, 9, 0, 2048, 4096, 6144) AXN_WAIT
+               : AXN_K(a), AXN_K(b) : "v"(pa), "v"(pb) : "memory");
+}
+__device__ __forceinline__ void read_block(Fragments<true, 4>& a, Fragments<false, 4>& b, uint32_t pa, uint32_t pb) {
+  asm volatile(AXN_RD4("b128", 0, 1, 2, 3, 8, 0, 2048, 4096, 6144) AXN_RD4("b128", 4, 5, 6, 7, 9, 0, 1024, 2048, 3072) AXN_WAIT
+               : AXN_K(a), AXN_M(b) : "v"(pa), "v"(pb) : "memory");
+}
+__device__ __forceinline__ void read_block(Fragments<false, 4>& a, Fragments<false, 4>& b, uint32_t pa, uint32_t pb) {
+  asm volatile(AXN_RD4("b128", 0, 1, 2, 3, 8, 0, 1024, 2048, 3072) AXN_RD4("b128", 4, 5, 6, 7, 9, 0, 1024, 2048, 3072) AXN_WAIT
+               : AXN_M(a), AXN_M(b) : "v"(pa), "v"(pb) : "memory");
+}
+#undef AXN_RD
+#undef AXN_RD4
+#undef AXN_WAIT
+#undef AXN_V4
+#undef AXN_M
+#undef AXN_K
+
+// Tile id of an output of tiles_m x tiles_n: the workgroups of a chiplet (every eighth) have neighbouring ones, in
+// groups of eight rows.
+__device__ __forceinline__ void chiplet_tile(unsigned id, int tiles_m, int tiles_n, int& tm, int& tn) {
+  constexpr unsigned kChiplets = 8, kRows = 8;
+  const unsigned tiles = tiles_m * tiles_n, each = tiles / kChiplets, rest = tiles % kChiplets;
+  const unsigned chiplet = id % kChiplets, t = chiplet * each + min(chiplet, rest) + id / kChiplets;
+  const unsigned group = t / (kRows * tiles_n), first = group * kRows, high = min(kRows, tiles_m - first);
+  const unsigned in = t - group * kRows * tiles_n;
+  tm = first + in % high, tn = in / high;
+}
+
+// What bounds gemm_f32_kernel is that a wave waits for each chunk's loads before it multiplies, 1 to 2 us from HBM, and
+// that an operand stored along the output is loaded 64 bytes a row and four bytes a lane.  Here a wave copies its own
+// operands to its own part of LDS, whole lines and up to 24 KB ahead, and waits for nobody: no barrier in the loop.
+// Its reads wait in the statement that issues them; a second workgroup on the CU (64 KB of LDS each up to F = 2) fills
+// that.  us, operands from HBM, gemm_f32_kernel / this:
+//   64 x 4096, contraction 1024, bias and GELU 18.0 / 10.9     1024 x 4096 weight gradient of 64 tokens  15.6 / 10.4
+//   64 x 1024, contraction 4096               22.3 / 13.6      the same of 256 tokens                   45.6 / 21.9
+//   256 x 4096, contraction 1024              41.0 / 26.6      1200 x 600, 1000 tokens                  41.2 / 23.4
+//   64 x 1024, contraction 4096, input gradient 55.3 / 18.5    256 x 1024, contraction 4096, input gradient 63.9 / 29.8
+// Twice the slots cost more (a workgroup a CU: 64 x 4096 above 13 -> 25 at F = 1); so do 32 x 32 tiles where 16 x 16 give a
+// workgroup for every CU (64 x 1024 above 29).  256 x 4096 x 1024 are 14 us at the rate of the matrix cores.
+//
+// TOGETHER: the four waves of a workgroup have one tile and the 64-deep chunks of its contraction in turn (what is left,
+// in blocks of 16); their sums are added in wave order.  Else a tile each, a square of two by two.
+template <bool AK, bool BKM, int EPI, int F, int SLOTS, bool TOGETHER>
+__global__ void __launch_bounds__(256)
+    gemm_f32_copied_kernel(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
+                           const float* __restrict__ bias, float* __restrict__ Z, int M, int N, int Kc, int tiles_m,
+                           int tiles_n, int beta) {
+  using OA = Copied<AK, F>;
+  using OB = Copied<BKM, F>;
+  constexpr int UNIT = OA::BYTES + OB::BYTES, EACH = OA::COPIES + OB::COPIES;
+  constexpr int STEP = F == 1 ? 2 : 1;   // units between two waits
+  static_assert(SLOTS % STEP == 0 && (SLOTS - STEP) * EACH <= 63, "the count of a wait has six bits");
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int tm, tn;
+  chiplet_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  if constexpr (!TOGETHER) tm = 2 * tm + (wave >> 1), tn = 2 * tn + (wave & 1);
+  const int m0 = tm * 16 * F, n0 = tn * 16 * F;
+  if (!TOGETHER && (m0 >= M || n0 >= N)) return;
+  OA a;
+  OB b;
+  a.start(A, m0, M, Kc);
+  b.start(B, n0, N, Kc);
+  const int chunks = Kc / 64, own = (chunks - wave + 3) / 4, tail = chunks * 64 + 16 * wave;
+  const int units = TOGETHER ? 2 * own + (tail < Kc) : (Kc + 31) / 32;
+  auto index_of = [&](int u) {
+    if constexpr (TOGETHER) return u < 2 * own ? 64 * (4 * (u >> 1) + wave) + 32 * (u & 1) : u == 2 * own ? tail : Kc;
+    else return 32 * u;
+  };
+  char* const mine = lds + wave * SLOTS * UNIT;
+  const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)mine;
+  const uint32_t ra[2] = {at + OA::read_at(0), at + OA::read_at(1)};
+  const uint32_t rb[2] = {at + OA::BYTES + OB::read_at(0), at + OA::BYTES + OB::read_at(1)};
+  f32x4 acc[F][F];
+  clear(acc);
+#pragma unroll
+  for (int u = 0; u < SLOTS; ++u) {
+    a.copy(index_of(u), mine + u * UNIT);
+    b.copy(index_of(u), mine + u * UNIT + OA::BYTES);
+  }
+  uint32_t slot = 0;
+#pragma unroll 1
+  for (int u = 0; u < units; u += STEP) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLOTS - STEP) * EACH) : "memory");
+    Fragments<AK, F> fa[2 * STEP];
+    Fragments<BKM, F> fb[2 * STEP];
+    auto multiply = [&](int h) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+          for (int j = 0; j < F; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[h].at(i, s), fb[h].at(j, s), acc[i][j], 0, 0, 0);
+    };
+    auto refill = [&]() {
+#pragma unroll
+      for (int v = 0; v < STEP; ++v) {
+        a.copy(index_of(u + SLOTS + v), mine + slot + v * UNIT);
+        b.copy(index_of(u + SLOTS + v), mine + slot + v * UNIT + OA::BYTES);
+      }
+    };
+    const uint32_t pa[2] = {ra[0] + slot, ra[1] + slot}, pb[2] = {rb[0] + slot, rb[1] + slot};
+    if constexpr (F == 4) {   // (two blocks' fragments would take half of the registers)
+      read_block(fa[0], fb[0], pa[0], pb[0]);
+      multiply(0);
+      read_block(fa[1], fb[1], pa[1], pb[1]);
+      refill();
+    } else {
+      read_step(fa, fb, pa, pb);
+      refill();
+      multiply(0);
+    }
+    if (!TOGETHER || u < 2 * own) {   // (else what is left: one block)
+#pragma unroll
+      for (int h = 1; h < 2 * STEP; ++h) multiply(h);
+    }
+    slot = slot + STEP * UNIT == SLOTS * UNIT ? 0 : slot + STEP * UNIT;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if constexpr (TOGETHER) {
+    // wave v adds and stores register v of every block
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+      for (int j = 0; j < F; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) ((float*)mine)[((i * F + j) * 4 + v) * 64 + lane] = acc[i][j][v];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < F; ++i) {
+      float x[F];
+#pragma unroll
+      for (int j = 0; j < F; ++j) {
+        const int o = ((i * F + j) * 4 + wave) * 64 + lane;
+        x[j] = ((const float*)lds)[o];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) x[j] += ((const float*)(lds + w * SLOTS * UNIT))[o];
+      }
+      store_row<EPI, F, true>(x, C, bias, Z, m0 + F * (4 * q + wave) + i, n0 + F * r, M, N, beta);
+    }
+  } else {
+    store_tile<EPI, F, F, true>(acc, C, bias, Z, m0, n0, M, N, beta);
+  }
 }
 
 // ---- fp32 products on the 16-bit matrix units ---------------------------------
@@ -639,12 +912,67 @@ int launch_parts(const float* ws, float* C, const float* bias, float* Z, int M, 
 // With fewer than 4096 of the native kernel's tiles and a contraction of KMIN or more (256 for the smallest
 // tile, 2048 for the middle one; measured: the split loses on the largest tile and on shorter contractions),
 // four waves share a tile.
+constexpr int kTogether16 = 256, kTogether32 = 2048;
 template <bool AK, bool BKM, int EPI, int FM, int FN, int U, int KMIN>
 int launch_waves(long long tiles, const float* A, const float* B, float* C, const float* bias,
                  float* Z, int M, int N, int Kc, int beta, hipStream_t stream) {
   if (tiles < 4096 && Kc >= KMIN)
     return launch_tile<AK, BKM, EPI, FM, FN, (U > 4 ? 4 : U), 4>(A, B, C, bias, Z, M, N, Kc, beta, stream);
   return launch_tile<AK, BKM, EPI, FM, FN, U, 1>(A, B, C, bias, Z, M, N, Kc, beta, stream);
+}
+
+// Whether gemm_f32_copied_kernel does a product faster than gemm_f32_kernel, and in which wave tiles: 16, 32 or 64
+// square (1, 2, 4 blocks), 0 for neither.  In us, fitted to 260 sizes of 8 to 6200 tokens and 64 to 8192 features, cold
+// operands, a layout and a tile each to 6 to 12 %; 5 % ahead counts.  What it picks takes 0.83 (forward), 0.53 (input
+// gradient) and 0.83 (weight gradient) of the time of gemm_f32_kernel on average and 1 to 2 % more than the best.  That one
+// stays ahead with short contractions (forward 924 x 336, contraction 164: 8.2 us, 8.9 here; weight gradients under 50 to
+// 100 tokens: 5696 x 960, 72 tokens 16.5, 19.1): there its waves have all they multiply in flight at once.
+int copied_blocks(GemmLayout layout, const NativeTiles& t, bool together, int64_t M, int64_t N, int64_t Kc) {
+  struct Fit {
+    double fixed, serial, load, round, out;   // a launch, a unit of a wave, of all on a CU, a round, 2^20 results or so
+  };
+  constexpr Fit kCopied[3][3] = {{{1.8, 0.098, 0.16, 1.6, 1.1}, {2.8, 0.31, 0.45, 1.1, 2.0}, {3.2, 2.1, 0.0, 4.2, 2.9}},
+                                 {{1.7, 0.12, 0.18, 1.2, 0.0}, {1.2, 0.35, 0.45, 1.3, 0.21}, {1.9, 2.1, 0.0, 1.7, 0.7}},
+                                 {{1e9, 0, 0, 0, 0}, {2.2, 0.22, 0.47, 0.51, 0.95}, {2.1, 2.0, 0.0, 1.7, 0.52}}};
+  double least = 1e9;
+  int best = 0;
+  for (int i = 0; i < 3; ++i) {
+    const int F = 1 << i, side = together ? 16 * F : 32 * F;
+    const double each = together ? 2.0 * ((Kc + 255) / 256) : (double)((Kc + 31) / 32);
+    const double load = (double)((((M + side - 1) / side) * ((N + side - 1) / side) + 255) / 256);
+    const double rounds = F == 4 ? load : std::ceil(load / 2);
+    const Fit& f = kCopied[layout][i];
+    const double us = f.fixed + f.serial * rounds * each + f.load * load * each + f.round * rounds + f.out * M * N * 1e-6;
+    if (us < least) least = us, best = F;
+  }
+  if (layout == GEMM_NN || (t.size == 32 && together)) return best;
+  struct Direct {
+    double fixed, chunk, chunks, load, bytes;   // a launch, a wave's 64 indices, a SIMD's, a wave on every SIMD, 1 MB loaded
+  };
+  // 16 x 16 tiles of a wave, of four waves, 32 x 32, 64 x 64
+  constexpr Direct kDirect[2][4] = {{{2.6, 0.57, 0.0, 0.61, 0.068}, {3.3, 0.17, 0.65, 0.0, 0.023}, {4.7, 0.23, 0.0, 1.4, 0.12}, {16.0, 1.1, 0.0, 0.0, 0.2}},
+                                    {{3.2, 0.0, 0.82, 0.15, 0.024}, {2.9, 0.86, 0.64, 0.16, 0.0}, {1.6, 4.0, 0.0, 1.1, 0.044}, {2.2, 4.9, 0.0, 3.1, 0.098}}};
+  const Direct& d = kDirect[layout == GEMM_NT ? 0 : 1][t.size == 64 ? 3 : t.size == 32 ? 2 : together ? 1 : 0];
+  const double chunks = Kc / (together ? 256.0 : 64.0), load = std::max(1.0, t.count * (together ? 4.0 : 1.0) / 1024);
+  const double us = d.fixed + d.chunk * chunks + d.chunks * load * chunks + d.load * load + d.bytes * t.count * 2.0 * t.size * Kc * 4e-6;
+  return least <= 0.95 * us ? best : 0;
+}
+
+template <bool AK, bool BKM, int EPI, int F, int SLOTS>
+int launch_copied(bool together, const float* A, const float* B, float* C, const float* bias, float* Z, int M, int N, int Kc,
+                  int beta, hipStream_t stream) {
+  if constexpr (F == 1 && !AK) return AXN_EINVAL;   // (not picked)
+  else {
+    constexpr size_t kLds = 4 * SLOTS * F * 4096;
+    const int side = together ? 16 * F : 32 * F, tiles_m = (int)ceil_div(M, side), tiles_n = (int)ceil_div(N, side);
+    const auto kern = together ? gemm_f32_copied_kernel<AK, BKM, EPI, F, SLOTS, true> : gemm_f32_copied_kernel<AK, BKM, EPI, F, SLOTS, false>;
+    static std::atomic<unsigned long long> allowed[2];   // per instance: devices it may have this LDS on
+    if (const int rc = allow_lds((const void*)kern, kLds, allowed[together])) return rc;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)tiles_m * tiles_n)), dim3(256), kLds, stream, A, B, C, bias, Z, M, N, Kc,
+                       tiles_m, tiles_n, beta);
+    AXN_HIP_TRY(hipGetLastError());
+    return AXN_OK;
+  }
 }
 
 // Contractions whose loops would step past 2^31 - 1 (by four waves' chunks of 128 at most).
@@ -668,13 +996,22 @@ int launch_epi(const float* A, const float* B, float* C, const float* bias, floa
   if (plan.parts == 1)
     return launch_split<AK, BKM, EPI>(A, B, C, bias, Z, M, N, Kc, beta, plan, stream);
   const NativeTiles t = native_tiles(M, N);
+  const uintptr_t ptrs = (uintptr_t)A | (uintptr_t)B | (uintptr_t)C | (uintptr_t)bias | (uintptr_t)Z;
+  if (N % 4 == 0 && (AK ? Kc % 4 == 0 : M % 4 == 0) && (ptrs & 15u) == 0 && std::max({M, N, Kc}) <= 1 << 22) {
+    const bool together = t.size < 64 && t.count < 4096 && Kc >= (t.size == 32 ? kTogether32 : kTogether16);
+    const int blocks = copied_blocks(layout, t, together, M, N, Kc);
+    if (AK && blocks == 1)
+      return launch_copied<AK, BKM, EPI, 1, 4>(together, A, B, C, bias, Z, M, N, Kc, beta, stream);
+    if (blocks == 2) return launch_copied<AK, BKM, EPI, 2, 2>(together, A, B, C, bias, Z, M, N, Kc, beta, stream);
+    if (blocks == 4) return launch_copied<AK, BKM, EPI, 4, 2>(together, A, B, C, bias, Z, M, N, Kc, beta, stream);
+  }
   if (Kc > kLongContraction)
     return launch_tile<AK, BKM, EPI, 1, 1, 4, 4, true>(A, B, C, bias, Z, M, N, Kc, beta, stream);
   if (t.size == 64)
     return launch_tile<AK, BKM, EPI, 4, 4, 2, 1>(A, B, C, bias, Z, M, N, Kc, beta, stream);
   if (t.size == 32)
-    return launch_waves<AK, BKM, EPI, 2, 2, 4, 2048>(t.count, A, B, C, bias, Z, M, N, Kc, beta, stream);
-  return launch_waves<AK, BKM, EPI, 1, 1, 8, 256>(t.count, A, B, C, bias, Z, M, N, Kc, beta, stream);
+    return launch_waves<AK, BKM, EPI, 2, 2, 4, kTogether32>(t.count, A, B, C, bias, Z, M, N, Kc, beta, stream);
+  return launch_waves<AK, BKM, EPI, 1, 1, 8, kTogether16>(t.count, A, B, C, bias, Z, M, N, Kc, beta, stream);
 }
 
 }  // namespace

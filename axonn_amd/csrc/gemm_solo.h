@@ -929,18 +929,5 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g) {
   solo_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, EDGE, ODD>(g, tm, tn, split);
 }
 
-// The dynamic LDS size a kernel may ask for is an attribute of the kernel on a device: set
-// on a kernel's first launch on each device, not on every launch.  `done` is the
-// per-kernel-instance record (one bit per device).
-int allow_lds(const void* kern, size_t lds, std::atomic<unsigned long long>& done) {
-  int dev = 0;
-  AXN_HIP_TRY(hipGetDevice(&dev));
-  const unsigned long long bit = 1ull << (dev & 63);
-  if (done.load(std::memory_order_acquire) & bit) return AXN_OK;
-  AXN_HIP_TRY(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  done.fetch_or(bit, std::memory_order_release);
-  return AXN_OK;
-}
-
 }  // namespace
 }  // namespace axn

@@ -202,6 +202,7 @@ int launch_gemm_edge_f16(GemmLayout layout, const GemmArgs& args, int epilogue, 
 // The same on a FED_* tile; row strides below kEdgeMaxLd / 2.
 int launch_gemm_fed_nt_bf16(const GemmArgs& args, int epilogue, bool out_f32, EdgeTile tile, hipStream_t stream);
 int launch_gemm_fed_nt_f16(const GemmArgs& args, int epilogue, bool out_f32, EdgeTile tile, hipStream_t stream);
+int launch_gemm_fed_rounds(const GemmArgs& args, bool half, EdgeTile tile, hipStream_t stream);
 int launch_gemm_fed_nn_tn_bf16(GemmLayout layout, const GemmArgs& args, bool out_f32, EdgeTile tile, hipStream_t stream);
 int launch_gemm_fed_nn_tn_f16(GemmLayout layout, const GemmArgs& args, bool out_f32, EdgeTile tile, hipStream_t stream);
 // Both gradients of a layer in one launch of 256 x 256 tiles; tiles_m, tiles_n and wg_first set.

@@ -25,7 +25,8 @@ FAST_PATH = os.path.join(LIB_DIR, "axn_fast.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = ["axn_api.hip", "gemm_bf16.hip", "gemm_edge_bf16.hip", "gemm_edge_f16.hip",
-           "gemm_fed_nt_bf16.hip", "gemm_fed_nt_f16.hip", "gemm_fed_nn_tn_bf16.hip", "gemm_fed_nn_tn_f16.hip", "gemm_gate_up.hip",
+           "gemm_fed_nt_bf16.hip", "gemm_fed_nt_f16.hip", "gemm_fed_nn_tn_bf16.hip", "gemm_fed_nn_tn_f16.hip", "gemm_fed_rounds.hip",
+           "gemm_gate_up.hip",
            "gemm_stream.hip", "gemm_far.hip", "gemm_f32.hip", "elementwise.hip", "embedding.hip", "optim.hip"]
 PROBE_SOURCES = ["stream_probe.hip"]
 

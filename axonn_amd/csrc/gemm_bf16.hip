@@ -308,6 +308,25 @@ const FedTile* fed_tile(GemmLayout layout, const GemmArgs& g, int epilogue, bool
   return us < 0.95 * other_microseconds(layout, other, g.M, g.N) ? t : nullptr;
 }
 
+// The tile of a 16-bit weight gradient that is done in more than two rounds of workgroups that stay
+// (gemm_fed_rounds.hip), or EDGE_256x256 where the others are ahead.  Such a launch saves what the tiles' ramps and
+// stores cost a short contraction, and ends on a finer last round than 256 x 256 tiles; what it loses is their rate.  So
+// the line lies at the contraction (the tokens): up to 448 it may take as many half rounds as they do, up to 800 it has to
+// save a sixteenth, and 264 and less are stores in any tile.  us, before / so, of 103 gradients of 265 to 800 tokens
+// over 1024 to 50264 features with more than 512 tiles, ragged ones most: where it is taken 0.90 of the time on average,
+// 1.02 at worst; 447 x 12288 x 2048 38.7 / 29.1, 404 x 9600 x 2368 35.7 / 28.1, 748 x 6016 x 2880 43.3 / 36.7,
+// 430 x 12096 x 2304 35.4 / 36.1.  Left out: 657 x 8960 x 3584 47.6 / 49.5, 768 x 8192 x 8192 98 / 112.  fp32 results and
+// adding to one are bound by the output (382 x 4160 x 5632 fp32 35.6 / 39.7, 349 x 6784 x 4808 added to 46 / 57).
+EdgeTile rounds_tile(const GemmArgs& g) {
+  if (g.Kc <= 264 || g.Kc > 800 || g.beta || g.splits > 1 || (g.lda > g.ldb ? g.lda : g.ldb) >= kEdgeMaxLd / 2) return EDGE_256x256;
+  const long long wide = ceil_div(g.M, 128) * ceil_div(g.N, 256), tall = ceil_div(g.M, 256) * ceil_div(g.N, 128);
+  const long long tiles = wide <= tall ? wide : tall, halves = 2 * ceil_div(ceil_div(g.M, 256) * ceil_div(g.N, 256), 256);
+  if (tiles <= 512 || tiles > 65536) return EDGE_256x256;
+  const long long rounds = ceil_div(tiles, 256);
+  if (16 * rounds > (g.Kc <= 448 ? 16 : 15) * halves) return EDGE_256x256;
+  return wide <= tall ? FED_128x256 : EDGE_256x128;
+}
+
 int launch_fed(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, bool half, EdgeTile tile,
                hipStream_t stream) {
   if (tile == EDGE_256x128)
@@ -428,6 +447,8 @@ template <bool AK, bool BKM, int EPI, bool OUT_F32, bool HALF>
 int launch_shape(const GemmArgs& g, hipStream_t stream) {
   if constexpr (EPI != EPI_PAIR) {
     constexpr GemmLayout order = !AK ? GEMM_TN : BKM ? GEMM_NT : GEMM_NN;
+    if constexpr (order == GEMM_TN && EPI == AXN_EPI_NONE && !OUT_F32)
+      if (const EdgeTile t = rounds_tile(g); t != EDGE_256x256) return launch_gemm_fed_rounds(g, HALF, t, stream);
     if (const FedTile* t = fed_tile(order, g, EPI, OUT_F32))
       return launch_fed(order, g, EPI, OUT_F32, HALF, t->tile, stream);
     // output rows that are not 16-byte aligned (axn_gemm_any_n): the kernels with bounds store them

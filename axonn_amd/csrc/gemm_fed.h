@@ -34,8 +34,10 @@ constexpr size_t kFedLds = (size_t)kFedStages<BM, BN> * (BM + BN) * 128;
 //
 // The operands' bounds are those of solo_gemm's EDGE (any contraction and operand size) throughout: they cost nothing
 // here, the copying waves have time for them.  EDGE: the output's (false: whole tiles, rows 16-byte aligned).
-// ODD, EPI_PAIR: as there.
-template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF, bool EDGE = true, bool ODD = false>
+// ODD, EPI_PAIR: as there.  ROUNDS: the workgroup takes tiles blockIdx.x, + gridDim.x, ... one after the other; the
+// stages of all of them are one sequence to the waves and the ring (gridDim.x is a multiple of the XCDs' number).
+template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF, bool EDGE = true, bool ODD = false,
+          bool ROUNDS = false>
 __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
   constexpr uint32_t kOutside = 0x80000000u;
   constexpr int FRM = BM / 32, FRN = BN / 32, PK = 64, NM = FRM * FRN, NFRAG = FRM + FRN;
@@ -51,6 +53,7 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
   static_assert(NST >= 3 && (NST - 1) * NC <= 63, "the count of a wait has six bits");
   static_assert(!PAIR || (A_KMAJOR && !B_KMAJOR), "the two-term product is the dgrad layout");
   static_assert(!ODD || (A_KMAJOR && B_KMAJOR), "the forward");
+  static_assert(!ROUNDS || (!A_KMAJOR && !B_KMAJOR && EPI == AXN_EPI_NONE), "weight gradients: their epilogue needs no LDS");
   static_assert(!SWIGLU || (BN % 128 == 0 && A_KMAJOR && B_KMAJOR && !OUT_F32), "gate and up rows of a wave column");
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -66,9 +69,18 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
     }
     tile_of_workgroup(pid, g.tiles_m, g.tiles_n, tm, tn);
   }
-  const int m0 = tm * BM, n0 = tn * (SWIGLU ? BN / 2 : BN);
+  [[maybe_unused]] int tile = blockIdx.x;   // ROUNDS
+  int m0 = tm * BM, n0 = tn * (SWIGLU ? BN / 2 : BN);
   const StageRange part = stages_of_part(g.Kc, split, g.splits);
   const int s0 = part.first, KP = part.count;
+  const int rounds = ROUNDS ? (g.tiles_m * g.tiles_n - tile + (int)gridDim.x - 1) / (int)gridDim.x : 1;
+  const int all = rounds * KP;   // stages
+  [[maybe_unused]] auto next_tile = [&]() {
+    tile += gridDim.x;
+    tile_of_workgroup(tile, g.tiles_m, g.tiles_n, tm, tn);
+    m0 = tm * BM;
+    n0 = tn * BN;
+  };
 
   if (wave8 >= 4) {
     OperandWalk wa, wb, wb2;   // (wb2: SWIGLU, the up weights')
@@ -94,6 +106,13 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
     uint32_t slot = 0;
     int next = 0;   // the stage to copy
     auto copy_stage = [&]() {
+      if constexpr (ROUNDS)
+        if (next == KP) {
+          next_tile();
+          wa.start(g.A, A_KMAJOR, g.M, kfirst, g.lda, m0, 0);
+          wb.start(g.B, B_KMAJOR, g.N, kfirst, g.ldb, n0, 0);
+          next = 0;
+        }
       if (PAIR && (s0 + next) * PK == g.k_first) {
         wa.start(g.A2, A_KMAJOR, g.M, g.Kc - g.k_first, g.lda, m0, 0);
         wb.start(g.B2, B_KMAJOR, g.N, g.Kc - g.k_first, g.ldb, n0, 0);
@@ -127,14 +146,14 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
       slot = slot + STAGE == NST * STAGE ? 0 : slot + STAGE;
       ++next;
     };
-    const int ahead = KP < NST ? KP : NST;
+    const int ahead = all < NST ? all : NST;
 #pragma unroll 1
     for (int p = 0; p < ahead; ++p) copy_stage();
-    if (KP >= NST) wait_vmcnt<(NST - 1) * NC>();
+    if (all >= NST) wait_vmcnt<(NST - 1) * NC>();
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
 #pragma unroll 1
-    for (int p = NST; p < KP; ++p) {
+    for (int p = NST; p < all; ++p) {
       wait_vmcnt<(NST - 2) * NC>();   // all but the youngest NST - 2 stages have landed
       __builtin_amdgcn_s_barrier();
       copy_stage();
@@ -210,6 +229,24 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
   };
   __builtin_amdgcn_s_barrier();
   static_for<NFRAG>([&](auto f_) { read(std::integral_constant<int, 0>{}, f_, s); });
+  if constexpr (ROUNDS) {
+#pragma unroll 1
+    for (int r = 1; r < rounds; ++r) {
+#pragma unroll 1
+      for (int p = 0; p < KP; ++p) stage(std::false_type{});
+      asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < FRM; ++i) tie_accumulators(acc[i]);
+      store_blocks<EPI, OUT_F32, HALF, EDGE, ODD, false>(acc, g, 0, m0 + wm * (BM / 2), n0 + wn * (BN / 2), lane, nullptr);
+#pragma unroll
+      for (int i = 0; i < FRM; ++i) {
+#pragma unroll
+        for (int j = 0; j < FRN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        tie_accumulators(acc[i]);
+      }
+      next_tile();
+    }
+  }
 #pragma unroll 1
   for (int p = 0; p < KP - 1; ++p) stage(std::false_type{});
   stage(std::true_type{});

@@ -234,6 +234,7 @@ __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {
     for (int r = 1; r < rounds; ++r) {
 #pragma unroll 1
       for (int p = 0; p < KP; ++p) stage(std::false_type{});
+      wait_all_fragments(fa0, fb0);   // the next tile's first: the stores' code may move registers
       asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
       for (int i = 0; i < FRM; ++i) tie_accumulators(acc[i]);

@@ -314,9 +314,9 @@ const FedTile* fed_tile(GemmLayout layout, const GemmArgs& g, int epilogue, bool
 // the line lies at the contraction (the tokens): up to 448 it may take as many half rounds as they do, up to 800 it has to
 // save a sixteenth, and 264 and less are stores in any tile.  us, before / so, of 103 gradients of 265 to 800 tokens
 // over 1024 to 50264 features with more than 512 tiles, ragged ones most: where it is taken 0.90 of the time on average,
-// 1.02 at worst, and of 70 drawn anew that it takes 0.91, three slower (763 x 50264 x 1792 148.5 / 150.5, 424 x 15872 x
-// 1792 36.4 / 37.2, 381 x 12416 x 1632 23.4 / 25.4); 447 x 12288 x 2048 38.7 / 29.1, 404 x 9600 x 2368 35.7 / 28.1, 748 x 6016 x 2880 43.3 / 36.7,
-// 430 x 12096 x 2304 35.4 / 36.1.  Left out: 657 x 8960 x 3584 47.6 / 49.5, 768 x 8192 x 8192 98 / 112.  fp32 results and
+// 1.02 at worst.  Since a tile's stores wait for the next tile's first fragments (2 %): of 70 drawn anew that it takes 0.93,
+// six slower (381 x 12416 x 1632 23.9 / 25.9, the others 2 to 5 %).  Before that wait 447 x 12288 x 2048 38.7 / 29.1,
+// 404 x 9600 x 2368 35.7 / 28.1, 748 x 6016 x 2880 43.3 / 36.7, 430 x 12096 x 2304 35.4 / 36.1.  Left out: 657 x 8960 x 3584 47.6 / 49.5, 768 x 8192 x 8192 98 / 112.  fp32 results and
 // adding to one are bound by the output (382 x 4160 x 5632 fp32 35.6 / 39.7, 349 x 6784 x 4808 added to 46 / 57).
 EdgeTile rounds_tile(const GemmArgs& g) {
   if (g.Kc <= 264 || g.Kc > 800 || g.beta || g.splits > 1 || (g.lda > g.ldb ? g.lda : g.ldb) >= kEdgeMaxLd / 2) return EDGE_256x256;

@@ -186,7 +186,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const at::Tensor bias = tensor_or_none(args[2]);
   const c10::DeviceIndex device = current_device_for(x);
   if (at::autocast::is_autocast_enabled(at::kCUDA) || !plain(x, device) || !plain(w, device) ||
-      x.dim() < 1 || !nothing_watches() || x._fw_grad(0).defined() || w._fw_grad(0).defined())
+      x.dim() < 1 || !nothing_watches() || x._fw_grad(0).defined() || w._fw_grad(0).defined() ||
+      (bias.defined() && bias._fw_grad(0).defined()))
     Py_RETURN_NONE;
   const int64_t N = PyLong_AsLongLong(args[3]), K = PyLong_AsLongLong(args[4]);
   if (N < 1 || K < 1 || x.size(-1) != K || w.numel() != N * K) Py_RETURN_NONE;

@@ -187,6 +187,20 @@ def test_what_is_left_to_the_general_way():
         assert back(*args) is None
 
 
+@pytest.mark.parametrize("dual", ["x", "weight", "bias"])
+def test_a_tangent_is_refused_as_the_general_way_refuses_it(dual):
+    """Of any operand, also where no gradients are recorded (forward mode goes on there): it is not dropped."""
+    layer = Linear(64, 48).cuda().bfloat16()
+    x = torch.randn(16, 64, device="cuda").bfloat16()
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        at = {"x": x, "weight": layer.weight, "bias": layer.bias}
+        made = torch.autograd.forward_ad.make_dual(at[dual].detach(), torch.ones_like(at[dual]))
+        if dual == "x":
+            x = made
+        with pytest.raises(NotImplementedError, match="jvp"):
+            torch.func.functional_call(layer, {} if dual == "x" else {dual: made}, (x,))
+
+
 def test_errors_are_those_of_the_general_way():
     layer = Linear(64, 48).cuda().bfloat16()
     with torch.no_grad():

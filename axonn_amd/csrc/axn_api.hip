@@ -593,6 +593,11 @@ int axn_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,
   REQUIRE(aligned16(dY) && aligned16(Z) && aligned16(dZ), AXN_EALIGN,
           "%s: pointers must be 16-byte aligned", name);
   REQUIRE(beta == 0 || beta == 1, AXN_EINVAL, "%s: beta must be 0 or 1", name);
+  // elements of half the size: a row of dZ lies where another one of dY has not been read
+  const unsigned __int128 elements = (unsigned __int128)(M - 1) * (uint64_t)ld + (uint64_t)N;
+  const uintptr_t y = (uintptr_t)dY, z = (uintptr_t)dZ;
+  REQUIRE(!wide || (y < z ? z - y >= 4 * elements : y - z >= 2 * elements), AXN_EINVAL,
+          "%s: an fp32 dY and dZ must not overlap", name);
   return launch_dgelu_dbias(dY, Z, dZ, dtype, wide, dbias, dbias16, M, N, ld, beta, workspace,
                             workspace_bytes, (hipStream_t)stream);
 }

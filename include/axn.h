@@ -110,8 +110,9 @@ AXN_API int axn_gemm_wgrad(const void* dY, const void* X, void* dW, int64_t M,
  * `workspace` (axn_dgelu_dbias_workspace_bytes, needed only when dbias is
  * given) and are reduced in a fixed order.  dZ may alias dY.
  * dtype | AXN_DY_F32 (16-bit types): dY is fp32 and rounded to dtype first (a 16-bit product
- * with an fp32 bias has an fp32 result and gradient); dZ is required, and without Z receives
- * the rounded dY.  dtype | AXN_DBIAS_16BIT (16-bit types, beta 0): dbias is of dtype. */
+ * with an fp32 bias has an fp32 result and gradient); dZ is required, must not overlap dY, and
+ * without Z receives the rounded dY.  dtype | AXN_DBIAS_16BIT (16-bit types, beta 0): dbias is
+ * of dtype. */
 #define AXN_DY_F32 0x100
 #define AXN_DBIAS_16BIT 0x200
 AXN_API int axn_dgelu_dbias(const void* dY, const void* Z, void* dZ, int dtype,

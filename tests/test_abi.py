@@ -296,6 +296,22 @@ def test_elementwise_argument_errors():
     assert "workspace" in _err()
 
 
+def test_an_fp32_gradient_is_not_rounded_in_place():
+    """dZ's elements are half as wide as dY's: its rows would overwrite others of dY that are still to be read.  (The
+    workspace is too small throughout: what gets past the check is refused for that.)"""
+    f = nv.load().axn_dgelu_dbias
+    M, N, ld, Y = 5, 16, 24, 0x100000
+    used = (M - 1) * ld + N
+    for dtype in (nv.BF16 | nv.DY_F32, nv.F16 | nv.DY_F32 | nv.DBIAS_16BIT):
+        for z, apart in [(Y, False), (Y + 16, False), (Y + 4 * used - 16, False), (Y + 4 * used, True),
+                         (Y - 2 * used + 16, False), (Y - 2 * used, True)]:
+            for Z in (None, 2 * Y):
+                assert f(Y, Z, z, dtype, Y, M, N, ld, 0, Y, 4, None) == nv.AXN_EINVAL
+                assert ("overlap" in _err()) != apart and ("workspace" in _err()) == apart, (z - Y, _err())
+    # of one type, in place: accepted as it was
+    assert f(Y, Y, Y, nv.BF16, Y, M, N, ld, 0, Y, 4, None) == nv.AXN_EINVAL and "workspace" in _err()
+
+
 def test_multi_tensor_argument_errors():
     lib = nv.load()
     ptrs = (ctypes.c_void_p * 2)(0x1000, 0x2001)

@@ -68,7 +68,7 @@ class GateUpSwiGLU(torch.autograd.Function):
             x2, w_gate.reshape(shape).to(dt), w_up.reshape(shape).to(dt), save=needs_grad, few=few,
             any_sizes=not few and not ops.gemm_swiglu_supported(x2.shape[0], *shape, dt))
         ctx.save_for_backward(x2, w_gate, w_up, gate, up)
-        ctx.shape, ctx.input_shape, ctx.compute_dtype = shape, x.shape, dt
+        ctx.shape, ctx.input_shape, ctx.input_dtype, ctx.compute_dtype = shape, x.shape, x.dtype, dt
         return h.reshape(*x.shape[:-1], shape[0])
 
     @staticmethod
@@ -82,12 +82,12 @@ class GateUpSwiGLU(torch.autograd.Function):
         dgate, dup = ops.swiglu_bwd(d2, gate, up)
         grad_x = grad_wg = grad_wu = None
         if not ops.gemm_dgrad_pair_supported(x2.shape[0], n, n, k, dt):
-            # as the two projections called by themselves, and autograd's sum
-            need = ctx.needs_input_grad
-            grad_x, grad_wg = _backward_products(dgate, w_gate.reshape(ctx.shape).to(dt), x2, w_gate, need[0], need[1])
-            dx_up, grad_wu = _backward_products(dup, w_up.reshape(ctx.shape).to(dt), x2, w_up, need[0], need[2])
+            # as the two projections called by themselves, and autograd's sum: in the input's type
+            need, widen = ctx.needs_input_grad, ctx.input_dtype == torch.float32
+            grad_x, grad_wg = _backward_products(dgate, w_gate.reshape(ctx.shape).to(dt), x2, w_gate, need[0], need[1], widen)
+            dx_up, grad_wu = _backward_products(dup, w_up.reshape(ctx.shape).to(dt), x2, w_up, need[0], need[2], widen)
             if need[0]:
-                grad_x = (grad_x + dx_up).reshape(ctx.input_shape)
+                grad_x = (grad_x.to(ctx.input_dtype) + dx_up.to(ctx.input_dtype)).reshape(ctx.input_shape)
             return grad_x, grad_wg, grad_wu, None, None
         if ctx.needs_input_grad[0]:
             # both products through one set of accumulators, rounded once (two products and

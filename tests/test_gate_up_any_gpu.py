@@ -87,3 +87,26 @@ def test_the_patched_mlp_of_any_number_of_tokens(tokens, hidden, ffn, grad, monk
     monkeypatch.setattr(modify_llama, "_one_launch_gate_up", lambda mlp, x: False)
     for a, b in zip(fused, step()):
         assert float((a.double() - b.double()).norm() / b.double().norm()) < 1e-2
+
+
+@pytest.mark.parametrize("tokens,hidden,ffn", [(301, 1024, 2752), (777, 512, 1408)])
+@pytest.mark.parametrize("x_dtype,dtype", [(torch.float32, torch.bfloat16), (torch.float32, torch.float16),
+                                           (torch.bfloat16, torch.float16), (torch.bfloat16, torch.bfloat16)])
+def test_input_gradients_are_added_in_the_inputs_type(tokens, hidden, ffn, x_dtype, dtype):
+    """Each rounded to the products' type, converted to the input's and then added, as autograd adds those of two
+    projections: an fp32 input under autocast has the fp32 sum of the two."""
+    from axonn_amd.models.transformers.modify_llama import GateUpSwiGLU
+
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    x = torch.randn(1, tokens, hidden, generator=gen, device="cuda").to(x_dtype).requires_grad_(True)
+    wg, wu = (torch.randn(ffn, hidden, generator=gen, device="cuda").mul_(0.02).to(dtype).requires_grad_(True) for _ in range(2))
+    dh = torch.randn(1, tokens, ffn, generator=gen, device="cuda").mul_(0.1).to(dtype)
+    with torch.autocast("cuda", dtype):
+        h = GateUpSwiGLU.apply(x, wg.view(-1), wu.view(-1), (ffn, hidden), True)
+    h.backward(dh)
+    x2 = x.detach()[0].to(dtype)
+    _, gate, up = ops.gemm_swiglu_fwd(x2, wg.detach(), wu.detach(), any_sizes=True)
+    (a, dwg), (b, dwu) = (ops.gemm_bwd(d, w.detach(), x2) for d, w in zip(ops.swiglu_bwd(dh[0], gate, up), (wg, wu)))
+    assert a.dtype == b.dtype == dtype and x.grad.dtype == x_dtype
+    assert torch.equal(x.grad[0], a.to(x_dtype) + b.to(x_dtype))
+    assert torch.equal(wg.grad, dwg) and torch.equal(wu.grad, dwu)

@@ -190,6 +190,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
       (bias.defined() && bias._fw_grad(0).defined()))
     Py_RETURN_NONE;
   const int64_t N = PyLong_AsLongLong(args[3]), K = PyLong_AsLongLong(args[4]);
+  const bool gelu = truth(args[5]);   // (here: objects are asked with the interpreter's lock held)
+  if (PyErr_Occurred()) return nullptr;
   if (N < 1 || K < 1 || x.size(-1) != K || w.numel() != N * K) Py_RETURN_NONE;
   std::vector<int64_t> shape = x.sizes().vec();
   shape.back() = N;
@@ -198,7 +200,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   {
     Unlocked unlocked;
     const bool out_f32 = bias.defined() && bias.scalar_type() == at::kFloat && x.scalar_type() != at::kFloat;
-    done = forward(x, w, bias, x.numel() / K, N, K, truth(args[5]), false, out_f32, shape, device, y, z);
+    done = forward(x, w, bias, x.numel() / K, N, K, gelu, false, out_f32, shape, device, y, z);
   }
   if (!done) Py_RETURN_NONE;
   return wrap(y);

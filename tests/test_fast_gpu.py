@@ -201,6 +201,25 @@ def test_a_tangent_is_refused_as_the_general_way_refuses_it(dual):
             torch.func.functional_call(layer, {} if dual == "x" else {dual: made}, (x,))
 
 
+def test_arguments_are_asked_with_the_interpreters_lock():
+    x, w, b = (torch.randn(s, device="cuda").bfloat16() for s in ((16, 64), (48 * 64,), (48,)))
+
+    class Asked:
+        def __init__(self, answer):
+            self.answer = answer
+
+        def __bool__(self):
+            return {"yes": True, "no": False}[self.answer]
+
+    with torch.no_grad():
+        for answer, plain in (("yes", True), ("no", False)):
+            assert torch.equal(FAST.linear(x, w, b, 48, 64, Asked(answer)), FAST.linear(x, w, b, 48, 64, plain))
+        with pytest.raises(KeyError):
+            FAST.linear(x, w, b, 48, 64, Asked("neither"))
+        with pytest.raises(TypeError):
+            FAST.linear(x, w, b, "48", 64, False)
+
+
 def test_errors_are_those_of_the_general_way():
     layer = Linear(64, 48).cuda().bfloat16()
     with torch.no_grad():

@@ -142,7 +142,7 @@ def _load_fast(lib):
     import torch
 
     dtype_code(torch.float32)   # (fills the table that callers of `fast` look types up in)
-    module.bind({name: ctypes.cast(getattr(lib, name), _vp).value for name in module.entry_points()})
+    module.bind(dict({name: ctypes.cast(getattr(lib, name), _vp).value for name in module.entry_points()}, check=check))
     return module
 
 

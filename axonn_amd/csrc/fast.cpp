@@ -1,8 +1,9 @@
 // The usual calls of a Linear layer without their way through Python: checks, output and workspace tensors and
 // the library's entry point in one function each.  Whatever is not usual - another layout, type, device or
-// alignment, an empty batch, a size that needs padding, a mode that watches tensors, an error of the library -
-// answers None, and the caller (axonn_amd/ops.py, fully_connected.py) goes the general way from the start (only an error
-// of the library can follow a launch, and none follows one that adds to a result).
+// alignment, an empty batch, a size that needs padding, a mode that watches tensors - answers None before anything is
+// launched, and the caller (axonn_amd/ops.py, fully_connected.py) goes the general way from the start.  An error of the
+// library is raised, as it is there: it can follow a launch (one that an earlier call left behind is reported by the
+// next), and a second one would add the weight gradient again.
 //
 // Host time of a forward of 8 x 1024 x 1024 bf16 through a Linear without gradients 15.6 us in Python, 5.4 here (3.7 of
 // it the library's call and its launch); forward and backward of 64 x 1024 x 1024, autograd's part included, 153 -> 99.
@@ -38,6 +39,7 @@ struct Library {
   ENTRY_POINTS(DECLARE)
 #undef DECLARE
 } lib;
+PyObject* check_status = nullptr;   // axonn_amd._native.check: raises the library's error
 
 // Rows further apart are packed first by the general way.
 constexpr int64_t kFarRows = 1 << 22;
@@ -120,23 +122,30 @@ at::ScalarType type_of(PyObject* o) {   // of AXN_*; anything else is no type
   return c == AXN_BF16 ? at::kBFloat16 : c == AXN_F16 ? at::kHalf : c == AXN_F32 ? at::kFloat : at::ScalarType::Undefined;
 }
 
+constexpr int kNotTaken = 1;   // beside the library's status: nothing was launched, the general way takes the call
+PyObject* no_result(int status) {
+  if (status == kNotTaken) Py_RETURN_NONE;
+  Py_XDECREF(PyObject_CallFunction(check_status, "i", status));
+  return nullptr;
+}
+
 // ---- forward -------------------------------------------------------------------------------
-// act(X W^T + b) into y [.., N] (and z); false: not launched.
-bool forward(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, int64_t M, int64_t N, int64_t K, bool gelu,
-             bool save_z, bool out_f32, at::IntArrayRef shape, c10::DeviceIndex device, at::Tensor& y, at::Tensor& z) {
+// act(X W^T + b) into y [.., N] (and z).
+int forward(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, int64_t M, int64_t N, int64_t K, bool gelu,
+            bool save_z, bool out_f32, at::IntArrayRef shape, c10::DeviceIndex device, at::Tensor& y, at::Tensor& z) {
   const at::ScalarType type = x.scalar_type();
   const bool half = is16(type);
   if (!(half || type == at::kFloat) || w.scalar_type() != type || M < 1 || N < 1 || K < 1 || K >= kFarRows ||
       M > 0x7fffffff || N > 0x7ffffff8)
-    return false;
-  if (half ? K % 8 != 0 : out_f32) return false;
+    return kNotTaken;
+  if (half ? K % 8 != 0 : out_f32) return kNotTaken;
   int epilogue = bias.defined() ? (gelu ? AXN_EPI_BIAS_GELU : AXN_EPI_BIAS) : (gelu ? AXN_EPI_GELU : AXN_EPI_NONE);
   if (bias.defined()) {
-    if (bias.numel() != N || !plain(bias, device)) return false;
+    if (bias.numel() != N || !plain(bias, device)) return kNotTaken;
     if (half && bias.scalar_type() == type) epilogue |= AXN_BIAS_16BIT;
-    else if (bias.scalar_type() != at::kFloat) return false;
+    else if (bias.scalar_type() != at::kFloat) return kNotTaken;
   } else if (out_f32) {
-    return false;
+    return kNotTaken;
   }
   y = empty(shape, out_f32 ? at::kFloat : type, x);
   if (gelu && save_z) z = empty(shape, type, x);
@@ -144,11 +153,11 @@ bool forward(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, i
   if (half) {
     const Workspace ws(out_f32 ? 0 : bytes_needed(FWD, M, N, K), x);
     return lib.axn_gemm_any_n(AXN_GEMM_FWD, pointer(x), pointer(w), pointer(bias), pointer(y), pointer(z), code_of(type),
-                              M, N, K, K, K, N, epilogue, 0, out_f32 ? AXN_F32 : code_of(type), ws.at, ws.bytes, stream) == AXN_OK;
+                              M, N, K, K, K, N, epilogue, 0, out_f32 ? AXN_F32 : code_of(type), ws.at, ws.bytes, stream);
   }
   const Workspace ws(bytes_needed(F32_FWD, M, N, K), x);
   return lib.axn_gemm_fwd_f32_ws((const float*)pointer(x), (const float*)pointer(w), (const float*)pointer(bias),
-                                 (float*)pointer(y), (float*)pointer(z), M, N, K, epilogue, ws.at, ws.bytes, stream) == AXN_OK;
+                                 (float*)pointer(y), (float*)pointer(z), M, N, K, epilogue, ws.at, ws.bytes, stream);
 }
 
 // gemm_fwd(x, w, bias, gelu, save_z, out_f32) -> (y, z) or None
@@ -162,12 +171,12 @@ PyObject* gemm_fwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t M = x.size(0), N = w.size(0);
   const bool gelu = truth(args[3]), save_z = truth(args[4]), out_f32 = truth(args[5]);
   at::Tensor y, z;
-  bool done;
+  int status;
   {
     Unlocked unlocked;
-    done = forward(x, w, bias, M, N, x.size(1), gelu, save_z, out_f32, {M, N}, device, y, z);
+    status = forward(x, w, bias, M, N, x.size(1), gelu, save_z, out_f32, {M, N}, device, y, z);
   }
-  if (!done) Py_RETURN_NONE;
+  if (status != AXN_OK) return no_result(status);
   PyObject* out = PyTuple_New(2);
   PyTuple_SET_ITEM(out, 0, wrap(y));
   PyTuple_SET_ITEM(out, 1, wrap(z));
@@ -196,13 +205,13 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   std::vector<int64_t> shape = x.sizes().vec();
   shape.back() = N;
   at::Tensor y, z;
-  bool done;
+  int status;
   {
     Unlocked unlocked;
     const bool out_f32 = bias.defined() && bias.scalar_type() == at::kFloat && x.scalar_type() != at::kFloat;
-    done = forward(x, w, bias, x.numel() / K, N, K, gelu, false, out_f32, shape, device, y, z);
+    status = forward(x, w, bias, x.numel() / K, N, K, gelu, false, out_f32, shape, device, y, z);
   }
-  if (!done) Py_RETURN_NONE;
+  if (status != AXN_OK) return no_result(status);
   return wrap(y);
   END_HANDLE_TH_ERRORS
 }
@@ -214,18 +223,18 @@ struct Backward {
   at::ScalarType bias_type, dw_type;   // of the bias gradient, if the kernels write it; of dW
   at::Tensor dx, dw, db;
 
-  bool run(c10::DeviceIndex device) {
+  int run(c10::DeviceIndex device) {
     const at::ScalarType type = x.scalar_type();
     const bool half = is16(type);
     const int64_t M = dy.size(0), N = dy.size(1), K = w.size(1);
     if (!(half || type == at::kFloat) || M < 1 || N % 8 != 0 || N < 8 || K < 1 || (half && K % 8 != 0) ||
         std::max(N, K) >= kFarRows || M > 0x7fffffff)
-      return false;
+      return kNotTaken;
     const at::ScalarType from = dy.scalar_type();
     const bool pass = z.defined() || want_db, wide = half && from == at::kFloat;
-    if (from != type && !(wide && pass)) return false;
-    if (z.defined() && (z.scalar_type() != type || z.sizes() != dy.sizes())) return false;
-    if (need_dw && dw_type != at::kFloat && dw_type != type) return false;
+    if (from != type && !(wide && pass)) return kNotTaken;
+    if (z.defined() && (z.scalar_type() != type || z.sizes() != dy.sizes())) return kNotTaken;
+    if (need_dw && dw_type != at::kFloat && dw_type != type) return kNotTaken;
     const auto stream = c10::hip::getCurrentHIPStream(device).stream();
     const int code = code_of(type);
     if (pass) {
@@ -236,9 +245,9 @@ struct Backward {
       if (db16) flags |= AXN_DBIAS_16BIT;
       if (want_db) db = empty({N}, db16 ? type : at::kFloat, x);
       const Workspace ws(want_db ? std::max<size_t>(bytes_needed(DBIAS, M, N, 0), 16) : 0, x);
-      if (lib.axn_dgelu_dbias(pointer(dy), pointer(z), pointer(dz), flags, (float*)pointer(db), M, N, N, 0, ws.at, ws.bytes,
-                              stream) != AXN_OK)
-        return false;
+      const int rc = lib.axn_dgelu_dbias(pointer(dy), pointer(z), pointer(dz), flags, (float*)pointer(db), M, N, N, 0, ws.at,
+                                         ws.bytes, stream);
+      if (rc != AXN_OK) return rc;
       if (dz.defined()) dy = dz;
     }
     const int beta = out.defined() ? 1 : 0;
@@ -250,26 +259,28 @@ struct Backward {
       if (need_dx) {
         void* pdx = make_dx();
         const Workspace ws(bytes_needed(F32_DGRAD, M, N, K), x);
-        if (lib.axn_gemm_dgrad_f32_ws((float*)pdy, (float*)pw, (float*)pdx, M, N, K, ws.at, ws.bytes, stream) != AXN_OK) return false;
+        const int rc = lib.axn_gemm_dgrad_f32_ws((float*)pdy, (float*)pw, (float*)pdx, M, N, K, ws.at, ws.bytes, stream);
+        if (rc != AXN_OK) return rc;
       }
       if (need_dw) {
         void* pdw = make_dw();
         const Workspace ws(bytes_needed(F32_WGRAD, M, N, K), x);
-        if (lib.axn_gemm_wgrad_f32_ws((float*)pdy, (float*)px, (float*)pdw, M, N, K, beta, ws.at, ws.bytes, stream) != AXN_OK) return false;
+        const int rc = lib.axn_gemm_wgrad_f32_ws((float*)pdy, (float*)px, (float*)pdw, M, N, K, beta, ws.at, ws.bytes, stream);
+        if (rc != AXN_OK) return rc;
       }
-      return true;
+      return AXN_OK;
     }
     const int dw_code = code_of(dw_type);
     const size_t both = need_dx && need_dw ? bytes_needed(beta ? BOTH_ADD : BOTH, M, N, K) : 0;
     if (both) {
       void *pdx = make_dx(), *pdw = make_dw();
       const Workspace ws(both, x);
-      return lib.axn_gemm_bwd_ws(pdy, pw, px, pdx, pdw, code, M, N, K, N, K, K, K, K, beta, dw_code, ws.at, ws.bytes, stream) == AXN_OK;
+      return lib.axn_gemm_bwd_ws(pdy, pw, px, pdx, pdw, code, M, N, K, N, K, K, K, K, beta, dw_code, ws.at, ws.bytes, stream);
     }
     const size_t ws_d = need_dx ? bytes_needed(DGRAD, M, N, K) : 0, ws_w = need_dw ? bytes_needed(WGRAD, M, N, K) : 0;
     if (need_dx && need_dw && ws_d == 0 && ws_w == 0) {
       void *pdx = make_dx(), *pdw = make_dw();
-      return lib.axn_gemm_bwd(pdy, pw, px, pdx, pdw, code, M, N, K, N, K, K, K, K, beta, dw_code, stream) == AXN_OK;
+      return lib.axn_gemm_bwd(pdy, pw, px, pdx, pdw, code, M, N, K, N, K, K, K, K, beta, dw_code, stream);
     }
     if (need_dx) {
       const bool wider = ws_d && widen;
@@ -285,14 +296,14 @@ struct Backward {
       } else {
         rc = (type == at::kHalf ? lib.axn_gemm_dgrad_f16 : lib.axn_gemm_dgrad)(pdy, pw, pdx, M, N, K, N, K, K, stream);
       }
-      if (rc != AXN_OK) return false;
+      if (rc != AXN_OK) return rc;
     }
-    if (!need_dw) return true;
+    if (!need_dw) return AXN_OK;
     void* pdw = make_dw();
     const Workspace ws(ws_w, x);
     if (ws_w)
-      return lib.axn_gemm_wgrad_ws(pdy, px, pdw, code, M, N, K, N, K, K, beta, dw_code, ws.at, ws.bytes, stream) == AXN_OK;
-    return (type == at::kHalf ? lib.axn_gemm_wgrad_f16 : lib.axn_gemm_wgrad)(pdy, px, pdw, M, N, K, N, K, K, beta, dw_code, stream) == AXN_OK;
+      return lib.axn_gemm_wgrad_ws(pdy, px, pdw, code, M, N, K, N, K, K, beta, dw_code, ws.at, ws.bytes, stream);
+    return (type == at::kHalf ? lib.axn_gemm_wgrad_f16 : lib.axn_gemm_wgrad)(pdy, px, pdw, M, N, K, N, K, K, beta, dw_code, stream);
   }
 };
 
@@ -322,12 +333,12 @@ PyObject* backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Py_RETURN_NONE;
   if (b.out.defined() && (!b.need_dw || !plain(b.out, device) || b.out.scalar_type() != b.dw_type || b.out.numel() != b.w.numel()))
     Py_RETURN_NONE;
-  bool done;
+  int status;
   {
     Unlocked unlocked;
-    done = b.run(device);
+    status = b.run(device);
   }
-  if (!done) Py_RETURN_NONE;
+  if (status != AXN_OK) return no_result(status);
   PyObject* out = PyTuple_New(3);
   PyTuple_SET_ITEM(out, 0, wrap(b.dx));
   PyTuple_SET_ITEM(out, 1, wrap(b.dw));
@@ -336,7 +347,7 @@ PyObject* backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind({name: address}): the library's entry points
+// bind({name: address, "check": axonn_amd._native.check}): the library's entry points, and what raises their errors
 PyObject* bind(PyObject*, PyObject* table) {
   Library bound;
 #define BIND(name)                                                                        \
@@ -349,6 +360,10 @@ PyObject* bind(PyObject*, PyObject* table) {
   }
   ENTRY_POINTS(BIND)
 #undef BIND
+  PyObject* check = PyMapping_GetItemString(table, "check");
+  if (check == nullptr) return nullptr;
+  Py_XDECREF(check_status);
+  check_status = check;
   lib = bound;
   Py_RETURN_NONE;
 }

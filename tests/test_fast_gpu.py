@@ -239,6 +239,38 @@ def test_errors_are_those_of_the_general_way():
         assert ops.gemm_fwd(torch.zeros(4, 64, device="cuda"), torch.zeros(48, 64, device="cuda"))[0].shape == (4, 48)
 
 
+# (each a different entry point: one launch, one in parts, two launches, full precision)
+@pytest.mark.parametrize("dtype,M,N,K", [(torch.bfloat16, 64, 128, 64), (torch.bfloat16, 777, 6144, 4096),
+                                         (torch.float16, 512, 8192, 3584), (torch.float32, 64, 128, 256)])
+def test_an_error_behind_a_launch_is_raised_and_adds_once(dtype, M, N, K):
+    """A launch that has been made and then reports an error (HIP reports one that an earlier call left behind): the
+    weight gradient has been added, and is not added again by another way."""
+    lib, calls = nv.load(), []
+
+    def reports_an_error(name):
+        def entry(*args):
+            assert getattr(lib, name)(*args) == nv.AXN_OK
+            calls.append(name)
+            return nv.AXN_EHIP
+        return ctypes.CFUNCTYPE(*[nv.SYMBOLS[name][0], *nv.SYMBOLS[name][1]])(entry)
+
+    table = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in FAST.entry_points()}
+    table["check"] = nv.check
+    adding = [name for name in table if name.startswith(("axn_gemm_bwd", "axn_gemm_wgrad")) and not name.endswith("_bytes")]
+    entries = {name: reports_an_error(name) for name in adding}
+    dy, w, x = (torch.randint(-2, 3, s, device="cuda").to(dtype) for s in ((M, N), (N, K), (M, K)))
+    grad = torch.full((N, K), 3.0, device="cuda")
+    once = ops.gemm_wgrad(dy, x, out=grad.clone(), accumulate=True)
+    FAST.bind(dict(table, **{name: ctypes.cast(e, ctypes.c_void_p).value for name, e in entries.items()}))
+    try:
+        with pytest.raises(nv.AxnError) as raised:
+            ops.gemm_bwd(dy, w, x, out=grad, accumulate=True)
+    finally:
+        FAST.bind(table)
+    assert raised.value.code == nv.AXN_EHIP and len(calls) == 1
+    assert torch.equal(grad, once)
+
+
 def test_streams_and_graphs():
     """On the current stream, and in a captured graph, replayed with other work between."""
     torch.manual_seed(4)

@@ -27,7 +27,7 @@ DY_F32, DBIAS_16BIT = 0x100, 0x200   # with the dtype of axn_dgelu_dbias: dY is 
 ROUNDED = 0x100      # with F32 as an input gradient's output type: 16-bit values
 ANY_SIZES = 0x100    # with the dtype of axn_gemm_swiglu_fwd: sizes that are not made of whole tiles
 
-ABI_VERSION = 15   # another one with every change of the entry points below
+ABI_VERSION = 16   # another one with every change of the entry points below or of the constants above
 
 # Every symbol include/axn.h declares: name -> (restype, argtypes)
 _c = ctypes

@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define AXN_ABI_VERSION 15
+#define AXN_ABI_VERSION 16
 
 #if defined(__GNUC__)
 #define AXN_API __attribute__((visibility("default")))

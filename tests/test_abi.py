@@ -6,6 +6,7 @@ import ctypes
 import os
 import re
 import subprocess
+import zlib
 
 import pytest
 
@@ -34,7 +35,15 @@ def test_library_loads_and_exports_every_declared_symbol():
 
 def test_the_version_goes_with_the_entry_points():
     """A change of the entry points takes a version of its own: raise it together with what is written here."""
-    assert (nv.ABI_VERSION, len(nv.SYMBOLS)) == (15, 43)
+    assert (nv.ABI_VERSION, len(nv.SYMBOLS)) == (16, 43)
+
+
+def test_the_version_goes_with_the_flags_and_arguments():
+    """So does a new constant or argument: a library that does not know it would fail in the middle of a step."""
+    text = open(os.path.join(ROOT, "include", "axn.h")).read()
+    text = re.sub(r"#define AXN_ABI_VERSION[^\n]*", "", re.sub(r"/\*.*?\*/", " ", text, flags=re.S))
+    assert "AXN_ANY_SIZES" in text and "axn_mt_adam" in text
+    assert (nv.ABI_VERSION, "%08x" % zlib.crc32(" ".join(text.split()).encode())) == (16, "eec76e83")
 
 
 def test_a_library_of_another_version_is_refused_by_its_version(tmp_path, monkeypatch):

@@ -9,7 +9,9 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sys
 import threading
+import warnings
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libaxn_gfx950.so")
 
@@ -113,7 +115,8 @@ SYMBOLS = {
 _lib = None
 _probe_lib = None
 # axn_fast.so (csrc/fast.cpp): the host side of the usual Linear calls, same kernels.  None before `load` and where it is
-# not built: every caller then goes the general way, which it also goes where a function of `fast` answers None.
+# not built or does not fit: every caller then goes the general way, which it also goes where a function of `fast` answers
+# None.
 fast = None
 _lock = threading.Lock()
 
@@ -131,19 +134,34 @@ def lib_path():
 
 
 def _load_fast(lib):
+    """axn_fast.so, or None.  Unlike the library it is tied to one PyTorch and one Python: built for others, or for another
+    version of this package, it is left alone with a warning."""
     path = os.path.join(os.path.dirname(_LIB_PATH), "axn_fast.so")
     if not os.path.exists(path):
         return None
-    loader = importlib.machinery.ExtensionFileLoader("axn_fast", path)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("axn_fast", loader))
-    loader.exec_module(module)
-    if module.ABI_VERSION != ABI_VERSION:
-        raise ImportError("axn_fast.so has ABI version %d, this package needs %d" % (module.ABI_VERSION, ABI_VERSION))
-    import torch
-
+    try:
+        import torch
+    except ImportError:
+        return None   # (nobody calls it)
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("axn_fast", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("axn_fast", loader))
+        loader.exec_module(module)
+        built, wanted = (module.ABI_VERSION, module.BUILT_FOR), (ABI_VERSION, fast_built_for(torch))
+        if built != wanted:
+            raise ImportError("it was built for %s, this is %s" % (built, wanted))
+        module.bind(dict({name: ctypes.cast(getattr(lib, name), _vp).value for name in module.entry_points()}, check=check))
+    except (ImportError, AttributeError) as error:
+        warnings.warn("axn_fast.so is not used, Linear calls take more host time (%s); run "
+                      "`python -m axonn_amd.csrc.build`" % error, stacklevel=3)
+        return None
     dtype_code(torch.float32)   # (fills the table that callers of `fast` look types up in)
-    module.bind(dict({name: ctypes.cast(getattr(lib, name), _vp).value for name in module.entry_points()}, check=check))
     return module
+
+
+def fast_built_for(torch):
+    """What axn_fast.so is built for beside the library's version."""
+    return "%s, PyTorch %s" % (sys.implementation.cache_tag, torch.__version__)
 
 
 def load():

@@ -63,16 +63,28 @@ def build_fast():
     """Compiles and links axn_fast.so.  Its libraries are PyTorch's, found by soname in the process that has them."""
     import torch
 
+    from .._native import fast_built_for
+
     base = os.path.dirname(torch.__file__)
     tmp = FAST_PATH + ".tmp"
     _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
-          *("-isystem" + d for d in (os.path.join(base, "include"), os.path.join(base, "include", "torch", "csrc", "api", "include"),
+          '-DAXN_BUILT_FOR="%s"' % fast_built_for(torch), *("-isystem" + d for d in (os.path.join(base, "include"), os.path.join(base, "include", "torch", "csrc", "api", "include"),
                                      os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
                                      sysconfig.get_paths()["include"])),
           "-I" + os.path.join(ROOT, "include"), os.path.join(HERE, "fast.cpp"), "-o", tmp, "-L" + os.path.join(base, "lib"),
           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"])
     os.replace(tmp, FAST_PATH)   # (a running process keeps the file it has mapped)
+
+
+def build_fast_if_possible():
+    """The package works without axn_fast.so: without a host compiler, or PyTorch's headers, the library alone is built."""
+    try:
+        build_fast()
+    except (ImportError, OSError, RuntimeError) as error:
+        if os.path.exists(FAST_PATH):
+            os.remove(FAST_PATH)   # (what is left of an earlier build is of other sources)
+        print("axn_fast.so is not built, Linear calls will take more host time: %s" % error, file=sys.stderr)
 
 
 def build_library(verbose=False, extra_flags=()):
@@ -89,7 +101,7 @@ def build_library(verbose=False, extra_flags=()):
 
     every = SOURCES + PROBE_SOURCES
     with ThreadPoolExecutor(max_workers=min(len(every) + 1, os.cpu_count() or 1)) as pool:
-        fast = pool.submit(build_fast)
+        fast = pool.submit(build_fast_if_possible)
         objs = list(pool.map(compile_one, every))
         fast.result()
     for path, part in ((LIB_PATH, objs[:len(SOURCES)]), (PROBE_LIB_PATH, objs[len(SOURCES):])):

@@ -394,7 +394,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "axn_fast", nullptr, -1, methods};
 
 PyMODINIT_FUNC PyInit_axn_fast() {
   PyObject* m = PyModule_Create(&module);
-  if (m != nullptr && PyModule_AddIntConstant(m, "ABI_VERSION", AXN_ABI_VERSION) != 0) {
+  if (m != nullptr && (PyModule_AddIntConstant(m, "ABI_VERSION", AXN_ABI_VERSION) != 0 ||
+                       PyModule_AddStringConstant(m, "BUILT_FOR", AXN_BUILT_FOR) != 0)) {
     Py_DECREF(m);
     return nullptr;
   }

@@ -6,6 +6,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sysconfig
 import zlib
 
 import pytest
@@ -395,3 +396,45 @@ def test_missing_library_fails_loudly(monkeypatch):
     monkeypatch.setattr(nv, "_LIB_PATH", "/nonexistent/libaxn_gfx950.so")
     with pytest.raises(ImportError, match="not built"):
         nv.load()
+
+
+FOREIGN = {
+    "a symbol that this PyTorch lacks": "extern int of_another_pytorch(void); void* PyInit_axn_fast(void) { of_another_pytorch(); return 0; }",
+    "no module": "int nothing;",
+    "another version": """
+        #include <Python.h>
+        static struct PyModuleDef def = {PyModuleDef_HEAD_INIT, "axn_fast", 0, -1, 0};
+        PyMODINIT_FUNC PyInit_axn_fast(void) {
+          PyObject* m = PyModule_Create(&def);
+          PyModule_AddIntConstant(m, "ABI_VERSION", %d);
+          PyModule_AddStringConstant(m, "BUILT_FOR", "cpython-310, PyTorch 1.0");
+          return m;
+        }""" % nv.ABI_VERSION,
+}
+
+
+@pytest.mark.parametrize("what", sorted(FOREIGN))
+def test_a_host_side_that_does_not_fit_is_left_alone(tmp_path, monkeypatch, what):
+    """axn_fast.so is tied to one PyTorch and one Python, the library is not: it is used without the other."""
+    source = tmp_path / "fast.c"
+    source.write_text(FOREIGN[what])
+    subprocess.run(["gcc", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"], "-o", str(tmp_path / "axn_fast.so"), str(source)],
+                   check=True)
+    os.symlink(nv.lib_path(), tmp_path / "libaxn_gfx950.so")
+    monkeypatch.setattr(nv, "_LIB_PATH", str(tmp_path / "libaxn_gfx950.so"))
+    monkeypatch.setattr(nv, "_lib", None)
+    monkeypatch.setattr(nv, "fast", None)
+    with pytest.warns(UserWarning, match="axn_fast.so is not used"):
+        lib = nv.load()
+    assert lib.axn_abi_version() == nv.ABI_VERSION and nv.fast is None
+
+
+def test_the_library_is_built_without_a_compiler_for_the_host_side(tmp_path, monkeypatch, capsys):
+    from axonn_amd.csrc import build
+
+    stale = tmp_path / "axn_fast.so"
+    stale.write_bytes(b"of an earlier build")
+    monkeypatch.setattr(build, "FAST_PATH", str(stale))
+    monkeypatch.setenv("CXX", str(tmp_path / "no_compiler"))
+    build.build_fast_if_possible()
+    assert not stale.exists() and "axn_fast.so is not built" in capsys.readouterr().err

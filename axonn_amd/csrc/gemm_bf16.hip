@@ -320,6 +320,7 @@ const FedTile* fed_tile(GemmLayout layout, const GemmArgs& g, int epilogue, bool
 // adding to one are bound by the output (382 x 4160 x 5632 fp32 35.6 / 39.7, 349 x 6784 x 4808 added to 46 / 57).
 EdgeTile rounds_tile(const GemmArgs& g) {
   if (g.Kc <= 264 || g.Kc > 800 || g.beta || g.splits > 1 || (g.lda > g.ldb ? g.lda : g.ldb) >= kEdgeMaxLd / 2) return EDGE_256x256;
+  if (g.N % 8 != 0 || g.ldc % 8 != 0) return EDGE_256x256;   // (columns that it does not store)
   const long long wide = ceil_div(g.M, 128) * ceil_div(g.N, 256), tall = ceil_div(g.M, 256) * ceil_div(g.N, 128);
   const long long tiles = wide <= tall ? wide : tall, halves = 2 * ceil_div(ceil_div(g.M, 256) * ceil_div(g.N, 256), 256);
   if (tiles <= 512 || tiles > 65536) return EDGE_256x256;

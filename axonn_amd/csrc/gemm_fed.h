@@ -35,7 +35,8 @@ constexpr size_t kFedLds = (size_t)kFedStages<BM, BN> * (BM + BN) * 128;
 // The operands' bounds are those of solo_gemm's EDGE (any contraction and operand size) throughout: they cost nothing
 // here, the copying waves have time for them.  EDGE: the output's (false: whole tiles, rows 16-byte aligned).
 // ODD, EPI_PAIR: as there.  ROUNDS: the workgroup takes tiles blockIdx.x, + gridDim.x, ... one after the other; the
-// stages of all of them are one sequence to the waves and the ring (gridDim.x is a multiple of the XCDs' number).
+// stages of all of them are one sequence to the waves and the ring (gridDim.x is a multiple of the XCDs' number); the output's
+// columns are a multiple of 8 (the others go through LDS, which the next tile's stages have).
 template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF, bool EDGE = true, bool ODD = false,
           bool ROUNDS = false>
 __device__ __forceinline__ void fed_gemm(const GemmArgs& g) {

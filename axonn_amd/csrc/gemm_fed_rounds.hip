@@ -38,6 +38,10 @@ int launch_rounds(const GemmArgs& in, hipStream_t stream) {
 }  // namespace
 
 int launch_gemm_fed_rounds(const GemmArgs& g, bool half, EdgeTile tile, hipStream_t stream) {
+  if (g.N % 8 != 0 || g.ldc % 8 != 0) {   // the epilogue has no LDS for columns behind the last multiple of 8
+    set_error("gemm_fed_rounds: rows of whole, aligned vectors expected (got N=%d, ldc=%lld)", g.N, (long long)g.ldc);
+    return AXN_ESHAPE;
+  }
   if (tile == FED_128x256) return half ? launch_rounds<128, 256, true>(g, stream) : launch_rounds<128, 256, false>(g, stream);
   return half ? launch_rounds<256, 128, true>(g, stream) : launch_rounds<256, 128, false>(g, stream);
 }

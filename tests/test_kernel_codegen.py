@@ -198,3 +198,33 @@ def test_update_kernel_streams_through_buffer_accesses_without_scratch(tmp_path_
         assert max(loads) < min(stores), name
         assert all(ins[i].endswith(" nt") for i in loads), name
         assert all(ins[i].endswith(" nt sc1") for i in stores), name
+
+
+def test_tiles_in_rounds_refuse_columns_that_they_do_not_store(tmp_path):
+    """Their epilogue has no LDS for the columns behind the last multiple of 8: the launch refuses such an output, and
+    rows that are not 16-byte aligned, whoever calls it."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    csrc = os.path.join(ROOT, "axonn_amd", "csrc")
+    source = tmp_path / "rounds.hip"
+    source.write_text("""
+        #include <stdio.h>
+        #include "gemm_fed_rounds.hip"
+        namespace axn {
+        void set_error(const char*, ...) {}
+        int hip_fail(hipError_t, const char*) { return AXN_EHIP; }
+        }
+        int main() {
+          const int sizes[][2] = {{2060, 2064}, {2056, 2060}, {8, 9}, {7, 8}};
+          for (auto& s : sizes) {
+            axn::GemmArgs g = {};
+            g.M = 8200, g.N = s[0], g.ldc = s[1], g.Kc = 320, g.lda = 8200, g.ldb = 2064;
+            printf("%d\\n", axn::launch_gemm_fed_rounds(g, false, axn::FED_128x256, nullptr));
+          }
+        }""")
+    program = tmp_path / "rounds"
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + csrc, str(source), "-o", str(program)],
+                   check=True, capture_output=True, timeout=900)
+    out = subprocess.run([str(program)], check=True, capture_output=True, text=True, timeout=120).stdout
+    assert [int(s) for s in out.split()] == [-3] * 4   # AXN_ESHAPE

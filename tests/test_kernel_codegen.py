@@ -118,6 +118,106 @@ def _device_asm(tmp_path_factory, name):
     return kernels
 
 
+def _vector_registers(s):
+    used = {int(v) for v in re.findall(r"\bv(\d+)\b", s)}
+    for a, b in re.findall(r"\bv\[(\d+):(\d+)\]", s):
+        used |= set(range(int(a), int(b) + 1))
+    return used
+
+
+def fragments_touched_in_flight(body):
+    """(instructions that name a register of an LDS read that may be on its way, number of such reads).  The reads are
+    asm statements, and so is the wait for them: nothing tells the compiler that their registers are not written yet.
+    Reads stay on their way from one block to the next, so the blocks' ends are followed until nothing is added."""
+    blocks, names, in_asm = [[]], {}, False
+    for line in body.split("\n"):
+        in_asm = (in_asm or "#APP" in line or "#ASMSTART" in line) and "#NO_APP" not in line and "#ASMEND" not in line
+        s = line.split(";")[0].strip()
+        label = re.fullmatch(r"(\.LBB\w+):", s)
+        if label:
+            blocks.append([])
+            names[label.group(1)] = len(blocks) - 1
+        elif s and not s.startswith("."):
+            blocks[-1].append((s, in_asm))
+            if s.startswith(("s_branch", "s_cbranch", "s_endpgm")):
+                blocks.append([])
+    found, reads = [], 0
+    seen, todo = [None] * len(blocks), [(0, frozenset())]
+    while todo:
+        at, pending = todo.pop()
+        if seen[at] is not None and pending <= seen[at]:
+            continue
+        seen[at] = pending = pending | (seen[at] or frozenset())
+        after = [at + 1]
+        for s, asm in blocks[at]:
+            assert not s.startswith(("s_setpc", "s_swappc", "s_call")), s
+            if s.startswith("s_endpgm"):
+                after = []
+            elif s.startswith("s_branch"):
+                after = [names[s.split()[1]]]
+            elif s.startswith("s_cbranch"):
+                after = [at + 1, names[s.split()[1]]]
+            elif s.startswith("s_waitcnt") and "lgkmcnt(0)" in s:
+                pending = frozenset()
+            else:
+                if _vector_registers(s) & pending:
+                    found.append(s)
+                if asm and re.match(r"ds_read_b(128|64_tr_b16)\b", s):   # (not the compiler's own reads)
+                    reads += 1
+                    pending |= _vector_registers(s.split(None, 1)[1].split(",")[0])
+        todo += [(b, pending) for b in after if b < len(blocks)]
+    return found, reads
+
+
+def _check_copied_ahead(kernels):
+    test_solo_kernels_do_not_spill(kernels)
+    test_accumulators_stay_in_their_registers_until_the_last_mfma_has_retired(kernels)
+    for name, body in kernels.items():
+        found, reads = fragments_touched_in_flight(body)
+        assert not found and reads > 0, (name, found[:3])
+
+
+def test_fragments_in_flight_are_found():
+    """What the check below is there for, in a few lines: a register moved in a loop's next turn, or behind a branch."""
+    loop = """
+.LBB0_1:
+  v_mfma_f32_16x16x32_bf16 a[0:3], v[0:3], v[4:7], a[0:3]
+  %s
+  ;;#ASMSTART
+  ds_read_b128 v[0:3], v9
+  ;;#ASMEND
+  s_cbranch_scc1 .LBB0_1
+  s_branch .LBB0_2
+.LBB0_2:
+  %s
+  v_mov_b32_e32 v20, v1
+  s_endpgm
+"""
+    wait = "s_waitcnt lgkmcnt(0)"
+    assert fragments_touched_in_flight(loop % (wait, wait))[0] == ["v_mfma_f32_16x16x32_bf16 a[0:3], v[0:3], v[4:7], a[0:3]"]
+    loop = loop.replace("  v_mfma", "  s_waitcnt lgkmcnt(0)\n  v_mfma")
+    assert fragments_touched_in_flight(loop % ("", wait)) == ([], 2)   # (the loop's block is gone through twice)
+    assert fragments_touched_in_flight(loop % ("", "s_waitcnt vmcnt(0)"))[0][0] == "v_mov_b32_e32 v20, v1"
+
+
+@pytest.mark.parametrize("source,count", [("gemm_fed_rounds", 4), ("gemm_gate_up", 14), ("gemm_fed_nt_bf16", 72),
+                                          ("gemm_fed_nt_f16", 72), ("gemm_fed_nn_tn_bf16", 36), ("gemm_fed_nn_tn_f16", 36)])
+def test_kernels_with_copying_waves_keep_the_same_properties(tmp_path_factory, source, count):
+    """And no instruction touches a fragment before its wait, on any way through the kernel: in gemm_fed_rounds the reads
+    of a tile's first fragments are on their way across the end of the loop over the tiles."""
+    kernels = {k: v for k, v in _device_asm(tmp_path_factory, source).items() if "gemm_" in k}
+    assert len(kernels) == count, sorted(kernels)
+    _check_copied_ahead(kernels)
+
+
+def test_main_loops_touch_no_fragment_before_its_wait(gemm_asm, tmp_path_factory):
+    """The same for the kernels of the other two files."""
+    for kernels in (gemm_asm, {k: v for k, v in _device_asm(tmp_path_factory, "gemm_edge_bf16").items() if "gemm_edge" in k}):
+        for name, body in kernels.items():
+            found, reads = fragments_touched_in_flight(body)
+            assert not found and reads > 0, (name, found[:3])
+
+
 def test_stream_kernels_touch_no_fragment_before_its_wait(tmp_path_factory):
     """The forward of a few tokens reads its fragments in asm statements and waits for them in another: until
     then no instruction names their registers."""

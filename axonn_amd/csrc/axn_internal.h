@@ -169,7 +169,7 @@ int launch_gemm_backward(const GemmArgs& dgrad, const GemmArgs& wgrad, bool half
 // FED_*: tiles of gemm_fed_tiles.h, one workgroup on a CU.
 enum EdgeTile {
   EDGE_256x256 = 0, EDGE_256x128 = 1, EDGE_128x128 = 2,
-  FED_64x64, FED_96x64, FED_64x128, FED_96x128, FED_128x128, FED_96x192, FED_128x192, FED_160x192, FED_128x256
+  FED_64x64, FED_96x64, FED_64x128, FED_96x128, FED_128x128, FED_96x192, FED_128x192, FED_160x192, FED_128x256, FED_256x128
 };
 constexpr int64_t kEdgeMaxLd = 1LL << 23;
 // Split contraction for problems with few output tiles: into how many parts and on which

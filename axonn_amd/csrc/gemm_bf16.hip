@@ -18,7 +18,8 @@
 //     works on a compact block of neighbouring tiles.
 //
 // One-wave-per-SIMD kernels (solo_gemm: gemm_*_solo_kernel at 256 x 256 and 128 x 128
-// tiles, gemm_*_swiglu_kernel; shapes made of whole tiles, contraction % 64 == 0, operands below 2 GiB): 4 waves, one per SIMD, each a
+// tiles, gemm_*_rest_kernel at 256 x 128, gemm_*_swiglu_kernel; shapes made of whole
+// tiles, contraction % 64 == 0, operands below 2 GiB): 4 waves, one per SIMD, each a
 // quarter of the tile on v_mfma_f32_16x16x32_{bf16,f16}; operand tiles go global -> LDS
 // directly (buffer loads to LDS, 16 bytes per lane, no registers) into a ring of five
 // 64-deep tiles; each wave pipelines its share of the copies and its LDS fragment reads
@@ -30,9 +31,8 @@
 // gate/up forward of a gated MLP gathers its column operand from two weight matrices
 // and applies silu(gate) * up in the epilogue.
 //
-// Kernels with copying waves of their own (fed_gemm: gemm_*_rest_kernel at 256 x 128, and the tiles of
-// gemm_fed_tiles.h): rests, and outputs that small tiles cover in one round of workgroups or two, of any shape
-// (fed_tile, gemm_plan).
+// Kernels with copying waves of their own (fed_gemm: the tiles of gemm_fed_tiles.h): rests, and outputs that small
+// tiles cover in one round of workgroups or two, of any shape (fed_tile, gemm_plan).
 //
 // Everything else (ragged shapes, contractions that are not multiples of 64, operands of
 // 2 GiB and more) runs on the same main loop with bounds: gemm_edge.h.
@@ -42,7 +42,7 @@
 #include <queue>
 #include <vector>
 
-#include "gemm_fed.h"
+#include "gemm_solo.h"
 
 namespace axn {
 namespace {
@@ -55,14 +55,17 @@ template <int TILE, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32>
 __global__ void __launch_bounds__(256) gemm_f16_solo_kernel(const GemmArgs g) {
   solo_gemm<TILE, TILE, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, true>(g);
 }
-// The 256 x 128 tile of the launches that finish a problem.
+// The 256 x 128 tile of the launches that finish a problem.  (As fed_gemm it takes longer, in one part or several: 260 input
+// gradients, 260 weight gradients and 231 forwards that the estimates give this tile, with bounds and without, 1.04, 1.02 and
+// 1.02 of the time on average, up to 1.16: 640 x 7936 over 3176 57.5 us, 63.9; 15872 x 256 over 4263 54.3, 61.8.  Rests of
+// more than 64 large tiles 1.00 to 1.015, whole problems of 65 to 128 of them 1.025.)
 template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32>
-__global__ void __launch_bounds__(512) gemm_bf16_rest_kernel(const GemmArgs g) {
-  fed_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, false, false>(g);
+__global__ void __launch_bounds__(256) gemm_bf16_rest_kernel(const GemmArgs g) {
+  solo_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, false>(g);
 }
 template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32>
-__global__ void __launch_bounds__(512) gemm_f16_rest_kernel(const GemmArgs g) {
-  fed_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, true, false>(g);
+__global__ void __launch_bounds__(256) gemm_f16_rest_kernel(const GemmArgs g) {
+  solo_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, true>(g);
 }
 
 // Weight gradient and input gradient of one layer in one launch, 256 x 256 tiles: the
@@ -130,7 +133,7 @@ int launch_rest(const GemmArgs& in, hipStream_t stream) {
   GemmArgs g = in;
   g.tiles_m = g.M / 256;
   g.tiles_n = g.N / 128;
-  constexpr size_t lds = kFedLds<256, 128>;
+  constexpr size_t lds = 5 * 256 * 64 * 2;   // five slots of the A tile's size
   void (*kern)(const GemmArgs) = gemm_bf16_rest_kernel<AK, BKM, EPI, OUT_F32>;
   if constexpr (HALF) kern = gemm_f16_rest_kernel<AK, BKM, EPI, OUT_F32>;
   {
@@ -139,7 +142,7 @@ int launch_rest(const GemmArgs& in, hipStream_t stream) {
     if (rc != AXN_OK) return rc;
   }
   const int splits = g.splits > 1 ? g.splits : 1;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(g.tiles_m * g.tiles_n * splits)), dim3(512), lds, stream, g);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(g.tiles_m * g.tiles_n * splits)), dim3(256), lds, stream, g);
   AXN_HIP_TRY(hipGetLastError());
   return AXN_OK;
 }
@@ -183,8 +186,8 @@ EpilogueTime epilogue_time(const GemmArgs& g, int epilogue, bool out_f32) {
   return t;
 }
 
-// The same for an unsplit M x N output as launch_edge_kind runs it: a last round of at most
-// half of the CUs goes to smaller tiles.
+// The same for an unsplit M x N output as launch_edge runs it: a last round of at most
+// half of the CUs goes to smaller tiles (fed ones among them, which this leaves out).
 double edge_microseconds(EdgeTile tile, long long M, long long N, long long Kc, const EpilogueTime& epilogue) {
   const int bm = tile == EDGE_128x128 ? 128 : 256, bn = tile == EDGE_256x256 ? 256 : 128;
   const long long w = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), full = w / 256, rest = w % 256;
@@ -248,7 +251,7 @@ constexpr FedTile kFedTiles[] = {
     {FED_128x192, 128, 192, {2.52f, 2.67f, 4.01f}, {0.564f, 0.595f, 0.528f}, {0.051f, 0.030f, 0.121f}, {0.45f, 0.48f, 0.15f}},
     {FED_160x192, 160, 192, {3.00f, 2.88f, 4.33f}, {0.609f, 0.662f, 0.620f}, {0.044f, 0.022f, 0.104f}, {0.41f, 0.44f, 0.15f}},
     {FED_128x256, 128, 256, {2.98f, 2.92f, 4.40f}, {0.683f, 0.686f, 0.627f}, {0.049f, 0.031f, 0.114f}, {0.39f, 0.42f, 0.15f}},
-    {EDGE_256x128, 256, 128, {3.35f, 2.45f, 4.41f}, {0.748f, 0.784f, 0.678f}, {0.010f, 0.000f, 0.091f}, {0.39f, 0.46f, 0.16f}},
+    {FED_256x128, 256, 128, {3.35f, 2.45f, 4.41f}, {0.748f, 0.784f, 0.678f}, {0.010f, 0.000f, 0.091f}, {0.39f, 0.46f, 0.16f}},
 };
 
 double fed_microseconds(const FedTile& t, GemmLayout layout, long long M, long long N, long long Kc, int parts,
@@ -326,14 +329,11 @@ EdgeTile rounds_tile(const GemmArgs& g) {
   if (tiles <= 512 || tiles > 65536) return EDGE_256x256;
   const long long rounds = ceil_div(tiles, 256);
   if (16 * rounds > (g.Kc <= 448 ? 16 : 15) * halves) return EDGE_256x256;
-  return wide <= tall ? FED_128x256 : EDGE_256x128;
+  return wide <= tall ? FED_128x256 : FED_256x128;
 }
 
 int launch_fed(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32, bool half, EdgeTile tile,
                hipStream_t stream) {
-  if (tile == EDGE_256x128)
-    return half ? launch_gemm_edge_f16(layout, g, epilogue, out_f32, tile, stream)
-                : launch_gemm_edge_bf16(layout, g, epilogue, out_f32, tile, stream);
   if (layout == GEMM_NT)
     return half ? launch_gemm_fed_nt_f16(g, epilogue, out_f32, tile, stream)
                 : launch_gemm_fed_nt_bf16(g, epilogue, out_f32, tile, stream);

@@ -14,18 +14,14 @@
 #pragma once
 #include <atomic>
 
-#include "gemm_fed.h"
+#include "gemm_solo.h"
 
 namespace axn {
 namespace {
 
-// Tiles that leave room for a second wave on a SIMD and give a CU one workgroup: fed_gemm.
-constexpr bool edge_tile_is_fed(int bm, int bn) { return bm != bn; }
-
 template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32, bool HALF, bool ODD = false>
-__global__ void __launch_bounds__(edge_tile_is_fed(BM, BN) ? 512 : 256) gemm_edge_kernel(const GemmArgs g) {
-  if constexpr (edge_tile_is_fed(BM, BN)) fed_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, true, ODD>(g);
-  else solo_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, true, ODD>(g);
+__global__ void __launch_bounds__(256) gemm_edge_kernel(const GemmArgs g) {
+  solo_gemm<BM, BN, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, HALF, true, ODD>(g);
 }
 
 // Both gradients of a layer in one launch, as gemm_backward_kernel.  PARTS: the input gradient's contraction is
@@ -55,15 +51,14 @@ int launch_edge_tile(const GemmArgs& in, hipStream_t stream) {
     set_error("gemm: too many output tiles (%lld)", nwg);
     return AXN_ELIMIT;
   }
-  constexpr bool fed = edge_tile_is_fed(BM, BN);
-  constexpr size_t lds = fed ? kFedLds<BM, BN> : 5 * BM * 64 * 2;   // else five slots of the A tile's size
+  constexpr size_t lds = 5 * BM * 64 * 2;   // five slots of the A tile's size
   void (*kern)(const GemmArgs) = gemm_edge_kernel<BM, BN, AK, BKM, EPI, OUT_F32, HALF, ODD>;
   {
     static std::atomic<unsigned long long> lds_allowed{0};   // per template instance
     const int rc = allow_lds((const void*)kern, lds, lds_allowed);
     if (rc != AXN_OK) return rc;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(fed ? 512 : 256), lds, stream, g);
+  hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(256), lds, stream, g);
   AXN_HIP_TRY(hipGetLastError());
   return AXN_OK;
 }

@@ -20,6 +20,8 @@ constexpr size_t kFedLds = (size_t)kFedStages<BM, BN> * (BM + BN) * 128;
 //   us of one round of 256 workgroups, contraction 4096, operands in the caches / from HBM:
 //     256 x 128 tiles   solo_gemm 60.0 / 64.7   here 52.5 / 59.7
 //     128 x 128 tiles             36.1 / 48.0        30.4 / 39.1
+//   That is a forward's whole round alone.  Between other launches, and over the sizes that take 256 x 128 tiles, solo_gemm is
+//   2 to 4 % ahead of this on them (gemm_*_rest_kernel); FED_256x128 runs where its own estimate is ahead (kFedTiles).
 //   Without its copies this kernel takes 43 us on 256 x 128 tiles, its copies alone 37 / 55: from HBM they are the bound.
 //   One, two or four copying waves, reads from the first or the fifth MFMA of a step on, s_setprio: all the same.
 //

@@ -46,6 +46,7 @@ int launch_fed_tile(const GemmArgs& g, EdgeTile tile, hipStream_t stream) {
     case FED_128x192: return launch_fed<128, 192, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
     case FED_160x192: return launch_fed<160, 192, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
     case FED_128x256: return launch_fed<128, 256, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
+    case FED_256x128: return launch_fed<256, 128, AK, BKM, EPI, OUT_F32, HALF>(g, stream);
     default: break;
   }
   set_error("gemm: no such tile");

@@ -585,6 +585,11 @@ __device__ __forceinline__ void store_gate_up(f32x4 (&acc)[FRM][FRN], const Gemm
 // fill the chip with 256 x 256 tiles: 64 x 64 per wave (4 x 4 blocks, 16 MFMAs per
 // step, 4 copies per tile and wave), an 80 KiB ring, two workgroups per CU.
 //
+// BM x BN = 256 x 128 is the tile of the launches that finish a problem after its full
+// rounds of 256 x 256 tiles: a rest of r <= 128 large tiles makes 2 r <= 256 of these,
+// one per CU, and needs 3/4 of the global -> LDS bytes per MFMA of the 128 x 128 tile.
+// Its ring has five slots of the larger (A) tile's size.
+//
 // EDGE: any M, N and contraction, operands of any size.  The main loop is the same; what is
 // added is
 //   * copies of rows past the end of an operand: the buffer's byte count ends at the last
@@ -619,7 +624,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g, const int tm, const
   constexpr int READ_EVERY = (NM / 2) / NFRAG;     // a fragment read every .. MFMAs, first half of a step
   constexpr int COPY_EVERY_A = (NM / 2) / NCA;     // a copy every .. MFMAs, second half
   constexpr int COPY_EVERY_B = (NM / 2) / NCB;
-  static_assert((BM == 128 && BN == 128) || (BM <= 256 && BN == 256), "tile sizes with a schedule below");
+  static_assert((BM <= 256 && BN == 256) || ((BM == 256 || BM == 128) && BN == 128), "tile sizes with a schedule below");
   static_assert(READ_EVERY >= 1 && COPY_EVERY_A >= 1 && COPY_EVERY_B >= 1, "schedule fits a step");
   // Gate/up forward (gate_up_copy): the tile covers 128 output columns.
   constexpr bool SWIGLU = EPI == EPI_SWIGLU;
@@ -630,7 +635,7 @@ __device__ __forceinline__ void solo_gemm(const GemmArgs& g, const int tm, const
   static_assert(!ODD || (A_KMAJOR && B_KMAJOR), "the forward");
   static_assert(!PAIR || (A_KMAJOR && !B_KMAJOR), "the two-term product is the dgrad layout");
   static_assert(!SWIGLU || (BN == 256 && A_KMAJOR && B_KMAJOR && !OUT_F32),
-                "the gate/up forward runs on the 256 x 256 tile with contraction-contiguous operands");
+                "the gate/up forward runs on tiles of 256 columns with contraction-contiguous operands");
 
   extern __shared__ __attribute__((aligned(16))) char lds[];
 

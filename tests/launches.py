@@ -13,8 +13,9 @@ class _KernelNodeParams(ctypes.Structure):   # hipKernelNodeParams
                 ("grid", ctypes.c_uint * 3), ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
 
 
-def launches(call):
-    """[(kernel name, number of workgroups), ...] of call(), which uses torch's current stream."""
+def launches(call, threads=False):
+    """[(kernel name, number of workgroups), ...] of call(), which uses torch's current stream; with `threads` the
+    threads of a workgroup behind them."""
     hip = ctypes.CDLL(glob.glob(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so*"))[0])
     hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
     hip.hipKernelNameRefByPtr.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
@@ -34,5 +35,6 @@ def launches(call):
         assert kind.value == 0, "a node that is no kernel"
         assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)) == 0
         name = hip.hipKernelNameRefByPtr(params.func, None)
-        found.append(((name or b"").decode(), params.grid[0] * params.grid[1] * params.grid[2]))
+        found.append(((name or b"").decode(), params.grid[0] * params.grid[1] * params.grid[2])
+                     + ((params.block[0] * params.block[1] * params.block[2],) if threads else ()))
     return found

@@ -16,7 +16,7 @@ from test_gemm_edge_gpu import canvas, check, numbers
 @pytest.mark.parametrize("source", ["gemm_fed_nt_f16", "gemm_fed_nn_tn_bf16"])
 def test_fed_kernels_keep_the_properties_of_the_others(tmp_path_factory, source):
     kernels = {k: v for k, v in codegen._device_asm(tmp_path_factory, source).items() if "gemm_fed_edge" in k}
-    assert len(kernels) == (72 if "nt" in source.split("_")[2] else 36), len(kernels)   # 9 tiles x 8 or 4 products
+    assert len(kernels) == (80 if "nt" in source.split("_")[2] else 40), len(kernels)   # 10 tiles x 8 or 4 products
     codegen.test_solo_kernels_do_not_spill(kernels)
     codegen.test_accumulators_stay_in_their_registers_until_the_last_mfma_has_retired(kernels)
 
@@ -100,3 +100,20 @@ def test_a_workspace_that_a_smaller_tile_does_without(M, N, K):
     if nbytes:
         with pytest.raises(nv.AxnError, match="workspace too small"):
             product(0, a, b, c, M, N, K, nv.BF16, nv.BF16, c.stride(0), ws[:-4])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op,M,N,K,workgroups", [
+    (1, 640, 3176, 7936, 186), (0, 704, 9856, 7392, 231),                           # one part, with bounds
+    (1, 1216, 5208, 2816, 220), (1, 320, 3648, 5376, 252), (2, 4263, 15872, 256, 248),   # parts
+    (1, 5120, 256, 1536, 240), (0, 256, 4096, 15360, 256),                          # whole tiles, and parts of them
+])
+def test_tiles_of_256_by_128_that_are_not_fed(op, M, N, K, workgroups):
+    """Where the estimate of the one-wave tile picks 256 x 128, that tile runs: four waves, not eight."""
+    shapes = (((M, K), (N, K), (M, N)), ((M, N), (N, K), (M, K)), ((M, N), (M, K), (N, K)))[op]
+    a, b, c = (torch.zeros(*s, device="cuda", dtype=torch.bfloat16) for s in shapes)
+    nbytes = nv.load().axn_gemm_workspace_bytes(op, M, N, K)
+    ws = torch.empty(nbytes // 4, device="cuda") if nbytes else None
+    found = launches(lambda: product(op, a, b, c, M, N, K, nv.BF16, nv.BF16, c.stride(0), ws), threads=True)
+    assert re.search(r"gemm_(edge|bf16_rest)_kernel", found[0][0]) and "fed" not in found[0][0], found
+    assert found[0][1:] == (workgroups, 256) and len(found) == (2 if nbytes else 1), found

@@ -200,8 +200,8 @@ def test_fragments_in_flight_are_found():
     assert fragments_touched_in_flight(loop % ("", "s_waitcnt vmcnt(0)"))[0][0] == "v_mov_b32_e32 v20, v1"
 
 
-@pytest.mark.parametrize("source,count", [("gemm_fed_rounds", 4), ("gemm_gate_up", 14), ("gemm_fed_nt_bf16", 72),
-                                          ("gemm_fed_nt_f16", 72), ("gemm_fed_nn_tn_bf16", 36), ("gemm_fed_nn_tn_f16", 36)])
+@pytest.mark.parametrize("source,count", [("gemm_fed_rounds", 4), ("gemm_gate_up", 14), ("gemm_fed_nt_bf16", 80),
+                                          ("gemm_fed_nt_f16", 80), ("gemm_fed_nn_tn_bf16", 40), ("gemm_fed_nn_tn_f16", 40)])
 def test_kernels_with_copying_waves_keep_the_same_properties(tmp_path_factory, source, count):
     """And no instruction touches a fragment before its wait, on any way through the kernel: in gemm_fed_rounds the reads
     of a tile's first fragments are on their way across the end of the loop over the tiles."""

@@ -342,7 +342,7 @@ static int gemm_ws(const char* name, int op, const void* a, const void* b, void*
     REQUIRE(given || !refused || workspace_bytes >= need, AXN_EINVAL,
             "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
     REQUIRE(given || !refused, AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
-    if (given) plan = gemm_plan(layout, g.M, g.N, g.Kc);
+    if (given) plan = gemm_plan(layout, g, epilogue, out_dtype == AXN_F32);
   }
   if (plan.parts > 1)
     return launch_gemm_splitk(layout, g, epilogue, half, out_dtype == AXN_F32, plan, (float*)workspace,
@@ -396,7 +396,7 @@ int axn_gemm_any_n(int op, const void* A, const void* B, const void* bias, void*
     REQUIRE(workspace_bytes >= need, AXN_EINVAL,
             "%s: workspace too small (%zu bytes given, %zu needed)", name, workspace_bytes, need);
     REQUIRE(aligned16(workspace), AXN_EALIGN, "%s: workspace must be 16-byte aligned", name);
-    plan = gemm_plan(layout, g.M, g.N, g.Kc);
+    plan = gemm_plan(layout, g, epilogue, out_f32);
     if (plan.parts > 1)
       return launch_gemm_splitk(layout, g, epilogue, half, out_f32, plan, (float*)workspace, (hipStream_t)stream, widen);
     if (widen) {   // in one part after all: 16 bits into the workspace, which is larger than that

@@ -183,7 +183,7 @@ struct SplitPlan {
 SplitPlan gemm_splits(GemmLayout layout, int64_t M, int64_t N, int64_t Kc, double* us = nullptr);
 // What a call with the workspace for gemm_splits' parts does: those parts or fewer, on the tile that is estimated to
 // be fastest.
-SplitPlan gemm_plan(GemmLayout layout, int64_t M, int64_t N, int64_t Kc);
+SplitPlan gemm_plan(GemmLayout layout, const GemmArgs& args, int epilogue, bool out_f32);
 // widen (input gradient): the result is rounded to the operands' type and stored as fp32.
 int launch_gemm_splitk(GemmLayout layout, const GemmArgs& args, int epilogue, bool half, bool out_f32,
                        const SplitPlan& plan, float* ws, hipStream_t stream, bool widen = false);

@@ -117,3 +117,23 @@ def test_tiles_of_256_by_128_that_are_not_fed(op, M, N, K, workgroups):
     found = launches(lambda: product(op, a, b, c, M, N, K, nv.BF16, nv.BF16, c.stride(0), ws), threads=True)
     assert re.search(r"gemm_(edge|bf16_rest)_kernel", found[0][0]) and "fed" not in found[0][0], found
     assert found[0][1:] == (workgroups, 256) and len(found) == (2 if nbytes else 1), found
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,epilogue", [(2366, 256, 3712, nv.EPI_GELU), (1007, 512, 3200, nv.EPI_GELU),
+                                            (3211, 1024, 5504, nv.EPI_BIAS | nv.BIAS_16BIT)])
+def test_a_round_of_tiles_has_its_epilogue_counted(M, N, K, epilogue):
+    """One part without an epilogue; parts, whose sum has it for little, with one.  Both are right."""
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    x, w = numbers(M, K, torch.bfloat16, gen, 16), numbers(N, K, torch.bfloat16, gen, 16)
+    bias = torch.randint(-3, 4, (N,), generator=gen, device="cuda").bfloat16() if epilogue & nv.BIAS_16BIT else None
+    y = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+    nbytes = nv.load().axn_gemm_workspace_bytes(0, M, N, K)
+    ws = torch.empty(nbytes // 4, device="cuda")
+    call = lambda epi: product(0, x, w, y, M, N, K, nv.BF16, nv.BF16, N, ws, bias=bias if epi else None, epilogue=epi)   # noqa: E731
+    assert [len(launches(lambda: call(epi))) for epi in (nv.EPI_NONE, epilogue)] == [1, 2]
+    call(epilogue)
+    want = (x.double() @ w.double().t())
+    want = want + bias.double() if bias is not None else torch.nn.functional.gelu(want)
+    # exact sums, one rounding to 8 bits; the activation's own error is 2^-20 of its argument at most
+    assert float(((y.double() - want).abs() / want.abs().clamp(min=1.0)).max()) <= 2.0 ** -8

@@ -318,22 +318,30 @@ const FedTile* fed_tile(GemmLayout layout, const GemmArgs& g, int epilogue, bool
 
 // The tile of a 16-bit weight gradient that is done in more than two rounds of workgroups that stay
 // (gemm_fed_rounds.hip), or EDGE_256x256 where the others are ahead.  Such a launch saves what the tiles' ramps and
-// stores cost a short contraction, and ends on a finer last round than 256 x 256 tiles; what it loses is their rate.  So
-// the line lies at the contraction (the tokens): up to 448 it may take as many half rounds as they do, up to 800 it has to
-// save a sixteenth, and 264 and less are stores in any tile.  us, before / so, of 103 gradients of 265 to 800 tokens
-// over 1024 to 50264 features with more than 512 tiles, ragged ones most: where it is taken 0.90 of the time on average,
-// 1.02 at worst.  Since a tile's stores wait for the next tile's first fragments (2 %): of 70 drawn anew that it takes 0.93,
-// six slower (381 x 12416 x 1632 23.9 / 25.9, the others 2 to 5 %).  Before that wait 447 x 12288 x 2048 38.7 / 29.1,
-// 404 x 9600 x 2368 35.7 / 28.1, 748 x 6016 x 2880 43.3 / 36.7, 430 x 12096 x 2304 35.4 / 36.1.  Left out: 657 x 8960 x 3584 47.6 / 49.5, 768 x 8192 x 8192 98 / 112.  fp32 results and
-// adding to one are bound by the output (382 x 4160 x 5632 fp32 35.6 / 39.7, 349 x 6784 x 4808 added to 46 / 57).
+// stores cost a short contraction, and ends on a finer last round than 256 x 256 tiles; what it loses is their rate.
+// Both sides are estimated in us: rounds, their stages, the output's and the operands' megabytes; the others' last round
+// of up to 128 tiles is one of smaller ones.  Fitted to 700 gradients of 265 to 800 tokens over 1024 to 50264 and 512 to
+// 8192 features with more than 512 tiles (7 and 5 % rms); 264 tokens and less are stores in any tile.  Of 700 drawn
+// anew 309 are taken, with 0.92 of the time that they have elsewhere, 12 of them 3 to 7 % slower (counting half rounds of
+// 256 x 256 tiles instead took 531, with 0.954 and 77 of them 3 to 18 % slower).  us, elsewhere / so, operands from HBM:
+// 447 x 12288 x 2048 44.7 / 34.3, 404 x 9600 x 2368 40.7 / 32.0, 320 x 16384 x 3584 64.2 / 59.8, 748 x 6016 x 2880 45.0 / 42.2;
+// left out 440 x 8288 x 3736 42.2 / 54.6, 708 x 8192 x 2304 36.0 / 44.5, 512 x 8192 x 3584 42.5 / 49.2, 768 x 8192 x 8192 112 /
+// 138.  fp32 results and adding to one are bound by the output (382 x 4160 x 5632 fp32 35.6 / 39.7, 349 x 6784 x 4808 added
+// to 46 / 57).
 EdgeTile rounds_tile(const GemmArgs& g) {
   if (g.Kc <= 264 || g.Kc > 800 || g.beta || g.splits > 1 || (g.lda > g.ldb ? g.lda : g.ldb) >= kEdgeMaxLd / 2) return EDGE_256x256;
   if (g.N % 8 != 0 || g.ldc % 8 != 0) return EDGE_256x256;   // (columns that it does not store)
   const long long wide = ceil_div(g.M, 128) * ceil_div(g.N, 256), tall = ceil_div(g.M, 256) * ceil_div(g.N, 128);
-  const long long tiles = wide <= tall ? wide : tall, halves = 2 * ceil_div(ceil_div(g.M, 256) * ceil_div(g.N, 256), 256);
+  const long long tiles = wide <= tall ? wide : tall;
   if (tiles <= 512 || tiles > 65536) return EDGE_256x256;
-  const long long rounds = ceil_div(tiles, 256);
-  if (16 * rounds > (g.Kc <= 448 ? 16 : 15) * halves) return EDGE_256x256;
+  const double stages = (double)ceil_div(g.Kc, 64), out = (double)g.M * (double)g.N * 2e-6;
+  const double in = ((double)g.M + (double)g.N) * (double)g.Kc * 2e-6;
+  const double here = 7.3 + (double)ceil_div(tiles, 256) * (0.688 * stages - 1.22) + 0.27 * out + 0.16 * in;
+  const long long tm = ceil_div(g.M, 256), tn = ceil_div(g.N, 256), full = tm * tn / 256, rest = tm * tn % 256;
+  const bool cut = full > 0 && rest > 0 && rest <= 128 && (full * 256 % tm == 0 || full * 256 % tn == 0);
+  const double last = rest == 0 ? 0.0 : !cut ? 0.78 + 1.217 * stages : rest > 64 ? 5.0 + 0.587 * stages : 3.8 + 0.28 * stages;
+  const double others = 4.8 + (double)full * (0.78 + 1.217 * stages) + last + 0.234 * out + 0.101 * in;
+  if (here > 0.95 * others) return EDGE_256x256;
   return wide <= tall ? FED_128x256 : FED_256x128;
 }
 

@@ -2,8 +2,9 @@
 //
 // What bounds them on other kernels: a tile is 5 to 13 stages, about 0.7 us each, and its ramp (2 to 3 us until the first
 // stage has come from HBM) and its stores are as long again.  Here the copying waves go on to the next tile's stages while
-// the matrix waves store.  us, 512 x 8192 x 3584 (tokens, out, in): 256 x 256 tiles 39 to 46, fed_gemm with a workgroup a
-// tile 43, here 37; 250 x 4096 x 14336 49.9, here 42.0; 1000 tokens and more are as fast or faster on 256 x 256 tiles.
+// the matrix waves store.  us (tokens x out x in), the other kernels / this: 447 x 12288 x 2048 44.7 / 34.3, 404 x 9600 x
+// 2368 40.7 / 32.0, 320 x 16384 x 3584 64.2 / 59.8; where rounds_tile leaves it out 512 x 8192 x 3584 42.5 / 49.2, 1000 x
+// 8192 x 3584 63.2 / 75.8.
 // 128 x 128 and 160 x 192 tiles are behind these two (404 to 1014 tokens: 0 to 25 %).  The sums' order is the same.
 #include <atomic>
 

@@ -14,9 +14,9 @@ pytestmark = pytest.mark.gpu
 SHAPES = [   # and the tile that covers the gradient in fewer of them
     (265, 8200, 2056, "256, 128"),     # the fewest tokens, a broken stage, rows and columns past the edges, 2 to 3 tiles each
     (320, 16384, 3584, "128, 256"),    # whole tiles, 7 rounds
-    (448, 12288, 2048, "128, 256"),    # the most tokens of the first rule, 3 whole rounds
+    (448, 12288, 2048, "128, 256"),    # whole tiles, 3 whole rounds
     (447, 3336, 5128, "128, 256"),     # the last of a CU's is another tile column
-    (799, 6016, 2880, "256, 128"),     # the second rule's end
+    (799, 6016, 2880, "256, 128"),     # nearly the most tokens
     (300, 33000, 520, "256, 128"),     # tall
 ]
 
@@ -33,6 +33,7 @@ def tile_in_rounds(call):
     (264, 8200, 2056, False, None), (801, 6016, 2880, False, None),          # fewer tokens, more
     (320, 8192, 2048, False, None),                                          # two rounds
     (449, 16384, 4096, False, None), (512, 8192, 3584, False, None),         # as many half rounds as large tiles take
+    (440, 8288, 3736, False, None), (708, 8192, 2304, False, None), (787, 34048, 1024, False, None),   # measured slower in rounds
     (320, 16384, 3584, True, None), (320, 16384, 3584, False, torch.float32),   # bound by the output
 ])
 def test_what_the_rule_leaves_to_others(tokens, out_features, in_features, add, dtype):

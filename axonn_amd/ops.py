@@ -563,11 +563,17 @@ def gemm_swiglu_few_supported(M, N, K, dtype):
 
 
 def gemm_swiglu_any_supported(M, N, K, dtype):
-    """The same for any number of tokens: products large enough that their launches are not all there is to them
-    (two products and the activation of 160 layers of 65 to 4096 tokens: 0.73 of their time in one launch on
-    average, 1.01 at worst)."""
-    return (dtype in _GEMM16 and M > 64 and N > 0 and N % 8 == 0 and K > 0 and K % 8 == 0 and M * N * K >= 1 << 28
-            and K < _FAR_ROWS and M <= 0x7fffffff and N <= 0x7fffffff)
+    """The same for any number of tokens: products large enough that their launches are not all there is to them, and
+    not so few tiles that each alone would have its contraction in many parts, which one launch of both does not (nor where
+    it is long and its rows do not fill 128-byte lines, in parts at all).  Of 700 layers of 65 to 4096 tokens, 512 to 16384
+    features and hidden sizes of 512 to 8192, 584 are so: one launch has 0.73 of the time of two products and the activation
+    on average, 13 take 3 to 15 % longer.  The others 74 x 512 over 7752 30 us, 71 in one launch; 124 x 1344 over 6024
+    36, 70; 226 x 8768 over 6840 128, 165."""
+    if not (dtype in _GEMM16 and M > 64 and N > 0 and N % 8 == 0 and K > 0 and K % 8 == 0 and M * N * K >= 1 << 28
+            and K < _FAR_ROWS and M <= 0x7fffffff and N <= 0x7fffffff):
+        return False
+    parts = _workspace_bytes(GEMM_FWD, M, N, K) // (4 * M * N)   # fp32 results of each
+    return parts <= (0 if K % 64 and K > 6000 else 5)
 
 
 def gemm_swiglu_fwd(x, w_gate, w_up, save=True, few=False, any_sizes=False):

@@ -341,3 +341,16 @@ def test_padded_rows_as_long_as_far_rows_are_not_packed_again(monkeypatch):
         dy8 = torch.zeros(2, ld).bfloat16()[:, :n8]
         at, stride = ops._prep_bf16(dy8)
         assert at.data_ptr() == dy8.data_ptr() and stride == ld
+
+
+@pytest.mark.parametrize("sizes, one", [
+    ((777, 14336, 4096), True), ((300, 11008, 4096), True), ((79, 2528, 1536), True), ((2006, 520, 4288), True),
+    ((549, 11392, 7168), True), ((4000, 10752, 3072), True),
+    ((74, 512, 7752), False), ((124, 1344, 6024), False), ((130, 768, 7296), False),    # few tiles, many parts
+    ((226, 8768, 6840), False), ((701, 3328, 6600), False),                            # few parts, broken lines
+    ((64, 14336, 4096), False), ((100, 512, 512), False), ((777, 14336, 4100), False),   # few tokens, small, no vectors
+])
+def test_gate_and_up_in_one_launch_where_their_contraction_is_not_in_many_parts(sizes, one):
+    """(tokens, features, hidden size).  One launch has no parts: 74 tokens took 71 us so, 30 in two products."""
+    assert ops.gemm_swiglu_any_supported(*sizes, torch.bfloat16) is one
+    assert not ops.gemm_swiglu_any_supported(*sizes, torch.float32)

@@ -927,7 +927,11 @@ int launch_waves(long long tiles, const float* A, const float* B, float* C, cons
 // gradient) and 0.83 (weight gradient) of the time of gemm_f32_kernel on average and 1 to 2 % more than the best.  That one
 // stays ahead with short contractions (forward 924 x 336, contraction 164: 8.2 us, 8.9 here; weight gradients under 50 to
 // 100 tokens: 5696 x 960, 72 tokens 16.5, 19.1): there its waves have all they multiply in flight at once.
+// Weight gradients of up to 32 tokens are one unit a wave: with less than two 16 x 16 tiles for a SIMD its copy and its wait
+// are all there is to them (128 x 128, 22 tokens 3.3 us, 3.7 here, added to 5.2, 7.2; 1088 x 128, 30 tokens, added to 5.6,
+// 7.6; from 2300 tiles on 0.7 to 0.8 of the time).
 int copied_blocks(GemmLayout layout, const NativeTiles& t, bool together, int64_t M, int64_t N, int64_t Kc) {
+  if (layout == GEMM_TN && Kc <= 32 && t.size == 16 && t.count < 2048) return 0;
   struct Fit {
     double fixed, serial, load, round, out;   // a launch, a unit of a wave, of all on a CU, a round, 2^20 results or so
   };

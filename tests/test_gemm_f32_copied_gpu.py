@@ -64,3 +64,17 @@ def test_infinities_and_nans_stay_where_they_belong():
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
     back, want = ops.gemm_dgrad(want.float().nan_to_num(1, 2, 3), w), want.float().nan_to_num(1, 2, 3).double() @ w.double()
     assert torch.equal(back.isnan(), want.isnan()) and torch.equal(back.isinf(), want.isinf())
+
+
+@pytest.mark.parametrize("tokens,out_features,in_features,copied", [
+    (22, 128, 128, False), (30, 1088, 128, False), (32, 64, 320, False), (21, 2240, 224, False), (24, 320, 1472, False),   # one unit a wave
+    (32, 512, 1408, True), (18, 240, 3840, True), (64, 1024, 1024, True),
+])
+def test_few_small_weight_gradients_are_loaded_directly(tokens, out_features, in_features, copied):
+    dy, x = torch.randn(tokens, out_features, device="cuda"), torch.randn(tokens, in_features, device="cuda")
+    out = torch.randn(out_features, in_features, device="cuda")
+    want = out.double() + dy.double().t() @ x.double()
+    dw = out.clone()
+    assert any("gemm_f32_copied_kernel" in n for n, _ in launches(lambda: ops.gemm_wgrad(dy, x, out=dw, accumulate=True))) == copied
+    got = ops.gemm_wgrad(dy, x, out=out, accumulate=True)
+    assert float((got.double() - want).norm() / want.norm()) < 2 * 2.0 ** -24 * (5 + (tokens / 4) ** 0.5)

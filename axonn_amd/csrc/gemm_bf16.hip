@@ -155,7 +155,7 @@ int launch_rest(const GemmArgs& in, hipStream_t stream) {
 //               times the rounds of workgroups;
 //   operands    never faster than 1.7 + their bytes at 5.7 TB/s, which they reach only with a
 //               workgroup on every CU (9 % of it with none, linear between).
-// The constants were fitted to 3479 launches: every tile size and split of 220 forward and
+// (256 x 128 tiles are the one-wave kernel's.)  The constants were fitted to 3479 launches: every tile size and split of 220 forward and
 // input-gradient problems of 33 to 3000 tokens and 768 to 14336 features, ragged and whole.
 // `epilogue`: what the output's epilogue adds to a round, on each of the four.
 struct EpilogueTime {
@@ -303,10 +303,11 @@ double other_microseconds(GemmLayout layout, double us, long long M, long long N
 }
 
 // The fed tile of a contraction in one part, or null where the others are ahead or less than 5 % behind.  With the parts
-// of gemm_plan, 700 products drawn anew have 0.85 (forward), 0.86 (input gradient) and 0.98 (weight gradient) of the
-// time they had on average; 18 got 4 to 11 % slower (385 x 2848 over 3648 26 -> 29 us).  us, before / so, outputs over
-// contractions, operands from HBM: 512 x 8192, 3584 43.0 / 38.5; 777 x 6144, 4096 60 / 51; 250 x 1024, 1024 14.8 / 7.7;
-// 2006 x 2432, 1088 19.3 / 17.1; weight gradient 2440 x 2240, 800 18.6 / 16.6.
+// of gemm_plan: of 1500 products drawn anew (1 to 8192 tokens, 256 to 16384 features; a third each forwards, input and weight
+// gradients) those that take a fed tile have 0.71 (forward), 0.73 and 0.77 of the time of the other tiles in one part, 0.82,
+// 0.86 and 0.93 in several; 18 got 3 to 15 % slower (315 x 2304 x 9024, weight gradient, 26 -> 30 us; 640 x 2560 over 4480 with
+// bias 32 -> 35).  us, before / so, outputs over contractions, operands from HBM: 512 x 8192, 3584 45.4 / 42.5; 777 x 6144, 4096
+// 57 / 49; 250 x 1024, 1024 15.0 / 8.2; 2006 x 2432, 1088 20.9 / 18.6; weight gradient 2440 x 2240, 800 18.9 / 17.5.
 const FedTile* fed_tile(GemmLayout layout, const GemmArgs& g, int epilogue, bool out_f32) {
   if (g.splits > 1 || (g.lda > g.ldb ? g.lda : g.ldb) >= kEdgeMaxLd / 2) return nullptr;
   double us = 0, other = 0;
@@ -940,7 +941,7 @@ int launch_gemm_splitk(GemmLayout layout, const GemmArgs& in, int epilogue, bool
 // ---- both gradients in one launch, the input gradient's contraction in parts -----------
 // An input gradient of few tiles and its weight gradient each end in a ramp and a last wave of their own; in one
 // launch the shorter tiles fill what the longer leave.  us, two launches and the sum / one and the sum: 1722 x 5888
-// x 1024 69 / 55, 1376 x 9088 x 2112 141 / 118, 599 x 32000 x 1088 143 / 118, 777 x 6144 x 4096 105 / 86.
+// x 1024 69 / 54, 1376 x 9088 x 2112 139 / 127, 599 x 32000 x 1088 128 / 121, 777 x 6144 x 4096 109 / 89.
 namespace {
 // Time until n1 tiles of s1 and then n2 of s2, each on the CU that is free first, are done.
 double filled(long long n1, double s1, long long n2, double s2) {
@@ -974,8 +975,10 @@ double filled(long long n1, double s1, long long n2, double s2) {
 //                                                                                         512 x 11008 x 8192 186 / 196
 //   adding to dW in tiles that reach past its edge where those of two launches do not      256 x 18560 x 5632 209 / 236
 //   adding to more than 256 tiles of dW from at most 256 rows with bounds                  237 x 13312 x 5376 154 / 180
-// Of 857 problems drawn anew that it then takes, one launch has 0.88 of the time of two on average, 13 take 3 to 13 %
-// longer (3223 x 11176 x 1920, fp32 dW, 257 / 285; 512 x 5632 x 3328 64 / 69).
+// The estimates of two launches know neither gemm_fed_tiles.h's tiles nor gemm_plan's parts, which make them faster than
+// that; measured against what two launches do with both, free to take other parts, the rule holds: of 500 problems drawn
+// anew that it takes, one launch has 0.877 of their time on average, 15 take 3 to 15 % longer (2549 x 4032 x 1088, added to an
+// fp32 dW, 76 / 88; 284 x 15040 x 4800 123 / 139; 3223 x 11176 x 1920, fp32 dW, 283 / 296).
 int gemm_backward_parts(int64_t M, int64_t N, int64_t K, bool add) {
   if (M <= 192) return 0;
   double apart_d = 0, apart_w = 0;

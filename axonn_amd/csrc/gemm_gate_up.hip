@@ -4,8 +4,8 @@
 // What bounds it: the same as any product of twice the columns.  What it saves against two products and the activation:
 // a launch's ramp and last round (777 rows x 14336: 224 tiles of 256 x 256 each, 256 CUs), the activation's pass over
 // both, and where nothing is saved for a backward pass the writing of both.  us, two products and the activation / this,
-// operands from HBM: 777 x 14336 over 4096 220 / 178, 300 x 11008 over 4096 94 / 70, 150 x 8192 over 3072 49 / 32,
-// 1000 x 4096 over 1024 35 / 20, 4000 x 10752 over 3072 477 / 387.  What it loses is the parts of a long contraction over few
+// operands from HBM: 777 x 14336 over 4096 188 / 161, 300 x 11008 over 4096 94 / 74, 150 x 8192 over 3072 50 / 38,
+// 1000 x 4096 over 1024 34 / 22, 4000 x 10752 over 3072 477 / 393.  What it loses is the parts of a long contraction over few
 // tiles (74 x 512 over 7752 30 / 71): callers leave those to two products (584 of 700 layers are taken, 0.73 of the time
 // on average, 1.15 at worst).
 #include <atomic>

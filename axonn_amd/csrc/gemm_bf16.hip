@@ -57,8 +57,8 @@ __global__ void __launch_bounds__(256) gemm_f16_solo_kernel(const GemmArgs g) {
 }
 // The 256 x 128 tile of the launches that finish a problem.  (As fed_gemm it takes longer, in one part or several: 260 input
 // gradients, 260 weight gradients and 231 forwards that the estimates give this tile, with bounds and without, 1.04, 1.02 and
-// 1.02 of the time on average, up to 1.16: 640 x 7936 over 3176 57.5 us, 63.9; 15872 x 256 over 4263 54.3, 61.8.  Rests of
-// more than 64 large tiles 1.00 to 1.015, whole problems of 65 to 128 of them 1.025.)
+// 1.02 of the time on average, up to 1.16: 640 x 7936 over 3176 57.5 us, 63.9; 15872 x 256 over 4263 54.3, 61.8.  Whole
+// problems of 65 to 128 large tiles 1.025; rests: launch_shape.)
 template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_F32>
 __global__ void __launch_bounds__(256) gemm_bf16_rest_kernel(const GemmArgs g) {
   solo_gemm<256, 128, A_KMAJOR, B_KMAJOR, EPI, OUT_F32, false>(g);
@@ -485,8 +485,13 @@ int launch_shape(const GemmArgs& g, hipStream_t stream) {
         // with the 256 x 128 tile).
         const int64_t a_span = (int64_t)(AK ? g2.M : g2.Kc) * g2.lda * 2;
         const int64_t b_span = (int64_t)(BKM ? g2.N : g2.Kc) * g2.ldb * 2;
-        if (rest > 64 && a_span < (1LL << 31) && b_span < (1LL << 31))
+        if (rest > 64 && a_span < (1LL << 31) && b_span < (1LL << 31)) {
+          // From contractions of 2048 on (70 to 73 problems of whole tiles each) the tile with copying waves takes 0.992 of
+          // the whole time in weight gradients, 1.005 in forwards, 1.008 in input gradients (0.96 to 1.04 in all three).
+          if constexpr (order == GEMM_TN && EPI == AXN_EPI_NONE)
+            if (g2.Kc >= 2048) return launch_fed(order, g2, EPI, OUT_F32, HALF, FED_256x128, stream);
           return launch_rest<AK, BKM, EPI, OUT_F32, HALF>(g2, stream);
+        }
         if constexpr (EPI != EPI_PAIR) {
           if (const FedTile* t = fed_tile(order, g2, EPI, OUT_F32))
             return launch_fed(order, g2, EPI, OUT_F32, HALF, t->tile, stream);

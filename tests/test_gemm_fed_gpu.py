@@ -137,3 +137,28 @@ def test_a_round_of_tiles_has_its_epilogue_counted(M, N, K, epilogue):
     want = want + bias.double() if bias is not None else torch.nn.functional.gelu(want)
     # exact sums, one rounding to 8 bits; the activation's own error is 2^-20 of its argument at most
     assert float(((y.double() - want).abs() / want.abs().clamp(min=1.0)).max()) <= 2.0 ** -8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op,M,N,K,fed", [(2, 2048, 6144, 4096, True), (2, 4096, 6144, 4096, True), (2, 1984, 6144, 4096, False),
+                                          (0, 4096, 6144, 2048, False), (1, 4096, 2048, 6144, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rests_of_more_than_64_large_tiles(op, M, N, K, fed, dtype):
+    """One whole round and 128 tiles: those of a weight gradient of 2048 tokens on are the ones with copying waves."""
+    out, beta = (torch.float32, 1) if op == 2 and dtype == torch.float16 else (dtype, 0)
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    shapes = (((M, K), (N, K), (M, N)), ((M, N), (N, K), (M, K)), ((M, N), (M, K), (N, K)))[op]
+    a, b = (torch.randint(-2, 3, s, generator=gen, device="cuda").to(dtype) for s in shapes[:2])
+    c = torch.full(shapes[2], 3.0, device="cuda", dtype=out)
+    call = lambda: product(op, a, b, c, M, N, K, nv.dtype_code(dtype), nv.dtype_code(out), c.stride(0), None, beta=beta)   # noqa: E731
+    (first, n1, t1), (rest, n2, t2) = launches(call, threads=True)
+    assert "solo_kernel" in first and (n1, t1) == (256, 256) and n2 == 256, (first, n1, t1)
+    assert t2 == (512 if fed else 256) and ("gemm_fed_edge" in rest) == fed, (rest, t2)
+    c.fill_(3.0)
+    call()
+    rows = torch.randint(0, shapes[2][0], (128,), generator=gen, device="cuda")
+    left = {0: lambda: a[rows], 1: lambda: a[rows], 2: lambda: a[:, rows].t()}[op]().double().contiguous()
+    right = (b.t() if op == 0 else b).double().contiguous()
+    want = left @ right + 3.0 * beta
+    # whole numbers: exact in fp32 (the sums are below 2^24), one rounding to a 16-bit result
+    assert torch.equal(c[rows].double(), want.to(out).double())
